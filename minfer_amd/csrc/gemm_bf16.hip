@@ -296,66 +296,212 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN)) void tile_kernel(const 
 }
 
 // ------------------------------------------------------------------ tiled kernel, loads straight into LDS
-// A tile of 256 rows by BN weight rows on 8 waves, but k tiles of 64 travel global -> LDS
-// without passing registers (global_load_lds_dwordx4: lane i's 16 bytes land at the wave's LDS
-// base + 16 i), in two or three stages of (256 + BN) * 128 bytes, and the staging registers are
-// gone.  The widths: 256 (waves of 128 x 64, two stages of 64 KB) has the most products per
-// byte copied and is the fastest where its tiles fill the chip's rounds; 192 (waves of 64 x 96)
-// and 128 (waves of 64 x 64, three stages) make more, smaller tiles for products whose 256-wide
-// tiles would leave a round half empty (q|k|v and o of a prompt of 2,048 tokens: 144 and 112
-// such tiles for 256 CUs).
+// BM x BN tiles on 8 waves whose k tiles of 64 travel global -> LDS without passing registers
+// (global_load_lds_dwordx4: lane i's 16 bytes land at the wave's LDS base + 16 i).  A row of a k tile is one
+// 128-byte line, fetched by 8 adjacent lanes: what a CU can have in flight towards L2 is counted in requests, so every
+// request should be a whole line.  There is no room for padding in such a copy, so a row's eight 16-byte chunks are
+// stored permuted: chunk c of row r sits at position c ^ ((r >> 1) & 7), which spreads the rows that one pass of a
+// 16-byte fragment read covers over all banks.  Which chunk a lane fetches is free (its global address), so the
+// permutation costs nothing on the way in.
 //
-// A row of a k tile is one 128-byte line, fetched by 8 adjacent lanes: what a CU can have in
-// flight towards L2 is counted in requests, so every request should be a whole line (k tiles of
-// 32, half lines, drew markedly less).
+// What bounds a large product here is the chip's power: with the same schedule, zeros run at 2.0 PFLOP/s and random
+// values at 1.5 (8192^3), so what counts is energy a product and matrix cores that never wait.
+//  * 16x16x32 MFMA.  The 32x32x16 form at the same tiles and schedule: 486 us for 413 at 2,048 rows against 37,888 of
+//    3,584, 775 for 708 at 8192^3 (the same machine, random values).
+//  * The two waves of a SIMD take turns: one reads its fragments while the other multiplies.  A wave's part of a k tile
+//    is four products of a half of its rows with a half of its columns (A0 W0, A1 W0, A1 W1, A0 W1: one half changes at
+//    a time); between two of them it reads the half that comes new (slot of the other wave's products), and a barrier
+//    ends every slot.  Waves 4..7 run one slot behind waves 0..3.
+//  * A half of a stage is set out again in the slot after its last read (STAGES tiles ahead), so that nearly all of LDS
+//    is always on its way: at two stages of 256 x 256 a copy has seven of a k tile's eight slots to land.  The waits
+//    count copies (vmcnt), they never drain them.
+// At the widths of the 7B model (2,048 rows, random values): q|k|v (256 x 192) 77 us before, 61 now; o (256 x 128) 62 and
+// 50; gate|up (256 x 256) 540 and 430; 8192^3 890 and 715.  (Before: 32x32x16 MFMA, a k tile's fragments read in two halves
+// by all waves at once, one barrier and one wait a tile, 2-byte stores.)
 //
-// There is no room for padding in such a copy, so a row's eight 16-byte chunks are stored
-// permuted: chunk c of row r sits at position c ^ ((r >> 1) & 7), which spreads the 16 rows
-// that one pass of a 16-byte fragment read covers over all 64 banks.  Which chunk a lane fetches
-// is free (its global address), so the permutation costs nothing on the way in.
-//
-// The compiler does not know that these loads write LDS and so does not wait for them; the
-// kernel does, with vmcnt counts it keeps itself (4 + BN / 64 loads per wave and tile, in order)
-// and one barrier per tile: behind it, tile kt + 1 has landed for every wave, and the stage of
-// tile kt, which every wave holds in registers by then, is free to take tile kt + STAGES.
-// Needs 16-byte aligned rows and K a multiple of 64.  What keeps this kernel from the matrix
-// cores' own rate is where the copies' lines come from (HBM and other dies' share of the data),
-// not how the copies are issued: blocks that run side by side on an XCD must walk K in step, so
-// that a line one of them fetches is in that XCD's L2 for the others.
-constexpr int DMA_BM = 256, DMA_BK = 64;
+// The order of the copies of a tile, W0 A0 A1 W1, is the order of the reads; LA, LW0 and LW1 copies a wave.  At the end
+// of a product's read slot the half that the next slot but one reads must have landed for this wave (the barrier makes
+// it everyone's): the number of younger copies allowed in flight stands at each wait.  Why a half may be overwritten:
+// both groups have its last read back (lgkmcnt(0) in front of a barrier) at the latest one slot before the first
+// group sets the new copy out.
+// The compiler does not know that these loads write LDS and so does not wait for them.
+// Needs 16-byte aligned rows and K a multiple of 64, and operands below 4 GB (32-bit byte offsets).
+constexpr int DMA_BK = 64;
 
-// 16 bytes per lane from base + off (a wave-uniform base and a 32-bit byte offset per lane: one
-// register where a 64-bit address takes two, and no address arithmetic per copy)
 __device__ __forceinline__ void dma16(const bf16* base, unsigned off, unsigned lds_byte) {
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds_byte)
-               : "memory", "m0");
+               : "m0");
+}
+// at most N of this wave's youngest copies are in flight, and all its LDS reads are back
+template <int N>
+__device__ __forceinline__ void dma_wait() {
+  static_assert(N >= 0 && N < 64, "vmcnt has six bits");
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory");
+}
+__device__ __forceinline__ void dma_meet() {
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_sched_barrier(0);
 }
 
-// waits until at most `tiles` of the youngest k tiles' copies (LOADS a wave and tile) are in flight
-template <int LOADS>
-__device__ __forceinline__ void dma_wait(int tiles) {
-  if (tiles <= 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  else if (tiles == 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS) : "memory");
-  else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * LOADS) : "memory");
+// How the 8 waves of a block share a BM x BN tile, in blocks of 16 x 16 results.
+template <int BM, int BN>
+struct DmaTile {
+  static constexpr int WAVES_M = BM == 256 && BN != 256 ? 4 : 2, WAVES_N = 8 / WAVES_M;
+  static constexpr int ROWS = BM / WAVES_M, COLS = BN / WAVES_N;      // of a wave
+  static constexpr int I = ROWS / 16, IH = I / 2;                     // row blocks of a wave, of a half of A
+  static constexpr int J = COLS / 16, J0 = BN == 192 ? 4 : J / 2, J1 = J - J0;      // column blocks, of the halves of W
+  // a wave's column block j is the tile's block first(n) + j * STEP: neighbours, except where a wave's columns would not
+  // hold whole pairs of a gate block and its up block (two blocks further)
+  static constexpr bool PAIRED = J % 4 != 0;
+  static constexpr int STEP = PAIRED ? 2 : 1;
+  static __device__ __forceinline__ int first(int n) {
+    return !PAIRED ? n * J : J == 2 ? (n >> 1) * 4 + (n & 1) : n;
+  }
+  // copies per wave: a half of A; the halves of W
+  static constexpr int LA = BM / 128, LW0 = J0 * WAVES_N / 4, LW1 = J1 * WAVES_N / 4;
+  static constexpr int T = LW0 + 2 * LA + LW1;
+  static constexpr int STAGE = (BM + BN) * DMA_BK * 2;
+  static constexpr int OWN = 16 * 1024;       // LDS bytes of a wave in the epilogue
+  template <int STAGES> static constexpr int lds() { return STAGES * STAGE > 8 * OWN ? STAGES * STAGE : 8 * OWN; }
+  static_assert(ROWS % 32 == 0 && BM % 128 == 0 && (J0 * WAVES_N) % 4 == 0 && (J1 * WAVES_N) % 4 == 0, "whole copies per wave");
+  static_assert(32 * (COLS + 4) * 4 <= OWN && 32 * (COLS + 8) * 2 <= OWN, "the epilogue's rows fit");
+};
+
+// A wave's results, acc[i][j]: the lane's row is 16 i + lane % 16, its columns 16 j + 4 (lane / 16) + e.  They go through the
+// wave's own LDS in runs of 32 rows and leave in rows of 16 bytes a lane: straight from the registers every store would be
+// pieces of lines, 2 bytes a lane (506 us for 469 at 2,048 x 37,888 x 3,584).
+template <typename TT>
+__device__ __forceinline__ void dma_epilogue(floatx4 (&acc)[TT::I][TT::J], unsigned char* __restrict__ own,
+                                             const float* __restrict__ bias, void* __restrict__ C, int ldc, int M, int N, int epi,
+                                             int mw, int n0, int wn, int lane) {
+  constexpr int J = TT::J, STEP = TT::STEP, COLS = TT::COLS;
+  const int row = lane & 15, sub = (lane >> 4) * 4;
+  const int b0 = TT::first(wn);
+  auto column = [&](int c) { return n0 + (b0 + (c >> 4) * STEP) * 16 + (c & 15); };      // of the wave's column c
+  if (epi == EPI_F32 || epi == EPI_ACC_F32) {
+    constexpr int LD = COLS + 4, CH = COLS / 4;              // floats a staged row takes; chunks of four in it
+    float* st = reinterpret_cast<float*>(own);
+    const bool vec = ldc % 4 == 0 && (uintptr_t)C % 16 == 0;
+#pragma unroll
+    for (int h = 0; h < TT::I / 2; ++h) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < J; ++j) {
+          const floatx4 v = acc[h * 2 + i][j];
+          *reinterpret_cast<float4*>(st + (i * 16 + row) * LD + j * 16 + sub) = float4{v[0], v[1], v[2], v[3]};
+        }
+#pragma unroll 4
+      for (int x = lane; x < 32 * CH; x += 64) {
+        const int r = x / CH, c = (x % CH) * 4, m = mw + h * 32 + r, n = column(c);
+        float4 v = *reinterpret_cast<const float4*>(st + r * LD + c);
+        if (m >= M || n >= N) continue;
+        float* o = (float*)C + (size_t)m * ldc + n;
+        if (vec && n + 4 <= N) {
+          if (bias) v = float4{v.x + bias[n], v.y + bias[n + 1], v.z + bias[n + 2], v.w + bias[n + 3]};
+          if (epi == EPI_ACC_F32) { const float4 p = *reinterpret_cast<const float4*>(o); v = float4{p.x + v.x, p.y + v.y, p.z + v.z, p.w + v.w}; }
+          *reinterpret_cast<float4*>(o) = v;
+        } else {
+          const float e4[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (n + e < N) {
+              const float s = e4[e] + (bias ? bias[n + e] : 0.f);
+              o[e] = epi == EPI_ACC_F32 ? o[e] + s : s;
+            }
+        }
+      }
+    }
+    return;
+  }
+  constexpr int LD = COLS + 8;                               // bfloat16 values a staged row takes
+  bf16* st = reinterpret_cast<bf16*>(own);
+  const bool vec = ldc % 8 == 0 && (uintptr_t)C % 16 == 0;
+  // 32 staged rows of WIDTH values leave in chunks of eight: chunk c of a row to column `at(c)`, below `end`
+  auto leave = [&](auto WIDTH, int h, int end, auto at) {
+    constexpr int CH = decltype(WIDTH)::value / 8;
+#pragma unroll 4
+    for (int x = lane; x < 32 * CH; x += 64) {
+      const int r = x / CH, c = (x % CH) * 8, m = mw + h * 32 + r, n = at(c);
+      const bf16x8 v = *reinterpret_cast<const bf16x8*>(st + r * LD + c);
+      if (m >= M) continue;
+      bf16* o = (bf16*)C + (size_t)m * ldc + n;
+      if (vec && n + 8 <= end) {
+        *reinterpret_cast<bf16x8*>(o) = v;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          if (n + e < end) o[e] = v[e];
+      }
+    }
+  };
+  if (epi == EPI_SWIGLU) {
+    // the tile's blocks of 16 columns: two of gates, the two of their ups, ...; block b's outputs are 16 ((b / 4) 2 + b % 2) on.
+    // A wave holds gate block and up block as j and j + 2 (neighbours) or j and j + 1 (every second block).
+    auto gated = [&](auto act) {
+#pragma unroll
+      for (int h = 0; h < TT::I / 2; ++h) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int p = 0; p < J / 2; ++p) {
+            const int jg = TT::PAIRED ? 2 * p : (p >> 1) * 4 + (p & 1), ju = jg + 2 / STEP;
+            bf16x4 v;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = (bf16)act(acc[h * 2 + i][jg][e], acc[h * 2 + i][ju][e]);
+            *reinterpret_cast<bf16x4*>(st + (i * 16 + row) * LD + p * 16 + sub) = v;
+          }
+        leave(std::integral_constant<int, COLS / 2>{}, h, ldc, [&](int c) {
+          const int p = c >> 4, b = b0 + (TT::PAIRED ? 2 * p * STEP : (p >> 1) * 4 + (p & 1));
+          return (n0 >> 1) + ((b >> 2) * 2 + (b & 1)) * 16 + (c & 15);
+        });
+      }
+    };
+    if (bias) {
+      const float limit = *bias;
+      gated([=](float g, float u) { return clamped_gate(g, u, limit); });
+    } else {
+      gated([](float g, float u) { return swiglu_f(g, u, nullptr); });
+    }
+    return;
+  }
+  const float ap = epi == EPI_XIELU ? bias[N] : 0.f, an = epi == EPI_XIELU ? bias[N + 1] : 0.f;
+#pragma unroll
+  for (int h = 0; h < TT::I / 2; ++h) {
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      float b[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int n = column(j * 16 + sub + e);
+        b[e] = bias && n < N ? bias[n] : 0.f;
+      }
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        bf16x4 v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float z = acc[h * 2 + i][j][e] + b[e];
+          v[e] = (bf16)(epi == EPI_XIELU ? xielu_f(z, ap, an) : z);
+        }
+        *reinterpret_cast<bf16x4*>(st + (i * 16 + row) * LD + j * 16 + sub) = v;
+      }
+    }
+    leave(std::integral_constant<int, COLS>{}, h, N, column);
+  }
 }
 
-// BN: the tile's width (256 or 128); WAVES_M x (8 / WAVES_M): the grid of the 8 waves over the
-// tile; STAGES: k tiles of a tile in LDS (2 or 3), (256 + BN) * 128 bytes each.
-template <int BN, int WAVES_M, int STAGES, bool GROUPED = false>
-__global__ __launch_bounds__(512) void tile_dma_kernel(const bf16* __restrict__ A, int lda,
+template <int BM, int BN, int STAGES, bool GROUPED = false>
+__global__ __launch_bounds__(512, 2) void tile_dma_kernel(const bf16* __restrict__ A, int lda,
                                                        const bf16* __restrict__ W, int ldw,
                                                        const float* __restrict__ bias, void* __restrict__ C,
                                                        int ldc, int M, int N, int K, int epi, int tiles_m,
                                                        int xcd_remap, int k_per_split,
                                                        const RowGroup* __restrict__ groups = nullptr) {
-  constexpr int WAVES_N = 8 / WAVES_M;
-  constexpr int WM = DMA_BM / WAVES_M, WN = BN / WAVES_N;
-  constexpr int TM = WM / 32, TN = WN / 32;
-  constexpr int ROW = DMA_BK * 2;              // bytes of a row in LDS
-  constexpr int STAGE_BYTES = (DMA_BM + BN) * ROW;
-  constexpr int WB = BN / 64;                  // 1 KB blocks of the W tile that a wave copies
-  constexpr int LOADS = 4 + WB;                // copies per wave and k tile
-  static_assert(STAGES == 2 || STAGES == 3, "the waits count one or two tiles in flight");
+  using TT = DmaTile<BM, BN>;
+  constexpr int ROW = DMA_BK * 2, A_ST = BM * ROW, W_ST = BN * ROW, W_AT = STAGES * A_ST;
+  constexpr int I = TT::I, IH = TT::IH, J = TT::J, J0 = TT::J0, J1 = TT::J1, LA = TT::LA, LW0 = TT::LW0, LW1 = TT::LW1, T = TT::T;
   if (k_per_split > 0) {
     // K split over blockIdx.y (k_per_split a multiple of 64): this block multiplies its part of K
     // and stores 32-bit sums into its own [M][N] slab of C; another kernel adds the slabs
@@ -365,7 +511,7 @@ __global__ __launch_bounds__(512) void tile_dma_kernel(const bf16* __restrict__ 
     K = min(k_per_split, K - kb);
     C = (float*)C + (size_t)blockIdx.y * M * N;
   }
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];      // [stage][BM][64] of A, [stage][BN][64] of W
   int tile = blockIdx.x;
   if (xcd_remap) {
     const int n_tiles = gridDim.x, per = n_tiles / 8, rem = n_tiles % 8;
@@ -382,145 +528,181 @@ __global__ __launch_bounds__(512) void tile_dma_kernel(const bf16* __restrict__ 
     C = (float*)C + (size_t)first * ldc;
     bm = 0;
   }
-  const int m0 = bm * DMA_BM, n0 = bn * BN;
+  const int m0 = bm * BM, n0 = bn * BN;
   const int lane = threadIdx.x & 63;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int wm = (wid % WAVES_M) * WM, wn = (wid / WAVES_M) * WN;
-  const int fr = lane & 31, fk = lane >> 5;
+  const int grp = wid >> 2;                                  // waves w and w + 4 share a SIMD
+  const int wave_m = TT::WAVES_M == 2 ? grp : wid & 3, wave_n = TT::WAVES_M == 2 ? wid & 3 : grp;
+  const int fr = lane & 15, fk = lane >> 4;
 
-  floatx16 acc[TM][TN];
+  floatx4 acc[I][J];
 #pragma unroll
-  for (int i = 0; i < TM; ++i)
+  for (int i = 0; i < I; ++i)
 #pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+    for (int j = 0; j < J; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
 
-  // this lane's share of a tile's copy: wave `wid` moves the 1 KB blocks wid, 8 + wid, ... (8 rows
-  // each) of the A tile and of the W tile; the lane fetches row 8 b + lane / 8, the chunk that
-  // belongs at position lane % 8
+  // What a wave copies: pieces of 8 rows (1 KB), the lane row lane / 8 of a piece and the chunk that belongs at position
+  // lane % 8.  Half h of A: the rows of the row blocks h IH .. + IH - 1 of every row of waves; half h of W: the rows of
+  // the column blocks of that half of every column of waves.
   const unsigned lds0 = (unsigned)(uintptr_t)smem;
-  unsigned ga[4], gw[WB];                      // byte offsets from A and W (the host checks that they fit)
+  unsigned ga[2][LA], gw[LW0 + LW1], la[2][LA], lw[LW0 + LW1];
 #pragma unroll
-  for (int jj = 0; jj < 4; ++jj) {
-    const int r = 8 * (jj * 8 + wid) + (lane >> 3);
-    const int chunk = (lane & 7) ^ ((r >> 1) & 7);
-    ga[jj] = ((unsigned)min(m0 + r, M - 1) * (unsigned)lda + chunk * 8) * 2u;
-    if (jj < WB) gw[jj] = ((unsigned)min(n0 + r, N - 1) * (unsigned)ldw + chunk * 8) * 2u;
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int q = 0; q < LA; ++q) {
+      const int p = q * 8 + wid;                             // piece of the half: 2 IH pieces a row of waves
+      const int r0 = (p / (2 * IH)) * TT::ROWS + h * IH * 16 + (p % (2 * IH)) * 8, r = r0 + (lane >> 3);
+      ga[h][q] = ((unsigned)min(m0 + r, M - 1) * (unsigned)lda + ((lane & 7) ^ ((r >> 1) & 7)) * 8) * 2u;
+      la[h][q] = lds0 + r0 * ROW;
+    }
+#pragma unroll
+  for (int q = 0; q < LW0 + LW1; ++q) {
+    const int jh = q < LW0 ? J0 : J1, p = (q < LW0 ? q : q - LW0) * 8 + wid;       // 2 jh pieces a column of waves
+    const int b = TT::first(p / (2 * jh)) + ((q < LW0 ? 0 : J0) + (p % (2 * jh)) / 2) * TT::STEP;
+    const int r0 = b * 16 + (p & 1) * 8, r = r0 + (lane >> 3);
+    gw[q] = ((unsigned)min(n0 + r, N - 1) * (unsigned)ldw + ((lane & 7) ^ ((r >> 1) & 7)) * 8) * 2u;
+    lw[q] = lds0 + W_AT + r0 * ROW;
   }
-  // the copies of a wave for tile kt into stage st: four blocks of the A tile, then WB of the W tile
-  auto issue = [&](int kt, int st) {
-    const unsigned base = lds0 + (unsigned)st * STAGE_BYTES + wid * 1024;
-    const int k = kt * DMA_BK;
+  auto copy_a = [&](int kt, int st, auto HALF) {
+    constexpr int h = decltype(HALF)::value;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) dma16(A + k, ga[q], __builtin_amdgcn_readfirstlane(base + q * 8192));
-#pragma unroll
-    for (int q = 0; q < WB; ++q)
-      dma16(W + k, gw[q], __builtin_amdgcn_readfirstlane(base + DMA_BM * ROW + q * 8192));
+    for (int q = 0; q < LA; ++q) dma16(A + kt * DMA_BK, ga[h][q], __builtin_amdgcn_readfirstlane(la[h][q] + st * A_ST));
   };
-  // fragment reads: row R of a tile, chunk 4 half + 2 ks + fk of its 8, at position chunk ^ ((R >> 1) & 7)
+  auto copy_w = [&](int kt, int st, auto HALF) {
+    constexpr int h = decltype(HALF)::value;
+#pragma unroll
+    for (int q = h ? LW0 : 0; q < (h ? LW0 + LW1 : LW0); ++q)
+      dma16(W + kt * DMA_BK, gw[q], __builtin_amdgcn_readfirstlane(lw[q] + st * W_ST));
+  };
+  // fragment reads (16x16x32): row R, chunk 4 ks + fk of its 8, at position chunk ^ ((R >> 1) & 7)
   const int sw = (fr >> 1) & 7;
-  int offa[TM], offw[TN];
+  unsigned pa[2], pw[2];
 #pragma unroll
-  for (int i = 0; i < TM; ++i) offa[i] = (wm + i * 32 + fr) * ROW;
-#pragma unroll
-  for (int j = 0; j < TN; ++j) offw[j] = DMA_BM * ROW + (wn + j * 32 + fr) * ROW;
-
-  const int nkt = K / DMA_BK;
-  // A tile is multiplied in two halves of two k-steps, from two register sets: the fragments of
-  // the next half are read from LDS while the second k-step of this one runs, so that behind the
-  // barrier there is always work for the matrix cores.
-  bf16x8 fa[2][2][TM], fw[2][2][TN];          // [set][k-step][tile]
-  auto read_frags = [&](int stage, auto HALF) {
-    constexpr int half = decltype(HALF)::value;          // which is also the register set
-    const unsigned char* st = smem + stage * STAGE_BYTES;
-    const int pos0 = ((half * 4 + fk) ^ sw) * 16, pos1 = ((half * 4 + 2 + fk) ^ sw) * 16;
-#pragma unroll
-    for (int i = 0; i < TM; ++i) fa[half][0][i] = *reinterpret_cast<const bf16x8*>(st + offa[i] + pos0);
-#pragma unroll
-    for (int j = 0; j < TN; ++j) fw[half][0][j] = *reinterpret_cast<const bf16x8*>(st + offw[j] + pos0);
-#pragma unroll
-    for (int i = 0; i < TM; ++i) fa[half][1][i] = *reinterpret_cast<const bf16x8*>(st + offa[i] + pos1);
-#pragma unroll
-    for (int j = 0; j < TN; ++j) fw[half][1][j] = *reinterpret_cast<const bf16x8*>(st + offw[j] + pos1);
-  };
-  auto multiply = [&](int ks, auto SET) {
-    constexpr int set = decltype(SET)::value;
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j)
-        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[set][ks][i], fw[set][ks][j], acc[i][j], 0, 0, 0);
-  };
-  using S0 = std::integral_constant<int, 0>;
-  using S1 = std::integral_constant<int, 1>;
-  // tiles 0 .. STAGES - 1 set out at once; tile 0 has landed (for this wave) when only the ones
-  // after it are in flight
-  int issued = 0;                              // tiles set out so far
-  for (; issued < STAGES && issued < nkt; ++issued) issue(issued, issued);
-  dma_wait<LOADS>(issued - 1);
-  __syncthreads();
-  read_frags(0, S0{});
-  int stage = 0;                               // of tile kt
-  // All tiles but the last run the same straight line of code, the last one a copy without the
-  // barrier section.  (With that section under an `if` inside one loop, the compiler joins the
-  // two paths in front of the last eight products and waits there for every LDS read in flight,
-  // the next tile's fragments included, which those products do not use.)
-  for (int kt = 0; kt + 1 < nkt; ++kt) {
-    // first half, from set 0; the second half of the same stage goes into set 1
-    multiply(0, S0{});
-    __builtin_amdgcn_sched_barrier(0);
-    read_frags(stage, S1{});
-    __builtin_amdgcn_sched_barrier(0);
-    multiply(1, S0{});
-    __builtin_amdgcn_sched_barrier(0);
-    // second half, from set 1; in its middle the barrier that makes tile kt + 1 readable and
-    // this tile's stage free
-    multiply(0, S1{});
-    __builtin_amdgcn_sched_barrier(0);
-    dma_wait<LOADS>(issued - kt - 2);          // tile kt + 1 has landed when only the later ones are in flight
-    __syncthreads();
-    // Tile kt + STAGES goes into the stage of tile kt: waves 0..3 set their copies out here, waves
-    // 4..7 (the other wave of each SIMD) behind the tile's last products, a quarter of a k tile
-    // later.  All eight at once measured 2 to 11 % slower (the down product of a prompt most):
-    // the copies' requests reach the L2 in one burst from every CU of the XCD, which walk K in
-    // step, and meet the fragment reads of the new tile in LDS.  (Four groups a quarter apart,
-    // or every wave's copies in two halves, measured worse than two groups: the last ones land late.)
-    const int freed = stage;
-    if (wid < 4 && issued < nkt) { issue(issued, freed); ++issued; }
-    stage = stage + 1 == STAGES ? 0 : stage + 1;
-    read_frags(stage, S0{});
-    __builtin_amdgcn_sched_barrier(0);
-    multiply(1, S1{});
-    __builtin_amdgcn_sched_barrier(0);
-    if (wid >= 4 && issued < nkt) { issue(issued, freed); ++issued; }
-    __builtin_amdgcn_sched_barrier(0);
+  for (int ks = 0; ks < 2; ++ks) {
+    const unsigned pos = ((4 * ks + fk) ^ sw) * 16;
+    pa[ks] = (wave_m * TT::ROWS + fr) * ROW + pos;
+    pw[ks] = W_AT + (TT::first(wave_n) * 16 + fr) * ROW + pos;
   }
-  multiply(0, S0{});
-  __builtin_amdgcn_sched_barrier(0);
-  read_frags(stage, S1{});
-  __builtin_amdgcn_sched_barrier(0);
-  multiply(1, S0{});
-  multiply(0, S1{});
-  multiply(1, S1{});
-  tile_epilogue<TM, TN>(acc, bias, C, ldc, M, N, epi, m0, wm, n0, wn, lane);
+  bf16x8 fa[2][IH][2], fw0[J0][2], fw1[J1][2];               // [half][block][k-step], [block][k-step]
+  auto read_a = [&](int st, auto HALF) {
+    constexpr int h = decltype(HALF)::value;
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int i = 0; i < IH; ++i) fa[h][i][ks] = *reinterpret_cast<const bf16x8*>(smem + pa[ks] + st * A_ST + (h * IH + i) * 16 * ROW);
+  };
+  auto read_w0 = [&](int st) {
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int j = 0; j < J0; ++j) fw0[j][ks] = *reinterpret_cast<const bf16x8*>(smem + pw[ks] + st * W_ST + j * TT::STEP * 16 * ROW);
+  };
+  auto read_w1 = [&](int st) {
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int j = 0; j < J1; ++j) fw1[j][ks] = *reinterpret_cast<const bf16x8*>(smem + pw[ks] + st * W_ST + (J0 + j) * TT::STEP * 16 * ROW);
+  };
+  auto multiply = [&](auto HA, auto HW) {
+    constexpr int ha = decltype(HA)::value, hw = decltype(HW)::value;
+    __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int i = 0; i < IH; ++i)
+#pragma unroll
+        for (int j = 0; j < (hw ? J1 : J0); ++j) {
+          floatx4& d = acc[ha * IH + i][(hw ? J0 : 0) + j];
+          d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hw ? fw1[j < J1 ? j : 0][ks] : fw0[j < J0 ? j : 0][ks], fa[ha][i][ks], d, 0, 0, 0);
+        }
+    __builtin_amdgcn_s_setprio(0);
+  };
+  using H0 = std::integral_constant<int, 0>;
+  using H1 = std::integral_constant<int, 1>;
+  const int nkt = K / DMA_BK;
+#pragma unroll
+  for (int t = 0; t < STAGES; ++t) {                         // (past the last tile: that one again, never read)
+    const int kt = min(t, nkt - 1);
+    copy_w(kt, t, H0{});
+    copy_a(kt, t, H0{});
+    copy_a(kt, t, H1{});
+    copy_w(kt, t, H1{});
+  }
+  dma_wait<STAGES * T - LW0 - LA>();                         // W0 and A0 of tile 0 are here
+  dma_meet();
+  read_w0(0);
+  dma_wait<STAGES * T - LW0 - LA>();
+  dma_meet();
+  if (grp == 1) dma_meet();                                  // the second group runs a slot behind the first
+  auto tile_pass = [&](int kt, int st, int st_next) {
+    const int ahead = min(kt + STAGES, nkt - 1);
+    read_a(st, H0{});
+    __builtin_amdgcn_sched_barrier(0);
+    copy_w(ahead, st, H0{});
+    dma_wait<STAGES * T - 2 * LA>();                         // A1
+    dma_meet();
+    multiply(H0{}, H0{});
+    dma_meet();
+    read_a(st, H1{});
+    __builtin_amdgcn_sched_barrier(0);
+    copy_a(ahead, st, H0{});
+    dma_wait<(STAGES - 1) * T + LW0 + LA>();                 // W1
+    dma_meet();
+    multiply(H1{}, H0{});
+    dma_meet();
+    read_w1(st);
+    __builtin_amdgcn_sched_barrier(0);
+    copy_a(ahead, st, H1{});
+    dma_wait<(STAGES - 1) * T + 2 * LA>();                   // the next tile's W0
+    dma_meet();
+    multiply(H1{}, H1{});
+    dma_meet();
+    read_w0(st_next);
+    __builtin_amdgcn_sched_barrier(0);
+    copy_w(ahead, st, H1{});
+    dma_wait<STAGES * T - LW0 - LA>();                       // the next tile's A0
+    dma_meet();
+    multiply(H0{}, H1{});
+    dma_meet();
+  };
+  if constexpr (STAGES == 2) {
+    int kt = 0;
+    for (; kt + 1 < nkt; kt += 2) {
+      tile_pass(kt, 0, 1);
+      tile_pass(kt + 1, 1, 0);
+    }
+    if (kt < nkt) tile_pass(kt, 0, 1);
+  } else {
+    int st = 0;
+    for (int kt = 0; kt < nkt; ++kt) {
+      const int next = st + 1 == STAGES ? 0 : st + 1;
+      tile_pass(kt, st, next);
+      st = next;
+    }
+  }
+  if (grp == 0) dma_meet();
+  dma_wait<0>();
+  dma_meet();
+  dma_epilogue<TT>(acc, smem + wid * TT::OWN, bias, C, ldc, M, N, epi, m0 + wave_m * TT::ROWS, n0, wave_n, lane);
 }
 
-template <int BN, int WAVES_M, int STAGES>
+template <int BM, int BN, int STAGES, bool GROUPED>
+int configure_tile_dma() {
+  static bool configured = false;
+  if (configured) return 0;
+  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(tile_dma_kernel<BM, BN, STAGES, GROUPED>),
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, DmaTile<BM, BN>::template lds<STAGES>());
+  configured = e == hipSuccess;
+  return (int)e;
+}
+
+template <int BM, int BN, int STAGES>
 int launch_tile_dma(const bf16* A, int lda, const bf16* W, int ldw, const float* bias, void* C, int ldc, int M,
                     int N, int K, int epi, hipStream_t stream, int splits = 1, int k_per_split = 0) {
-  constexpr int smem = STAGES * (DMA_BM + BN) * DMA_BK * 2;
-  static bool configured = false;
-  auto kern = tile_dma_kernel<BN, WAVES_M, STAGES>;
-  if (!configured) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, smem);
-    if (e != hipSuccess) return (int)e;
-    configured = true;
-  }
-  const int tiles_m = (M + DMA_BM - 1) / DMA_BM, tiles_n = (N + BN - 1) / BN;
-  kern<<<dim3(tiles_m * tiles_n, splits), 512, smem, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi, tiles_m,
-                                                               tiles_m * tiles_n >= 16, k_per_split, nullptr);
+  if (const int e = configure_tile_dma<BM, BN, STAGES, false>()) return e;
+  const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
+  tile_dma_kernel<BM, BN, STAGES><<<dim3(tiles_m * tiles_n, splits), 512, DmaTile<BM, BN>::template lds<STAGES>(), stream>>>(
+      A, lda, W, ldw, bias, C, ldc, M, N, K, epi, tiles_m, tiles_m * tiles_n >= 16, k_per_split, nullptr);
   return mf_launch_status();
 }
 
@@ -554,20 +736,13 @@ int launch_tile(const bf16* A, int lda, const bf16* W, int ldw, const float* bia
 }
 
 // The grouped forms: a tile row per entry of `groups` (int32 [n_groups][4] on the device), 32-bit sums stored.
-template <int BN, int WAVES_M, int STAGES>
+template <int BM, int BN, int STAGES>
 int launch_grouped_dma(const bf16* A, int lda, const bf16* W, int ldw, float* C, int ldc, const RowGroup* groups, int n_groups,
                        int N, int K, hipStream_t stream) {
-  constexpr int smem = STAGES * (DMA_BM + BN) * DMA_BK * 2;
-  static bool configured = false;
-  auto kern = tile_dma_kernel<BN, WAVES_M, STAGES, true>;
-  if (!configured) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, smem);
-    if (e != hipSuccess) return (int)e;
-    configured = true;
-  }
+  if (const int e = configure_tile_dma<BM, BN, STAGES, true>()) return e;
   const int tiles_n = (N + BN - 1) / BN;
-  kern<<<dim3(n_groups * tiles_n), 512, smem, stream>>>(A, lda, W, ldw, nullptr, C, ldc, 0, N, K, EPI_F32, n_groups,
-                                                        n_groups * tiles_n >= 16, 0, groups);
+  tile_dma_kernel<BM, BN, STAGES, true><<<dim3(n_groups * tiles_n), 512, DmaTile<BM, BN>::template lds<STAGES>(), stream>>>(
+      A, lda, W, ldw, nullptr, C, ldc, 0, N, K, EPI_F32, n_groups, n_groups * tiles_n >= 16, 0, groups);
   return mf_launch_status();
 }
 
@@ -1956,20 +2131,61 @@ int launch_panel(const bf16* A, int lda, const bf16* W, const bf16* Wt, int ldw,
 
 // ---- which tile kernel a product of many rows takes
 // Variants: 2: 128 x 128 tiles through registers (two blocks a CU), 3: 64 x 64, 9: 256 x 256 through
-// registers, and the direct-to-LDS kernel (aligned operands, K in 64s) with tiles of 256 x 256
-// (12), 256 x 192 (15, no SwiGLU) and 256 x 128 in three stages (13).  With `splits` > 1 the K
-// dimension is cut over blocks (variants 12 and 2) and skinny_reduce_kernel adds the parts.
+// registers, and the direct-to-LDS kernel (aligned operands, K in 64s): 12 the largest tiles (256 x 256; SwiGLU products
+// 256 x 192 where their rounds are the shorter), 15 256 x 192 (no SwiGLU), 13 the smaller ones (256 x 128, 128 x 256 or
+// 128 x 128).  With `splits` > 1 the K dimension is cut over blocks (variants 12 and 2, the latter with the smaller
+// direct-to-LDS tiles where the operands allow) and skinny_reduce_kernel adds the parts.
 struct TilePlan { int variant, splits, k_per_split; double us; };
 
+// The direct-to-LDS kernel's tiles: microseconds a k tile of 64 with every CU busy (random values, 2,048 rows at the 7B
+// widths; a chip that is not full runs up to 0.7 of it) and how many of them a round adds for its start and end.
+struct DmaForm { int bm, bn; double step_us; };
+enum { FORM_256, FORM_192, FORM_128, FORM_128T, FORM_SMALL, N_FORMS };
+constexpr DmaForm DMA_FORMS[N_FORMS] = {{256, 256, 1.36}, {256, 192, 1.08}, {256, 128, 0.84}, {128, 256, 0.84}, {128, 128, 0.58}};
+constexpr double ROUND_US = 5.;
+
 // The estimate behind the choice: a kernel's tiles go over its slots (blocks that fit the chip at
-// once) in rounds; a round takes the product's k tiles of 64 times the variant's time per k tile
-// (measured at the 7B widths with every CU busy), a last round that is not full somewhat less
-// (fewer blocks pull on the fabric); a start, the epilogue's traffic, and for a K split the
-// parts' way to memory and back come on top.
-double rounds_us(long blocks, long slots, double step_us, long nkt) {
+// once) in rounds; a round takes the product's k tiles of 64 times the variant's time per k tile, a last round that is
+// not full somewhat less (fewer blocks pull on the fabric and on the power); a start, the epilogue's traffic, and for a K
+// split the parts' way to memory and back come on top.
+double rounds_us(long blocks, long slots, double step_us, long nkt, double round_us) {
   const long full = blocks / slots;
   const double fill = (double)(blocks % slots) / (double)slots;
-  return (double)nkt * step_us * ((double)full + (fill > 0. ? 0.7 + 0.3 * fill : 0.));
+  return ((double)nkt * step_us) * ((double)full + (fill > 0. ? 0.7 + 0.3 * fill : 0.)) + round_us * (double)(full + (fill > 0.));
+}
+
+double form_us(int form, int M, int N, long nkt, int splits, long cu) {
+  const DmaForm& f = DMA_FORMS[form];
+  const long tiles = (long)((M + f.bm - 1) / f.bm) * ((N + f.bn - 1) / f.bn);
+  return rounds_us(tiles * splits, cu, f.step_us, nkt, ROUND_US);
+}
+
+// the cheapest of the forms first .. last
+int best_form(int first, int last, int M, int N, long nkt, int splits, long cu) {
+  int best = first;
+  for (int f = first + 1; f <= last; ++f)
+    if (form_us(f, M, N, nkt, splits, cu) < form_us(best, M, N, nkt, splits, cu)) best = f;
+  return best;
+}
+
+// which tiles variant 12, 13 or 15, or variant 2 cut over K, runs
+int dma_form(int variant, int M, int N, int epi, long nkt, int splits, long cu) {
+  switch (variant) {
+    case 12: return epi == EPI_SWIGLU && splits == 1 ? best_form(FORM_256, FORM_192, M, N, nkt, 1, cu) : FORM_256;
+    case 15: return FORM_192;
+  }
+  return best_form(FORM_128, FORM_SMALL, M, N, nkt, splits, cu);
+}
+
+int launch_form(int form, const bf16* A, int lda, const bf16* W, int ldw, const float* bias, void* C, int ldc, int M, int N, int K,
+                int epi, hipStream_t stream, int splits = 1, int k_per_split = 0) {
+  switch (form) {
+    case FORM_256: return launch_tile_dma<256, 256, 2>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi, stream, splits, k_per_split);
+    case FORM_192: return launch_tile_dma<256, 192, 2>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi, stream, splits, k_per_split);
+    case FORM_128: return launch_tile_dma<256, 128, 3>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi, stream, splits, k_per_split);
+    case FORM_128T: return launch_tile_dma<128, 256, 3>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi, stream, splits, k_per_split);
+  }
+  return launch_tile_dma<128, 128, 4>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi, stream, splits, k_per_split);
 }
 
 TilePlan plan_tiles(int M, int N, int K, bool dma_ok, int epi, int n_cu) {
@@ -1977,7 +2193,7 @@ TilePlan plan_tiles(int M, int N, int K, bool dma_ok, int epi, int n_cu) {
   const long nkt = (K + 63) / 64, chunks = (K + 255) / 256;
   const double mn = (double)M * (double)N;
   const double epi_us = (epi == EPI_ACC_F32 ? 8. : epi == EPI_F32 ? 4. : (epi == EPI_BF16 || epi == EPI_XIELU) ? 2. : 1.) * mn / 4e6;
-  const double start_us = 12.;
+  const double start_us = dma_ok ? 4. : 12.;
   auto tiles = [&](int bm, int bn) { return (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
   auto cut = [&](long parts, int& splits, int& per) {          // K in `parts` runs of whole chunks of 256
     const long c = (chunks + parts - 1) / parts;
@@ -1989,12 +2205,13 @@ TilePlan plan_tiles(int M, int N, int K, bool dma_ok, int epi, int n_cu) {
   auto offer = [&](int variant, int splits, int per, double us) {
     if (us < best.us) best = TilePlan{variant, splits, per, us};
   };
+  auto form = [&](int variant, int splits, long steps) {
+    return form_us(dma_form(variant, M, N, epi, steps, splits, cu), M, N, steps, splits, cu);
+  };
   if (dma_ok) {
-    offer(12, 1, K, rounds_us(tiles(256, 256), cu, 1.75, nkt) + start_us + epi_us);
-    // (the narrower tiles must promise 4 % to be taken: where the estimates are that close, the
-    // 256-wide tile has measured the faster)
-    offer(13, 1, K, 1.04 * (rounds_us(tiles(256, 128), cu, 1.00, nkt) + start_us + epi_us));
-    if (epi != EPI_SWIGLU) offer(15, 1, K, 1.04 * (rounds_us(tiles(256, 192), cu, 1.35, nkt) + start_us + epi_us));
+    offer(12, 1, K, form(12, 1, nkt) + start_us + epi_us);
+    offer(13, 1, K, form(13, 1, nkt) + start_us + epi_us);
+    if (epi != EPI_SWIGLU) offer(15, 1, K, form(15, 1, nkt) + start_us + epi_us);
     // many rows against few weight rows and a long K (the down product of a prompt): K cut over
     // the big tiles, each part at least 2,048 of K
     if (epi != EPI_SWIGLU && M >= 768)
@@ -2002,22 +2219,24 @@ TilePlan plan_tiles(int M, int N, int K, bool dma_ok, int epi, int n_cu) {
         int splits, per;
         cut(parts, splits, per);
         if (splits < 2) continue;
-        offer(12, splits, per, rounds_us(tiles(256, 256) * splits, cu, 1.75, per / 64) + start_us + parts_us(splits));
+        offer(12, splits, per, form(12, splits, per / 64) + start_us + parts_us(splits));
       }
   } else {
-    offer(9, 1, K, rounds_us(tiles(256, 256), cu, 2.1, nkt) + start_us + epi_us);
+    offer(9, 1, K, rounds_us(tiles(256, 256), cu, 2.1, nkt, 0.) + start_us + epi_us);
+    offer(M <= 64 && tiles(128, 128) < 64 && epi != EPI_SWIGLU ? 3 : 2, 1, K,
+          rounds_us(tiles(128, 128), 2 * cu, 1.45, nkt, 0.) + start_us + epi_us);
   }
-  const long t128 = tiles(128, 128);
-  offer(M <= 64 && t128 < 64 && epi != EPI_SWIGLU ? 3 : 2, 1, K,
-        rounds_us(t128, 2 * cu, 1.45, nkt) + start_us + epi_us);
   // a few hundred rows against a few thousand weight rows (some 50 tiles of 128 x 128, bound by
-  // the weight stream): K over about two blocks per CU, each with at least 512 of K
-  const long parts = std::min(chunks / 2, (2 * cu) / std::max(1L, t128));
-  if (t128 < cu && parts >= 2) {
-    int splits, per;
-    cut(parts, splits, per);
-    if (splits >= 2) offer(2, splits, per, rounds_us(t128 * splits, 2 * cu, 1.45, per / 64) + start_us + parts_us(splits));
-  }
+  // the weight stream): K over the chip, each part at least 512 of K
+  const long t128 = tiles(128, 128);
+  if (t128 < cu)
+    for (long parts = 2; parts <= std::min(chunks / 2, (2 * cu) / std::max(1L, t128)); ++parts) {
+      int splits, per;
+      cut(parts, splits, per);
+      if (splits < 2 || splits * t128 > 2 * cu) continue;
+      const double us = dma_ok ? form(2, splits, per / 64) : rounds_us(t128 * splits, 2 * cu, 1.45, per / 64, 0.);
+      offer(2, splits, per, us + start_us + parts_us(splits));
+    }
   return best;
 }
 
@@ -2061,9 +2280,11 @@ MF_API int mf_gemm_bf16_grouped(const void* A, const void* W, float* C, const in
   const bf16* w = (const bf16*)W;
   const RowGroup* g = (const RowGroup*)groups;
   switch (variant) {
-    case 2: return launch_grouped_tile<128, 128, 64, 64, 64>(a, K, w, K, C, N, g, n_groups, N, K, stream);
-    case 12: return launch_grouped_dma<256, 2, 2>(a, K, w, K, C, N, g, n_groups, N, K, stream);
-    case 13: return launch_grouped_dma<128, 4, 3>(a, K, w, K, C, N, g, n_groups, N, K, stream);
+    case 2:
+      return K % DMA_BK == 0 ? launch_grouped_dma<128, 128, 4>(a, K, w, K, C, N, g, n_groups, N, K, stream)
+                             : launch_grouped_tile<128, 128, 64, 64, 64>(a, K, w, K, C, N, g, n_groups, N, K, stream);
+    case 12: return launch_grouped_dma<256, 256, 2>(a, K, w, K, C, N, g, n_groups, N, K, stream);
+    case 13: return launch_grouped_dma<256, 128, 3>(a, K, w, K, C, N, g, n_groups, N, K, stream);
   }
   return (int)hipErrorInvalidValue;
 }
@@ -2095,15 +2316,9 @@ MF_API int mf_gemm_bf16(const void* A, int lda, const void* W, int ldw, const fl
     case 3: return launch_tile<64, 64, 32, 32>(a, lda, w, ldw, bias, C, ldc, M, N, K, epi, vec_ok, stream);
     case 6: return launch_tile<256, 128, 64, 64, 32>(a, lda, w, ldw, bias, C, ldc, M, N, K, epi, vec_ok, stream);
     case 9: return launch_tile<256, 256, 128, 64, 64>(a, lda, w, ldw, bias, C, ldc, M, N, K, epi, vec_ok, stream);
-    case 12:
-      if (!dma_ok) return (int)hipErrorInvalidValue;
-      return launch_tile_dma<256, 2, 2>(a, lda, w, ldw, bias, C, ldc, M, N, K, epi, stream);
-    case 13:
-      if (!dma_ok) return (int)hipErrorInvalidValue;
-      return launch_tile_dma<128, 4, 3>(a, lda, w, ldw, bias, C, ldc, M, N, K, epi, stream);
-    case 15:
-      if (!dma_ok || epi == EPI_SWIGLU) return (int)hipErrorInvalidValue;
-      return launch_tile_dma<192, 4, 2>(a, lda, w, ldw, bias, C, ldc, M, N, K, epi, stream);
+    case 12: case 13: case 15:
+      if (!dma_ok || (variant == 15 && epi == EPI_SWIGLU)) return (int)hipErrorInvalidValue;
+      return launch_form(dma_form(variant, M, N, epi, K / DMA_BK, 1, cu_count()), a, lda, w, ldw, bias, C, ldc, M, N, K, epi, stream);
   }
   return (int)hipErrorInvalidValue;
 }
@@ -2124,16 +2339,14 @@ MF_API int mf_gemm_bf16_splitk(const void* A, int lda, const void* W, int ldw, c
   const int vec_ok = (lda % 8 == 0) && (ldw % 8 == 0) && ((uintptr_t)A % 16 == 0) &&
                      ((uintptr_t)W % 16 == 0) && (K % 8 == 0);
   // variant 12: 256 x 256 tiles through the direct-to-LDS pipeline (many rows against few weight
-  // rows and a long K: the down product of a prompt); 2: 128 x 128 (few rows)
+  // rows and a long K: the down product of a prompt); 2: the smaller tiles (few rows)
   if (variant != 12 && variant != 2) return (int)hipErrorInvalidValue;
-  const bool big_tiles = variant == 12;
-  if (big_tiles && (!vec_ok || K % DMA_BK != 0 || (size_t)M * lda * 2 >= (1ull << 32) ||
-                    (size_t)N * ldw * 2 >= (1ull << 32)))
-    return (int)hipErrorInvalidValue;
-  int rc = big_tiles ? launch_tile_dma<256, 2, 2>((const bf16*)A, lda, (const bf16*)W, ldw, nullptr, part, N, M, N, K,
-                                       EPI_F32, stream, splits, k_per_split)
-                     : launch_tile<128, 128, 64, 64>((const bf16*)A, lda, (const bf16*)W, ldw, nullptr, part, N, M,
-                                                     N, K, EPI_F32, vec_ok, stream, splits, k_per_split);
+  const bool dma_ok = vec_ok && K % DMA_BK == 0 && (size_t)M * lda * 2 < (1ull << 32) && (size_t)N * ldw * 2 < (1ull << 32);
+  if (variant == 12 && !dma_ok) return (int)hipErrorInvalidValue;
+  int rc = dma_ok ? launch_form(dma_form(variant, M, N, EPI_F32, k_per_split / DMA_BK, splits, cu_count()), (const bf16*)A, lda,
+                                (const bf16*)W, ldw, nullptr, part, N, M, N, K, EPI_F32, stream, splits, k_per_split)
+                  : launch_tile<128, 128, 64, 64>((const bf16*)A, lda, (const bf16*)W, ldw, nullptr, part, N, M,
+                                                  N, K, EPI_F32, vec_ok, stream, splits, k_per_split);
   if (rc) return rc;
   return launch_reduce(part, bias, C, ldc, M, N, K, splits, epi, FusedNorm{}, stream);
 }
