@@ -2,10 +2,18 @@
 // out[t][o] = dot(W[o][:], x[t][:]) + b[o], as src/graph/cpu_backend.rs:214-248 of
 // yusiwen/minfer.  Plain fp32 FMA, no reduced-precision matrix mode: this is the path
 // that shows faults bfloat16 hides.  Any M, N, K; vector loads only where they are aligned.
+//
+// Three kernels:
+//  * `rows_f32_kernel`: at most 8 rows, K in 4s: the weight stream, a wave a few weight rows.
+//  * `tile_f32_kernel`: aligned operands and K in 32s: 64 x 64 tiles on the 32-bit matrix instruction (an FMA a product,
+//    twice the vector units' rate), K split over blocks where the tiles leave CUs idle.
+//  * `gemm_f32_kernel`: everything else, from LDS with vector FMA.
 // A dot product is summed in blocks of 128 terms whose sums are then added up: the rounding
 // error of one long chain grows with the root of its length (18944 terms in the down product;
 // the reference's scalar path sums in 64 bits, src/vec_ops.rs:31-35), that of blocks with the
 // roots of the block's and of the number of blocks.
+#include <algorithm>
+
 #include "common.h"
 
 namespace {
@@ -94,14 +102,261 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__
   }
 }
 
+// ---- many rows on the matrix cores
+// A 64 x 64 tile on 4 waves of 32 x 32 (16x16x4 products).  k tiles of 32 (a row is a 128-byte line) travel global -> LDS
+// in three stages, chunk c of row r at position c ^ ((r >> 1) & 7); a lane reads four neighbouring k of its row at once
+// and the e-th of them goes into the e-th product, so a product's four k are 4 apart (the order of a sum's terms within
+// sixteen).  The products are what bounds it (1,024 cycles a k tile for 256 of LDS reads); 48 KB of LDS let three
+// blocks share a CU, whose waves cover each other's waits.
+// 611 rows (0.5B widths), with vector FMA before and now: gate|up 9,728 x 896 152 us and 98 (113 TFLOP/s); q|k|v 1,152 x 896
+// 74 and 24 (a third of K a block, and the kernel that adds the parts); down 896 x 4,864 and o 896 x 896 together 450 and 85.
+constexpr int T_BM = 64, T_BK = 32, T_STAGES = 3, T_ROW = T_BK * 4, T_STAGE = 2 * T_BM * T_ROW;
+
+__device__ __forceinline__ void dma16(const float* base, unsigned off, unsigned lds_byte) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds_byte)
+               : "memory", "m0");
+}
+
+// SPLIT: sums without bias into this part's slab of C, [parts][M][N]; else the product's own epilogue
+template <bool ACCUMULATE, bool SPLIT>
+__global__ __launch_bounds__(256) void tile_f32_kernel(const float* __restrict__ A, int lda, const float* __restrict__ W, int ldw,
+                                                       const float* __restrict__ bias, float* __restrict__ C, int ldc, int M, int N,
+                                                       int K, int tiles_m, int k_per_split) {
+  __shared__ __attribute__((aligned(16))) unsigned char smem[T_STAGES * T_STAGE];
+  if (SPLIT) {
+    const int kb = blockIdx.y * k_per_split;
+    A += kb;
+    W += kb;
+    K = min(k_per_split, K - kb);
+    C += (size_t)blockIdx.y * M * N;
+  }
+  const int m0 = (blockIdx.x % tiles_m) * T_BM, n0 = (blockIdx.x / tiles_m) * T_BM;
+  const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = (wid & 1) * 32, wn = (wid >> 1) * 32;
+  const int fr = lane & 15, fk = lane >> 4;
+  const unsigned lds0 = (unsigned)(uintptr_t)smem;
+  // a wave copies pieces of 8 rows: 2 of A's 8 and 2 of W's 8
+  unsigned ga[2], gw[2];
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const int r = (q * 4 + wid) * 8 + (lane >> 3), c = ((lane & 7) ^ ((r >> 1) & 7)) * 4;
+    ga[q] = ((unsigned)min(m0 + r, M - 1) * (unsigned)lda + c) * 4u;
+    gw[q] = ((unsigned)min(n0 + r, N - 1) * (unsigned)ldw + c) * 4u;
+  }
+  const int nkt = K / T_BK;
+  auto copy = [&](int kt, int st) {               // (past the last tile: that one again, never read)
+    const int k = min(kt, nkt - 1) * T_BK;
+    const unsigned base = lds0 + st * T_STAGE + wid * 1024;
+#pragma unroll
+    for (int q = 0; q < 2; ++q) dma16(A + k, ga[q], __builtin_amdgcn_readfirstlane(base + q * 4096));
+#pragma unroll
+    for (int q = 0; q < 2; ++q) dma16(W + k, gw[q], __builtin_amdgcn_readfirstlane(base + T_BM * T_ROW + q * 4096));
+  };
+  floatx4 acc[2][2], tot[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[i][j] = tot[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+  copy(0, 0);
+  copy(1, 1);
+  const int sw = (fr >> 1) & 7;
+  int st = 0;
+  for (int kt = 0; kt < nkt; ++kt) {
+    // tile kt has landed for this wave (tile kt + 1's four copies may be in flight), and behind the barrier for all; the
+    // stage of tile kt - 1, which every wave holds in registers by then, takes tile kt + 2
+    asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+    __syncthreads();
+    copy(kt + 2, st == 0 ? 2 : st - 1);
+    const unsigned char* s = smem + st * T_STAGE;
+    float4 a[2][2], w[2][2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int pos = ((4 * h + fk) ^ sw) * 16;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        a[h][i] = *reinterpret_cast<const float4*>(s + (wm + i * 16 + fr) * T_ROW + pos);
+        w[h][i] = *reinterpret_cast<const float4*>(s + T_BM * T_ROW + (wn + i * 16 + fr) * T_ROW + pos);
+      }
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int j = 0; j < 2; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32((&w[h][j].x)[e], (&a[h][i].x)[e], acc[i][j], 0, 0, 0);
+    if ((kt & 3) == 3) {                          // 128 terms
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          tot[i][j] += acc[i][j];
+          acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+        }
+    }
+    st = st == T_STAGES - 1 ? 0 : st + 1;
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  // D: the lane's row is lane % 16, its columns 4 (lane / 16) + e
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int m = m0 + wm + i * 16 + fr;
+    if (m >= M) continue;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int n = n0 + wn + j * 16 + fk * 4;
+      const floatx4 v = acc[i][j] + tot[i][j];
+      float* c = C + (size_t)m * ldc + n;
+      if (SPLIT && n + 4 <= N && ldc % 4 == 0 && (uintptr_t)C % 16 == 0) {
+        *reinterpret_cast<floatx4*>(c) = v;
+        continue;
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (n + e < N) {
+          const float x = SPLIT || !bias ? v[e] : v[e] + bias[n + e];
+          c[e] = ACCUMULATE ? c[e] + x : x;
+        }
+    }
+  }
+}
+
+// adds the parts of a K split in their order, then the bias, then (ACCUMULATE) what C held
+template <bool ACCUMULATE>
+__global__ __launch_bounds__(256) void add_parts_f32_kernel(const float* __restrict__ part, const float* __restrict__ bias,
+                                                            float* __restrict__ C, int ldc, int M, int N, int splits) {
+  const size_t x = (size_t)blockIdx.x * 256 + threadIdx.x, mn = (size_t)M * N;
+  if (x >= mn) return;
+  const int m = x / N, n = x % N;
+  float v = 0.f;
+  for (int s0 = 0; s0 < splits; s0 += 8) {        // eight parts' loads in flight together
+    float p[8];
+#pragma unroll
+    for (int s = 0; s < 8; ++s) p[s] = s0 + s < splits ? part[(size_t)(s0 + s) * mn + x] : 0.f;
+#pragma unroll
+    for (int s = 0; s < 8; ++s) v += p[s];
+  }
+  if (bias) v += bias[n];
+  float* c = C + (size_t)m * ldc + n;
+  *c = ACCUMULATE ? *c + v : v;
+}
+
+// How many blocks share a tile's K: the chip holds three blocks a CU and is busy with one, so K is cut, in parts of at
+// least 256, until every CU has about two (140 tiles of 64 x 64 for 611 rows against 896: whole, a CU in two would idle).
+int tile_splits(int M, int N, int K, int n_cu) {
+  const long tiles = (long)((M + T_BM - 1) / T_BM) * ((N + T_BM - 1) / T_BM);
+  if (tiles >= n_cu) return 1;
+  const long parts = std::min<long>(std::min<long>(K / 256, 16), (2L * n_cu + tiles - 1) / tiles);
+  if (parts < 2) return 1;
+  const int per = (int)((K / T_BK + parts - 1) / parts) * T_BK;
+  return (K + per - 1) / per;
+}
+
+bool tile_takes(int M, int N, int K, int lda, int ldw, const void* A, const void* W) {
+  return K % T_BK == 0 && lda % 4 == 0 && ldw % 4 == 0 && (uintptr_t)A % 16 == 0 && (uintptr_t)W % 16 == 0 &&
+         (size_t)M * lda * 4 < (1ull << 32) && (size_t)N * ldw * 4 < (1ull << 32);
+}
+
+// ---- few rows: the weight stream
+// A wave takes NR weight rows (four where the matrix is tall enough to keep every SIMD busy all the same: the activations
+// are then read once for four rows) and walks K in runs of 256, a float4 a lane; its sums meet by shuffles.
+// The head of the 0.5B widths (151,936 x 896, one row): 204 us before, 92 now, 5.9 TB/s.
+template <int MR, int NR, bool ACCUMULATE>
+__global__ __launch_bounds__(256) void rows_f32_kernel(const float* __restrict__ A, int lda, const float* __restrict__ W, int ldw,
+                                                       const float* __restrict__ bias, float* __restrict__ C, int ldc, int M, int N,
+                                                       int K) {
+  const int lane = threadIdx.x & 63;
+  const int n0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * NR;
+  if (n0 >= N) return;
+  const float* w[NR];
+#pragma unroll
+  for (int j = 0; j < NR; ++j) w[j] = W + (size_t)min(n0 + j, N - 1) * ldw;
+  float acc[MR][NR] = {};
+#pragma unroll 2
+  for (int k = lane * 4; k < K; k += 256) {
+    float4 x[NR];
+#pragma unroll
+    for (int j = 0; j < NR; ++j) x[j] = *reinterpret_cast<const float4*>(w[j] + k);
+#pragma unroll
+    for (int i = 0; i < MR; ++i) {
+      const float4 a = *reinterpret_cast<const float4*>(A + (size_t)min(i, M - 1) * lda + k);
+#pragma unroll
+      for (int j = 0; j < NR; ++j)
+        acc[i][j] = fmaf(a.w, x[j].w, fmaf(a.z, x[j].z, fmaf(a.y, x[j].y, fmaf(a.x, x[j].x, acc[i][j]))));
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < MR; ++i)
+#pragma unroll
+    for (int j = 0; j < NR; ++j) acc[i][j] = wave_sum(acc[i][j]);
+  // lane i NR + j stores sum (i, j)
+#pragma unroll
+  for (int i = 0; i < MR; ++i)
+#pragma unroll
+    for (int j = 0; j < NR; ++j)
+      if (lane == i * NR + j && i < M && n0 + j < N) {
+        const float v = bias ? acc[i][j] + bias[n0 + j] : acc[i][j];
+        float* c = C + (size_t)i * ldc + n0 + j;
+        *c = ACCUMULATE ? *c + v : v;
+      }
+}
+
+template <int MR, int NR>
+int launch_rows(const float* A, int lda, const float* W, int ldw, const float* bias, float* C, int ldc, int M, int N, int K,
+                int accumulate, hipStream_t stream) {
+  const int grid = (N + 4 * NR - 1) / (4 * NR);
+  if (accumulate) rows_f32_kernel<MR, NR, true><<<grid, 256, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K);
+  else rows_f32_kernel<MR, NR, false><<<grid, 256, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K);
+  return mf_launch_status();
+}
+
+template <int MR>
+int launch_rows_n(const float* A, int lda, const float* W, int ldw, const float* bias, float* C, int ldc, int M, int N, int K,
+                  int accumulate, hipStream_t stream) {
+  return N >= 16384 ? launch_rows<MR, 4>(A, lda, W, ldw, bias, C, ldc, M, N, K, accumulate, stream)
+                    : launch_rows<MR, 1>(A, lda, W, ldw, bias, C, ldc, M, N, K, accumulate, stream);
+}
+
 }  // namespace
 
-MF_API int mf_gemm_f32(const float* A, int lda, const float* W, int ldw, const float* bias, float* C,
-                       int ldc, int M, int N, int K, int accumulate, hipStream_t stream) {
+// How many parts K is cut into (1: none): `mf_gemm_f32` with more than one needs part [parts][M][N].
+// `aligned`: 16-byte aligned operands with row strides in multiples of 4.
+MF_API int mf_gemm_f32_splits(int M, int N, int K, int aligned, int n_cu) {
+  if (M <= 8 || N <= 0 || !aligned || K % T_BK || (size_t)M * K * 4 >= (1ull << 32) || (size_t)N * K * 4 >= (1ull << 32)) return 1;
+  return tile_splits(M, N, K, n_cu);
+}
+
+MF_API int mf_gemm_f32(const float* A, int lda, const float* W, int ldw, const float* bias, float* C, int ldc, float* part,
+                       int M, int N, int K, int splits, int accumulate, hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
   if (K <= 0 || lda < K || ldw < K || ldc < N) return (int)hipErrorInvalidValue;
   const int vec_ok = (lda % 4 == 0) && (ldw % 4 == 0) && ((uintptr_t)A % 16 == 0) &&
                      ((uintptr_t)W % 16 == 0);
+  if (M <= 8 && vec_ok && K % 4 == 0) {
+    if (M == 1) return launch_rows_n<1>(A, lda, W, ldw, bias, C, ldc, M, N, K, accumulate, stream);
+    if (M == 2) return launch_rows_n<2>(A, lda, W, ldw, bias, C, ldc, M, N, K, accumulate, stream);
+    if (M <= 4) return launch_rows_n<4>(A, lda, W, ldw, bias, C, ldc, M, N, K, accumulate, stream);
+    return launch_rows_n<8>(A, lda, W, ldw, bias, C, ldc, M, N, K, accumulate, stream);
+  }
+  if (tile_takes(M, N, K, lda, ldw, A, W)) {
+    const int tiles_m = (M + T_BM - 1) / T_BM, tiles = tiles_m * ((N + T_BM - 1) / T_BM);
+    if (splits > 1) {
+      const int per = (K / T_BK + splits - 1) / splits * T_BK;
+      if (!part || (long)(splits - 1) * per >= K) return (int)hipErrorInvalidValue;
+      tile_f32_kernel<false, true><<<dim3(tiles, splits), 256, 0, stream>>>(A, lda, W, ldw, nullptr, part, N, M, N, K, tiles_m, per);
+      const int rc = mf_launch_status();
+      if (rc) return rc;
+      const unsigned blocks = (unsigned)(((size_t)M * N + 255) / 256);
+      if (accumulate) add_parts_f32_kernel<true><<<blocks, 256, 0, stream>>>(part, bias, C, ldc, M, N, splits);
+      else add_parts_f32_kernel<false><<<blocks, 256, 0, stream>>>(part, bias, C, ldc, M, N, splits);
+      return mf_launch_status();
+    }
+    if (accumulate) tile_f32_kernel<true, false><<<tiles, 256, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, tiles_m, 0);
+    else tile_f32_kernel<false, false><<<tiles, 256, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, tiles_m, 0);
+    return mf_launch_status();
+  }
   dim3 grid((N + BN - 1) / BN, (M + BM - 1) / BM);
   if (accumulate)
     gemm_f32_kernel<true><<<grid, 256, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, vec_ok);

@@ -129,7 +129,8 @@ _PROTOTYPES = {
         "mf_fill_normal_host": [_P, c_int, c_size_t, c_uint64, c_float, c_int, c_int],
     },
     "gemm_f32": {
-        "mf_gemm_f32": [_P, c_int, _P, c_int, _P, _P, c_int, c_int, c_int, c_int, c_int, _P],
+        "mf_gemm_f32": [_P, c_int, _P, c_int, _P, _P, c_int, _P, c_int, c_int, c_int, c_int, c_int, _P],
+        "mf_gemm_f32_splits": [c_int, c_int, c_int, c_int, c_int],
     },
     "gemm_bf16": {
         "mf_gemm_bf16": [_P, c_int, _P, c_int, _P, _P, c_int, c_int, c_int, c_int, c_int, c_int, _P],
@@ -1768,8 +1769,11 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], 
         return
     if x.dtype == torch.float32:
         _need(out, "linear.out", torch.float32)
-        _check(_fn("gemm_f32", "mf_gemm_f32")(_ptr(x), k, _ptr(weight), k, _ptr(bias), _ptr(out), n, m,
-                                               n, k, 1 if accumulate else 0, _stream()), f"gemm_f32 {m}x{n}x{k}")
+        aligned = not (x.data_ptr() % 16 or weight.data_ptr() % 16 or k % 4)
+        splits = _fn("gemm_f32", "mf_gemm_f32_splits")(m, n, k, 1 if aligned else 0, cu_count())
+        part = torch.empty(splits * m * n, dtype=torch.float32, device=x.device) if splits > 1 else None
+        _check(_fn("gemm_f32", "mf_gemm_f32")(_ptr(x), k, _ptr(weight), k, _ptr(bias), _ptr(out), n, _ptr(part), m,
+                                               n, k, splits, 1 if accumulate else 0, _stream()), f"gemm_f32 {m}x{n}x{k}")
         return
     if accumulate and out.dtype != torch.float32:
         raise KernelError("linear: accumulation needs a float32 output")

@@ -222,6 +222,16 @@ def test_gemm_f32(ops, m, n, k):
     close(acc, ref - b.double() + base.double(), 1e-5 * math.sqrt(k) / 8, 1e-5)
 
 
+# the 32-bit product's kernels: few rows (one to eight, one or four weight rows a wave), the matrix cores (one k tile and
+# more than its stages, rows and columns that leave remainders, K cut into parts that are not all equal), row lengths that go
+# to the general kernel
+@pytest.mark.parametrize("m,n,k", [(1, 16387, 896), (2, 33, 36), (3, 16385, 260), (4, 896, 4864), (7, 130, 128), (8, 20001, 64),
+                                   (9, 65, 32), (64, 64, 64), (65, 127, 96), (611, 896, 896), (100, 130, 4864), (33, 1001, 2080),
+                                   (1000, 1537, 160), (12, 100, 48), (5, 50, 35)])
+def test_gemm_f32_kernels(ops, m, n, k):
+    test_gemm_f32(ops, m, n, k)
+
+
 @pytest.mark.parametrize("variant", [0, 1, 2, 3, 6, 9, 12, 13, 15])
 @pytest.mark.parametrize("m,n,k", GEMM_SHAPES + [(2048, 512, 256), (1, 152064, 64), (64, 3584, 3584),
                                                  # at most 16 rows with K of 1536..4096: activations in registers
