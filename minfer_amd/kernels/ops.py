@@ -6,6 +6,7 @@ cached workspaces below.
 from __future__ import annotations
 
 import ctypes
+import functools
 import sys
 from ctypes import c_char_p, c_double, c_float, c_int, c_int64, c_size_t, c_uint64, c_void_p
 from typing import Dict, Optional, Tuple
@@ -189,8 +190,10 @@ def _fn(lib: str, name: str, variant: Optional[str] = None):
     return f
 
 
-def _stream() -> c_void_p:
-    return c_void_p(torch.cuda.current_stream().cuda_stream)
+def _stream() -> int:
+    """The current stream of the current device, as the launches take it.  (By way of `torch.cuda.current_stream()` it costs
+    three microseconds a launch, a tenth of what a layer of a short prompt takes on the host.)"""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _check(rc: int, what: str) -> None:
@@ -212,8 +215,8 @@ def _check(rc: int, what: str) -> None:
         print(f"[minfer_amd] {what} OK", file=sys.stderr, flush=True)
 
 
-def _ptr(t: Optional[torch.Tensor]) -> c_void_p:
-    return c_void_p(0 if t is None else t.data_ptr())
+def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
+    return None if t is None else t.data_ptr()
 
 
 # ------------------------------------------------------------------ per-launch timing
@@ -241,6 +244,10 @@ def stop_trace():
 
 
 def _need(t: torch.Tensor, name: str, dtype=None, shape=None) -> None:
+    # (a launch checks some seven tensors: what is right is found so in one expression, what is not is named below)
+    if isinstance(t, torch.Tensor) and t.is_cuda and t.is_contiguous() and \
+            (dtype is None or t.dtype is dtype or dtype is _FLOATS and t.dtype in _FLOATS) and (shape is None or t.shape == shape):
+        return
     if not isinstance(t, torch.Tensor) or not t.is_cuda:
         raise KernelError(f"{name}: must be a tensor on the GPU (there is no CPU path)")
     if not t.is_contiguous():
@@ -1665,8 +1672,11 @@ def skinny_plan(m: int, n: int, k: int, target_blocks: Optional[int] = None,
     against 30.4) and where a CU's share of the weight rows fills its 16-row tiles poorly, unless
     the matrix is small (the down product of the 3B shape, 2048 x 11008, at 8 rows: 13.5 us in one
     kernel, half-filled tiles and all, against 15.0 in two; at 16 rows 17.1 against 15.4)."""
-    if target_blocks is None:
-        target_blocks = tuning.SKINNY_TARGET or cu_count()
+    return _skinny_plan(m, n, k, tuning.SKINNY_TARGET or cu_count() if target_blocks is None else target_blocks, swiglu, tiled)
+
+
+@functools.lru_cache(maxsize=4096)
+def _skinny_plan(m: int, n: int, k: int, target_blocks: int, swiglu: bool, tiled: bool) -> Tuple[int, int]:
     if m <= 16:
         share = (n + target_blocks - 1) // target_blocks          # weight rows of a block in the one-kernel form
         fill = share / float((share + 15) // 16 * 16)
@@ -1684,18 +1694,28 @@ def tile_plan(m: int, n: int, k: int, epi: int, aligned: bool = True, n_cu: Opti
     """(variant, splits, k_per_split) of a bfloat16 product of more than 64 rows, as the library
     chooses among its tile kernels (an estimate of the rounds their tiles take over the CUs); with
     splits > 1, K is cut over blocks and a second kernel adds the parts."""
+    return _tile_plan(m, n, k, epi, bool(aligned), n_cu or cu_count())
+
+
+@functools.lru_cache(maxsize=4096)           # (a plan depends on these numbers alone; a prompt asks for each of a few once a layer)
+def _tile_plan(m: int, n: int, k: int, epi: int, aligned: bool, n_cu: int) -> Tuple[int, int, int]:
     out = (c_int * 3)()
-    rc = _fn("gemm_bf16", "mf_gemm_bf16_tile_plan")(m, n, k, 1 if aligned else 0, epi, n_cu or cu_count(), out)
+    rc = _fn("gemm_bf16", "mf_gemm_bf16_tile_plan")(m, n, k, 1 if aligned else 0, epi, n_cu, out)
     if rc != 0:
         raise KernelError(f"tile_plan: error {rc} for m {m}, n {n}, k {k}")
     return out[0], out[1], out[2]
 
 
+@functools.lru_cache(maxsize=4096)
+def _f32_splits(m: int, n: int, k: int, aligned: bool, n_cu: int) -> int:
+    """Parts that the 32-bit product's K is cut into, as the library decides it."""
+    return _fn("gemm_f32", "mf_gemm_f32_splits")(m, n, k, 1 if aligned else 0, n_cu)
+
+
 def _k_split(m: int, n: int, k: int, swiglu: bool, aligned: bool, n_cu: Optional[int] = None,
              tiled: bool = False) -> Tuple[int, int]:
     """(splits, k_per_split) as `linear` and `linear_swiglu` cut a bfloat16 product of at most 64 rows."""
-    target = tuning.SKINNY_TARGET or n_cu
-    return skinny_plan(m, n, k, target_blocks=target, swiglu=swiglu, tiled=tiled)
+    return _skinny_plan(m, n, k, tuning.SKINNY_TARGET or n_cu or cu_count(), swiglu, tiled)
 
 
 def plan_linear(m: int, n: int, k: int, swiglu: bool = False, normed: bool = False, aligned: bool = True,
@@ -1770,7 +1790,7 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], 
     if x.dtype == torch.float32:
         _need(out, "linear.out", torch.float32)
         aligned = not (x.data_ptr() % 16 or weight.data_ptr() % 16 or k % 4)
-        splits = _fn("gemm_f32", "mf_gemm_f32_splits")(m, n, k, 1 if aligned else 0, cu_count())
+        splits = _f32_splits(m, n, k, aligned, cu_count())
         part = torch.empty(splits * m * n, dtype=torch.float32, device=x.device) if splits > 1 else None
         _check(_fn("gemm_f32", "mf_gemm_f32")(_ptr(x), k, _ptr(weight), k, _ptr(bias), _ptr(out), n, _ptr(part), m,
                                                n, k, splits, 1 if accumulate else 0, _stream()), f"gemm_f32 {m}x{n}x{k}")
@@ -2153,6 +2173,12 @@ def attn_decode_rope(qkv: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, kc
         float(scale), int(window or 0), n_splits, base, 1 if write_kv else 0, _stream()), "attn_decode_rope_bf16")
 
 
+@functools.lru_cache(maxsize=256)
+def _prefill_per_cu(head_dim: int) -> int:
+    return _fn("attn_prefill_bf16", "mf_attn_prefill_per_cu")(head_dim)
+
+
+@functools.lru_cache(maxsize=256)
 def prefill_tile(n_heads: int, n_kv_heads: int, head_dim: int):
     """(tq, gh, workgroups per block of queries): a workgroup of the prompt attention takes `gh` heads
     of a kv head's group (all of them, unless there are more than it has rows) times `tq` consecutive
@@ -2191,7 +2217,7 @@ def attn_prefill(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor, pa
     # workgroups, which take the pages in turn.
     window = int(window or 0)
     tq, gh, per_tile = prefill_tile(n_heads, n_kv_heads, head_dim)
-    per_cu = _fn("attn_prefill_bf16", "mf_attn_prefill_per_cu")(head_dim)
+    per_cu = _prefill_per_cu(head_dim)
     shared = None if tuning.NO_SHARED_PAGES else ctx.shared_query_tiles(
         tq, PAGE, window, per_tile, cu_count(), per_cu, PREFILL_MIN_PAGES, PREFILL_MAX_SHARES)
     if shared is None:
