@@ -483,6 +483,9 @@ __global__ __launch_bounds__(64) void rope_kvwrite_kernel(
 // a thread takes four neighbouring pairs at a time (float4 loads of x, cos and sin, one 8- or
 // 16-byte store per half), q and k heads first, then v: the same bytes as one wave per token and
 // head with 4-byte accesses moves, in wide accesses.
+// The rows may come in `parts` of a product whose K was split ([parts][tokens][row], added in their order, then the bias):
+// the launch and the pass of the kernel that would add them are saved (203 tokens of 36 heads in 7 parts: 6.6 + 5.6 us as
+// two kernels, 11.1 as one).
 template <typename OT>
 __device__ __forceinline__ void store4(OT* dst, float a, float b, float c, float d);
 template <>
@@ -499,19 +502,37 @@ __global__ __launch_bounds__(256) void rope_kvwrite_vec_kernel(
     const float* __restrict__ qkv, const float* __restrict__ cs, const float* __restrict__ sn,
     const int* __restrict__ positions, const int* __restrict__ seq_of_tok,
     const int* __restrict__ page_table, int pt_stride, OT* __restrict__ q_out,
-    OT* __restrict__ kcache, OT* __restrict__ vcache, int nh, int nk, int hd, int write_kv) {
+    OT* __restrict__ kcache, OT* __restrict__ vcache, int nh, int nk, int hd, int write_kv, int parts,
+    const float* __restrict__ bias) {
   const int t = blockIdx.x;
   const int half = hd >> 1, groups = half >> 2;           // groups of four pairs per head
   const int pos = positions[t];
-  const float* row = qkv + (size_t)t * (nh + 2 * nk) * hd;
+  const size_t row0 = (size_t)t * (nh + 2 * nk) * hd, stride = (size_t)gridDim.x * (nh + 2 * nk) * hd;
+  auto four = [&](int at) {                               // values at .. at + 3 of the token's row
+    const float* p = qkv + row0 + at;
+    if (parts == 1) return *reinterpret_cast<const float4*>(p);
+    float4 v = float4{0.f, 0.f, 0.f, 0.f};
+    for (int s0 = 0; s0 < parts; s0 += 8) {
+      float4 x[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        x[j] = s0 + j < parts ? *reinterpret_cast<const float4*>(p + (size_t)(s0 + j) * stride) : float4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int j = 0; j < 8; ++j) { v.x += x[j].x; v.y += x[j].y; v.z += x[j].z; v.w += x[j].w; }
+    }
+    if (bias) {
+      const float4 b = *reinterpret_cast<const float4*>(bias + at);
+      v = float4{v.x + b.x, v.y + b.y, v.z + b.z, v.w + b.w};
+    }
+    return v;
+  };
   const int page = write_kv ? page_table[(size_t)seq_of_tok[t] * pt_stride + pos / MF_PAGE] : -1;
   const int off = pos % MF_PAGE;
   const int n_rot = (nh + (write_kv && page >= 0 ? nk : 0)) * groups;
   for (int it = threadIdx.x; it < n_rot; it += 256) {
     const int head = it / groups, i = (it % groups) * 4;
-    const float* src = row + (size_t)head * hd;
-    const float4 x0 = *reinterpret_cast<const float4*>(src + i);
-    const float4 x1 = *reinterpret_cast<const float4*>(src + i + half);
+    const float4 x0 = four(head * hd + i);
+    const float4 x1 = four(head * hd + i + half);
     const float4 c = cs ? *reinterpret_cast<const float4*>(cs + (size_t)pos * half + i) : make_float4(1.f, 1.f, 1.f, 1.f);
     const float4 s = cs ? *reinterpret_cast<const float4*>(sn + (size_t)pos * half + i) : make_float4(0.f, 0.f, 0.f, 0.f);
     OT* dst = head < nh ? q_out + ((size_t)t * nh + head) * hd
@@ -522,10 +543,9 @@ __global__ __launch_bounds__(256) void rope_kvwrite_vec_kernel(
                x0.w * s.w + x1.w * c.w);
   }
   if (!write_kv || page < 0) return;
-  const float* vsrc = row + (size_t)(nh + nk) * hd;
   for (int it = threadIdx.x; it < nk * (hd >> 2); it += 256) {
     const int hk = it / (hd >> 2), i = (it % (hd >> 2)) * 4;
-    const float4 v = *reinterpret_cast<const float4*>(vsrc + (size_t)hk * hd + i);
+    const float4 v = four((nh + nk + hk) * hd + i);
     if (V_TRANSPOSED) {                   // a page of V is [2][hd][32 keys]
       constexpr int VH = MF_PAGE / 2;
       OT* dst = vcache + ((((size_t)page * nk + hk) * 2 + off / VH) * hd + i) * VH + off % VH;
@@ -596,23 +616,24 @@ MF_API int mf_rope_pairs_inplace(float* x, const float* cs, const float* sn, con
 MF_API int mf_rope_kvwrite(const float* qkv, const float* cs, const float* sn, const int* positions,
                            const int* seq_of_tok, const int* page_table, int pt_stride, void* q_out,
                            void* kcache, void* vcache, int is_bf16, int n_tok, int nh, int nk, int hd,
-                           int write_kv, hipStream_t stream) {
+                           int write_kv, int parts, const float* bias, hipStream_t stream) {
   if (n_tok <= 0) return 0;
-  if ((cs == nullptr) != (sn == nullptr)) return (int)hipErrorInvalidValue;
-  const bool vec = hd % 8 == 0 && (uintptr_t)qkv % 16 == 0 && (uintptr_t)cs % 16 == 0 && (uintptr_t)sn % 16 == 0 &&
+  if ((cs == nullptr) != (sn == nullptr) || parts < 1 || (parts == 1 && bias)) return (int)hipErrorInvalidValue;
+  const bool vec = hd % 8 == 0 && (uintptr_t)bias % 16 == 0 && (uintptr_t)qkv % 16 == 0 && (uintptr_t)cs % 16 == 0 && (uintptr_t)sn % 16 == 0 &&
                    (uintptr_t)q_out % 16 == 0 && (uintptr_t)kcache % 16 == 0 && (uintptr_t)vcache % 16 == 0;
   if (vec) {
     if (is_bf16)
       rope_kvwrite_vec_kernel<bf16, true><<<n_tok, 256, 0, stream>>>(qkv, cs, sn, positions, seq_of_tok, page_table,
                                                                      pt_stride, (bf16*)q_out, (bf16*)kcache,
-                                                                     (bf16*)vcache, nh, nk, hd, write_kv);
+                                                                     (bf16*)vcache, nh, nk, hd, write_kv, parts, bias);
     else
       rope_kvwrite_vec_kernel<float, false><<<n_tok, 256, 0, stream>>>(qkv, cs, sn, positions, seq_of_tok,
                                                                        page_table, pt_stride, (float*)q_out,
                                                                        (float*)kcache, (float*)vcache, nh, nk, hd,
-                                                                       write_kv);
+                                                                       write_kv, parts, bias);
     return mf_launch_status();
   }
+  if (parts > 1) return (int)hipErrorInvalidValue;        // (the caller asks for parts only where the kernel above runs)
   dim3 grid(n_tok, write_kv ? nh + 2 * nk : nh);
   if (is_bf16)
     rope_kvwrite_kernel<bf16, true><<<grid, 64, 0, stream>>>(qkv, cs, sn, positions, seq_of_tok, page_table,

@@ -2018,6 +2018,76 @@ __global__ __launch_bounds__(256) void skinny_reduce4_kernel(const float* __rest
   }
 }
 
+// The kernel that adds the parts of a K split into the residual stream and norms the new rows for the product that reads
+// them next (more than 64 rows, where that product takes them normed): a block a row, which it holds in registers between
+// the sum of squares and the scaling.  The additions are those of `skinny_reduce4_kernel` and the norm that of
+// `rmsnorm_kernel`, in their order.  One launch for two, and the rows are not read again: 203 rows of 3,584 values in 9
+// parts 6.6 + 4.7 us as two kernels, 9.1 as this one; 2,048 rows in two parts 20.9 + 10.2 and 23.6.
+template <int KEEP>
+__global__ __launch_bounds__(256) void reduce_norm_kernel(const float* __restrict__ part, const float* __restrict__ bias,
+                                                          float* __restrict__ C, int ldc, int M, int N, int splits, int accumulate,
+                                                          const float* __restrict__ g, float eps, bf16* __restrict__ normed) {
+  __shared__ float scratch[4];
+  const int m = blockIdx.x;
+  const size_t stride = (size_t)M * N;
+  const float* p = part + (size_t)m * N;
+  float* c = C + (size_t)m * ldc;
+  float4 v[KEEP];
+  float ss = 0.f;
+#pragma unroll
+  for (int q = 0; q < KEEP; ++q) {
+    const int n = (q * 256 + threadIdx.x) * 4;
+    v[q] = float4{0.f, 0.f, 0.f, 0.f};
+    if (n < N) {
+      const float4 old = accumulate ? *reinterpret_cast<const float4*>(c + n) : v[q];
+      for (int s0 = 0; s0 < splits; s0 += 8) {               // eight parts' loads in flight together, added in their order
+        float4 x[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          x[j] = s0 + j < splits ? *reinterpret_cast<const float4*>(p + (size_t)(s0 + j) * stride + n) : float4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < 8; ++j) { v[q].x += x[j].x; v[q].y += x[j].y; v[q].z += x[j].z; v[q].w += x[j].w; }
+      }
+      if (bias) {
+        const float4 b = *reinterpret_cast<const float4*>(bias + n);
+        v[q] = float4{v[q].x + b.x, v[q].y + b.y, v[q].z + b.z, v[q].w + b.w};
+      }
+      if (accumulate) v[q] = float4{v[q].x + old.x, v[q].y + old.y, v[q].z + old.z, v[q].w + old.w};
+      *reinterpret_cast<float4*>(c + n) = v[q];
+    }
+    ss = fmaf(v[q].x, v[q].x, ss);
+    ss = fmaf(v[q].y, v[q].y, ss);
+    ss = fmaf(v[q].z, v[q].z, ss);
+    ss = fmaf(v[q].w, v[q].w, ss);
+  }
+  ss = block_sum<256>(ss, scratch);
+  const float scale = 1.0f / sqrtf(ss / (float)N + eps);
+#pragma unroll
+  for (int q = 0; q < KEEP; ++q) {
+    const int n = (q * 256 + threadIdx.x) * 4;
+    if (n < N) {
+      const float4 w = *reinterpret_cast<const float4*>(g + n);
+      *reinterpret_cast<bf16x4*>(normed + (size_t)m * N + n) =
+          bf16x4{(bf16)(v[q].x * scale * w.x), (bf16)(v[q].y * scale * w.y), (bf16)(v[q].z * scale * w.z), (bf16)(v[q].w * scale * w.w)};
+    }
+  }
+}
+
+constexpr int REDUCE_NORM_MAX = 256 * 4 * 16;                // a row's values that a block holds
+
+int launch_reduce_norm(const float* part, const float* bias, float* C, int ldc, int M, int N, int splits, int accumulate,
+                       const float* g, float eps, bf16* normed, hipStream_t stream) {
+  auto run = [&](auto KEEP) {
+    reduce_norm_kernel<decltype(KEEP)::value><<<M, 256, 0, stream>>>(part, bias, C, ldc, M, N, splits, accumulate, g, eps, normed);
+  };
+  if (N <= 1024) run(std::integral_constant<int, 1>{});
+  else if (N <= 2048) run(std::integral_constant<int, 2>{});
+  else if (N <= 4096) run(std::integral_constant<int, 4>{});
+  else if (N <= 8192) run(std::integral_constant<int, 8>{});
+  else run(std::integral_constant<int, 16>{});
+  return mf_launch_status();
+}
+
 // adds the parts of a K split and runs the epilogue: the kernel in fours where the operands allow it
 int launch_reduce(const float* part, const float* bias, void* C, int ldc, int M, int N, int K, int splits, int epi,
                   const FusedNorm& fused, hipStream_t stream) {
@@ -2200,7 +2270,7 @@ TilePlan plan_tiles(int M, int N, int K, bool dma_ok, int epi, int n_cu) {
     splits = (int)((chunks + c - 1) / c);
     per = (int)(c * 256);
   };
-  auto parts_us = [&](int splits) { return (double)(splits + 2) * mn * 4. / 3.5e6 + 5.; };
+  auto parts_us = [&](int splits) { return (double)(splits + 2) * mn * 4. / 6e6 + 4.; };
   TilePlan best{0, 1, K, 1e30};
   auto offer = [&](int variant, int splits, int per, double us) {
     if (us < best.us) best = TilePlan{variant, splits, per, us};
@@ -2325,16 +2395,13 @@ MF_API int mf_gemm_bf16(const void* A, int lda, const void* W, int ldw, const fl
 
 // Few rows for the tile kernel (a prompt of a few hundred tokens against 3584 weight rows makes
 // some 50 tiles for 256 CUs): K is split over `splits` blocks per tile, which store 32-bit sums
-// into part[splits][M][N], and skinny_reduce_kernel adds them and runs the epilogue.
+// into part[splits][M][N] (`mf_gemm_bf16_parts`), and skinny_reduce_kernel adds them and runs the epilogue.
 // k_per_split is a multiple of 64.
-MF_API int mf_gemm_bf16_splitk(const void* A, int lda, const void* W, int ldw, const float* bias, void* C,
-                               int ldc, float* part, int M, int N, int K, int splits, int k_per_split,
-                               int epi, int variant, hipStream_t stream) {
+MF_API int mf_gemm_bf16_parts(const void* A, int lda, const void* W, int ldw, float* part, int M, int N, int K, int splits,
+                              int k_per_split, int variant, hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
-  if (K <= 0 || lda < K || ldw < K || epi < 0 || epi > EPI_XIELU || (epi == EPI_XIELU && !bias) || splits < 2 || !part || k_per_split % 64 != 0 ||
-      (long)splits * k_per_split < K || (long)(splits - 1) * k_per_split >= K)
-    return (int)hipErrorInvalidValue;
-  if (epi == EPI_SWIGLU ? (N % 64 != 0 || ldc > N / 2 || ldc <= N / 2 - 32) : ldc < N)
+  if (K <= 0 || lda < K || ldw < K || splits < 2 || !part || k_per_split % 64 != 0 || (long)splits * k_per_split < K ||
+      (long)(splits - 1) * k_per_split >= K)
     return (int)hipErrorInvalidValue;
   const int vec_ok = (lda % 8 == 0) && (ldw % 8 == 0) && ((uintptr_t)A % 16 == 0) &&
                      ((uintptr_t)W % 16 == 0) && (K % 8 == 0);
@@ -2343,12 +2410,38 @@ MF_API int mf_gemm_bf16_splitk(const void* A, int lda, const void* W, int ldw, c
   if (variant != 12 && variant != 2) return (int)hipErrorInvalidValue;
   const bool dma_ok = vec_ok && K % DMA_BK == 0 && (size_t)M * lda * 2 < (1ull << 32) && (size_t)N * ldw * 2 < (1ull << 32);
   if (variant == 12 && !dma_ok) return (int)hipErrorInvalidValue;
-  int rc = dma_ok ? launch_form(dma_form(variant, M, N, EPI_F32, k_per_split / DMA_BK, splits, cu_count()), (const bf16*)A, lda,
-                                (const bf16*)W, ldw, nullptr, part, N, M, N, K, EPI_F32, stream, splits, k_per_split)
-                  : launch_tile<128, 128, 64, 64>((const bf16*)A, lda, (const bf16*)W, ldw, nullptr, part, N, M,
-                                                  N, K, EPI_F32, vec_ok, stream, splits, k_per_split);
+  return dma_ok ? launch_form(dma_form(variant, M, N, EPI_F32, k_per_split / DMA_BK, splits, cu_count()), (const bf16*)A, lda,
+                              (const bf16*)W, ldw, nullptr, part, N, M, N, K, EPI_F32, stream, splits, k_per_split)
+                : launch_tile<128, 128, 64, 64>((const bf16*)A, lda, (const bf16*)W, ldw, nullptr, part, N, M,
+                                                N, K, EPI_F32, vec_ok, stream, splits, k_per_split);
+}
+
+MF_API int mf_gemm_bf16_splitk(const void* A, int lda, const void* W, int ldw, const float* bias, void* C,
+                               int ldc, float* part, int M, int N, int K, int splits, int k_per_split,
+                               int epi, int variant, hipStream_t stream) {
+  if (M <= 0 || N <= 0) return 0;
+  if (epi < 0 || epi > EPI_XIELU || (epi == EPI_XIELU && !bias)) return (int)hipErrorInvalidValue;
+  if (epi == EPI_SWIGLU ? (N % 64 != 0 || ldc > N / 2 || ldc <= N / 2 - 32) : ldc < N)
+    return (int)hipErrorInvalidValue;
+  const int rc = mf_gemm_bf16_parts(A, lda, W, ldw, part, M, N, K, splits, k_per_split, variant, stream);
   if (rc) return rc;
   return launch_reduce(part, bias, C, ldc, M, N, K, splits, epi, FusedNorm{}, stream);
+}
+
+// The same into the residual stream (32-bit C, stored or added to), with the RMS norm of the new rows beside it: normed =
+// bfloat16 C / sqrt(mean(C^2) + eps) g, [M][N].  N in fours, at most 16,384, every operand 16-byte aligned; MF_NOT_BUILT
+// (nothing launched) for any other.
+MF_API int mf_gemm_bf16_splitk_norm(const void* A, int lda, const void* W, int ldw, const float* bias, float* C, int ldc,
+                                    float* part, int M, int N, int K, int splits, int k_per_split, int accumulate, int variant,
+                                    const float* g, float eps, void* normed, hipStream_t stream) {
+  if (M <= 0 || N <= 0) return 0;
+  if (N % 4 || N > REDUCE_NORM_MAX || ldc % 4 || (uintptr_t)C % 16 || (uintptr_t)part % 16 || (uintptr_t)bias % 16 ||
+      (uintptr_t)g % 16 || (uintptr_t)normed % 8 || !g || !normed)
+    return MF_NOT_BUILT;
+  if (ldc < N) return (int)hipErrorInvalidValue;
+  const int rc = mf_gemm_bf16_parts(A, lda, W, ldw, part, M, N, K, splits, k_per_split, variant, stream);
+  if (rc) return rc;
+  return launch_reduce_norm(part, bias, C, ldc, M, N, splits, accumulate, g, eps, (bf16*)normed, stream);
 }
 
 // The register-resident kernel for the shapes it is built for (K = 256 NS with enough tiles to

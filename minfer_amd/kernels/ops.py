@@ -39,7 +39,7 @@ _PROTOTYPES = {
         "mf_convert": [_P, c_int, _P, c_int, c_size_t, _P],
         "mf_rope_table": [_P, _P, c_int, c_int, c_double, c_double, _P],
         "mf_rope_kvwrite": [_P, _P, _P, _P, _P, _P, c_int, _P, _P, _P, c_int, c_int, c_int, c_int,
-                            c_int, c_int, _P],
+                            c_int, c_int, c_int, _P, _P],
         "mf_rope_inplace": [_P, _P, _P, _P, c_int, c_int, c_int, c_int, _P],
         "mf_fill_normal": [_P, c_int, c_size_t, c_uint64, c_float, c_int, _P],
         "mf_group_rmsnorm": [_P, _P, _P, _P, c_int, c_int, _P, c_int, c_int, c_int, c_float, _P],
@@ -138,6 +138,9 @@ _PROTOTYPES = {
         "mf_gemm_bf16_grouped": [_P, _P, _P, _P, c_int, c_int, c_int, c_int, _P],
         "mf_gemm_bf16_splitk": [_P, c_int, _P, c_int, _P, _P, c_int, _P, c_int, c_int, c_int, c_int, c_int, c_int,
                                 c_int, _P],
+        "mf_gemm_bf16_parts": [_P, c_int, _P, c_int, _P, c_int, c_int, c_int, c_int, c_int, c_int, _P],
+        "mf_gemm_bf16_splitk_norm": [_P, c_int, _P, c_int, _P, _P, c_int, _P, c_int, c_int, c_int, c_int, c_int, c_int, c_int,
+                                     _P, c_float, _P, _P],
         "mf_gemm_bf16_skinny": [_P, c_int, _P, _P, c_int, _P, _P, c_int, _P, c_int, c_int, c_int, c_int,
                                 c_int, c_int, _P],
         "mf_gemm_bf16_normed": [_P, c_int, _P, _P, c_float, _P, _P, c_int, _P, _P, c_int, c_int, c_int, c_int,
@@ -510,12 +513,19 @@ def rope_inplace(qkv: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, positi
 def rope_kvwrite(qkv: torch.Tensor, cos: Optional[torch.Tensor], sin: Optional[torch.Tensor],
                  positions: torch.Tensor, seq_of_tok: torch.Tensor, page_table: torch.Tensor, q_out: torch.Tensor,
                  kcache: Optional[torch.Tensor], vcache: Optional[torch.Tensor], n_heads: int,
-                 n_kv_heads: int, head_dim: int, write_kv: bool = True) -> None:
+                 n_kv_heads: int, head_dim: int, write_kv: bool = True, bias: Optional[torch.Tensor] = None) -> None:
     """Rotates q and k, and stores k and v of the tokens at their positions in the cache pages
     (`v_page_shape` says how V lies in a page).  Without tables (cos and sin None) nothing is
-    rotated: q is rounded into q_out and k, v are stored as they come."""
-    n_tok = positions.numel()
-    _need(qkv, "rope.qkv", torch.float32, (n_tok, (n_heads + 2 * n_kv_heads) * head_dim))
+    rotated: q is rounded into q_out and k, v are stored as they come.  `qkv` may be the parts
+    `[parts][tokens][row]` of a product whose K was split (`linear_parts`), added up on the way, `bias`
+    then the product's (head sizes in 8s, operands 16-byte aligned)."""
+    n_tok, width = positions.numel(), (n_heads + 2 * n_kv_heads) * head_dim
+    parts = qkv.shape[0] if qkv.dim() == 3 else 1
+    _need(qkv, "rope.qkv", torch.float32, (n_tok, width) if qkv.dim() != 3 else (parts, n_tok, width))
+    if bias is not None:
+        if parts == 1:
+            raise KernelError("rope: a bias belongs to the parts of a split product")
+        _need(bias, "rope.bias", torch.float32, (width,))
     if (cos is None) != (sin is None):
         raise KernelError("rope: cos and sin come together or not at all")
     if cos is not None:
@@ -533,7 +543,7 @@ def rope_kvwrite(qkv: torch.Tensor, cos: Optional[torch.Tensor], sin: Optional[t
         _ptr(qkv), _ptr(cos), _ptr(sin), _ptr(positions), _ptr(seq_of_tok), _ptr(page_table),
         page_table.shape[1], _ptr(q_out), _ptr(kcache if write_kv else None),
         _ptr(vcache if write_kv else None), _is_bf16(q_out), n_tok, n_heads, n_kv_heads, head_dim,
-        1 if write_kv else 0, _stream()), "rope_kvwrite")
+        1 if write_kv else 0, parts, _ptr(bias), _stream()), "rope_kvwrite")
 
 
 # ------------------------------------------------------------------ norm in groups, xIELU, frequency tables
@@ -1817,6 +1827,57 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], 
             return
     _check(_fn("gemm_bf16", "mf_gemm_bf16")(_ptr(x), k, _ptr(weight), k, _ptr(bias), _ptr(out), n, m,
                                              n, k, epi, variant, _stream()), f"gemm_bf16 {m}x{n}x{k}")
+
+
+def linear_parts(x: torch.Tensor, weight: torch.Tensor) -> Optional[torch.Tensor]:
+    """The product of more than 64 bfloat16 rows as `linear` would cut it over K, its parts not yet added: float32
+    `[parts][m][n]` in the scratch the next split product reuses (without bias), or None, nothing launched, where `linear`
+    does not cut it."""
+    _need(x, "linear_parts.x", torch.bfloat16)
+    _need(weight, "linear_parts.weight", torch.bfloat16)
+    m, k = x.shape
+    n = weight.shape[0]
+    if weight.shape[1] != k:
+        raise KernelError(f"linear_parts: x is [{m},{k}], weight is {tuple(weight.shape)}")
+    if m <= 64:
+        return None
+    variant, splits, per = tile_plan(m, n, k, EPI_F32, not (x.data_ptr() % 16 or weight.data_ptr() % 16 or k % 8))
+    if splits <= 1:
+        return None
+    part = workspace("skinny", splits * m * n, x.device)[:splits * m * n].view(splits, m, n)
+    _check(_fn("gemm_bf16", "mf_gemm_bf16_parts")(_ptr(x), k, _ptr(weight), k, _ptr(part), m, n, k, splits, per, variant,
+                                                   _stream()), f"gemm_bf16_parts {m}x{n}x{k}")
+    return part
+
+
+def linear_norm_out(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], out: torch.Tensor, accumulate: bool,
+                    g: torch.Tensor, eps: float) -> Optional[torch.Tensor]:
+    """out (+)= x weight^T (+ bias) for more than 64 bfloat16 rows into float32 `out`, where `linear` would cut the product
+    over K, and out / sqrt(mean(out^2) + eps) g in bfloat16, which the kernel that adds the parts leaves beside it and
+    which is returned.  None, nothing launched, for any other shape."""
+    m, k = x.shape
+    n = weight.shape[0]
+    if m <= 64 or x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 or weight.shape[1] != k:
+        return None
+    variant, splits, per = tile_plan(m, n, k, EPI_ACC_F32 if accumulate else EPI_F32,
+                                     not (x.data_ptr() % 16 or weight.data_ptr() % 16 or k % 8))
+    if splits <= 1:
+        return None
+    _need(x, "linear_norm_out.x")
+    _need(weight, "linear_norm_out.weight")
+    _need(out, "linear_norm_out.out", torch.float32, (m, n))
+    _need(g, "linear_norm_out.g", torch.float32, (n,))
+    if bias is not None:
+        _need(bias, "linear_norm_out.bias", torch.float32, (n,))
+    normed = torch.empty((m, n), dtype=torch.bfloat16, device=x.device)
+    part = workspace("skinny", splits * m * n, x.device)
+    rc = _fn("gemm_bf16", "mf_gemm_bf16_splitk_norm")(_ptr(x), k, _ptr(weight), k, _ptr(bias), _ptr(out), n, _ptr(part), m, n, k,
+                                                      splits, per, 1 if accumulate else 0, variant, _ptr(g), float(eps),
+                                                      _ptr(normed), _stream())
+    if rc == NOT_BUILT:
+        return None
+    _check(rc, f"gemm_bf16_splitk_norm {m}x{n}x{k}")
+    return normed
 
 
 # variants of the grouped product: (tile rows, tile columns, blocks a CU, microseconds a k tile of 64 with every CU

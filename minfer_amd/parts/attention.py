@@ -73,10 +73,21 @@ class GQAttention(Mixer):
     def forward(self, x, h, ctx, entry: int, writes_cache: bool) -> None:
         kc, vc, group = ctx.cache.kv(entry)
         table = ctx.page_table(group)
-        qkv = self.qkv(x, out_dtype=torch.float32)
         window = 0 if self.window is None else int(self.window)
         o = torch.empty((x.shape[0], self.nh * self.hd), dtype=self.rt.dtype, device=x.device)
         tables = self.position.rotation_tables(ctx.max_len)
+        # a product cut over K leaves its parts to the kernel that rotates and stores
+        parts = None
+        if tables is not None and self.rt.is_bf16 and not ctx.all_decode and self.hd % 8 == 0:
+            parts = self.qkv.parts(x)
+        if parts is not None:
+            q = torch.empty_like(o)
+            ops.rope_kvwrite(parts, tables[0], tables[1], ctx.positions, ctx.seq_of_tok, table, q, kc, vc,
+                             self.nh, self.nk, self.hd, writes_cache, bias=self.qkv.bias)
+            self._attend(q, kc, vc, table, ctx, o, window)
+            self.o(o, out=h, accumulate=True, ctx=ctx)
+            return
+        qkv = self.qkv(x, out_dtype=torch.float32)
         if tables is not None and self.rt.is_bf16 and ctx.all_decode:
             # decode: rotation, cache write and attention in one kernel
             ops.attn_decode_rope(qkv, tables[0], tables[1], kc, vc, table, ctx.positions, ctx.seq_of_tok, o,
@@ -94,9 +105,13 @@ class GQAttention(Mixer):
             else:
                 ops.rope_kvwrite(qkv, None, None, ctx.positions, ctx.seq_of_tok, table, q, None, None,
                                  self.nh, self.nk, self.hd, False)
+        self._attend(q, kc, vc, table, ctx, o, window)
+        self.o(o, out=h, accumulate=True, ctx=ctx)
+
+    def _attend(self, q, kc, vc, table, ctx, o, window: int) -> None:
+        """Every new token of a step over its sequence's cache rows, the step's own stored already."""
         if self.rt.is_bf16 and not ctx.all_decode and ops.HAVE_PREFILL_ATTENTION:
             ops.attn_prefill(q, kc, vc, table, ctx, o, self.nh, self.nk, self.hd, self.scale, window)
         else:
             ops.attn_tokens(q, kc, vc, table, ctx.positions, ctx.seq_of_tok, o, self.nh, self.nk,
                             self.hd, self.scale, window, ctx.max_len)
-        self.o(o, out=h, accumulate=True, ctx=ctx)

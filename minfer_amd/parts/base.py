@@ -85,11 +85,12 @@ class Norm(Part):
 class NormAhead:
     """What a product that added into the residual stream `h` left for `norm`, the norm that reads
     the stream next: bf16(h g) and, per row, partial sums of h^2 (`ops.linear_fused`).  The product
-    that follows the norm may take these instead of the normed rows."""
+    that follows the norm may take these instead of the normed rows.  Without sums, `xg` is the
+    normed rows themselves (`ops.linear_norm_out`)."""
     norm: "Norm"
     h: torch.Tensor
     xg: torch.Tensor
-    sums: torch.Tensor
+    sums: Optional[torch.Tensor]
 
 
 class Normed:
@@ -102,8 +103,10 @@ class Normed:
     def __init__(self, norm: "Norm", h: torch.Tensor, row_idx: Optional[torch.Tensor] = None,
                  ahead: Optional[NormAhead] = None):
         self.norm, self.h, self.row_idx = norm, h, row_idx
-        self.ahead = ahead
         self._rows: Optional[torch.Tensor] = None
+        if ahead is not None and ahead.sums is None:     # the product before has normed them already
+            self._rows, ahead = ahead.xg, None
+        self.ahead = ahead
 
     @property
     def shape(self):
@@ -130,6 +133,8 @@ def normed_input(norm: "Norm", part, h: torch.Tensor, row_idx: Optional[torch.Te
             ahead = None
     if getattr(part, "takes_normed", False):
         return Normed(norm, h, row_idx, ahead)
+    if ahead is not None and ahead.sums is None:
+        return ahead.xg
     return norm.forward(h, row_idx=row_idx)
 
 

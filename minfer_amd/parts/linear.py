@@ -83,17 +83,37 @@ class Linear:
         ops.linear(x, self.weight, self.bias, out, accumulate=accumulate, tiled=self.tiled)
         return out
 
+    def parts(self, x):
+        """The product's parts `[parts][rows][out_features]` (float32, without the bias) where it is cut over K and a kernel
+        behind it can add them up (`ops.linear_parts`), else None, nothing launched."""
+        if isinstance(x, Normed):
+            if x.shape[0] <= 64:
+                return None
+            x = x.tensor()
+        if x.device.type != "cuda" or x.shape[0] <= 64 or x.dtype != torch.bfloat16 or self.weight.dtype != torch.bfloat16:
+            return None
+        return ops.linear_parts(x, self.weight)
+
     def _prepare_norm(self, x: torch.Tensor, out: torch.Tensor, accumulate: bool, ctx) -> bool:
         """Runs the product with the next norm's input prepared beside it (bf16(out g) and the rows'
         partial sums of squares, left in `ctx.norm_ahead`) where the block has said which norm
         that is, the norm is of the RMS form and the product's kernels have a place for it (steps of
         17 to 64 rows whose K is split over blocks; steps of at most 16 rows in the one-kernel
-        forms).  False: nothing ran."""
+        forms; steps of more rows whose K is split: there the normed rows themselves).  False: nothing ran."""
         norm = getattr(ctx, "norm_next", None)
-        if norm is None or not 0 < x.shape[0] <= 64 or x.dtype != torch.bfloat16 or out.dtype != torch.float32:
+        if norm is None or x.shape[0] == 0 or x.dtype != torch.bfloat16 or out.dtype != torch.float32:
             return False
         if tuning.NO_NORM_AHEAD or x.device.type != "cuda":
             return False
+        if x.shape[0] > 64:
+            fold = norm.rms_scale()
+            if fold is None or fold[0].numel() != self.out_features:
+                return False
+            normed = ops.linear_norm_out(x, self.weight, self.bias, out, accumulate, fold[0], fold[1])
+            if normed is None:
+                return False
+            ctx.norm_ahead = NormAhead(norm, out, normed, None)
+            return True
         lo, hi = ops.NORM_AHEAD_16_WIDTHS
         if x.shape[0] <= 16 and not lo <= self.out_features <= hi:
             return False

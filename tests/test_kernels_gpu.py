@@ -759,6 +759,47 @@ def test_gemm_bf16_swiglu_tile_forms(ops, variant, m, nf, k):
     test_gemm_bf16_swiglu(ops, variant, m, nf, k)
 
 
+# a product cut over K whose parts the next kernel adds: into the stream with the norm of the new rows (rows of one, two, four,
+# eight and sixteen runs of 1,024 values, whole and not), and under the rotation; the same bits as one kernel after the other
+@pytest.mark.parametrize("m,n,k", [(65, 896, 4864), (203, 3584, 3584), (100, 1028, 2048), (100, 8192, 8192), (66, 9000, 8192),
+                                   (1030, 776, 6144)])
+def test_split_product_with_norm(ops, m, n, k):
+    x, w = rnd((m, k), torch.bfloat16, 8).to(DEV), rnd((n, k), torch.bfloat16, 9, 0.05).to(DEV)
+    b, g, base = rnd((n,), seed=10).to(DEV), rnd((n,), seed=11).to(DEV), rnd((m, n), seed=12).to(DEV)
+    assert ops.tile_plan(m, n, k, ops.EPI_ACC_F32)[1] > 1
+    for accumulate, bias in ((True, None), (False, b)):
+        want, got = base.clone(), base.clone()
+        ops.linear(x, w, bias, want, accumulate=accumulate)
+        want_n = torch.empty(m, n, dtype=torch.bfloat16, device=DEV)
+        ops.rmsnorm(want, g, 1e-6, want_n)
+        normed = ops.linear_norm_out(x, w, bias, got, accumulate, g, 1e-6)
+        assert torch.equal(got, want) and torch.equal(normed, want_n)
+    assert ops.linear_norm_out(x[:64], w, None, got[:64], True, g, 1e-6) is None
+
+
+@pytest.mark.parametrize("nh,nk,hd,k", [(28, 4, 128, 3584), (3, 1, 24, 4096), (14, 2, 64, 4864)])
+def test_rope_kvwrite_of_parts(ops, nh, nk, hd, k):
+    t, width = 67, (nh + 2 * nk) * hd
+    x, w, b = rnd((t, k), torch.bfloat16, 8).to(DEV), rnd((width, k), torch.bfloat16, 9, 0.05).to(DEV), rnd((width,), seed=10).to(DEV)
+    pos = torch.arange(t, dtype=torch.int32, device=DEV)
+    seq, table = torch.zeros(t, dtype=torch.int32, device=DEV), torch.tensor([[3, 1]], dtype=torch.int32, device=DEV)
+    cs, sn = ops.rope_table(128, hd // 2, 1e4, 1.0, DEV)
+    got = []
+    for split in (False, True):
+        kc, vc = make_cache(4, nk, hd, torch.bfloat16, 7)
+        kd, vd = kc.to(DEV), stored_v(vc).to(DEV)
+        q = torch.empty(t, nh * hd, dtype=torch.bfloat16, device=DEV)
+        qkv = ops.linear_parts(x, w) if split else torch.empty(t, width, device=DEV)
+        if not split:
+            ops.linear(x, w, b, qkv)
+        assert not split or (qkv.dim() == 3 and qkv.shape[0] > 1)
+        ops.rope_kvwrite(qkv, cs, sn, pos, seq, table, q, kd, vd, nh, nk, hd, bias=b if split else None)
+        got.append((q, kd, vd))
+    for a, c in zip(*got):
+        assert torch.equal(a, c)
+    assert ops.linear_parts(x[:64], w) is None
+
+
 @pytest.mark.parametrize("m,n,k,idx", [(1, 2100, 1536, False), (5, 4608, 2048, True), (8, 4001, 3584, False),
                                        (16, 2048, 4096, True), (3, 152064, 3584, True),
                                        (2, 2100, 5120, True), (9, 5000, 5120, False), (7, 5000, 8192, True),
