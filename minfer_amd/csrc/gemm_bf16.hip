@@ -356,7 +356,7 @@ struct DmaTile {
   static constexpr bool PAIRED = J % 4 != 0;
   static constexpr int STEP = PAIRED ? 2 : 1;
   static __device__ __forceinline__ int first(int n) {
-    return !PAIRED ? n * J : J == 2 ? (n >> 1) * 4 + (n & 1) : n;
+    return PAIRED ? n : n * J;
   }
   // copies per wave: a half of A; the halves of W
   static constexpr int LA = BM / 128, LW0 = J0 * WAVES_N / 4, LW1 = J1 * WAVES_N / 4;
@@ -684,6 +684,145 @@ __global__ __launch_bounds__(512, 2) void tile_dma_kernel(const bf16* __restrict
   dma_wait<0>();
   dma_meet();
   dma_epilogue<TT>(acc, smem + wid * TT::OWN, bias, C, ldc, M, N, epi, m0 + wave_m * TT::ROWS, n0, wave_n, lane);
+}
+
+// ---- the smaller tiles: one barrier a k tile
+// 128 x 128 on 8 waves and 64 x 64 on 4, for products whose larger tiles would leave most of the chip idle: a block's time
+// is then its own chain of k tiles, whatever the others do, and a k tile's chain is what is kept short: wait for the copies
+// of one k tile, meet, set out the copies STAGES - 1 tiles on, read every fragment, multiply.  (The quarter products of
+// `tile_dma_kernel` meet eight times a k tile, which 128 x 128 cannot fill: 203 rows against 9,728 of 896 15.5 us so, 12.6
+// here; 2,048 x 2,048 x 2,048 27.2 and 23.3.  At 256 x 128 the two are level.)  64 x 64: 203 rows against 1,152 of 896 (the
+// narrowest model's q|k|v) 11.6 us as 128 x 128, 6.4 so.
+template <int BM, int BN, int WAVES_M_, int WAVES_N_>
+struct StepTile {
+  static constexpr int WAVES_M = WAVES_M_, WAVES_N = WAVES_N_, WAVES = WAVES_M * WAVES_N;
+  static constexpr int ROWS = BM / WAVES_M, COLS = BN / WAVES_N, I = ROWS / 16, J = COLS / 16;
+  // a wave's two column blocks are a gate block and its up block (see DmaTile)
+  static constexpr bool PAIRED = true;
+  static constexpr int STEP = 2;
+  static __device__ __forceinline__ int first(int n) { return (n >> 1) * 4 + (n & 1); }
+  static constexpr int LA = BM / 8 / WAVES, LW = BN / 8 / WAVES;       // copies per wave
+  static constexpr int OWN = 32 * (COLS + 4) * 4;
+  template <int STAGES> static constexpr int lds() {
+    return STAGES * (BM + BN) * DMA_BK * 2 > WAVES * OWN ? STAGES * (BM + BN) * DMA_BK * 2 : WAVES * OWN;
+  }
+  static_assert(J == 2 && I % 2 == 0 && BM % (8 * WAVES) == 0 && BN % (8 * WAVES) == 0, "pairs of blocks, whole copies per wave");
+};
+
+template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, bool GROUPED = false>
+__global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void tile_step_kernel(const bf16* __restrict__ A, int lda,
+                                                       const bf16* __restrict__ W, int ldw,
+                                                       const float* __restrict__ bias, void* __restrict__ C,
+                                                       int ldc, int M, int N, int K, int epi, int tiles_m,
+                                                       int xcd_remap, int k_per_split,
+                                                       const RowGroup* __restrict__ groups = nullptr) {
+  using TT = StepTile<BM, BN, WAVES_M, WAVES_N>;
+  constexpr int ROW = DMA_BK * 2, ST = (BM + BN) * ROW, WAVES = TT::WAVES, I = TT::I, J = TT::J, LA = TT::LA, LW = TT::LW;
+  if (k_per_split > 0) {                                     // as in tile_dma_kernel
+    const int kb = blockIdx.y * k_per_split;
+    A += kb;
+    W += kb;
+    K = min(k_per_split, K - kb);
+    C = (float*)C + (size_t)blockIdx.y * M * N;
+  }
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];      // [stage][BM rows of A, BN rows of W][64]
+  int tile = blockIdx.x;
+  if (xcd_remap) {
+    const int n_tiles = gridDim.x, per = n_tiles / 8, rem = n_tiles % 8;
+    const int x = blockIdx.x % 8, qq = blockIdx.x / 8;
+    tile = x * per + min(x, rem) + qq;
+  }
+  int bm, bn;
+  tile_position(tile, tiles_m, gridDim.x / tiles_m, bm, bn);
+  if (GROUPED) {
+    const int first = __builtin_amdgcn_readfirstlane(groups[bm].first), matrix = __builtin_amdgcn_readfirstlane(groups[bm].matrix);
+    M = __builtin_amdgcn_readfirstlane(groups[bm].rows);
+    A += (size_t)first * lda;
+    W += (size_t)matrix * N * ldw;
+    C = (float*)C + (size_t)first * ldc;
+    bm = 0;
+  }
+  const int m0 = bm * BM, n0 = bn * BN;
+  const int lane = threadIdx.x & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wave_m = wid % WAVES_M, wave_n = wid / WAVES_M;
+  const int fr = lane & 15, fk = lane >> 4;
+  floatx4 acc[I][J];
+#pragma unroll
+  for (int i = 0; i < I; ++i)
+#pragma unroll
+    for (int j = 0; j < J; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+  const unsigned lds0 = (unsigned)(uintptr_t)smem;
+  unsigned ga[LA], gw[LW];                                   // a wave copies pieces wid, WAVES + wid, ... of 8 rows
+#pragma unroll
+  for (int q = 0; q < LA; ++q) {
+    const int r = (q * WAVES + wid) * 8 + (lane >> 3);
+    ga[q] = ((unsigned)min(m0 + r, M - 1) * (unsigned)lda + ((lane & 7) ^ ((r >> 1) & 7)) * 8) * 2u;
+  }
+#pragma unroll
+  for (int q = 0; q < LW; ++q) {
+    const int r = (q * WAVES + wid) * 8 + (lane >> 3);
+    gw[q] = ((unsigned)min(n0 + r, N - 1) * (unsigned)ldw + ((lane & 7) ^ ((r >> 1) & 7)) * 8) * 2u;
+  }
+  const int nkt = K / DMA_BK;
+  auto copy = [&](int kt, int st) {                          // (past the last tile: that one again, never read)
+    const int k = min(kt, nkt - 1) * DMA_BK;
+    const unsigned base = lds0 + st * ST + wid * 1024;
+#pragma unroll
+    for (int q = 0; q < LW; ++q) dma16(W + k, gw[q], __builtin_amdgcn_readfirstlane(base + BM * ROW + q * (WAVES * 1024)));
+#pragma unroll
+    for (int q = 0; q < LA; ++q) dma16(A + k, ga[q], __builtin_amdgcn_readfirstlane(base + q * (WAVES * 1024)));
+  };
+  const int sw = (fr >> 1) & 7;
+#pragma unroll
+  for (int t = 0; t < STAGES - 1; ++t) copy(t, t);
+  int st = 0;
+  for (int kt = 0; kt < nkt; ++kt) {
+    // tile kt has landed for this wave, and behind the barrier for all; the stage of tile kt - 1, whose fragments every
+    // wave has back by then (its products used them), takes tile kt + STAGES - 1
+    dma_wait<(STAGES - 2) * (LA + LW)>();
+    dma_meet();
+    copy(kt + STAGES - 1, st == 0 ? STAGES - 1 : st - 1);
+    const unsigned char* s = smem + st * ST;
+    bf16x8 fa[2][I], fw[2][J];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int pos = ((4 * h + fk) ^ sw) * 16;
+#pragma unroll
+      for (int i = 0; i < I; ++i) fa[h][i] = *reinterpret_cast<const bf16x8*>(s + (wave_m * TT::ROWS + i * 16 + fr) * ROW + pos);
+#pragma unroll
+      for (int j = 0; j < J; ++j)
+        fw[h][j] = *reinterpret_cast<const bf16x8*>(s + (BM + (TT::first(wave_n) + j * TT::STEP) * 16 + fr) * ROW + pos);
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int i = 0; i < I; ++i)
+#pragma unroll
+        for (int j = 0; j < J; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[h][j], fa[h][i], acc[i][j], 0, 0, 0);
+    st = st == STAGES - 1 ? 0 : st + 1;
+  }
+  dma_wait<0>();
+  dma_meet();
+  dma_epilogue<TT>(acc, smem + wid * TT::OWN, bias, C, ldc, M, N, epi, m0 + wave_m * TT::ROWS, n0, wave_n, lane);
+}
+
+template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, bool GROUPED>
+int launch_tile_step(const bf16* A, int lda, const bf16* W, int ldw, const float* bias, void* C, int ldc, int M, int N, int K, int epi,
+                     hipStream_t stream, int splits, int k_per_split, const RowGroup* groups, int n_groups) {
+  using TT = StepTile<BM, BN, WAVES_M, WAVES_N>;
+  auto kern = tile_step_kernel<BM, BN, WAVES_M, WAVES_N, STAGES, GROUPED>;
+  static bool configured = false;
+  if (!configured) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                             TT::template lds<STAGES>());
+    if (e != hipSuccess) return (int)e;
+    configured = true;
+  }
+  const int tiles_m = GROUPED ? n_groups : (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
+  kern<<<dim3(tiles_m * tiles_n, splits), 64 * TT::WAVES, TT::template lds<STAGES>(), stream>>>(
+      A, lda, W, ldw, bias, C, ldc, M, N, K, epi, tiles_m, tiles_m * tiles_n >= 16, k_per_split, groups);
+  return mf_launch_status();
 }
 
 template <int BM, int BN, int STAGES, bool GROUPED>
@@ -2202,32 +2341,33 @@ int launch_panel(const bf16* A, int lda, const bf16* W, const bf16* Wt, int ldw,
 // ---- which tile kernel a product of many rows takes
 // Variants: 2: 128 x 128 tiles through registers (two blocks a CU), 3: 64 x 64, 9: 256 x 256 through
 // registers, and the direct-to-LDS kernel (aligned operands, K in 64s): 12 the largest tiles (256 x 256; SwiGLU products
-// 256 x 192 where their rounds are the shorter), 15 256 x 192 (no SwiGLU), 13 the smaller ones (256 x 128, 128 x 256 or
-// 128 x 128).  With `splits` > 1 the K dimension is cut over blocks (variants 12 and 2, the latter with the smaller
+// 256 x 192 where their rounds are the shorter), 15 256 x 192 (no SwiGLU), 13 the smaller ones (256 x 128, 128 x 256,
+// 128 x 128 or 64 x 64).  With `splits` > 1 the K dimension is cut over blocks (variants 12 and 2, the latter with the smaller
 // direct-to-LDS tiles where the operands allow) and skinny_reduce_kernel adds the parts.
 struct TilePlan { int variant, splits, k_per_split; double us; };
 
-// The direct-to-LDS kernel's tiles: microseconds a k tile of 64 with every CU busy (random values, 2,048 rows at the 7B
-// widths; a chip that is not full runs up to 0.7 of it) and how many of them a round adds for its start and end.
-struct DmaForm { int bm, bn; double step_us; };
-enum { FORM_256, FORM_192, FORM_128, FORM_128T, FORM_SMALL, N_FORMS };
-constexpr DmaForm DMA_FORMS[N_FORMS] = {{256, 256, 1.36}, {256, 192, 1.08}, {256, 128, 0.84}, {128, 256, 0.84}, {128, 128, 0.58}};
+// The direct-to-LDS kernels' tiles: blocks a CU, microseconds a k tile of 64 with every CU busy (random values, 2,048 rows
+// at the 7B widths), and what a chip that is nearly empty takes of it (the smaller tiles are their own chains of waits).
+struct DmaForm { int bm, bn, per_cu; double step_us, low; };
+enum { FORM_256, FORM_192, FORM_128, FORM_128T, FORM_SMALL, FORM_TINY, N_FORMS };
+constexpr DmaForm DMA_FORMS[N_FORMS] = {{256, 256, 1, 1.36, 0.7}, {256, 192, 1, 1.08, 0.7}, {256, 128, 1, 0.84, 0.9},
+                                        {128, 256, 1, 0.84, 0.9}, {128, 128, 1, 0.62, 0.9}, {64, 64, 2, 0.56, 0.55}};
 constexpr double ROUND_US = 5.;
 
 // The estimate behind the choice: a kernel's tiles go over its slots (blocks that fit the chip at
 // once) in rounds; a round takes the product's k tiles of 64 times the variant's time per k tile, a last round that is
 // not full somewhat less (fewer blocks pull on the fabric and on the power); a start, the epilogue's traffic, and for a K
 // split the parts' way to memory and back come on top.
-double rounds_us(long blocks, long slots, double step_us, long nkt, double round_us) {
+double rounds_us(long blocks, long slots, double step_us, long nkt, double round_us, double low = 0.7) {
   const long full = blocks / slots;
   const double fill = (double)(blocks % slots) / (double)slots;
-  return ((double)nkt * step_us) * ((double)full + (fill > 0. ? 0.7 + 0.3 * fill : 0.)) + round_us * (double)(full + (fill > 0.));
+  return ((double)nkt * step_us) * ((double)full + (fill > 0. ? low + (1. - low) * fill : 0.)) + round_us * (double)(full + (fill > 0.));
 }
 
 double form_us(int form, int M, int N, long nkt, int splits, long cu) {
   const DmaForm& f = DMA_FORMS[form];
   const long tiles = (long)((M + f.bm - 1) / f.bm) * ((N + f.bn - 1) / f.bn);
-  return rounds_us(tiles * splits, cu, f.step_us, nkt, ROUND_US);
+  return rounds_us(tiles * splits, cu * f.per_cu, f.step_us, nkt, ROUND_US, f.low);
 }
 
 // the cheapest of the forms first .. last
@@ -2244,7 +2384,7 @@ int dma_form(int variant, int M, int N, int epi, long nkt, int splits, long cu) 
     case 12: return epi == EPI_SWIGLU && splits == 1 ? best_form(FORM_256, FORM_192, M, N, nkt, 1, cu) : FORM_256;
     case 15: return FORM_192;
   }
-  return best_form(FORM_128, FORM_SMALL, M, N, nkt, splits, cu);
+  return best_form(FORM_128, FORM_TINY, M, N, nkt, splits, cu);
 }
 
 int launch_form(int form, const bf16* A, int lda, const bf16* W, int ldw, const float* bias, void* C, int ldc, int M, int N, int K,
@@ -2255,7 +2395,9 @@ int launch_form(int form, const bf16* A, int lda, const bf16* W, int ldw, const 
     case FORM_128: return launch_tile_dma<256, 128, 3>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi, stream, splits, k_per_split);
     case FORM_128T: return launch_tile_dma<128, 256, 3>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi, stream, splits, k_per_split);
   }
-  return launch_tile_dma<128, 128, 4>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi, stream, splits, k_per_split);
+  return form == FORM_SMALL
+             ? launch_tile_step<128, 128, 2, 4, 3, false>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi, stream, splits, k_per_split, nullptr, 0)
+             : launch_tile_step<64, 64, 2, 2, 4, false>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi, stream, splits, k_per_split, nullptr, 0);
 }
 
 TilePlan plan_tiles(int M, int N, int K, bool dma_ok, int epi, int n_cu) {
@@ -2351,7 +2493,7 @@ MF_API int mf_gemm_bf16_grouped(const void* A, const void* W, float* C, const in
   const RowGroup* g = (const RowGroup*)groups;
   switch (variant) {
     case 2:
-      return K % DMA_BK == 0 ? launch_grouped_dma<128, 128, 4>(a, K, w, K, C, N, g, n_groups, N, K, stream)
+      return K % DMA_BK == 0 ? launch_tile_step<128, 128, 2, 4, 3, true>(a, K, w, K, nullptr, C, N, 0, N, K, EPI_F32, stream, 1, 0, g, n_groups)
                              : launch_grouped_tile<128, 128, 64, 64, 64>(a, K, w, K, C, N, g, n_groups, N, K, stream);
     case 12: return launch_grouped_dma<256, 256, 2>(a, K, w, K, C, N, g, n_groups, N, K, stream);
     case 13: return launch_grouped_dma<256, 128, 3>(a, K, w, K, C, N, g, n_groups, N, K, stream);

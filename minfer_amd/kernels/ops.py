@@ -1882,7 +1882,7 @@ def linear_norm_out(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.
 
 # variants of the grouped product: (tile rows, tile columns, blocks a CU, microseconds a k tile of 64 with every CU
 # busy), as the plan of the single product has them
-GROUPED_TILES = {12: (256, 256, 1, 1.75), 13: (256, 128, 1, 1.0), 2: (128, 128, 2, 1.45)}
+GROUPED_TILES = {12: (256, 256, 1, 1.36), 13: (256, 128, 1, 0.84), 2: (128, 128, 1, 0.62)}
 
 
 def grouped_takes(dtype, n: int, k: int) -> bool:

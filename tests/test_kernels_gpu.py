@@ -745,16 +745,17 @@ def test_gemm_bf16_swiglu(ops, variant, m, nf, k):
 # its stages of k tiles), rows and columns that leave remainders, row lengths without 16-byte stores
 @pytest.mark.parametrize("variant,m,n,k", [(13, 700, 11000, 64), (13, 511, 16001, 192), (13, 130, 16390, 256),     # 256 x 128
                                            (13, 600, 22016, 128), (13, 513, 9000, 320), (13, 1025, 8201, 64),      # 128 x 256
-                                           (13, 129, 101, 64), (13, 127, 333, 320), (13, 65, 1002, 576),           # 128 x 128
+                                           (13, 257, 8200, 192), (13, 300, 6403, 64), (13, 257, 8201, 320),        # 128 x 128
+                                           (13, 129, 101, 64), (13, 127, 333, 320), (13, 65, 1002, 576),           # 64 x 64
                                            (15, 257, 193, 64), (15, 300, 579, 192),                                # 256 x 192
                                            (12, 255, 259, 64), (12, 513, 510, 192)])                               # 256 x 256
 def test_gemm_bf16_tile_forms(ops, variant, m, n, k):
     test_gemm_bf16(ops, variant, m, n, k)
 
 
-# SwiGLU: 256 x 256 (512 rows and 16,380 outputs fill the chip once), 256 x 192, 256 x 128, 128 x 256, 128 x 128
+# SwiGLU: 256 x 256 (512 rows and 16,380 outputs fill the chip once), 256 x 192, 256 x 128, 128 x 256, 128 x 128, 64 x 64
 @pytest.mark.parametrize("variant,m,nf,k", [(12, 500, 16380, 128), (12, 257, 95, 192), (12, 300, 201, 64), (13, 700, 5500, 64),
-                                            (13, 600, 11008, 128), (13, 129, 97, 320)])
+                                            (13, 600, 11008, 128), (13, 257, 4101, 192), (13, 129, 97, 320)])
 def test_gemm_bf16_swiglu_tile_forms(ops, variant, m, nf, k):
     test_gemm_bf16_swiglu(ops, variant, m, nf, k)
 
