@@ -689,7 +689,7 @@ __global__ __launch_bounds__(512, 2) void tile_dma_kernel(const bf16* __restrict
 // ---- the smaller tiles: one barrier a k tile
 // 128 x 128 on 8 waves and 64 x 64 on 4, for products whose larger tiles would leave most of the chip idle: a block's time
 // is then its own chain of k tiles, whatever the others do, and a k tile's chain is what is kept short: wait for the copies
-// of one k tile, meet, set out the copies STAGES - 1 tiles on, read every fragment, multiply.  (The quarter products of
+// of the next k tile, meet, set out the copies STAGES - 1 tiles on, read the next tile's fragments, multiply this one's.  (The quarter products of
 // `tile_dma_kernel` meet eight times a k tile, which 128 x 128 cannot fill: 203 rows against 9,728 of 896 15.5 us so, 12.6
 // here; 2,048 x 2,048 x 2,048 27.2 and 23.3.  At 256 x 128 the two are level.)  64 x 64: 203 rows against 1,152 of 896 (the
 // narrowest model's q|k|v) 11.6 us as 128 x 128, 6.4 so.
@@ -709,13 +709,17 @@ struct StepTile {
   static_assert(J == 2 && I % 2 == 0 && BM % (8 * WAVES) == 0 && BN % (8 * WAVES) == 0, "pairs of blocks, whole copies per wave");
 };
 
-template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, bool GROUPED = false>
+// SCALED: the rows' sums are multiplied by 1 / sqrt(mean + eps) of the row, `in_parts` partial sums of squares of which stand
+// in in_ssq [M][in_parts] (FusedNorm::in_*; one launch, K whole).
+template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, bool GROUPED = false, bool SCALED = false>
 __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void tile_step_kernel(const bf16* __restrict__ A, int lda,
                                                        const bf16* __restrict__ W, int ldw,
                                                        const float* __restrict__ bias, void* __restrict__ C,
                                                        int ldc, int M, int N, int K, int epi, int tiles_m,
                                                        int xcd_remap, int k_per_split,
-                                                       const RowGroup* __restrict__ groups = nullptr) {
+                                                       const RowGroup* __restrict__ groups = nullptr,
+                                                       const float* __restrict__ in_ssq = nullptr, int in_parts = 0,
+                                                       float in_eps = 0.f) {
   using TT = StepTile<BM, BN, WAVES_M, WAVES_N>;
   constexpr int ROW = DMA_BK * 2, ST = (BM + BN) * ROW, WAVES = TT::WAVES, I = TT::I, J = TT::J, LA = TT::LA, LW = TT::LW;
   if (k_per_split > 0) {                                     // as in tile_dma_kernel
@@ -774,44 +778,97 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void tile_step_kernel(const
     for (int q = 0; q < LA; ++q) dma16(A + k, ga[q], __builtin_amdgcn_readfirstlane(base + q * (WAVES * 1024)));
   };
   const int sw = (fr >> 1) & 7;
+  // the rows' partial sums are asked for in front of the first copies and added up behind them (what waits for the sums then
+  // waits for the first k tiles, which the loop needs anyway)
+  constexpr int PART_LOADS = 4;
+  float fac[I], part0[I][PART_LOADS];
+  if constexpr (SCALED) {
+#pragma unroll
+    for (int i = 0; i < I; ++i)
+#pragma unroll
+      for (int p = 0; p < PART_LOADS; ++p)
+        part0[i][p] = in_ssq[(size_t)min(m0 + wave_m * TT::ROWS + i * 16 + fr, M - 1) * in_parts + min(p, in_parts - 1)];
+    __builtin_amdgcn_sched_barrier(0);
+  }
 #pragma unroll
   for (int t = 0; t < STAGES - 1; ++t) copy(t, t);
-  int st = 0;
-  for (int kt = 0; kt < nkt; ++kt) {
-    // tile kt has landed for this wave, and behind the barrier for all; the stage of tile kt - 1, whose fragments every
-    // wave has back by then (its products used them), takes tile kt + STAGES - 1
-    dma_wait<(STAGES - 2) * (LA + LW)>();
-    dma_meet();
-    copy(kt + STAGES - 1, st == 0 ? STAGES - 1 : st - 1);
+  if constexpr (SCALED) {
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < I; ++i) {
+      const float* p = in_ssq + (size_t)min(m0 + wave_m * TT::ROWS + i * 16 + fr, M - 1) * in_parts;
+      float t = 0.f;
+#pragma unroll
+      for (int q = 0; q < PART_LOADS; ++q) t += q < in_parts ? part0[i][q] : 0.f;
+      for (int q = PART_LOADS; q < in_parts; ++q) t += p[q];
+      fac[i] = 1.0f / sqrtf(t / (float)K + in_eps);
+    }
+  }
+  bf16x8 fa[2][2][I], fw[2][2][J];                           // [set][k-step][block]
+  auto read = [&](int st, auto SET) {
+    constexpr int set = decltype(SET)::value;
     const unsigned char* s = smem + st * ST;
-    bf16x8 fa[2][I], fw[2][J];
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       const int pos = ((4 * h + fk) ^ sw) * 16;
 #pragma unroll
-      for (int i = 0; i < I; ++i) fa[h][i] = *reinterpret_cast<const bf16x8*>(s + (wave_m * TT::ROWS + i * 16 + fr) * ROW + pos);
+      for (int i = 0; i < I; ++i) fa[set][h][i] = *reinterpret_cast<const bf16x8*>(s + (wave_m * TT::ROWS + i * 16 + fr) * ROW + pos);
 #pragma unroll
       for (int j = 0; j < J; ++j)
-        fw[h][j] = *reinterpret_cast<const bf16x8*>(s + (BM + (TT::first(wave_n) + j * TT::STEP) * 16 + fr) * ROW + pos);
+        fw[set][h][j] = *reinterpret_cast<const bf16x8*>(s + (BM + (TT::first(wave_n) + j * TT::STEP) * 16 + fr) * ROW + pos);
     }
+  };
+  auto multiply = [&](auto SET) {
+    constexpr int set = decltype(SET)::value;
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
       for (int i = 0; i < I; ++i)
 #pragma unroll
-        for (int j = 0; j < J; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[h][j], fa[h][i], acc[i][j], 0, 0, 0);
+        for (int j = 0; j < J; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[set][h][j], fa[set][h][i], acc[i][j], 0, 0, 0);
+  };
+  using S0 = std::integral_constant<int, 0>;
+  using S1 = std::integral_constant<int, 1>;
+  constexpr int L = LA + LW;
+  dma_wait<(STAGES - 2) * L>();
+  dma_meet();
+  read(0, S0{});
+  int st = 0;                                                // of tile kt
+  // one k tile: its fragments are in set NOW; those of the next one are read into the other set under its products
+  auto pass = [&](int kt, auto NOW, auto OTHER) {
+    // tile kt + 1 has landed for this wave, and behind the barrier for all; the stage of tile kt - 1, whose fragments every
+    // wave's products have used by then, takes tile kt + STAGES - 1
+    dma_wait<(STAGES - 3) * L>();
+    dma_meet();
+    copy(kt + STAGES - 1, st == 0 ? STAGES - 1 : st - 1);
     st = st == STAGES - 1 ? 0 : st + 1;
+    read(st, OTHER);                                         // (behind the last tile: that one again, never used)
+    multiply(NOW);
+  };
+  int kt = 0;
+  for (; kt + 1 < nkt; kt += 2) {
+    pass(kt, S0{}, S1{});
+    pass(kt + 1, S1{}, S0{});
   }
+  if (kt < nkt) multiply(S0{});
   dma_wait<0>();
   dma_meet();
+  if constexpr (SCALED) {
+#pragma unroll
+    for (int i = 0; i < I; ++i)
+#pragma unroll
+      for (int j = 0; j < J; ++j) acc[i][j] *= fac[i];
+  }
   dma_epilogue<TT>(acc, smem + wid * TT::OWN, bias, C, ldc, M, N, epi, m0 + wave_m * TT::ROWS, n0, wave_n, lane);
 }
 
-template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, bool GROUPED>
+template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, bool GROUPED, bool SCALED = false>
 int launch_tile_step(const bf16* A, int lda, const bf16* W, int ldw, const float* bias, void* C, int ldc, int M, int N, int K, int epi,
-                     hipStream_t stream, int splits, int k_per_split, const RowGroup* groups, int n_groups) {
+                     hipStream_t stream, int splits, int k_per_split, const RowGroup* groups, int n_groups,
+                     const float* in_ssq = nullptr, int in_parts = 0, float in_eps = 0.f) {
   using TT = StepTile<BM, BN, WAVES_M, WAVES_N>;
-  auto kern = tile_step_kernel<BM, BN, WAVES_M, WAVES_N, STAGES, GROUPED>;
+  auto kern = tile_step_kernel<BM, BN, WAVES_M, WAVES_N, STAGES, GROUPED, SCALED>;
   static bool configured = false;
   if (!configured) {
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -821,8 +878,16 @@ int launch_tile_step(const bf16* A, int lda, const bf16* W, int ldw, const float
   }
   const int tiles_m = GROUPED ? n_groups : (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
   kern<<<dim3(tiles_m * tiles_n, splits), 64 * TT::WAVES, TT::template lds<STAGES>(), stream>>>(
-      A, lda, W, ldw, bias, C, ldc, M, N, K, epi, tiles_m, tiles_m * tiles_n >= 16, k_per_split, groups);
+      A, lda, W, ldw, bias, C, ldc, M, N, K, epi, tiles_m, tiles_m * tiles_n >= 16, k_per_split, groups, in_ssq, in_parts, in_eps);
   return mf_launch_status();
+}
+
+// 64 x 64: five stages, so that two blocks fit a CU (ten for blocks that have a CU to themselves: level)
+template <bool SCALED>
+int launch_tile64(const bf16* A, int lda, const bf16* W, int ldw, const float* bias, void* C, int ldc, int M, int N, int K, int epi,
+                  hipStream_t stream, int splits, int k_per_split, const float* in_ssq = nullptr, int in_parts = 0, float in_eps = 0.f) {
+  return launch_tile_step<64, 64, 2, 2, 5, false, SCALED>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi, stream, splits, k_per_split,
+                                                          nullptr, 0, in_ssq, in_parts, in_eps);
 }
 
 template <int BM, int BN, int STAGES, bool GROUPED>
@@ -2396,8 +2461,8 @@ int launch_form(int form, const bf16* A, int lda, const bf16* W, int ldw, const 
     case FORM_128T: return launch_tile_dma<128, 256, 3>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi, stream, splits, k_per_split);
   }
   return form == FORM_SMALL
-             ? launch_tile_step<128, 128, 2, 4, 3, false>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi, stream, splits, k_per_split, nullptr, 0)
-             : launch_tile_step<64, 64, 2, 2, 4, false>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi, stream, splits, k_per_split, nullptr, 0);
+             ? launch_tile_step<128, 128, 2, 4, 4, false>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi, stream, splits, k_per_split, nullptr, 0)
+             : launch_tile64<false>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi, stream, splits, k_per_split);
 }
 
 TilePlan plan_tiles(int M, int N, int K, bool dma_ok, int epi, int n_cu) {
@@ -2455,8 +2520,16 @@ TilePlan plan_tiles(int M, int N, int K, bool dma_ok, int epi, int n_cu) {
 // Which kernel a product of at most 64 rows takes.
 enum SkinnyChoice {
   SK_STATIONARY, SK_ROLLING, SK_GUARDED_PAIR, SK_GUARDED_4X2, SK_GUARDED_8X2, SK_GUARDED_8X1, SK_PANEL, SK_RING,
-  SK_STAGED
+  SK_STAGED, SK_TILE
 };
+
+// 17 to 64 rows against a short K: a tile of 64 x 64 over the whole of K, with the norm's factors, the bias and SwiGLU in its
+// epilogue, where the K-split kernels need a second one (32 to 40 rows, K-split and added / one tile kernel: gate|up 9,728 x 896
+// 15.0 / 9.0 us, 17,920 x 1,536 19.9 / 19.2, 22,016 x 2,048 28.3 / 26.6; q|k|v 1,152 x 896 11.6 / 9.0, 2,048 x 1,536 level).
+// At most two tiles a CU, all at once; fewer than eight tiles are a launch whichever kernel it is.
+bool tile64_takes(int M, int N, int K, bool aligned, int epi, int n_cu) {
+  return M > 16 && aligned && K % DMA_BK == 0 && N >= 512 && (N + 63) / 64 <= 2 * n_cu && K <= (epi == EPI_SWIGLU ? 2048 : 1024);
+}
 
 SkinnyChoice skinny_choice(int M, int N, int K, bool aligned, int epi, int splits, int k_per_split, int n_cu) {
   if (M <= 16 && splits == 1) {
@@ -2474,6 +2547,7 @@ SkinnyChoice skinny_choice(int M, int N, int K, bool aligned, int epi, int split
     return SK_GUARDED_8X1;
   }
   if (M > 16 && panel_takes(M, N, K, aligned, epi, n_cu)) return SK_PANEL;
+  if (tile64_takes(M, N, K, aligned, epi, n_cu)) return SK_TILE;
   return ring_takes(aligned, K, splits, k_per_split) ? SK_RING : SK_STAGED;
 }
 
@@ -2493,7 +2567,7 @@ MF_API int mf_gemm_bf16_grouped(const void* A, const void* W, float* C, const in
   const RowGroup* g = (const RowGroup*)groups;
   switch (variant) {
     case 2:
-      return K % DMA_BK == 0 ? launch_tile_step<128, 128, 2, 4, 3, true>(a, K, w, K, nullptr, C, N, 0, N, K, EPI_F32, stream, 1, 0, g, n_groups)
+      return K % DMA_BK == 0 ? launch_tile_step<128, 128, 2, 4, 4, true>(a, K, w, K, nullptr, C, N, 0, N, K, EPI_F32, stream, 1, 0, g, n_groups)
                              : launch_grouped_tile<128, 128, 64, 64, 64>(a, K, w, K, C, N, g, n_groups, N, K, stream);
     case 12: return launch_grouped_dma<256, 256, 2>(a, K, w, K, C, N, g, n_groups, N, K, stream);
     case 13: return launch_grouped_dma<256, 128, 3>(a, K, w, K, C, N, g, n_groups, N, K, stream);
@@ -2648,6 +2722,12 @@ static int skinny_product(const void* A, int lda, const void* W, const void* Wt,
     case SK_GUARDED_8X2: return launch_skinny16<8, 2, 4>(a, lda, w, ldw, bias, C, ldc, M, N, K, epi, vec_ok, stream);
     case SK_GUARDED_8X1: return launch_skinny16<8, 1, 8>(a, lda, w, ldw, bias, C, ldc, M, N, K, epi, vec_ok, stream);
     case SK_PANEL: return launch_panel(a, lda, w, wt, ldw, bias, C, ldc, M, N, K, epi, fused, stream);
+    case SK_TILE:
+      // (the next norm's sums of squares come from the K-split kernels' second one; operands beyond 4 GB go to them as well)
+      if (fused.out_g || (size_t)N * ldw * 2 >= (1ull << 32)) break;
+      return fused.in_ssq ? launch_tile64<true>(a, lda, w, ldw, bias, C, ldc, M, N, K, epi, stream, 1, 0, fused.in_ssq, fused.in_parts,
+                                                fused.in_eps)
+                          : launch_tile64<false>(a, lda, w, ldw, bias, C, ldc, M, N, K, epi, stream, 1, 0);
     default: break;
   }
   switch ((M + 15) / 16) {
@@ -2739,6 +2819,7 @@ MF_API int mf_gemm_bf16_plan(int M, int N, int K, int aligned, int epi, int spli
       case SK_PANEL: what = "panel_kernel"; break;
       case SK_RING: what = "skinny_ring_kernel"; break;
       case SK_STAGED: what = "skinny_kernel"; break;
+      case SK_TILE: what = "tile_step_kernel<64,64>"; break;
     }
   } else {
     const bool dma_ok = aligned && K % DMA_BK == 0 && (size_t)M * K * 2 < (1ull << 32) && (size_t)N * K * 2 < (1ull << 32);

@@ -947,6 +947,15 @@ def test_product_takes_a_prepared_norm(ops, m, n, k, swiglu):
     close(acc, ref - b.double() + base.double(), 2e-5 * math.sqrt(k), 1e-5)
 
 
+# ... and by 64 x 64 tiles over the whole of a short K (one to eight partial sums a row, rows and columns that leave remainders)
+@pytest.mark.parametrize("m,n,k,swiglu", [(17, 1152, 896, False), (40, 1001, 1024, False), (64, 9728, 896, True), (33, 17920, 1536, True),
+                                          (50, 22016, 2048, True), (64, 515, 64, False), (31, 2000, 192, True)])
+def test_product_takes_a_prepared_norm_in_tiles(ops, m, n, k, swiglu):
+    n_run = (n + 63) // 64 * 64 if swiglu else n
+    assert ops.plan_linear(m, n_run, k, swiglu=swiglu)["kernel"] == "tile_step_kernel<64,64>"
+    test_product_takes_a_prepared_norm(ops, m, n, k, swiglu)
+
+
 def test_fused_norm_declines_where_no_kernel_has_a_place_for_it(ops):
     """A K that is not split at 17 rows and more, a shape of few rows that the register-resident
     kernel does not take: nothing is written, the caller is told."""
