@@ -48,24 +48,29 @@ struct RopeArgs {
   int write_kv;
 };
 
-// 8 rotated elements d .. d + 7 of one head (src, hd floats) at position pos
+// 8 rotated elements d .. d + 7 of one head (src, hd floats) at position pos: what they need, asked for, and their values
+struct Rot8 { float4 a0, a1, b0, b1, c0, c1, s0, s1; };
 template <int HD>
-__device__ __forceinline__ bf16x8 rotated8(const float* __restrict__ src, const float* __restrict__ cs,
-                                           const float* __restrict__ sn, int pos, int d) {
+__device__ __forceinline__ void load8(Rot8& r, const float* __restrict__ src, const float* __restrict__ cs,
+                                      const float* __restrict__ sn, int pos, int d) {
   constexpr int HALF = HD / 2;
-  const bool upper = d >= HALF;
-  const int i = upper ? d - HALF : d;               // index into the table and of the lower partner
-  const float4 a0 = *reinterpret_cast<const float4*>(src + i), a1 = *reinterpret_cast<const float4*>(src + i + 4);
-  const float4 b0 = *reinterpret_cast<const float4*>(src + i + HALF);
-  const float4 b1 = *reinterpret_cast<const float4*>(src + i + HALF + 4);
-  const float4 c0 = *reinterpret_cast<const float4*>(cs + (size_t)pos * HALF + i);
-  const float4 c1 = *reinterpret_cast<const float4*>(cs + (size_t)pos * HALF + i + 4);
-  const float4 s0 = *reinterpret_cast<const float4*>(sn + (size_t)pos * HALF + i);
-  const float4 s1 = *reinterpret_cast<const float4*>(sn + (size_t)pos * HALF + i + 4);
-  const float x0[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
-  const float x1[8] = {b0.x, b0.y, b0.z, b0.w, b1.x, b1.y, b1.z, b1.w};
-  const float c[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
-  const float sv[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
+  const int i = d >= HALF ? d - HALF : d;           // index into the table and of the lower partner
+  r.a0 = *reinterpret_cast<const float4*>(src + i);
+  r.a1 = *reinterpret_cast<const float4*>(src + i + 4);
+  r.b0 = *reinterpret_cast<const float4*>(src + i + HALF);
+  r.b1 = *reinterpret_cast<const float4*>(src + i + HALF + 4);
+  r.c0 = *reinterpret_cast<const float4*>(cs + (size_t)pos * HALF + i);
+  r.c1 = *reinterpret_cast<const float4*>(cs + (size_t)pos * HALF + i + 4);
+  r.s0 = *reinterpret_cast<const float4*>(sn + (size_t)pos * HALF + i);
+  r.s1 = *reinterpret_cast<const float4*>(sn + (size_t)pos * HALF + i + 4);
+}
+template <int HD>
+__device__ __forceinline__ bf16x8 rotated8(const Rot8& o, int d) {
+  const bool upper = d >= HD / 2;
+  const float x0[8] = {o.a0.x, o.a0.y, o.a0.z, o.a0.w, o.a1.x, o.a1.y, o.a1.z, o.a1.w};
+  const float x1[8] = {o.b0.x, o.b0.y, o.b0.z, o.b0.w, o.b1.x, o.b1.y, o.b1.z, o.b1.w};
+  const float c[8] = {o.c0.x, o.c0.y, o.c0.z, o.c0.w, o.c1.x, o.c1.y, o.c1.z, o.c1.w};
+  const float sv[8] = {o.s0.x, o.s0.y, o.s0.z, o.s0.w, o.s1.x, o.s1.y, o.s1.z, o.s1.w};
   bf16x8 r;
 #pragma unroll
   for (int e = 0; e < 8; ++e) r[e] = (bf16)(upper ? x0[e] * sv[e] + x1[e] * c[e] : x0[e] * c[e] - x1[e] * sv[e]);
@@ -168,71 +173,33 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(
     return;
   }
 
-  // B operand of the first product: row = head r16, 8 elements of head_dim at 32 ks + 8 q4.
-  // ROPE: the block rotates its 16 heads once, one 8-element chunk per thread, into LDS.
-  __shared__ __attribute__((aligned(16))) bf16 sm_q[ROPE ? 16 * KS * 32 : 8];
-  if constexpr (ROPE) {
-    for (int c = threadIdx.x; c < 16 * KS * 4; c += 256) {
-      const int head = c / (KS * 4), d = (c % (KS * 4)) * 8;
-      bf16x8 q8 = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
-      if (head < gcount && d < HD)
-        q8 = rotated8<HD>(rope.qkv + ((size_t)t * (nh + 2 * nk) + h0 + head) * HD, rope.cs, rope.sn, p, d);
-      *reinterpret_cast<bf16x8*>(&sm_q[head * KS * 32 + d]) = q8;
-    }
-  }
-  // ROPE: the token's own key and value, for the blocks whose split ends at its position:
-  // rotated (k) and rounded once here, kept in LDS until the step that holds position p.
-  // Key p is row `krow + 4 a` of tile a in its step for exactly one a, in the four lanes of one
-  // r16; value p is element p % 8 of the lanes with q4 = (p % 32) / 8.
+  // ROPE: the block rotates its 16 heads once, one 8-element chunk per thread, into LDS, and the blocks whose split ends at
+  // the token's position its own key and value: rotated (k) and rounded once, kept in LDS until the step that holds position
+  // p.  Key p is row `krow + 4 a` of tile a in its step for exactly one a, in the four lanes of one r16; value p is element
+  // p % 8 of the lanes with q4 = (p % 32) / 8.
+  // All that is asked for before the first product is asked for at once (loads come back in order, so the rotation's, from
+  // the chip's caches, go first): the kernel is a chain of such trips at short lengths, and with the keys asked for behind the
+  // rotation's barrier a decode step of the 0.5B widths took 0.3 us a layer longer (step 810 -> 803 us).
   const int krow = 8 * (r16 >> 2) + (r16 & 3);
   const bool own_split = ROPE && rope.write_kv && j_end == p + 1 && j_begin <= p;
   const int po = p % STEP;
   const int own_a = (po - krow) >> 2;                      // 0 or 1 where this lane holds key p
   const bool own_k = own_split && (po - krow == 0 || po - krow == 4);
   const bool own_v = own_split && q4 == (po >> 3);
+  __shared__ __attribute__((aligned(16))) bf16 sm_q[ROPE ? 16 * KS * 32 : 8];
   __shared__ __attribute__((aligned(16))) bf16 sm_k[ROPE ? KS * 32 : 8];
   __shared__ bf16 sm_v[ROPE ? HD : 8];
-  if constexpr (ROPE) {
-    if (own_split) {
-      const int tid = threadIdx.x;
-      const float* row = rope.qkv + (size_t)t * (nh + 2 * nk) * HD;
-      const bool store = g0 == 0;                          // one block per kv head fills the cache
-      const int page = pt[p / MF_PAGE];
-      if (tid < KS * 4) {
-        bf16x8 k8 = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
-        if (tid * 8 < HD) {
-          k8 = rotated8<HD>(row + (size_t)(nh + hk) * HD, rope.cs, rope.sn, p, tid * 8);
-          if (store)
-            *reinterpret_cast<bf16x8*>(kc + (((size_t)page * nk + hk) * MF_PAGE + p % MF_PAGE) * HD + tid * 8) = k8;
-        }
-        *reinterpret_cast<bf16x8*>(&sm_k[tid * 8]) = k8;
-      }
-      for (int d = tid; d < HD; d += 256) {
-        const bf16 v = (bf16)row[(size_t)(nh + nk + hk) * HD + d];
-        sm_v[d] = v;
-        if (store)
-          vt[((((size_t)page * nk + hk) * 2 + (p % MF_PAGE) / STEP) * HD + d) * STEP + p % STEP] = v;
-      }
-    }
-    __syncthreads();
-  }
-  bf16x8 qf[KS];
-#pragma unroll
-  for (int ks = 0; ks < KS; ++ks) {
-    const int d = ks * 32 + q4 * 8;
-    if constexpr (ROPE) {
-      qf[ks] = *reinterpret_cast<const bf16x8*>(&sm_q[r16 * KS * 32 + d]);
-    } else {
-      qf[ks] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
-      if (r16 < gcount && d < HD) qf[ks] = *reinterpret_cast<const bf16x8*>(q + ((size_t)t * nh + h0 + r16) * HD + d);
-    }
-  }
-
-  floatx4 oacc[CT];                       // O^T: head r16, columns 16 c + 4 q4 + r
-#pragma unroll
-  for (int c = 0; c < CT; ++c) oacc[c] = floatx4{0.f, 0.f, 0.f, 0.f};
-  float m_run = -INFINITY, l_run = 0.f;   // of head r16 (the same in the four lanes that share it)
-
+  constexpr int QCH = (16 * KS * 4 + 255) / 256;           // chunks of q a thread rotates
+  static_assert(HD <= 256, "a thread takes one value of v");
+  const int tid = threadIdx.x;
+  Rot8 rq[ROPE ? QCH : 1], rk;
+  float rv = 0.f;
+  auto q_chunk = [&](int u, int& head, int& d) {
+    const int c = tid + u * 256;
+    head = c / (KS * 4);
+    d = (c % (KS * 4)) * 8;
+    return head < gcount && d < HD;
+  };
   // Steps are 32-key blocks of the cache, so a step lies in one page.  Row r16 of K tile a is
   // key 8 (r16 / 4) + 4 a + r16 % 4 of the step: the scores of lane (r16, q4) then belong to
   // keys 8 q4 + 4 a + r, r = 0..3, eight consecutive keys over the two tiles.
@@ -258,12 +225,68 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(
 #pragma unroll
     for (int c = 0; c < CT; ++c) vn[c] = *reinterpret_cast<const bf16x8*>(vp + (size_t)(16 * c) * STEP);
   };
+  const int page_first = w < n_steps ? page_of(w) : 0;
+  if constexpr (ROPE) {
+    const float* row = rope.qkv + (size_t)t * (nh + 2 * nk) * HD;
+#pragma unroll
+    for (int u = 0; u < QCH; ++u) {
+      int head, d;
+      if (q_chunk(u, head, d)) load8<HD>(rq[u], row + (size_t)(h0 + head) * HD, rope.cs, rope.sn, p, d);
+    }
+    if (own_split) {
+      if (tid * 8 < HD) load8<HD>(rk, row + (size_t)(nh + hk) * HD, rope.cs, rope.sn, p, tid * 8);
+      if (tid < HD) rv = row[(size_t)(nh + nk + hk) * HD + tid];
+    }
+  }
   int page_ahead = 0;                    // of the step after the one in flight
   if (w < n_steps) {
-    const int page_first = page_of(w);
     if (w + 4 < n_steps) page_ahead = page_of(w + 4);
     issue(w, page_first);
   }
+  if constexpr (ROPE) {
+#pragma unroll
+    for (int u = 0; u < QCH; ++u) {
+      int head, d;
+      const bool have = q_chunk(u, head, d);
+      const bf16x8 q8 = have ? rotated8<HD>(rq[u], d) : bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+      if (head < 16) *reinterpret_cast<bf16x8*>(&sm_q[head * KS * 32 + d]) = q8;
+    }
+    if (own_split) {
+      const bool store = g0 == 0;                          // one block per kv head fills the cache
+      const int page = pt[p / MF_PAGE];
+      if (tid < KS * 4) {
+        const bf16x8 k8 = tid * 8 < HD ? rotated8<HD>(rk, tid * 8) : bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+        if (store && tid * 8 < HD)
+          *reinterpret_cast<bf16x8*>(kc + (((size_t)page * nk + hk) * MF_PAGE + p % MF_PAGE) * HD + tid * 8) = k8;
+        *reinterpret_cast<bf16x8*>(&sm_k[tid * 8]) = k8;
+      }
+      if (tid < HD) {
+        const bf16 v = (bf16)rv;
+        sm_v[tid] = v;
+        if (store)
+          vt[((((size_t)page * nk + hk) * 2 + (p % MF_PAGE) / STEP) * HD + tid) * STEP + p % STEP] = v;
+      }
+    }
+    __syncthreads();
+  }
+  // B operand of the first product: row = head r16, 8 elements of head_dim at 32 ks + 8 q4.
+  bf16x8 qf[KS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) {
+    const int d = ks * 32 + q4 * 8;
+    if constexpr (ROPE) {
+      qf[ks] = *reinterpret_cast<const bf16x8*>(&sm_q[r16 * KS * 32 + d]);
+    } else {
+      qf[ks] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+      if (r16 < gcount && d < HD) qf[ks] = *reinterpret_cast<const bf16x8*>(q + ((size_t)t * nh + h0 + r16) * HD + d);
+    }
+  }
+
+  floatx4 oacc[CT];                       // O^T: head r16, columns 16 c + 4 q4 + r
+#pragma unroll
+  for (int c = 0; c < CT; ++c) oacc[c] = floatx4{0.f, 0.f, 0.f, 0.f};
+  float m_run = -INFINITY, l_run = 0.f;   // of head r16 (the same in the four lanes that share it)
+
   for (int i = w; i < n_steps; i += 4) {
     bf16x8 kf[2][KS], vf[CT];
 #pragma unroll
