@@ -242,6 +242,15 @@ __global__ __launch_bounds__(NT) void sample_kernel(const float* __restrict__ lo
   sample_row(logits + (size_t)blockIdx.x * ld, blockIdx.x, vocab, temp, streams, steps, forced_r, out);
 }
 
+__device__ __forceinline__ float penalised(float v, int count, float repeat, float frequency, float presence) {
+  if (fabsf(frequency) >= 1e-6f || fabsf(presence) >= 1e-6f) {
+    v -= (float)count * frequency;
+    v -= presence;
+  }
+  if (fabsf(repeat - 1.0f) >= 1e-6f && repeat >= 1.0f) v = (v <= 0.f) ? v * repeat : v / repeat;
+  return v;
+}
+
 // penalties in place; prev is [rows][max_prev], n_prev[row] entries are used
 __global__ __launch_bounds__(64) void penalties_kernel(float* __restrict__ logits, int ld, int vocab,
                                                        const int* __restrict__ prev, int max_prev,
@@ -250,6 +259,23 @@ __global__ __launch_bounds__(64) void penalties_kernel(float* __restrict__ logit
   const int rowi = blockIdx.x;
   float* row = logits + (size_t)rowi * ld;
   const int* pv = prev + (size_t)rowi * max_prev;
+  if (max_prev <= 64) {
+    // a lane for each place of the window: three trips to memory (the window, the entries, back), 6.6 us -> 4.2 against a
+    // walk over the window in memory for every token
+    const int lane = threadIdx.x;
+    const int all = pv[min(lane, max_prev - 1)], n = min(n_prev[rowi], max_prev);
+    const bool mine = lane < n && all >= 0 && all < vocab;
+    const float at = mine ? row[all] : 0.f;
+    int count = 0;
+    bool first = true;
+    for (int j = 0; j < n; ++j) {
+      const bool same = __builtin_amdgcn_readlane(all, j) == all;
+      count += same ? 1 : 0;
+      first = first && !(same && j < lane);
+    }
+    if (mine && first) row[all] = penalised(at, count, repeat, frequency, presence);
+    return;
+  }
   const int n = min(n_prev[rowi], max_prev);
   for (int i = threadIdx.x; i < n; i += 64) {
     const int tok = pv[i];
@@ -262,14 +288,7 @@ __global__ __launch_bounds__(64) void penalties_kernel(float* __restrict__ logit
         if (j < i) first = false;
       }
     }
-    if (!first) continue;
-    float v = row[tok];
-    if (fabsf(frequency) >= 1e-6f || fabsf(presence) >= 1e-6f) {
-      v -= (float)count * frequency;
-      v -= presence;
-    }
-    if (fabsf(repeat - 1.0f) >= 1e-6f && repeat >= 1.0f) v = (v <= 0.f) ? v * repeat : v / repeat;
-    row[tok] = v;
+    if (first) row[tok] = penalised(row[tok], count, repeat, frequency, presence);
   }
 }
 
@@ -464,10 +483,20 @@ __global__ __launch_bounds__(256) void piece_max_kernel(const float* __restrict_
   if (lane == 0) piece_max[rowi * CAND_CHUNKS + chunk] = best <= 0x007FFFFFu ? 0u : best;
 }
 
+__device__ __forceinline__ void wave_sync() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }   // LDS that one wave shares
+// An entry's place among others: the larger key first, the lower index among equals, as one whole number (larger first).
+__device__ __forceinline__ uint64_t entry_of(uint32_t key, int idx) { return ((uint64_t)key << 32) | (uint32_t)~idx; }
+__device__ __forceinline__ int entry_index(uint64_t e) { return (int)~(uint32_t)e; }
+__device__ __forceinline__ uint64_t entry_at(uint64_t e, int lane) {        // another lane's (`lane` the same in every lane)
+  return ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(e >> 32), lane) << 32) |
+         (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)e, lane);
+}
+
 // One wave lists one piece (no barrier anywhere: a block is four pieces that know nothing of each
-// other): each lane holds its entries of the piece as keys, the wave takes the largest that is
-// still in play until the k-th and its ties are out or the next one is below the row's bound,
-// lane 0 writes it out.
+// other): each lane holds its entries of the piece as keys; those of at least the row's bound, a handful, go through
+// LDS to a lane each, which counts the ones before its own.  Only a piece with more of them than the list holds (or no
+// bound at all) is taken one largest at a time until the k-th and its ties are out, at a chain of shuffles for each
+// entry: with that for every piece a row of 151,936 took 15.0 us, now 7.5.
 template <int EPT>      // entries per lane: a piece has at most 64 EPT
 __global__ __launch_bounds__(256) void topk_candidates_kernel(const float* __restrict__ logits, int ld,
                                                               int vocab, int k,
@@ -475,31 +504,60 @@ __global__ __launch_bounds__(256) void topk_candidates_kernel(const float* __res
                                                               float* __restrict__ cand_val,
                                                               int* __restrict__ cand_idx,
                                                               int* __restrict__ cand_n) {
-  const int lane = threadIdx.x & 63;
-  const int rowi = blockIdx.y, chunk = blockIdx.x * 4 + (threadIdx.x >> 6);
+  __shared__ uint64_t s_list[4][CAND_CAP];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int rowi = blockIdx.y, chunk = blockIdx.x * 4 + w;
   const float* row = logits + (size_t)rowi * ld;
   const int per = (vocab + CAND_CHUNKS - 1) / CAND_CHUNKS;
   const int lo = chunk * per, n = max(0, min(per, vocab - lo));
+  static_assert(CAND_CHUNKS == 64 && CAND_CAP == 64 && FAST_K_MAX <= CAND_CHUNKS, "a lane for every piece, k pieces at least");
+  const uint32_t mine = piece_max[rowi * CAND_CHUNKS + lane];
+  // this lane's entries: lo + j * 64 + lane, as keys; 0 marks one that is out of play (no entry
+  // above -inf has a key that small, and those at or below -inf are never listed)
+  float x[EPT];
+#pragma unroll
+  for (int j = 0; j < EPT; ++j) x[j] = j * 64 < n ? row[lo + min(j * 64 + lane, n - 1)] : 0.f;
   // the bound: lane c holds piece c's maximum; its place among the 64 (larger first, the lower piece
   // among equals) is the number of lanes that come before it; the one at place k - 1 is the bound
-  static_assert(CAND_CHUNKS == 64 && FAST_K_MAX <= CAND_CHUNKS, "a lane for every piece, k pieces at least");
-  const uint32_t mine = piece_max[rowi * CAND_CHUNKS + lane];
   int place = 0;
+#pragma unroll
   for (int c = 0; c < 64; ++c) {
-    const uint32_t other = (uint32_t)__shfl((int)mine, c, MF_WAVE);
+    const uint32_t other = (uint32_t)__builtin_amdgcn_readlane((int)mine, c);
     place += (other > mine || (other == mine && c < lane)) ? 1 : 0;
   }
   const unsigned long long at = __builtin_amdgcn_ballot_w64(place == k - 1);
   const uint32_t bound = (uint32_t)__shfl((int)mine, (int)__builtin_ctzll(at), MF_WAVE);    // 0: no bound
-  // this lane's entries: lo + j * 64 + lane, as keys; 0 marks one that is out of play (no entry
-  // above -inf has a key that small, and those at or below -inf are never listed)
+  const uint32_t least = max(bound, 0x00800000u);      // of a listed key: the bound, and above -inf
   uint32_t key[EPT];
+  int total = 0;                                       // entries of the piece with at least that
 #pragma unroll
   for (int j = 0; j < EPT; ++j) {
     const int i = j * 64 + lane;
-    key[j] = i < n ? order_key(row[lo + i]) : 0u;
+    key[j] = i < n ? order_key(x[j]) : 0u;
+    const unsigned long long in = __builtin_amdgcn_ballot_w64(key[j] >= least);
+    if (in) {
+      const int to = total + __popcll(in & ((1ull << lane) - 1));
+      if (key[j] >= least && to < CAND_CAP) s_list[w][to] = entry_of(key[j], lo + i);
+      total += __popcll(in);
+    }
   }
   const size_t base = ((size_t)rowi * CAND_CHUNKS + chunk) * CAND_CAP;
+  if (total <= CAND_CAP) {
+    wave_sync();
+    const uint64_t e = lane < total ? s_list[w][lane] : 0;
+    int before = 0;
+    for (int c = 0; c < total; ++c) before += entry_at(e, c) > e ? 1 : 0;
+    const unsigned long long last = __builtin_amdgcn_ballot_w64(lane < total && before == k - 1);
+    const uint32_t kth = last ? (uint32_t)(entry_at(e, (int)__builtin_ctzll(last)) >> 32) : 0u;
+    const bool listed = lane < total && (uint32_t)(e >> 32) >= kth;
+    if (listed) {
+      cand_val[base + before] = key_value((uint32_t)(e >> 32));
+      cand_idx[base + before] = entry_index(e);
+    }
+    const unsigned long long all = __builtin_amdgcn_ballot_w64(listed);
+    if (lane == 0) cand_n[rowi * CAND_CHUNKS + chunk] = __popcll(all);
+    return;
+  }
   int count = 0, over = 0;
   uint32_t kth = 0;
   for (;;) {
@@ -537,27 +595,34 @@ __global__ __launch_bounds__(256) void topk_candidates_kernel(const float* __res
   if (lane == 0) cand_n[rowi * CAND_CHUNKS + chunk] = over ? -1 : count;
 }
 
-// Sums that have to run one after the other (doubles, in a fixed order) run in wave 0 with the
-// terms in registers, place r in lane r % 64 (register r / 64), read out by lane number: a
-// thread that walks an LDS array instead waits for every element in turn.
-__device__ __forceinline__ float at_place(float lo, float hi, int r) {       // r the same in every lane
-  const int l = __builtin_amdgcn_readfirstlane(r & 63);
-  return __int_as_float(r < 64 ? __builtin_amdgcn_readlane(__float_as_int(lo), l)
-                               : __builtin_amdgcn_readlane(__float_as_int(hi), l));
+// Sums that have to run one after the other (doubles, in a fixed order) are run by every lane of a wave over terms in LDS,
+// eight terms a read and no branch between them (places from n to the next multiple of eight hold zeros).
+__device__ __forceinline__ double sum_in_order(const double* terms, int n) {
+  double t = 0.0;
+  for (int i = 0; i < n; i += 8)
+#pragma unroll
+    for (int u = 0; u < 8; ++u) t += terms[i + u];
+  return t;
 }
-__device__ __forceinline__ int at_place(int lo, int hi, int r) {
-  const int l = __builtin_amdgcn_readfirstlane(r & 63);
-  return r < 64 ? __builtin_amdgcn_readlane(lo, l) : __builtin_amdgcn_readlane(hi, l);
-}
-__device__ __forceinline__ double at_place(double lo, double hi, int r) {
-  const int l = __builtin_amdgcn_readfirstlane(r & 63);
-  const double x = r < 64 ? lo : hi;
-  const int a = __builtin_amdgcn_readlane(__double2loint(x), l), b = __builtin_amdgcn_readlane(__double2hiint(x), l);
-  return __hiloint2double(b, a);
+// how many of the running sums satisfy `f` (which, once it is false, stays false)
+template <typename F>
+__device__ __forceinline__ int prefix_count(const float* terms, int n, F f) {
+  double cum = 0.0;
+  int count = 0;
+  for (int i = 0; i < n && f(cum); i += 8)
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      cum += (double)terms[i + u];
+      count += f(cum) ? 1 : 0;
+    }
+  return count;
 }
 
 constexpr int RANK_MAX = 512;        // candidates up to which each finds its place by counting the ones before it
 
+// The block's part is the survivors and their places; from there on they are a wave's own, two places a lane, with no
+// barrier.  A chain of waits throughout (one block a row, some 100 candidates and 40 survivors): what it reads is asked for
+// at once, 21.2 -> 7.2 us at a row of 151,936.
 __global__ __launch_bounds__(NT) void sample_filtered_kernel(float* __restrict__ logits, int ld, int vocab, int k,
                                                              float top_p, float temp,
                                                              const long long* __restrict__ streams,
@@ -567,111 +632,91 @@ __global__ __launch_bounds__(NT) void sample_filtered_kernel(float* __restrict__
                                                              const int* __restrict__ cand_idx,
                                                              const int* __restrict__ cand_n,
                                                              int* __restrict__ out) {
-  __shared__ float v[SURV_CAP];        // survivors: value, index, probability, alive
-  __shared__ int ix[SURV_CAP];
-  __shared__ float pr[SURV_CAP];
-  __shared__ int alive[SURV_CAP];
-  __shared__ int order[SURV_CAP];      // survivor at a place
-  __shared__ int s_n, s_over, s_total, s_keep;
+  __shared__ uint64_t d_entry[CAND_CHUNKS * CAND_CAP];         // the pieces' lists one after the other
+  __shared__ uint64_t s_surv[SURV_CAP];                        // survivors at their places
+  __shared__ __attribute__((aligned(16))) double s_sum[SURV_CAP];
+  __shared__ __attribute__((aligned(16))) float s_pr[SURV_CAP];
+  __shared__ __attribute__((aligned(16))) int s_x[SURV_CAP];
+  __shared__ int s_n, s_over;
   __shared__ uint32_t s_kth;
-  __shared__ uint32_t d_key[CAND_CHUNKS * CAND_CAP];   // the pieces' lists one after the other, as keys
-  __shared__ int d_idx[CAND_CHUNKS * CAND_CAP];
-  __shared__ int c_n[CAND_CHUNKS], c_off[CAND_CHUNKS];
   const int rowi = blockIdx.x;
   float* row = logits + (size_t)rowi * ld;
   const int tid = threadIdx.x, lane = tid & 63;
-  if (tid == 0) { s_n = 0; s_over = 0; s_kth = 0; }
-  __syncthreads();
-  if (tid < 64) {
-    // where each piece's list begins in the row's list
-    static_assert(CAND_CHUNKS == 64, "a lane for every piece");
-    const int cn = cand_n[rowi * CAND_CHUNKS + lane];
-    const bool piece_over = __builtin_amdgcn_ballot_w64(cn < 0) != 0;
-    const int cnt = max(cn, 0);
-    int incl = cnt;
+  // thread: entries tid / 64 + 16 i of piece tid % 64.  The first of them (inside the work space whatever the list holds)
+  // and the draw's numbers are asked for with the lists' lengths
+  static_assert(CAND_CHUNKS == 64, "a lane for every piece");
+  const size_t src = ((size_t)rowi * CAND_CHUNKS + lane) * CAND_CAP + tid / 64;
+  const int cn = cand_n[rowi * CAND_CHUNKS + lane];
+  const float first_val = cand_val[src];
+  const int first_idx = cand_idx[src];
+  const float rnd = forced_r ? forced_r[rowi] : uniform01((uint64_t)streams[rowi], (uint64_t)(uint32_t)steps[rowi]);
+  if (tid == 0) { s_n = 0; s_kth = 0; }
+  // where each piece's list begins in the row's list (every wave for itself)
+  bool over = __builtin_amdgcn_ballot_w64(cn < 0) != 0;        // the same in every thread up to the second barrier
+  const int cnt = max(cn, 0);
+  int incl = cnt;
 #pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int up = __shfl_up(incl, o, MF_WAVE);
-      if (lane >= o) incl += up;
-    }
-    c_n[lane] = cnt;
-    c_off[lane] = incl - cnt;
-    if (lane == 63) s_total = incl;
-    if (lane == 0 && piece_over) s_over = 1;
+  for (int o = 1; o < 64; o <<= 1) {
+    const int up = __shfl_up(incl, o, MF_WAVE);
+    if (lane >= o) incl += up;
+  }
+  const int C = __builtin_amdgcn_readlane(incl, 63), begin = incl - cnt;
+  if (tid == 0) s_over = over;
+  if (!over) {
+    if (tid / 64 < cnt) d_entry[begin + tid / 64] = entry_of(order_key(first_val), first_idx);
+    for (int i = NT / 64; tid / 64 + i < cnt; i += NT / 64)
+      d_entry[begin + tid / 64 + i] = entry_of(order_key(cand_val[src + i]), cand_idx[src + i]);
   }
   __syncthreads();
-  const int C = s_total;
-  if (!s_over) {
-    // every piece's first entries in the first round (the lists are short as a rule: one wait for
-    // memory, not one per piece)
-    for (int s0 = 0; s0 < CAND_CAP; s0 += NT / CAND_CHUNKS) {
-      const int piece = tid % CAND_CHUNKS, slot = s0 + tid / CAND_CHUNKS;
-      if (slot < c_n[piece]) {
-        const size_t src = (size_t)rowi * CAND_CHUNKS * CAND_CAP + piece * CAND_CAP + slot;
-        d_key[c_off[piece] + slot] = order_key(cand_val[src]);
-        d_idx[c_off[piece] + slot] = cand_idx[src];
-      }
+  if (!over && C <= RANK_MAX) {
+    // Few candidates (the rule): each counts the ones that come before it, which is its place; the one at place k - 1
+    // names the k-th value, and what is at least that survives, at its place.  2 to 16 threads a candidate.
+    static_assert(2 * RANK_MAX <= NT, "two threads for every candidate");
+    const int lg = C > 256 ? 1 : C > 128 ? 2 : C > 64 ? 3 : 4, share = 1 << lg;
+    const int c = tid >> lg;
+    const uint64_t e = c < C ? d_entry[c] : 0;
+    int place = 0;
+    if (c < C) {
+#pragma unroll 4
+      for (int j = tid & (share - 1); j < C; j += share) place += d_entry[j] > e ? 1 : 0;
     }
-  }
-  __syncthreads();
-  if (!s_over && C <= RANK_MAX) {
-    // Few candidates (the rule): each counts the ones that come before it (larger first, the lower
-    // index among equals), which is its place; the one at place k - 1 names the k-th value, and
-    // what is at least that survives, at its place.
-    static_assert(RANK_MAX <= NT, "a thread for every candidate");
-    uint32_t mk = 0;
-    int mi = 0, place = 0;
-    if (tid < C) {
-      mk = d_key[tid];
-      mi = d_idx[tid];
-      for (int j = 0; j < C; ++j) {
-        const uint32_t ok = d_key[j];
-        const int oi = d_idx[j];
-        place += (ok > mk || (ok == mk && oi < mi)) ? 1 : 0;
-      }
-      if (place == k - 1) s_kth = mk;
-    }
+    for (int o = 1; o < share; o <<= 1) place += __shfl_xor(place, o, MF_WAVE);
+    const bool one = c < C && (tid & (share - 1)) == 0;
+    if (one && place == k - 1) s_kth = (uint32_t)(e >> 32);
     __syncthreads();
-    if (tid < C && mk >= s_kth) {
-      if (place < SURV_CAP) {
-        v[place] = key_value(mk);
-        ix[place] = mi;
-      } else {
-        s_over = 1;
-      }
-      atomicAdd(&s_n, 1);
+    const bool stays = one && (uint32_t)(e >> 32) >= s_kth;
+    if (stays) {
+      if (place < SURV_CAP) s_surv[place] = e;
+      else s_over = 1;
     }
-  } else if (!s_over && tid < 64) {
+    const int stay = __popcll(__builtin_amdgcn_ballot_w64(stays));
+    if (lane == 0 && stay) atomicAdd(&s_n, stay);
+  } else if (!over && tid < 64) {
     // many candidates: the pieces' lists are sorted, lane c holds the head of piece c's, the wave
-    // takes the best head (the lower piece among equals, which is the lower index) until the k-th
-    // and its ties are out
-    const int c = lane;
-    const int cn = c_n[c], base = c_off[c];
-    int head = 0, count = 0, over = 0;
+    // takes the best head until the k-th and its ties are out
+    int head = 0, count = 0, full = 0;
     uint32_t kth = 0;
     for (;;) {
-      const bool has = head < cn;
-      const uint32_t hk = has ? d_key[base + head] : 0;
-      uint32_t rk = hk;
-      int rc = has ? c : 0x7fffffff;
+      const uint64_t he = head < cnt ? d_entry[begin + head] : 0;       // (no entry is 0)
+      uint64_t best = he;
 #pragma unroll
       for (int o = 32; o > 0; o >>= 1) {
-        const uint32_t ok = __shfl_xor(rk, o, MF_WAVE);
-        const int oc = __shfl_xor(rc, o, MF_WAVE);
-        if (oc != 0x7fffffff && (rc == 0x7fffffff || ok > rk || (ok == rk && oc < rc))) { rk = ok; rc = oc; }
+        const uint64_t other = ((uint64_t)(uint32_t)__shfl_xor((int)(best >> 32), o, MF_WAVE) << 32) |
+                               (uint32_t)__shfl_xor((int)(uint32_t)best, o, MF_WAVE);
+        if (other > best) best = other;
       }
-      if (rc == 0x7fffffff) break;
+      if (best == 0) break;
+      const uint32_t rk = (uint32_t)(best >> 32);
       if (count >= k && rk != kth) break;
-      if (count == SURV_CAP) { over = 1; break; }
+      if (count == SURV_CAP) { full = 1; break; }
       if (count == k - 1) kth = rk;
-      if (c == rc) {
-        v[count] = key_value(d_key[base + head]);
-        ix[count] = d_idx[base + head];
+      if (he == best) {
+        s_surv[count] = best;
         ++head;
       }
       ++count;
     }
-    if (lane == 0) { s_n = count; if (over) s_over = 1; }
+    if (lane == 0) { s_n = count; if (full) s_over = 1; }
   }
   __syncthreads();
   if (s_over) {            // too many equal values for the lists: the whole-row kernels, in place
@@ -680,83 +725,84 @@ __global__ __launch_bounds__(NT) void sample_filtered_kernel(float* __restrict__
     sample_row(row, rowi, vocab, temp, streams, steps, forced_r, out);
     return;
   }
-  const int n = s_n;       // survivors, largest first, equal values in index order
-  if (tid < n) alive[tid] = 1;
-  __syncthreads();
-  const float mx = n > 0 ? v[0] : -INFINITY;
-  const int r0 = lane, r1 = lane + 64;                 // wave 0: the two places of a lane
+  if (tid >= 64) return;
+  // wave 0 alone from here on: lane holds the survivors at places r0 and r1 (largest first, equal values in index order)
+  const int n = s_n;
+  const int r0 = lane, r1 = lane + 64;
+  const uint64_t u0 = r0 < n ? s_surv[r0] : 0, u1 = r1 < n ? s_surv[r1] : 0;
+  const float v0 = key_value((uint32_t)(u0 >> 32)), v1 = key_value((uint32_t)(u1 >> 32));
+  const int x0 = entry_index(u0), x1 = entry_index(u1);
+  bool alive0 = r0 < n, alive1 = r1 < n;
+  const float mx = n > 0 ? key_value((uint32_t)(s_surv[0] >> 32)) : -INFINITY;
   if (top_p > 0.f && top_p < 1.f && mx > -INFINITY) {
     // as top_p_row: p_i = exp(l_i - max) / sum over finite entries, the sum in double
-    __shared__ double s_tot;
-    if (tid < 64) {
-      const double e0 = r0 < n && v[r0] > -INFINITY ? exp((double)(v[r0] - mx)) : 0.0;
-      const double e1 = r1 < n && v[r1] > -INFINITY ? exp((double)(v[r1] - mx)) : 0.0;
-      double t = 0.0;
-      for (int i = 0; i < n; ++i) t += at_place(e0, e1, i);
-      if (lane == 0) s_tot = t;
-    }
-    __syncthreads();
-    const float tot_f = (float)s_tot;
-    if (tid < n) pr[tid] = v[tid] > -INFINITY ? share_of(v[tid], mx, tot_f) : -1.f;    // -1: not finite, last
-    __syncthreads();
-    if (tid < n) {
-      int r = 0;
-      for (int j = 0; j < n; ++j)
-        if (pr[j] > pr[tid] || (pr[j] == pr[tid] && ix[j] < ix[tid])) ++r;
-      order[r] = tid;
-    }
-    __syncthreads();
-    if (tid < 64) {
-      // descending, stable: the shortest prefix whose mass exceeds p stays
-      const float p0 = r0 < n ? pr[order[r0]] : -1.f, p1 = r1 < n ? pr[order[r1]] : -1.f;
-      double cum = 0.0;
-      int keep = n;
-      for (int r = 0; r < n; ++r) {
-        const float p = at_place(p0, p1, r);
-        if (p < 0.f) { keep = min(keep, r); break; }           // entries that are not finite stay as they are
-        cum += (double)p;
-        if (cum > (double)top_p) { keep = r + 1; break; }
+    s_sum[r0] = r0 < n && v0 > -INFINITY ? exp((double)(v0 - mx)) : 0.0;
+    s_sum[r1] = 0.0;
+    if (r1 < n && v1 > -INFINITY) s_sum[r1] = exp((double)(v1 - mx));
+    wave_sync();
+    const float tot_f = (float)sum_in_order(s_sum, n);
+    const float p0 = r0 < n ? share_of(v0, mx, tot_f) : 0.f, p1 = r1 < n ? share_of(v1, mx, tot_f) : 0.f;
+    // descending, the lower index among equals: the places' own order unless two neighbours have one probability
+    int o0 = r0, o1 = r1;
+    s_pr[r0] = p0;
+    s_pr[r1] = p1;
+    s_x[r0] = x0;
+    s_x[r1] = x1;
+    wave_sync();
+    auto in_order = [&](int r, float p, int x) {
+      if (r + 1 >= n) return true;
+      const float next = s_pr[r + 1];
+      return p > next || (p == next && x < s_x[r + 1]);
+    };
+    if (__builtin_amdgcn_ballot_w64(!in_order(r0, p0, x0) || !in_order(r1, p1, x1))) {
+      o0 = o1 = 0;
+      for (int j = 0; j < n; ++j) {
+        const float p = s_pr[j];
+        const int x = s_x[j];
+        o0 += p > p0 || (p == p0 && x < x0) ? 1 : 0;
+        o1 += p > p1 || (p == p1 && x < x1) ? 1 : 0;
       }
-      if (r0 < n && r0 >= keep && p0 >= 0.f) alive[order[r0]] = 0;
-      if (r1 < n && r1 >= keep && p1 >= 0.f) alive[order[r1]] = 0;
+      wave_sync();
+      if (r0 < n) s_pr[o0] = p0;
+      if (r1 < n) s_pr[o1] = p1;
+      wave_sync();
     }
-    __syncthreads();
+    // descending, stable: the shortest prefix whose mass exceeds p stays
+    const int keep = min(n, 1 + prefix_count(s_pr, n, [=](double cum) { return !(cum > (double)top_p); }));
+    if (o0 >= keep) alive0 = false;
+    if (o1 >= keep) alive1 = false;
   }
-  // as sample_row on what is left, in index order
-  if (tid < n) {
-    int r = 0;
-    for (int j = 0; j < n; ++j)
-      if (ix[j] < ix[tid]) ++r;
-    order[r] = tid;
-  }
-  __syncthreads();
-  if (tid >= 64) return;
-  // wave 0 alone from here on: lane holds the survivors at places r0 and r1 of the index order
-  const float inv_t = 1.0f / temp;
-  const int i0 = r0 < n ? order[r0] : 0, i1 = r1 < n ? order[r1] : 0;
-  const bool on0 = r0 < n && alive[i0], on1 = r1 < n && alive[i1];
-  const float l0 = on0 ? scaled(v[i0], inv_t) : -INFINITY, l1 = on1 ? scaled(v[i1], inv_t) : -INFINITY;
-  float mxt = fmaxf(l0, l1);
+  // as sample_row on what is left, in index order (what is not alive adds nothing there)
+  wave_sync();
+  s_x[r0] = alive0 ? x0 : 0x7fffffff;
+  s_x[r1] = alive1 ? x1 : 0x7fffffff;
+  wave_sync();
+  int o0 = 0, o1 = 0;
+  for (int j = 0; j < n; j += 8)
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) mxt = fmaxf(mxt, __shfl_xor(mxt, o, MF_WAVE));
+    for (int u = 0; u < 8; ++u) o0 += s_x[j + u] < x0 ? 1 : 0;
+  if (n > 64)
+    for (int j = 0; j < n; ++j) o1 += s_x[j] < x1 ? 1 : 0;
+  if (alive0) d_entry[o0] = u0;
+  if (alive1) d_entry[o1] = u1;
+  wave_sync();
+  const int left = __popcll(__builtin_amdgcn_ballot_w64(alive0)) + __popcll(__builtin_amdgcn_ballot_w64(alive1));
+  const uint64_t y0 = r0 < left ? d_entry[r0] : 0, y1 = r1 < left ? d_entry[r1] : 0;
+  const float inv_t = 1.0f / temp;
+  const float l0 = r0 < left ? scaled(key_value((uint32_t)(y0 >> 32)), inv_t) : -INFINITY;
+  const float l1 = r1 < left ? scaled(key_value((uint32_t)(y1 >> 32)), inv_t) : -INFINITY;
+  const float mxt = wave_max(fmaxf(l0, l1));
   const float e0 = l0 > -INFINITY ? exp_rel(l0, mxt) : 0.f, e1 = l1 > -INFINITY ? exp_rel(l1, mxt) : 0.f;
-  double total = 0.0;
-  for (int r = 0; r < n; ++r) total += (double)at_place(e0, e1, r);
-  const float inv = (float)(1.0 / total);
-  const float q0 = e0 * inv, q1 = e1 * inv;            // the probability, as prob_of forms it
-  const int x0 = r0 < n ? ix[i0] : 0, x1 = r1 < n ? ix[i1] : 0;
-  const float rnd = forced_r ? forced_r[rowi]
-                             : uniform01((uint64_t)streams[rowi], (uint64_t)(uint32_t)steps[rowi]);
+  s_sum[r0] = (double)e0;
+  s_sum[r1] = (double)e1;
+  wave_sync();
+  const float inv = (float)(1.0 / sum_in_order(s_sum, left));
+  s_pr[r0] = e0 * inv;                                 // the probability, as prob_of forms it
+  s_pr[r1] = e1 * inv;
+  wave_sync();
   const double rr = fmax((double)rnd, 1e-30);
-  double cum = 0.0;
-  int pick = vocab - 1;                // fallback: the last index (src/sampler.rs:266)
-  for (int r = 0; r < n; ++r) {
-    const float p = at_place(q0, q1, r);
-    if (p <= 0.f) continue;
-    cum += (double)p;
-    if (rr <= cum) { pick = at_place(x0, x1, r); break; }
-  }
-  if (lane == 0) out[rowi] = pick;
+  const int at = prefix_count(s_pr, left, [=](double cum) { return !(rr <= cum); });
+  if (lane == 0) out[rowi] = at < left ? entry_index(d_entry[at]) : vocab - 1;     // fallback: the last index (src/sampler.rs:266)
 }
 
 // after a decode step: feed the sampled token back, move every sequence on by one, and (when

@@ -192,6 +192,27 @@ def test_sample_filtered_with_many_candidates(ops):
     assert torch.equal(d.cpu(), l)
 
 
+@pytest.mark.parametrize("count", [64, 65, 128, 129, 256, 257, 512, 513])
+def test_sample_filtered_by_number_of_candidates(ops, count):
+    """As many candidates as a share of the threads takes and one more: ten that survive, in one piece, and the rest at the
+    bound, dealt over the other 63; with a piece of 70 at the bound instead (more than its list holds) for the second row."""
+    vocab, k = 152064, 10
+    per = (vocab + 63) // 64
+    l = logits_rows(2, vocab, 31).clamp(-1.0, 1.0)
+    l[:, 50:50 + k] = 10.0 + 0.25 * torch.arange(k)
+    for i in range(count - k):
+        l[:, (1 + i % 63) * per + 11 * (i // 63)] = 5.0
+    l[1, per:per + 70] = 5.0
+    rs = torch.tensor([0.4, 0.9], device=DEV)
+    keys, steps = torch.zeros(2, dtype=torch.int64, device=DEV), torch.zeros(2, dtype=torch.int32, device=DEV)
+    chain, want, got = l.to(DEV), torch.empty(2, dtype=torch.int32, device=DEV), torch.empty(2, dtype=torch.int32, device=DEV)
+    ops.top_k(chain, k)
+    ops.top_p(chain, 0.95)
+    ops.sample(chain, 0.8, keys, steps, want, rs)
+    ops.sample_filtered(l.to(DEV), k, 0.95, 0.8, keys, steps, got, rs)
+    assert got.cpu().tolist() == want.cpu().tolist() and all(50 <= t < 50 + k for t in got.cpu().tolist())
+
+
 def test_device_uniform_is_the_host_uniform_and_draws_follow_softmax(ops):
     rows, vocab = 4000, 3
     small = torch.tensor([0.0, 1.0, 2.0]).repeat(rows, 1).to(DEV)
