@@ -8,9 +8,10 @@
 // half pages first and then jumps to the half page of its window's first key; with `sink`, a number per head, the
 // denominator also holds e^sink[h] (split 0 starts from it as from a key without a value).
 //
-// A wave (a workgroup of its own) owns 16 consecutive new tokens of one sequence times RB query heads of one kv
-// head and walks the tokens' keys 32 at a time (half a page), with no LDS and no barrier; the key rows of a
-// step are asked for a step ahead, the value rows before the step's scores are formed:
+// A workgroup of WK waves owns 16 consecutive new tokens of one sequence times RB query heads of one kv head; its
+// waves take the tokens' keys 32 at a time (half a page) in turn, with no LDS and no barrier until they add up their
+// sums at the end; the key rows of a step are asked for a step ahead, their page a step before that, the value rows
+// before the step's scores are formed:
 //   S^T[key][token] = K Q^T      16x16x32 MFMA, A = 16 key rows straight from the cache, B = Q kept in registers
 //   a lane holds, for its token (lane % 16), the scores of keys 4 (lane / 16) + i of both key tiles:
 //   the softmax statistics are per lane, shared by the four lanes of a token through two shuffles
@@ -72,8 +73,13 @@ __device__ __forceinline__ float fast_tanh(float y) {
   return fmaf(-2.0f, __builtin_amdgcn_rcpf(e + 1.0f), 1.0f);
 }
 
-template <int RB>
-__global__ __launch_bounds__(64) void capped_mfma_kernel(
+// A step is a chain (page, keys, scores, softmax, values) that one wave a SIMD leaves waiting most of the time, a tile's
+// last keys decide how long a launch takes, and a group's keys want to stay in one die's L2.  Two heads a wave and four waves
+// a tile, two of them on a SIMD (256 registers: so the next keys go where this step's were), every group on its dies: 16 heads
+// of 128 over two kv heads, 2,048 tokens 144 -> 78 us, over 16 kv heads 237 -> 129; 8,192 tokens over four 1,350 -> 940; 203
+// tokens 15.6 -> 11.
+template <int RB, int WK>
+__global__ __launch_bounds__(64 * WK, WK > 1 ? 2 : 1) void capped_mfma_kernel(
     const bf16* __restrict__ q, const bf16* __restrict__ kc, const bf16* __restrict__ vc,
     const int* __restrict__ page_table, int pt_stride, const int* __restrict__ cu_seqlens,
     const int* __restrict__ start_pos, const int* __restrict__ tile_seq, const int* __restrict__ tile_q0, int n_tiles,
@@ -82,12 +88,19 @@ __global__ __launch_bounds__(64) void capped_mfma_kernel(
     const float* __restrict__ far_b, int keep_first, const float* __restrict__ bias, int n_bias,
     const float* __restrict__ sink) {
   const int lane = threadIdx.x & 63;
-  const int tile = blockIdx.x;                    // a workgroup is one wave: the waves drift apart freely
-  if (tile >= n_tiles) return;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // Consecutive workgroups go to consecutive dies, each with an L2 of its own: a die takes every eighth group of heads (or,
+  // with fewer groups, a group shares itself over 8 / groups dies), all of its tiles, the tiles in their order.
   const int G = nh / nk;
-  const int n_hc = G / RB;
-  const int hk = blockIdx.y / n_hc;
-  const int h0 = hk * G + (blockIdx.y % n_hc) * RB;
+  const int n_hc = G / RB, n_hg = nk * n_hc;
+  const int die = blockIdx.x % 8, turn = blockIdx.x / 8;
+  int tile, hg;
+  if (n_hg % 8 == 0) { hg = die + 8 * (turn % (n_hg / 8)); tile = turn / (n_hg / 8); }
+  else if (8 % n_hg == 0) { hg = die % n_hg; tile = turn * (8 / n_hg) + die / n_hg; }
+  else { hg = blockIdx.x / n_tiles; tile = blockIdx.x % n_tiles; }
+  if (tile >= n_tiles || hg >= n_hg) return;
+  const int hk = hg / n_hc;
+  const int h0 = hk * G + (hg % n_hc) * RB;
   const int col = lane & 15, g = lane >> 4;
 
   const int b = tile_seq[tile], q0 = tile_q0[tile];
@@ -111,7 +124,9 @@ __global__ __launch_bounds__(64) void capped_mfma_kernel(
   // the kept first keys, in half pages [0, kept_stop), where they lie before the first half page of the window;
   // the keys between them and the window are seen by none of the tile's tokens
   const int kept_stop = (keep_first > 0 && split == 0) ? min((keep_first + 31) & ~31, k_first) : 0;
-  auto next_step = [&](int kb) { return (kb < kept_stop && kb + 32 >= kept_stop) ? k_first : kb + 32; };
+  const int n_kept = kept_stop / 32, n_steps = n_kept + max(0, (k_stop - k_first + 31) / 32);
+  auto step_key = [&](int i) { return i < n_kept ? i * 32 : k_first + (i - n_kept) * 32; };       // the first key of step i
+  auto step_page = [&](int i) { return pt[step_key(min(i, n_steps - 1)) / MF_PAGE]; };
 
   // Q fragments: token `col`, values 32 ks + 8 g .. + 8 of head h0 + r
   bf16x8 qf[RB][DKS];
@@ -140,17 +155,18 @@ __global__ __launch_bounds__(64) void capped_mfma_kernel(
 #pragma unroll
   for (int r = 0; r < RB; ++r) {
     // the sink weighs one against itself; a token's weight is spread over four lanes, of which one counts it
-    m[r] = sink && split == 0 ? sink[h0 + r] : -INFINITY;
-    l[r] = sink && split == 0 && g == 0 ? 1.f : 0.f;
+    m[r] = sink && split == 0 && w == 0 ? sink[h0 + r] : -INFINITY;
+    l[r] = sink && split == 0 && w == 0 && g == 0 ? 1.f : 0.f;
 #pragma unroll
     for (int c = 0; c < NVT; ++c) oacc[r][c] = floatx4{0.f, 0.f, 0.f, 0.f};
   }
 
   // K fragments of both key tiles of the 32 keys from kb: key row `col` (+ 16), values 32 ks + 8 g .. + 8;
-  // they are asked for one step ahead
+  // the next step's are asked for as soon as this step's scores are formed (four heads: a step ahead, their scores one
+  // after the other: it is the scores that there are no registers for)
+  constexpr bool COPY = RB > 2;
   bf16x8 kn[2][DKS];
-  auto ask_k = [&](int kb) {
-    const int page = pt[kb / MF_PAGE];
+  auto ask_k = [&](int kb, int page) {
     const bf16* kbase = kc + (((size_t)page * nk + hk) * MF_PAGE + kb % MF_PAGE + col) * D + g * 8;
 #pragma unroll
     for (int a = 0; a < 2; ++a)
@@ -161,17 +177,26 @@ __global__ __launch_bounds__(64) void capped_mfma_kernel(
         kn[a][ks] = v;
       }
   };
-  const int kb_first = kept_stop > 0 ? 0 : k_first;
-  if (kb_first < k_stop) ask_k(kb_first);
-  for (int kb = kb_first; kb < k_stop; kb = next_step(kb)) {
-    const int page = pt[kb / MF_PAGE];
+  int page_next = 0, page_ahead = 0;              // of the step whose keys are on their way, of the step after it
+  if (w < n_steps) {
+    page_next = step_page(w);
+    page_ahead = step_page(w + WK);
+    ask_k(step_key(w), page_next);
+  }
+  for (int i = w; i < n_steps; i += WK) {
+    const int kb = step_key(i), page = page_next;
     const int in_page = kb % MF_PAGE;              // 0 or 32
+    auto ask_next = [&]() {
+      page_next = page_ahead;
+      if (i + WK < n_steps) ask_k(step_key(i + WK), page_next);
+      page_ahead = step_page(i + 2 * WK);
+    };
     bf16x8 kf[2][DKS];
 #pragma unroll
     for (int a = 0; a < 2; ++a)
 #pragma unroll
       for (int ks = 0; ks < DKS; ++ks) kf[a][ks] = kn[a][ks];
-    if (next_step(kb) < k_stop) ask_k(next_step(kb));
+    if constexpr (COPY) ask_next();
     // V^T fragments: value row 16 c + col, keys 4 g .. + 4 and 16 + 4 g .. + 4 of this half page, asked for
     // before the scores are formed
     const bf16* vbase = vc + ((((size_t)page * nk + hk) * 2 + in_page / 32) * V + col) * 32 + 4 * g;
@@ -192,15 +217,24 @@ __global__ __launch_bounds__(64) void capped_mfma_kernel(
       seen[j] = all_seen || (row_ok && key <= p_mine && (window <= 0 || p_mine - key < window || key < keep_first) && key >= chunk_lo);
       dist[j] = (float)max(0, p_mine - key);
     }
+    floatx4 s0[RB], s1[RB];
+    auto scores = [&](int r) {
+      s0[r] = s1[r] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int ks = 0; ks < DKS; ++ks) {
+        s0[r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[0][ks], qf[r][ks], s0[r], 0, 0, 0);
+        s1[r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[1][ks], qf[r][ks], s1[r], 0, 0, 0);
+      }
+    };
+    if constexpr (!COPY) {
+#pragma unroll
+      for (int r = 0; r < RB; ++r) scores(r);
+      ask_next();
+    }
     bf16x8 pf[RB];
 #pragma unroll
     for (int r = 0; r < RB; ++r) {
-      floatx4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int ks = 0; ks < DKS; ++ks) {
-        s0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[0][ks], qf[r][ks], s0, 0, 0, 0);
-        s1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[1][ks], qf[r][ks], s1, 0, 0, 0);
-      }
+      if constexpr (COPY) scores(r);
       float x[8];
       float add_lo[4] = {0.f, 0.f, 0.f, 0.f}, add_hi[4] = {0.f, 0.f, 0.f, 0.f};
       if (bias) {        // this lane's keys are two runs of four neighbours, 16 keys apart
@@ -209,7 +243,7 @@ __global__ __launch_bounds__(64) void capped_mfma_kernel(
         bias_run(brow, n_bias, p_mine - (kb + 16 + 4 * g), add_hi);
       }
 #pragma unroll
-      for (int j = 0; j < 8; ++j) x[j] = (j < 4 ? s0[j] : s1[j - 4]) * sc[r];
+      for (int j = 0; j < 8; ++j) x[j] = (j < 4 ? s0[r][j] : s1[r][j - 4]) * sc[r];
       if (cap > 0.f) {
 #pragma unroll
         for (int j = 0; j < 8; ++j) x[j] = cap * fast_tanh(x[j] * inv_cap);
@@ -274,6 +308,58 @@ __global__ __launch_bounds__(64) void capped_mfma_kernel(
     }
   }
 
+  if constexpr (WK > 1) {
+    // the waves' sums relative to the largest of their references, head after head, in the order of the waves
+    constexpr int LD = V + 4;
+    __shared__ __attribute__((aligned(16))) float sm_o[WK][16][LD];
+    __shared__ float sm_m[WK][RB][16], sm_l[WK][RB][16];
+#pragma unroll
+    for (int r = 0; r < RB; ++r) {
+      float L = l[r];
+      L += __shfl_xor(L, 16, MF_WAVE);
+      L += __shfl_xor(L, 32, MF_WAVE);
+      if (g == 0) { sm_m[w][r][col] = m[r]; sm_l[w][r][col] = L; }
+    }
+#pragma unroll
+    for (int r = 0; r < RB; ++r) {
+      if (r) __syncthreads();
+#pragma unroll
+      for (int c = 0; c < NVT; ++c) *(floatx4*)&sm_o[w][col][c * 16 + 4 * g] = oacc[r][c];
+      __syncthreads();
+      for (int x = threadIdx.x; x < 16 * (V / 8); x += 64 * WK) {
+        const int tok = x / (V / 8), d = x % (V / 8) * 8;
+        float top = sm_m[0][r][tok];
+#pragma unroll
+        for (int u = 1; u < WK; ++u) top = fmaxf(top, sm_m[u][r][tok]);
+        float sum[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, L = 0.f;
+#pragma unroll
+        for (int u = 0; u < WK; ++u) {
+          const float f = sm_m[u][r][tok] == -INFINITY ? 0.f : __expf(sm_m[u][r][tok] - top);      // (a wave without keys)
+          L = fmaf(f, sm_l[u][r][tok], L);
+          const floatx4 a0 = *(const floatx4*)&sm_o[u][tok][d], a1 = *(const floatx4*)&sm_o[u][tok][d + 4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            sum[e] = fmaf(f, a0[e], sum[e]);
+            sum[4 + e] = fmaf(f, a1[e], sum[4 + e]);
+          }
+        }
+        const float inv = L > 0.f ? 1.0f / L : 0.f;
+        bf16x4 lo4, hi4;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          lo4[e] = (bf16)(sum[e] * inv);
+          hi4[e] = (bf16)(sum[4 + e] * inv);
+        }
+        if (tok < rows) {
+          bf16* o = out + ((size_t)(t_first + tok) * nh + h0 + r) * V + d;
+          *(bf16x4*)o = lo4;
+          *(bf16x4*)(o + 4) = hi4;
+        }
+      }
+    }
+    return;
+  }
+
   // O^T[d = 16 c + 4 g + i][token col] -> out[token][head][d]
 #pragma unroll
   for (int r = 0; r < RB; ++r) {
@@ -331,15 +417,21 @@ MF_API int mf_capped_mfma(const void* q, const void* kc, const void* vc, const i
   // heads of a kv head a wave takes together: four where that still leaves waves for all SIMDs
   int rb = G % 2 == 0 ? 2 : 1;
   if (G % 4 == 0 && (long long)n_tiles * nk * (G / 4) >= 4096) rb = 4;
-  dim3 grid(n_tiles, nk * (G / rb), n_splits);
-#define MF_GO(RB)                                                                                                          \
-  capped_mfma_kernel<RB><<<grid, 64, 0, stream>>>((const bf16*)q, (const bf16*)kc, (const bf16*)vc, page_table, pt_stride, \
+  // waves a tile: four, but one where the tiles' keys are split already and for four heads (whose sums leave no registers
+  // for a second wave a SIMD; 16 heads over four kv heads, four heads a wave / two heads and four waves: 8,192 tokens 873 /
+  // 940 us, 12,000 2,038 / 1,966, 16,384 3,410 / 3,616)
+  const int wk = n_splits == 1 && rb <= 2 ? 4 : 1;
+  dim3 grid((n_tiles * nk * (G / rb) + 7) / 8 * 8, 1, n_splits);          // (whole rounds of the eight dies)
+#define MF_GO(RB, WK)                                                                                                      \
+  capped_mfma_kernel<RB, WK><<<grid, 64 * WK, 0, stream>>>((const bf16*)q, (const bf16*)kc, (const bf16*)vc, page_table, pt_stride, \
                                                    cu_seqlens, start_pos, tile_seq, tile_q0, n_tiles, temp, (bf16*)out, part, \
                                                    n_splits, split_len, nh, nk, scale, cap, window, chunk, far_a, far_b, \
                                                    keep_first, bias, n_bias, sink)
-  if (rb == 4) MF_GO(4);
-  else if (rb == 2) MF_GO(2);
-  else MF_GO(1);
+  if (rb == 4) MF_GO(4, 1);
+  else if (rb == 2 && wk == 4) MF_GO(2, 4);
+  else if (rb == 2) MF_GO(2, 1);
+  else if (wk == 4) MF_GO(1, 4);
+  else MF_GO(1, 1);
 #undef MF_GO
   int rc = mf_launch_status();
   if (rc == 0 && n_splits > 1) {
