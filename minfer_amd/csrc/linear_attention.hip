@@ -302,6 +302,8 @@ static_assert(MF_LA_CHUNK == 64, "a wave of memory_gates_kernel takes a chunk");
 // staged in LDS with rows 4 floats longer than they are, which spreads a fragment's 64 reads over the banks.
 #define MF_LA_VS (64 + 4)     // row stride of tiles of 64 columns
 
+__host__ __device__ constexpr int la_max(int a, int b) { return a > b ? a : b; }
+
 // Staging of a [MF_LA_CHUNK][W] tile of 32-bit rows into LDS, silu applied or not: rows tt >= n and
 // columns beyond `valid` are zero.  With `vec` (every row start and `valid` multiples of 4 floats) a thread's
 // loads are 16 bytes each and all issued before the first is used.
@@ -439,7 +441,9 @@ __global__ __launch_bounds__(256) void lightning_chunk_fold_kernel(const int* __
 // First the decayed scores a[t][s] = decay^(t - s) (q_t . k_s), s <= t, tile by tile (the tiles above the
 // diagonal are neither formed nor read), then for every 16 tokens x 16 columns
 // o = decay^(t + 1) (Q S_in) + a V: the first product's sums are scaled row by row before the second
-// product adds onto them.
+// product adds onto them.  A wave's columns of S_in and V are no other wave's and come straight into its registers, asked for
+// with the rest, and the scores take the keys' place, so that two workgroups (68 KB each at 128 values a head) share a CU and
+// one's loads run under the other's products (2,048 tokens, 16 heads of 128 x 128: memory 76 -> 54 us, decays 66 -> 45).
 template <int DS, int KIND>
 __global__ __launch_bounds__(256) void lightning_chunk_out_kernel(const float* __restrict__ proj, int row_len,
                                                                   const int* __restrict__ chunk_t0,
@@ -454,11 +458,9 @@ __global__ __launch_bounds__(256) void lightning_chunk_out_kernel(const float* _
   __shared__ float s_take[MF_LA_CHUNK];
   extern __shared__ float lds[];
   float* sq = lds;                                   // [CHUNK][DPS]
-  float* sk = sq + MF_LA_CHUNK * DPS;                 // [CHUNK][DPS]
-  float* sa = sk + MF_LA_CHUNK * DPS;                 // [CHUNK][VS]: decayed scores
-  float* sv = sa + MF_LA_CHUNK * MF_LA_VS;            // [CHUNK][VS]
-  float* ss = sv + MF_LA_CHUNK * MF_LA_VS;            // [DP][VS]: S_in of this head and these columns
-  float* dpow = ss + DP * MF_LA_VS;                   // [CHUNK + 1]: decay^i; what S_in is worth after i tokens
+  float* sk = sq + MF_LA_CHUNK * DPS;                 // [CHUNK][DPS], then
+  float* sa = sk;                                    // [CHUNK][VS]: decayed scores
+  float* dpow = sk + MF_LA_CHUNK * la_max(DPS, MF_LA_VS);     // [CHUNK + 1]: decay^i; what S_in is worth after i tokens
   const int c = blockIdx.x, h = blockIdx.y, v0 = blockIdx.z * 64;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int t0 = chunk_t0[c], n = chunk_n[c];
@@ -466,10 +468,21 @@ __global__ __launch_bounds__(256) void lightning_chunk_out_kernel(const float* _
   const int off_k = H * D, off_v = 2 * H * D;
   const bool vec = D % 4 == 0 && V % 4 == 0 && row_len % 4 == 0;
   const float* rows = proj + (size_t)t0 * row_len;
+  const int col = lane & 15, g = lane >> 4, cc = v0 + 16 * w + col;
+  // the second operands of the output's products: S_in and v at column cc, rows 4 i + g
+  float sf[DP / 4], vf[MF_LA_CHUNK / 4];
+  const float* s_col = s_in + (((size_t)c * H + h) * D) * V + cc;
+#pragma unroll
+  for (int i = 0; i < DP / 4; ++i) sf[i] = 4 * i + g < D && cc < V ? s_col[(size_t)(4 * i + g) * V] : 0.f;
+#pragma unroll
+  for (int i = 0; i < MF_LA_CHUNK / 4; ++i)
+    vf[i] = 4 * i + g < n && cc < V ? rows[(size_t)(4 * i + g) * row_len + off_v + h * V + cc] : 0.f;
   stage_tile<DP, SILU>(sq, DPS, rows + h * D, row_len, MF_LA_CHUNK, n, D, vec, SILU ? 1.f : ex.q_scale);
   stage_tile<DP, SILU>(sk, DPS, rows + off_k + h * D, row_len, MF_LA_CHUNK, n, D, vec, SILU ? 1.f : ex.k_scale);
-  stage_tile<64, SILU>(sv, MF_LA_VS, rows + off_v + h * V + v0, row_len, MF_LA_CHUNK, n, min(64, V - v0), vec);
-  stage_tile<64, false>(ss, MF_LA_VS, s_in + (((size_t)c * H + h) * D) * V + v0, V, DP, D, min(64, V - v0), vec);
+  if (SILU) {
+#pragma unroll
+    for (int i = 0; i < MF_LA_CHUNK / 4; ++i) vf[i] = la_silu(vf[i]);
+  }
   if (KIND == MF_LA_MEMORY) {
     if (threadIdx.x < MF_LA_CHUNK) {
       // (tokens beyond the chunk's weigh nothing: their v is zero, and no output row reads their scores)
@@ -482,12 +495,17 @@ __global__ __launch_bounds__(256) void lightning_chunk_out_kernel(const float* _
     dpow[threadIdx.x] = powf(decay, (float)threadIdx.x);
   }
   __syncthreads();
-  const int col = lane & 15, g = lane >> 4;
   // the ten score tiles on and below the diagonal, in turn over the waves
-  for (int tile = w; tile < 10; tile += 4) {
-    int ti = 0, rest = tile;
-    while (rest > ti) { rest -= ti + 1; ++ti; }       // tile -> (ti, sj = rest), sj <= ti
-    const int sj = rest;
+  floatx4 scores[3];
+  auto tile_of = [](int tile, int& ti, int& sj) {       // tile -> (ti, sj), sj <= ti
+    ti = tile < 1 ? 0 : tile < 3 ? 1 : tile < 6 ? 2 : 3;
+    sj = tile - ti * (ti + 1) / 2;
+  };
+#pragma unroll
+  for (int u = 0; u < 3; ++u) {
+    if (w + 4 * u >= 10) continue;
+    int ti, sj;
+    tile_of(w + 4 * u, ti, sj);
     floatx4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 4
     for (int kk = 0; kk < DP / 4; ++kk)
@@ -500,8 +518,17 @@ __global__ __launch_bounds__(256) void lightning_chunk_out_kernel(const float* _
       float weight = 0.f;
       if (sidx <= t)
         weight = KIND == MF_LA_MEMORY ? (t < n ? expf((float)(s_decay[t] - s_decay[sidx]) + s_take[sidx]) : 0.f) : dpow[t - sidx];
-      sa[t * MF_LA_VS + sidx] = acc[r] * weight;
+      scores[u][r] = acc[r] * weight;
     }
+  }
+  __syncthreads();                                      // (the last read of the keys)
+#pragma unroll
+  for (int u = 0; u < 3; ++u) {
+    if (w + 4 * u >= 10) continue;
+    int ti, sj;
+    tile_of(w + 4 * u, ti, sj);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) sa[(16 * ti + 4 * g + r) * MF_LA_VS + 16 * sj + col] = scores[u][r];
   }
   __syncthreads();
   if (KIND == MF_LA_MEMORY && blockIdx.z == 0) {
@@ -521,19 +548,18 @@ __global__ __launch_bounds__(256) void lightning_chunk_out_kernel(const float* _
       ex.floor[(size_t)(t0 + t) * H + h] = ex.gates[(size_t)(t0 + t) * H + h].floor;
     }
   }
-  const int cc = v0 + 16 * w + col;
-  for (int ti = 0; ti < MF_LA_CHUNK / 16 && 16 * ti < n; ++ti) {
+#pragma unroll
+  for (int ti = 0; ti < MF_LA_CHUNK / 16; ++ti) {
+    if (16 * ti >= n) break;
     floatx4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
+#pragma unroll
     for (int kk = 0; kk < DP / 4; ++kk)
-      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(sq[(16 * ti + col) * DPS + 4 * kk + g], ss[(4 * kk + g) * MF_LA_VS + 16 * w + col],
-                                                 acc, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(sq[(16 * ti + col) * DPS + 4 * kk + g], sf[kk], acc, 0, 0, 0);
 #pragma unroll
     for (int r = 0; r < 4; ++r) acc[r] *= dpow[16 * ti + 4 * g + r + 1];
-#pragma unroll 4
+#pragma unroll
     for (int kk = 0; kk < 4 * (ti + 1); ++kk)
-      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(sa[(16 * ti + col) * MF_LA_VS + 4 * kk + g], sv[(4 * kk + g) * MF_LA_VS + 16 * w + col],
-                                                 acc, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(sa[(16 * ti + col) * MF_LA_VS + 4 * kk + g], vf[kk], acc, 0, 0, 0);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int t = 16 * ti + 4 * g + r;
@@ -643,8 +669,8 @@ int scan_chunks(const float* proj, int row_len, const int* chunks, int n_chunks,
   if (rc) return rc;
 #define MF_CALL(DS)                                                                                                   \
   {                                                                                                                   \
-    const size_t lds = sizeof(float) * (2 * MF_LA_CHUNK * (4 * DS + 4) + 2 * MF_LA_CHUNK * MF_LA_VS +                 \
-                                        4 * DS * MF_LA_VS + MF_LA_CHUNK + 1);                                         \
+    const size_t lds = sizeof(float) * (MF_LA_CHUNK * (4 * DS + 4) + MF_LA_CHUNK * la_max(4 * DS + 4, MF_LA_VS) +     \
+                                        MF_LA_CHUNK + 1);                                                             \
     static bool raised = false;                                                                                       \
     if (!raised && lds > 48 * 1024) {                                                                                 \
       rc = (int)hipFuncSetAttribute((const void*)lightning_chunk_out_kernel<DS, KIND>,                                \
