@@ -4,11 +4,12 @@
 // yusiwen/minfer; the reference's own matrix kernels are quantised and are not followed.)
 //
 // The kernels:
-//  * `tile_kernel`: many rows (prompts).  A BM x BN block tile per 4 or 8 waves, K walked in
-//    steps of BK through double-buffered LDS, 32x32x16 MFMA, each wave a WM x WN tile.
-//  * `tile_dma_kernel`: tiles of 256 x 256, 256 x 192 or 256 x 128 with their k tiles copied
-//    straight into LDS; the choice for large aligned products (the width by how the tiles fill
-//    the chip's rounds).
+//  * `tile_dma_kernel`: many rows (prompts), aligned operands: tiles of 256 x 256, 256 x 192, 256 x 128 or 128 x 256 with
+//    their k tiles copied straight into LDS, 16x16x32 MFMA, two groups of four waves a quarter product apart.
+//  * `tile_step_kernel`: the same copies for tiles of 128 x 128 and 64 x 64 (fewer rows, and 17 to 64 rows against a short
+//    K), one barrier a k tile.
+//  * `tile_kernel`: many rows of any alignment, through registers and double-buffered LDS, 32x32x16 MFMA.
+//  * `reduce_norm_kernel`: adds the parts of a K split into the stream and norms the new rows.
 //  * `stationary16_kernel`: at most 16 rows and K of 896, 1536, 2048, 3584, 4096, 5120 or 8192 (decode):
 //    one block per CU keeps the activations in registers and walks over weight tiles.
 //  * `rolling16_kernel`, `skinny16_kernel`: at most 16 rows, any K (decode).  The time is the
