@@ -73,13 +73,18 @@ __device__ __forceinline__ float fast_tanh(float y) {
   return fmaf(-2.0f, __builtin_amdgcn_rcpf(e + 1.0f), 1.0f);
 }
 
+// What a wave that takes RB heads keeps in registers: queries, 32 keys, sums, 32 keys' values, and scores and addresses (the
+// compiler's counts for sizes between 16 and 256 lie within 12 of it).
+constexpr int wave_registers(int rb) { return rb * D / 8 + D / 4 + rb * V / 4 + V / 4 + 64 + 16 * rb; }
+
 // A step is a chain (page, keys, scores, softmax, values) that one wave a SIMD leaves waiting most of the time, a tile's
-// last keys decide how long a launch takes, and a group's keys want to stay in one die's L2.  Two heads a wave and four waves
-// a tile, two of them on a SIMD (256 registers: so the next keys go where this step's were), every group on its dies: 16 heads
-// of 128 over two kv heads, 2,048 tokens 144 -> 78 us, over 16 kv heads 237 -> 129; 8,192 tokens over four 1,350 -> 940; 203
-// tokens 15.6 -> 11.
+// last keys decide how long a launch takes, and a group's keys want to stay in one die's L2.  Several waves a tile, two of them
+// on a SIMD where 256 registers hold one (so the next keys go where this step's were; two heads of 128, one of 192), every
+// group on its dies: 16 heads of 128 over two kv heads, 2,048 tokens 144 -> 78 us, over 16 kv heads 237 -> 129; 203 tokens
+// 15.6 -> 11.  Wider heads have a SIMD to themselves: in 256 registers two heads of 192 spill 146 (2,048 tokens over two kv
+// heads 220 us so, 124 in 512), two of 128 with values of 256 190.
 template <int RB, int WK>
-__global__ __launch_bounds__(64 * WK, WK > 1 ? 2 : 1) void capped_mfma_kernel(
+__global__ __launch_bounds__(64 * WK, WK > 1 && wave_registers(RB) <= 256 ? 2 : 1) void capped_mfma_kernel(
     const bf16* __restrict__ q, const bf16* __restrict__ kc, const bf16* __restrict__ vc,
     const int* __restrict__ page_table, int pt_stride, const int* __restrict__ cu_seqlens,
     const int* __restrict__ start_pos, const int* __restrict__ tile_seq, const int* __restrict__ tile_q0, int n_tiles,
@@ -400,38 +405,37 @@ MF_API int mf_capped_mfma_sizes(int* d, int* v) {
   return 0;
 }
 
-// tiles: blocks of 16 consecutive new tokens of a sequence (tile_seq, tile_q0), n_tiles of them
+// tiles: blocks of 16 consecutive new tokens of a sequence (tile_seq, tile_q0), n_tiles of them; heads: of a kv head that a
+// wave takes together; waves: of a tile (one where the tiles' keys are split)
 MF_API int mf_capped_mfma(const void* q, const void* kc, const void* vc, const int* page_table, int pt_stride,
                           const int* cu_seqlens, const int* start_pos, const int* tile_seq, const int* tile_q0,
                           int n_tiles, const float* temp, void* out, float* part, int n_splits, int split_len, int n_tok,
                           int nh, int nk, int d, int v, float scale, float cap, int window, int chunk, const float* far_a,
-                          const float* far_b, int keep_first, const float* bias, int n_bias, const float* sink,
-                          hipStream_t stream) {
+                          const float* far_b, int keep_first, const float* bias, int n_bias, const float* sink, int heads,
+                          int waves, hipStream_t stream) {
   if (n_tiles <= 0) return 0;
   if (d != D || v != V || nk <= 0 || nh % nk || !temp || n_splits < 1 || n_splits > 64 ||
-      (n_splits > 1 && (!part || split_len < 32 || split_len % 32)) || chunk < 0 ||
-      (far_b && !far_a) || keep_first < 0 || (keep_first > 0 && chunk > 0) || (bias && n_bias < 1))
+      (n_splits > 1 && (!part || split_len < 32 || split_len % 32 || waves != 1)) || chunk < 0 ||
+      (far_b && !far_a) || keep_first < 0 || (keep_first > 0 && chunk > 0) || (bias && n_bias < 1) || heads <= 0 ||
+      (nh / nk) % heads)
     return (int)hipErrorInvalidValue;
   if (!bias) n_bias = 1;
-  const int G = nh / nk;
-  // heads of a kv head a wave takes together: four where that still leaves waves for all SIMDs
-  int rb = G % 2 == 0 ? 2 : 1;
-  if (G % 4 == 0 && (long long)n_tiles * nk * (G / 4) >= 4096) rb = 4;
-  // waves a tile: four, but one where the tiles' keys are split already and for four heads (whose sums leave no registers
-  // for a second wave a SIMD; 16 heads over four kv heads, four heads a wave / two heads and four waves: 8,192 tokens 873 /
-  // 940 us, 12,000 2,038 / 1,966, 16,384 3,410 / 3,616)
-  const int wk = n_splits == 1 && rb <= 2 ? 4 : 1;
-  dim3 grid((n_tiles * nk * (G / rb) + 7) / 8 * 8, 1, n_splits);          // (whole rounds of the eight dies)
+  dim3 grid((n_tiles * (nh / heads) + 7) / 8 * 8, 1, n_splits);          // (whole rounds of the eight dies)
 #define MF_GO(RB, WK)                                                                                                      \
   capped_mfma_kernel<RB, WK><<<grid, 64 * WK, 0, stream>>>((const bf16*)q, (const bf16*)kc, (const bf16*)vc, page_table, pt_stride, \
                                                    cu_seqlens, start_pos, tile_seq, tile_q0, n_tiles, temp, (bf16*)out, part, \
                                                    n_splits, split_len, nh, nk, scale, cap, window, chunk, far_a, far_b, \
                                                    keep_first, bias, n_bias, sink)
-  if (rb == 4) MF_GO(4, 1);
-  else if (rb == 2 && wk == 4) MF_GO(2, 4);
-  else if (rb == 2) MF_GO(2, 1);
-  else if (wk == 4) MF_GO(1, 4);
-  else MF_GO(1, 1);
+  switch (heads * 8 + waves) {
+    case 4 * 8 + 1: MF_GO(4, 1); break;
+    case 2 * 8 + 4: MF_GO(2, 4); break;
+    case 2 * 8 + 2: MF_GO(2, 2); break;
+    case 2 * 8 + 1: MF_GO(2, 1); break;
+    case 1 * 8 + 4: MF_GO(1, 4); break;
+    case 1 * 8 + 2: MF_GO(1, 2); break;
+    case 1 * 8 + 1: MF_GO(1, 1); break;
+    default: return (int)hipErrorInvalidValue;
+  }
 #undef MF_GO
   int rc = mf_launch_status();
   if (rc == 0 && n_splits > 1) {

@@ -68,6 +68,23 @@ class StepContext:
             self._memo[key] = (both[0], both[1])
         return self._memo[key]
 
+    def keys_in_sight(self, window: int = 0, chunk: int = 0):
+        """(mean, most) keys that the step's new tokens see, from the host's copy of the step: how even a launch's work is
+        and how long its longest walk.  `window`, `chunk`: 0 for none; with chunks the mean is rough (half a chunk)."""
+        key = ("keys_in_sight", window, chunk)
+        if key not in self._memo:
+            reach = min(window or self.max_len, chunk or self.max_len)
+            if self.host_start is None:                                   # (a decode step: the bound is all there is)
+                self._memo[key] = (min(self.max_len, reach),) * 2
+            else:
+                total = 0.0
+                for n, s in zip(self.host_new, self.host_start):
+                    short = min(n, max(0, (window or s + n) - s))         # tokens that see all before them, then full windows
+                    keys = short * (s + 0.5 * (short + 1)) + (n - short) * window
+                    total += min(keys, 0.5 * n * chunk) if chunk else keys
+                self._memo[key] = (total / max(1, self.n_tokens), min(self.max_len, reach))
+        return self._memo[key]
+
     def shared_query_tiles(self, block: int, page: int, window: int, n_heads: int, n_cu: int, per_cu: int,
                            min_pages: int, max_shares: int, min_imbalance: float = 1.5):
         """(tile_seq, tile_q0, tile_share, n_slots, most shares): as `query_tiles`, but a block of queries with

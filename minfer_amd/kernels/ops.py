@@ -77,7 +77,7 @@ _PROTOTYPES = {
     },
     "attn_capped_mfma": {
         "mf_capped_mfma": [_P, _P, _P, _P, c_int, _P, _P, _P, _P, c_int, _P, _P, _P, c_int, c_int, c_int, c_int, c_int, c_int,
-                           c_int, c_float, c_float, c_int, c_int, _P, _P, c_int, _P, c_int, _P, _P],
+                           c_int, c_float, c_float, c_int, c_int, _P, _P, c_int, _P, c_int, _P, c_int, c_int, _P],
     },
     "attn_normed": {
         "mf_qk_norm_prep": [_P, _P, _P, c_float, c_int, _P, _P, _P, _P, c_int, c_int, c_int, _P, _P, c_int, _P, c_int, _P, _P, _P,
@@ -1276,6 +1276,45 @@ def capped_mfma_takes(dtype, dim: int, v_dim: int) -> bool:
     return dtype == torch.bfloat16 and dim % 16 == 0 and v_dim % 16 == 0 and 16 <= dim <= 256 and 16 <= v_dim <= 256
 
 
+def _capped_registers(heads: int, dim: int, v_dim: int) -> int:
+    """Registers of a wave of the matrix-core form with so many heads (`wave_registers` in csrc/attn_capped_mfma.hip)."""
+    return heads * dim // 8 + dim // 4 + heads * v_dim // 4 + v_dim // 4 + 64 + 16 * heads
+
+
+def capped_form(n_tiles: int, n_heads: int, n_kv_heads: int, dim: int, v_dim: int, mean_keys: float, most_keys: int,
+                n_cu: Optional[int] = None) -> Tuple[int, int]:
+    """(heads a wave, waves a tile) of the matrix-core form without key splits, for tiles that see `mean_keys` keys on
+    average and `most_keys` at most.
+
+    Heads: two where the group is even and a SIMD's 512 registers hold them (up to 224 values; at 256 and 256 two heads spill
+    94 of them: 2,048 tokens of 16 heads over two kv heads 488 us, 239 one by one).  Four of them where a group has them and
+    there are waves for all SIMDs all the same.
+
+    Waves: several finish a tile sooner, each pays for its own start and end, and they share a SIMD only where 256 registers
+    hold one.  Four where they do.  Where they do not, the least estimate in steps of 32 keys: a wave's own walk, or the
+    chip's rounds of walks (whole rounds where all walks are alike); two heads of 192 over two kv heads, one / two / four
+    waves: 1,000 tokens 95 / 53 / 42 us, 2,048 171 / 105 / 124, 4,096 366 / 373 / 423, 16 prompts of 1,000 399 / 462 / 606."""
+    group = n_heads // n_kv_heads
+    heads = 2 if group % 2 == 0 and _capped_registers(2, dim, v_dim) <= 376 else 1
+    narrow = _capped_registers(heads, dim, v_dim) <= 256
+    if group % 4 == 0 and n_tiles * n_heads >= 4 * 4096 and (narrow or dim >= 2 * v_dim and
+                                                             _capped_registers(4, dim, v_dim) <= 400):
+        return 4, 1
+    if narrow:
+        return heads, 4
+    walks, slots = n_tiles * n_heads // heads, 4 * (n_cu or cu_count())
+    mean, most = -(-mean_keys // 32), -(-most_keys // 32)
+    best, best_steps = 4, 0.0
+    for waves, start in ((4, 2.0), (2, 3.0), (1, 2.5)):
+        if most < 1.25 * mean:
+            steps = -(-walks * waves // slots) * (-(-mean // waves) + start)
+        else:
+            steps = max(most / waves + start, walks * waves * (mean / waves + start) / slots)
+        if not best_steps or steps < 0.95 * best_steps:
+            best, best_steps = waves, steps
+    return heads, best
+
+
 def capped_attn_prefill(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor, page_table: torch.Tensor, ctx,
                         temp: torch.Tensor, out: torch.Tensor, n_heads: int, n_kv_heads: int, dim: int, v_dim: int,
                         scale: float, cap: float, window: int, chunk: int = 0, far=None, keep_first: int = 0,
@@ -1303,6 +1342,7 @@ def capped_attn_prefill(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Ten
         _need(sink, "capped_attn_prefill.sink", torch.float32, (n_heads,))
     keep_first, n_bias = _kept_and_bias("capped_attn_prefill", keep_first, window, chunk, bias, n_heads)
     n_splits, split_len, part = 1, 0, None
+    form = None
     if ctx.all_decode:
         # every sequence is a tile of one token; nothing comes from the host (the step may be captured)
         tile_seq = ctx.seq_of_tok
@@ -1316,14 +1356,17 @@ def capped_attn_prefill(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Ten
         n_splits = (reach + 31 + split_len - 1) // split_len
         if n_splits > 1:
             part = workspace("attn", n_tok * n_heads * n_splits * (v_dim + 2), q.device)
+            form = (1 + (n_heads // n_kv_heads + 1) % 2, 1)
     else:
         tile_seq, tile_q0 = ctx.query_tiles(CAPPED_MFMA_ROWS)
+    if form is None:
+        form = capped_form(tile_seq.numel(), n_heads, n_kv_heads, dim, v_dim, *ctx.keys_in_sight(int(window or 0) + keep_first, int(chunk or 0)))
     lib = build.variant("attn_capped_mfma", MF_CAPM_D=dim, MF_CAPM_V=v_dim)
     _check(_fn("attn_capped_mfma", "mf_capped_mfma", lib)(
         _ptr(q), _ptr(kcache), _ptr(vcache), _ptr(page_table), page_table.shape[1], _ptr(ctx.cu_seqlens),
         _ptr(ctx.start_pos), _ptr(tile_seq), _ptr(tile_q0), tile_seq.numel(), _ptr(temp), _ptr(out), _ptr(part), n_splits,
         split_len, n_tok, n_heads, n_kv_heads, dim, v_dim, float(scale), float(cap or 0.0), int(window or 0),
-        int(chunk or 0), _ptr(far_a), _ptr(far_b), keep_first, _ptr(bias), n_bias, _ptr(sink), _stream()),
+        int(chunk or 0), _ptr(far_a), _ptr(far_b), keep_first, _ptr(bias), n_bias, _ptr(sink), form[0], form[1], _stream()),
         "capped_attn_decode" if ctx.all_decode else "capped_attn_prefill")
 
 

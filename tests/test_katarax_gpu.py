@@ -111,6 +111,19 @@ def test_window_kept_first_positions_and_bias_in_both_attention_kernels(form, dt
     assert torch.isfinite(got).all() and err < (2e-5 if dtype == torch.float32 else 4e-2), float(err)
 
 
+# heads a wave x waves a tile, as a plan may choose them, at a narrow size and at the widest
+@pytest.mark.parametrize("form", [(1, 1), (1, 2), (1, 4), (2, 1), (2, 2), (2, 4), (4, 1)])
+@pytest.mark.parametrize("H, G, D, V, window, keep, n_bias", [(8, 2, 96, 48, 0, 0, 40), (8, 2, 128, 64, 70, 5, 300), (4, 2, 256, 256, 40, 3, 50)])
+@pytest.mark.parametrize("new", [(1, 130, 3, 1, 40), (1, 64, 64, 300, 65)])
+def test_every_form_of_the_matrix_core_attention(monkeypatch, form, H, G, D, V, window, keep, n_bias, new):
+    """The same bound as above, for the forms that the sizes there do not choose by themselves."""
+    from minfer_amd.kernels import ops
+    if H // G % form[0]:
+        pytest.skip("a group has no such number of heads")
+    monkeypatch.setattr(ops, "capped_form", lambda *a, **k: form)
+    test_window_kept_first_positions_and_bias_in_both_attention_kernels("matrix cores", torch.bfloat16, H, G, D, V, window, keep, n_bias, new)
+
+
 # the last query stands at position 299: (window, kept first positions, the key's position, seen or not)
 EDGES = [(17, 0, 283, True), (17, 0, 282, False), (64, 4, 236, True), (64, 4, 235, False), (64, 4, 3, True), (64, 4, 4, False),
          (65, 1, 0, True), (65, 1, 1, False), (100, 64, 63, True), (100, 64, 64, False), (100, 70, 69, True), (100, 70, 70, False),

@@ -1,6 +1,11 @@
 """The launch plans are plain functions of shapes: what the kernels' host checks rely on holds
 for every shape (no empty split, whole chunks and pages, bounds on the number of splits)."""
 import itertools
+import os
+import re
+import subprocess
+
+import pytest
 
 from minfer_amd.kernels import ops
 
@@ -199,3 +204,55 @@ def test_skinny_plan_keeps_a_small_matrix_in_one_kernel():
     assert ops.skinny_plan(8, 2048, 11008, target_blocks=256, tiled=True)[0] == 1      # the 3B shape's down product
     assert ops.skinny_plan(16, 2048, 11008, target_blocks=256, tiled=True)[0] > 1
     assert ops.skinny_plan(8, 5120, 13824, target_blocks=256, tiled=True)[0] > 1       # the 14B shape's: 141 MB
+
+
+def test_capped_form_of_wide_heads():
+    """Heads too wide for two waves a SIMD (192 and more of keys and values together in pairs): no form of four waves where
+    there are walks for every SIMD anyway, one head a wave where two would not fit a SIMD at all; narrow heads keep four waves."""
+    form = lambda tiles, h, kv, d, v, mean, most: ops.capped_form(tiles, h, kv, d, v, mean, most, n_cu=256)
+    for d, v in ((192, 192), (256, 128), (128, 256), (160, 160)):
+        assert form(16 * 63, 16, 2, d, v, 500, 1000) == (2, 1)          # sixteen prompts of 1,000 tokens
+        assert form(128, 16, 2, d, v, 512, 512) == (2, 1)               # 2,048 tokens, a window of 512: one round
+        assert form(63, 16, 2, d, v, 500, 1000) == (2, 4)               # 1,000 tokens
+        assert form(13, 16, 16, d, v, 102, 203)[0] == 1
+    assert form(63, 16, 2, 256, 256, 500, 1000)[0] == 1 and form(63, 16, 2, 224, 224, 500, 1000)[0] == 2
+    assert form(63, 16, 2, 128, 128, 500, 1000) == (2, 4) and form(63, 16, 16, 128, 128, 500, 1000) == (1, 4)
+    assert form(16 * 63, 32, 4, 256, 64, 500, 1000) == (4, 1) and form(16 * 63, 32, 4, 256, 128, 500, 1000) == (2, 1)
+
+
+def test_keys_in_sight():
+    """Mean and most keys of a step's new tokens, against a count over the tokens."""
+    import torch
+    from minfer_amd.engine.batch import StepContext
+    for new, start, window in (([5, 300], [0, 40], 0), ([100], [0], 64), ([7, 900], [500, 30], 128), ([1, 1], [10, 99], 50)):
+        n, top = sum(new), max(a + b for a, b in zip(new, start))
+        c = StepContext(cache=None, n_tokens=n, n_seqs=len(new), token_ids=torch.zeros(n, dtype=torch.int32), positions=None,
+                        seq_of_tok=None, cu_seqlens=None, start_pos=None, slot_ids=None, logit_rows=None, page_tables={},
+                        max_len=top, max_new=max(new), all_decode=False, host_new=list(new), host_start=list(start))
+        keys = [min(s + i + 1, window or top) for k, s in zip(new, start) for i in range(k)]
+        mean, most = c.keys_in_sight(window)
+        assert abs(mean - sum(keys) / n) < 0.5 and most == min(top, window or top)
+        assert c.keys_in_sight(0, 64)[0] <= 32 and c.keys_in_sight(0, 64)[1] == min(top, 64)
+
+
+# the sizes at which two heads a wave stop to fit 256 registers, and 512; one head at the largest
+@pytest.mark.parametrize("dim,v_dim", [(128, 128), (192, 80), (160, 160), (192, 192), (256, 128), (224, 224), (256, 256)])
+def test_capped_forms_keep_to_their_registers(dim, v_dim):
+    """The compiler's own report of the matrix-core attention: of the forms that a plan may choose at a size (heads a wave up
+    to what `capped_form` takes, any number of waves), none with one or two heads spills a register."""
+    from minfer_amd.kernels import build
+    flags = [f for f in build.HIPCC_FLAGS if f != "-shared"]
+    out = subprocess.run([build._hipcc(), *flags, f"-DMF_CAPM_D={dim}", f"-DMF_CAPM_V={v_dim}", "-I", build.CSRC, "-c", "--cuda-device-only",
+                          "-Rpass-analysis=kernel-resource-usage", os.path.join(build.CSRC, "attn_capped_mfma.hip"), "-o", os.devnull],
+                         capture_output=True, text=True)
+    assert out.returncode == 0, out.stderr[-2000:]
+    spills, form = {}, None
+    for line in out.stderr.splitlines():
+        if "Function Name" in line:
+            m = re.search(r"capped_mfma_kernelILi(\d)ELi(\d)E", line)
+            form = (int(m.group(1)), int(m.group(2))) if m else None
+        elif form and "VGPRs Spill:" in line:
+            spills[form] = int(re.search(r"VGPRs Spill: (\d+)", line).group(1))
+    heads = ops.capped_form(13, 2, 1, dim, v_dim, 100, 203, n_cu=256)[0]
+    assert (heads, 1) in spills and (heads, 4) in spills and (1, 4) in spills
+    assert not {f: n for f, n in spills.items() if f[0] <= heads and n}, spills
