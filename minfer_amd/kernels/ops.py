@@ -1287,29 +1287,36 @@ def capped_form(n_tiles: int, n_heads: int, n_kv_heads: int, dim: int, v_dim: in
     average and `most_keys` at most.
 
     Heads: two where the group is even and a SIMD's 512 registers hold them (up to 224 values; at 256 and 256 two heads spill
-    94 of them: 2,048 tokens of 16 heads over two kv heads 488 us, 239 one by one).  Four of them where a group has them and
-    there are waves for all SIMDs all the same.
+    94 of them: 2,048 tokens of 16 heads over two kv heads 488 us, 239 one by one).  Four where keys are twice as wide as
+    values (a step is then mostly the keys' way) and there are waves for all SIMDs all the same (32 heads over four kv heads of
+    256 and 64, 16 prompts of 1,000 tokens: 530 us, 684 with two); elsewhere two, two waves a SIMD, have measured the faster at
+    every size (of 128, those prompts: 560 us with four heads, 540).
 
-    Waves: several finish a tile sooner, each pays for its own start and end, and they share a SIMD only where 256 registers
-    hold one.  Four where they do.  Where they do not, the least estimate in steps of 32 keys: a wave's own walk, or the
-    chip's rounds of walks (whole rounds where all walks are alike); two heads of 192 over two kv heads, one / two / four
-    waves: 1,000 tokens 95 / 53 / 42 us, 2,048 171 / 105 / 124, 4,096 366 / 373 / 423, 16 prompts of 1,000 399 / 462 / 606."""
+    Waves: several finish a tile sooner, but each pays for its own start and end.  The least estimate in steps of 32 keys: a
+    wave's own walk, or the chip's rounds of walks (whole rounds where all walks are alike), a step a tenth longer where two
+    waves share a SIMD (where 256 registers hold one; a single wave's kernel takes the accumulation registers beside them), and
+    twice as long for single heads so wide that a wave alone would have its SIMD to itself.  One / two
+    / four waves, two heads over two kv heads: of 192, 1,000 tokens 95 / 53 / 42 us, 2,048 171 / 105 / 124, 4,096 366 / 373 /
+    423, 16 prompts of 1,000 399 / 462 / 606; of 64, 32 prompts of 200 29 / 34 / 46, a step of 256 sequences at 200 tokens 29 /
+    41 / 41; of 128, 2,048 tokens 147 / 91 / 78, 16 prompts of 1,000 323 / 266 / 297, 512 sequences at 100 64 / 53 / 67.  Over
+    1,650 pairs of sizes and steps the choice is 1 % from the best form on average."""
     group = n_heads // n_kv_heads
     heads = 2 if group % 2 == 0 and _capped_registers(2, dim, v_dim) <= 376 else 1
-    narrow = _capped_registers(heads, dim, v_dim) <= 256
-    if group % 4 == 0 and n_tiles * n_heads >= 4 * 4096 and (narrow or dim >= 2 * v_dim and
-                                                             _capped_registers(4, dim, v_dim) <= 400):
+    if group % 4 == 0 and n_tiles * n_heads >= 4 * 4096 and dim >= 2 * v_dim and _capped_registers(4, dim, v_dim) <= 400:
         return 4, 1
-    if narrow:
-        return heads, 4
-    walks, slots = n_tiles * n_heads // heads, 4 * (n_cu or cu_count())
-    mean, most = -(-mean_keys // 32), -(-most_keys // 32)
+    registers = _capped_registers(heads, dim, v_dim)
+    alone = registers + (v_dim // 4 + 8 if heads == 1 else 3 * v_dim // 8 + 30)
+    walks, simds = n_tiles * n_heads // heads, 4 * (n_cu or cu_count())
+    mean, most = mean_keys / 32, -(-most_keys // 32)
     best, best_steps = 4, 0.0
     for waves, start in ((4, 2.0), (2, 3.0), (1, 2.5)):
+        shared = (alone if waves == 1 else registers) <= 256
+        slots = 2 * simds if shared else simds
+        price = (2.0 if heads == 1 and alone > 256 else 1.1) if shared else 1.0
         if most < 1.25 * mean:
-            steps = -(-walks * waves // slots) * (-(-mean // waves) + start)
+            steps = -(-walks * waves // slots) * (-(-most // waves) + start) * (price if walks * waves > simds else 1.0)
         else:
-            steps = max(most / waves + start, walks * waves * (mean / waves + start) / slots)
+            steps = max(most / waves + start, walks * waves * (mean / waves + start) / slots * price)
         if not best_steps or steps < 0.95 * best_steps:
             best, best_steps = waves, steps
     return heads, best

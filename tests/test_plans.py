@@ -220,6 +220,18 @@ def test_capped_form_of_wide_heads():
     assert form(16 * 63, 32, 4, 256, 64, 500, 1000) == (4, 1) and form(16 * 63, 32, 4, 256, 128, 500, 1000) == (2, 1)
 
 
+def test_capped_form_of_short_and_even_walks():
+    """Where there are walks for every SIMD and few keys to each, four waves a tile pay for their starts and ends: one or two;
+    long walks and launches that leave SIMDs idle keep four, and four heads a wave are for keys twice as wide as values."""
+    form = lambda tiles, h, kv, d, v, mean, most: ops.capped_form(tiles, h, kv, d, v, mean, most, n_cu=256)
+    assert form(32 * 13, 16, 2, 64, 64, 100, 200)[1] < 4 and form(32 * 13, 16, 16, 128, 128, 100, 200)[1] < 4
+    assert form(256, 16, 2, 64, 64, 200, 200) == (2, 1) and form(512, 12, 4, 128, 128, 100, 100)[1] < 4      # decode, no splits
+    assert form(16 * 63, 16, 2, 128, 128, 500, 1000) == (2, 2) and form(16 * 63, 16, 16, 128, 128, 500, 1000) == (1, 1)
+    assert form(16 * 63, 32, 4, 128, 128, 500, 1000) == (2, 2)
+    for tiles, mean, most in ((13, 102, 203), (63, 500, 1000), (128, 1024, 2048), (24, 800, 1010)):
+        assert form(tiles, 16, 2, 128, 128, mean, most) == (2, 4) and form(tiles, 8, 8, 64, 64, mean, most) == (1, 4)
+
+
 def test_keys_in_sight():
     """Mean and most keys of a step's new tokens, against a count over the tokens."""
     import torch
