@@ -2471,14 +2471,23 @@ TilePlan plan_tiles(int M, int N, int K, bool dma_ok, int epi, int n_cu) {
   const long nkt = (K + 63) / 64, chunks = (K + 255) / 256;
   const double mn = (double)M * (double)N;
   const double epi_us = (epi == EPI_ACC_F32 ? 8. : epi == EPI_F32 ? 4. : (epi == EPI_BF16 || epi == EPI_XIELU) ? 2. : 1.) * mn / 4e6;
-  const double start_us = dma_ok ? 4. : 12.;
+  // The kernels through registers have costs of their own: a launch's epilogue is a chain (SwiGLU's stores 4 us, of 16 or 32
+  // bits 7, a read and a store 25), the second kernel of a SwiGLU product adds its parts one value at a time, and rows that are
+  // no whole 16 bytes are read in eights of single values.  1,888 products of K not in 64s, from 65 x 192 x 100 on: the choice is
+  // 0.5 % from the best kernel on average; with the costs of the direct-to-LDS kernels 1.3 %, and SwiGLU of 200 rows against
+  // 8,000 of 1,000 34.7 us in two parts for 21.2 whole.
+  const double start_us = dma_ok ? 4. : epi == EPI_ACC_F32 ? 25. : epi == EPI_SWIGLU ? 4. : 7.;
+  const double slow = K % 8 ? 4. : 1.;
   auto tiles = [&](int bm, int bn) { return (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
   auto cut = [&](long parts, int& splits, int& per) {          // K in `parts` runs of whole chunks of 256
     const long c = (chunks + parts - 1) / parts;
     splits = (int)((chunks + c - 1) / c);
     per = (int)(c * 256);
   };
-  auto parts_us = [&](int splits) { return (double)(splits + 2) * mn * 4. / 6e6 + 4.; };
+  auto parts_us = [&](int splits) {                            // the start of both kernels and the parts' way
+    const double bytes = (double)(splits + 2) * mn * 4.;
+    return dma_ok ? bytes / 6e6 + 8. : bytes / (epi == EPI_SWIGLU ? 3e6 : 8e6) + 14.25;
+  };
   TilePlan best{0, 1, K, 1e30};
   auto offer = [&](int variant, int splits, int per, double us) {
     if (us < best.us) best = TilePlan{variant, splits, per, us};
@@ -2497,12 +2506,12 @@ TilePlan plan_tiles(int M, int N, int K, bool dma_ok, int epi, int n_cu) {
         int splits, per;
         cut(parts, splits, per);
         if (splits < 2) continue;
-        offer(12, splits, per, form(12, splits, per / 64) + start_us + parts_us(splits));
+        offer(12, splits, per, form(12, splits, per / 64) + parts_us(splits));
       }
   } else {
-    offer(9, 1, K, rounds_us(tiles(256, 256), cu, 2.1, nkt, 0.) + start_us + epi_us);
+    offer(9, 1, K, rounds_us(tiles(256, 256), cu, 2.1 * slow, nkt, 0.) + start_us + epi_us);
     offer(M <= 64 && tiles(128, 128) < 64 && epi != EPI_SWIGLU ? 3 : 2, 1, K,
-          rounds_us(tiles(128, 128), 2 * cu, 1.45, nkt, 0.) + start_us + epi_us);
+          rounds_us(tiles(128, 128), 2 * cu, 1.45 * slow, nkt, 0.) + start_us + epi_us);
   }
   // a few hundred rows against a few thousand weight rows (some 50 tiles of 128 x 128, bound by
   // the weight stream): K over the chip, each part at least 512 of K
@@ -2512,8 +2521,8 @@ TilePlan plan_tiles(int M, int N, int K, bool dma_ok, int epi, int n_cu) {
       int splits, per;
       cut(parts, splits, per);
       if (splits < 2 || splits * t128 > 2 * cu) continue;
-      const double us = dma_ok ? form(2, splits, per / 64) : rounds_us(t128 * splits, 2 * cu, 1.45, per / 64, 0.);
-      offer(2, splits, per, us + start_us + parts_us(splits));
+      const double us = dma_ok ? form(2, splits, per / 64) : rounds_us(t128 * splits, 2 * cu, 1.45 * slow, per / 64, 0.);
+      offer(2, splits, per, us + parts_us(splits));
     }
   return best;
 }

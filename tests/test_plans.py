@@ -86,6 +86,22 @@ def test_decode_split_plan_bounds():
     assert ops.decode_split_plan(8, 4, 7, 4096, target_blocks=64) == (2, 2)        # a chip of 64 CUs splits less
 
 
+def test_tile_plan_of_k_not_in_64s():
+    """A product that cannot be copied straight into LDS is cut over K where its own kernels gain by it: not for the cheap
+    epilogues of a K of a thousand (200 x 8000 SwiGLU 21.2 us whole, 34.7 in two parts), for sums added to 32 bits at the
+    same sizes, and for any epilogue against a long K."""
+    splits = lambda m, n, k, epi: ops.tile_plan(m, n, k, epi, k % 8 == 0, n_cu=256)[1]
+    for m, n, k in ((200, 8000, 1000), (128, 8000, 1000), (2048, 512, 1000), (300, 4096, 1000), (700, 512, 808), (65, 4096, 808),
+                    (700, 4096, 2000)):
+        assert splits(m, n, k, ops.EPI_SWIGLU) == 1, (m, n, k)
+    for m, n, k in ((512, 3000, 1000), (1500, 1000, 1000), (700, 2000, 1000), (128, 12000, 1000), (300, 4096, 1000)):
+        assert splits(m, n, k, ops.EPI_BF16) == 1, (m, n, k)
+    for m, n, k in ((200, 200, 808), (128, 1000, 808), (65, 20000, 1000)):
+        assert splits(m, n, k, ops.EPI_ACC_F32) > 1, (m, n, k)
+    for epi in (ops.EPI_ACC_F32, ops.EPI_F32, ops.EPI_BF16, ops.EPI_SWIGLU):
+        assert splits(128, 1024, 5000, epi) > 1 and splits(65, 4096, 18000, epi) > 1
+
+
 def test_plan_linear_names_the_kernels_of_the_model_shapes():
     """Which kernel a product takes, as the library decides it (nothing is launched): the decode
     shapes of the 7B, 32B and 72B widths get the kernels the design describes, and widths off the
