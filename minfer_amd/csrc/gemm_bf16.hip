@@ -2536,12 +2536,19 @@ enum SkinnyChoice {
 // 17 to 64 rows against a short K: a tile of 64 x 64 over the whole of K, with the norm's factors, the bias and SwiGLU in its
 // epilogue, where the K-split kernels need a second one (32 to 40 rows, K-split and added / one tile kernel: gate|up 9,728 x 896
 // 15.0 / 9.0 us, 17,920 x 1,536 19.9 / 19.2, 22,016 x 2,048 28.3 / 26.6; q|k|v 1,152 x 896 11.6 / 9.0, 2,048 x 1,536 level).
-// At most two tiles a CU, all at once; fewer than eight tiles are a launch whichever kernel it is.
-bool tile64_takes(int M, int N, int K, bool aligned, int epi, int n_cu) {
-  return M > 16 && aligned && K % DMA_BK == 0 && N >= 512 && (N + 63) / 64 <= 2 * n_cu && K <= (epi == EPI_SWIGLU ? 2048 : 1024);
+// At most two tiles a CU, all at once; fewer than eight tiles are a launch whichever kernel it is.  A tile's chain over K is the
+// same however few rows and tiles there are, while the K-split kernels' two launches get shorter with them in the ring form with
+// the tiled copy to read: SwiGLU of 17 rows of 2,048 against 512 to 2,048 9.3 us so and 7.6 split, level where rows times weight
+// rows reach some 110,000 at that K and 22,000 at 1,536; with a second tile a CU and no SwiGLU to save, 17 rows against 24,576
+// of 768 10.9 us and 8.9, 48 rows 12.4 and 13.1 (12.2 so and 18.1 split without the copy).
+bool tile64_takes(int M, int N, int K, bool aligned, bool tiled, int epi, int n_cu) {
+  if (M <= 16 || !aligned || K % DMA_BK || N < 512 || (N + 63) / 64 > 2 * n_cu) return false;
+  const bool fast_split = tiled && K % 256 == 0;             // (`ring_takes`)
+  if (epi == EPI_SWIGLU) return K <= 2048 && (!fast_split || (long)M * N >= 176L * (K - 1408));
+  return K <= 1024 && (!fast_split || M > 32 || K <= 512 || N <= 64 * n_cu);
 }
 
-SkinnyChoice skinny_choice(int M, int N, int K, bool aligned, int epi, int splits, int k_per_split, int n_cu) {
+SkinnyChoice skinny_choice(int M, int N, int K, bool aligned, bool tiled, int epi, int splits, int k_per_split, int n_cu) {
   if (M <= 16 && splits == 1) {
     // the register-resident kernel where it is built; other aligned shapes the rolling K-split
     // kernel; the rest (and SwiGLU outside the first) the guarded kernel
@@ -2557,7 +2564,7 @@ SkinnyChoice skinny_choice(int M, int N, int K, bool aligned, int epi, int split
     return SK_GUARDED_8X1;
   }
   if (M > 16 && panel_takes(M, N, K, aligned, epi, n_cu)) return SK_PANEL;
-  if (tile64_takes(M, N, K, aligned, epi, n_cu)) return SK_TILE;
+  if (tile64_takes(M, N, K, aligned, tiled, epi, n_cu)) return SK_TILE;
   return ring_takes(aligned, K, splits, k_per_split) ? SK_RING : SK_STAGED;
 }
 
@@ -2716,7 +2723,7 @@ static int skinny_product(const void* A, int lda, const void* W, const void* Wt,
   const bf16* w = (const bf16*)W;
   const bf16* wt = (K % 32 == 0 && (uintptr_t)Wt % 16 == 0) ? (const bf16*)Wt : nullptr;
   const bool folds = fused.in_ssq || fused.out_g;
-  const SkinnyChoice choice = skinny_choice(M, N, K, vec_ok, epi, splits, k_per_split, cu_count());
+  const SkinnyChoice choice = skinny_choice(M, N, K, vec_ok, wt != nullptr, epi, splits, k_per_split, cu_count());
   // at most 16 rows: the register-resident kernel takes a prepared norm and prepares the next one, the
   // rolling kernel prepares the next one; the K-split kernels' second kernel counts its parts otherwise
   if (folds && M <= 16 && choice != SK_STATIONARY && choice != SK_RING && choice != SK_STAGED &&
@@ -2812,17 +2819,17 @@ MF_API int mf_gemm_bf16_tile_plan(int M, int N, int K, int aligned, int epi, int
 
 // The name of the kernel that a product of this shape takes, without launching anything: `rows`
 // activation rows against `N` weight rows of length `K`; `aligned`: 16-byte aligned operands with
-// row strides and K in multiples of 8; for at most 64 rows `splits`, `k_per_split`: the caller's K
+// row strides and K in multiples of 8; `tiled`: there is the tiled copy; for at most 64 rows `splits`, `k_per_split`: the caller's K
 // split (1, K for none); `normed`: the RMS norm is to be folded in (an empty name then means "no
 // such kernel": norm and product run one after the other); `n_cu`: compute units of the device.
-MF_API int mf_gemm_bf16_plan(int M, int N, int K, int aligned, int epi, int splits, int k_per_split,
+MF_API int mf_gemm_bf16_plan(int M, int N, int K, int aligned, int tiled, int epi, int splits, int k_per_split,
                              int normed, int n_cu, char* name, int cap) {
   if (!name || cap < 48 || M <= 0 || N <= 0 || K <= 0 || epi < 0 || epi > EPI_XIELU || n_cu <= 0) return (int)hipErrorInvalidValue;
   const char* what = "";
   if (normed) {
     what = (aligned && stationary_takes(M, N, K, epi, true)) ? "stationary16_kernel(norm)" : "";
   } else if (M <= 64) {
-    switch (skinny_choice(M, N, K, aligned != 0, epi, splits, k_per_split, n_cu)) {
+    switch (skinny_choice(M, N, K, aligned != 0, tiled != 0 && K % 32 == 0, epi, splits, k_per_split, n_cu)) {
       case SK_STATIONARY: what = "stationary16_kernel"; break;
       case SK_ROLLING: what = "rolling16_kernel"; break;
       case SK_GUARDED_PAIR: case SK_GUARDED_4X2: case SK_GUARDED_8X2: case SK_GUARDED_8X1: what = "skinny16_kernel"; break;

@@ -147,7 +147,7 @@ _PROTOTYPES = {
                                 c_int, _P],
         "mf_gemm_bf16_skinny_fused": [_P, c_int, _P, _P, c_int, _P, _P, c_int, _P, c_int, c_int, c_int, c_int,
                                       c_int, c_int, _P, c_int, c_float, _P, _P, _P, c_int, _P],
-        "mf_gemm_bf16_plan": [c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_char_p, c_int],
+        "mf_gemm_bf16_plan": [c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_char_p, c_int],
         "mf_gemm_bf16_tile_plan": [c_int, c_int, c_int, c_int, c_int, c_int, _P],
     },
     "attn_tokens_f32": {
@@ -1798,7 +1798,7 @@ def plan_linear(m: int, n: int, k: int, swiglu: bool = False, normed: bool = Fal
     else:
         _, splits, per = tile_plan(m, n, k, epi, aligned, n_cu)
     name = ctypes.create_string_buffer(64)
-    rc = _fn("gemm_bf16", "mf_gemm_bf16_plan")(m, n, k, 1 if aligned else 0, epi, splits, per,
+    rc = _fn("gemm_bf16", "mf_gemm_bf16_plan")(m, n, k, 1 if aligned else 0, 1 if tiled else 0, epi, splits, per,
                                                1 if normed else 0, n_cu, name, 64)
     if rc != 0:
         raise KernelError(f"plan_linear: error {rc} for m {m}, n {n}, k {k}")

@@ -86,6 +86,22 @@ def test_decode_split_plan_bounds():
     assert ops.decode_split_plan(8, 4, 7, 4096, target_blocks=64) == (2, 2)        # a chip of 64 CUs splits less
 
 
+def test_where_64_x_64_tiles_take_a_short_k():
+    """17 to 64 rows: one tile kernel over the whole of a short K, but not where a tile's chain outlasts the K-split kernels
+    (few rows against few weight rows of 2,048; few rows against more than a tile a CU without SwiGLU)."""
+    tiles = lambda m, n, k, **kw: ops.plan_linear(m, n, k, n_cu=256, **kw)["kernel"] == "tile_step_kernel<64,64>"
+    for m, n, k in ((17, 512, 2048), (17, 2048, 2048), (24, 1024, 2048), (32, 2560, 2048), (48, 512, 2048), (17, 512, 1536)):
+        assert not tiles(m, n, k, swiglu=True, tiled=True) and tiles(m, n, k, swiglu=True), (m, n, k)
+    for m, n, k in ((64, 2048, 2048), (33, 4096, 2048), (17, 12288, 2048), (64, 512, 1536), (17, 2048, 1536), (17, 512, 896),
+                    (40, 22016, 2048), (32, 17920, 1536), (17, 9728, 896)):
+        assert tiles(m, n, k, swiglu=True, tiled=True) and tiles(m, n, k, swiglu=True), (m, n, k)
+    for m, n, k in ((17, 24576, 768), (24, 20480, 1024), (32, 24576, 768)):
+        assert not tiles(m, n, k, accumulate=True, tiled=True) and tiles(m, n, k, accumulate=True), (m, n, k)
+    for m, n, k in ((48, 24576, 768), (64, 20480, 1024), (17, 24576, 256), (17, 16384, 768), (17, 512, 1024), (32, 1152, 896),
+                    (24, 16448, 896), (32, 24576, 640)):
+        assert tiles(m, n, k, accumulate=True, tiled=True) and tiles(m, n, k, accumulate=True), (m, n, k)
+
+
 def test_tile_plan_of_k_not_in_64s():
     """A product that cannot be copied straight into LDS is cut over K where its own kernels gain by it: not for the cheap
     epilogues of a K of a thousand (200 x 8000 SwiGLU 21.2 us whole, 34.7 in two parts), for sums added to 32 bits at the
