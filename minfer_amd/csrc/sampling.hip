@@ -252,6 +252,10 @@ __device__ __forceinline__ float penalised(float v, int count, float repeat, flo
 }
 
 // penalties in place; prev is [rows][max_prev], n_prev[row] entries are used
+// SHORT: windows of at most 64, a lane for each place: three trips to memory (the window, the entries, back), 6.6 us -> 4.2
+// against a walk over the window in memory for every token.  (Kernels of their own: as one, the walk of longer windows took
+// 3 us more of 65, at 256 places.)
+template <bool SHORT>
 __global__ __launch_bounds__(64) void penalties_kernel(float* __restrict__ logits, int ld, int vocab,
                                                        const int* __restrict__ prev, int max_prev,
                                                        const int* __restrict__ n_prev, float repeat,
@@ -259,9 +263,7 @@ __global__ __launch_bounds__(64) void penalties_kernel(float* __restrict__ logit
   const int rowi = blockIdx.x;
   float* row = logits + (size_t)rowi * ld;
   const int* pv = prev + (size_t)rowi * max_prev;
-  if (max_prev <= 64) {
-    // a lane for each place of the window: three trips to memory (the window, the entries, back), 6.6 us -> 4.2 against a
-    // walk over the window in memory for every token
+  if constexpr (SHORT) {
     const int lane = threadIdx.x;
     const int all = pv[min(lane, max_prev - 1)], n = min(n_prev[rowi], max_prev);
     const bool mine = lane < n && all >= 0 && all < vocab;
@@ -274,21 +276,22 @@ __global__ __launch_bounds__(64) void penalties_kernel(float* __restrict__ logit
       first = first && !(same && j < lane);
     }
     if (mine && first) row[all] = penalised(at, count, repeat, frequency, presence);
-    return;
-  }
-  const int n = min(n_prev[rowi], max_prev);
-  for (int i = threadIdx.x; i < n; i += 64) {
-    const int tok = pv[i];
-    if (tok < 0 || tok >= vocab) continue;
-    int count = 0;
-    bool first = true;
-    for (int j = 0; j < n; ++j) {
-      if (pv[j] == tok) {
-        ++count;
-        if (j < i) first = false;
+  } else {
+    const int n = min(n_prev[rowi], max_prev);
+    for (int i = threadIdx.x; i < n; i += 64) {
+      const int tok = pv[i];
+      if (tok < 0 || tok >= vocab) continue;
+      int count = 0;
+      bool first = true;
+      for (int j = 0; j < n; ++j) {
+        if (pv[j] == tok) {
+          ++count;
+          if (j < i) first = false;
+        }
       }
+      if (!first) continue;
+      row[tok] = penalised(row[tok], count, repeat, frequency, presence);
     }
-    if (first) row[tok] = penalised(row[tok], count, repeat, frequency, presence);
   }
 }
 
@@ -890,8 +893,10 @@ MF_API int mf_penalties(float* logits, int ld, int rows, int vocab, const int* p
                         hipStream_t stream) {
   if (rows <= 0 || max_prev <= 0) return 0;
   if (vocab <= 0 || ld < vocab) return (int)hipErrorInvalidValue;
-  penalties_kernel<<<rows, 64, 0, stream>>>(logits, ld, vocab, prev, max_prev, n_prev, repeat, frequency,
-                                            presence);
+  if (max_prev <= 64)
+    penalties_kernel<true><<<rows, 64, 0, stream>>>(logits, ld, vocab, prev, max_prev, n_prev, repeat, frequency, presence);
+  else
+    penalties_kernel<false><<<rows, 64, 0, stream>>>(logits, ld, vocab, prev, max_prev, n_prev, repeat, frequency, presence);
   return mf_launch_status();
 }
 

@@ -57,6 +57,21 @@ def test_reference_vectors(ops):
     assert run(ops.penalties, [4., -4, 0, 0], prev0, n2, 2.0, 1.0, 1.0) == [1, -4, 0, 0]  # :411-427, :448-452
 
 
+@pytest.mark.parametrize("window", [1, 2, 63, 64, 65, 200])
+def test_penalties_by_window(ops, window):
+    """Both kernels' windows (up to 64 places, more) and their edges: repeated tokens, rows that use a part of their window,
+    none of it, all of it; the same bits as the plain sampler's 32-bit steps give, to the last place."""
+    vocab, rows = 500, 4
+    l = logits_rows(rows, vocab, 3)
+    prev = torch.randint(0, 40, (rows, window), generator=torch.Generator().manual_seed(window), dtype=torch.int32)
+    n = torch.tensor([0, 1, max(1, window - 1), window], dtype=torch.int32)
+    for repeat, frequency, presence in ((1.3, 0.0, 0.0), (1.1, 0.25, 0.5), (1.0, 0.1, 0.0)):
+        got = l.to(DEV)
+        ops.penalties(got, prev.to(DEV), n.to(DEV), repeat, frequency, presence)
+        want = np.stack([pq.apply_penalties(l[i].numpy(), prev[i, :int(n[i])].tolist(), repeat, frequency, presence) for i in range(rows)])
+        np.testing.assert_allclose(got.cpu().numpy(), want, rtol=3e-7, atol=1e-6)      # (two roundings of values up to 12)
+
+
 @pytest.mark.parametrize("vocab,k", [(1000, 40), (152064, 40), (777, 1), (50, 49), (3000, 700)])
 def test_top_k_matches_plain(ops, vocab, k):
     l = logits_rows(4, vocab, 2)
