@@ -1,18 +1,20 @@
 // True 32-bit matrix product: C[M][N] (+)= A[M][K] * W[N][K]^T (+ bias[N]).
 // out[t][o] = dot(W[o][:], x[t][:]) + b[o], as src/graph/cpu_backend.rs:214-248 of
-// yusiwen/minfer.  Plain fp32 FMA, no reduced-precision matrix mode: this is the path
-// that shows faults bfloat16 hides.  Any M, N, K; vector loads only where they are aligned.
+// yusiwen/minfer.  32-bit operands, products and sums throughout, no reduced-precision matrix mode: this is the
+// path that shows faults bfloat16 hides.  Any M, N, K; vector loads only where they are aligned.
 //
 // Three kernels:
 //  * `rows_f32_kernel`: at most 8 rows, K in 4s: the weight stream, a wave a few weight rows.
 //  * `tile_f32_kernel`: aligned operands and K in 32s: 64 x 64 tiles on the 32-bit matrix instruction (an FMA a product,
 //    twice the vector units' rate), K split over blocks where the tiles leave CUs idle.
 //  * `gemm_f32_kernel`: everything else, from LDS with vector FMA.
-// A dot product is summed in blocks of 128 terms whose sums are then added up: the rounding
+// A dot product is summed in chains of 128 terms whose sums are then added up: the rounding
 // error of one long chain grows with the root of its length (18944 terms in the down product;
-// the reference's scalar path sums in 64 bits, src/vec_ops.rs:31-35), that of blocks with the
-// roots of the block's and of the number of blocks.
+// the reference's scalar path sums in 64 bits, src/vec_ops.rs:31-35), that of short chains with the
+// roots of a chain's and of the number of chains.  (`rows_f32_kernel`: 128 chains of K / 128 terms, which errs less
+// than chains of 128 at any K.)
 #include <algorithm>
+#include <type_traits>
 
 #include "common.h"
 
@@ -273,31 +275,46 @@ __global__ __launch_bounds__(256) void rows_f32_kernel(const float* __restrict__
   const float* w[NR];
 #pragma unroll
   for (int j = 0; j < NR; ++j) w[j] = W + (size_t)min(n0 + j, N - 1) * ldw;
-  float acc[MR][NR] = {};
-#pragma unroll 2
-  for (int k = lane * 4; k < K; k += 256) {
-    float4 x[NR];
+  float acc[MR][NR][2] = {};
+  // U runs of 256 at a time, all their loads on their way before the first is waited for (left to the scheduler, the loads of
+  // eight rows are waited for one by one: 8 rows against 1,536 of 8,960 26 us so, 78)
+  constexpr int U = MR * NR >= 16 ? 1 : 2;
+  auto runs = [&](auto COUNT, int k) {
+    constexpr int C = decltype(COUNT)::value;
+    float4 x[C][NR], a[C][MR];
 #pragma unroll
-    for (int j = 0; j < NR; ++j) x[j] = *reinterpret_cast<const float4*>(w[j] + k);
+    for (int u = 0; u < C; ++u) {
 #pragma unroll
-    for (int i = 0; i < MR; ++i) {
-      const float4 a = *reinterpret_cast<const float4*>(A + (size_t)min(i, M - 1) * lda + k);
+      for (int j = 0; j < NR; ++j) x[u][j] = *reinterpret_cast<const float4*>(w[j] + k + 256 * u);
 #pragma unroll
-      for (int j = 0; j < NR; ++j)
-        acc[i][j] = fmaf(a.w, x[j].w, fmaf(a.z, x[j].z, fmaf(a.y, x[j].y, fmaf(a.x, x[j].x, acc[i][j]))));
+      for (int i = 0; i < MR; ++i) a[u][i] = *reinterpret_cast<const float4*>(A + (size_t)min(i, M - 1) * lda + k + 256 * u);
     }
-  }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < C; ++u)
+#pragma unroll
+      for (int i = 0; i < MR; ++i)
+#pragma unroll
+        for (int j = 0; j < NR; ++j) {
+          acc[i][j][0] = fmaf(a[u][i].y, x[u][j].y, fmaf(a[u][i].x, x[u][j].x, acc[i][j][0]));
+          acc[i][j][1] = fmaf(a[u][i].w, x[u][j].w, fmaf(a[u][i].z, x[u][j].z, acc[i][j][1]));
+        }
+  };
+  int k = lane * 4;
+  for (; k + 256 * (U - 1) < K; k += 256 * U) runs(std::integral_constant<int, U>{}, k);
+  if (U > 1 && k < K) runs(std::integral_constant<int, 1>{}, k);
+  float tot[MR][NR];
 #pragma unroll
   for (int i = 0; i < MR; ++i)
 #pragma unroll
-    for (int j = 0; j < NR; ++j) acc[i][j] = wave_sum(acc[i][j]);
+    for (int j = 0; j < NR; ++j) tot[i][j] = wave_sum(acc[i][j][0] + acc[i][j][1]);
   // lane i NR + j stores sum (i, j)
 #pragma unroll
   for (int i = 0; i < MR; ++i)
 #pragma unroll
     for (int j = 0; j < NR; ++j)
       if (lane == i * NR + j && i < M && n0 + j < N) {
-        const float v = bias ? acc[i][j] + bias[n0 + j] : acc[i][j];
+        const float v = bias ? tot[i][j] + bias[n0 + j] : tot[i][j];
         float* c = C + (size_t)i * ldc + n0 + j;
         *c = ACCUMULATE ? *c + v : v;
       }

@@ -232,6 +232,19 @@ def test_gemm_f32_kernels(ops, m, n, k):
     test_gemm_f32(ops, m, n, k)
 
 
+@pytest.mark.parametrize("m", [1, 8, 9])
+def test_gemm_f32_error_over_a_long_k(ops, m):
+    """Sums in short chains.  Rounding a sum errs by 0.41 units of 2^-24 of it (root of squares), so a dot product of K unit
+    normal pairs by that times the root of the sum of its partial sums' variances: chains of 128 added up, 64 K + K^2 / 256 =
+    7.6e7 at K = 131,072; 128 chains of K / 128 terms (the kernel of few rows) 6.8e7, one chain for each of 64 lanes 1.3e8."""
+    n, k = 256, 131072
+    x, w = (torch.randn(r, k, generator=torch.Generator().manual_seed(s)).to(DEV) for r, s in ((m, 1), (n, 2)))
+    out = torch.empty(m, n, device=DEV)
+    ops.linear(x, w, None, out)
+    err = (out.double() - x.double() @ w.double().t()).pow(2).mean().sqrt().item()
+    assert err < 0.41 * 2.0 ** -24 * math.sqrt(7.6e7) * 1.15
+
+
 @pytest.mark.parametrize("variant", [0, 1, 2, 3, 6, 9, 12, 13, 15])
 @pytest.mark.parametrize("m,n,k", GEMM_SHAPES + [(2048, 512, 256), (1, 152064, 64), (64, 3584, 3584),
                                                  # at most 16 rows with K of 1536..4096: activations in registers
