@@ -2466,6 +2466,17 @@ int launch_form(int form, const bf16* A, int lda, const bf16* W, int ldw, const 
              : launch_tile64<false>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi, stream, splits, k_per_split);
 }
 
+// by their columns where the tile has 256 rows
+const char* form_name(int form, bool split) {
+  static const char* names[N_FORMS][2] = {{"tile_dma_kernel<256>", "tile_dma_kernel<256>(split K)"},
+                                          {"tile_dma_kernel<192>", "tile_dma_kernel<192>(split K)"},
+                                          {"tile_dma_kernel<128>", "tile_dma_kernel<128>(split K)"},
+                                          {"tile_dma_kernel<128,256>", "tile_dma_kernel<128,256>(split K)"},
+                                          {"tile_step_kernel<128,128>", "tile_step_kernel<128,128>(split K)"},
+                                          {"tile_step_kernel<64,64>", "tile_step_kernel<64,64>(split K)"}};
+  return names[form][split];
+}
+
 TilePlan plan_tiles(int M, int N, int K, bool dma_ok, int epi, int n_cu) {
   const long cu = n_cu > 0 ? n_cu : 1;
   const long nkt = (K + 63) / 64, chunks = (K + 255) / 256;
@@ -2594,7 +2605,7 @@ MF_API int mf_gemm_bf16_grouped(const void* A, const void* W, float* C, const in
 
 // `variant`: 0 picks by shape among the whole-K kernels; 1: 256x256 tile with 4 waves, 2: 128x128,
 // 3: 64x64, 6: 256x128 with 8 waves, 9: 256x256 with 8 waves; through the direct-to-LDS pipeline, K in
-// 64s: 12: 256x256, 13: 256x128 in three stages, 15: 256x192 (tests name them).
+// 64s: 12: 256x256 (SwiGLU: or 256x192), 13: the cheapest of 256x128, 128x256, 128x128 and 64x64, 15: 256x192 (tests name them).
 MF_API int mf_gemm_bf16(const void* A, int lda, const void* W, int ldw, const float* bias, void* C,
                         int ldc, int M, int N, int K, int epi, int variant, hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
@@ -2821,14 +2832,15 @@ MF_API int mf_gemm_bf16_tile_plan(int M, int N, int K, int aligned, int epi, int
 // activation rows against `N` weight rows of length `K`; `aligned`: 16-byte aligned operands with
 // row strides and K in multiples of 8; `tiled`: there is the tiled copy; for at most 64 rows `splits`, `k_per_split`: the caller's K
 // split (1, K for none); `normed`: the RMS norm is to be folded in (an empty name then means "no
-// such kernel": norm and product run one after the other); `n_cu`: compute units of the device.
+// such kernel": norm and product run one after the other); `variant`: of the tile kernels, as `mf_gemm_bf16` takes it (0: the
+// plan's own choice, K split or whole); `n_cu`: compute units of the device.
 MF_API int mf_gemm_bf16_plan(int M, int N, int K, int aligned, int tiled, int epi, int splits, int k_per_split,
-                             int normed, int n_cu, char* name, int cap) {
+                             int normed, int variant, int n_cu, char* name, int cap) {
   if (!name || cap < 48 || M <= 0 || N <= 0 || K <= 0 || epi < 0 || epi > EPI_XIELU || n_cu <= 0) return (int)hipErrorInvalidValue;
   const char* what = "";
   if (normed) {
     what = (aligned && stationary_takes(M, N, K, epi, true)) ? "stationary16_kernel(norm)" : "";
-  } else if (M <= 64) {
+  } else if (M <= 64 && !variant) {
     switch (skinny_choice(M, N, K, aligned != 0, tiled != 0 && K % 32 == 0, epi, splits, k_per_split, n_cu)) {
       case SK_STATIONARY: what = "stationary16_kernel"; break;
       case SK_ROLLING: what = "rolling16_kernel"; break;
@@ -2840,14 +2852,20 @@ MF_API int mf_gemm_bf16_plan(int M, int N, int K, int aligned, int tiled, int ep
     }
   } else {
     const bool dma_ok = aligned && K % DMA_BK == 0 && (size_t)M * K * 2 < (1ull << 32) && (size_t)N * K * 2 < (1ull << 32);
-    const TilePlan plan = plan_tiles(M, N, K, dma_ok, epi, n_cu);
+    const TilePlan plan = variant ? TilePlan{variant, 1, K, 0.} : plan_tiles(M, N, K, dma_ok, epi, n_cu);
+    const bool split = plan.splits > 1;
+    if (variant >= 12 && !dma_ok) return (int)hipErrorInvalidValue;
     switch (plan.variant) {
-      case 12: what = plan.splits > 1 ? "tile_dma_kernel<256>(split K)" : "tile_dma_kernel<256>"; break;
-      case 13: what = "tile_dma_kernel<128>"; break;
-      case 15: what = "tile_dma_kernel<192>"; break;
+      case 12: case 13: case 15:
+        what = form_name(dma_form(plan.variant, M, N, epi, (split ? plan.k_per_split : K) / DMA_BK, plan.splits, n_cu), split);
+        break;
       case 9: what = "tile_kernel<256,256>"; break;
-      case 2: what = plan.splits > 1 ? "tile_kernel<128,128>(split K)" : "tile_kernel<128,128>"; break;
-      default: what = "tile_kernel<64,64>"; break;
+      case 2:
+        what = split && dma_ok ? form_name(dma_form(2, M, N, EPI_F32, plan.k_per_split / DMA_BK, plan.splits, n_cu), true)
+               : split         ? "tile_kernel<128,128>(split K)" : "tile_kernel<128,128>";
+        break;
+      case 3: what = "tile_kernel<64,64>"; break;
+      default: return (int)hipErrorInvalidValue;
     }
   }
   snprintf(name, (size_t)cap, "%s", what);

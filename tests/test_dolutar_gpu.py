@@ -209,8 +209,9 @@ GATED_SHAPES = {
     (5, 2048, 896): "stationary16_kernel", (8, 3000, 1024): "stationary16_kernel", (16, 64, 8192): "skinny_ring_kernel",
     (17, 112, 96): "skinny_kernel", (40, 100, 1024): "skinny_ring_kernel", (33, 16416, 512): "panel_kernel",
     (64, 33, 77): "skinny_kernel", (65, 112, 96): "tile_kernel<128,128>", (300, 37, 60): "tile_kernel<128,128>",
-    (256, 192, 4096): "tile_kernel<128,128>(split K)", (513, 1024, 512): "tile_dma_kernel<128>",
-    (1501, 8170, 128): "tile_dma_kernel<256>", (1000, 8192, 100): "tile_kernel<256,256>"}
+    (256, 192, 4096): "tile_step_kernel<64,64>(split K)", (513, 1024, 512): "tile_step_kernel<64,64>",
+    (257, 3331, 64): "tile_step_kernel<128,128>", (257, 5551, 64): "tile_dma_kernel<128,256>", (700, 2776, 64): "tile_dma_kernel<128>",
+    (257, 10990, 64): "tile_dma_kernel<192>", (1501, 8170, 128): "tile_dma_kernel<256>", (1000, 8192, 100): "tile_kernel<256,256>"}
 
 
 @pytest.mark.parametrize("m, nf, k", list(GATED_SHAPES))

@@ -144,7 +144,7 @@ def test_plan_linear_names_the_kernels_of_the_model_shapes():
     assert p(4096, 3584, 3584, accumulate=True) == "tile_dma_kernel<256>"     # 224 tiles: one round nearly full
     assert p(4096, 37888, 3584, swiglu=True) == "tile_dma_kernel<256>"
     assert p(2048, 3584, 3584 + 8, accumulate=True) == "tile_kernel<128,128>"      # K not in 64s
-    assert p(200, 3584, 18944, accumulate=True) == "tile_kernel<128,128>(split K)"
+    assert p(200, 3584, 18944, accumulate=True) == "tile_dma_kernel<128>(split K)"
     # other widths: multiples of 256 that are instantiated take the register-resident kernel, the
     # rest the rolling one; unaligned operands the guarded ones
     for k in (1024, 2560, 3072, 6144, 7168):
