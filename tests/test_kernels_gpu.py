@@ -754,30 +754,43 @@ def test_gemm_bf16_swiglu(ops, variant, m, nf, k):
     assert torch.equal(out, again)
 
 
-# the direct-to-LDS kernel's tiles: sizes at which each of them is the one that runs (with fewer than, exactly and more than
-# its stages of k tiles), rows and columns that leave remainders, row lengths without 16-byte stores
-@pytest.mark.parametrize("variant,m,n,k", [(13, 700, 11000, 64), (13, 511, 16001, 192), (13, 130, 16390, 256),     # 256 x 128
-                                           (13, 600, 22016, 128), (13, 513, 9000, 320), (13, 1025, 8201, 64),      # 128 x 256
-                                           (13, 257, 8200, 192), (13, 300, 6403, 64), (13, 257, 8201, 320),        # 128 x 128
-                                           (13, 129, 101, 64), (13, 127, 333, 320), (13, 65, 1002, 576),           # 64 x 64
-                                           (15, 257, 193, 64), (15, 300, 579, 192),                                # 256 x 192
-                                           (12, 255, 259, 64), (12, 513, 510, 192)])                               # 256 x 256
-def test_gemm_bf16_tile_forms(ops, variant, m, n, k):
+# the direct-to-LDS kernels' tiles by name: sizes at which each of them is the one that runs (with fewer k tiles than its
+# stages, as many, and more), rows and columns that leave remainders, row lengths without 16-byte stores
+DMA_TILES = {"tile_dma_kernel<256>": [(12, 255, 259, 64), (12, 513, 510, 192), (12, 300, 700, 128)],                     # two stages
+             "tile_dma_kernel<192>": [(15, 257, 193, 64), (15, 300, 579, 192), (15, 300, 201, 128)],                     # two
+             "tile_dma_kernel<128>": [(13, 700, 11000, 64), (13, 511, 16001, 192), (13, 130, 16390, 256)],               # three
+             "tile_dma_kernel<128,256>": [(13, 600, 22016, 128), (13, 513, 9000, 320), (13, 1025, 8201, 64), (13, 513, 9001, 192)],
+             "tile_step_kernel<128,128>": [(13, 300, 7203, 64), (13, 300, 7003, 128), (13, 257, 8200, 192), (13, 257, 8201, 256),
+                                           (13, 257, 8201, 320)],                                                       # four
+             "tile_step_kernel<64,64>": [(13, 129, 101, 64), (13, 127, 333, 320), (13, 65, 1002, 576), (13, 300, 6403, 64)]}    # five
+SWIGLU_TILES = {"tile_dma_kernel<256>": [(12, 500, 16380, 128)], "tile_dma_kernel<192>": [(12, 257, 95, 192), (12, 300, 201, 64)],
+                "tile_dma_kernel<128>": [(13, 700, 5500, 64)], "tile_dma_kernel<128,256>": [(13, 600, 11008, 128)],
+                "tile_step_kernel<128,128>": [(13, 257, 4101, 192)], "tile_step_kernel<64,64>": [(13, 129, 97, 320)]}
+
+
+@pytest.mark.parametrize("name,variant,m,n,k", [(f, *s) for f, sizes in DMA_TILES.items() for s in sizes])
+def test_gemm_bf16_tile_forms(ops, name, variant, m, n, k):
+    if ops.cu_count() == 256:
+        assert ops.plan_linear(m, n, k, variant=variant)["kernel"] == name
     test_gemm_bf16(ops, variant, m, n, k)
 
 
-# SwiGLU: 256 x 256 (512 rows and 16,380 outputs fill the chip once), 256 x 192, 256 x 128, 128 x 256, 128 x 128, 64 x 64
-@pytest.mark.parametrize("variant,m,nf,k", [(12, 500, 16380, 128), (12, 257, 95, 192), (12, 300, 201, 64), (13, 700, 5500, 64),
-                                            (13, 600, 11008, 128), (13, 257, 4101, 192), (13, 129, 97, 320)])
-def test_gemm_bf16_swiglu_tile_forms(ops, variant, m, nf, k):
+@pytest.mark.parametrize("name,variant,m,nf,k", [(f, *s) for f, sizes in SWIGLU_TILES.items() for s in sizes])
+def test_gemm_bf16_swiglu_tile_forms(ops, name, variant, m, nf, k):
+    if ops.cu_count() == 256:
+        assert ops.plan_linear(m, (nf + 31) // 32 * 64, k, swiglu=True, variant=variant)["kernel"] == name
     test_gemm_bf16_swiglu(ops, variant, m, nf, k)
 
 
 # a product cut over K whose parts the next kernel adds: into the stream with the norm of the new rows (rows of one, two, four,
 # eight and sixteen runs of 1,024 values, whole and not), and under the rotation; the same bits as one kernel after the other
-@pytest.mark.parametrize("m,n,k", [(65, 896, 4864), (203, 3584, 3584), (100, 1028, 2048), (100, 8192, 8192), (66, 9000, 8192),
-                                   (1030, 776, 6144)])
-def test_split_product_with_norm(ops, m, n, k):
+@pytest.mark.parametrize("m,n,k,name", [(65, 896, 4864, "tile_step_kernel<64,64>"), (203, 3584, 3584, "tile_dma_kernel<128>"),
+                                        (100, 1028, 2048, "tile_step_kernel<64,64>"), (100, 8192, 8192, "tile_dma_kernel<128,256>"),
+                                        (66, 9000, 8192, "tile_dma_kernel<128,256>"), (1030, 776, 6144, "tile_dma_kernel<128>"),
+                                        (720, 896, 4864, "tile_step_kernel<128,128>")])
+def test_split_product_with_norm(ops, m, n, k, name):
+    if ops.cu_count() == 256:
+        assert ops.plan_linear(m, n, k, accumulate=True)["kernel"] == name + "(split K)"
     x, w = rnd((m, k), torch.bfloat16, 8).to(DEV), rnd((n, k), torch.bfloat16, 9, 0.05).to(DEV)
     b, g, base = rnd((n,), seed=10).to(DEV), rnd((n,), seed=11).to(DEV), rnd((m, n), seed=12).to(DEV)
     assert ops.tile_plan(m, n, k, ops.EPI_ACC_F32)[1] > 1
