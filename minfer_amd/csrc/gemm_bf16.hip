@@ -158,15 +158,12 @@ struct RowGroup { int first, rows, matrix, unused; };
 
 // ------------------------------------------------------------------ tiled kernel
 // LDS row stride is BK + 8 elements (144 bytes for BK 64, 80 for BK 32): conflict-free b128 reads
-// GROUPED: rows in groups, each with a matrix of its own (experts): entry bm of `groups` names the rows of tile row bm
-// and the matrix, one of a stack [matrices][N][ldw] (see RowGroup).
-template <int BM, int BN, int WM, int WN, int BK, bool VEC, bool GROUPED = false>
+template <int BM, int BN, int WM, int WN, int BK, bool VEC>
 __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN)) void tile_kernel(const bf16* __restrict__ A, int lda,
                                                    const bf16* __restrict__ W, int ldw,
                                                    const float* __restrict__ bias, void* __restrict__ C,
                                                    int ldc, int M, int N, int K, int epi, int tiles_m,
-                                                   int xcd_remap, int k_per_split,
-                                                   const RowGroup* __restrict__ groups = nullptr) {
+                                                   int xcd_remap, int k_per_split) {
   constexpr int NTHR = 64 * (BM / WM) * (BN / WN);
   constexpr int LDS_LD = BK + 8;
   if (k_per_split > 0) {
@@ -197,14 +194,6 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN)) void tile_kernel(const 
   }
   int bm, bn;
   tile_position(tile, tiles_m, gridDim.x / tiles_m, bm, bn);
-  if (GROUPED) {
-    const RowGroup rg = groups[bm];
-    A += (size_t)rg.first * lda;
-    W += (size_t)rg.matrix * N * ldw;
-    C = (float*)C + (size_t)rg.first * ldc;
-    M = rg.rows;
-    bm = 0;
-  }
   const int m0 = bm * BM, n0 = bn * BN;
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
   const int wm = (wid % (BM / WM)) * WM, wn = (wid / (BM / WM)) * WN;
@@ -926,7 +915,7 @@ int launch_tile_v(const bf16* A, int lda, const bf16* W, int ldw, const float* b
   }
   const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
   kern<<<dim3(tiles_m * tiles_n, splits), NTHR, smem, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi,
-                                                                tiles_m, tiles_m * tiles_n >= 16, k_per_split, nullptr);
+                                                                tiles_m, tiles_m * tiles_n >= 16, k_per_split);
   return mf_launch_status();
 }
 
@@ -948,23 +937,6 @@ int launch_grouped_dma(const bf16* A, int lda, const bf16* W, int ldw, float* C,
   const int tiles_n = (N + BN - 1) / BN;
   tile_dma_kernel<BM, BN, STAGES, true><<<dim3(n_groups * tiles_n), 512, DmaTile<BM, BN>::template lds<STAGES>(), stream>>>(
       A, lda, W, ldw, nullptr, C, ldc, 0, N, K, EPI_F32, n_groups, n_groups * tiles_n >= 16, 0, groups);
-  return mf_launch_status();
-}
-
-template <int BM, int BN, int WM, int WN, int BK>
-int launch_grouped_tile(const bf16* A, int lda, const bf16* W, int ldw, float* C, int ldc, const RowGroup* groups, int n_groups,
-                        int N, int K, hipStream_t stream) {
-  constexpr int smem = 2 * (BM + BN) * (BK + 8) * (int)sizeof(bf16);
-  static bool configured = false;
-  auto kern = tile_kernel<BM, BN, WM, WN, BK, true, true>;
-  if (!configured) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, smem);
-    if (e != hipSuccess) return (int)e;
-    configured = true;
-  }
-  const int tiles_n = (N + BN - 1) / BN;
-  kern<<<dim3(n_groups * tiles_n), 64 * (BM / WM) * (BN / WN), smem, stream>>>(A, lda, W, ldw, nullptr, C, ldc, 0, N, K, EPI_F32,
-                                                                               n_groups, n_groups * tiles_n >= 16, 0, groups);
   return mf_launch_status();
 }
 
@@ -2583,20 +2555,17 @@ SkinnyChoice skinny_choice(int M, int N, int K, bool aligned, bool tiled, int ep
 
 // Products of rows that stand in groups with a matrix each: rows first .. first + rows - 1 of A (a row group's, at most
 // the variant's tile rows) with matrix `matrix` of the stack W [matrices][N][K], 32-bit sums into the same rows of C.
-// variant 2: tiles of 128 x 128, 12: 256 x 256 (K in 64s), 13: 256 x 128 (K in 64s).
+// variant 2: tiles of 128 x 128, 12: 256 x 256, 13: 256 x 128; K in 64s.
 MF_API int mf_gemm_bf16_grouped(const void* A, const void* W, float* C, const int* groups, int n_groups, int N, int K,
                                 int variant, hipStream_t stream) {
   if (n_groups <= 0 || N <= 0) return 0;
-  if (K <= 0 || K % 8 || !groups || (uintptr_t)A % 16 || (uintptr_t)W % 16 || (variant != 2 && K % DMA_BK) ||
-      (size_t)N * K * 2 >= (1ull << 32))
+  if (K <= 0 || K % DMA_BK || !groups || (uintptr_t)A % 16 || (uintptr_t)W % 16 || (size_t)N * K * 2 >= (1ull << 32))
     return (int)hipErrorInvalidValue;
   const bf16* a = (const bf16*)A;
   const bf16* w = (const bf16*)W;
   const RowGroup* g = (const RowGroup*)groups;
   switch (variant) {
-    case 2:
-      return K % DMA_BK == 0 ? launch_tile_step<128, 128, 2, 4, 4, true>(a, K, w, K, nullptr, C, N, 0, N, K, EPI_F32, stream, 1, 0, g, n_groups)
-                             : launch_grouped_tile<128, 128, 64, 64, 64>(a, K, w, K, C, N, g, n_groups, N, K, stream);
+    case 2: return launch_tile_step<128, 128, 2, 4, 4, true>(a, K, w, K, nullptr, C, N, 0, N, K, EPI_F32, stream, 1, 0, g, n_groups);
     case 12: return launch_grouped_dma<256, 256, 2>(a, K, w, K, C, N, g, n_groups, N, K, stream);
     case 13: return launch_grouped_dma<256, 128, 3>(a, K, w, K, C, N, g, n_groups, N, K, stream);
   }

@@ -1934,7 +1934,9 @@ def linear_norm_out(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.
 
 
 # variants of the grouped product: (tile rows, tile columns, blocks a CU, microseconds a k tile of 64 with every CU
-# busy), as the plan of the single product has them
+# busy).  The times are those in the plan of the single product, which also prices a round's start and each tile's own
+# nearly empty chip; here one share for every tile is enough: over 132 products of 4 to 128 groups of 20 to 1,500 rows
+# each (matrices of 512 x 256 to 14,336 x 4,096) the choice is 0.4 % from the best tile on average, 16 % at most.
 GROUPED_TILES = {12: (256, 256, 1, 1.36), 13: (256, 128, 1, 0.84), 2: (128, 128, 1, 0.62)}
 
 
