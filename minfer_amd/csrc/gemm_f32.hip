@@ -202,6 +202,8 @@ __global__ __launch_bounds__(256) void tile_f32_kernel(const float* __restrict__
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   // D: the lane's row is lane % 16, its columns 4 (lane / 16) + e
+  // (what a short K takes is the stores: 1,500 rows against 24,000 of 32 92 us with 4-byte ones, 45 so)
+  const bool vec = ldc % 4 == 0 && (uintptr_t)C % 16 == 0;
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     const int m = m0 + wm + i * 16 + fr;
@@ -209,18 +211,20 @@ __global__ __launch_bounds__(256) void tile_f32_kernel(const float* __restrict__
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       const int n = n0 + wn + j * 16 + fk * 4;
-      const floatx4 v = acc[i][j] + tot[i][j];
+      floatx4 v = acc[i][j] + tot[i][j];
       float* c = C + (size_t)m * ldc + n;
-      if (SPLIT && n + 4 <= N && ldc % 4 == 0 && (uintptr_t)C % 16 == 0) {
+      if (!SPLIT && bias) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] += n + e < N ? bias[n + e] : 0.f;
+      }
+      if (vec && n + 4 <= N) {
+        if (ACCUMULATE) v = *reinterpret_cast<const floatx4*>(c) + v;
         *reinterpret_cast<floatx4*>(c) = v;
         continue;
       }
 #pragma unroll
       for (int e = 0; e < 4; ++e)
-        if (n + e < N) {
-          const float x = SPLIT || !bias ? v[e] : v[e] + bias[n + e];
-          c[e] = ACCUMULATE ? c[e] + x : x;
-        }
+        if (n + e < N) c[e] = ACCUMULATE ? c[e] + v[e] : v[e];
     }
   }
 }
