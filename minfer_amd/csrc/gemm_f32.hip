@@ -4,7 +4,7 @@
 // path that shows faults bfloat16 hides.  Any M, N, K; vector loads only where they are aligned.
 //
 // Three kernels:
-//  * `rows_f32_kernel`: at most 8 rows, K in 4s: the weight stream, a wave a few weight rows.
+//  * `rows_f32_kernel`: at most 8 rows, K in 4s (and not short for many weight rows): the weight stream, a wave a few weight rows.
 //  * `tile_f32_kernel`: aligned operands and K in 32s: 64 x 64 tiles on the 32-bit matrix instruction (an FMA a product,
 //    twice the vector units' rate), K split over blocks where the tiles leave CUs idle.
 //  * `gemm_f32_kernel`: everything else, from LDS with vector FMA.
@@ -266,6 +266,24 @@ bool tile_takes(int M, int N, int K, int lda, int ldw, const void* A, const void
 }
 
 // ---- few rows: the weight stream
+// The sums of a wave's lanes: a lane's N sums meet those of the lane O away, which keeps the one half of them and hands over the
+// other while there are several: the additions of a `wave_sum` for each, in their order, with a sixth of the shuffles for
+// 32 sums (8 rows against 24,000 of 64 16.5 us with a `wave_sum` each, 6.6 so).  Sum s ends in the lanes s 64 / N on.
+template <int N, int O>
+__device__ __forceinline__ void meet(float* sum, int lane) {
+  if constexpr (N > 1) {
+    const bool upper = lane & O;
+#pragma unroll
+    for (int x = 0; x < N / 2; ++x) {
+      const float lo = sum[x], hi = sum[x + N / 2];
+      sum[x] = (upper ? hi : lo) + __shfl_xor(upper ? lo : hi, O, MF_WAVE);
+    }
+  } else {
+    sum[0] += __shfl_xor(sum[0], O, MF_WAVE);
+  }
+  if constexpr (O > 1) meet<(N > 1 ? N / 2 : 1), O / 2>(sum, lane);
+}
+
 // A wave takes NR weight rows (four where the matrix is tall enough to keep every SIMD busy all the same: the activations
 // are then read once for four rows) and walks K in runs of 256, a float4 a lane; its sums meet by shuffles.
 // The head of the 0.5B widths (151,936 x 896, one row): 204 us before, 92 now, 5.9 TB/s.
@@ -280,8 +298,11 @@ __global__ __launch_bounds__(256) void rows_f32_kernel(const float* __restrict__
 #pragma unroll
   for (int j = 0; j < NR; ++j) w[j] = W + (size_t)min(n0 + j, N - 1) * ldw;
   float acc[MR][NR][2] = {};
-  // U runs of 256 at a time, all their loads on their way before the first is waited for (left to the scheduler, the loads of
-  // eight rows are waited for one by one: 8 rows against 1,536 of 8,960 26 us so, 78)
+  // Eight sums or more: U runs of 256 at a time, all their loads on their way before the first is waited for (left to the
+  // scheduler the loads of eight rows are waited for one by one: 8 rows against 1,536 of 8,960 26 us so, 78).  Fewer: the
+  // scheduler's order, which mixes the next run's loads with this one's products (4 rows against 512 of 8,960 10.0 us in runs
+  // of two, 8.4 so; four rows against four weight rows each the other way round: 24,000 of 260 6.4 and 8.0).
+  constexpr bool ORDERED = MR * NR >= 8;
   constexpr int U = MR * NR >= 16 ? 1 : 2;
   auto runs = [&](auto COUNT, int k) {
     constexpr int C = decltype(COUNT)::value;
@@ -293,7 +314,7 @@ __global__ __launch_bounds__(256) void rows_f32_kernel(const float* __restrict__
 #pragma unroll
       for (int i = 0; i < MR; ++i) a[u][i] = *reinterpret_cast<const float4*>(A + (size_t)min(i, M - 1) * lda + k + 256 * u);
     }
-    __builtin_amdgcn_sched_barrier(0);
+    if (ORDERED) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int u = 0; u < C; ++u)
 #pragma unroll
@@ -305,23 +326,27 @@ __global__ __launch_bounds__(256) void rows_f32_kernel(const float* __restrict__
         }
   };
   int k = lane * 4;
-  for (; k + 256 * (U - 1) < K; k += 256 * U) runs(std::integral_constant<int, U>{}, k);
-  if (U > 1 && k < K) runs(std::integral_constant<int, 1>{}, k);
-  float tot[MR][NR];
+  if constexpr (ORDERED) {
+    for (; k + 256 * (U - 1) < K; k += 256 * U) runs(std::integral_constant<int, U>{}, k);
+    if (U > 1 && k < K) runs(std::integral_constant<int, 1>{}, k);
+  } else {
+#pragma unroll 2
+    for (; k < K; k += 256) runs(std::integral_constant<int, 1>{}, k);
+  }
+  constexpr int SUMS = MR * NR;
+  float sum[SUMS];
 #pragma unroll
   for (int i = 0; i < MR; ++i)
 #pragma unroll
-    for (int j = 0; j < NR; ++j) tot[i][j] = wave_sum(acc[i][j][0] + acc[i][j][1]);
-  // lane i NR + j stores sum (i, j)
-#pragma unroll
-  for (int i = 0; i < MR; ++i)
-#pragma unroll
-    for (int j = 0; j < NR; ++j)
-      if (lane == i * NR + j && i < M && n0 + j < N) {
-        const float v = bias ? tot[i][j] + bias[n0 + j] : tot[i][j];
-        float* c = C + (size_t)i * ldc + n0 + j;
-        *c = ACCUMULATE ? *c + v : v;
-      }
+    for (int j = 0; j < NR; ++j) sum[i * NR + j] = acc[i][j][0] + acc[i][j][1];
+  meet<SUMS, 32>(sum, lane);
+  constexpr int EACH = 64 / SUMS;
+  const int i = lane / EACH / NR, n = n0 + lane / EACH % NR;
+  if (lane % EACH == 0 && i < M && n < N) {
+    const float v = bias ? sum[0] + bias[n] : sum[0];
+    float* c = C + (size_t)i * ldc + n;
+    *c = ACCUMULATE ? *c + v : v;
+  }
 }
 
 template <int MR, int NR>
@@ -333,11 +358,21 @@ int launch_rows(const float* A, int lda, const float* W, int ldw, const float* b
   return mf_launch_status();
 }
 
+constexpr int TALL = 16384;                       // weight rows from which a wave takes four of them
 template <int MR>
 int launch_rows_n(const float* A, int lda, const float* W, int ldw, const float* bias, float* C, int ldc, int M, int N, int K,
                   int accumulate, hipStream_t stream) {
-  return N >= 16384 ? launch_rows<MR, 4>(A, lda, W, ldw, bias, C, ldc, M, N, K, accumulate, stream)
-                    : launch_rows<MR, 1>(A, lda, W, ldw, bias, C, ldc, M, N, K, accumulate, stream);
+  return N >= TALL ? launch_rows<MR, 4>(A, lda, W, ldw, bias, C, ldc, M, N, K, accumulate, stream)
+                   : launch_rows<MR, 1>(A, lda, W, ldw, bias, C, ldc, M, N, K, accumulate, stream);
+}
+
+// At most 8 rows, K in 4s, except many weight rows of a short K: a wave's time does not fall with K below 256 (fewer of its lanes
+// have work, and its sums meet all the same), a tile's does.  As tiles / so: 8 rows against 100,000 of 48 11.4 us / 16.9, of
+// 80 17.0 / 17.9, one row of 16 5.2 / 6.7; 8 rows against 9,728 of 16 4.3 / 5.9, against 2,048 of 16 5.1 / 3.9.
+bool rows_take(int M, int N, int K) {
+  if (M > 8 || K % 4) return false;
+  const int mr = M <= 2 ? M : M <= 4 ? 4 : 8;
+  return K > (N >= TALL ? 8 * mr + (mr > 1 ? 16 : 8) : N >= 8192 ? 4 * mr : 0);
 }
 
 }  // namespace
@@ -355,7 +390,7 @@ MF_API int mf_gemm_f32(const float* A, int lda, const float* W, int ldw, const f
   if (K <= 0 || lda < K || ldw < K || ldc < N) return (int)hipErrorInvalidValue;
   const int vec_ok = (lda % 4 == 0) && (ldw % 4 == 0) && ((uintptr_t)A % 16 == 0) &&
                      ((uintptr_t)W % 16 == 0);
-  if (M <= 8 && vec_ok && K % 4 == 0) {
+  if (vec_ok && rows_take(M, N, K)) {
     if (M == 1) return launch_rows_n<1>(A, lda, W, ldw, bias, C, ldc, M, N, K, accumulate, stream);
     if (M == 2) return launch_rows_n<2>(A, lda, W, ldw, bias, C, ldc, M, N, K, accumulate, stream);
     if (M <= 4) return launch_rows_n<4>(A, lda, W, ldw, bias, C, ldc, M, N, K, accumulate, stream);

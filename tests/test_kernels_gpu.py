@@ -227,7 +227,10 @@ def test_gemm_f32(ops, m, n, k):
 # to the general kernel
 @pytest.mark.parametrize("m,n,k", [(1, 16387, 896), (2, 33, 36), (3, 16385, 260), (4, 896, 4864), (7, 130, 128), (8, 20001, 64),
                                    (9, 65, 32), (64, 64, 64), (65, 127, 96), (611, 896, 896), (100, 130, 4864), (33, 1001, 2080),
-                                   (1000, 1537, 160), (12, 100, 48), (5, 50, 35)])
+                                   (1000, 1537, 160), (12, 100, 48), (5, 50, 35),
+                                   # few rows against many weight rows, K at both sides of where tiles take them
+                                   (1, 16384, 16), (1, 16384, 20), (2, 16385, 32), (2, 16385, 36), (4, 16387, 48), (4, 16387, 52),
+                                   (8, 16390, 80), (7, 16390, 84), (8, 8193, 32), (6, 8193, 36), (3, 8191, 4)])
 def test_gemm_f32_kernels(ops, m, n, k):
     test_gemm_f32(ops, m, n, k)
 
