@@ -22,8 +22,9 @@ Kernel choice, for measurements (each overrides what `ops` would pick by shape):
 * MF_NO_FOLD=1          the RMS norm is a kernel of its own instead of being folded into the
                         product that follows it (steps of at most 16 rows)
 * MF_NO_LATENT_MFMA=1   the latent attention runs its plain kernel in bfloat16 as well, not the matrix-core one
-* MF_NO_NORM_AHEAD=1    in steps of 17 to 64 rows, a product that adds into the residual stream does
-                        not prepare the next norm's input: the norm is a kernel of its own
+* MF_NO_NORM_AHEAD=1    a product that adds into the residual stream does not prepare the next norm's
+                        input (steps of at most 64 rows) or norm the new rows behind its K split (more):
+                        the norm is a kernel of its own
 """
 from __future__ import annotations
 
