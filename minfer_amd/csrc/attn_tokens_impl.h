@@ -17,7 +17,7 @@
 // `attn_combine_kernel` merges them; the merge order is fixed, so results are the same
 // bits run to run.
 //
-// Used for decode in both precisions and for whole prompts in the 32-bit path.
+// Used for decode in both precisions; 32-bit prompts with heads of more than 128 too (`attn_prompt_f32.hip` takes the others).
 #pragma once
 #include <type_traits>
 #include "common.h"

@@ -68,6 +68,20 @@ class StepContext:
             self._memo[key] = (both[0], both[1])
         return self._memo[key]
 
+    def row_tiles(self, group: int, rows: int):
+        """(tile_seq, tile_row) int32 on the device: each sequence's (new token, head of a group of `group`) pairs in runs
+        of `rows`, the run with the most keys in sight first; kept like `query_tiles`."""
+        key = ("row_tiles", group, rows)
+        if key not in self._memo:
+            tiles = []
+            for b, n in enumerate(self.host_new):
+                first = self.host_start[b] if self.host_start else 0
+                tiles += [(first + min(r + rows - 1, n * group - 1) // group, b, r) for r in range(0, n * group, rows)]
+            tiles.sort(key=lambda t: -t[0])
+            both = torch.tensor([[t[1] for t in tiles], [t[2] for t in tiles]], dtype=torch.int32).to(self.token_ids.device)
+            self._memo[key] = (both[0], both[1])
+        return self._memo[key]
+
     def keys_in_sight(self, window: int = 0, chunk: int = 0):
         """(mean, most) keys that the step's new tokens see, from the host's copy of the step: how even a launch's work is
         and how long its longest walk.  `window`, `chunk`: 0 for none; with chunks the mean is rough (half a chunk)."""

@@ -28,6 +28,7 @@ LIBRARIES: Dict[str, str] = {
     "gemm_f32": "gemm_f32.hip",
     "gemm_bf16": "gemm_bf16.hip",
     "attn_tokens_f32": "attn_tokens_f32.hip",
+    "attn_prompt_f32": "attn_prompt_f32.hip",
     "attn_decode_bf16": "attn_decode_bf16.hip",
     "attn_prefill_bf16": "attn_prefill_bf16.hip",
     "attn_latent": "attn_latent.hip",
@@ -47,6 +48,7 @@ DEFINES: Dict[str, List[str]] = {}
 HEADERS = {"host_random": ["random_normal.h"],
            "elementwise": ["common.h", "random_normal.h"],
            "attn_tokens_f32": ["common.h", "attn_tokens_impl.h"],
+           "attn_prompt_f32": ["common.h", "attn_tokens_impl.h"],
            "attn_decode_bf16": ["common.h", "attn_tokens_impl.h", "noalloc.h"],
            "attn_capped": ["common.h", "attn_tokens_impl.h"],
            "attn_capped_mfma": ["common.h", "attn_tokens_impl.h"]}

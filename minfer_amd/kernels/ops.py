@@ -154,6 +154,12 @@ _PROTOTYPES = {
         "mf_attn_tokens_f32": [_P, _P, _P, _P, c_int, _P, _P, _P, _P, c_int, c_int, c_int, c_int,
                                c_float, c_int, c_int, c_int, _P],
     },
+    "attn_prompt_f32": {
+        "mf_attn_prompt_f32": [_P, _P, _P, _P, c_int, _P, _P, _P, _P, _P, _P, c_int, c_int, c_int, c_int, c_int, c_float, c_int,
+                               c_int, c_int, _P],
+        "mf_attn_prompt_f32_rows": [c_int],
+        "mf_attn_prompt_f32_keys": [],
+    },
     "attn_decode_bf16": {
         "mf_attn_decode_bf16": [_P, _P, _P, _P, c_int, _P, _P, _P, _P, c_int, c_int, c_int, c_int,
                                 c_float, c_int, c_int, c_int, _P],
@@ -2254,6 +2260,49 @@ def attn_tokens(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor, pag
         _ptr(q), _ptr(kcache), _ptr(vcache), _ptr(page_table), page_table.shape[1], _ptr(positions),
         _ptr(seq_of_tok), _ptr(out), _ptr(part), n_tok, n_heads, n_kv_heads, head_dim, float(scale),
         int(window or 0), n_splits, split_len, _stream()), "attn_tokens_f32")
+
+
+@functools.lru_cache(maxsize=256)
+def prompt_f32_rows(head_dim: int) -> int:
+    """Rows of a block of the 32-bit prompt attention; 0: a head size that it does not take (`attn_tokens` does)."""
+    return _fn("attn_prompt_f32", "mf_attn_prompt_f32_rows")(head_dim)
+
+
+def attn_prompt_f32(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor, page_table: torch.Tensor, ctx, out: torch.Tensor,
+                    n_heads: int, n_kv_heads: int, head_dim: int, scale: float, window: int) -> None:
+    """32-bit attention of a step that brings several tokens per sequence (what `attn_tokens` gives for it, on the 32-bit
+    matrix instruction).  `ctx` gives the ragged layout (cu_seqlens, start_pos, the rows in runs)."""
+    n_tok = ctx.n_tokens
+    _need(q, "attn_prompt.q", torch.float32, (n_tok, n_heads * head_dim))
+    _need(out, "attn_prompt.out", torch.float32, (n_tok, n_heads * head_dim))
+    _need_caches("attn_prompt", kcache, vcache, torch.float32, n_kv_heads, head_dim)
+    _need(page_table, "attn_prompt.page_table", torch.int32)
+    _need(ctx.cu_seqlens, "attn_prompt.cu_seqlens", torch.int32, (ctx.n_seqs + 1,))
+    _need(ctx.start_pos, "attn_prompt.start_pos", torch.int32, (ctx.n_seqs,))
+    rows = prompt_f32_rows(head_dim)
+    if not rows:
+        raise KernelError(f"attn_prompt: head_dim {head_dim} is not a multiple of 16 in [16, 128]")
+    if n_heads % n_kv_heads:
+        raise KernelError(f"attention: {n_heads} heads are not a multiple of {n_kv_heads} kv heads")
+    if ctx.max_len > page_table.shape[1] * PAGE or page_table.shape[0] != ctx.n_seqs:
+        raise KernelError(f"attention: page table {tuple(page_table.shape)} does not cover "
+                          f"{ctx.n_seqs} sequences of up to {ctx.max_len} positions")
+    tile_seq, tile_row = ctx.row_tiles(n_heads // n_kv_heads, rows)
+    n_splits, split_len = prompt_f32_splits(tile_seq.numel() * n_kv_heads, _fn("attn_prompt_f32", "mf_attn_prompt_f32_keys")(),
+                                            ctx.max_len, cu_count())
+    part = workspace("attn", n_tok * n_heads * n_splits * (head_dim + 2), q.device) if n_splits > 1 else None
+    _check(_fn("attn_prompt_f32", "mf_attn_prompt_f32")(
+        _ptr(q), _ptr(kcache), _ptr(vcache), _ptr(page_table), page_table.shape[1], _ptr(ctx.cu_seqlens), _ptr(ctx.start_pos),
+        _ptr(tile_seq), _ptr(tile_row), _ptr(out), _ptr(part), tile_seq.numel(), n_tok, n_heads, n_kv_heads, head_dim,
+        float(scale), int(window or 0), n_splits, split_len, _stream()), "attn_tokens_f32 (rows)")
+
+
+def prompt_f32_splits(blocks: int, keys: int, max_len: int, n_cu: int) -> Tuple[int, int]:
+    """(splits, keys of a split): the keys of the 32-bit prompt attention are cut where its blocks are fewer than two a CU (a
+    few new tokens on a long context), each part at least four turns of a block's waves (`keys` each)."""
+    n_splits = max(1, min(2 * n_cu // max(1, blocks), max_len // (4 * keys), 64))
+    split_len = ((max_len + n_splits - 1) // n_splits + PAGE - 1) // PAGE * PAGE
+    return (max_len + split_len - 1) // split_len, split_len
 
 
 def attn_decode_rope(qkv: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, kcache: torch.Tensor,

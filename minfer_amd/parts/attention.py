@@ -112,6 +112,8 @@ class GQAttention(Mixer):
         """Every new token of a step over its sequence's cache rows, the step's own stored already."""
         if self.rt.is_bf16 and not ctx.all_decode and ops.HAVE_PREFILL_ATTENTION:
             ops.attn_prefill(q, kc, vc, table, ctx, o, self.nh, self.nk, self.hd, self.scale, window)
+        elif not self.rt.is_bf16 and not ctx.all_decode and q.device.type == "cuda" and ops.prompt_f32_rows(self.hd):
+            ops.attn_prompt_f32(q, kc, vc, table, ctx, o, self.nh, self.nk, self.hd, self.scale, window)
         else:
             ops.attn_tokens(q, kc, vc, table, ctx.positions, ctx.seq_of_tok, o, self.nh, self.nk,
                             self.hd, self.scale, window, ctx.max_len)
