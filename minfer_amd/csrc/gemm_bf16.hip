@@ -153,6 +153,33 @@ __device__ __forceinline__ void tile_position(int tile, int tiles_m, int tiles_n
   bn = in_band / rows;
 }
 
+// The tile and the part of K that a block of a grid of (tiles, parts) takes.  Workgroups go to the 8 XCDs in turn, each with an
+// L2 of its own: every XCD gets one contiguous eighth of the tiles, so that what it has in flight are neighbours and share their
+// operands' rows in its L2 (ORDER_TILES: the same eighth of every part); or of the tiles of all parts, part by part
+// (ORDER_PARTS), so that an XCD brings in the activations of one part of K or two, and not those of all of K: for activations
+// that an L2 does not hold (`tile_order`).
+enum { ORDER_PLAIN = 0, ORDER_TILES = 1, ORDER_PARTS = 2 };
+__device__ __forceinline__ void block_work(int order, int& tile, int& part) {
+  int at = blockIdx.x, n = gridDim.x;
+  if (order == ORDER_PARTS) {
+    at += blockIdx.y * gridDim.x;
+    n *= gridDim.y;
+  }
+  if (order != ORDER_PLAIN) {
+    const int per = n / 8, rem = n % 8, x = at % 8;
+    at = x * per + min(x, rem) + at / 8;
+  }
+  part = order == ORDER_PARTS ? at / (int)gridDim.x : blockIdx.y;
+  tile = order == ORDER_PARTS ? at - part * (int)gridDim.x : at;
+}
+// Part by part where the activations of all of K are more than an XCD's L2 of 4 MB.  (rows x weight rows x K, microseconds with the
+// kernel behind it, the same eighth of every part / part by part: 2,048 x 2,048 x 8,192 78.1 / 73.8, 203 x 3,584 x 18,944 56.8 /
+// 53.9, 604 x 2,048 x 11,008 48.3 / 46.9, 400 x 1,536 x 8,960 29.5 / 28.2; but 604 x 2,048 x 2,048 22.2 / 24.8 and 400 x 896 x
+// 4,864 17.1 / 17.9.)
+int tile_order(int tiles, int splits, int M, int K) {
+  return splits > 1 && (size_t)M * K * 2 > (4u << 20) ? ORDER_PARTS : tiles >= 16 ? ORDER_TILES : ORDER_PLAIN;
+}
+
 // Rows of a product that belong to one of several matrices: `rows` of them (at most a tile's) from row `first` on.
 struct RowGroup { int first, rows, matrix, unused; };
 
@@ -163,17 +190,19 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN)) void tile_kernel(const 
                                                    const bf16* __restrict__ W, int ldw,
                                                    const float* __restrict__ bias, void* __restrict__ C,
                                                    int ldc, int M, int N, int K, int epi, int tiles_m,
-                                                   int xcd_remap, int k_per_split) {
+                                                   int order, int k_per_split) {
   constexpr int NTHR = 64 * (BM / WM) * (BN / WN);
   constexpr int LDS_LD = BK + 8;
+  int tile, part;
+  block_work(order, tile, part);
   if (k_per_split > 0) {
-    // K split over blockIdx.y: this block multiplies k_per_split of K and stores its sums, 32-bit
+    // K cut into parts: this block multiplies k_per_split of K and stores its sums, 32-bit
     // and without bias, into its own [M][N] slab of C; another kernel adds the slabs
-    const int kb = blockIdx.y * k_per_split;
+    const int kb = part * k_per_split;
     A += kb;
     W += kb;
     K = min(k_per_split, K - kb);
-    C = (float*)C + (size_t)blockIdx.y * M * N;
+    C = (float*)C + (size_t)part * M * N;
   }
   constexpr int TM = WM / 32, TN = WN / 32;
   constexpr int RP = NTHR / (BK / 8);         // rows per load pass
@@ -183,15 +212,6 @@ __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN)) void tile_kernel(const 
   bf16* As = reinterpret_cast<bf16*>(smem);               // [2][BM][LDS_LD]
   bf16* Ws = As + 2 * BM * LDS_LD;                        // [2][BN][LDS_LD]
 
-  // Workgroups go to the 8 XCDs in turn, each with an L2 of its own: give every XCD one
-  // contiguous eighth of the tile numbers, so that the tiles an XCD has in flight are neighbours
-  // and share their operands' rows in its L2.
-  int tile = blockIdx.x;
-  if (xcd_remap) {
-    const int n_tiles = gridDim.x, per = n_tiles / 8, rem = n_tiles % 8;
-    const int x = blockIdx.x % 8, qq = blockIdx.x / 8;
-    tile = x * per + min(x, rem) + qq;
-  }
   int bm, bn;
   tile_position(tile, tiles_m, gridDim.x / tiles_m, bm, bn);
   const int m0 = bm * BM, n0 = bn * BN;
@@ -487,27 +507,23 @@ __global__ __launch_bounds__(512, 2) void tile_dma_kernel(const bf16* __restrict
                                                        const bf16* __restrict__ W, int ldw,
                                                        const float* __restrict__ bias, void* __restrict__ C,
                                                        int ldc, int M, int N, int K, int epi, int tiles_m,
-                                                       int xcd_remap, int k_per_split,
+                                                       int order, int k_per_split,
                                                        const RowGroup* __restrict__ groups = nullptr) {
   using TT = DmaTile<BM, BN>;
   constexpr int ROW = DMA_BK * 2, A_ST = BM * ROW, W_ST = BN * ROW, W_AT = STAGES * A_ST;
   constexpr int I = TT::I, IH = TT::IH, J = TT::J, J0 = TT::J0, J1 = TT::J1, LA = TT::LA, LW0 = TT::LW0, LW1 = TT::LW1, T = TT::T;
+  int tile, part;
+  block_work(order, tile, part);
   if (k_per_split > 0) {
-    // K split over blockIdx.y (k_per_split a multiple of 64): this block multiplies its part of K
+    // K cut into parts (k_per_split a multiple of 64): this block multiplies its part of K
     // and stores 32-bit sums into its own [M][N] slab of C; another kernel adds the slabs
-    const int kb = blockIdx.y * k_per_split;
+    const int kb = part * k_per_split;
     A += kb;
     W += kb;
     K = min(k_per_split, K - kb);
-    C = (float*)C + (size_t)blockIdx.y * M * N;
+    C = (float*)C + (size_t)part * M * N;
   }
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];      // [stage][BM][64] of A, [stage][BN][64] of W
-  int tile = blockIdx.x;
-  if (xcd_remap) {
-    const int n_tiles = gridDim.x, per = n_tiles / 8, rem = n_tiles % 8;
-    const int x = blockIdx.x % 8, qq = blockIdx.x / 8;
-    tile = x * per + min(x, rem) + qq;
-  }
   int bm, bn;
   tile_position(tile, tiles_m, gridDim.x / tiles_m, bm, bn);
   if (GROUPED) {
@@ -706,26 +722,22 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void tile_step_kernel(const
                                                        const bf16* __restrict__ W, int ldw,
                                                        const float* __restrict__ bias, void* __restrict__ C,
                                                        int ldc, int M, int N, int K, int epi, int tiles_m,
-                                                       int xcd_remap, int k_per_split,
+                                                       int order, int k_per_split,
                                                        const RowGroup* __restrict__ groups = nullptr,
                                                        const float* __restrict__ in_ssq = nullptr, int in_parts = 0,
                                                        float in_eps = 0.f) {
   using TT = StepTile<BM, BN, WAVES_M, WAVES_N>;
   constexpr int ROW = DMA_BK * 2, ST = (BM + BN) * ROW, WAVES = TT::WAVES, I = TT::I, J = TT::J, LA = TT::LA, LW = TT::LW;
+  int tile, part;
+  block_work(order, tile, part);
   if (k_per_split > 0) {                                     // as in tile_dma_kernel
-    const int kb = blockIdx.y * k_per_split;
+    const int kb = part * k_per_split;
     A += kb;
     W += kb;
     K = min(k_per_split, K - kb);
-    C = (float*)C + (size_t)blockIdx.y * M * N;
+    C = (float*)C + (size_t)part * M * N;
   }
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];      // [stage][BM rows of A, BN rows of W][64]
-  int tile = blockIdx.x;
-  if (xcd_remap) {
-    const int n_tiles = gridDim.x, per = n_tiles / 8, rem = n_tiles % 8;
-    const int x = blockIdx.x % 8, qq = blockIdx.x / 8;
-    tile = x * per + min(x, rem) + qq;
-  }
   int bm, bn;
   tile_position(tile, tiles_m, gridDim.x / tiles_m, bm, bn);
   if (GROUPED) {
@@ -868,7 +880,7 @@ int launch_tile_step(const bf16* A, int lda, const bf16* W, int ldw, const float
   }
   const int tiles_m = GROUPED ? n_groups : (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
   kern<<<dim3(tiles_m * tiles_n, splits), 64 * TT::WAVES, TT::template lds<STAGES>(), stream>>>(
-      A, lda, W, ldw, bias, C, ldc, M, N, K, epi, tiles_m, tiles_m * tiles_n >= 16, k_per_split, groups, in_ssq, in_parts, in_eps);
+      A, lda, W, ldw, bias, C, ldc, M, N, K, epi, tiles_m, tile_order(tiles_m * tiles_n, splits, M, K), k_per_split, groups, in_ssq, in_parts, in_eps);
   return mf_launch_status();
 }
 
@@ -896,7 +908,7 @@ int launch_tile_dma(const bf16* A, int lda, const bf16* W, int ldw, const float*
   if (const int e = configure_tile_dma<BM, BN, STAGES, false>()) return e;
   const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
   tile_dma_kernel<BM, BN, STAGES><<<dim3(tiles_m * tiles_n, splits), 512, DmaTile<BM, BN>::template lds<STAGES>(), stream>>>(
-      A, lda, W, ldw, bias, C, ldc, M, N, K, epi, tiles_m, tiles_m * tiles_n >= 16, k_per_split, nullptr);
+      A, lda, W, ldw, bias, C, ldc, M, N, K, epi, tiles_m, tile_order(tiles_m * tiles_n, splits, M, K), k_per_split, nullptr);
   return mf_launch_status();
 }
 
@@ -915,7 +927,7 @@ int launch_tile_v(const bf16* A, int lda, const bf16* W, int ldw, const float* b
   }
   const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
   kern<<<dim3(tiles_m * tiles_n, splits), NTHR, smem, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi,
-                                                                tiles_m, tiles_m * tiles_n >= 16, k_per_split);
+                                                                tiles_m, tile_order(tiles_m * tiles_n, splits, M, K), k_per_split);
   return mf_launch_status();
 }
 
@@ -2199,21 +2211,28 @@ __global__ __launch_bounds__(256) void skinny_reduce4_kernel(const float* __rest
 // them next (more than 64 rows, where that product takes them normed): a block a row, which it holds in registers between
 // the sum of squares and the scaling.  The additions are those of `skinny_reduce4_kernel` and the norm that of
 // `rmsnorm_kernel`, in their order.  One launch for two, and the rows are not read again: 203 rows of 3,584 values in 9
-// parts 6.6 + 4.7 us as two kernels, 9.1 as this one; 2,048 rows in two parts 20.9 + 10.2 and 23.6.
-template <int KEEP>
-__global__ __launch_bounds__(256) void reduce_norm_kernel(const float* __restrict__ part, const float* __restrict__ bias,
+// parts 6.6 + 4.7 us as two kernels, 7.5 as this one; 2,048 rows in two parts 20.9 + 10.2 and 23.4.
+template <int KEEP, int NT>
+__global__ __launch_bounds__(NT) void reduce_norm_kernel(const float* __restrict__ part, const float* __restrict__ bias,
                                                           float* __restrict__ C, int ldc, int M, int N, int splits, int accumulate,
                                                           const float* __restrict__ g, float eps, bf16* __restrict__ normed) {
-  __shared__ float scratch[4];
+  __shared__ float scratch[NT / 64];
+  extern __shared__ __attribute__((aligned(16))) float row[];      // [N] (more than 256 threads)
   const int m = blockIdx.x;
   const size_t stride = (size_t)M * N;
   const float* p = part + (size_t)m * N;
   float* c = C + (size_t)m * ldc;
   float4 v[KEEP];
   float ss = 0.f;
+  auto squares = [&](const float4& x) {
+    ss = fmaf(x.x, x.x, ss);
+    ss = fmaf(x.y, x.y, ss);
+    ss = fmaf(x.z, x.z, ss);
+    ss = fmaf(x.w, x.w, ss);
+  };
 #pragma unroll
   for (int q = 0; q < KEEP; ++q) {
-    const int n = (q * 256 + threadIdx.x) * 4;
+    const int n = (q * NT + threadIdx.x) * 4;
     v[q] = float4{0.f, 0.f, 0.f, 0.f};
     if (n < N) {
       const float4 old = accumulate ? *reinterpret_cast<const float4*>(c + n) : v[q];
@@ -2232,16 +2251,19 @@ __global__ __launch_bounds__(256) void reduce_norm_kernel(const float* __restric
       if (accumulate) v[q] = float4{v[q].x + old.x, v[q].y + old.y, v[q].z + old.z, v[q].w + old.w};
       *reinterpret_cast<float4*>(c + n) = v[q];
     }
-    ss = fmaf(v[q].x, v[q].x, ss);
-    ss = fmaf(v[q].y, v[q].y, ss);
-    ss = fmaf(v[q].z, v[q].z, ss);
-    ss = fmaf(v[q].w, v[q].w, ss);
+    if (NT == 256) squares(v[q]);
+    else if (n < N) *reinterpret_cast<float4*>(row + n) = v[q];
   }
-  ss = block_sum<256>(ss, scratch);
+  if constexpr (NT > 256) {                                  // in the order in which 256 threads add them up
+    __syncthreads();
+    if (threadIdx.x < 256)
+      for (int n = threadIdx.x * 4; n < N; n += 1024) squares(*reinterpret_cast<const float4*>(row + n));
+  }
+  ss = block_sum<NT>(ss, scratch);
   const float scale = 1.0f / sqrtf(ss / (float)N + eps);
 #pragma unroll
   for (int q = 0; q < KEEP; ++q) {
-    const int n = (q * 256 + threadIdx.x) * 4;
+    const int n = (q * NT + threadIdx.x) * 4;
     if (n < N) {
       const float4 w = *reinterpret_cast<const float4*>(g + n);
       *reinterpret_cast<bf16x4*>(normed + (size_t)m * N + n) =
@@ -2254,14 +2276,23 @@ constexpr int REDUCE_NORM_MAX = 256 * 4 * 16;                // a row's values t
 
 int launch_reduce_norm(const float* part, const float* bias, float* C, int ldc, int M, int N, int splits, int accumulate,
                        const float* g, float eps, bf16* normed, hipStream_t stream) {
-  auto run = [&](auto KEEP) {
-    reduce_norm_kernel<decltype(KEEP)::value><<<M, 256, 0, stream>>>(part, bias, C, ldc, M, N, splits, accumulate, g, eps, normed);
+  auto run = [&](auto KEEP, auto NT) {
+    reduce_norm_kernel<decltype(KEEP)::value, decltype(NT)::value>
+        <<<M, decltype(NT)::value, NT > 256 ? N * sizeof(float) : 0, stream>>>(part, bias, C, ldc, M, N, splits, accumulate, g, eps, normed);
   };
-  if (N <= 1024) run(std::integral_constant<int, 1>{});
-  else if (N <= 2048) run(std::integral_constant<int, 2>{});
-  else if (N <= 4096) run(std::integral_constant<int, 4>{});
-  else if (N <= 8192) run(std::integral_constant<int, 8>{});
-  else run(std::integral_constant<int, 16>{});
+  auto with = [&](auto NT) {                                 // the values of a row that a thread holds, in fours
+    const int keep = (N + NT * 4 - 1) / (NT * 4);
+    if (keep <= 1) run(std::integral_constant<int, 1>{}, NT);
+    else if (keep <= 2) run(std::integral_constant<int, 2>{}, NT);
+    else if (keep <= 4) run(std::integral_constant<int, 4>{}, NT);
+    else if (NT == 256 && keep <= 8) run(std::integral_constant<int, NT == 256 ? 8 : 4>{}, NT);
+    else run(std::integral_constant<int, NT == 256 ? 16 : 4>{}, NT);
+  };
+  // Where no CU has two rows, a row's loads should all be on their way at once: 203 rows of 3,584 in 9 parts 9.9 us with 256
+  // threads a row, 7.5 with 1,024.  With more rows the blocks of a CU do that for each other: 604 rows of 2,048 in 6 parts 8.1
+  // and 8.5, 2,048 rows of 3,584 in 2 23.4 and 25.0.
+  if (M <= cu_count()) with(std::integral_constant<int, 1024>{});
+  else with(std::integral_constant<int, 256>{});
   return mf_launch_status();
 }
 
