@@ -18,6 +18,7 @@ from ..parts.base import (BLOCKS, COMBINERS, EMBEDDING_ENTRY, EMBEDDINGS, FEED_F
                           normed_input)
 from ..parts.spec import BlockSpec, ModelSpec
 from ..weights.loader import TensorSpec
+from .alike import AlikeLayers
 
 
 def _build_block(bs: BlockSpec, rt: Runtime):
@@ -157,6 +158,7 @@ class DecoderModel:
         rows = ctx.logit_rows
         last = len(s.schedule) - 1
         ctx.norm_ahead = None
+        alike = AlikeLayers() if self.rt.device.type == "cuda" and not ctx.all_decode else None      # (decode steps run captured)
         for n, e in enumerate(s.schedule):
             keep = rows if (n == last and rows is not None) else None
             ctx.kept_rows = keep                 # which of the step's tokens the block's feed-forward sees
@@ -167,7 +169,10 @@ class DecoderModel:
             if e.adds_embedding:
                 ops.add_rows(h, first)
                 ctx.norm_ahead = None
-            h = self.blocks[e.block].forward(h, ctx, e.cache, e.writes_cache, keep_rows=keep)
+            if alike is not None and keep is None:
+                h = alike.forward(self.blocks[e.block], h, ctx, e.cache, e.writes_cache)
+            else:
+                h = self.blocks[e.block].forward(h, ctx, e.cache, e.writes_cache, keep_rows=keep)
             ahead = ctx.norm_ahead
             if ahead is not None and (ahead.norm is not ctx.norm_after_block or ahead.h is not h):
                 ctx.norm_ahead = None            # prepared for someone who will not come

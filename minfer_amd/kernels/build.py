@@ -21,9 +21,11 @@ CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
 LIB_DIR = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "_lib")
 
 # library name -> source file; HEADERS: what each includes (default: common.h).  A `.cpp` source is
-# host code only and is built with the host compiler.
+# host code only and is built with the host compiler.  EXTENSIONS: those that are Python modules against torch's headers
+# (`load_extension`).
 LIBRARIES: Dict[str, str] = {
     "host_random": "host_random.cpp",
+    "host_call": "host_call.cpp",
     "elementwise": "elementwise.hip",
     "gemm_f32": "gemm_f32.hip",
     "gemm_bf16": "gemm_bf16.hip",
@@ -43,9 +45,11 @@ LIBRARIES: Dict[str, str] = {
     "sampling": "sampling.hip",
     "probe": "probe.hip",
 }
+EXTENSIONS = {"host_call": "mf_host_call"}
 # library name -> extra -D definitions (variants of one source compiled for given sizes, see `variant`)
 DEFINES: Dict[str, List[str]] = {}
 HEADERS = {"host_random": ["random_normal.h"],
+           "host_call": [],
            "elementwise": ["common.h", "random_normal.h"],
            "attn_tokens_f32": ["common.h", "attn_tokens_impl.h"],
            "attn_prompt_f32": ["common.h", "attn_tokens_impl.h"],
@@ -61,6 +65,28 @@ HOST_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-shared", "-pthread", "-ffp-contrac
 
 class KernelBuildError(RuntimeError):
     pass
+
+
+def _host_flags(name: str) -> List[str]:
+    """What a host library is compiled with; for an extension also where torch's and Python's headers and torch's
+    libraries are."""
+    if name not in EXTENSIONS:
+        return HOST_FLAGS
+    import sysconfig
+    import torch
+    root = os.path.dirname(torch.__file__)
+    return HOST_FLAGS + ["-I" + os.path.join(root, "include"), "-I" + sysconfig.get_paths()["include"],
+                         f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-L" + os.path.join(root, "lib"),
+                         "-ltorch_python", "-ltorch_cpu", "-lc10"]
+
+
+def _stamp_flags(name: str) -> List[str]:
+    """What besides its sources decides whether a built file is current: the flags, and for an extension the versions of
+    the interpreter and torch."""
+    if name not in EXTENSIONS:
+        return HOST_FLAGS if is_host_library(name) else HIPCC_FLAGS
+    import torch
+    return HOST_FLAGS + [sys.version, torch.__version__]
 
 
 def variant(base: str, **sizes: int) -> str:
@@ -126,7 +152,7 @@ def _host_compiler() -> str:
 
 def source_hash(name: str) -> str:
     h = hashlib.sha256()
-    h.update(" ".join((HOST_FLAGS if is_host_library(name) else HIPCC_FLAGS) + DEFINES.get(name, [])).encode())
+    h.update(" ".join(_stamp_flags(name) + DEFINES.get(name, [])).encode())
     for fname in [LIBRARIES[name]] + HEADERS.get(name, ["common.h"]):
         with open(os.path.join(CSRC, fname), "rb") as f:
             h.update(fname.encode())
@@ -177,7 +203,9 @@ def compile_library(name: str, quiet: bool = False) -> str:
     so = lib_path(name)
     tmp = f"{so}.{os.getpid()}.tmp"
     if is_host_library(name):
-        cmd = [_host_compiler()] + HOST_FLAGS + ["-I", CSRC, os.path.join(CSRC, LIBRARIES[name]), "-o", tmp]
+        flags = _host_flags(name)
+        libs = [f for f in flags if f.startswith("-l")]
+        cmd = [_host_compiler()] + [f for f in flags if f not in libs] + ["-I", CSRC, os.path.join(CSRC, LIBRARIES[name]), "-o", tmp] + libs
     else:
         cmd = [_hipcc()] + HIPCC_FLAGS + DEFINES.get(name, []) + ["-I", CSRC, os.path.join(CSRC, LIBRARIES[name]), "-o", tmp]
     if not quiet:
@@ -239,6 +267,27 @@ def build_all(force: bool = True, jobs: int = 4) -> List[str]:
 
 _loaded: Dict[str, ctypes.CDLL] = {}
 _load_lock = threading.Lock()
+_modules: Dict[str, object] = {}
+
+
+def load_extension(name: str):
+    """The Python module built from an extension's source, compiled first if it is missing or its source changed."""
+    import importlib.machinery
+    import importlib.util
+    with _load_lock:
+        module = _modules.get(name)
+        if module is None:
+            if not is_current(name):
+                compile_library(name)
+            loader = importlib.machinery.ExtensionFileLoader(EXTENSIONS[name], lib_path(name))
+            spec = importlib.util.spec_from_file_location(EXTENSIONS[name], lib_path(name), loader=loader)
+            try:
+                module = importlib.util.module_from_spec(spec)
+                loader.exec_module(module)
+            except ImportError as e:
+                raise KernelBuildError(f"cannot load {lib_path(name)}: {e}") from None
+            _modules[name] = module
+        return module
 
 
 def load(name: str) -> ctypes.CDLL:

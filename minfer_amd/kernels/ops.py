@@ -186,17 +186,45 @@ _PROTOTYPES = {
 _functions: Dict[str, object] = {}
 
 
+_KINDS = {c_void_p: "p", c_char_p: "p", c_int: "i", c_int64: "q", c_size_t: "q", c_uint64: "q", c_float: "f", c_double: "d"}
+_launch = None           # `Launch` of csrc/host_call.cpp, once a library is called
+
+
+def _native_calls():
+    """Loads the extension that checks operands and calls the libraries, and puts its check in `_need`'s place."""
+    global _launch, _need
+    module = build.load_extension("host_call")
+    module.otherwise(_need_in_general)
+    _launch, _need = module.Launch, module.need
+    return _launch
+
+
 def _fn(lib: str, name: str, variant: Optional[str] = None):
-    """`variant`: the name of a sized variant of `lib` (`build.variant`), whose functions have the
-    prototypes of `lib`."""
+    """A library's entry point, called with tensors, numbers and None.  `variant`: the name of a sized variant of `lib`
+    (`build.variant`), whose functions have the prototypes of `lib`."""
     key = name if variant is None else f"{variant}:{name}"
     f = _functions.get(key)
     if f is None:
-        f = getattr(build.load(variant or lib), name)
-        f.argtypes = _PROTOTYPES[lib][name]
-        f.restype = c_int
+        address = ctypes.cast(getattr(build.load(variant or lib), name), c_void_p).value
+        kinds = "".join(_KINDS[t] for t in _PROTOTYPES[lib][name])
+        # (what launches ends with the stream; the tile plan ends with the place for its answer)
+        f = (_launch or _native_calls())(address, kinds, kinds.endswith("p") and name != "mf_gemm_bf16_tile_plan")
         _functions[key] = f
     return f
+
+
+def record_launches():
+    """A `Record` of csrc/host_call.cpp: the launches made under `with record:`, to be made again with other tensors in
+    some places.  None while launches are timed or waited for one by one (those go through `_check`)."""
+    if _trace is not None or tuning.DEBUG_SYNC:
+        return None
+    if _launch is None:
+        _native_calls()
+    return build.load_extension("host_call").Record()
+
+
+def check_recorded(rc: int) -> None:
+    _check(rc, "recorded launches of a layer")
 
 
 def _stream() -> int:
@@ -224,10 +252,6 @@ def _check(rc: int, what: str) -> None:
         print(f"[minfer_amd] {what} OK", file=sys.stderr, flush=True)
 
 
-def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
-    return None if t is None else t.data_ptr()
-
-
 # ------------------------------------------------------------------ per-launch timing
 _trace: Optional[list] = None
 
@@ -252,11 +276,8 @@ def stop_trace():
     return [(name, events[i - 1][1].elapsed_time(ev) * 1e3) for i, (name, ev) in enumerate(events) if i]
 
 
-def _need(t: torch.Tensor, name: str, dtype=None, shape=None) -> None:
-    # (a launch checks some seven tensors: what is right is found so in one expression, what is not is named below)
-    if isinstance(t, torch.Tensor) and t.is_cuda and t.is_contiguous() and \
-            (dtype is None or t.dtype is dtype or dtype is _FLOATS and t.dtype in _FLOATS) and (shape is None or t.shape == shape):
-        return
+def _need_in_general(t: torch.Tensor, name: str, dtype=None, shape=None) -> None:
+    """Raises, naming it, where `t` is no contiguous tensor on the GPU of that type (one, or several) and shape."""
     if not isinstance(t, torch.Tensor) or not t.is_cuda:
         raise KernelError(f"{name}: must be a tensor on the GPU (there is no CPU path)")
     if not t.is_contiguous():
@@ -267,6 +288,9 @@ def _need(t: torch.Tensor, name: str, dtype=None, shape=None) -> None:
             raise KernelError(f"{name}: dtype {t.dtype}, expected {dtype}")
     if shape is not None and tuple(t.shape) != tuple(shape):
         raise KernelError(f"{name}: shape {tuple(t.shape)}, expected {tuple(shape)}")
+
+
+_need = _need_in_general          # (`need` of csrc/host_call.cpp, which passes what is right, once a library is called)
 
 
 def _is_bf16(t: torch.Tensor) -> int:
@@ -384,7 +408,7 @@ def embed(table: torch.Tensor, ids: torch.Tensor, out: torch.Tensor, scale: floa
     _need(ids, "embed.ids", torch.int32)
     n, d = ids.numel(), table.shape[1]
     _need(out, "embed.out", torch.float32, (n, d))
-    _check(_fn("elementwise", "mf_embed")(_ptr(table), _is_bf16(table), _ptr(ids), _ptr(out), n, d,
+    _check(_fn("elementwise", "mf_embed")(table, _is_bf16(table), ids, out, n, d,
                                            table.shape[0], float(scale), _stream()), "embed")
 
 
@@ -407,8 +431,8 @@ def embed_pairs(table: torch.Tensor, pairs: torch.Tensor, ids: torch.Tensor, pos
     if buckets < 1 or max(abs(int(mul_prev)), abs(int(mul_cur))) >= 1 << 31:
         raise KernelError(f"embed_pairs: {buckets} buckets, factors {mul_prev} and {mul_cur}")
     _check(_fn("elementwise", "mf_embed_pairs")(
-        _ptr(table), _ptr(pairs), _is_bf16(table), _ptr(ids), _ptr(positions), _ptr(seq_of_tok), _ptr(cu_seqlens), _ptr(slot_ids),
-        _ptr(last), _ptr(out), n, d, table.shape[0], buckets, int(mul_prev), int(mul_cur), float(scale), _stream()), "embed_pairs")
+        table, pairs, _is_bf16(table), ids, positions, seq_of_tok, cu_seqlens, slot_ids,
+        last, out, n, d, table.shape[0], buckets, int(mul_prev), int(mul_cur), float(scale), _stream()), "embed_pairs")
 
 
 def rmsnorm(x: torch.Tensor, weight: Optional[torch.Tensor], eps: float, out: torch.Tensor,
@@ -423,7 +447,7 @@ def rmsnorm(x: torch.Tensor, weight: Optional[torch.Tensor], eps: float, out: to
         _need(out, "rmsnorm.out", _FLOATS, (rows, cols))
         if weight is not None:
             _need(weight, "rmsnorm.weight", torch.float32, (cols,))
-        _check(_fn("elementwise", "mf_rmsnorm_cols")(_ptr(x), x.shape[1], _ptr(weight), _ptr(out), _is_bf16(out), rows, cols,
+        _check(_fn("elementwise", "mf_rmsnorm_cols")(x, x.shape[1], weight, out, _is_bf16(out), rows, cols,
                                                       float(eps), _stream()), "rmsnorm")
         return
     d = x.shape[-1]
@@ -435,7 +459,7 @@ def rmsnorm(x: torch.Tensor, weight: Optional[torch.Tensor], eps: float, out: to
         _need(row_idx, "rmsnorm.row_idx", torch.int32, (rows,))
     elif x.shape[0] != rows:
         raise KernelError(f"rmsnorm: x has {x.shape[0]} rows, out has {rows}")
-    _check(_fn("elementwise", "mf_rmsnorm")(_ptr(x), _ptr(row_idx), _ptr(weight), _ptr(out),
+    _check(_fn("elementwise", "mf_rmsnorm")(x, row_idx, weight, out,
                                              _is_bf16(out), rows, d, float(eps), _stream()), "rmsnorm")
 
 
@@ -443,7 +467,7 @@ def gather_rows(x: torch.Tensor, idx: torch.Tensor, out: torch.Tensor) -> None:
     _need(x, "gather_rows.x", torch.float32)
     _need(idx, "gather_rows.idx", torch.int32)
     _need(out, "gather_rows.out", torch.float32, (idx.numel(), x.shape[1]))
-    _check(_fn("elementwise", "mf_gather_rows")(_ptr(x), _ptr(idx), _ptr(out), idx.numel(),
+    _check(_fn("elementwise", "mf_gather_rows")(x, idx, out, idx.numel(),
                                                  x.shape[1], _stream()), "gather_rows")
 
 
@@ -457,7 +481,7 @@ def swiglu(gate_up: torch.Tensor, out: torch.Tensor, limit: float = 0.0) -> None
     _need(out, "swiglu.out", _FLOATS, (rows, two_nf // 2))
     if _is_bf16(gate_up) and not _is_bf16(out):
         raise KernelError("swiglu: bfloat16 input with float32 output is not provided")
-    _check(_fn("elementwise", "mf_swiglu")(_ptr(gate_up), _is_bf16(gate_up), _ptr(out), _is_bf16(out),
+    _check(_fn("elementwise", "mf_swiglu")(gate_up, _is_bf16(gate_up), out, _is_bf16(out),
                                             rows, two_nf // 2, float(limit), _stream()), "swiglu")
 
 
@@ -466,7 +490,7 @@ def convert(src: torch.Tensor, dst: torch.Tensor) -> None:
     _need(dst, "convert.dst", _FLOATS)
     if src.numel() != dst.numel() or src.dtype == dst.dtype:
         raise KernelError("convert: needs equal sizes and different types")
-    _check(_fn("elementwise", "mf_convert")(_ptr(src), _is_bf16(src), _ptr(dst), _is_bf16(dst),
+    _check(_fn("elementwise", "mf_convert")(src, _is_bf16(src), dst, _is_bf16(dst),
                                              src.numel(), _stream()), "convert")
 
 
@@ -474,7 +498,7 @@ def fill_normal(out: torch.Tensor, seed: int, std: float, round_bf16: bool = Tru
     """N(0, std) values that depend on (seed, index) only, the same bits as `fill_normal_host`
     gives.  `round_bf16`: a float32 tensor gets values that bfloat16 represents."""
     _need(out, "fill_normal.out", _FLOATS)
-    _check(_fn("elementwise", "mf_fill_normal")(_ptr(out), _is_bf16(out), out.numel(),
+    _check(_fn("elementwise", "mf_fill_normal")(out, _is_bf16(out), out.numel(),
                                                  seed & 0xFFFFFFFFFFFFFFFF, float(std), 1 if round_bf16 else 0,
                                                  _stream()), "fill_normal")
 
@@ -485,7 +509,7 @@ def fill_normal_host(out: torch.Tensor, seed: int, std: float, round_bf16: bool 
     if not isinstance(out, torch.Tensor) or out.is_cuda or not out.is_contiguous() or out.dtype not in _FLOATS:
         raise KernelError("fill_normal_host: needs a contiguous float32 or bfloat16 tensor on the CPU")
     threads = threads or max(1, min(16, os.cpu_count() or 1))
-    rc = _fn("host_random", "mf_fill_normal_host")(c_void_p(out.data_ptr()), _is_bf16(out), out.numel(),
+    rc = _fn("host_random", "mf_fill_normal_host")(out.data_ptr(), _is_bf16(out), out.numel(),
                                                     seed & 0xFFFFFFFFFFFFFFFF, float(std),
                                                     1 if round_bf16 else 0, threads)
     if rc != 0:
@@ -496,7 +520,7 @@ def rope_table(n_pos: int, half: int, theta: float, freq_scale: float, device):
     cs = torch.empty((n_pos, half), dtype=torch.float32, device=device)
     sn = torch.empty((n_pos, half), dtype=torch.float32, device=device)
     _need(cs, "rope_table.out")
-    _check(_fn("elementwise", "mf_rope_table")(_ptr(cs), _ptr(sn), n_pos, half, float(theta),
+    _check(_fn("elementwise", "mf_rope_table")(cs, sn, n_pos, half, float(theta),
                                                 float(freq_scale), _stream()), "rope_table")
     return cs, sn
 
@@ -512,7 +536,7 @@ def rope_inplace(qkv: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, positi
     if cos.shape[1] != head_dim // 2 or head_dim % 2 or n_rot_heads > n_heads_total:
         raise KernelError(f"rope_inplace: table {tuple(cos.shape)}, head_dim {head_dim}, {n_rot_heads} of {n_heads_total} heads")
     _need(positions, "rope_inplace.positions", torch.int32, (n_tok,))
-    _check(_fn("elementwise", "mf_rope_inplace")(_ptr(qkv), _ptr(cos), _ptr(sin), _ptr(positions), n_tok,
+    _check(_fn("elementwise", "mf_rope_inplace")(qkv, cos, sin, positions, n_tok,
                                                   n_rot_heads, n_heads_total, head_dim, _stream()), "rope_inplace")
 
 
@@ -546,10 +570,10 @@ def rope_kvwrite(qkv: torch.Tensor, cos: Optional[torch.Tensor], sin: Optional[t
     if write_kv:
         _need_caches("rope", kcache, vcache, q_out.dtype, n_kv_heads, head_dim)
     _check(_fn("elementwise", "mf_rope_kvwrite")(
-        _ptr(qkv), _ptr(cos), _ptr(sin), _ptr(positions), _ptr(seq_of_tok), _ptr(page_table),
-        page_table.shape[1], _ptr(q_out), _ptr(kcache if write_kv else None),
-        _ptr(vcache if write_kv else None), _is_bf16(q_out), n_tok, n_heads, n_kv_heads, head_dim,
-        1 if write_kv else 0, parts, _ptr(bias), _stream()), "rope_kvwrite")
+        qkv, cos, sin, positions, seq_of_tok, page_table,
+        page_table.shape[1], q_out, kcache if write_kv else None,
+        vcache if write_kv else None, _is_bf16(q_out), n_tok, n_heads, n_kv_heads, head_dim,
+        1 if write_kv else 0, parts, bias, _stream()), "rope_kvwrite")
 
 
 # ------------------------------------------------------------------ norm in groups, xIELU, frequency tables
@@ -574,8 +598,8 @@ def group_rmsnorm(x: torch.Tensor, weight: Optional[torch.Tensor], eps: float, g
         raise KernelError(f"group_rmsnorm: x has {x.shape[0]} rows, out has {rows}")
     if cast_out is not None:
         _need(cast_out, "group_rmsnorm.cast_out", torch.bfloat16, (rows, d))
-    _check(_fn("elementwise", "mf_group_rmsnorm")(_ptr(x), _ptr(row_idx), _ptr(weight), _ptr(out), _is_bf16(out),
-                                                   1 if add else 0, _ptr(cast_out), rows, d, int(groups), float(eps),
+    _check(_fn("elementwise", "mf_group_rmsnorm")(x, row_idx, weight, out, _is_bf16(out),
+                                                   1 if add else 0, cast_out, rows, d, int(groups), float(eps),
                                                    _stream()), "group_rmsnorm")
 
 
@@ -583,7 +607,7 @@ def xielu(x: torch.Tensor, out: torch.Tensor, a_pos: float, a_neg: float) -> Non
     """out = a_pos x^2 + x/2 where x > 0, a_neg (e^x - 1 - x) + x/2 elsewhere; x float32, out run type."""
     _need(x, "xielu.x", torch.float32)
     _need(out, "xielu.out", _FLOATS, tuple(x.shape))
-    _check(_fn("elementwise", "mf_xielu")(_ptr(x), _ptr(out), _is_bf16(out), x.numel(), float(a_pos), float(a_neg),
+    _check(_fn("elementwise", "mf_xielu")(x, out, _is_bf16(out), x.numel(), float(a_pos), float(a_neg),
                                            _stream()), "xielu")
 
 
@@ -595,7 +619,7 @@ def rope_table_freqs(n_pos: int, freqs, magnitude: float, device):
     cs = torch.empty((n_pos, half), dtype=torch.float32, device=device)
     sn = torch.empty((n_pos, half), dtype=torch.float32, device=device)
     _need(cs, "rope_table_freqs.out")
-    _check(_fn("elementwise", "mf_rope_table_freqs")(_ptr(cs), _ptr(sn), _ptr(f), n_pos, half, float(magnitude),
+    _check(_fn("elementwise", "mf_rope_table_freqs")(cs, sn, f, n_pos, half, float(magnitude),
                                                       _stream()), "rope_table_freqs")
     return cs, sn
 
@@ -613,7 +637,7 @@ def rope_pairs_inplace(qkv: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, 
         raise KernelError(f"rope_pairs_inplace: table {tuple(cos.shape)}, head_dim {head_dim}, "
                           f"{n_rot_heads} of {n_heads_total} heads")
     _need(positions, "rope_pairs_inplace.positions", torch.int32, (n_tok,))
-    _check(_fn("elementwise", "mf_rope_pairs_inplace")(_ptr(qkv), _ptr(cos), _ptr(sin), _ptr(positions), n_tok,
+    _check(_fn("elementwise", "mf_rope_pairs_inplace")(qkv, cos, sin, positions, n_tok,
                                                         n_rot_heads, n_heads_total, head_dim, cos.shape[1],
                                                         _stream()), "rope_pairs_inplace")
 
@@ -632,15 +656,15 @@ def embed_pos(table: torch.Tensor, pos_table: torch.Tensor, ids: torch.Tensor, p
     _need(ids, "embed_pos.ids", torch.int32)
     _need(positions, "embed_pos.positions", torch.int32, (n,))
     _need(out, "embed_pos.out", torch.float32, (n, d))
-    _check(_fn("elementwise", "mf_embed_pos")(_ptr(table), _ptr(pos_table), _is_bf16(table), _ptr(ids), _ptr(positions),
-                                               _ptr(out), n, d, table.shape[0], pos_table.shape[0], _stream()), "embed_pos")
+    _check(_fn("elementwise", "mf_embed_pos")(table, pos_table, _is_bf16(table), ids, positions,
+                                               out, n, d, table.shape[0], pos_table.shape[0], _stream()), "embed_pos")
 
 
 def gelu_tanh(x: torch.Tensor, out: torch.Tensor) -> None:
     """out = 0.5 x (1 + tanh(sqrt(2/pi) (x + 0.044715 x^3))) from 32-bit values, rounded once."""
     _need(x, "gelu_tanh.x", torch.float32)
     _need(out, "gelu_tanh.out", _FLOATS, tuple(x.shape))
-    _check(_fn("elementwise", "mf_gelu_tanh")(_ptr(x), _ptr(out), _is_bf16(out), x.numel(), _stream()), "gelu_tanh")
+    _check(_fn("elementwise", "mf_gelu_tanh")(x, out, _is_bf16(out), x.numel(), _stream()), "gelu_tanh")
 
 
 def softcap(x: torch.Tensor, cap: float) -> None:
@@ -648,7 +672,7 @@ def softcap(x: torch.Tensor, cap: float) -> None:
     _need(x, "softcap.x", torch.float32)
     if not cap > 0:
         raise KernelError(f"softcap: cap {cap} must be positive")
-    _check(_fn("elementwise", "mf_softcap")(_ptr(x), float(cap), x.numel(), _stream()), "softcap")
+    _check(_fn("elementwise", "mf_softcap")(x, float(cap), x.numel(), _stream()), "softcap")
 
 
 def weighted_sum(buffers, weights: torch.Tensor, out: torch.Tensor, row_idx: Optional[torch.Tensor] = None,
@@ -670,22 +694,22 @@ def weighted_sum(buffers, weights: torch.Tensor, out: torch.Tensor, row_idx: Opt
     if rows == 0:
         return
     ptrs = (c_void_p * n)(*[b.data_ptr() for b in buffers])
-    _check(_fn("elementwise", "mf_weighted_sum")(ptrs, n, int(n_indexed), _ptr(row_idx if n_indexed else None),
-                                                  _ptr(weights), _ptr(out), rows, d, _stream()), "weighted_sum")
+    _check(_fn("elementwise", "mf_weighted_sum")(ptrs, n, int(n_indexed), row_idx if n_indexed else None,
+                                                  weights, out, rows, d, _stream()), "weighted_sum")
 
 
 def add_rows(h: torch.Tensor, x: torch.Tensor) -> None:
     """h += x, both float32 of one shape."""
     _need(h, "add_rows.h", torch.float32)
     _need(x, "add_rows.x", torch.float32, tuple(h.shape))
-    _check(_fn("elementwise", "mf_add_rows")(_ptr(h), _ptr(x), h.numel(), _stream()), "add_rows")
+    _check(_fn("elementwise", "mf_add_rows")(h, x, h.numel(), _stream()), "add_rows")
 
 
 def relu2(x: torch.Tensor, out: torch.Tensor) -> None:
     """out = max(x, 0)^2; x float32, out run type."""
     _need(x, "relu2.x", torch.float32)
     _need(out, "relu2.out", _FLOATS, tuple(x.shape))
-    _check(_fn("elementwise", "mf_relu2")(_ptr(x), _ptr(out), _is_bf16(out), x.numel(), _stream()), "relu2")
+    _check(_fn("elementwise", "mf_relu2")(x, out, _is_bf16(out), x.numel(), _stream()), "relu2")
 
 
 def layernorm(x: torch.Tensor, weight: torch.Tensor, eps: float, out: torch.Tensor,
@@ -700,7 +724,7 @@ def layernorm(x: torch.Tensor, weight: torch.Tensor, eps: float, out: torch.Tens
         _need(row_idx, "layernorm.row_idx", torch.int32, (rows,))
     elif x.shape[0] != rows:
         raise KernelError(f"layernorm: x has {x.shape[0]} rows, out has {rows}")
-    _check(_fn("elementwise", "mf_layernorm")(_ptr(x), _ptr(row_idx), _ptr(weight), _ptr(out), _is_bf16(out), rows, d,
+    _check(_fn("elementwise", "mf_layernorm")(x, row_idx, weight, out, _is_bf16(out), rows, d,
                                                float(eps), _stream()), "layernorm")
 
 
@@ -714,7 +738,7 @@ def layernorm_join(h: torch.Tensor, y: torch.Tensor, alpha: float, weight: torch
     _need(weight, "layernorm_join.weight", torch.float32, (d,))
     if cast_out is not None:
         _need(cast_out, "layernorm_join.cast_out", torch.bfloat16, (rows, d))
-    _check(_fn("elementwise", "mf_layernorm_join")(_ptr(h), _ptr(y), float(alpha), _ptr(weight), _ptr(cast_out), rows, d,
+    _check(_fn("elementwise", "mf_layernorm_join")(h, y, float(alpha), weight, cast_out, rows, d,
                                                     float(eps), _stream()), "layernorm_join")
 
 
@@ -727,7 +751,7 @@ def rmsnorm_pair(a: torch.Tensor, wa: torch.Tensor, b: torch.Tensor, wb: torch.T
     _need(wa, "rmsnorm_pair.wa", torch.float32, (d,))
     _need(wb, "rmsnorm_pair.wb", torch.float32, (d,))
     _need(out, "rmsnorm_pair.out", torch.float32, (rows, d))
-    _check(_fn("elementwise", "mf_rmsnorm_pair")(_ptr(a), _ptr(wa), _ptr(b), _ptr(wb), _ptr(out), rows, d, float(eps),
+    _check(_fn("elementwise", "mf_rmsnorm_pair")(a, wa, b, wb, out, rows, d, float(eps),
                                                   float(scale), 1 if accumulate else 0, _stream()), "rmsnorm_pair")
 
 
@@ -773,8 +797,8 @@ def gated_scan(proj: torch.Tensor, lower: torch.Tensor, cu_seqlens: torch.Tensor
     if dim > 256:
         raise KernelError(f"gated_scan: key width {dim} is beyond 256")
     if chunks is None:
-        _check(_fn("gated_recurrence", "mf_gated_scan")(_ptr(proj), _ptr(lower), _ptr(cu_seqlens), _ptr(slot_ids),
-                                                        _ptr(state), _ptr(out), n_seqs, n_heads, dim, v_dim, _stream()),
+        _check(_fn("gated_recurrence", "mf_gated_scan")(proj, lower, cu_seqlens, slot_ids,
+                                                        state, out, n_seqs, n_heads, dim, v_dim, _stream()),
                "gated_scan")
         return
     table, n_chunks = chunks
@@ -782,8 +806,8 @@ def gated_scan(proj: torch.Tensor, lower: torch.Tensor, cu_seqlens: torch.Tensor
     per = n_heads * dim * v_dim
     ws = workspace("gr_chunks", n_chunks * (per + n_heads * dim), proj.device)
     _check(_fn("gated_recurrence", "mf_gated_scan_chunked")(
-        _ptr(proj), _ptr(lower), _ptr(table), n_chunks, c_void_p(table.data_ptr() + 16 * n_chunks), _ptr(slot_ids),
-        _ptr(state), _ptr(ws), c_void_p(ws.data_ptr() + 4 * n_chunks * per), _ptr(out), n_seqs, n_heads, dim, v_dim,
+        proj, lower, table, n_chunks, table.data_ptr() + 16 * n_chunks, slot_ids,
+        state, ws, ws.data_ptr() + 4 * n_chunks * per, out, n_seqs, n_heads, dim, v_dim,
         _stream()), "gated_scan_chunked")
 
 
@@ -812,14 +836,14 @@ def low_rank_scan(proj: torch.Tensor, a2: torch.Tensor, bias: torch.Tensor, off_
     if chunks is not None:
         table, n_chunks = chunks
         _need(table, "low_rank_scan.chunks", torch.int32, (4 * n_chunks + n_seqs + 1,))
-        first = c_void_p(table.data_ptr() + 16 * n_chunks)
+        first = table.data_ptr() + 16 * n_chunks
         per = n_heads * dim * v_dim
         buf = workspace("gr_chunks", n_chunks * (per + n_heads * dim) + n_tok * n_heads * dim, proj.device)
-        ws, ws_a = _ptr(buf), c_void_p(buf.data_ptr() + 4 * n_chunks * per)
-        decays = c_void_p(buf.data_ptr() + 4 * n_chunks * (per + n_heads * dim))
+        ws, ws_a = buf, buf.data_ptr() + 4 * n_chunks * per
+        decays = buf.data_ptr() + 4 * n_chunks * (per + n_heads * dim)
     _check(_fn("gated_recurrence", "mf_low_rank_scan")(
-        _ptr(proj), row_len, _ptr(a2), _ptr(bias), rank, int(off_r), 1.0 / float(tau), float(q_scale), _ptr(cu_seqlens),
-        _ptr(table), n_chunks, first, _ptr(slot_ids), _ptr(state), ws, ws_a, decays, _ptr(out), n_tok, n_seqs, n_heads, dim,
+        proj, row_len, a2, bias, rank, int(off_r), 1.0 / float(tau), float(q_scale), cu_seqlens,
+        table, n_chunks, first, slot_ids, state, ws, ws_a, decays, out, n_tok, n_seqs, n_heads, dim,
         v_dim, _stream()), "low_rank_scan" if chunks is None else "low_rank_scan_chunked")
 
 
@@ -834,7 +858,7 @@ def head_rmsnorm(o: torch.Tensor, weight: Optional[torch.Tensor], eps: float, ou
     if weight is not None:
         _need(weight, "head_rmsnorm.weight", torch.float32, (n // n_heads,))
     _need(out, "head_rmsnorm.out", _FLOATS, (rows, n))
-    _check(_fn("gated_recurrence", "mf_head_rmsnorm")(_ptr(o), _ptr(weight), _ptr(out), _is_bf16(out), rows, n_heads,
+    _check(_fn("gated_recurrence", "mf_head_rmsnorm")(o, weight, out, _is_bf16(out), rows, n_heads,
                                                       n // n_heads, float(eps), float(scale), _stream()), "head_rmsnorm")
 
 
@@ -881,10 +905,10 @@ def qk_norm_prep(qkv: torch.Tensor, q_gain: Optional[torch.Tensor], k_gain: Opti
     _need(seq_of_tok, "qk_norm_prep.seq_of_tok", torch.int32, (n_tok,))
     _need(positions, "qk_norm_prep.positions", torch.int32, (n_tok,))
     _check(_fn("attn_normed", "mf_qk_norm_prep")(
-        _ptr(qkv), _ptr(q_gain), _ptr(k_gain), float(eps), 1 if normed else 0, _ptr(seq_of_tok), _ptr(positions),
-        _ptr(cos_r), _ptr(sin_r), rot, 1 if halves else 0, 1 if q_only else 0, _ptr(cos_v), _ptr(sin_v),
-        1 if v_from_k else 0, _ptr(page_table),
-        page_table.shape[1], _ptr(q_out), _ptr(kcache), _ptr(vcache), _is_bf16(q_out), n_tok, n_heads, n_kv_heads, dim,
+        qkv, q_gain, k_gain, float(eps), 1 if normed else 0, seq_of_tok, positions,
+        cos_r, sin_r, rot, 1 if halves else 0, 1 if q_only else 0, cos_v, sin_v,
+        1 if v_from_k else 0, page_table,
+        page_table.shape[1], q_out, kcache, vcache, _is_bf16(q_out), n_tok, n_heads, n_kv_heads, dim,
         v_dim, 1 if write_cache else 0, _stream()), "qk_norm_prep")
 
 
@@ -907,8 +931,8 @@ def qk_row_prep(qkv: torch.Tensor, q_gain: torch.Tensor, k_gain: torch.Tensor, e
     _need(positions, "qk_row_prep.positions", torch.int32, (n_tok,))
     coef, every = (0.0, 0) if temperature is None else (float(temperature[0]), int(temperature[1]))
     _check(_fn("attn_normed", "mf_qk_row_prep")(
-        _ptr(qkv), _ptr(q_gain), _ptr(k_gain), float(eps), coef, every, _ptr(seq_of_tok), _ptr(positions), _ptr(page_table),
-        page_table.shape[1], _ptr(q_out), _ptr(kcache), _ptr(vcache), _is_bf16(q_out), n_tok, n_heads, n_kv_heads, dim, v_dim,
+        qkv, q_gain, k_gain, float(eps), coef, every, seq_of_tok, positions, page_table,
+        page_table.shape[1], q_out, kcache, vcache, _is_bf16(q_out), n_tok, n_heads, n_kv_heads, dim, v_dim,
         1 if write_cache else 0, _stream()), "qk_row_prep")
 
 
@@ -929,7 +953,7 @@ def unrotate(rows: torch.Tensor, value_tables, positions: torch.Tensor, n_heads:
         if 2 * cos_v.shape[1] != v_dim:
             raise KernelError(f"unrotate: tables of {cos_v.shape[1]} pairs for values of {v_dim}")
     _need(positions, "unrotate.positions", torch.int32, (n_tok,))
-    _check(_fn("attn_normed", "mf_unrotate")(_ptr(rows), _is_bf16(rows), _ptr(cos_v), _ptr(sin_v), _ptr(positions), n_tok,
+    _check(_fn("attn_normed", "mf_unrotate")(rows, _is_bf16(rows), cos_v, sin_v, positions, n_tok,
                                               n_heads, v_dim, float(scale), _stream()), "unrotate")
 
 
@@ -973,16 +997,16 @@ def lightning_scan(proj: torch.Tensor, cu_seqlens: torch.Tensor, slot_ids: torch
     if dim > 256:
         raise KernelError(f"lightning_scan: key width {dim} is beyond 256")
     if chunks is None or dim > LA_CHUNKED_MAX_DIM:
-        _check(_fn("linear_attention", "mf_lightning_scan")(_ptr(proj), _ptr(cu_seqlens), _ptr(slot_ids), _ptr(decays),
-                                                            _ptr(state), _ptr(out), n_seqs, n_heads, dim, v_dim,
+        _check(_fn("linear_attention", "mf_lightning_scan")(proj, cu_seqlens, slot_ids, decays,
+                                                            state, out, n_seqs, n_heads, dim, v_dim,
                                                             _stream()), "lightning_scan")
         return
     table, n_chunks = chunks
     _need(table, "lightning_scan.chunks", torch.int32, (2 * n_chunks + n_seqs + 1,))
     ws = workspace("la_chunks", n_chunks * n_heads * dim * v_dim, proj.device)
-    first = c_void_p(table.data_ptr() + 8 * n_chunks)
+    first = table.data_ptr() + 8 * n_chunks
     _check(_fn("linear_attention", "mf_lightning_scan_chunked")(
-        _ptr(proj), _ptr(table), n_chunks, first, _ptr(slot_ids), _ptr(decays), _ptr(state), _ptr(ws), _ptr(out),
+        proj, table, n_chunks, first, slot_ids, decays, state, ws, out,
         n_seqs, n_heads, dim, v_dim, _stream()), "lightning_scan_chunked")
 
 
@@ -993,7 +1017,7 @@ def _la_chunk_args(what: str, chunks, n_seqs: int, dim: int):
         return None, 0, None
     table, n_chunks = chunks
     _need(table, what + ".chunks", torch.int32, (2 * n_chunks + n_seqs + 1,))
-    return table, n_chunks, c_void_p(table.data_ptr() + 8 * n_chunks)
+    return table, n_chunks, table.data_ptr() + 8 * n_chunks
 
 
 def _need_la(what: str, proj, cu_seqlens, slot_ids, state, state_shape, out, n_heads: int, dim: int, v_dim: int):
@@ -1033,8 +1057,8 @@ def retention_scan(proj: torch.Tensor, cu_seqlens: torch.Tensor, slot_ids: torch
     table, n_chunks, first = _la_chunk_args("retention_scan", chunks, n_seqs, dim)
     ws = workspace("la_chunks", n_chunks * n_heads * dim * v_dim, proj.device) if n_chunks else None
     _check(_fn("linear_attention", "mf_retention_scan")(
-        _ptr(proj), row_len, _ptr(cu_seqlens), _ptr(table), n_chunks, first, _ptr(slot_ids), _ptr(decays), float(q_scale),
-        float(k_scale), _ptr(cos), _ptr(sin), rot, _ptr(positions), _ptr(state), _ptr(ws), _ptr(out), n_tok, n_seqs, n_heads,
+        proj, row_len, cu_seqlens, table, n_chunks, first, slot_ids, decays, float(q_scale),
+        float(k_scale), cos, sin, rot, positions, state, ws, out, n_tok, n_seqs, n_heads,
         dim, v_dim, _stream()), "retention_scan_chunked" if n_chunks else "retention_scan")
 
 
@@ -1069,10 +1093,10 @@ def memory_scan(proj: torch.Tensor, off_i: int, off_f: int, cap: float, q_scale:
         g, s, n = MEMORY_GATE_FLOATS * n_tok * n_heads, n_chunks * n_heads * dim * v_dim, n_chunks * n_heads * dim
         buf = workspace("la_memory", g + s + n + n_chunks * n_heads, proj.device)
         at = buf.data_ptr()
-        gates, ws, n_ws, decay = (c_void_p(at), c_void_p(at + 4 * g), c_void_p(at + 4 * (g + s)), c_void_p(at + 4 * (g + s + n)))
+        gates, ws, n_ws, decay = (at, at + 4 * g, at + 4 * (g + s), at + 4 * (g + s + n))
     _check(_fn("linear_attention", "mf_memory_scan")(
-        _ptr(proj), row_len, _ptr(cu_seqlens), _ptr(table), n_chunks, first, _ptr(slot_ids), float(q_scale), 1.0, int(off_i),
-        int(off_f), float(cap), _ptr(state), gates, decay, n_ws, ws, _ptr(out), _ptr(den), _ptr(floor), n_seqs, n_heads, dim,
+        proj, row_len, cu_seqlens, table, n_chunks, first, slot_ids, float(q_scale), 1.0, int(off_i),
+        int(off_f), float(cap), state, gates, decay, n_ws, ws, out, den, floor, n_seqs, n_heads, dim,
         v_dim, _stream()), "memory_scan_chunked" if n_chunks else "memory_scan")
 
 
@@ -1099,8 +1123,8 @@ def gated_head_norm(o: torch.Tensor, proj: torch.Tensor, gate_offset: int, weigh
         _need(floor, "gated_head_norm.floor", torch.float32, (rows, n_heads))
     _need(out, "gated_head_norm.out", _FLOATS, (rows, n))
     _check(_fn("linear_attention", "mf_gated_head_norm")(
-        _ptr(o), _ptr(den), _ptr(floor), c_void_p(proj.data_ptr() + 4 * gate_offset), proj.shape[1], _ptr(weight), per_head,
-        _ptr(out), _is_bf16(out), rows, n_heads, n // n_heads, 1 if act == "silu" else 0, float(eps), _stream()),
+        o, den, floor, proj.data_ptr() + 4 * gate_offset, proj.shape[1], weight, per_head,
+        out, _is_bf16(out), rows, n_heads, n // n_heads, 1 if act == "silu" else 0, float(eps), _stream()),
         "gated_head_norm")
 
 
@@ -1115,8 +1139,8 @@ def gated_rmsnorm(o: torch.Tensor, proj: torch.Tensor, gate_offset: int, weight:
         raise KernelError(f"gated_rmsnorm: gate columns {gate_offset}..{gate_offset + n} of rows {tuple(proj.shape)}")
     _need(weight, "gated_rmsnorm.weight", torch.float32, (n,))
     _need(out, "gated_rmsnorm.out", _FLOATS, (rows, n))
-    _check(_fn("linear_attention", "mf_gated_rmsnorm")(_ptr(o), c_void_p(proj.data_ptr() + 4 * gate_offset), proj.shape[1],
-                                                       _ptr(weight), _ptr(out), _is_bf16(out), rows, n, float(eps),
+    _check(_fn("linear_attention", "mf_gated_rmsnorm")(o, proj.data_ptr() + 4 * gate_offset, proj.shape[1],
+                                                       weight, out, _is_bf16(out), rows, n, float(eps),
                                                        _stream()), "gated_rmsnorm")
 
 
@@ -1136,7 +1160,7 @@ def rope_half_inplace(rows: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, 
     _need(positions, "rope_half.positions", torch.int32)
     if rot > head_dim:
         raise KernelError(f"rope_half: {rot} rotated values in heads of {head_dim}")
-    _check(_fn("attn_capped", "mf_rope_half_inplace")(_ptr(rows), _ptr(cos), _ptr(sin), _ptr(positions), n_tok,
+    _check(_fn("attn_capped", "mf_rope_half_inplace")(rows, cos, sin, positions, n_tok,
                                                       n_rot_heads, n_heads_total, head_dim, rot, _stream()), "rope_half_inplace")
 
 
@@ -1183,9 +1207,9 @@ def qkv_conv_prep(qkv: torch.Tensor, conv_w: Optional[torch.Tensor], conv_state:
                            ("slot_ids", slot_ids, (n_seqs,)), ("positions", positions, (n_tok,))):
         _need(t, "qkv_conv_prep." + name, torch.int32, shape)
     _check(_fn("attn_capped", "mf_qkv_conv_prep")(
-        _ptr(qkv), _ptr(conv_w), taps, _ptr(conv_state if taps > 1 else None), _ptr(cu_seqlens), _ptr(seq_of_tok),
-        _ptr(slot_ids), _ptr(positions), _ptr(cos), _ptr(sin), rot, float(blend), _ptr(v_first), _ptr(v_own),
-        _ptr(page_table), page_table.shape[1], _ptr(q_out), _ptr(kcache), _ptr(vcache), _is_bf16(q_out), n_tok, n_seqs,
+        qkv, conv_w, taps, conv_state if taps > 1 else None, cu_seqlens, seq_of_tok,
+        slot_ids, positions, cos, sin, rot, float(blend), v_first, v_own,
+        page_table, page_table.shape[1], q_out, kcache, vcache, _is_bf16(q_out), n_tok, n_seqs,
         n_heads, n_kv_heads, dim, v_dim, 1 if write_cache else 0, _stream()), "qkv_conv_prep")
 
 
@@ -1241,10 +1265,10 @@ def capped_attn(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor, pag
     n_splits = (reach + split_len - 1) // split_len
     part = workspace("attn", n_tok * n_heads * n_splits * (v_dim + 2), q.device) if n_splits > 1 else None
     _check(_fn("attn_capped", "mf_capped_attn")(
-        _ptr(q), _ptr(kcache), _ptr(vcache), _ptr(page_table), page_table.shape[1], _ptr(positions), _ptr(seq_of_tok),
-        _ptr(temp), _ptr(out), _ptr(part), _is_bf16(q), n_tok, n_heads, n_kv_heads, dim, v_dim, float(scale),
-        float(cap or 0.0), int(window or 0), int(chunk or 0), _ptr(far_a), _ptr(far_b), keep_first, _ptr(bias), n_bias,
-        _ptr(sink), n_splits, split_len, _stream()), "capped_attn")
+        q, kcache, vcache, page_table, page_table.shape[1], positions, seq_of_tok,
+        temp, out, part, _is_bf16(q), n_tok, n_heads, n_kv_heads, dim, v_dim, float(scale),
+        float(cap or 0.0), int(window or 0), int(chunk or 0), far_a, far_b, keep_first, bias, n_bias,
+        sink, n_splits, split_len, _stream()), "capped_attn")
 
 
 def _kept_and_bias(what: str, keep_first, window, chunk, bias: Optional[torch.Tensor], n_heads: int):
@@ -1376,10 +1400,10 @@ def capped_attn_prefill(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Ten
         form = capped_form(tile_seq.numel(), n_heads, n_kv_heads, dim, v_dim, *ctx.keys_in_sight(int(window or 0) + keep_first, int(chunk or 0)))
     lib = build.variant("attn_capped_mfma", MF_CAPM_D=dim, MF_CAPM_V=v_dim)
     _check(_fn("attn_capped_mfma", "mf_capped_mfma", lib)(
-        _ptr(q), _ptr(kcache), _ptr(vcache), _ptr(page_table), page_table.shape[1], _ptr(ctx.cu_seqlens),
-        _ptr(ctx.start_pos), _ptr(tile_seq), _ptr(tile_q0), tile_seq.numel(), _ptr(temp), _ptr(out), _ptr(part), n_splits,
+        q, kcache, vcache, page_table, page_table.shape[1], ctx.cu_seqlens,
+        ctx.start_pos, tile_seq, tile_q0, tile_seq.numel(), temp, out, part, n_splits,
         split_len, n_tok, n_heads, n_kv_heads, dim, v_dim, float(scale), float(cap or 0.0), int(window or 0),
-        int(chunk or 0), _ptr(far_a), _ptr(far_b), keep_first, _ptr(bias), n_bias, _ptr(sink), form[0], form[1], _stream()),
+        int(chunk or 0), far_a, far_b, keep_first, bias, n_bias, sink, form[0], form[1], _stream()),
         "capped_attn_decode" if ctx.all_decode else "capped_attn_prefill")
 
 
@@ -1418,8 +1442,8 @@ def moe_route(x: torch.Tensor, router: torch.Tensor, dense: Optional[torch.Tenso
         _need(correction, "moe_route.correction", torch.float32, (E,))
     if score not in MOE_SCORES or group_top < 1:
         raise KernelError(f"moe_route: scores {score!r} (one of {sorted(MOE_SCORES)}), group_top {group_top}")
-    _check(_fn("moe", "mf_moe_route")(_ptr(x), _is_bf16(x), _ptr(router), _ptr(bias), K, _ptr(dense), _ptr(chosen), _ptr(weights),
-                                       n_tok, E, n_groups, keep, top, MOE_SCORES[score], _ptr(correction), int(group_top),
+    _check(_fn("moe", "mf_moe_route")(x, _is_bf16(x), router, bias, K, dense, chosen, weights,
+                                       n_tok, E, n_groups, keep, top, MOE_SCORES[score], correction, int(group_top),
                                        float(weight_scale), 1 if normalize else 0, _stream()), "moe_route")
 
 
@@ -1438,7 +1462,7 @@ def moe_act(gu: torch.Tensor, dense: torch.Tensor, out: torch.Tensor, limit: flo
         raise KernelError(f"moe_act: rows {tuple(gu.shape)} for {E} experts")
     F = gu.shape[1] // (2 * E)
     _need(out, "moe_act.out", _FLOATS, (n_tok, E * F))
-    _check(_fn("moe", "mf_moe_act")(_ptr(gu), _ptr(dense), _ptr(out), _is_bf16(out), n_tok, E, F, float(limit),
+    _check(_fn("moe", "mf_moe_act")(gu, dense, out, _is_bf16(out), n_tok, E, F, float(limit),
                                      int(act), _stream()), "moe_act")
 
 
@@ -1465,7 +1489,7 @@ def moe_sparse(x: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, chose
                           f"{MOE_SPARSE_PAIRS} pairs")
     y = torch.empty((n_tok, top, F), dtype=x.dtype, device=x.device)
     rows = torch.empty((n_tok * top, N), dtype=torch.float32, device=x.device)
-    _check(_fn("moe", "mf_moe_sparse")(_ptr(x), _ptr(gate_up), _ptr(down), _ptr(chosen), _ptr(weights), _ptr(y), _ptr(rows), _ptr(out),
+    _check(_fn("moe", "mf_moe_sparse")(x, gate_up, down, chosen, weights, y, rows, out,
                                         _is_bf16(x), n_tok, top, n_experts, F, K, N, float(limit), int(act),
                                         1 if accumulate else 0, 1 if hands_on else 0, _stream()), "moe_sparse")
 
@@ -1508,7 +1532,7 @@ def mingru_scan(zug: torch.Tensor, cu_seqlens: torch.Tensor, slot_ids: torch.Ten
         raise KernelError(f"mingru_scan: state {tuple(state.shape)} for a width of {w}")
     _need(out, "mingru_scan.out", _FLOATS, (n_tok, w))
     if chunks is None:
-        _check(_fn("recurrence", "mf_mingru_scan")(_ptr(zug), _ptr(cu_seqlens), _ptr(slot_ids), _ptr(state), _ptr(out),
+        _check(_fn("recurrence", "mf_mingru_scan")(zug, cu_seqlens, slot_ids, state, out,
                                                     _is_bf16(out), n_seqs, w, _stream()), "mingru_scan")
         return
     _need(chunks, "mingru_scan.chunks", torch.int32)
@@ -1517,8 +1541,8 @@ def mingru_scan(zug: torch.Tensor, cu_seqlens: torch.Tensor, slot_ids: torch.Ten
     n_chunks = chunks.shape[1]
     ws = workspace("scan", (2 * n_chunks + n_seqs) * w, zug.device)
     _check(_fn("recurrence", "mf_mingru_scan_chunked")(
-        _ptr(zug), _ptr(chunks), n_chunks, _ptr(slot_ids), _ptr(state), _ptr(ws), c_void_p(ws.data_ptr() + 8 * n_chunks * w),
-        _ptr(out), _is_bf16(out), n_seqs, w, _stream()), "mingru_scan_chunked")
+        zug, chunks, n_chunks, slot_ids, state, ws, ws.data_ptr() + 8 * n_chunks * w,
+        out, _is_bf16(out), n_seqs, w, _stream()), "mingru_scan_chunked")
 
 
 # ------------------------------------------------------------------ latent attention
@@ -1565,9 +1589,9 @@ def latent_prep(proj: torch.Tensor, off_dkv: int, off_gate: int, latent_weight: 
     if cache.dim() < 2 or cache.shape[-1] != dk or cache.numel() % (PAGE * dk):
         raise KernelError(f"latent_prep: cache {tuple(cache.shape)} does not hold pages of {PAGE} rows of {dk}")
     _check(_fn("attn_latent", "mf_latent_prep")(
-        _ptr(proj), ld, off_dkv, off_gate, gate_w, _ptr(q_src), q_src.shape[1], _ptr(latent_weight), float(eps), _ptr(cos),
-        _ptr(sin), rd, _ptr(positions),
-        _ptr(seq_of_tok), _ptr(page_table), page_table.shape[1], _ptr(cache), _ptr(q_plain), _ptr(q_abs), _ptr(gate),
+        proj, ld, off_dkv, off_gate, gate_w, q_src, q_src.shape[1], latent_weight, float(eps), cos,
+        sin, rd, positions,
+        seq_of_tok, page_table, page_table.shape[1], cache, q_plain, q_abs, gate,
         _is_bf16(q_plain), n_tok, n_heads, dim, rot_dim, rank, 1 if write_cache else 0, _stream()), "latent_prep")
 
 
@@ -1598,7 +1622,7 @@ def headwise_linear(x: torch.Tensor, n_in: int, wt: torch.Tensor, out: torch.Ten
     if n_in * 32 > 64 * 1024:
         raise KernelError(f"headwise_linear: inputs of {n_in} values do not fit the kernel's staging")
     gate_w = _gate_width("headwise_linear", gate, n_tok, heads, n_out)
-    _check(_fn("attn_latent", "mf_headwise_linear")(_ptr(x), in_stride, _ptr(wt), _ptr(out), out.shape[2], _ptr(gate),
+    _check(_fn("attn_latent", "mf_headwise_linear")(x, in_stride, wt, out, out.shape[2], gate,
                                                      gate_w, _is_bf16(x), n_tok, heads, n_in, n_out, _stream()),
            "headwise_linear")
 
@@ -1623,7 +1647,7 @@ def headwise_linear_mfma(x: torch.Tensor, n_in: int, wo: torch.Tensor, out: torc
     if not headwise_mfma_takes(x.dtype, n_in, in_stride):
         raise KernelError(f"headwise_linear_mfma: inputs of {n_in} in rows of {in_stride} are not 16-byte pieces")
     gate_w = _gate_width("headwise_linear_mfma", gate, n_tok, heads, n_out)
-    _check(_fn("attn_latent", "mf_headwise_mfma")(_ptr(x), in_stride, _ptr(wo), _ptr(out), out.shape[2], _ptr(gate),
+    _check(_fn("attn_latent", "mf_headwise_mfma")(x, in_stride, wo, out, out.shape[2], gate,
                                                    gate_w, n_tok, heads, n_in, n_out, _stream()), "headwise_linear_mfma")
 
 
@@ -1684,8 +1708,8 @@ def latent_attn(q_abs: torch.Tensor, cache: torch.Tensor, page_table: torch.Tens
         part = workspace("latent_attn", n_tok * heads * n_splits * (rank + 2), q_abs.device) if n_splits > 1 else None
         lib = build.variant("attn_latent_mfma", MF_LAT_DKP=(dk + 31) // 32 * 32, MF_LAT_RP=(rank + 31) // 32 * 32)
         _check(_fn("attn_latent_mfma", "mf_latent_mfma", lib)(
-            _ptr(q_abs), _ptr(cache), _ptr(page_table), page_table.shape[1], _ptr(positions), _ptr(cu),
-            _ptr(tile_seq), _ptr(tile_q0), n_tiles, _ptr(out), _ptr(part), n_tok, heads, rank, dk, hc, tq, float(scale),
+            q_abs, cache, page_table, page_table.shape[1], positions, cu,
+            tile_seq, tile_q0, n_tiles, out, part, n_tok, heads, rank, dk, hc, tq, float(scale),
             int(window), n_splits, split_len, _stream()), "latent_attn_mfma")
         return
     if rank > 1024 or (4 * dk + 4 * 256 + 4) * 4 > 64 * 1024:
@@ -1693,8 +1717,8 @@ def latent_attn(q_abs: torch.Tensor, cache: torch.Tensor, page_table: torch.Tens
     n_splits, split_len = latent_split_plan(n_tok * ((heads + 3) // 4), max_len)
     part = workspace("latent_attn", n_tok * heads * n_splits * (rank + 2), q_abs.device) if n_splits > 1 else None
     _check(_fn("attn_latent", "mf_latent_attn")(
-        _ptr(q_abs), _ptr(cache), _ptr(page_table), page_table.shape[1], _ptr(positions), _ptr(seq_of_tok), _ptr(out),
-        _ptr(part), _is_bf16(q_abs), n_tok, heads, rank, dk, float(scale), int(window), n_splits, split_len,
+        q_abs, cache, page_table, page_table.shape[1], positions, seq_of_tok, out,
+        part, _is_bf16(q_abs), n_tok, heads, rank, dk, float(scale), int(window), n_splits, split_len,
         _stream()), "latent_attn")
 
 
@@ -1861,7 +1885,7 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], 
         aligned = not (x.data_ptr() % 16 or weight.data_ptr() % 16 or k % 4)
         splits = _f32_splits(m, n, k, aligned, cu_count())
         part = torch.empty(splits * m * n, dtype=torch.float32, device=x.device) if splits > 1 else None
-        _check(_fn("gemm_f32", "mf_gemm_f32")(_ptr(x), k, _ptr(weight), k, _ptr(bias), _ptr(out), n, _ptr(part), m,
+        _check(_fn("gemm_f32", "mf_gemm_f32")(x, k, weight, k, bias, out, n, part, m,
                                                n, k, splits, 1 if accumulate else 0, _stream()), f"gemm_f32 {m}x{n}x{k}")
         return
     if accumulate and out.dtype != torch.float32:
@@ -1872,19 +1896,19 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], 
         splits, per = _k_split(m, n, k, False, aligned, tiled=tiled is not None)
         part = workspace("skinny", splits * m * n, x.device) if splits > 1 else None
         _need_tiled(tiled, "linear.tiled", n, k)
-        _check(_fn("gemm_bf16", "mf_gemm_bf16_skinny")(_ptr(x), k, _ptr(weight), _ptr(tiled), k, _ptr(bias),
-                                                        _ptr(out), n, _ptr(part), m, n, k, splits, per,
+        _check(_fn("gemm_bf16", "mf_gemm_bf16_skinny")(x, k, weight, tiled, k, bias,
+                                                        out, n, part, m, n, k, splits, per,
                                                         epi, _stream()), f"gemm_bf16_skinny {m}x{n}x{k}")
         return
     if variant == 0:
         variant, splits, per = tile_plan(m, n, k, epi, aligned)
         if splits > 1:
             part = workspace("skinny", splits * m * n, x.device)
-            _check(_fn("gemm_bf16", "mf_gemm_bf16_splitk")(_ptr(x), k, _ptr(weight), k, _ptr(bias), _ptr(out), n,
-                                                            _ptr(part), m, n, k, splits, per, epi, variant,
+            _check(_fn("gemm_bf16", "mf_gemm_bf16_splitk")(x, k, weight, k, bias, out, n,
+                                                            part, m, n, k, splits, per, epi, variant,
                                                             _stream()), f"gemm_bf16_splitk {m}x{n}x{k}")
             return
-    _check(_fn("gemm_bf16", "mf_gemm_bf16")(_ptr(x), k, _ptr(weight), k, _ptr(bias), _ptr(out), n, m,
+    _check(_fn("gemm_bf16", "mf_gemm_bf16")(x, k, weight, k, bias, out, n, m,
                                              n, k, epi, variant, _stream()), f"gemm_bf16 {m}x{n}x{k}")
 
 
@@ -1904,7 +1928,7 @@ def linear_parts(x: torch.Tensor, weight: torch.Tensor) -> Optional[torch.Tensor
     if splits <= 1:
         return None
     part = workspace("skinny", splits * m * n, x.device)[:splits * m * n].view(splits, m, n)
-    _check(_fn("gemm_bf16", "mf_gemm_bf16_parts")(_ptr(x), k, _ptr(weight), k, _ptr(part), m, n, k, splits, per, variant,
+    _check(_fn("gemm_bf16", "mf_gemm_bf16_parts")(x, k, weight, k, part, m, n, k, splits, per, variant,
                                                    _stream()), f"gemm_bf16_parts {m}x{n}x{k}")
     return part
 
@@ -1930,9 +1954,9 @@ def linear_norm_out(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.
         _need(bias, "linear_norm_out.bias", torch.float32, (n,))
     normed = torch.empty((m, n), dtype=torch.bfloat16, device=x.device)
     part = workspace("skinny", splits * m * n, x.device)
-    rc = _fn("gemm_bf16", "mf_gemm_bf16_splitk_norm")(_ptr(x), k, _ptr(weight), k, _ptr(bias), _ptr(out), n, _ptr(part), m, n, k,
-                                                      splits, per, 1 if accumulate else 0, variant, _ptr(g), float(eps),
-                                                      _ptr(normed), _stream())
+    rc = _fn("gemm_bf16", "mf_gemm_bf16_splitk_norm")(x, k, weight, k, bias, out, n, part, m, n, k,
+                                                      splits, per, 1 if accumulate else 0, variant, g, float(eps),
+                                                      normed, _stream())
     if rc == NOT_BUILT:
         return None
     _check(rc, f"gemm_bf16_splitk_norm {m}x{n}x{k}")
@@ -1986,7 +2010,7 @@ def linear_grouped(x: torch.Tensor, weights: torch.Tensor, groups: torch.Tensor,
     _need(out, "linear_grouped.out", torch.float32, (rows, n))
     if not grouped_takes(x.dtype, n, k) or variant not in GROUPED_TILES or groups.dim() != 2 or groups.shape[1] != 4:
         raise KernelError(f"linear_grouped: matrices [{n}][{k}], variant {variant}, groups {tuple(groups.shape)}")
-    _check(_fn("gemm_bf16", "mf_gemm_bf16_grouped")(_ptr(x), _ptr(weights), _ptr(out), _ptr(groups), groups.shape[0], n, k, variant,
+    _check(_fn("gemm_bf16", "mf_gemm_bf16_grouped")(x, weights, out, groups, groups.shape[0], n, k, variant,
                                                      _stream()), f"gemm_bf16_grouped {rows}x{n}x{k}")
 
 
@@ -2024,19 +2048,19 @@ def linear_swiglu(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor, vari
         splits, per = _k_split(m, n, k, True, aligned, tiled=tiled is not None)
         part = workspace("skinny", splits * m * n, x.device) if m > 16 or splits > 1 else None
         _need_tiled(tiled, "linear_swiglu.tiled", n, k)
-        _check(_fn("gemm_bf16", "mf_gemm_bf16_skinny")(_ptr(x), k, _ptr(weight), _ptr(tiled), k, _ptr(limit), _ptr(out), nf,
-                                                        _ptr(part), m, n, k, splits, per, EPI_SWIGLU, _stream()),
+        _check(_fn("gemm_bf16", "mf_gemm_bf16_skinny")(x, k, weight, tiled, k, limit, out, nf,
+                                                        part, m, n, k, splits, per, EPI_SWIGLU, _stream()),
                f"gemm_bf16_skinny(swiglu) {m}x{n}x{k}")
         return
     if variant == 0:
         variant, splits, per = tile_plan(m, n, k, EPI_SWIGLU, aligned)
         if splits > 1:
             part = workspace("skinny", splits * m * n, x.device)
-            _check(_fn("gemm_bf16", "mf_gemm_bf16_splitk")(_ptr(x), k, _ptr(weight), k, _ptr(limit), _ptr(out), nf,
-                                                            _ptr(part), m, n, k, splits, per, EPI_SWIGLU, variant,
+            _check(_fn("gemm_bf16", "mf_gemm_bf16_splitk")(x, k, weight, k, limit, out, nf,
+                                                            part, m, n, k, splits, per, EPI_SWIGLU, variant,
                                                             _stream()), f"gemm_bf16_splitk(swiglu) {m}x{n}x{k}")
             return
-    _check(_fn("gemm_bf16", "mf_gemm_bf16")(_ptr(x), k, _ptr(weight), k, _ptr(limit), _ptr(out), nf, m, n, k,
+    _check(_fn("gemm_bf16", "mf_gemm_bf16")(x, k, weight, k, limit, out, nf, m, n, k,
                                              EPI_SWIGLU, variant, _stream()), f"gemm_bf16(swiglu) {m}x{n}x{k}")
 
 
@@ -2080,8 +2104,8 @@ def linear_normed(x: torch.Tensor, norm_weight: torch.Tensor, eps: float, row_id
     if m > 16 or tuning.NO_FOLD:
         return False
     _need_tiled(tiled, "linear_normed.tiled", n, k)
-    rc = _fn("gemm_bf16", "mf_gemm_bf16_normed")(_ptr(x), k, _ptr(row_idx), _ptr(norm_weight), float(eps),
-                                                 _ptr(weight), _ptr(tiled), k, _ptr(bias), _ptr(out), ldc, m, n, k,
+    rc = _fn("gemm_bf16", "mf_gemm_bf16_normed")(x, k, row_idx, norm_weight, float(eps),
+                                                 weight, tiled, k, bias, out, ldc, m, n, k,
                                                  epi, _stream())
     if rc == NOT_BUILT:
         return False
@@ -2167,8 +2191,8 @@ def linear_fused(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Ten
     part = workspace("skinny", splits * m * n, x.device) if (splits > 1 or (swiglu and m > 16)) else None
     _need_tiled(tiled, "linear_fused.tiled", n, k)
     rc = _fn("gemm_bf16", "mf_gemm_bf16_skinny_fused")(
-        _ptr(x), k, _ptr(weight), _ptr(tiled), k, _ptr(bias), _ptr(out), ldc, _ptr(part), m, n, k, splits, per, epi,
-        _ptr(in_ssq), in_parts, float(in_eps), _ptr(out_g), _ptr(out_xg), _ptr(out_ssq),
+        x, k, weight, tiled, k, bias, out, ldc, part, m, n, k, splits, per, epi,
+        in_ssq, in_parts, float(in_eps), out_g, out_xg, out_ssq,
         out_ssq.shape[1] if out_ssq is not None else 0, _stream())
     if rc == NOT_BUILT:
         return False
@@ -2250,15 +2274,15 @@ def attn_tokens(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor, pag
         n_splits, base = decode_split_plan(n_tok, n_kv_heads, n_heads // n_kv_heads, max_len)
         part = workspace("attn", n_tok * n_heads * n_splits * (head_dim + 2), q.device) if n_splits > 1 else None
         _check(_fn("attn_decode_bf16", "mf_attn_decode_bf16")(
-            _ptr(q), _ptr(kcache), _ptr(vcache), _ptr(page_table), page_table.shape[1], _ptr(positions),
-            _ptr(seq_of_tok), _ptr(out), _ptr(part), n_tok, n_heads, n_kv_heads, head_dim, float(scale),
+            q, kcache, vcache, page_table, page_table.shape[1], positions,
+            seq_of_tok, out, part, n_tok, n_heads, n_kv_heads, head_dim, float(scale),
             int(window or 0), n_splits, base, _stream()), "attn_decode_bf16")
         return
     n_splits, split_len = split_plan(n_tok, n_kv_heads, n_heads // n_kv_heads, head_dim, max_len)
     part = workspace("attn", n_tok * n_heads * n_splits * (head_dim + 2), q.device) if n_splits > 1 else None
     _check(_fn("attn_tokens_f32", "mf_attn_tokens_f32")(
-        _ptr(q), _ptr(kcache), _ptr(vcache), _ptr(page_table), page_table.shape[1], _ptr(positions),
-        _ptr(seq_of_tok), _ptr(out), _ptr(part), n_tok, n_heads, n_kv_heads, head_dim, float(scale),
+        q, kcache, vcache, page_table, page_table.shape[1], positions,
+        seq_of_tok, out, part, n_tok, n_heads, n_kv_heads, head_dim, float(scale),
         int(window or 0), n_splits, split_len, _stream()), "attn_tokens_f32")
 
 
@@ -2292,8 +2316,8 @@ def attn_prompt_f32(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor,
                                             ctx.max_len, cu_count())
     part = workspace("attn", n_tok * n_heads * n_splits * (head_dim + 2), q.device) if n_splits > 1 else None
     _check(_fn("attn_prompt_f32", "mf_attn_prompt_f32")(
-        _ptr(q), _ptr(kcache), _ptr(vcache), _ptr(page_table), page_table.shape[1], _ptr(ctx.cu_seqlens), _ptr(ctx.start_pos),
-        _ptr(tile_seq), _ptr(tile_row), _ptr(out), _ptr(part), tile_seq.numel(), n_tok, n_heads, n_kv_heads, head_dim,
+        q, kcache, vcache, page_table, page_table.shape[1], ctx.cu_seqlens, ctx.start_pos,
+        tile_seq, tile_row, out, part, tile_seq.numel(), n_tok, n_heads, n_kv_heads, head_dim,
         float(scale), int(window or 0), n_splits, split_len, _stream()), "attn_tokens_f32 (rows)")
 
 
@@ -2333,8 +2357,8 @@ def attn_decode_rope(qkv: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, kc
     n_splits, base = decode_split_plan(n_tok, n_kv_heads, n_heads // n_kv_heads, max_len)
     part = workspace("attn", n_tok * n_heads * n_splits * (head_dim + 2), qkv.device) if n_splits > 1 else None
     _check(_fn("attn_decode_bf16", "mf_attn_decode_rope_bf16")(
-        _ptr(qkv), _ptr(cos), _ptr(sin), _ptr(kcache), _ptr(vcache), _ptr(page_table), page_table.shape[1],
-        _ptr(positions), _ptr(seq_of_tok), _ptr(out), _ptr(part), n_tok, n_heads, n_kv_heads, head_dim,
+        qkv, cos, sin, kcache, vcache, page_table, page_table.shape[1],
+        positions, seq_of_tok, out, part, n_tok, n_heads, n_kv_heads, head_dim,
         float(scale), int(window or 0), n_splits, base, 1 if write_kv else 0, _stream()), "attn_decode_rope_bf16")
 
 
@@ -2394,9 +2418,9 @@ def attn_prefill(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor, pa
         parts = workspace("prefill_parts", n_slots * per_tile * most_shares * part, q.device)
         arrived = _zeroed_counters("prefill_arrived", n_slots * per_tile, q.device)
     rc = _fn("attn_prefill_bf16", "mf_attn_prefill_bf16")(
-        _ptr(q), _ptr(kcache), _ptr(vcache), _ptr(page_table), page_table.shape[1], _ptr(ctx.cu_seqlens),
-        _ptr(ctx.start_pos), _ptr(tile_seq), _ptr(tile_q0), _ptr(tile_share), _ptr(parts), _ptr(arrived),
-        most_shares if shared is not None else 1, _ptr(out), tile_seq.numel(), n_heads, n_kv_heads, head_dim,
+        q, kcache, vcache, page_table, page_table.shape[1], ctx.cu_seqlens,
+        ctx.start_pos, tile_seq, tile_q0, tile_share, parts, arrived,
+        most_shares if shared is not None else 1, out, tile_seq.numel(), n_heads, n_kv_heads, head_dim,
         gh, tq, float(scale), window, _stream())
     if rc != 0 and arrived is not None:
         arrived.zero_()                  # a launch that failed may have left workgroups counted in
@@ -2418,7 +2442,7 @@ def argmax(logits: torch.Tensor, out: torch.Tensor) -> None:
     if vocab >= 16384 and rows < 256:          # few long rows: several blocks per row
         chunks = max(1, min(64, 512 // rows, vocab // 4096))
     work = workspace("argmax", 2 * rows * chunks, logits.device) if chunks > 1 else None
-    _check(_fn("sampling", "mf_argmax")(_ptr(logits), vocab, rows, vocab, _ptr(out), _ptr(work), chunks,
+    _check(_fn("sampling", "mf_argmax")(logits, vocab, rows, vocab, out, work, chunks,
                                          _stream()), "argmax")
 
 
@@ -2433,8 +2457,8 @@ def sample(logits: torch.Tensor, temp: float, streams: torch.Tensor, steps: torc
     _need(out, "sample.out", torch.int32, (rows,))
     if forced_r is not None:
         _need(forced_r, "sample.forced_r", torch.float32, (rows,))
-    _check(_fn("sampling", "mf_sample")(_ptr(logits), vocab, rows, vocab, float(temp), _ptr(streams),
-                                         _ptr(steps), _ptr(forced_r), _ptr(out), _stream()), "sample")
+    _check(_fn("sampling", "mf_sample")(logits, vocab, rows, vocab, float(temp), streams,
+                                         steps, forced_r, out, _stream()), "sample")
 
 
 def penalties(logits: torch.Tensor, prev: torch.Tensor, n_prev: torch.Tensor, repeat: float,
@@ -2444,19 +2468,19 @@ def penalties(logits: torch.Tensor, prev: torch.Tensor, n_prev: torch.Tensor, re
     if prev.dim() != 2 or prev.shape[0] != rows:
         raise KernelError(f"penalties.prev: expected [{rows}][window], got {tuple(prev.shape)}")
     _need(n_prev, "penalties.n_prev", torch.int32, (rows,))
-    _check(_fn("sampling", "mf_penalties")(_ptr(logits), vocab, rows, vocab, _ptr(prev), prev.shape[1],
-                                            _ptr(n_prev), float(repeat), float(frequency),
+    _check(_fn("sampling", "mf_penalties")(logits, vocab, rows, vocab, prev, prev.shape[1],
+                                            n_prev, float(repeat), float(frequency),
                                             float(presence), _stream()), "penalties")
 
 
 def top_k(logits: torch.Tensor, k: int) -> None:
     rows, vocab = _logit_rows(logits, "top_k.logits")
-    _check(_fn("sampling", "mf_top_k")(_ptr(logits), vocab, rows, vocab, int(k), _stream()), "top_k")
+    _check(_fn("sampling", "mf_top_k")(logits, vocab, rows, vocab, int(k), _stream()), "top_k")
 
 
 def top_p(logits: torch.Tensor, p: float) -> None:
     rows, vocab = _logit_rows(logits, "top_p.logits")
-    _check(_fn("sampling", "mf_top_p")(_ptr(logits), vocab, rows, vocab, float(p), _stream()), "top_p")
+    _check(_fn("sampling", "mf_top_p")(logits, vocab, rows, vocab, float(p), _stream()), "top_p")
 
 
 FILTERED_K_MAX = 48            # the largest top-k that `sample_filtered` takes
@@ -2484,9 +2508,9 @@ def sample_filtered(logits: torch.Tensor, k: int, p: float, temp: float, streams
     if forced_r is not None:
         _need(forced_r, "sample_filtered.forced_r", torch.float32, (rows,))
     work = workspace("sample_filtered", rows * 64 * (2 * 64 + 2), logits.device)
-    _check(_fn("sampling", "mf_sample_filtered")(_ptr(logits), vocab, rows, vocab, int(k), float(p), float(temp),
-                                                  _ptr(streams), _ptr(steps), _ptr(forced_r), _ptr(work),
-                                                  _ptr(out), _stream()),
+    _check(_fn("sampling", "mf_sample_filtered")(logits, vocab, rows, vocab, int(k), float(p), float(temp),
+                                                  streams, steps, forced_r, work,
+                                                  out, _stream()),
            "sample_filtered")
 
 
@@ -2507,9 +2531,9 @@ def advance(next_ids: torch.Tensor, sampled: torch.Tensor, positions: torch.Tens
         max_prev = prev.shape[1]
         _need(n_prev, "advance.n_prev", torch.int32, (n,))
         _need(cursor, "advance.cursor", torch.int32, (n,))
-    _check(_fn("sampling", "mf_advance")(_ptr(next_ids), _ptr(sampled), _ptr(positions), _ptr(steps), n,
-                                          _ptr(prev), max_prev, _ptr(n_prev if prev is not None else None),
-                                          _ptr(cursor if prev is not None else None), _stream()), "advance")
+    _check(_fn("sampling", "mf_advance")(next_ids, sampled, positions, steps, n,
+                                          prev, max_prev, n_prev if prev is not None else None,
+                                          cursor if prev is not None else None, _stream()), "advance")
 
 
 # ------------------------------------------------------------------ measuring kernels
@@ -2520,7 +2544,7 @@ def probe_read(buffer: torch.Tensor, blocks: Optional[int] = None) -> None:
     nbytes = buffer.numel() * buffer.element_size() // 16 * 16
     blocks = blocks or cu_count()
     sink = workspace("probe", blocks, buffer.device)
-    _check(_fn("probe", "mf_probe_read")(_ptr(buffer), nbytes, _ptr(sink), blocks, _stream()), "probe_read")
+    _check(_fn("probe", "mf_probe_read")(buffer, nbytes, sink, blocks, _stream()), "probe_read")
 
 
 def probe_mfma(rounds: int, blocks: Optional[int] = None, device="cuda") -> float:
@@ -2528,7 +2552,7 @@ def probe_mfma(rounds: int, blocks: Optional[int] = None, device="cuda") -> floa
     of floating-point operations it performs (time it from outside)."""
     blocks = blocks or cu_count()
     sink = workspace("probe", blocks, device)
-    _check(_fn("probe", "mf_probe_mfma")(int(rounds), _ptr(sink), blocks, _stream()), "probe_mfma")
+    _check(_fn("probe", "mf_probe_mfma")(int(rounds), sink, blocks, _stream()), "probe_mfma")
     return float(blocks) * 8 * rounds * 8 * 2 * 32 * 32 * 16
 
 
@@ -2547,7 +2571,7 @@ def moe_table(table: torch.Tensor, ids: torch.Tensor, rows: Optional[torch.Tenso
         raise KernelError(f"moe_table: {ids.numel()} token ids for {n_tok} rows")
     _need(chosen, "moe_table.chosen", torch.int32)
     _need(weights, "moe_table.weights", torch.float32, (n_tok, top))
-    _check(_fn("moe", "mf_moe_table")(_ptr(table), _ptr(ids), _ptr(rows), _ptr(chosen), _ptr(weights), n_tok, top, table.shape[0],
+    _check(_fn("moe", "mf_moe_table")(table, ids, rows, chosen, weights, n_tok, top, table.shape[0],
                                        float(weight), _stream()), "moe_table")
 
 
@@ -2558,7 +2582,7 @@ def gated_expert_act(gu: torch.Tensor, out: torch.Tensor) -> None:
     if gu.shape[0] != n_tok or gu.shape[1] < 2 * F + 1:
         raise KernelError(f"gated_expert_act: rows {tuple(gu.shape)} for {n_tok} tokens of {F} values")
     _need(out, "gated_expert_act.out", _FLOATS, (n_tok, F))
-    _check(_fn("moe", "mf_gated_expert_act")(_ptr(gu), gu.shape[1], _ptr(out), _is_bf16(out), n_tok, F, _stream()),
+    _check(_fn("moe", "mf_gated_expert_act")(gu, gu.shape[1], out, _is_bf16(out), n_tok, F, _stream()),
            "gated_expert_act")
 
 
@@ -2568,7 +2592,7 @@ def moe_group(chosen: torch.Tensor, n_experts: int, rank: torch.Tensor, counts: 
     _need(chosen, "moe_group.chosen", torch.int32)
     _need(rank, "moe_group.rank", torch.int32, tuple(chosen.shape))
     _need(counts, "moe_group.counts", torch.int32, (n_experts,))
-    _check(_fn("moe", "mf_moe_group")(_ptr(chosen), chosen.numel(), n_experts, _ptr(rank), _ptr(counts), _stream()), "moe_group")
+    _check(_fn("moe", "mf_moe_group")(chosen, chosen.numel(), n_experts, rank, counts, _stream()), "moe_group")
 
 
 ALL_REAL = 0x7fffffff      # every expert number a router can name has matrices
@@ -2592,7 +2616,7 @@ def moe_gather(x: torch.Tensor, chosen: torch.Tensor, rank: torch.Tensor, offset
     _need(rank, "moe_gather.rank", torch.int32, (n_tok, top))
     _need(offsets, "moe_gather.offsets", torch.int32)
     _need_pair_rows(xs, "moe_gather.xs", x.dtype, n_tok * top, K, n_real is None)
-    _check(_fn("moe", "mf_moe_gather")(_ptr(x), _is_bf16(x), _ptr(chosen), _ptr(rank), _ptr(offsets), _ptr(xs), n_tok * top,
+    _check(_fn("moe", "mf_moe_gather")(x, _is_bf16(x), chosen, rank, offsets, xs, n_tok * top,
                                         top, K, ALL_REAL if n_real is None else int(n_real), _stream()), "moe_gather")
 
 
@@ -2612,6 +2636,6 @@ def moe_combine(rows: torch.Tensor, chosen: torch.Tensor, rank: torch.Tensor, of
     _need(offsets, "moe_combine.offsets", torch.int32)
     _need(weights, "moe_combine.weights", torch.float32, (n_tok, top))
     _need(out, "moe_combine.out", torch.float32, (n_tok, N))
-    _check(_fn("moe", "mf_moe_combine")(_ptr(rows), _ptr(chosen), _ptr(rank), _ptr(offsets), _ptr(weights), _ptr(x),
-                                         0 if x is None else _is_bf16(x), ALL_REAL if n_real is None else int(n_real), _ptr(out),
+    _check(_fn("moe", "mf_moe_combine")(rows, chosen, rank, offsets, weights, x,
+                                         0 if x is None else _is_bf16(x), ALL_REAL if n_real is None else int(n_real), out,
                                          n_tok, top, N, 1 if accumulate else 0, _stream()), "moe_combine")

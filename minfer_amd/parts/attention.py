@@ -15,6 +15,7 @@ from ..kernels import ops
 from ..weights.loader import TensorSpec
 from .base import Mixer, POSITIONS, make_part, register_mixer
 from .linear import Linear
+from .rotary import RotaryNeoX
 
 
 @register_mixer("gqa_attention")
@@ -69,6 +70,13 @@ class GQAttention(Mixer):
         self.position.prepare(max_len)
 
     takes_normed = True
+
+    def alike(self, ctx, entry: int):
+        if type(self) is not GQAttention or type(self.position) is not RotaryNeoX:
+            return None
+        kc, vc, group = ctx.cache.kv(entry)
+        constants = (GQAttention, self.hidden, self.nh, self.nk, self.hd, self.scale, self.window, group)
+        return constants, self.qkv.tensors() + self.o.tensors() + (kc, vc) + self.position.rotation_tables(ctx.max_len)
 
     def forward(self, x, h, ctx, entry: int, writes_cache: bool) -> None:
         kc, vc, group = ctx.cache.kv(entry)

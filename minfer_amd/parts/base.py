@@ -57,6 +57,11 @@ class Part:
 
 
 class Norm(Part):
+    def alike(self):
+        """(constants, tensors) that decide what `forward` and the folds of this norm launch (tuples), or None: not said.
+        Norms with equal constants make the same launches with tensors of the same types and shapes, each with its own."""
+        return None
+
     def forward(self, h: torch.Tensor, out: Optional[torch.Tensor] = None,
                 row_idx: Optional[torch.Tensor] = None) -> torch.Tensor:
         """float32 rows in, run-type rows out; row r reads h[row_idx[r]] when given."""
@@ -164,6 +169,10 @@ class PositionEncoding(Part):
 
 
 class Mixer(Part):
+    def alike(self, ctx, entry: int):
+        """As `Norm.alike`, for `forward` on the cache entry `entry` in the step `ctx`."""
+        return None
+
     def cache_request(self):
         """A `KVRequest`, a `StateRequest` or None."""
         return None
@@ -179,6 +188,10 @@ class Mixer(Part):
 
 
 class FeedForward(Part):
+    def alike(self):
+        """As `Norm.alike`."""
+        return None
+
     takes_normed = False     # True: `x` may arrive as a `Normed`
     can_overwrite = False    # True: `forward(..., accumulate=False)` stores its output instead of adding it
 
@@ -269,6 +282,10 @@ class Block:
     @property
     def feed_forward_norm(self) -> Optional[Norm]:
         return self.norms.get("feed_forward")
+
+    def alike(self, ctx, entry: int, writes_cache: bool):
+        """(constants, tensors) that decide what `forward` without `keep_rows` launches, or None: not said (`Norm.alike`)."""
+        return None
 
     def parts(self):
         """Every part of the block that exists, norms in the order of `norm_names`."""

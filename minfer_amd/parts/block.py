@@ -32,6 +32,14 @@ class PreNormBlock(Block):
     def first_norm(self):
         return self.mixer_norm if self.mixer is not None else self.feed_forward_norm
 
+    def alike(self, ctx, entry: int, writes_cache: bool):
+        if type(self) is not PreNormBlock or self.mixer is None or self.feed_forward is None:
+            return None
+        parts = (self.mixer.alike(ctx, entry), self.feed_forward.alike(), self.mixer_norm.alike(), self.feed_forward_norm.alike())
+        if None in parts:
+            return None
+        return (writes_cache,) + tuple(p[0] for p in parts), sum((p[1] for p in parts), ())
+
     def forward(self, h, ctx, entry: int, writes_cache: bool, keep_rows=None):
         after = getattr(ctx, "norm_after_block", None)      # the norm that reads the stream behind this block
         if self.mixer is not None:

@@ -61,6 +61,12 @@ class SwiGLU(FeedForward):
 
     takes_normed = True
 
+    def alike(self):
+        if type(self) is not SwiGLU:
+            return None
+        gate_up = (None, None, None) if self.gate_up is None else self.gate_up.tensors()
+        return (SwiGLU, self.hidden, self.inter, self.limit), (self.fused, self.fused_tiled, self.limit_on_device) + gate_up + self.down.tensors()
+
     def forward(self, x, h, ctx, accumulate: bool = True) -> None:
         y = torch.empty((x.shape[0], self.inter), dtype=self.rt.dtype, device=x.device)
         if self.fused is not None:

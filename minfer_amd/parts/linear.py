@@ -28,6 +28,9 @@ class Linear:
         self.out_features, self.in_features = weight.shape
         self.tiled: Optional[torch.Tensor] = None      # ops.tile_weight(weight), where the model keeps one
 
+    def tensors(self):
+        return self.weight, self.tiled, self.bias
+
     def decode_copy(self, make: bool, min_row_length: int = 0) -> int:
         """Bytes of the tiled copy of this matrix, which the products of few rows read faster than
         the matrix itself (0: it has none: 32-bit, a row length that is no multiple of 32, or a

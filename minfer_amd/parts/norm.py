@@ -31,6 +31,9 @@ class RMSNorm(Norm):
     def rms_scale(self):
         return self.weight, self.eps
 
+    def alike(self):
+        return ((RMSNorm, self.size, self.eps), (self.weight,)) if type(self) is RMSNorm else None
+
     def forward(self, h, out: Optional[torch.Tensor] = None, row_idx: Optional[torch.Tensor] = None):
         rows = h.shape[0] if row_idx is None else row_idx.numel()
         if out is None:
