@@ -106,13 +106,14 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__
 
 // ---- many rows on the matrix cores
 // A 64 x 64 tile on 4 waves of 32 x 32 (16x16x4 products).  k tiles of 32 (a row is a 128-byte line) travel global -> LDS
-// in three stages, chunk c of row r at position c ^ ((r >> 1) & 7); a lane reads four neighbouring k of its row at once
+// in two stages, chunk c of row r at position c ^ ((r >> 1) & 7); a lane reads four neighbouring k of its row at once
 // and the e-th of them goes into the e-th product, so a product's four k are 4 apart (the order of a sum's terms within
-// sixteen).  The products are what bounds it (1,024 cycles a k tile for 256 of LDS reads); 48 KB of LDS let three
-// blocks share a CU, whose waves cover each other's waits.
-// 611 rows (0.5B widths), with vector FMA before and now: gate|up 9,728 x 896 152 us and 98 (113 TFLOP/s); q|k|v 1,152 x 896
-// 74 and 24 (a third of K a block, and the kernel that adds the parts); down 896 x 4,864 and o 896 x 896 together 450 and 85.
-constexpr int T_BM = 64, T_BK = 32, T_STAGES = 3, T_ROW = T_BK * 4, T_STAGE = 2 * T_BM * T_ROW;
+// sixteen).  The products are what bounds it (1,024 cycles a k tile for 256 of LDS reads); 32 KB of LDS let five
+// blocks share a CU, whose waves cover each other's waits (three stages and three blocks: level to 3 % slower).
+// 4,096^3 runs at 136 TFLOP/s.  611 rows (0.5B widths): gate|up 9,728 x 896 104 us (95 with the weights in the memory-side
+// cache; 640 rows at 136 TFLOP/s are 82), with vector FMA 152; q|k|v 1,152 x 896 74 and 21 (K in 4 parts);
+// down 896 x 4,864 61 (in 5).
+constexpr int T_BM = 64, T_BK = 32, T_STAGES = 2, T_ROW = T_BK * 4, T_STAGE = 2 * T_BM * T_ROW;
 
 __device__ __forceinline__ void dma16(const float* base, unsigned off, unsigned lds_byte) {
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds_byte)
@@ -120,19 +121,26 @@ __device__ __forceinline__ void dma16(const float* base, unsigned off, unsigned 
 }
 
 // SPLIT: sums without bias into this part's slab of C, [parts][M][N]; else the product's own epilogue
+// by_xcd: every XCD takes one contiguous eighth of the tiles of all parts (`tiles_by_xcd`)
 template <bool ACCUMULATE, bool SPLIT>
 __global__ __launch_bounds__(256) void tile_f32_kernel(const float* __restrict__ A, int lda, const float* __restrict__ W, int ldw,
                                                        const float* __restrict__ bias, float* __restrict__ C, int ldc, int M, int N,
-                                                       int K, int tiles_m, int k_per_split) {
+                                                       int K, int tiles_m, int k_per_split, int by_xcd) {
   __shared__ __attribute__((aligned(16))) unsigned char smem[T_STAGES * T_STAGE];
+  int at = blockIdx.y * gridDim.x + blockIdx.x;
+  if (by_xcd) {
+    const int n = gridDim.x * gridDim.y, per = n / 8, rem = n % 8, x = at % 8;
+    at = x * per + min(x, rem) + at / 8;
+  }
+  const int part = at / (int)gridDim.x, tile = at - part * (int)gridDim.x;
   if (SPLIT) {
-    const int kb = blockIdx.y * k_per_split;
+    const int kb = part * k_per_split;
     A += kb;
     W += kb;
     K = min(k_per_split, K - kb);
-    C += (size_t)blockIdx.y * M * N;
+    C += (size_t)part * M * N;
   }
-  const int m0 = (blockIdx.x % tiles_m) * T_BM, n0 = (blockIdx.x / tiles_m) * T_BM;
+  const int m0 = (tile % tiles_m) * T_BM, n0 = (tile / tiles_m) * T_BM;
   const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = (wid & 1) * 32, wn = (wid >> 1) * 32;
   const int fr = lane & 15, fk = lane >> 4;
@@ -159,16 +167,16 @@ __global__ __launch_bounds__(256) void tile_f32_kernel(const float* __restrict__
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j) acc[i][j] = tot[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
-  copy(0, 0);
-  copy(1, 1);
+#pragma unroll
+  for (int t = 0; t < T_STAGES - 1; ++t) copy(t, t);
   const int sw = (fr >> 1) & 7;
   int st = 0;
   for (int kt = 0; kt < nkt; ++kt) {
-    // tile kt has landed for this wave (tile kt + 1's four copies may be in flight), and behind the barrier for all; the
-    // stage of tile kt - 1, which every wave holds in registers by then, takes tile kt + 2
-    asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+    // tile kt has landed for this wave (the younger ones' four copies each may be in flight), and behind the barrier for all;
+    // the stage of tile kt - 1, which every wave holds in registers by then, takes the next one
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(4 * (T_STAGES - 2)) : "memory");
     __syncthreads();
-    copy(kt + 2, st == 0 ? 2 : st - 1);
+    copy(kt + T_STAGES - 1, st == 0 ? T_STAGES - 1 : st - 1);
     const unsigned char* s = smem + st * T_STAGE;
     float4 a[2][2], w[2][2];
 #pragma unroll
@@ -249,15 +257,34 @@ __global__ __launch_bounds__(256) void add_parts_f32_kernel(const float* __restr
   *c = ACCUMULATE ? *c + v : v;
 }
 
-// How many blocks share a tile's K: the chip holds three blocks a CU and is busy with one, so K is cut, in parts of at
-// least 256, until every CU has about two (140 tiles of 64 x 64 for 611 rows against 896: whole, a CU in two would idle).
+// How many blocks share a tile's K.  The chip's time is that of the CU with the most tiles, times their k tiles (and some three
+// more a tile for its start), at 0.43 us a k tile where three or more share a CU and somewhat more where two or one do; the
+// parts' way to memory and back and the second kernel come on top.  (611 rows against 896 of 4,864, 140 tiles: 4 parts, 560 on
+// 256 CUs, 71 us; 5 parts 60.5.)
 int tile_splits(int M, int N, int K, int n_cu) {
-  const long tiles = (long)((M + T_BM - 1) / T_BM) * ((N + T_BM - 1) / T_BM);
-  if (tiles >= n_cu) return 1;
-  const long parts = std::min<long>(std::min<long>(K / 256, 16), (2L * n_cu + tiles - 1) / tiles);
-  if (parts < 2) return 1;
-  const int per = (int)((K / T_BK + parts - 1) / parts) * T_BK;
-  return (K + per - 1) / per;
+  const long tiles = (long)((M + T_BM - 1) / T_BM) * ((N + T_BM - 1) / T_BM), nkt = K / T_BK;
+  long best = 1;
+  double best_us = 1e30;
+  for (long parts = 1; parts <= std::min<long>(std::max<long>(1, nkt / 7), 16); ++parts) {
+    const long per = (nkt + parts - 1) / parts, most = (tiles * parts + n_cu - 1) / n_cu;
+    if ((nkt + per - 1) / per != parts) continue;
+    const double step_us = most >= 3 ? 0.43 : most == 2 ? 0.54 : 0.75;
+    const double us = (double)(most * (per + 3)) * step_us + (parts > 1 ? 4. + (double)(parts + 1) * M * N * 4. / 3e6 : 0.);
+    if (us < best_us * 0.95) {
+      best_us = us;
+      best = parts;
+    }
+  }
+  return (int)best;
+}
+
+// An eighth of the tiles an XCD, each with an L2 of 4 MB: whole products whose activations stay in it beside the weights (each
+// XCD then reads an eighth of these: 611 rows against 9,728 of 896 109 us and 104, 400 against 17,920 of 1,536 219 and 202; 2,000 against 9,728
+// of 896 274 and 284), and parts of
+// activations that would not (an XCD then reads a part or two: 400 x 1,536 x 8,960 119 us and 112; 611 x 1,152 x 896 24 and 25).
+int tiles_by_xcd(int M, int K, int splits) {
+  const size_t bytes = (size_t)M * K * 4;
+  return splits > 1 ? bytes > (4u << 20) : bytes <= (3u << 20);
 }
 
 bool tile_takes(int M, int N, int K, int lda, int ldw, const void* A, const void* W) {
@@ -398,10 +425,11 @@ MF_API int mf_gemm_f32(const float* A, int lda, const float* W, int ldw, const f
   }
   if (tile_takes(M, N, K, lda, ldw, A, W)) {
     const int tiles_m = (M + T_BM - 1) / T_BM, tiles = tiles_m * ((N + T_BM - 1) / T_BM);
+    const int by_xcd = tiles_by_xcd(M, K, splits);
     if (splits > 1) {
       const int per = (K / T_BK + splits - 1) / splits * T_BK;
       if (!part || (long)(splits - 1) * per >= K) return (int)hipErrorInvalidValue;
-      tile_f32_kernel<false, true><<<dim3(tiles, splits), 256, 0, stream>>>(A, lda, W, ldw, nullptr, part, N, M, N, K, tiles_m, per);
+      tile_f32_kernel<false, true><<<dim3(tiles, splits), 256, 0, stream>>>(A, lda, W, ldw, nullptr, part, N, M, N, K, tiles_m, per, by_xcd);
       const int rc = mf_launch_status();
       if (rc) return rc;
       const unsigned blocks = (unsigned)(((size_t)M * N + 255) / 256);
@@ -409,8 +437,8 @@ MF_API int mf_gemm_f32(const float* A, int lda, const float* W, int ldw, const f
       else add_parts_f32_kernel<false><<<blocks, 256, 0, stream>>>(part, bias, C, ldc, M, N, splits);
       return mf_launch_status();
     }
-    if (accumulate) tile_f32_kernel<true, false><<<tiles, 256, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, tiles_m, 0);
-    else tile_f32_kernel<false, false><<<tiles, 256, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, tiles_m, 0);
+    if (accumulate) tile_f32_kernel<true, false><<<tiles, 256, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, tiles_m, 0, by_xcd);
+    else tile_f32_kernel<false, false><<<tiles, 256, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, tiles_m, 0, by_xcd);
     return mf_launch_status();
   }
   dim3 grid((N + BN - 1) / BN, (M + BM - 1) / BM);

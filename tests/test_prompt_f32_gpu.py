@@ -94,3 +94,26 @@ def test_attn_prompt_f32_keeps_values_that_are_no_numbers_apart(ops):
     assert torch.isinf(out[~same]).all()
     # (a run with such a value is added up key by key: other roundings in the other columns)
     close(out[same].double(), clean[same].double(), 1e-6)
+
+
+@pytest.mark.parametrize("m,n,k", [(65, 130, 896),          # whole, few tiles
+                                   (611, 1152, 896),        # in parts of which the last is shorter
+                                   (611, 9728, 896),        # whole, an eighth of the tiles an XCD
+                                   (300, 200, 4128),        # in parts, 4.9 MB of activations: part by part
+                                   (1000, 4100, 1088),      # whole, 4.4 MB of activations: tile by tile
+                                   (9, 64, 32)])            # one tile of one k tile
+def test_products_of_many_rows(ops, m, n, k):
+    """The 32-bit product's parts and tile orders.  Bound: a sum of k terms in chains of 128 whose sums are added in turn errs by at
+    most (128 + k / 128 + parts + 2) half units in the last place of the sum of the terms' sizes; a quarter of that is far above
+    what roundings of either sign come to."""
+    gen = torch.Generator().manual_seed(m + n + k)
+    x, w = torch.randn((m, k), generator=gen), torch.randn((n, k), generator=gen)
+    b, base = torch.randn(n, generator=gen), torch.randn((m, n), generator=gen)
+    want = x.double() @ w.double().t() + b.double()
+    size = x.abs().double() @ w.abs().double().t()
+    bound = 0.25 * (128 + k / 128 + 18) * 2.0 ** -24 * size + 1e-6
+    for accumulate in (False, True):
+        out = base.to(DEV)
+        ops.linear(x.to(DEV), w.to(DEV), b.to(DEV), out, accumulate=accumulate)
+        err = (out.cpu().double() - want - (base.double() if accumulate else 0.0)).abs()
+        assert bool((err <= bound).all()), (err / bound).max().item()
