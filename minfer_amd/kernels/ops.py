@@ -167,7 +167,7 @@ _PROTOTYPES = {
                                      c_int, c_float, c_int, c_int, c_int, c_int, _P],
     },
     "attn_prefill_bf16": {
-        "mf_attn_prefill_bf16": [_P, _P, _P, _P, c_int, _P, _P, _P, _P, _P, _P, _P, c_int, _P, c_int, c_int, c_int,
+        "mf_attn_prefill_bf16": [_P, _P, _P, _P, c_int, _P, _P, _P, _P, _P, _P, c_int, _P, c_int, c_int, c_int,
                                  c_int, c_int, c_int, c_float, c_int, _P],
         "mf_attn_prefill_part_floats": [c_int],
         "mf_attn_prefill_rows": [c_int],
@@ -2411,20 +2411,16 @@ def attn_prefill(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor, pa
         tq, PAGE, window, per_tile, cu_count(), per_cu, PREFILL_MIN_PAGES, PREFILL_MAX_SHARES)
     if shared is None:
         tile_seq, tile_q0 = ctx.query_tiles(tq)
-        tile_share = parts = arrived = None
+        tile_share = parts = None
     else:
         tile_seq, tile_q0, tile_share, n_slots, most_shares = shared
         part = _fn("attn_prefill_bf16", "mf_attn_prefill_part_floats")(head_dim)
         parts = workspace("prefill_parts", n_slots * per_tile * most_shares * part, q.device)
-        arrived = _zeroed_counters("prefill_arrived", n_slots * per_tile, q.device)
-    rc = _fn("attn_prefill_bf16", "mf_attn_prefill_bf16")(
+    _check(_fn("attn_prefill_bf16", "mf_attn_prefill_bf16")(
         q, kcache, vcache, page_table, page_table.shape[1], ctx.cu_seqlens,
-        ctx.start_pos, tile_seq, tile_q0, tile_share, parts, arrived,
+        ctx.start_pos, tile_seq, tile_q0, tile_share, parts,
         most_shares if shared is not None else 1, out, tile_seq.numel(), n_heads, n_kv_heads, head_dim,
-        gh, tq, float(scale), window, _stream())
-    if rc != 0 and arrived is not None:
-        arrived.zero_()                  # a launch that failed may have left workgroups counted in
-    _check(rc, "attn_prefill_bf16")
+        gh, tq, float(scale), window, _stream()), "attn_prefill_bf16")
 
 
 # ------------------------------------------------------------------ sampling
