@@ -108,7 +108,7 @@ __global__ __launch_bounds__(64 * WK, WK > 1 && wave_registers(RB) <= 256 ? 2 : 
   const int h0 = hk * G + (hg % n_hc) * RB;
   const int col = lane & 15, g = lane >> 4;
 
-  const int b = tile_seq[tile], q0 = tile_q0[tile];
+  const int b = tile_seq[tile], q0 = tile_q0 ? tile_q0[tile] : 0;
   const int t_first = cu_seqlens[b] + q0;
   const int n_new = cu_seqlens[b + 1] - cu_seqlens[b];
   const int rows = min(16, n_new - q0);
@@ -405,7 +405,7 @@ MF_API int mf_capped_mfma_sizes(int* d, int* v) {
   return 0;
 }
 
-// tiles: blocks of 16 consecutive new tokens of a sequence (tile_seq, tile_q0), n_tiles of them; heads: of a kv head that a
+// tiles: blocks of 16 consecutive new tokens of a sequence (tile_seq, tile_q0; null: each from the sequence's first), n_tiles of them; heads: of a kv head that a
 // wave takes together; waves: of a tile (one where the tiles' keys are split)
 MF_API int mf_capped_mfma(const void* q, const void* kc, const void* vc, const int* page_table, int pt_stride,
                           const int* cu_seqlens, const int* start_pos, const int* tile_seq, const int* tile_q0,

@@ -1381,9 +1381,8 @@ def capped_attn_prefill(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Ten
     n_splits, split_len, part = 1, 0, None
     form = None
     if ctx.all_decode:
-        # every sequence is a tile of one token; nothing comes from the host (the step may be captured)
-        tile_seq = ctx.seq_of_tok
-        tile_q0 = torch.zeros(n_tok, dtype=torch.int32, device=q.device)
+        # every sequence is a tile of one token, its first; nothing comes from the host (the step may be captured)
+        tile_seq, tile_q0 = ctx.seq_of_tok, None
         reach = min(ctx.max_len, window) if window else ctx.max_len
         if chunk:
             reach = min(reach, int(chunk))
