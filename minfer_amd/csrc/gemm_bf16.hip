@@ -2469,6 +2469,15 @@ int launch_form(int form, const bf16* A, int lda, const bf16* W, int ldw, const 
              : launch_tile64<false>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi, stream, splits, k_per_split);
 }
 
+// A few weight rows past whole tiles (a gate beside q|k|v, a low-rank factor) can cost a whole round of them: 2,048 rows against
+// 8,192 of 2,048 are 256 tiles of 256 x 256, a CU each, against 8,224 264.  Up to 64 of them are then a product of their own, in
+// small tiles behind the large ones (variant 16).  The weight rows of the first product, or 0: none are left over, or the
+// epilogue takes its columns together.
+int main_rows(int N, int epi) {
+  const int rest = N % 256;
+  return N > 256 && rest > 0 && rest <= 64 && (epi == EPI_F32 || epi == EPI_ACC_F32 || epi == EPI_BF16) ? N - rest : 0;
+}
+
 // by their columns where the tile has 256 rows
 const char* form_name(int form, bool split) {
   static const char* names[N_FORMS][2] = {{"tile_dma_kernel<256>", "tile_dma_kernel<256>(split K)"},
@@ -2513,6 +2522,9 @@ TilePlan plan_tiles(int M, int N, int K, bool dma_ok, int epi, int n_cu) {
     offer(12, 1, K, form(12, 1, nkt) + start_us + epi_us);
     offer(13, 1, K, form(13, 1, nkt) + start_us + epi_us);
     if (epi != EPI_SWIGLU) offer(15, 1, K, form(15, 1, nkt) + start_us + epi_us);
+    if (const int n0 = main_rows(N, epi))
+      offer(16, 1, K, form_us(best_form(0, N_FORMS - 1, M, n0, nkt, 1, cu), M, n0, nkt, 1, cu) +
+                          form_us(best_form(FORM_128, FORM_TINY, M, N - n0, nkt, 1, cu), M, N - n0, nkt, 1, cu) + 2 * start_us + epi_us);
     // many rows against few weight rows and a long K (the down product of a prompt): K cut over
     // the big tiles, each part at least 2,048 of K
     if (epi != EPI_SWIGLU && M >= 768)
@@ -2605,7 +2617,8 @@ MF_API int mf_gemm_bf16_grouped(const void* A, const void* W, float* C, const in
 
 // `variant`: 0 picks by shape among the whole-K kernels; 1: 256x256 tile with 4 waves, 2: 128x128,
 // 3: 64x64, 6: 256x128 with 8 waves, 9: 256x256 with 8 waves; through the direct-to-LDS pipeline, K in
-// 64s: 12: 256x256 (SwiGLU: or 256x192), 13: the cheapest of 256x128, 128x256, 128x128 and 64x64, 15: 256x192 (tests name them).
+// 64s: 12: 256x256 (SwiGLU: or 256x192), 13: the cheapest of 256x128, 128x256, 128x128 and 64x64, 15: 256x192 (tests name them),
+// 16: the cheapest of all for the weight rows up to a multiple of 256, and of the small ones for up to 64 behind them.
 MF_API int mf_gemm_bf16(const void* A, int lda, const void* W, int ldw, const float* bias, void* C,
                         int ldc, int M, int N, int K, int epi, int variant, hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
@@ -2622,6 +2635,16 @@ MF_API int mf_gemm_bf16(const void* A, int lda, const void* W, int ldw, const fl
     const TilePlan plan = plan_tiles(M, N, K, dma_ok, epi, cu_count());
     if (plan.splits > 1) return (int)hipErrorInvalidValue;       // a K split needs the caller's workspace
     variant = plan.variant;
+  }
+  if (variant == 16) {
+    const int n0 = main_rows(N, epi), cu = cu_count();
+    if (!n0 || !dma_ok || cu <= 0) return (int)hipErrorInvalidValue;
+    const long nkt = K / DMA_BK;
+    const int rc = launch_form(best_form(0, N_FORMS - 1, M, n0, nkt, 1, cu), a, lda, w, ldw, bias, C, ldc, M, n0, K, epi, stream);
+    if (rc) return rc;
+    void* rest = (char*)C + (size_t)n0 * (epi == EPI_BF16 ? 2 : 4);
+    return launch_form(best_form(FORM_128, FORM_TINY, M, N - n0, nkt, 1, cu), a, lda, w + (size_t)n0 * ldw, ldw, bias ? bias + n0 : nullptr,
+                       rest, ldc, M, N - n0, K, epi, stream);
   }
   if (epi == EPI_SWIGLU && variant == 3) variant = 2;      // needs two 32-column tiles per wave
   switch (variant) {
@@ -2859,6 +2882,7 @@ MF_API int mf_gemm_bf16_plan(int M, int N, int K, int aligned, int tiled, int ep
       case 12: case 13: case 15:
         what = form_name(dma_form(plan.variant, M, N, epi, (split ? plan.k_per_split : K) / DMA_BK, plan.splits, n_cu), split);
         break;
+      case 16: what = "tile kernels (the last weight rows apart)"; break;
       case 9: what = "tile_kernel<256,256>"; break;
       case 2:
         what = split && dma_ok ? form_name(dma_form(2, M, N, EPI_F32, plan.k_per_split / DMA_BK, plan.splits, n_cu), true)
