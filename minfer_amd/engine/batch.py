@@ -100,7 +100,7 @@ class StepContext:
         return self._memo[key]
 
     def shared_query_tiles(self, block: int, page: int, window: int, n_heads: int, n_cu: int, per_cu: int,
-                           min_pages: int, max_shares: int, min_imbalance: float = 1.5):
+                           min_pages: int, max_shares: int, min_imbalance: float = 1.5, at_once: bool = False):
         """(tile_seq, tile_q0, tile_share, n_slots, most shares): as `query_tiles`, but a block of queries with
         many pages of keys is listed several times, once for each of the workgroups that are to
         take its pages in turn.  A workgroup should get at most its even share of the step's pages
@@ -110,9 +110,9 @@ class StepContext:
         sharing, or where sharing cannot gain: the step takes at least as long as a CU's even
         share of all pages and as its longest block, and only where the longest block is
         `min_imbalance` times that share is there time to win by cutting it (putting the parts
-        together has a price).  Kept per set of arguments: layers with other head counts plan for
-        themselves."""
-        key = ("shared_query_tiles", block, page, window, n_heads, n_cu, per_cu, min_pages, max_shares, min_imbalance)
+        together has a price).  `at_once`: shares grow until all workgroups run at once, where the blocks
+        alone do.  Kept per set of arguments: layers with other head counts plan for themselves."""
+        key = ("shared_query_tiles", block, page, window, n_heads, n_cu, per_cu, min_pages, max_shares, min_imbalance, at_once)
         if key not in self._memo:
             tiles = []
             for b, n in enumerate(self.host_new):
@@ -127,11 +127,11 @@ class StepContext:
                 self._memo[key] = None
                 return None
             target = max(1, int(min_pages), -(-total * n_heads // max(1, n_cu * per_cu)))
-            # all of them at once, where the blocks of queries themselves are: a few workgroups that wait for a place double the
-            # time (604 tokens on up to 5,000 keys, 16 heads on 2: 560 workgroups in 512 places 79 us, 480 65)
+            # (a few workgroups that wait for a place double the time: 604 tokens on up to 5,000 keys, 16 heads on 2, 560
+            # workgroups in 512 places 79 us, 480 of them 65)
             def in_all(t):
                 return n_heads * sum(min(max_shares, (pages + t - 1) // t) for pages, _, _ in tiles)
-            if len(tiles) * n_heads <= n_cu * per_cu:
+            if at_once and len(tiles) * n_heads <= n_cu * per_cu:
                 while in_all(target) > n_cu * per_cu:
                     target += 1
             entries, n_slots, most = [], 0, 1

@@ -2407,7 +2407,7 @@ def attn_prefill(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor, pa
     tq, gh, per_tile = prefill_tile(n_heads, n_kv_heads, head_dim)
     per_cu = _prefill_per_cu(head_dim)
     shared = None if tuning.NO_SHARED_PAGES else ctx.shared_query_tiles(
-        tq, PAGE, window, per_tile, cu_count(), per_cu, PREFILL_MIN_PAGES, PREFILL_MAX_SHARES)
+        tq, PAGE, window, per_tile, cu_count(), per_cu, PREFILL_MIN_PAGES, PREFILL_MAX_SHARES, at_once=True)
     if shared is None:
         tile_seq, tile_q0 = ctx.query_tiles(tq)
         tile_share = parts = None

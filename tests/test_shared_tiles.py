@@ -21,7 +21,7 @@ def step(new, start):
 ])
 def test_shares_fit_the_chip_and_cover_every_page_once(new, start, block, heads, per_cu, window):
     places = 256 * per_cu
-    got = step(new, start).shared_query_tiles(block, 64, window, heads, 256, per_cu, 4, 8)
+    got = step(new, start).shared_query_tiles(block, 64, window, heads, 256, per_cu, 4, 8, at_once=True)
     blocks = [(b, q) for b, n in enumerate(new) for q in range(0, n, block)]
     if got is None:
         assert len(blocks) * heads > places
