@@ -15,7 +15,8 @@
 //  * `rolling16_kernel`, `skinny16_kernel`: at most 16 rows, any K (decode).  The time is the
 //    weight stream: the waves of a block split K, each reads weights and activations straight
 //    into MFMA operands (16x16x32) and the partial sums meet in LDS.
-//  * `panel_kernel`: 17 to 64 rows against a wide matrix: one block per CU over the whole of K.
+//  * `panel_kernel`: 17 to 64 rows against a wide matrix: one block per CU over the whole of K; `panel_dma_kernel`: the same for up to
+//    128 rows with copies straight into LDS, where all its tiles are on the chip at once.
 //  * `skinny_ring_kernel`, `skinny_kernel` (any alignment): 17 to 64 rows.  Each wave owns 16
 //    weight rows and reads them from HBM straight into MFMA operands, the activation rows are
 //    staged in LDS and shared by the block, K may be split over blocks with a fixed-order
@@ -2065,6 +2066,222 @@ __global__ __launch_bounds__(512) void panel_kernel(const bf16* __restrict__ A, 
   }
 }
 
+// ---- one tile row against a wide matrix, a block per CU over the whole of K
+// A block takes RA rows (at least M) and 32 J weight rows and copies k tiles of both straight into LDS, STAGES of them: what
+// bounds it is the stream of weights and, from 100 rows on, how much a CU's copies bring in at once (some 55 GB/s of weights from
+// memory and activations from L2 together), so rows past M are not copied (lanes switched off; the copies still count), the
+// weight rows are cut to the number of CUs (tiles of 160 for 37,888: 237 blocks where tiles of 256 make 148), and the results of
+// a block meet in LDS, where gates and ups of a SwiGLU pair up whichever waves held them.
+// TURNS: the two waves of a SIMD in turns, one reading a k tile's fragments while the other multiplies (one group of waves a half
+// k tile behind the other); without, all read and all multiply.
+// SwiGLU of 37,888 x 3,584: 64 rows 50.8 us (5.3 TB/s of weights; `panel_kernel` 58.7), 100 rows 55.6 (tiles of 128 x 256 66.7),
+// without TURNS 2 us more.
+template <int I, int J, int RA, int STAGES>
+struct PanelTile {
+  static constexpr int WM = 4, WN = 2, BN = 32 * J, P = (RA + BN) / 8, L = (P + 7) / 8, ST = (RA + BN) * DMA_BK * 2, OLD = BN + 4;
+  static constexpr int LDS = STAGES * ST > RA * OLD * 4 ? STAGES * ST : RA * OLD * 4;
+  static_assert(RA <= 16 * I * WM && RA % 8 == 0 && LDS <= 160 * 1024, "the rows fit the waves, the stages LDS");
+};
+
+template <int I, int J, int RA, int STAGES, bool TURNS>
+__global__ __launch_bounds__(512, 2) void panel_dma_kernel(const bf16* __restrict__ A, int lda, const bf16* __restrict__ W, int ldw,
+                                                           const float* __restrict__ bias, void* __restrict__ C, int ldc, int M, int N,
+                                                           int K, int epi, const float* __restrict__ in_ssq, int in_parts, float in_eps) {
+  using T = PanelTile<I, J, RA, STAGES>;
+  constexpr int WM = T::WM, BN = T::BN, P = T::P, L = T::L, ST = T::ST, ROW = DMA_BK * 2;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];      // [stage][RA rows of A, BN rows of W][64]
+  int at = blockIdx.x;
+  {
+    const int n = gridDim.x, per = n / 8, rem = n % 8, x = at % 8;          // (neighbours on one die)
+    at = x * per + min(x, rem) + at / 8;
+  }
+  const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wid % WM, wn = wid / WM, fr = lane & 15, fk = lane >> 4;
+  const bool pair = epi == EPI_SWIGLU;
+  // the block's weight rows: units u0 .. u0 + J - 1 of 32; of a pair (16 gate rows and the 16 up rows of the same outputs) the gates
+  // of all units first, then the ups
+  const int u0 = at * J;
+  auto weight_row = [&](int r) {
+    if (!pair) return u0 * 32 + r;
+    const int c = r >> 4, u = u0 + c % J;
+    return (u >> 1) * 64 + (u & 1) * 16 + (c / J) * 32 + (r & 15);
+  };
+  floatx4 acc[I][J];
+#pragma unroll
+  for (int i = 0; i < I; ++i)
+#pragma unroll
+    for (int j = 0; j < J; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+  // the rows' partial sums of squares are asked for here and added up behind the products (8 lanes a row)
+  constexpr int SUMS = (RA + 63) / 64;
+  float part[SUMS][2];
+#pragma unroll
+  for (int q = 0; q < SUMS; ++q)
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+      part[q][e] = in_ssq ? in_ssq[(size_t)min(q * 64 + wid * 8 + (lane >> 3), M - 1) * in_parts + min((lane & 7) + 8 * e, in_parts - 1)] : 0.f;
+  __builtin_amdgcn_sched_barrier(0);
+  // what a wave copies: pieces wid, 8 + wid, ... of 8 rows (chunk c of a row at position c ^ ((row >> 1) & 7))
+  const unsigned lds0 = (unsigned)(uintptr_t)smem;
+  unsigned g[L], dst[L];
+  unsigned long long lanes[L];
+#pragma unroll
+  for (int q = 0; q < L; ++q) {
+    const int p = q * 8 + wid, r = p * 8 + (lane >> 3), c = (lane & 7) ^ ((r >> 1) & 7);
+    const bool of_a = p * 8 < RA;
+    const int row = of_a ? r : weight_row(r - RA);
+    lanes[q] = __builtin_amdgcn_ballot_w64(p < P && row < (of_a ? M : N));
+    g[q] = ((unsigned)min(row, (of_a ? M : N) - 1) * (unsigned)(of_a ? lda : ldw) + c * 8) * 2u;
+    dst[q] = lds0 + min(p, P - 1) * 1024;
+  }
+  const int nkt = K / DMA_BK;
+  auto copy = [&](int kt, int st) {                          // (past the last tile: that one again, never read)
+    const int k = min(kt, nkt - 1) * DMA_BK;
+#pragma unroll
+    for (int q = 0; q < L; ++q)
+      asm volatile("s_mov_b32 m0, %2\n\ts_mov_b64 exec, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1\n\ts_mov_b64 exec, -1" ::"v"(g[q]),
+                   "s"((q * 8 + wid) * 8 < RA ? A + k : W + k), "s"(__builtin_amdgcn_readfirstlane(dst[q] + st * ST)), "s"(lanes[q])
+                   : "m0");
+  };
+  const int sw = (fr >> 1) & 7;
+  bf16x8 fa[2][I], fw[2][J];
+  auto read = [&](int st) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int pos = ((4 * h + fk) ^ sw) * 16;
+      const unsigned char* s = smem + st * ST + fr * ROW + pos;
+#pragma unroll
+      for (int i = 0; i < I; ++i) fa[h][i] = *reinterpret_cast<const bf16x8*>(s + min((wm * I + i) * 16, RA - 16) * ROW);
+#pragma unroll
+      for (int j = 0; j < J; ++j) fw[h][j] = *reinterpret_cast<const bf16x8*>(s + (RA + (wn * J + j) * 16) * ROW);
+    }
+  };
+  auto multiply = [&]() {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int i = 0; i < I; ++i)
+#pragma unroll
+        for (int j = 0; j < J; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[h][j], fa[h][i], acc[i][j], 0, 0, 0);
+  };
+#pragma unroll
+  for (int t = 0; t < STAGES - 1; ++t) copy(t, t);
+  int st = 0;
+  if constexpr (TURNS) {
+    // Waves w and w + 4 share a SIMD.  A stage is set out again in a group's read slot of the tile behind it: both groups have
+    // its fragments in registers then (lgkmcnt(0) in front of the barriers between).  Tile kt + 1 has landed for every wave at
+    // the end of the second group's read slot of tile kt, which is the first one's product slot.
+    const bool second = wid >= 4;
+    dma_wait<(STAGES - 2) * L>();
+    dma_meet();
+    if (second) dma_meet();
+    for (int kt = 0; kt < nkt; ++kt) {
+      read(st);
+      __builtin_amdgcn_sched_barrier(0);
+      copy(kt + STAGES - 1, st == 0 ? STAGES - 1 : st - 1);
+      st = st == STAGES - 1 ? 0 : st + 1;
+      if (second) dma_wait<(STAGES - 2) * L>();
+      else asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      dma_meet();
+      __builtin_amdgcn_s_setprio(1);
+      multiply();
+      __builtin_amdgcn_s_setprio(0);
+      if (!second) dma_wait<(STAGES - 2) * L>();
+      dma_meet();
+    }
+    if (!second) dma_meet();
+  } else {
+    for (int kt = 0; kt < nkt; ++kt) {
+      dma_wait<(STAGES - 2) * L>();                          // tile kt is here, and the one before in every wave's registers
+      dma_meet();
+      copy(kt + STAGES - 1, st == 0 ? STAGES - 1 : st - 1);
+      read(st);
+      multiply();
+      st = st == STAGES - 1 ? 0 : st + 1;
+    }
+  }
+  dma_wait<0>();
+  dma_meet();
+  // the results, [RA][BN + 4]; D: the lane's row is lane % 16, its columns 4 (lane / 16) + e
+  float* out = reinterpret_cast<float*>(smem);
+  __shared__ float fac[RA];
+#pragma unroll
+  for (int q = 0; q < SUMS; ++q) {
+    const int r = q * 64 + wid * 8 + (lane >> 3);
+    float t = (lane & 7) < in_parts ? part[q][0] : 0.f;
+    t += (lane & 7) + 8 < in_parts ? part[q][1] : 0.f;
+    for (int p = (lane & 7) + 16; p < in_parts; p += 8) t += in_ssq[(size_t)min(r, M - 1) * in_parts + p];
+#pragma unroll
+    for (int o = 1; o < 8; o <<= 1) t += __shfl_xor(t, o, MF_WAVE);
+    if ((lane & 7) == 0 && r < RA) fac[r] = in_ssq ? 1.0f / sqrtf(t / (float)K + in_eps) : 1.0f;
+  }
+#pragma unroll
+  for (int i = 0; i < I; ++i)
+#pragma unroll
+    for (int j = 0; j < J; ++j)
+      if ((wm * I + i) * 16 < RA) {
+        const floatx4 v = acc[i][j];
+        *reinterpret_cast<float4*>(out + ((wm * I + i) * 16 + fr) * T::OLD + (wn * J + j) * 16 + fk * 4) = float4{v[0], v[1], v[2], v[3]};
+      }
+  __syncthreads();
+  if (pair) {
+    const bool vec = ldc % 4 == 0 && (uintptr_t)C % 8 == 0;
+    auto gated = [&](auto act) {
+      for (int x = threadIdx.x; x < M * 4 * J; x += 512) {
+        const int r = x / (4 * J), c = (x % (4 * J)) * 4, col = u0 * 16 + c;
+        const float4 gt = *reinterpret_cast<const float4*>(out + r * T::OLD + c), up = *reinterpret_cast<const float4*>(out + r * T::OLD + BN / 2 + c);
+        const float f = fac[r];
+        const bf16x4 v = {(bf16)act(gt.x * f, up.x * f), (bf16)act(gt.y * f, up.y * f), (bf16)act(gt.z * f, up.z * f), (bf16)act(gt.w * f, up.w * f)};
+        bf16* o = (bf16*)C + (size_t)r * ldc + col;
+        if (vec && col + 4 <= ldc) *reinterpret_cast<bf16x4*>(o) = v;
+        else
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (col + e < ldc) o[e] = v[e];
+      }
+    };
+    if (bias) {
+      const float limit = *bias;
+      gated([=](float gt, float up) { return clamped_gate(gt, up, limit); });
+    } else {
+      gated([](float gt, float up) { return swiglu_f(gt, up, nullptr); });
+    }
+    return;
+  }
+  const bool vec = epi != EPI_BF16 && epi != EPI_XIELU && ldc % 4 == 0 && (uintptr_t)C % 16 == 0;
+  for (int x = threadIdx.x; x < M * (BN / 4); x += 512) {
+    const int r = x / (BN / 4), c = (x % (BN / 4)) * 4, n = u0 * 32 + c;
+    if (n >= N) continue;
+    const float4 v4 = *reinterpret_cast<const float4*>(out + r * T::OLD + c);
+    float v[4] = {v4.x, v4.y, v4.z, v4.w};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = v[e] * fac[r] + (bias && n + e < N ? bias[n + e] : 0.f);
+    if (vec && n + 4 <= N) {
+      float4* o = reinterpret_cast<float4*>((float*)C + (size_t)r * ldc + n);
+      float4 old = epi == EPI_ACC_F32 ? *o : float4{0.f, 0.f, 0.f, 0.f};
+      *o = float4{old.x + v[0], old.y + v[1], old.z + v[2], old.w + v[3]};
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (n + e < N) store_out(C, ldc, r, n + e, v[e], epi, bias, N);
+    }
+  }
+}
+
+template <int I, int J, int RA, int STAGES, bool TURNS>
+int launch_panel_dma(const bf16* A, int lda, const bf16* W, int ldw, const float* bias, void* C, int ldc, int M, int N, int K, int epi,
+                     const FusedNorm& fused, hipStream_t stream) {
+  using T = PanelTile<I, J, RA, STAGES>;
+  auto kern = panel_dma_kernel<I, J, RA, STAGES, TURNS>;
+  static bool configured = false;
+  if (!configured) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, T::LDS);
+    if (e != hipSuccess) return (int)e;
+    configured = true;
+  }
+  kern<<<((N + 31) / 32 + J - 1) / J, 512, T::LDS, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi, fused.in_ssq, fused.in_parts, fused.in_eps);
+  return mf_launch_status();
+}
+
 // The parts of a split are added in rounds of up to eight, a round's loads in flight together, in
 // the order of the splits (a plain loop over a count that is not known here is left to run split
 // by split, a trip to memory each).
@@ -2489,6 +2706,8 @@ const char* form_name(int form, bool split) {
   return names[form][split];
 }
 
+int panel_dma_units(int M, int N, int K, int epi, int n_cu);
+
 TilePlan plan_tiles(int M, int N, int K, bool dma_ok, int epi, int n_cu) {
   const long cu = n_cu > 0 ? n_cu : 1;
   const long nkt = (K + 63) / 64, chunks = (K + 255) / 256;
@@ -2519,6 +2738,7 @@ TilePlan plan_tiles(int M, int N, int K, bool dma_ok, int epi, int n_cu) {
     return form_us(dma_form(variant, M, N, epi, steps, splits, cu), M, N, steps, splits, cu);
   };
   if (dma_ok) {
+    if (M > 64 && panel_dma_units(M, N, K, epi, n_cu)) return TilePlan{13, 1, K, 0.};
     offer(12, 1, K, form(12, 1, nkt) + start_us + epi_us);
     offer(13, 1, K, form(13, 1, nkt) + start_us + epi_us);
     if (epi != EPI_SWIGLU) offer(15, 1, K, form(15, 1, nkt) + start_us + epi_us);
@@ -2553,10 +2773,34 @@ TilePlan plan_tiles(int M, int N, int K, bool dma_ok, int epi, int n_cu) {
   return best;
 }
 
+// Where `panel_dma_kernel` runs: J of its tiles (32 J weight rows), or 0.  All tiles are on the chip at once.
+//  * 17 to 64 rows: in `panel_kernel`'s place up to 160 weight rows a CU (SwiGLU of 37,888 x 3,584, 17 / 48 / 64 rows 50.5 / 53.9 /
+//    58.7 us there and 48.9 / 49.8 / 50.8 so; 40,960 x 512 17.2 and 11.9); beyond, that kernel's blocks go on from pass to pass.
+//  * 51 to 64 rows, SwiGLU, more than 64 and up to 96 weight rows a CU against a K of up to 2,048, where 64 x 64 tiles are two a CU:
+//    22,016 x 2,048, 64 rows 27.6 and 23.9; 17,920 x 1,536 20.7 and 16.3.  (Fewer rows gain less, 33 rows 25.5 and 23.2, and are left
+//    with the tiles, as are 64 weight rows a CU and fewer: 9,728 x 896 6.0 and 7.7.)
+//  * 65 to 128 rows, more than 128 and up to 160 weight rows a CU, where tiles of 128 x 128 take two rounds and tiles of 128 x 256
+//    leave a third of the CUs idle: SwiGLU of 37,888 x 3,584, 65 / 100 / 128 rows 63.5 / 66.7 / 68.9 and 52.6 / 55.6 / 58.7.  (32,768 x
+//    2,048, a round of 128 x 128: 36.2 and 38.5; 208 rows, in tiles of 208 x 160: level with 256 x 192.)
+int panel_dma_units(int M, int N, int K, int epi, int n_cu) {
+  const int units = (N + 31) / 32;
+  if (M <= 16 || M > 128 || K % DMA_BK || n_cu <= 0 || units > 5 * n_cu) return 0;
+  if (units > 4 * n_cu || (M <= 64 && units == 4 * n_cu)) return 5;
+  return M > 50 && M <= 64 && epi == EPI_SWIGLU && K <= 2048 && units > 2 * n_cu && units <= 3 * n_cu ? 3 : 0;
+}
+
+int launch_panel_rows(int J, const bf16* A, int lda, const bf16* W, int ldw, const float* bias, void* C, int ldc, int M, int N, int K,
+                      int epi, const FusedNorm& fused, hipStream_t stream) {
+#define MF_PANEL(I_, J_, RA_, STAGES_, TURNS_) launch_panel_dma<I_, J_, RA_, STAGES_, TURNS_>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi, fused, stream)
+  if (M > 64) return MF_PANEL(2, 5, 128, 4, true);
+  return J == 5 ? MF_PANEL(1, 5, 64, 5, false) : MF_PANEL(1, 3, 64, 6, false);
+#undef MF_PANEL
+}
+
 // Which kernel a product of at most 64 rows takes.
 enum SkinnyChoice {
   SK_STATIONARY, SK_ROLLING, SK_GUARDED_PAIR, SK_GUARDED_4X2, SK_GUARDED_8X2, SK_GUARDED_8X1, SK_PANEL, SK_RING,
-  SK_STAGED, SK_TILE
+  SK_STAGED, SK_TILE, SK_PANEL_SHORT
 };
 
 // 17 to 64 rows against a short K: a tile of 64 x 64 over the whole of K, with the norm's factors, the bias and SwiGLU in its
@@ -2590,6 +2834,7 @@ SkinnyChoice skinny_choice(int M, int N, int K, bool aligned, bool tiled, int ep
     return SK_GUARDED_8X1;
   }
   if (M > 16 && panel_takes(M, N, K, aligned, epi, n_cu)) return SK_PANEL;
+  if (aligned && panel_dma_units(M, N, K, epi, n_cu) == 3) return SK_PANEL_SHORT;
   if (tile64_takes(M, N, K, aligned, tiled, epi, n_cu)) return SK_TILE;
   return ring_takes(aligned, K, splits, k_per_split) ? SK_RING : SK_STAGED;
 }
@@ -2617,8 +2862,10 @@ MF_API int mf_gemm_bf16_grouped(const void* A, const void* W, float* C, const in
 
 // `variant`: 0 picks by shape among the whole-K kernels; 1: 256x256 tile with 4 waves, 2: 128x128,
 // 3: 64x64, 6: 256x128 with 8 waves, 9: 256x256 with 8 waves; through the direct-to-LDS pipeline, K in
-// 64s: 12: 256x256 (SwiGLU: or 256x192), 13: the cheapest of 256x128, 128x256, 128x128 and 64x64, 15: 256x192 (tests name them),
-// 16: the cheapest of all for the weight rows up to a multiple of 256, and of the small ones for up to 64 behind them.
+// 64s: 12: 256x256 (SwiGLU: or 256x192), 13: the cheapest of 256x128, 128x256, 128x128 and 64x64 (or the
+// panel kernel where it runs), 15: 256x192 (tests name them),
+// 16: the cheapest of all for the weight rows up to a multiple of 256, and of the small ones for up to 64 behind them; 17: the panel
+// kernel with copies straight into LDS.
 MF_API int mf_gemm_bf16(const void* A, int lda, const void* W, int ldw, const float* bias, void* C,
                         int ldc, int M, int N, int K, int epi, int variant, hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
@@ -2635,6 +2882,11 @@ MF_API int mf_gemm_bf16(const void* A, int lda, const void* W, int ldw, const fl
     const TilePlan plan = plan_tiles(M, N, K, dma_ok, epi, cu_count());
     if (plan.splits > 1) return (int)hipErrorInvalidValue;       // a K split needs the caller's workspace
     variant = plan.variant;
+  }
+  if (variant == 17 || (variant == 13 && M > 64 && dma_ok && panel_dma_units(M, N, K, epi, cu_count()))) {
+    const int J = panel_dma_units(M, N, K, epi, cu_count());
+    if (!J || !dma_ok) return (int)hipErrorInvalidValue;
+    return launch_panel_rows(J, a, lda, w, ldw, bias, C, ldc, M, N, K, epi, FusedNorm{}, stream);
   }
   if (variant == 16) {
     const int n0 = main_rows(N, epi), cu = cu_count();
@@ -2772,7 +3024,14 @@ static int skinny_product(const void* A, int lda, const void* W, const void* Wt,
     case SK_GUARDED_4X2: return launch_skinny16<4, 2, 4>(a, lda, w, ldw, bias, C, ldc, M, N, K, epi, vec_ok, stream);
     case SK_GUARDED_8X2: return launch_skinny16<8, 2, 4>(a, lda, w, ldw, bias, C, ldc, M, N, K, epi, vec_ok, stream);
     case SK_GUARDED_8X1: return launch_skinny16<8, 1, 8>(a, lda, w, ldw, bias, C, ldc, M, N, K, epi, vec_ok, stream);
-    case SK_PANEL: return launch_panel(a, lda, w, wt, ldw, bias, C, ldc, M, N, K, epi, fused, stream);
+    case SK_PANEL:
+    case SK_PANEL_SHORT: {
+      // (the panel kernels take a prepared norm and prepare none; 32-bit byte offsets)
+      const int J = (size_t)N * ldw * 2 < (1ull << 32) && !fused.out_g ? panel_dma_units(M, N, K, epi, cu_count()) : 0;
+      if (J) return launch_panel_rows(J, a, lda, w, ldw, bias, C, ldc, M, N, K, epi, fused, stream);
+      if (choice == SK_PANEL_SHORT) break;
+      return launch_panel(a, lda, w, wt, ldw, bias, C, ldc, M, N, K, epi, fused, stream);
+    }
     case SK_TILE:
       // (the next norm's sums of squares come from the K-split kernels' second one; operands beyond 4 GB go to them as well)
       if (fused.out_g || (size_t)N * ldw * 2 >= (1ull << 32)) break;
@@ -2868,7 +3127,8 @@ MF_API int mf_gemm_bf16_plan(int M, int N, int K, int aligned, int tiled, int ep
       case SK_STATIONARY: what = "stationary16_kernel"; break;
       case SK_ROLLING: what = "rolling16_kernel"; break;
       case SK_GUARDED_PAIR: case SK_GUARDED_4X2: case SK_GUARDED_8X2: case SK_GUARDED_8X1: what = "skinny16_kernel"; break;
-      case SK_PANEL: what = "panel_kernel"; break;
+      case SK_PANEL: what = "panel_kernel"; break;           // (either form: `panel_dma_units`)
+      case SK_PANEL_SHORT: what = "panel_dma_kernel"; break;
       case SK_RING: what = "skinny_ring_kernel"; break;
       case SK_STAGED: what = "skinny_kernel"; break;
       case SK_TILE: what = "tile_step_kernel<64,64>"; break;
@@ -2880,9 +3140,11 @@ MF_API int mf_gemm_bf16_plan(int M, int N, int K, int aligned, int tiled, int ep
     if (variant >= 12 && !dma_ok) return (int)hipErrorInvalidValue;
     switch (plan.variant) {
       case 12: case 13: case 15:
-        what = form_name(dma_form(plan.variant, M, N, epi, (split ? plan.k_per_split : K) / DMA_BK, plan.splits, n_cu), split);
+        if (plan.variant == 13 && M > 64 && panel_dma_units(M, N, K, epi, n_cu)) what = "panel_dma_kernel";
+        else what = form_name(dma_form(plan.variant, M, N, epi, (split ? plan.k_per_split : K) / DMA_BK, plan.splits, n_cu), split);
         break;
       case 16: what = "tile kernels (the last weight rows apart)"; break;
+      case 17: what = "panel_dma_kernel"; break;
       case 9: what = "tile_kernel<256,256>"; break;
       case 2:
         what = split && dma_ok ? form_name(dma_form(2, M, N, EPI_F32, plan.k_per_split / DMA_BK, plan.splits, n_cu), true)
