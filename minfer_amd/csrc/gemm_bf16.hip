@@ -173,12 +173,16 @@ __device__ __forceinline__ void block_work(int order, int& tile, int& part) {
   part = order == ORDER_PARTS ? at / (int)gridDim.x : blockIdx.y;
   tile = order == ORDER_PARTS ? at - part * (int)gridDim.x : at;
 }
-// Part by part where the activations of all of K are more than an XCD's L2 of 4 MB.  (rows x weight rows x K, microseconds with the
-// kernel behind it, the same eighth of every part / part by part: 2,048 x 2,048 x 8,192 78.1 / 73.8, 203 x 3,584 x 18,944 56.8 /
-// 53.9, 604 x 2,048 x 11,008 48.3 / 46.9, 400 x 1,536 x 8,960 29.5 / 28.2; but 604 x 2,048 x 2,048 22.2 / 24.8 and 400 x 896 x
-// 4,864 17.1 / 17.9.)
+// Part by part where the activations of all of K are more than an XCD's L2 of 4 MB and all parts' tiles are at most two a CU.  (rows x
+// weight rows x K, microseconds with the kernel behind it, the same eighth of every part / part by part: 203 x 3,584 x 18,944 54.8 /
+// 52.2, 2,048 x 2,048 x 8,192 79.1 / 74.8, 2,048 x 2,048 x 11,008 102.8 / 91.2, 2,048 x 896 x 4,864 38.7 / 33.5; less than an L2: 604 x
+// 2,048 x 2,048 22.2 / 24.8, 400 x 896 x 4,864 17.1 / 17.9.)  With more tiles the XCDs stand in different parts of K at one time: level
+// at 462 tiles (2,600 x 3,584 x 18,944 312.6 / 313), slower beyond: 3,300 x 5,120 x 13,824 (780) 455 / 469, 5,754 x 3,584 x 18,944
+// (966) 647 / 664, 8,192 x 5,120 x 13,824 (1,280) 913 / 932.
+static int cu_count();
 int tile_order(int tiles, int splits, int M, int K) {
-  return splits > 1 && (size_t)M * K * 2 > (4u << 20) ? ORDER_PARTS : tiles >= 16 ? ORDER_TILES : ORDER_PLAIN;
+  if (splits > 1 && (size_t)M * K * 2 > (4u << 20) && (long)tiles * splits <= 2L * cu_count()) return ORDER_PARTS;
+  return tiles >= 16 ? ORDER_TILES : ORDER_PLAIN;
 }
 
 // Rows of a product that belong to one of several matrices: `rows` of them (at most a tile's) from row `first` on.
