@@ -479,13 +479,12 @@ __global__ __launch_bounds__(64) void rope_kvwrite_kernel(
   }
 }
 
-// The same for head sizes that are multiples of 8 and 16-byte aligned rows: one block per token,
-// a thread takes four neighbouring pairs at a time (float4 loads of x, cos and sin, one 8- or
-// 16-byte store per half), q and k heads first, then v: the same bytes as one wave per token and
-// head with 4-byte accesses moves, in wide accesses.
+// The same for head sizes that are multiples of 8 and 16-byte aligned rows: one block per token, four neighbouring pairs at a time
+// (float4 loads of x, cos and sin, one 8- or 16-byte store per half), q and k heads first, then v: the same bytes as one wave per
+// token and head with 4-byte accesses moves, in wide accesses.
 // The rows may come in `parts` of a product whose K was split ([parts][tokens][row], added in their order, then the bias):
 // the launch and the pass of the kernel that would add them are saved (203 tokens of 36 heads in 7 parts: 6.6 + 5.6 us as
-// two kernels, 11.1 as one).
+// two kernels, 8.8 as one).
 template <typename OT>
 __device__ __forceinline__ void store4(OT* dst, float a, float b, float c, float d);
 template <>
@@ -496,14 +495,37 @@ template <>
 __device__ __forceinline__ void store4<bf16>(bf16* dst, float a, float b, float c, float d) {
   *reinterpret_cast<bf16x4*>(dst) = bf16x4{(bf16)a, (bf16)b, (bf16)c, (bf16)d};
 }
+__device__ __forceinline__ void add4(float4& v, const float4& x) { v.x += x.x; v.y += x.y; v.z += x.z; v.w += x.w; }
 
-// A thread takes four pairs of a rotated head or eight values of a v head, a block a token.  What few tokens in parts wait for is
-// one trip to memory: a thread asks for all parts of both halves of its pairs at once, and there is a thread for every item (up
-// to 1,024).  203 tokens of 36 heads of 128 in 7 parts: 12.2 us with 256 threads that went round three times and asked for one half
-// after the other, 8.8 so; 604 tokens of 20 heads in 4 parts 11.6 and 9.5.  2,048 tokens of one part have enough in flight
-// (17.8 us with 256 threads, 27 with a thread an item).
+// Four pairs rotated and stored, at dst and `half` behind it.  Which product of a sum the FMA takes in is written out: left to the
+// compiler it depends on the code around it, and one part and several would give other last bits.
+template <typename OT>
+__device__ __forceinline__ void store_rotated(OT* dst, int half, const float4& x0, const float4& x1, const float4& c, const float4& s) {
+  auto low = [](float a, float b, float cos, float sin) { return fmaf(a, cos, -(b * sin)); };
+  auto high = [](float a, float b, float cos, float sin) { return fmaf(b, cos, a * sin); };
+  store4<OT>(dst, low(x0.x, x1.x, c.x, s.x), low(x0.y, x1.y, c.y, s.y), low(x0.z, x1.z, c.z, s.z), low(x0.w, x1.w, c.w, s.w));
+  store4<OT>(dst + half, high(x0.x, x1.x, c.x, s.x), high(x0.y, x1.y, c.y, s.y), high(x0.z, x1.z, c.z, s.z),
+             high(x0.w, x1.w, c.w, s.w));
+}
+
+// Values i .. i + 3 of a v head of a token (`head`: number of its page and head, off: its row there) into the cache; a transposed page
+// is [2][hd][32 keys].
 template <typename OT, bool V_TRANSPOSED>
-__global__ __launch_bounds__(1024) void rope_kvwrite_vec_kernel(
+__device__ __forceinline__ void store_values(OT* vcache, size_t head, int off, int hd, int i, const float4& v) {
+  if (V_TRANSPOSED) {
+    constexpr int VH = MF_PAGE / 2;
+    OT* dst = vcache + ((head * 2 + off / VH) * hd + i) * VH + off % VH;
+    dst[0] = from_f32<OT>(v.x);
+    dst[VH] = from_f32<OT>(v.y);
+    dst[2 * VH] = from_f32<OT>(v.z);
+    dst[3 * VH] = from_f32<OT>(v.w);
+  } else {
+    store4<OT>(vcache + (head * MF_PAGE + off) * hd + i, v.x, v.y, v.z, v.w);
+  }
+}
+
+template <typename OT, bool V_TRANSPOSED>
+__global__ __launch_bounds__(256) void rope_kvwrite_vec_kernel(
     const float* __restrict__ qkv, const float* __restrict__ cs, const float* __restrict__ sn,
     const int* __restrict__ positions, const int* __restrict__ seq_of_tok,
     const int* __restrict__ page_table, int pt_stride, OT* __restrict__ q_out,
@@ -513,11 +535,64 @@ __global__ __launch_bounds__(1024) void rope_kvwrite_vec_kernel(
   const int half = hd >> 1, groups = half >> 2;           // groups of four pairs per head
   const int pos = positions[t];
   const size_t row0 = (size_t)t * (nh + 2 * nk) * hd, stride = (size_t)gridDim.x * (nh + 2 * nk) * hd;
-  auto add = [](float4& v, const float4& x) { v.x += x.x; v.y += x.y; v.z += x.z; v.w += x.w; };
+  auto four = [&](int at) {                               // values at .. at + 3 of the token's row
+    const float* p = qkv + row0 + at;
+    if (parts == 1) return *reinterpret_cast<const float4*>(p);
+    float4 v = float4{0.f, 0.f, 0.f, 0.f};
+    for (int s0 = 0; s0 < parts; s0 += 8) {
+      float4 x[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        x[j] = s0 + j < parts ? *reinterpret_cast<const float4*>(p + (size_t)(s0 + j) * stride) : float4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int j = 0; j < 8; ++j) add4(v, x[j]);
+    }
+    if (bias) add4(v, *reinterpret_cast<const float4*>(bias + at));
+    return v;
+  };
+  const int page = write_kv ? page_table[(size_t)seq_of_tok[t] * pt_stride + pos / MF_PAGE] : -1;
+  const int off = pos % MF_PAGE;
+  const int n_rot = (nh + (write_kv && page >= 0 ? nk : 0)) * groups;
+  for (int it = threadIdx.x; it < n_rot; it += 256) {
+    const int head = it / groups, i = (it % groups) * 4;
+    const float4 x0 = four(head * hd + i);
+    const float4 x1 = four(head * hd + i + half);
+    const float4 c = cs ? *reinterpret_cast<const float4*>(cs + (size_t)pos * half + i) : make_float4(1.f, 1.f, 1.f, 1.f);
+    const float4 s = cs ? *reinterpret_cast<const float4*>(sn + (size_t)pos * half + i) : make_float4(0.f, 0.f, 0.f, 0.f);
+    OT* dst = head < nh ? q_out + ((size_t)t * nh + head) * hd
+                        : kcache + (((size_t)page * nk + (head - nh)) * MF_PAGE + off) * hd;
+    store_rotated<OT>(dst + i, half, x0, x1, c, s);
+  }
+  if (!write_kv || page < 0) return;
+  for (int it = threadIdx.x; it < nk * (hd >> 2); it += 256) {
+    const int hk = it / (hd >> 2), i = (it % (hd >> 2)) * 4;
+    const float4 v = four((nh + nk + hk) * hd + i);
+    store_values<OT, V_TRANSPOSED>(vcache, (size_t)page * nk + hk, off, hd, i, v);
+  }
+}
+
+// The same for few tokens, which wait for their trips to memory: q, k and v heads in one loop, four pairs of a rotated head or eight
+// values of a v head at a time.  PARTS: there is a thread for every item (up to 1,024), and it asks for all parts of both halves at once:
+// 203 tokens of 36 heads of 128 in 6 parts 8.7 us by the kernel above, which goes round three times and asks for one half after the
+// other, 7.2 so; 604 tokens of 20 heads in 3 parts 9.0 and 7.5.  These loads cost 94 registers, five waves a SIMD, so it is only for
+// tokens that are on the chip at once (`few_tokens`): more have enough in flight by themselves, and go through faster with the eight
+// waves a SIMD of the kernel above (36 heads of 128: 604 tokens in 3 parts 12.3 us there and 13.6 here, 2,048 in 3 26.3 and 32.4).
+// One part: 256 threads, up to a token a CU (203 tokens of 18 heads of 64 3.4 us above and 3.0 here; 604 level).
+template <typename OT, bool V_TRANSPOSED, bool PARTS>
+__global__ __launch_bounds__(PARTS ? 1024 : 256) void rope_kvwrite_few_kernel(
+    const float* __restrict__ qkv, const float* __restrict__ cs, const float* __restrict__ sn,
+    const int* __restrict__ positions, const int* __restrict__ seq_of_tok,
+    const int* __restrict__ page_table, int pt_stride, OT* __restrict__ q_out,
+    OT* __restrict__ kcache, OT* __restrict__ vcache, int nh, int nk, int hd, int write_kv, int parts,
+    const float* __restrict__ bias) {
+  const int t = blockIdx.x;
+  const int half = hd >> 1, groups = half >> 2;
+  const int pos = positions[t];
+  const size_t row0 = (size_t)t * (nh + 2 * nk) * hd, stride = (size_t)gridDim.x * (nh + 2 * nk) * hd;
   // values at .. at + 3 of the token's row, and at + next .. : the parts in their order, then the bias
   auto fours = [&](int at, int next, float4& v0, float4& v1) {
     const float* p = qkv + row0 + at;
-    if (parts == 1) {
+    if (!PARTS) {
       v0 = *reinterpret_cast<const float4*>(p);
       v1 = *reinterpret_cast<const float4*>(p + next);
       return;
@@ -533,13 +608,13 @@ __global__ __launch_bounds__(1024) void rope_kvwrite_vec_kernel(
       }
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        add(v0, x[j]);
-        add(v1, y[j]);
+        add4(v0, x[j]);
+        add4(v1, y[j]);
       }
     }
     if (bias) {
-      add(v0, *reinterpret_cast<const float4*>(bias + at));
-      add(v1, *reinterpret_cast<const float4*>(bias + at + next));
+      add4(v0, *reinterpret_cast<const float4*>(bias + at));
+      add4(v1, *reinterpret_cast<const float4*>(bias + at + next));
     }
   };
   const int page = write_kv ? page_table[(size_t)seq_of_tok[t] * pt_stride + pos / MF_PAGE] : -1;
@@ -555,31 +630,28 @@ __global__ __launch_bounds__(1024) void rope_kvwrite_vec_kernel(
       fours(head * hd + i, half, x0, x1);
       OT* dst = head < nh ? q_out + ((size_t)t * nh + head) * hd
                           : kcache + (((size_t)page * nk + (head - nh)) * MF_PAGE + off) * hd;
-      store4<OT>(dst + i, x0.x * c.x - x1.x * s.x, x0.y * c.y - x1.y * s.y, x0.z * c.z - x1.z * s.z,
-                 x0.w * c.w - x1.w * s.w);
-      store4<OT>(dst + i + half, x0.x * s.x + x1.x * c.x, x0.y * s.y + x1.y * c.y, x0.z * s.z + x1.z * c.z,
-                 x0.w * s.w + x1.w * c.w);
+      store_rotated<OT>(dst + i, half, x0, x1, c, s);
       continue;
     }
     const int iv = it - n_rot, hk = iv / groups, i = (iv % groups) * 8;
     fours((nh + nk + hk) * hd + i, 4, x0, x1);
-    if (V_TRANSPOSED) {                   // a page of V is [2][hd][32 keys]
-      constexpr int VH = MF_PAGE / 2;
-      OT* dst = vcache + ((((size_t)page * nk + hk) * 2 + off / VH) * hd + i) * VH + off % VH;
-      dst[0] = from_f32<OT>(x0.x);
-      dst[VH] = from_f32<OT>(x0.y);
-      dst[2 * VH] = from_f32<OT>(x0.z);
-      dst[3 * VH] = from_f32<OT>(x0.w);
-      dst[4 * VH] = from_f32<OT>(x1.x);
-      dst[5 * VH] = from_f32<OT>(x1.y);
-      dst[6 * VH] = from_f32<OT>(x1.z);
-      dst[7 * VH] = from_f32<OT>(x1.w);
-    } else {
-      OT* dst = vcache + (((size_t)page * nk + hk) * MF_PAGE + off) * hd + i;
-      store4<OT>(dst, x0.x, x0.y, x0.z, x0.w);
-      store4<OT>(dst + 4, x1.x, x1.y, x1.z, x1.w);
-    }
+    store_values<OT, V_TRANSPOSED>(vcache, (size_t)page * nk + hk, off, hd, i, x0);
+    store_values<OT, V_TRANSPOSED>(vcache, (size_t)page * nk + hk, off, hd, i + 4, x1);
   }
+}
+
+// Threads of a block where `rope_kvwrite_few_kernel` takes `n_tok` tokens of `items` items, or 0.  In parts: blocks of as many waves as
+// five a SIMD leave room for on every CU.
+int few_tokens(int n_tok, int items, int parts) {
+  static int n_cu = 0;
+  if (n_cu == 0) {
+    int dev = 0, n = 0;
+    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
+    n_cu = n;
+  }
+  if (parts == 1) return n_tok <= n_cu ? 256 : 0;
+  const int waves = items >= 1024 ? 16 : items < 256 ? 4 : (items + 63) / 64;
+  return n_tok <= n_cu * (20 / waves) ? 64 * waves : 0;
 }
 
 // The rotation alone, in place, on the first n_rot heads of every token's [n_heads_total][hd] row
@@ -645,17 +717,17 @@ MF_API int mf_rope_kvwrite(const float* qkv, const float* cs, const float* sn, c
   const bool vec = hd % 8 == 0 && (uintptr_t)bias % 16 == 0 && (uintptr_t)qkv % 16 == 0 && (uintptr_t)cs % 16 == 0 && (uintptr_t)sn % 16 == 0 &&
                    (uintptr_t)q_out % 16 == 0 && (uintptr_t)kcache % 16 == 0 && (uintptr_t)vcache % 16 == 0;
   if (vec) {
-    const int items = (nh + (write_kv ? 2 * nk : 0)) * (hd / 8);
-    const int threads = parts == 1 || items < 256 ? 256 : items < 1024 ? (items + 63) / 64 * 64 : 1024;
+    const int few = few_tokens(n_tok, (nh + (write_kv ? 2 * nk : 0)) * (hd / 8), parts);
+    auto run = [&](auto kern, auto out) {
+      using OT = decltype(out);
+      kern<<<n_tok, few ? few : 256, 0, stream>>>(qkv, cs, sn, positions, seq_of_tok, page_table, pt_stride, (OT*)q_out, (OT*)kcache,
+                                                  (OT*)vcache, nh, nk, hd, write_kv, parts, bias);
+    };
+    const bool one = parts == 1;
     if (is_bf16)
-      rope_kvwrite_vec_kernel<bf16, true><<<n_tok, threads, 0, stream>>>(qkv, cs, sn, positions, seq_of_tok, page_table,
-                                                                     pt_stride, (bf16*)q_out, (bf16*)kcache,
-                                                                     (bf16*)vcache, nh, nk, hd, write_kv, parts, bias);
+      run(!few ? rope_kvwrite_vec_kernel<bf16, true> : one ? rope_kvwrite_few_kernel<bf16, true, false> : rope_kvwrite_few_kernel<bf16, true, true>, bf16{});
     else
-      rope_kvwrite_vec_kernel<float, false><<<n_tok, threads, 0, stream>>>(qkv, cs, sn, positions, seq_of_tok,
-                                                                       page_table, pt_stride, (float*)q_out,
-                                                                       (float*)kcache, (float*)vcache, nh, nk, hd,
-                                                                       write_kv, parts, bias);
+      run(!few ? rope_kvwrite_vec_kernel<float, false> : one ? rope_kvwrite_few_kernel<float, false, false> : rope_kvwrite_few_kernel<float, false, true>, 0.f);
     return mf_launch_status();
   }
   if (parts > 1) return (int)hipErrorInvalidValue;        // (the caller asks for parts only where the kernel above runs)
