@@ -35,3 +35,23 @@ def test_shares_fit_the_chip_and_cover_every_page_once(new, start, block, heads,
     for shares in listed.values():
         assert sorted(s for s, _ in shares) == list(range(shares[0][1])) and shares[0][1] <= most <= 8
     assert n_slots == len({w >> 16 for w in words if w})
+
+
+@pytest.mark.parametrize("shorts", [0, 60, 100, 119, 120, 121, 124, 125, 126, 127, 128, 140])
+@pytest.mark.parametrize("heads,long_start", [(4, 30000), (4, 9000), (2, 30000), (3, 120000)])
+def test_the_longest_walk_stays_short_beside_many_short_prompts(shorts, heads, long_start):
+    """A step's time is its longest walk: fitting the workgroups to the chip lengthens it by a quarter at most, however many prompts
+    of one block there are beside a turn on a long context."""
+    new, start = [18] * shorts + [36], [0] * shorts + [long_start]
+    blocks = shorts + 2
+    pages = (long_start + 36 - 1) // 64 + 1
+
+    def longest(got):
+        if got is None:
+            return pages
+        seqs, starts, words, _, _ = (x.tolist() if isinstance(x, torch.Tensor) else x for x in got)
+        return max(-(-((s + min(q + 18, n) - 1) // 64 + 1) // max(1, (w >> 8) & 255))
+                   for b, q, w in zip(seqs, starts, words) for n, s in [(new[b], start[b])])
+    even = longest(step(new, start).shared_query_tiles(18, 64, 0, heads, 256, 2, 4, 8))
+    fitted = longest(step(new, start).shared_query_tiles(18, 64, 0, heads, 256, 2, 4, 8, at_once=True))
+    assert fitted <= 1.25 * even and even <= -(-pages // 8) + 1, (blocks, even, fitted, pages)
