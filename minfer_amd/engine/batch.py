@@ -14,6 +14,9 @@ from typing import Dict, List, Optional
 
 import torch
 
+# Pages that a workgroup could walk in the time it takes to start, to leave its part and to make place for the next one.
+SHARE_START = 4
+
 
 @dataclass
 class StepContext:
@@ -112,7 +115,7 @@ class StepContext:
         share of all pages and as its longest block, and only where the longest block is
         `min_imbalance` times that share is there time to win by cutting it (putting the parts
         together has a price).  `at_once`: shares grow until all workgroups run at once, where the blocks
-        alone do and the longest walk grows by a quarter at most.  Kept per set of arguments: layers with other head counts plan for themselves."""
+        alone do and the last workgroup ends no later for it.  Kept per set of arguments: layers with other head counts plan for themselves."""
         key = ("shared_query_tiles", block, page, window, n_heads, n_cu, per_cu, min_pages, max_shares, min_imbalance, at_once)
         if key not in self._memo:
             tiles = []
@@ -133,12 +136,18 @@ class StepContext:
 
             of_pages = Counter(pages for pages, _, _ in tiles)
 
-            def walk(t):                                     # pages of the longest workgroup
-                return max(-(-pages // shares_of(pages, t)) for pages in of_pages)
-            # (a few workgroups that wait for a place double the time: 604 tokens on up to 5,000 keys, 16 heads on 2, 560
-            # workgroups in 512 places 79 us, 480 of them 65.  But what the step waits for is its longest walk, and blocks that
-            # leave their place almost at once count as much as one of 470 pages: 125 prompts of 18 tokens and 36 tokens on
-            # 30,000 keys, 28 heads on 4, 97 us in shares of 59 pages, 598 with all workgroups at once)
+            def ends(t):                                     # when the last workgroup does, in pages (SHARE_START for starting and leaving)
+                walks = sorted((-(-(pages - s) // shares_of(pages, t)) for pages, c in of_pages.items()
+                                for s in range(shares_of(pages, t)) for _ in range(c)), reverse=True)
+                places = n_cu * per_cu // n_heads            # of each head: the longest start, the others as places become free
+                last = walks[0] + SHARE_START
+                for i, w in enumerate(walks[places:]):
+                    last = max(last, w + walks[max(0, places - 1 - i)] + 2 * SHARE_START)
+                return last
+            # A few workgroups that wait for a place can double the time (28 heads on 4, 611 tokens on 8,000 keys: 544 workgroups in
+            # 512 places 121 us, all at once 96; 16 on 2, 180 + 101 + 168 + 155 on 5,000: 61 and 46).  But blocks that leave their place
+            # almost at once count as much as one of 470 pages: 125 prompts of 18 tokens and 36 tokens on 30,000 keys, 28 heads on 4,
+            # 93 us in shares of 59 pages, 595 with all at once.  So the two are compared by when their last workgroup ends.
             if at_once and len(tiles) * n_heads <= n_cu * per_cu:
                 low, high = target, max(target, longest)     # the least target at which all run at once
                 while low < high:
@@ -147,7 +156,7 @@ class StepContext:
                         low = mid + 1
                     else:
                         high = mid
-                if 4 * walk(low) <= 5 * walk(target):
+                if low > target and ends(low) <= ends(target):
                     target = low
             entries, n_slots, most = [], 0, 1
             for pages, b, q0 in tiles:

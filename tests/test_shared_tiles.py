@@ -1,4 +1,6 @@
 """How blocks of queries of the prompt attention are shared out (host side only)."""
+import heapq
+
 import pytest
 import torch
 
@@ -37,21 +39,35 @@ def test_shares_fit_the_chip_and_cover_every_page_once(new, start, block, heads,
     assert n_slots == len({w >> 16 for w in words if w})
 
 
-@pytest.mark.parametrize("shorts", [0, 60, 100, 119, 120, 121, 124, 125, 126, 127, 128, 140])
-@pytest.mark.parametrize("heads,long_start", [(4, 30000), (4, 9000), (2, 30000), (3, 120000)])
-def test_the_longest_walk_stays_short_beside_many_short_prompts(shorts, heads, long_start):
-    """A step's time is its longest walk: fitting the workgroups to the chip lengthens it by a quarter at most, however many prompts
-    of one block there are beside a turn on a long context."""
-    new, start = [18] * shorts + [36], [0] * shorts + [long_start]
-    blocks = shorts + 2
-    pages = (long_start + 36 - 1) // 64 + 1
+def last_end(new, start, block, heads, places, at_once):
+    """When the last workgroup of a step's plan ends, in pages: each takes the place that is free first, the longest first; four
+    pages' time to start and leave."""
+    got = step(new, start).shared_query_tiles(block, 64, 0, heads, 256, places // 256, 4, 8, at_once=at_once)
+    if got is None:
+        entries = [(b, q, 0) for b, n in enumerate(new) for q in range(0, n, block)]
+    else:
+        entries = list(zip(*(x.tolist() for x in got[:3])))
+    walks = []
+    for b, q, w in entries:
+        pages, shares = (start[b] + min(q + block, new[b]) - 1) // 64 + 1, max(1, (w >> 8) & 255)
+        walks += [(pages - (w & 255) + shares - 1) // shares + 4] * heads
+    free = [0] * places
+    for w in sorted(walks, reverse=True):
+        heapq.heapreplace(free, free[0] + w)
+    return max(free)
 
-    def longest(got):
-        if got is None:
-            return pages
-        seqs, starts, words, _, _ = (x.tolist() if isinstance(x, torch.Tensor) else x for x in got)
-        return max(-(-((s + min(q + 18, n) - 1) // 64 + 1) // max(1, (w >> 8) & 255))
-                   for b, q, w in zip(seqs, starts, words) for n, s in [(new[b], start[b])])
-    even = longest(step(new, start).shared_query_tiles(18, 64, 0, heads, 256, 2, 4, 8))
-    fitted = longest(step(new, start).shared_query_tiles(18, 64, 0, heads, 256, 2, 4, 8, at_once=True))
-    assert fitted <= 1.25 * even and even <= -(-pages // 8) + 1, (blocks, even, fitted, pages)
+
+@pytest.mark.parametrize("shorts", [0, 60, 100, 119, 120, 121, 124, 125, 126, 127, 128, 140])
+@pytest.mark.parametrize("heads,long_new,long_start", [(4, 36, 30000), (4, 36, 9000), (2, 36, 30000), (3, 36, 120000), (4, 611, 8000), (4, 300, 3000)])
+def test_fitting_shares_to_the_chip_costs_no_time(shorts, heads, long_new, long_start):
+    """However many prompts of one block there are beside a turn on a long context, the last workgroup ends no later than by the even
+    share (a tenth for the rounding of walks)."""
+    new, start = [18] * shorts + [long_new], [0] * shorts + [long_start]
+    even, fitted = (last_end(new, start, 18, heads, 512, at_once) for at_once in (False, True))
+    assert fitted <= 1.1 * even
+
+
+def test_fitting_shares_to_the_chip_gains_where_a_few_workgroups_would_wait():
+    new, start = [180, 101, 168, 155], [5000, 4997, 4994, 4991]
+    assert last_end(new, start, 16, 2, 512, True) < 0.75 * last_end(new, start, 16, 2, 512, False)
+    assert last_end([611], [8000], 18, 4, 512, True) < 0.8 * last_end([611], [8000], 18, 4, 512, False)
