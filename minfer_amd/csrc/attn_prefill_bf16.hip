@@ -16,11 +16,11 @@
 // group the pages' way into the CU, not the matrix cores, set the time.)
 // The time of a prompt's attention is that of its last tile, whose block walks every page of the
 // sequence one after the other, so the host may give a tile to several blocks, which take its
-// pages in turn (block s of n the pages first + s, first + s + n, ...): each leaves its maxima,
-// sums and output in `parts`, and a kernel behind this one adds them up, in the order of s, and writes the result.  (A
-// form in which the block that came last added them up read half a megabyte alone: 604 tokens on up to 5,000 keys, 16 heads on
-// 2, 65 us so and 41 + 10
-// in two kernels; 120 tokens on 4,000, 28 heads on 4, 31 and 21 + 7; a prompt of 1,500, 14 heads of 64 on 2, 29 and 14 + 7.)
+// pages in turn (block s of n the pages first + s, first + s + n, ...): each leaves its maxima, sums and output in `parts`, which are
+// added up in the order of s, in one of two ways.  Few parts: each block counts itself in, and the one that comes last adds them
+// (MEET), no second kernel.  Many: that block would read half a megabyte alone, and a kernel behind this one adds them up.
+// (604 tokens on up to 5,000 keys, 16 heads on 2, 8 parts: 65 us so and 41 + 10 in two kernels; a prompt of 300, 14 heads of 64
+// on 2, 2 parts: 10.2 and 12.2.)
 // A page (64 keys) of K and of V travels from the cache straight into LDS (global_load_lds, no
 // registers in between), one or two pages ahead of the one being multiplied, one barrier a
 // page.  LDS holds K as stored, [64 keys][head_dim], and V as stored, transposed in two halves
@@ -31,6 +31,8 @@
 //   O^T[d][row]  += V^T P^T  A = V^T from LDS, B = P^T, which is S^T's own register layout
 // The k index of the second product is permuted the same way on both operands (the sum
 // does not care), which is what lets P stay in registers.
+#include <type_traits>
+
 #include "common.h"
 
 namespace {
@@ -86,13 +88,13 @@ __device__ __forceinline__ int kswz(int row) {
   return S::POW2 ? (row / S::KDIV) & (S::CPR - 1) : 0;
 }
 
-template <int NKS>
+template <int NKS, bool MEET>
 __global__ __launch_bounds__(Shape<NKS>::NW * 64, Shape<NKS>::PER_CU) void attn_prefill_kernel(
     const bf16* __restrict__ q, const bf16* __restrict__ kc, const bf16* __restrict__ vc,
     const int* __restrict__ page_table, int pt_stride, const int* __restrict__ cu_seqlens,
     const int* __restrict__ start_pos, const int* __restrict__ tile_seq,
     const int* __restrict__ tile_q0, const int* __restrict__ tile_share, float* __restrict__ parts,
-    int max_shares, bf16* __restrict__ out, int nh, int nk, int gh, int tq,
+    int* __restrict__ arrived, int max_shares, bf16* __restrict__ out, int nh, int nk, int gh, int tq,
     float scale, int window, int pair_slots) {
   using S = Shape<NKS>;
   constexpr int HD = S::HD, NW = S::NW, NT = NW * 64, NDT = S::NDT, HDP = S::HDP, CPR = S::CPR;
@@ -115,7 +117,7 @@ __global__ __launch_bounds__(Shape<NKS>::NW * 64, Shape<NKS>::PER_CU) void attn_
   const int h0 = hk * G + chunk * gh, ghc = min(gh, G - chunk * gh);      // this block's heads: h0 .. h0 + ghc - 1
   const int b = tile_seq[tile], q0 = tile_q0[tile];
   // tile_share[tile]: which of how many blocks of these queries this one is, and the number of the
-  // queries' slot in `parts`: share + 256 * shares + 65536 * slot (0 shares: alone)
+  // queries' slot in `parts` and `arrived`: share + 256 * shares + 65536 * slot (0 shares: alone)
   const int share_word = tile_share ? tile_share[tile] : 0;
   const int share = share_word & 255, n_shares = max(1, (share_word >> 8) & 255), share_slot = share_word >> 16;
   const int tok0 = cu_seqlens[b], n_new = cu_seqlens[b + 1] - tok0, start = start_pos[b];
@@ -355,7 +357,7 @@ __global__ __launch_bounds__(Shape<NKS>::NW * 64, Shape<NKS>::PER_CU) void attn_
   }
   __syncthreads();            // every wave is past its last read of the pages: LDS is free
 
-  if (n_shares > 1) {         // this block's part, value v of thread t at v * NT + t, for `attn_prefill_merge_kernel`
+  if (!MEET && n_shares > 1) {         // this block's part, value v of thread t at v * NT + t, for `attn_prefill_merge_kernel`
     float* mine = parts + (((size_t)share_slot * ipt + it) * max_shares + share) * XW * NT + tid;
     mine[0] = m_run;
     mine[NT] = l_run;
@@ -364,6 +366,58 @@ __global__ __launch_bounds__(Shape<NKS>::NW * 64, Shape<NKS>::PER_CU) void attn_
 #pragma unroll
       for (int e = 0; e < 16; ++e) mine[(2 + dt * 16 + e) * NT] = oacc[dt][e];
     return;
+  }
+  if (MEET && n_shares > 1) {
+    // This block's part goes to memory (lane-major: value v of thread t at v * NT + t), written
+    // through and read past the caches, since the blocks of a tile may sit behind different L2s.
+    float* slot0 = parts + ((size_t)share_slot * ipt + it) * max_shares * XW * NT + tid;
+    float* mine = slot0 + (size_t)share * XW * NT;
+    __hip_atomic_store(mine, m_run, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(mine + NT, l_run, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+#pragma unroll
+    for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+      for (int e = 0; e < 16; ++e)
+        __hip_atomic_store(mine + (2 + dt * 16 + e) * NT, oacc[dt][e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __builtin_amdgcn_s_waitcnt(0);                       // this wave's stores have reached memory
+    __syncthreads();
+    int* last = reinterpret_cast<int*>(smem);
+    if (tid == 0) {
+      // Counting in releases this block's part and, for the block that arrives last, acquires the
+      // others': the block's stores are ordered before the increment by the barrier above (and are
+      // atomic stores themselves), the increments on one counter form a release sequence, and the
+      // last arriver's loads below are ordered behind its increment by the barrier that follows.
+      int* count = arrived + share_slot * ipt + it;
+      const int before = __hip_atomic_fetch_add(count, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+      if (before == n_shares - 1) __hip_atomic_store(count, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // as it was found
+      *last = before == n_shares - 1;
+    }
+    __syncthreads();
+    const bool is_last = *last != 0;
+    __syncthreads();                                     // the word is in the output staging's place
+    if (!is_last) return;
+    m_run = -INFINITY;
+    l_run = 0.f;
+#pragma unroll
+    for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) oacc[dt][e] = 0.f;
+    for (int s = 0; s < n_shares; ++s) {                 // every part, this block's own too, in the order of s
+      const float* theirs = slot0 + (size_t)s * XW * NT;
+      const float m_o = __hip_atomic_load(theirs, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      const float l_o = __hip_atomic_load(theirs + NT, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      const float m_new = fmaxf(m_run, m_o);
+      const float c_mine = (m_run == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(m_run - m_new);
+      const float c_theirs = (m_o == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(m_o - m_new);
+      l_run = l_run * c_mine + l_o * c_theirs;
+#pragma unroll
+      for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+          oacc[dt][e] = oacc[dt][e] * c_mine +
+                        __hip_atomic_load(theirs + (2 + dt * 16 + e) * NT, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) * c_theirs;
+      m_run = m_new;
+    }
   }
   // normalise; O^T regs: d = 32 dt + 8 (e / 4) + 4 hf + e % 4 for this lane's row
   const float l_tot = l_run + __shfl_xor(l_run, 32, MF_WAVE);
@@ -446,18 +500,10 @@ __global__ __launch_bounds__(Shape<NKS>::NW * 64) void attn_prefill_merge_kernel
 template <int NKS>
 int launch(const bf16* q, const bf16* kc, const bf16* vc, const int* page_table, int pt_stride,
            const int* cu_seqlens, const int* start_pos, const int* tile_seq, const int* tile_q0,
-           const int* tile_share, float* parts, int max_shares, bf16* out, int n_tiles, int nh, int nk,
+           const int* tile_share, float* parts, int* arrived, int max_shares, bf16* out, int n_tiles, int nh, int nk,
            int gh, int tq, float scale, int window, hipStream_t stream) {
   using S = Shape<NKS>;
   if (gh * tq > S::ROWS) return (int)hipErrorInvalidValue;
-  static bool configured = false;
-  auto kern = attn_prefill_kernel<NKS>;
-  if (!configured) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, S::SMEM);
-    if (e != hipSuccess) return (int)e;
-    configured = true;
-  }
   static int n_cu = 0;                 // compute units of the device (asked once)
   if (n_cu == 0) {
     int dev = 0;
@@ -466,11 +512,21 @@ int launch(const bf16* q, const bf16* kc, const bf16* vc, const int* page_table,
     n_cu = prop.multiProcessorCount;
   }
   const int G = nh / nk, ipt = nk * ((G + gh - 1) / gh);
-  kern<<<n_tiles * ipt, S::NW * 64, S::SMEM, stream>>>(q, kc, vc, page_table, pt_stride, cu_seqlens, start_pos, tile_seq,
-                                                       tile_q0, tile_share, parts, max_shares, out, nh, nk, gh, tq, scale,
-                                                       window, S::PER_CU == 2 && !tile_share ? n_cu : 0);
-  const int rc = mf_launch_status();
-  if (rc || !tile_share) return rc;
+  auto run = [&](auto MEET) {
+    static bool configured = false;
+    auto kern = attn_prefill_kernel<NKS, decltype(MEET)::value>;
+    if (!configured) {
+      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, S::SMEM);
+      if (e != hipSuccess) return (int)e;
+      configured = true;
+    }
+    kern<<<n_tiles * ipt, S::NW * 64, S::SMEM, stream>>>(q, kc, vc, page_table, pt_stride, cu_seqlens, start_pos, tile_seq,
+                                                         tile_q0, tile_share, parts, arrived, max_shares, out, nh, nk, gh, tq, scale,
+                                                         window, S::PER_CU == 2 && !tile_share ? n_cu : 0);
+    return mf_launch_status();
+  };
+  if (!tile_share || arrived) return run(std::true_type{});
+  if (const int rc = run(std::false_type{})) return rc;
   attn_prefill_merge_kernel<NKS><<<dim3(n_tiles * ipt, S::NDT), S::NW * 64, 0, stream>>>(parts, cu_seqlens, tile_seq, tile_q0, tile_share,
                                                                                         max_shares, out, nh, nk, gh, tq);
   return mf_launch_status();
@@ -491,8 +547,9 @@ MF_API int mf_attn_prefill_per_cu(int hd) { return hd <= 128 ? 2 : 1; }
 // its group.  tile_share (or null: every workgroup has its rows to itself): entry i is share + 256 *
 // shares + 65536 * slot, workgroup `share` of `shares` (at most max_shares, which is at most 255)
 // that take the pages of these queries in turn; their parts meet in
-// parts[slot][workgroup of the block][max_shares][mf_attn_prefill_part_floats(hd)], and a second kernel adds them up.  Calls
-// that use the same parts run on one stream.
+// parts[slot][workgroup of the block][max_shares][mf_attn_prefill_part_floats(hd)], and where `arrived` is given in
+// arrived[slot][workgroup of the block], which is zero before the call and after it: the workgroup that comes last adds them up.
+// Without `arrived` a second kernel does.  Calls that use the same parts and arrived run on one stream.
 MF_API int mf_attn_prefill_part_floats(int hd) {
   return (((hd / 16 + 1) / 2) * 16 + 2) * 256;
 }
@@ -500,7 +557,7 @@ MF_API int mf_attn_prefill_part_floats(int hd) {
 MF_API int mf_attn_prefill_bf16(const void* q, const void* kc, const void* vc, const int* page_table,
                                 int pt_stride, const int* cu_seqlens, const int* start_pos,
                                 const int* tile_seq, const int* tile_q0, const int* tile_share, float* parts,
-                                int max_shares, void* out, int n_tiles, int nh, int nk, int hd,
+                                int* arrived, int max_shares, void* out, int n_tiles, int nh, int nk, int hd,
                                 int gh, int tq, float scale, int window, hipStream_t stream) {
   if (n_tiles <= 0) return 0;
   if (hd % 16 != 0 || hd < 16 || hd > 256 || nk <= 0 || nh % nk != 0) return (int)hipErrorInvalidValue;
@@ -509,7 +566,7 @@ MF_API int mf_attn_prefill_bf16(const void* q, const void* kc, const void* vc, c
 #define MF_CASE(E)                                                                                        \
   case E:                                                                                                 \
     return launch<E>((const bf16*)q, (const bf16*)kc, (const bf16*)vc, page_table, pt_stride, cu_seqlens, \
-                     start_pos, tile_seq, tile_q0, tile_share, parts, max_shares, (bf16*)out, n_tiles, nh, \
+                     start_pos, tile_seq, tile_q0, tile_share, parts, arrived, max_shares, (bf16*)out, n_tiles, nh, \
                      nk, gh, tq, scale, window, stream);
   switch (hd / 16) {
     MF_CASE(1) MF_CASE(2) MF_CASE(3) MF_CASE(4) MF_CASE(5) MF_CASE(6) MF_CASE(7) MF_CASE(8)

@@ -167,7 +167,7 @@ _PROTOTYPES = {
                                      c_int, c_float, c_int, c_int, c_int, c_int, _P],
     },
     "attn_prefill_bf16": {
-        "mf_attn_prefill_bf16": [_P, _P, _P, _P, c_int, _P, _P, _P, _P, _P, _P, c_int, _P, c_int, c_int, c_int,
+        "mf_attn_prefill_bf16": [_P, _P, _P, _P, c_int, _P, _P, _P, _P, _P, _P, _P, c_int, _P, c_int, c_int, c_int,
                                  c_int, c_int, c_int, c_float, c_int, _P],
         "mf_attn_prefill_part_floats": [c_int],
         "mf_attn_prefill_rows": [c_int],
@@ -2377,6 +2377,18 @@ def prefill_tile(n_heads: int, n_kv_heads: int, head_dim: int):
     return rows // gh, gh, n_kv_heads * (-(-group // gh))
 
 
+def prefill_parts_meet(head_dim: int, most_shares: int, shared: int, workgroups: int, n_cu: int) -> bool:
+    """Whether the parts of shared blocks (`shared` of them, heads counted; `workgroups` in all) are added up by the workgroup that
+    comes last, which saves a second kernel and reads its parts alone.  That is level to a fifth faster with two parts a block, or
+    with up to four where there are enough blocks to fill the second kernel, as long as every workgroup has a CU to itself
+    (microseconds so / with a second kernel: 300 tokens, 14 heads of 64 on 2, 2 parts 10.2 / 12.2; 1,000 with a window of 256, 16 of
+    128 on 2, 2 parts 18.0 / 20.8; 611 on 200 keys, 4 parts 20.1 / 21.9; otherwise: 60 tokens on 500 keys, 40 heads of 128 on 8, 3
+    parts of few blocks 15.3 / 13.2; 1,000 tokens, 28 heads on 4, 560 workgroups 36.0 / 28.7; heads of 256: 1.1 to 10 times slower)."""
+    if head_dim > 128 or workgroups > n_cu:
+        return False
+    return most_shares == 2 or (most_shares <= 4 and 8 * shared >= n_cu and 5 * workgroups <= 18 * shared)
+
+
 def attn_prefill(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor, page_table: torch.Tensor,
                  ctx, out: torch.Tensor, n_heads: int, n_kv_heads: int, head_dim: int, scale: float,
                  window: int) -> None:
@@ -2410,16 +2422,22 @@ def attn_prefill(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor, pa
         tq, PAGE, window, per_tile, cu_count(), per_cu, PREFILL_MIN_PAGES, PREFILL_MAX_SHARES, at_once=True)
     if shared is None:
         tile_seq, tile_q0 = ctx.query_tiles(tq)
-        tile_share = parts = None
+        tile_share = parts = arrived = None
     else:
         tile_seq, tile_q0, tile_share, n_slots, most_shares = shared
         part = _fn("attn_prefill_bf16", "mf_attn_prefill_part_floats")(head_dim)
         parts = workspace("prefill_parts", n_slots * per_tile * most_shares * part, q.device)
-    _check(_fn("attn_prefill_bf16", "mf_attn_prefill_bf16")(
+        arrived = None
+        if prefill_parts_meet(head_dim, most_shares, n_slots * per_tile, tile_seq.numel() * per_tile, cu_count()):
+            arrived = _zeroed_counters("prefill_arrived", n_slots * per_tile, q.device)
+    rc = _fn("attn_prefill_bf16", "mf_attn_prefill_bf16")(
         q, kcache, vcache, page_table, page_table.shape[1], ctx.cu_seqlens,
-        ctx.start_pos, tile_seq, tile_q0, tile_share, parts,
+        ctx.start_pos, tile_seq, tile_q0, tile_share, parts, arrived,
         most_shares if shared is not None else 1, out, tile_seq.numel(), n_heads, n_kv_heads, head_dim,
-        gh, tq, float(scale), window, _stream()), "attn_prefill_bf16")
+        gh, tq, float(scale), window, _stream())
+    if rc != 0 and arrived is not None:
+        arrived.zero_()                  # a launch that failed may have left workgroups counted in
+    _check(rc, "attn_prefill_bf16")
 
 
 # ------------------------------------------------------------------ sampling

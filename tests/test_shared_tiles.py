@@ -71,3 +71,10 @@ def test_fitting_shares_to_the_chip_gains_where_a_few_workgroups_would_wait():
     new, start = [180, 101, 168, 155], [5000, 4997, 4994, 4991]
     assert last_end(new, start, 16, 2, 512, True) < 0.75 * last_end(new, start, 16, 2, 512, False)
     assert last_end([611], [8000], 18, 4, 512, True) < 0.8 * last_end([611], [8000], 18, 4, 512, False)
+
+def test_how_parts_are_added_up():
+    """The last workgroup of a block adds its parts where they are few and every workgroup has a CU; heads beyond 128 never."""
+    from minfer_amd.kernels.ops import prefill_parts_meet as meet
+    assert meet(64, 2, 6, 40, 256) and meet(128, 2, 126, 252, 256) and not meet(128, 2, 168, 360, 256)
+    assert meet(128, 4, 72, 198, 256) and not meet(128, 3, 8, 24, 256) and not meet(128, 4, 48, 192, 256)
+    assert not meet(128, 8, 32, 200, 256) and not meet(144, 2, 6, 40, 256) and not meet(256, 2, 6, 12, 256)
