@@ -2511,8 +2511,10 @@ int launch_reduce_norm(const float* part, const float* bias, float* C, int ldc, 
   };
   // Where no CU has two rows, a row's loads should all be on their way at once: 203 rows of 3,584 in 9 parts 9.9 us with 256
   // threads a row, 7.5 with 1,024.  With more rows the blocks of a CU do that for each other: 604 rows of 2,048 in 6 parts 8.1
-  // and 8.5, 2,048 rows of 3,584 in 2 23.4 and 25.0.
-  if (M <= cu_count()) with(std::integral_constant<int, 1024>{});
+  // and 8.5, 2,048 rows of 3,584 in 2 23.4 and 25.0; and of at most 1,024 values 256 threads ask for all at once as well (65 rows of
+  // 896 with their product 9.4 us and 9.9).  1,024 threads hold the row in LDS, which a launch gives 64 KB of without being asked.
+  const bool fits = N * sizeof(float) + 1024 / 64 * sizeof(float) <= 64 * 1024;
+  if (M <= cu_count() && N > 1024 && fits) with(std::integral_constant<int, 1024>{});
   else with(std::integral_constant<int, 256>{});
   return mf_launch_status();
 }
