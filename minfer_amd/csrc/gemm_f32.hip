@@ -407,7 +407,7 @@ bool rows_take(int M, int N, int K) {
 // How many parts K is cut into (1: none): `mf_gemm_f32` with more than one needs part [parts][M][N].
 // `aligned`: 16-byte aligned operands with row strides in multiples of 4.
 MF_API int mf_gemm_f32_splits(int M, int N, int K, int aligned, int n_cu) {
-  if (M <= 8 || N <= 0 || !aligned || K % T_BK || (size_t)M * K * 4 >= (1ull << 32) || (size_t)N * K * 4 >= (1ull << 32)) return 1;
+  if (M <= 8 || N <= 0 || K < T_BK || n_cu <= 0 || !aligned || K % T_BK || (size_t)M * K * 4 >= (1ull << 32) || (size_t)N * K * 4 >= (1ull << 32)) return 1;
   return tile_splits(M, N, K, n_cu);
 }
 
