@@ -257,10 +257,12 @@ __global__ __launch_bounds__(256) void add_parts_f32_kernel(const float* __restr
   *c = ACCUMULATE ? *c + v : v;
 }
 
-// How many blocks share a tile's K.  The chip's time is that of the CU with the most tiles, times their k tiles (and some three
-// more a tile for its start), at 0.43 us a k tile where three or more share a CU and somewhat more where two or one do; the
+// How many blocks share a tile's K.  The chip's time is that of the CU with the most tiles, times their k tiles (and some four
+// more a tile for its start), at 0.46 us a k tile where three or more share a CU and somewhat more where two or one do; the
 // parts' way to memory and back and the second kernel come on top.  (611 rows against 896 of 4,864, 140 tiles: 4 parts, 560 on
-// 256 CUs, 71 us; 5 parts 60.5.)
+// 256 CUs, 71 us; 5 parts 54.  The constants are those with the least loss over 233 shapes of 9 to 4,000 rows timed at up to 11
+// numbers of parts each: 6 % above the best of each on the average, and nowhere more than 3 % above cutting in parts of 256 until
+// every CU has two tiles.)
 int tile_splits(int M, int N, int K, int n_cu) {
   const long tiles = (long)((M + T_BM - 1) / T_BM) * ((N + T_BM - 1) / T_BM), nkt = K / T_BK;
   long best = 1;
@@ -268,9 +270,9 @@ int tile_splits(int M, int N, int K, int n_cu) {
   for (long parts = 1; parts <= std::min<long>(std::max<long>(1, nkt / 7), 16); ++parts) {
     const long per = (nkt + parts - 1) / parts, most = (tiles * parts + n_cu - 1) / n_cu;
     if ((nkt + per - 1) / per != parts) continue;
-    const double step_us = most >= 3 ? 0.43 : most == 2 ? 0.54 : 0.75;
-    const double us = (double)(most * (per + 3)) * step_us + (parts > 1 ? 4. + (double)(parts + 1) * M * N * 4. / 3e6 : 0.);
-    if (us < best_us * 0.95) {
+    const double step_us = most >= 3 ? 0.46 : most == 2 ? 0.54 : 0.7;
+    const double us = (double)(most * (per + 4)) * step_us + (parts > 1 ? 3. + (double)(parts + 1) * M * N * 4. / 3.5e6 : 0.);
+    if (us < best_us) {
       best_us = us;
       best = parts;
     }
@@ -278,10 +280,10 @@ int tile_splits(int M, int N, int K, int n_cu) {
   return (int)best;
 }
 
-// An eighth of the tiles an XCD, each with an L2 of 4 MB: whole products whose activations stay in it beside the weights (each
-// XCD then reads an eighth of these: 611 rows against 9,728 of 896 109 us and 104, 400 against 17,920 of 1,536 219 and 202; 2,000 against 9,728
-// of 896 274 and 284), and parts of
-// activations that would not (an XCD then reads a part or two: 400 x 1,536 x 8,960 119 us and 112; 611 x 1,152 x 896 24 and 25).
+// An eighth of the tiles an XCD, each with an L2 of 4 MB: whole products whose activations stay in it beside the weights (each XCD
+// then reads an eighth of these: 611 rows against 9,728 of 896 109 us and 104, 400 against 17,920 of 1,536 219 and 202; 2,000
+// against 9,728 of 896 274 and 284), and parts of activations that would not (an XCD then reads a part or two: 400 x 1,536 x
+// 8,960 119 us and 112; 611 x 1,152 x 896 24 and 25).
 int tiles_by_xcd(int M, int K, int splits) {
   const size_t bytes = (size_t)M * K * 4;
   return splits > 1 ? bytes > (4u << 20) : bytes <= (3u << 20);
