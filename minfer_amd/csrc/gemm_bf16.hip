@@ -2078,8 +2078,9 @@ __global__ __launch_bounds__(512) void panel_kernel(const bf16* __restrict__ A, 
 // a block meet in LDS, where gates and ups of a SwiGLU pair up whichever waves held them.
 // TURNS: the two waves of a SIMD in turns, one reading a k tile's fragments while the other multiplies (one group of waves a half
 // k tile behind the other); without, all read and all multiply.
+// PAIR: SwiGLU, in a kernel of its own: every block runs its epilogue once, so what it takes is also the fetch of its code.
 // SwiGLU of 37,888 x 3,584: 64 rows 50.8 us (5.3 TB/s of weights; `panel_kernel` 58.7), 100 rows 55.6 (tiles of 128 x 256 66.7),
-// without TURNS 2 us more.
+// without TURNS 2 us more.  33,000 x 512, bfloat16 results, 128 rows: 17.8 us with 2-byte stores, 15.7 with 8-byte ones.
 template <int I, int J, int RA, int STAGES>
 struct PanelTile {
   static constexpr int WM = 4, WN = 2, BN = 32 * J, P = (RA + BN) / 8, L = (P + 7) / 8, ST = (RA + BN) * DMA_BK * 2, OLD = BN + 4;
@@ -2087,7 +2088,7 @@ struct PanelTile {
   static_assert(RA <= 16 * I * WM && RA % 8 == 0 && LDS <= 160 * 1024, "the rows fit the waves, the stages LDS");
 };
 
-template <int I, int J, int RA, int STAGES, bool TURNS>
+template <int I, int J, int RA, int STAGES, bool TURNS, bool PAIR>
 __global__ __launch_bounds__(512, 2) void panel_dma_kernel(const bf16* __restrict__ A, int lda, const bf16* __restrict__ W, int ldw,
                                                            const float* __restrict__ bias, void* __restrict__ C, int ldc, int M, int N,
                                                            int K, int epi, const float* __restrict__ in_ssq, int in_parts, float in_eps) {
@@ -2101,12 +2102,11 @@ __global__ __launch_bounds__(512, 2) void panel_dma_kernel(const bf16* __restric
   }
   const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = wid % WM, wn = wid / WM, fr = lane & 15, fk = lane >> 4;
-  const bool pair = epi == EPI_SWIGLU;
   // the block's weight rows: units u0 .. u0 + J - 1 of 32; of a pair (16 gate rows and the 16 up rows of the same outputs) the gates
   // of all units first, then the ups
   const int u0 = at * J;
   auto weight_row = [&](int r) {
-    if (!pair) return u0 * 32 + r;
+    if (!PAIR) return u0 * 32 + r;
     const int c = r >> 4, u = u0 + c % J;
     return (u >> 1) * 64 + (u & 1) * 16 + (c / J) * 32 + (r & 15);
   };
@@ -2227,7 +2227,7 @@ __global__ __launch_bounds__(512, 2) void panel_dma_kernel(const bf16* __restric
         *reinterpret_cast<float4*>(out + ((wm * I + i) * 16 + fr) * T::OLD + (wn * J + j) * 16 + fk * 4) = float4{v[0], v[1], v[2], v[3]};
       }
   __syncthreads();
-  if (pair) {
+  if constexpr (PAIR) {
     const bool vec = ldc % 4 == 0 && (uintptr_t)C % 8 == 0;
     auto gated = [&](auto act) {
       for (int x = threadIdx.x; x < M * 4 * J; x += 512) {
@@ -2251,7 +2251,8 @@ __global__ __launch_bounds__(512, 2) void panel_dma_kernel(const bf16* __restric
     }
     return;
   }
-  const bool vec = epi != EPI_BF16 && epi != EPI_XIELU && ldc % 4 == 0 && (uintptr_t)C % 16 == 0;
+  const bool half = epi == EPI_BF16 || epi == EPI_XIELU;
+  const bool vec = ldc % 4 == 0 && (uintptr_t)C % (half ? 8 : 16) == 0;
   for (int x = threadIdx.x; x < M * (BN / 4); x += 512) {
     const int r = x / (BN / 4), c = (x % (BN / 4)) * 4, n = u0 * 32 + c;
     if (n >= N) continue;
@@ -2259,7 +2260,12 @@ __global__ __launch_bounds__(512, 2) void panel_dma_kernel(const bf16* __restric
     float v[4] = {v4.x, v4.y, v4.z, v4.w};
 #pragma unroll
     for (int e = 0; e < 4; ++e) v[e] = v[e] * fac[r] + (bias && n + e < N ? bias[n + e] : 0.f);
-    if (vec && n + 4 <= N) {
+    if (vec && n + 4 <= N && half) {
+      bf16x4 h;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) h[e] = (bf16)(epi == EPI_XIELU ? xielu_f(v[e], bias[N], bias[N + 1]) : v[e]);
+      *reinterpret_cast<bf16x4*>((bf16*)C + (size_t)r * ldc + n) = h;
+    } else if (vec && n + 4 <= N) {
       float4* o = reinterpret_cast<float4*>((float*)C + (size_t)r * ldc + n);
       float4 old = epi == EPI_ACC_F32 ? *o : float4{0.f, 0.f, 0.f, 0.f};
       *o = float4{old.x + v[0], old.y + v[1], old.z + v[2], old.w + v[3]};
@@ -2275,15 +2281,18 @@ template <int I, int J, int RA, int STAGES, bool TURNS>
 int launch_panel_dma(const bf16* A, int lda, const bf16* W, int ldw, const float* bias, void* C, int ldc, int M, int N, int K, int epi,
                      const FusedNorm& fused, hipStream_t stream) {
   using T = PanelTile<I, J, RA, STAGES>;
-  auto kern = panel_dma_kernel<I, J, RA, STAGES, TURNS>;
-  static bool configured = false;
-  if (!configured) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, T::LDS);
-    if (e != hipSuccess) return (int)e;
-    configured = true;
-  }
-  kern<<<((N + 31) / 32 + J - 1) / J, 512, T::LDS, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi, fused.in_ssq, fused.in_parts, fused.in_eps);
-  return mf_launch_status();
+  auto run = [&](auto PAIR) {
+    auto kern = panel_dma_kernel<I, J, RA, STAGES, TURNS, decltype(PAIR)::value>;
+    static bool configured = false;
+    if (!configured) {
+      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, T::LDS);
+      if (e != hipSuccess) return (int)e;
+      configured = true;
+    }
+    kern<<<((N + 31) / 32 + J - 1) / J, 512, T::LDS, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi, fused.in_ssq, fused.in_parts, fused.in_eps);
+    return mf_launch_status();
+  };
+  return epi == EPI_SWIGLU ? run(std::true_type{}) : run(std::false_type{});
 }
 
 // The parts of a split are added in rounds of up to eight, a round's loads in flight together, in

@@ -83,3 +83,23 @@ def test_which_products_take_it():
     for m, n, k in ((129, 37888, 3584), (100, 32768, 2048), (100, 41024, 2048), (50, 22016, 2048), (64, 16384, 1536), (64, 9728, 896)):
         assert name(m, n, k, swiglu=True) != "panel_dma_kernel"
     assert name(64, 22016, 2048) != "panel_dma_kernel" and name(100, 37888, 3584, aligned=False) != "panel_dma_kernel"
+
+
+@pytest.mark.parametrize("m", [17, 65, 128])
+@pytest.mark.parametrize("which,at", [(0, 0), (1, 0), (2, 0), (2, 1), (2, 4)])
+def test_bf16_results_are_the_32_bit_ones_rounded(wide, m, which, at):
+    """Rows of results that four values do and do not divide, from an address that 8 bytes do and do not; plain and through xIELU."""
+    from minfer_amd.kernels import ops
+    n, k = wide[which], 192
+    x, w, b = operands(m, n, k, m + n)
+    out = torch.empty((m, n), device=DEV)
+    ops.linear(x, w, b, out, variant=17)
+    flat = torch.empty(m * n + at, dtype=torch.bfloat16, device=DEV)
+    half = flat[at:].view(m, n)
+    ops.linear(x, w, b, half, variant=17)
+    assert torch.equal(half, out.to(torch.bfloat16))
+    a_pos, a_neg = 0.8, 0.3
+    ops.linear(x, w, torch.cat([b, torch.tensor([a_pos, a_neg], device=DEV)]), half, xielu=True, variant=17)
+    want = torch.empty((m, n), dtype=torch.bfloat16, device=DEV)
+    ops.xielu(out, want, a_pos, a_neg)
+    assert torch.equal(half, want)
