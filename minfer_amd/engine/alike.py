@@ -5,11 +5,18 @@ the device.  Within a step the launches of one layer are recorded as they are ma
 alike (the same parts with the same constants, tensors of the same types and shapes: `Block.alike`) they are made again from
 native code with the layer's own tensors in their places (35 us).  Nothing outlives the step, and a layer that is not alike, or
 a step whose launches are timed one by one, takes the general path.
+
+What a recorded layer launched with stays allocated together until its record is dropped (the 7B shape: some 85 KB a token, where
+52 are live at once in the general path).  So only steps of up to MOST_VALUES values in the stream are recorded (585 tokens of the
+7B shape, 50 MB; 2,340 of the 0.5B one), beyond which the device takes longer for a layer than the host does without a record, and
+the record is dropped before the last block and the head.
 """
 from __future__ import annotations
 
 from ..kernels import ops
 from ..parts.base import NormAhead
+
+MOST_VALUES = 1 << 21
 
 
 def _pair(ahead):

@@ -18,7 +18,7 @@ from ..parts.base import (BLOCKS, COMBINERS, EMBEDDING_ENTRY, EMBEDDINGS, FEED_F
                           normed_input)
 from ..parts.spec import BlockSpec, ModelSpec
 from ..weights.loader import TensorSpec
-from .alike import AlikeLayers
+from .alike import MOST_VALUES, AlikeLayers
 
 
 def _build_block(bs: BlockSpec, rt: Runtime):
@@ -158,7 +158,8 @@ class DecoderModel:
         rows = ctx.logit_rows
         last = len(s.schedule) - 1
         ctx.norm_ahead = None
-        alike = AlikeLayers() if self.rt.device.type == "cuda" and not ctx.all_decode else None      # (decode steps run captured)
+        # (decode steps run captured)
+        alike = AlikeLayers() if self.rt.device.type == "cuda" and not ctx.all_decode and h.numel() <= MOST_VALUES else None
         for n, e in enumerate(s.schedule):
             keep = rows if (n == last and rows is not None) else None
             ctx.kept_rows = keep                 # which of the step's tokens the block's feed-forward sees
@@ -172,11 +173,12 @@ class DecoderModel:
             if alike is not None and keep is None:
                 h = alike.forward(self.blocks[e.block], h, ctx, e.cache, e.writes_cache)
             else:
+                alike = None                     # (it holds a layer's scratch, and the last one's is freed as it goes)
                 h = self.blocks[e.block].forward(h, ctx, e.cache, e.writes_cache, keep_rows=keep)
             ahead = ctx.norm_ahead
             if ahead is not None and (ahead.norm is not ctx.norm_after_block or ahead.h is not h):
                 ctx.norm_ahead = None            # prepared for someone who will not come
-        ctx.norm_after_block = None
+        ctx.norm_after_block = alike = None
         if not s.schedule and rows is not None:
             kept = torch.empty((rows.numel(), s.hidden_size), dtype=torch.float32, device=h.device)
             ops.gather_rows(h, rows, kept)

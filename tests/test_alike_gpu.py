@@ -85,6 +85,53 @@ def test_layers_that_are_not_alike(monkeypatch):
     assert 0 < few <= 8 and all(torch.equal(a, b) for a, b in zip(got, want))
 
 
+def test_only_short_steps_are_recorded(monkeypatch):
+    """A record holds all scratch of its layer: long steps have none."""
+    from minfer_amd import Engine
+    from minfer_amd.engine import alike
+    from minfer_amd.kernels import ops
+    model = build(WIDE, torch.bfloat16)
+    eng = Engine(model, max_tokens=8192, max_seqs=2)
+    made, record = [], ops.record_launches
+    monkeypatch.setattr(ops, "record_launches", lambda: (made.append(1), record())[1])
+    most = alike.MOST_VALUES // WIDE["hidden_size"]
+    for n, recorded in ((most, True), (most + 1, False)):
+        slots = [eng.new_sequence(), eng.new_sequence()]
+        eng.step(slots, [random_tokens(600, n - 1000, n), random_tokens(600, 1000, n)], "last")
+        assert bool(made) == recorded
+        made.clear()
+        for slot in slots:
+            eng.end_sequence(slot)
+
+
+def test_the_record_is_gone_before_the_last_block(monkeypatch):
+    """As much memory is allocated when the last block begins, and at most as much when the head does, as layer by layer."""
+    from minfer_amd import Engine
+    from minfer_amd.engine import alike
+    model = build(WIDE, torch.bfloat16)
+    eng = Engine(model, max_tokens=4096, max_seqs=2)
+    last, head, seen = model.blocks[-1].forward, model.head.forward, []
+
+    def at(fn):
+        def call(*args, **kw):
+            seen.append(torch.cuda.memory_allocated())
+            return fn(*args, **kw)
+        return call
+    monkeypatch.setattr(model.blocks[-1], "forward", at(last))
+    monkeypatch.setattr(model.head, "forward", at(head))
+    got = []
+    for general in (False, True, False, True):                  # (the first two settle what is kept between steps)
+        with monkeypatch.context() as m:
+            if general:
+                m.setattr(alike.AlikeLayers, "forward", lambda self, block, h, ctx, e, w: block.forward(h, ctx, e, w))
+            slot = eng.new_sequence()
+            seen.clear()
+            eng.step([slot], [random_tokens(600, 900, 1)], "last")
+            got.append(tuple(seen))
+            eng.end_sequence(slot)
+    assert len(got[2]) == 2 and got[2] == got[3]
+
+
 def test_a_launch_that_fails_is_told(monkeypatch):
     """A recorded launch's error code ends the step with the kernels' error."""
     from minfer_amd.kernels import ops
