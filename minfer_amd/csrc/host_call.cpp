@@ -6,12 +6,15 @@
 //                                           them) and shape; anything else goes to the function given to `otherwise`, which
 //                                           names what is wrong
 //   Launch(address, kinds)(...)             calls the C function at `address`; kinds, a letter an argument: p pointer (a tensor:
-//                                           its data; None; a number; an object with a buffer: that), i int, q 64 bits, f float,
-//                                           d double.  Returns its int.  The call runs without the interpreter's lock.
+//                                           its data; None; a number; a ctypes array: its place; a ctypes pointer: its value),
+//                                           i int, q 64 bits, f float, d double.  Returns its int.  The call runs without the
+//                                           interpreter's lock.
 //   Record()                                the launches that a thread makes between `with record:` and its end (those of Launches
 //                                           whose `recorded` is set and that returned 0), to be made again with other tensors
 //                                           in some places: `bind(olds)`, then `run(news)` for each set.  It holds the objects
-//                                           that the launches were given, so their memory stays theirs.
+//                                           that the launches were given, so their memory stays theirs.  A pointer is replaced
+//                                           where it is a tensor's first address; a launch that was given a number as a pointer
+//                                           (other than its last, the stream) may have an address inside one, and does not bind.
 #include <Python.h>
 #include <stdint.h>
 #include <string.h>
@@ -36,6 +39,7 @@ struct Call {
   uint64_t w[MAX_INT];
   double f[MAX_FP];
   uint64_t pointers;                                 // bit i: w[i] is one
+  bool numbers;                                      // one of them, not the last argument, came as a number
 };
 struct Place { int call, word, tensor; };
 struct Recorded {
@@ -72,6 +76,37 @@ PyObject* wrong_kind(const char* what, Py_ssize_t at, PyObject* got) {
   return nullptr;
 }
 
+PyObject *g_array = nullptr, *g_pointer = nullptr;   // ctypes.Array and ctypes.c_void_p
+
+// The address that a ctypes array lies at or a ctypes pointer holds; false (and no error): it is neither.  Nothing else with a
+// buffer is taken: the array of a numerical library is host memory, which no kernel may be given by mistake.  The caller holds
+// the object, and with it the memory.
+bool ctypes_address(PyObject* a, uint64_t& address) {
+  const int array = PyObject_IsInstance(a, g_array), pointer = array == 0 ? PyObject_IsInstance(a, g_pointer) : 0;
+  Py_buffer b;
+  if ((array <= 0 && pointer <= 0) || PyObject_GetBuffer(a, &b, PyBUF_SIMPLE) != 0) {
+    PyErr_Clear();
+    return false;
+  }
+  if (array > 0) address = reinterpret_cast<uint64_t>(b.buf);
+  else memcpy(&address, b.buf, sizeof address);
+  PyBuffer_Release(&b);
+  return true;
+}
+
+// a whole number, or what says which one it is (`__index__`); false: neither, with the error set
+bool whole(PyObject* a, Py_ssize_t at, uint64_t& v) {
+  PyObject* n = PyNumber_Index(a);
+  if (!n) {
+    PyErr_Clear();
+    wrong_kind("int", at, a);
+    return false;
+  }
+  v = PyLong_AsUnsignedLongLongMask(n);
+  Py_DECREF(n);
+  return true;
+}
+
 PyObject* launch_call(PyObject* self, PyObject* const* args, size_t nargsf, PyObject* kwnames) {
   Launch* l = reinterpret_cast<Launch*>(self);
   const Py_ssize_t n = PyVectorcall_NARGS(nargsf);
@@ -82,6 +117,7 @@ PyObject* launch_call(PyObject* self, PyObject* const* args, size_t nargsf, PyOb
   uint64_t w[MAX_INT] = {};
   double f[MAX_FP] = {};
   uint64_t pointers = 0;
+  bool numbers = false;
   int nw = 0, nf = 0;
   for (Py_ssize_t i = 0; i < n; ++i) {
     PyObject* a = args[i];
@@ -98,24 +134,21 @@ PyObject* launch_call(PyObject* self, PyObject* const* args, size_t nargsf, PyOb
             return nullptr;
           }
         } else if (PyLong_Check(a)) {
-          w[nw++] = PyLong_AsUnsignedLongLongMask(a);
+          w[nw] = PyLong_AsUnsignedLongLongMask(a);
+          numbers |= w[nw++] != 0 && i + 1 < n;
+        } else if (ctypes_address(a, w[nw])) {
+          ++nw;
         } else {
-          Py_buffer b;                               // the caller holds the object, and with it the memory
-          if (PyObject_GetBuffer(a, &b, PyBUF_SIMPLE) != 0) {
-            PyErr_Clear();
-            return wrong_kind("a tensor, a number, None or a buffer", i, a);
-          }
-          w[nw++] = reinterpret_cast<uint64_t>(b.buf);
-          PyBuffer_Release(&b);
+          return wrong_kind("a tensor, a number, None or a ctypes array or pointer", i, a);
         }
         break;
       case 'i':
-        if (!PyLong_Check(a)) return wrong_kind("int", i, a);
-        w[nw++] = static_cast<uint32_t>(PyLong_AsUnsignedLongMask(a));
+        if (!whole(a, i, w[nw])) return nullptr;
+        w[nw] = static_cast<uint32_t>(w[nw]);
+        ++nw;
         break;
       case 'q':
-        if (!PyLong_Check(a)) return wrong_kind("int", i, a);
-        w[nw++] = PyLong_AsUnsignedLongLongMask(a);
+        if (!whole(a, i, w[nw++])) return nullptr;
         break;
       default: {
         const double v = PyFloat_AsDouble(a);
@@ -141,6 +174,7 @@ PyObject* launch_call(PyObject* self, PyObject* const* args, size_t nargsf, PyOb
       memcpy(c.w, w, sizeof w);
       memcpy(c.f, f, sizeof f);
       c.pointers = pointers;
+      c.numbers = numbers;
       for (Py_ssize_t i = 0; i < n; ++i)
         if (l->kinds[i] == 'p') {
           t_recording->held.push_back(args[i]);
@@ -228,10 +262,11 @@ bool place_tensor(PyObject* o, at::Tensor& t) {
   if (o == Py_None) return true;
   if (!THPVariable_Check(o)) return false;
   t = THPVariable_Unpack(o);
-  return t.is_cuda() && t.is_contiguous();
+  return t.is_contiguous();
 }
 
-// bind(olds): the places at which these tensors (None: no such tensor) begin.  False where two of them begin at the same address.
+// bind(olds): the places at which these tensors (None: no such tensor) begin.  False where two of them begin at the same address,
+// or where a launch was given a pointer as a number.
 PyObject* record_bind(PyObject* self, PyObject* olds) {
   Recorded& r = *reinterpret_cast<Record*>(self)->r;
   if (!PyTuple_Check(olds)) {
@@ -241,6 +276,8 @@ PyObject* record_bind(PyObject* self, PyObject* olds) {
   try {
     r.places.clear();
     r.olds.clear();
+    for (const Call& c : r.calls)
+      if (c.numbers) Py_RETURN_FALSE;
     for (Py_ssize_t j = 0; j < PyTuple_GET_SIZE(olds); ++j) {
       at::Tensor t;
       if (!place_tensor(PyTuple_GET_ITEM(olds, j), t)) Py_RETURN_FALSE;
@@ -374,6 +411,12 @@ PyMODINIT_FUNC PyInit_mf_host_call() {
   RecordType.tp_dealloc = record_free;
   RecordType.tp_methods = record_methods;
   if (PyType_Ready(&LaunchType) < 0 || PyType_Ready(&RecordType) < 0) return nullptr;
+  PyObject* ctypes = PyImport_ImportModule("ctypes");
+  if (!ctypes) return nullptr;
+  Py_XSETREF(g_array, PyObject_GetAttrString(ctypes, "Array"));
+  Py_XSETREF(g_pointer, PyObject_GetAttrString(ctypes, "c_void_p"));
+  Py_DECREF(ctypes);
+  if (!g_array || !g_pointer) return nullptr;
   PyObject* m = PyModule_Create(&module);
   if (!m) return nullptr;
   Py_INCREF(&LaunchType);
