@@ -59,7 +59,12 @@ class Part:
 class Norm(Part):
     def alike(self):
         """(constants, tensors) that decide what `forward` and the folds of this norm launch (tuples), or None: not said.
-        Norms with equal constants make the same launches with tensors of the same types and shapes, each with its own."""
+        Norms with equal constants make the same launches with tensors of the same types and shapes, each with its own.
+
+        What may be said is therefore a part whose forward does everything by launches of `ops` and gives them its own tensors
+        whole, each among `tensors` by its first address: no torch operation that computes or copies (it would not be made
+        again), and no view that begins inside a tensor of the part (its address would stay the first layer's).  An address that
+        is handed over as a number (`t.data_ptr() + offset`) is found out, and such a layer runs as if nothing were said."""
         return None
 
     def forward(self, h: torch.Tensor, out: Optional[torch.Tensor] = None,

@@ -132,8 +132,9 @@ def test_the_record_is_gone_before_the_last_block(monkeypatch):
     assert len(got[2]) == 2 and got[2] == got[3]
 
 
-def test_a_launch_that_fails_is_told(monkeypatch):
-    """A recorded launch's error code ends the step with the kernels' error."""
+def test_a_recorded_launch_that_fails_raises_the_kernels_error():
+    """(`test_host_call.py`: it ends the layer's launches and the step.)"""
     from minfer_amd.kernels import ops
+    ops.check_recorded(0)
     with pytest.raises(ops.KernelError):
         ops.check_recorded(1)
