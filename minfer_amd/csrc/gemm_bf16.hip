@@ -173,15 +173,19 @@ __device__ __forceinline__ void block_work(int order, int& tile, int& part) {
   part = order == ORDER_PARTS ? at / (int)gridDim.x : blockIdx.y;
   tile = order == ORDER_PARTS ? at - part * (int)gridDim.x : at;
 }
-// Part by part where the activations of all of K are more than an XCD's L2 of 4 MB and all parts' tiles are at most two a CU.  (rows x
-// weight rows x K, microseconds with the kernel behind it, the same eighth of every part / part by part: 203 x 3,584 x 18,944 54.8 /
-// 52.2, 2,048 x 2,048 x 8,192 79.1 / 74.8, 2,048 x 2,048 x 11,008 102.8 / 91.2, 2,048 x 896 x 4,864 38.7 / 33.5; less than an L2: 604 x
-// 2,048 x 2,048 22.2 / 24.8, 400 x 896 x 4,864 17.1 / 17.9.)  With more tiles the XCDs stand in different parts of K at one time: level
-// at 462 tiles (2,600 x 3,584 x 18,944 312.6 / 313), slower beyond: 3,300 x 5,120 x 13,824 (780) 455 / 469, 5,754 x 3,584 x 18,944
-// (966) 647 / 664, 8,192 x 5,120 x 13,824 (1,280) 913 / 932.
+// Part by part where the activations of all of K are half as much again as an XCD's L2 of 4 MB and all parts' tiles are at most two a
+// CU.  (rows x weight rows x K, microseconds with the kernel behind it, the same eighth of every part / part by part: 800 x 1,536 x
+// 8,960 41.7 / 38.8, 1,000 x 1,024 x 8,192 38.9 / 32.2, 2,048 x 2,048 x 11,008 101.3 / 90.0, 2,048 x 896 x 4,864 38.5 / 32.8; less than
+// an L2: 604 x 2,048 x 2,048 22.2 / 24.8.)  In between what an XCD reads again is little, and so it pays only for few weight rows
+// of a long K: 300 x 1,024 x 8,192 24.5 / 23.2, 256 x 1,536 x 8,960 23.2 / 22.7, but 604 x 896 x 4,864 20.1 / 21.4, 129 x 3,584 x
+// 18,944 46.9 / 48.6.  With more tiles the XCDs stand in different parts of K at one time: level at 462 tiles (2,600 x 3,584 x 18,944
+// 312.6 / 313), slower beyond: 3,300 x 5,120 x 13,824 (780) 455 / 469, 5,754 x 3,584 x 18,944 (966) 647 / 664, 8,192 x 5,120 x 13,824
+// (1,280) 913 / 932.
 static int cu_count();
-int tile_order(int tiles, int splits, int M, int K) {
-  if (splits > 1 && (size_t)M * K * 2 > (4u << 20) && (long)tiles * splits <= 2L * cu_count()) return ORDER_PARTS;
+int tile_order(int tiles, int splits, int M, int N, int K) {
+  const size_t bytes = (size_t)M * K * 2;
+  const bool pays = bytes > (6u << 20) || (bytes > (4u << 20) && N <= 2048 && K >= 8192);
+  if (splits > 1 && pays && (long)tiles * splits <= 2L * cu_count()) return ORDER_PARTS;
   return tiles >= 16 ? ORDER_TILES : ORDER_PLAIN;
 }
 
@@ -885,7 +889,7 @@ int launch_tile_step(const bf16* A, int lda, const bf16* W, int ldw, const float
   }
   const int tiles_m = GROUPED ? n_groups : (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
   kern<<<dim3(tiles_m * tiles_n, splits), 64 * TT::WAVES, TT::template lds<STAGES>(), stream>>>(
-      A, lda, W, ldw, bias, C, ldc, M, N, K, epi, tiles_m, tile_order(tiles_m * tiles_n, splits, M, K), k_per_split, groups, in_ssq, in_parts, in_eps);
+      A, lda, W, ldw, bias, C, ldc, M, N, K, epi, tiles_m, tile_order(tiles_m * tiles_n, splits, M, N, K), k_per_split, groups, in_ssq, in_parts, in_eps);
   return mf_launch_status();
 }
 
@@ -913,7 +917,7 @@ int launch_tile_dma(const bf16* A, int lda, const bf16* W, int ldw, const float*
   if (const int e = configure_tile_dma<BM, BN, STAGES, false>()) return e;
   const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
   tile_dma_kernel<BM, BN, STAGES><<<dim3(tiles_m * tiles_n, splits), 512, DmaTile<BM, BN>::template lds<STAGES>(), stream>>>(
-      A, lda, W, ldw, bias, C, ldc, M, N, K, epi, tiles_m, tile_order(tiles_m * tiles_n, splits, M, K), k_per_split, nullptr);
+      A, lda, W, ldw, bias, C, ldc, M, N, K, epi, tiles_m, tile_order(tiles_m * tiles_n, splits, M, N, K), k_per_split, nullptr);
   return mf_launch_status();
 }
 
@@ -932,7 +936,7 @@ int launch_tile_v(const bf16* A, int lda, const bf16* W, int ldw, const float* b
   }
   const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
   kern<<<dim3(tiles_m * tiles_n, splits), NTHR, smem, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi,
-                                                                tiles_m, tile_order(tiles_m * tiles_n, splits, M, K), k_per_split);
+                                                                tiles_m, tile_order(tiles_m * tiles_n, splits, M, N, K), k_per_split);
   return mf_launch_status();
 }
 

@@ -18,3 +18,9 @@ def test_every_tile_of_every_part(m, n, k):
     ops.linear(x, w, None, out, accumulate=True)
     # two 32-bit sums of k exact products, each some sqrt(k) roundings of at most half a unit of the largest sum
     assert (out - want).abs().max() <= 2.0 ** -22 * float(want.abs().max()) * k ** 0.5
+
+
+@pytest.mark.parametrize("m,n,k", [(604, 896, 4864), (680, 896, 4864), (300, 1024, 8192), (300, 2048, 8192), (300, 2112, 8192)])
+def test_either_side_of_the_activations_that_change_the_order(m, n, k):
+    """Between one and one and a half times an XCD's L2, and more; few weight rows of a long K and others."""
+    test_every_tile_of_every_part(m, n, k)
