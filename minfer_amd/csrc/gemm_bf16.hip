@@ -2795,12 +2795,15 @@ TilePlan plan_tiles(int M, int N, int K, bool dma_ok, int epi, int n_cu) {
 // Where `panel_dma_kernel` runs: J of its tiles (32 J weight rows), or 0.  All tiles are on the chip at once.
 //  * 17 to 64 rows: in `panel_kernel`'s place up to 160 weight rows a CU (SwiGLU of 37,888 x 3,584, 17 / 48 / 64 rows 50.5 / 53.9 /
 //    58.7 us there and 48.9 / 49.8 / 50.8 so; 40,960 x 512 17.2 and 11.9); beyond, that kernel's blocks go on from pass to pass.
+//    (Timed at 32,768 to 40,960 weight rows of 512 to 8,192, all epilogues: 0.53 to 1.01 of its time, except 17 to 40 rows against
+//    34,816 to 37,888 of 6,144 or 8,192, which begin 12 or 16 KB apart: up to 1.06, 36,864 x 8,192 122.5 and 129.1.)
 //  * 51 to 64 rows, SwiGLU, more than 64 and up to 96 weight rows a CU against a K of up to 2,048, where 64 x 64 tiles are two a CU:
-//    22,016 x 2,048, 64 rows 27.6 and 23.9; 17,920 x 1,536 20.7 and 16.3.  (Fewer rows gain less, 33 rows 25.5 and 23.2, and are left
-//    with the tiles, as are 64 weight rows a CU and fewer: 9,728 x 896 6.0 and 7.7.)
+//    22,016 x 2,048, 64 rows 27.6 and 23.9; 17,920 x 1,536 20.7 and 16.3.  (17 to 50 rows would gain there too, 33 rows 25.5 and 23.2,
+//    and still run as tiles.  With 64 weight rows a CU and fewer the tiles are the faster: 9,728 x 896 6.0 and 7.7.)
 //  * 65 to 128 rows, more than 128 and up to 160 weight rows a CU, where tiles of 128 x 128 take two rounds and tiles of 128 x 256
-//    leave a third of the CUs idle: SwiGLU of 37,888 x 3,584, 65 / 100 / 128 rows 63.5 / 66.7 / 68.9 and 52.6 / 55.6 / 58.7.  (32,768 x
-//    2,048, a round of 128 x 128: 36.2 and 38.5; 208 rows, in tiles of 208 x 160: level with 256 x 192.)
+//    leave a third of the CUs idle: SwiGLU of 37,888 x 3,584, 65 / 100 / 128 rows 63.5 / 66.7 / 68.9 and 52.6 / 55.6 / 58.7.  No other
+//    plan is asked for its price there: at 32,800 to 40,960 weight rows of 512 to 8,192, all epilogues, 0.80 to 1.0 of the tiles' time.
+//    (32,768 x 2,048, a round of 128 x 128: 36.2 and 38.5; 208 rows, in tiles of 208 x 160: level with 256 x 192.)
 int panel_dma_units(int M, int N, int K, int epi, int n_cu) {
   const int units = (N + 31) / 32;
   if (M <= 16 || M > 128 || K % DMA_BK || n_cu <= 0 || units > 5 * n_cu) return 0;
