@@ -18,6 +18,50 @@ import torch
 SHARE_START = 4
 
 
+def _fitted_target(blocks, target: int, max_shares: int, places: int) -> int:
+    """The least number of pages a workgroup, from `target` on, at which all workgroups of a head run at once, or `target` where that
+    would end later.  `blocks`: pages of a block -> how many blocks have them; `places`: workgroups of a head that run at once."""
+    def too_many(t):
+        return sum(c * min(max_shares, (pages + t - 1) // t) for pages, c in blocks.items()) > places
+
+    if not too_many(target):
+        return target
+    low, high, step = target, target + 1, 2
+    while too_many(high):
+        low, high, step = high, high + step, 2 * step
+    while high - low > 1:
+        mid = (low + high) // 2
+        low, high = (mid, high) if too_many(mid) else (low, mid)
+    return high if _last_end(blocks, high, max_shares, places) <= _last_end(blocks, target, max_shares, places) else target
+
+
+def _last_end(blocks, target: int, max_shares: int, places: int) -> int:
+    """When the last workgroup of a head ends, in pages: the longest start, and each of the others in the place that is free first."""
+    lengths = Counter()
+    for pages, c in blocks.items():
+        shares = min(max_shares, (pages + target - 1) // target)
+        walk, more = divmod(pages, shares)
+        lengths[walk + 1] += c * more
+        lengths[walk] += c * (shares - more)
+    walks = sorted(((w, c) for w, c in lengths.items() if c), reverse=True)
+    last = walks[0][0] + SHARE_START
+    at, left = 0, places                             # runs of equal walks up to the last one that starts, and behind it
+    while at < len(walks) and walks[at][1] <= left:
+        left -= walks[at][1]
+        at += 1
+    started, waiting = walks[:at], walks[at:]
+    if waiting and left:
+        started.append((waiting[0][0], left))
+        waiting[0] = (waiting[0][0], waiting[0][1] - left)
+    while waiting and started:                       # the longest that waits follows the shortest that started
+        (w, n), (s, m) = waiting[0], started[-1]
+        last = max(last, w + s + 2 * SHARE_START)
+        both = min(n, m)
+        waiting[:1] = [(w, n - both)] if n > both else []
+        started[-1:] = [(s, m - both)] if m > both else []
+    return last
+
+
 @dataclass
 class StepContext:
     cache: object                        # minfer_amd.cache.Cache
@@ -131,36 +175,15 @@ class StepContext:
                 self._memo[key] = None
                 return None
             target = max(1, int(min_pages), -(-total * n_heads // max(1, n_cu * per_cu)))
-            def shares_of(pages, t):
-                return min(max_shares, (pages + t - 1) // t)
-
-            of_pages = Counter(pages for pages, _, _ in tiles)
-
-            def ends(t):                                     # when the last workgroup does, in pages (SHARE_START for starting and leaving)
-                walks = sorted((-(-(pages - s) // shares_of(pages, t)) for pages, c in of_pages.items()
-                                for s in range(shares_of(pages, t)) for _ in range(c)), reverse=True)
-                places = n_cu * per_cu // n_heads            # of each head: the longest start, the others as places become free
-                last = walks[0] + SHARE_START
-                for i, w in enumerate(walks[places:]):
-                    last = max(last, w + walks[max(0, places - 1 - i)] + 2 * SHARE_START)
-                return last
             # A few workgroups that wait for a place can double the time (28 heads on 4, 611 tokens on 8,000 keys: 544 workgroups in
             # 512 places 121 us, all at once 96; 16 on 2, 180 + 101 + 168 + 155 on 5,000: 61 and 46).  But blocks that leave their place
             # almost at once count as much as one of 470 pages: 125 prompts of 18 tokens and 36 tokens on 30,000 keys, 28 heads on 4,
             # 93 us in shares of 59 pages, 595 with all at once.  So the two are compared by when their last workgroup ends.
             if at_once and len(tiles) * n_heads <= n_cu * per_cu:
-                low, high = target, max(target, longest)     # the least target at which all run at once
-                while low < high:
-                    mid = (low + high) // 2
-                    if n_heads * sum(c * shares_of(pages, mid) for pages, c in of_pages.items()) > n_cu * per_cu:
-                        low = mid + 1
-                    else:
-                        high = mid
-                if low > target and ends(low) <= ends(target):
-                    target = low
+                target = _fitted_target(Counter(t[0] for t in tiles), target, max_shares, n_cu * per_cu // n_heads)
             entries, n_slots, most = [], 0, 1
             for pages, b, q0 in tiles:
-                shares = shares_of(pages, target)
+                shares = min(max_shares, (pages + target - 1) // target)
                 most = max(most, shares)
                 if shares <= 1:
                     entries.append((pages, b, q0, 0))
