@@ -723,11 +723,16 @@ MF_API int mf_rope_kvwrite(const float* qkv, const float* cs, const float* sn, c
       kern<<<n_tok, few ? few : 256, 0, stream>>>(qkv, cs, sn, positions, seq_of_tok, page_table, pt_stride, (OT*)q_out, (OT*)kcache,
                                                   (OT*)vcache, nh, nk, hd, write_kv, parts, bias);
     };
-    const bool one = parts == 1;
-    if (is_bf16)
-      run(!few ? rope_kvwrite_vec_kernel<bf16, true> : one ? rope_kvwrite_few_kernel<bf16, true, false> : rope_kvwrite_few_kernel<bf16, true, true>, bf16{});
-    else
-      run(!few ? rope_kvwrite_vec_kernel<float, false> : one ? rope_kvwrite_few_kernel<float, false, false> : rope_kvwrite_few_kernel<float, false, true>, 0.f);
+    if (few && parts == 1) {
+      if (is_bf16) run(rope_kvwrite_few_kernel<bf16, true, false>, bf16{});
+      else run(rope_kvwrite_few_kernel<float, false, false>, 0.f);
+    } else if (few) {
+      if (is_bf16) run(rope_kvwrite_few_kernel<bf16, true, true>, bf16{});
+      else run(rope_kvwrite_few_kernel<float, false, true>, 0.f);
+    } else {
+      if (is_bf16) run(rope_kvwrite_vec_kernel<bf16, true>, bf16{});
+      else run(rope_kvwrite_vec_kernel<float, false>, 0.f);
+    }
     return mf_launch_status();
   }
   if (parts > 1) return (int)hipErrorInvalidValue;        // (the caller asks for parts only where the kernel above runs)
