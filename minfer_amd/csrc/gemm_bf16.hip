@@ -17,6 +17,7 @@
 //    into MFMA operands (16x16x32) and the partial sums meet in LDS.
 //  * `panel_kernel`: 17 to 64 rows against a wide matrix: one block per CU over the whole of K; `panel_dma_kernel`: the same for up to
 //    128 rows with copies straight into LDS, where all its tiles are on the chip at once.
+//  * `whole_kernel`: 17 to 64 rows with a norm folded in on either side, a short K: one kernel over the whole of K.
 //  * `skinny_ring_kernel`, `skinny_kernel` (any alignment): 17 to 64 rows.  Each wave owns 16
 //    weight rows and reads them from HBM straight into MFMA operands, the activation rows are
 //    staged in LDS and shared by the block, K may be split over blocks with a fixed-order
@@ -701,6 +702,46 @@ __global__ __launch_bounds__(512, 2) void tile_dma_kernel(const bf16* __restrict
   dma_epilogue<TT>(acc, smem + wid * TT::OWN, bias, C, ldc, M, N, epi, m0 + wave_m * TT::ROWS, n0, wave_n, lane);
 }
 
+// The sum of a row's `parts` numbers by LANES lanes that stand side by side (l: the lane's place among them), in two steps so that a
+// kernel asks early and adds late: every lane asks for Q x 4 of them at once, in fours where the rows allow 16-byte loads, and what is
+// left of a longer row when it adds up.  A row without parts (p null) asks for nothing and gives 0.
+template <int LANES, int Q>
+struct LanesSum {
+  float x[Q][4];
+  __device__ __forceinline__ static bool fours(const float* p, int parts) { return parts % 4 == 0 && (uintptr_t)p % 16 == 0; }
+  __device__ __forceinline__ void ask(const float* __restrict__ p, int parts, int l) {
+#pragma unroll
+    for (int q = 0; q < Q; ++q)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[q][e] = 0.f;
+    if (!p) return;
+    if (fours(p, parts)) {
+#pragma unroll
+      for (int q = 0; q < Q; ++q)
+        if ((q * LANES + l) * 4 < parts) {
+          const float4 v = *reinterpret_cast<const float4*>(p + (q * LANES + l) * 4);
+          x[q][0] = v.x; x[q][1] = v.y; x[q][2] = v.z; x[q][3] = v.w;
+        }
+    } else {
+#pragma unroll
+      for (int q = 0; q < Q; ++q)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if ((q * 4 + e) * LANES + l < parts) x[q][e] = p[(q * 4 + e) * LANES + l];
+    }
+  }
+  __device__ __forceinline__ float add(const float* __restrict__ p, int parts, int l) const {
+    float t = 0.f;
+#pragma unroll
+    for (int q = 0; q < Q; ++q) t += (x[q][0] + x[q][1]) + (x[q][2] + x[q][3]);
+    if (p)
+      for (int i = Q * LANES * 4 + l; i < parts; i += LANES) t += p[i];
+#pragma unroll
+    for (int o = LANES / 2; o > 0; o >>= 1) t += __shfl_xor(t, o, MF_WAVE);
+    return t;
+  }
+};
+
 // ---- the smaller tiles: one barrier a k tile
 // 128 x 128 on 8 waves and 64 x 64 on 4, for products whose larger tiles would leave most of the chip idle: a block's time
 // is then its own chain of k tiles, whatever the others do, and a k tile's chain is what is kept short: wait for the copies
@@ -789,32 +830,20 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void tile_step_kernel(const
     for (int q = 0; q < LA; ++q) dma16(A + k, ga[q], __builtin_amdgcn_readfirstlane(base + q * (WAVES * 1024)));
   };
   const int sw = (fr >> 1) & 7;
-  // the rows' partial sums are asked for in front of the first copies and added up behind them (what waits for the sums then
-  // waits for the first k tiles, which the loop needs anyway)
-  constexpr int PART_LOADS = 4;
-  float fac[I], part0[I][PART_LOADS];
+  // the rows' partial sums are asked for in front of the first copies and added up behind the products, eight lanes a row
+  constexpr int GROUPS = (BM + WAVES * 8 - 1) / (WAVES * 8);
+  LanesSum<8, 4> sums[SCALED ? GROUPS : 1];
+  auto part_row = [&](int q) {
+    const int r = m0 + (q * WAVES + wid) * 8 + (lane >> 3);
+    return r < M ? in_ssq + (size_t)r * in_parts : nullptr;
+  };
   if constexpr (SCALED) {
 #pragma unroll
-    for (int i = 0; i < I; ++i)
-#pragma unroll
-      for (int p = 0; p < PART_LOADS; ++p)
-        part0[i][p] = in_ssq[(size_t)min(m0 + wave_m * TT::ROWS + i * 16 + fr, M - 1) * in_parts + min(p, in_parts - 1)];
+    for (int q = 0; q < GROUPS; ++q) sums[q].ask(part_row(q), in_parts, lane & 7);
     __builtin_amdgcn_sched_barrier(0);
   }
 #pragma unroll
   for (int t = 0; t < STAGES - 1; ++t) copy(t, t);
-  if constexpr (SCALED) {
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int i = 0; i < I; ++i) {
-      const float* p = in_ssq + (size_t)min(m0 + wave_m * TT::ROWS + i * 16 + fr, M - 1) * in_parts;
-      float t = 0.f;
-#pragma unroll
-      for (int q = 0; q < PART_LOADS; ++q) t += q < in_parts ? part0[i][q] : 0.f;
-      for (int q = PART_LOADS; q < in_parts; ++q) t += p[q];
-      fac[i] = 1.0f / sqrtf(t / (float)K + in_eps);
-    }
-  }
   bf16x8 fa[2][2][I], fw[2][2][J];                           // [set][k-step][block]
   auto read = [&](int st, auto SET) {
     constexpr int set = decltype(SET)::value;
@@ -866,10 +895,21 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void tile_step_kernel(const
   dma_wait<0>();
   dma_meet();
   if constexpr (SCALED) {
+    static_assert(WAVES * TT::OWN + BM * 4 <= TT::template lds<STAGES>(), "the factors stand behind the waves' own LDS");
+    float* fac = reinterpret_cast<float*>(smem + WAVES * TT::OWN);
 #pragma unroll
-    for (int i = 0; i < I; ++i)
+    for (int q = 0; q < GROUPS; ++q) {
+      const float t = sums[q].add(part_row(q), in_parts, lane & 7);
+      const int r = (q * WAVES + wid) * 8 + (lane >> 3);
+      if ((lane & 7) == 0 && r < BM) fac[r] = 1.0f / sqrtf(t / (float)K + in_eps);
+    }
+    __syncthreads();
 #pragma unroll
-      for (int j = 0; j < J; ++j) acc[i][j] *= fac[i];
+    for (int i = 0; i < I; ++i) {
+      const float f = fac[wave_m * TT::ROWS + i * 16 + fr];
+#pragma unroll
+      for (int j = 0; j < J; ++j) acc[i][j] *= f;
+    }
   }
   dma_epilogue<TT>(acc, smem + wid * TT::OWN, bias, C, ldc, M, N, epi, m0 + wave_m * TT::ROWS, n0, wave_n, lane);
 }
@@ -1339,7 +1379,7 @@ bool ring_takes(bool aligned, int K, int splits, int k_per_split) {
 //    the stream next leaves, beside the stream's new rows, xg = bf16(x g) and for every row the
 //    sums of x^2 in parts (`out_*`): over runs of 256 columns where the kernel that adds the parts
 //    of a K split does it (17 to 64 rows: it has every new value of x in its hands), one part per
-//    block where a one-kernel product of at most 16 rows does it in its epilogue (every block
+//    block where a one-kernel product does it in its epilogue (at most 16 rows, or `whole_kernel`: every block
 //    owns some columns; `out_parts` places a row, the ones past the grid set to zero);
 //  * the product that follows takes xg as its activations and multiplies its own sums by the
 //    row's 1 / sqrt(sum / K + eps) in its epilogue (`in_*`), the partial sums of squares added up
@@ -1365,11 +1405,20 @@ struct FusedNorm {
 // rows' loads in flight together, and add up in a fixed tree.
 template <int NR>
 __device__ __forceinline__ void row_sums_ask(const FusedNorm& f, const int (&rows)[NR], int M, int lane, float (&t)[NR]) {
+  constexpr int AT_ONCE = 4;             // of a row, asked for at once (as many as a product of one block a CU leaves)
+  float x[NR][AT_ONCE];
+#pragma unroll
+  for (int i = 0; i < NR; ++i)
+#pragma unroll
+    for (int q = 0; q < AT_ONCE; ++q)
+      x[i][q] = rows[i] >= 0 && rows[i] < M && lane + q * 64 < f.in_parts ? f.in_ssq[(size_t)rows[i] * f.in_parts + lane + q * 64] : 0.f;
 #pragma unroll
   for (int i = 0; i < NR; ++i) {
     t[i] = 0.f;
+#pragma unroll
+    for (int q = 0; q < AT_ONCE; ++q) t[i] += x[i][q];
     if (rows[i] >= 0 && rows[i] < M)
-      for (int p = lane; p < f.in_parts; p += 64) t[i] += f.in_ssq[(size_t)rows[i] * f.in_parts + p];
+      for (int p = lane + AT_ONCE * 64; p < f.in_parts; p += 64) t[i] += f.in_ssq[(size_t)rows[i] * f.in_parts + p];
   }
 }
 
@@ -1568,6 +1617,169 @@ int launch_skinny16(const bf16* A, int lda, const bf16* W, int ldw, const float*
   else
     skinny16_kernel<NW, NT, S, false, PAIR><<<blocks, NW * 64, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M,
                                                                             N, K, k_per_wave, epi);
+  return mf_launch_status();
+}
+
+// ---- 17 to 64 rows over the whole of K, with a norm folded in
+// The K-split kernels (below) need a second one to add their parts, 4 to 5 us of every product, and against a short K that is as
+// much as the product itself.  Here a block takes 16 MT rows and up to 16 NT weight rows over the whole of K, its waves share K and
+// read both operands straight into MFMA operands, the whole slice or S steps of it in flight (nothing is staged: no wave reads what
+// another does), their sums meet in LDS, and the epilogue takes the norm's factors, adds to the stream and prepares the next norm.
+// What bounds it is how many of these gathered loads (16 rows of 64 bytes) a CU gets through, activations above all: some 3.1 us
+// and 0.175 us for each of a wave's loads, blocks of a CU added up (measured over 12 shapes of 896 to 18,944, 20 to 64 rows).
+// Hence the choice of `whole_plan`.  q|k|v and o of 32 rows, this / K split or 64 x 64 tiles: 1,152 x 896 3.8 / 8.5 us, 896 x 896
+// 4.3 / 10.2, 2,048 x 1,536 4.7 / 10.5, 2,560 x 2,048 5.9 / 10.7; 896 x 4,864 9.2 / 11.0.
+template <int MT, int NT, int S>
+__global__ __launch_bounds__(512) void whole_kernel(const bf16* __restrict__ A, int lda, const bf16* __restrict__ W,
+                                                    const float* __restrict__ bias, float* __restrict__ C, int ldc, int M, int N, int K,
+                                                    int accumulate, int rpb, FusedNorm fused) {
+  constexpr int NW = 8, COLS = 16 * NT, RS = COLS + 4, ROWS = 16 * MT;
+  __shared__ float red[NW][ROWS][RS];
+  const int lane = threadIdx.x & 63, r16 = lane & 15;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int m0 = blockIdx.y * ROWS, n0 = blockIdx.x * rpb;             // rpb: weight rows of a block, as in rolling16_kernel
+  const int total = K / 32, share = (total + NW - 1) / NW;
+  const int first = min(wid * share, total);
+  const int T = min(share, total - first);                             // steps of this wave
+  const int kq = first * 32 + (lane >> 4) * 8;
+  const bf16 *arow[MT], *wrow[NT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i) arow[i] = A + (size_t)min(m0 + i * 16 + r16, M - 1) * lda + kq;
+#pragma unroll
+  for (int j = 0; j < NT; ++j) wrow[j] = w_operand<true>(W, 0, K, min(n0 + min(j * 16 + r16, rpb - 1), N - 1), kq);
+  // the epilogue's places of this lane, what it needs of them asked for in front of the stream
+  constexpr int PER_WAVE = 64 / COLS, PASS = NW * PER_WAVE, PASSES = (ROWS + PASS - 1) / PASS;
+  const int e_c = lane % COLS, e_n = n0 + e_c;
+  const bool e_col = e_c < rpb && e_n < N;
+  const float e_g = fused.out_g && e_col ? fused.out_g[e_n] : 0.f, e_b = bias && e_col ? bias[e_n] : 0.f;
+  float old[PASSES];
+  LanesSum<COLS, 2> sums[PASSES];                                      // of the lane's own row
+  auto part_row = [&](int p) {
+    const int r = p * PASS + wid * PER_WAVE + lane / COLS, m = m0 + r;
+    return fused.in_ssq && r < ROWS && m < M ? fused.in_ssq + (size_t)m * fused.in_parts : nullptr;
+  };
+#pragma unroll
+  for (int p = 0; p < PASSES; ++p) {
+    const int r = p * PASS + wid * PER_WAVE + lane / COLS, m = m0 + r;
+    old[p] = accumulate && r < ROWS && m < M && e_col ? C[(size_t)m * ldc + e_n] : 0.f;
+  }
+  floatx4 acc[MT][NT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+  bf16x8 a[S][MT], w[S][NT];
+  auto load = [&](int s, int at) {
+#pragma unroll
+    for (int j = 0; j < NT; ++j) w[s][j] = *reinterpret_cast<const bf16x8*>(wrow[j] + (size_t)at * 512);
+#pragma unroll
+    for (int i = 0; i < MT; ++i) a[s][i] = *reinterpret_cast<const bf16x8*>(arow[i] + at * 32);
+  };
+  auto multiply = [&](int s) {
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int j = 0; j < NT; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[s][i], w[s][j], acc[i][j], 0, 0, 0);
+  };
+#pragma unroll
+  for (int s = 0; s < S; ++s)
+    if (s < T) load(s, s);
+#pragma unroll
+  for (int p = 0; p < PASSES; ++p) sums[p].ask(part_row(p), fused.in_parts, e_c);
+  __builtin_amdgcn_sched_barrier(0);
+  int base = 0;
+  for (; base + 2 * S <= T; base += S) {                               // rounds whose refills all exist
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      multiply(s);
+      load(s, base + S + s);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  const int rem = T - base - S;                                        // steps behind those in registers (none if not above 0)
+#pragma unroll
+  for (int s = 0; s < S; ++s) {
+    if (base + s < T) multiply(s);
+    if (s < rem) load(s, base + S + s);
+  }
+#pragma unroll
+  for (int s = 0; s < S; ++s)
+    if (s < rem) multiply(s);
+  // D[m][n]: n = lane % 16, m = 4 (lane / 16) + r
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) red[wid][i * 16 + (lane >> 4) * 4 + r][j * 16 + r16] = acc[i][j][r];
+  float fac[PASSES];
+#pragma unroll
+  for (int p = 0; p < PASSES; ++p)
+    fac[p] = fused.in_ssq ? 1.0f / sqrtf(sums[p].add(part_row(p), fused.in_parts, e_c) / (float)K + fused.in_eps) : 1.f;
+  __syncthreads();
+#pragma unroll
+  for (int p = 0; p < PASSES; ++p) {
+    const int r = p * PASS + wid * PER_WAVE + lane / COLS, m = m0 + r;
+    const bool mine = r < ROWS && m < M && e_col;
+    float sq = 0.f;
+    if (mine) {
+      float v = 0.f;
+#pragma unroll
+      for (int ww = 0; ww < NW; ++ww) v += red[ww][r][e_c];
+      v *= fac[p];
+      v = v + e_b + old[p];
+      C[(size_t)m * ldc + e_n] = v;
+      if (fused.out_g) {
+        fused.out_xg[(size_t)m * N + e_n] = (bf16)(v * e_g);
+        sq = v * v;
+      }
+    }
+    if (fused.out_g) {                                                 // this block's part of the row
+#pragma unroll
+      for (int o = COLS / 2; o > 0; o >>= 1) sq += __shfl_xor(sq, o, MF_WAVE);
+      if (e_c == 0 && r < ROWS && m < M) {
+        fused.out_ssq[(size_t)m * fused.out_parts + blockIdx.x] = sq;
+        if (blockIdx.x == 0)                                           // (a row's places past the grid: zero)
+          for (int x = gridDim.x; x < fused.out_parts; ++x) fused.out_ssq[(size_t)m * fused.out_parts + x] = 0.f;
+      }
+    }
+  }
+}
+
+// How `whole_kernel` cuts a product: tiles of rows and of weight rows a block, weight rows a block, blocks; `loads`: a wave's loads
+// by the cost above, those of the blocks that share a CU added up.  Every CU gets a block where there are rows enough.
+struct WholePlan { int mt, nt, rpb, gx, gy; long loads; };
+WholePlan whole_plan(int M, int N, int K, int n_cu) {
+  WholePlan best{0, 0, 0, 0, 0, 1L << 40};
+  for (int mt = 1; mt <= 2; ++mt)
+    for (int nt = 1; nt <= 2; ++nt) {
+      const int gy = (M + 16 * mt - 1) / (16 * mt), columns = std::max(1, n_cu / gy);
+      const int rpb = std::min(16 * nt, (N + columns - 1) / columns), gx = (N + rpb - 1) / rpb;
+      if (nt == 2 && rpb <= 16) continue;                              // (nothing to gain)
+      const long loads = ((long)gx * gy + n_cu - 1) / n_cu * (mt + nt) * ((K / 32 + 7) / 8);
+      if (loads < best.loads) best = WholePlan{mt, nt, rpb, gx, gy, loads};
+    }
+  return best;
+}
+// Up to 38 loads, where both ways take some 10 us: 896 x 4,864 (38) 9.2 here and 11.0 with K split, 3,584 x 3,584 at 32 rows (42) 11.9
+// and 12.5, 1,536 x 8,960 (70) 16.3 and 13.4.
+bool whole_takes(int M, int N, int K, bool aligned, bool tiled, int epi, int n_cu) {
+  if (M <= 16 || M > 64 || !aligned || !tiled || K % 32 || n_cu <= 0 || (epi != EPI_F32 && epi != EPI_ACC_F32)) return false;
+  return whole_plan(M, N, K, n_cu).loads <= 38;
+}
+
+int launch_whole(const bf16* A, int lda, const bf16* Wt, const float* bias, float* C, int ldc, int M, int N, int K, int epi,
+                 const FusedNorm& fused, hipStream_t stream) {
+  const WholePlan p = whole_plan(M, N, K, cu_count());
+  if (fused.out_g && fused.out_parts < p.gx) return MF_NOT_BUILT;
+  auto run = [&](auto MT, auto NT) {
+    whole_kernel<decltype(MT)::value, decltype(NT)::value, 8>
+        <<<dim3(p.gx, p.gy), 512, 0, stream>>>(A, lda, Wt, bias, C, ldc, M, N, K, epi == EPI_ACC_F32, p.rpb, fused);
+  };
+  using One = std::integral_constant<int, 1>;
+  using Two = std::integral_constant<int, 2>;
+  if (p.mt == 1) p.nt == 1 ? run(One{}, One{}) : run(One{}, Two{});
+  else p.nt == 1 ? run(Two{}, One{}) : run(Two{}, Two{});
   return mf_launch_status();
 }
 
@@ -2119,14 +2331,16 @@ __global__ __launch_bounds__(512, 2) void panel_dma_kernel(const bf16* __restric
   for (int i = 0; i < I; ++i)
 #pragma unroll
     for (int j = 0; j < J; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
-  // the rows' partial sums of squares are asked for here and added up behind the products (8 lanes a row)
+  // the rows' partial sums of squares are asked for here and added up behind the products, eight lanes a row (products of more than 64
+  // rows have none)
   constexpr int SUMS = (RA + 63) / 64;
-  float part[SUMS][2];
+  LanesSum<8, SUMS == 1 ? 4 : 1> sums[SUMS];
+  auto part_row = [&](int q) {
+    const int r = q * 64 + wid * 8 + (lane >> 3);
+    return in_ssq && r < M ? in_ssq + (size_t)r * in_parts : nullptr;
+  };
 #pragma unroll
-  for (int q = 0; q < SUMS; ++q)
-#pragma unroll
-    for (int e = 0; e < 2; ++e)
-      part[q][e] = in_ssq ? in_ssq[(size_t)min(q * 64 + wid * 8 + (lane >> 3), M - 1) * in_parts + min((lane & 7) + 8 * e, in_parts - 1)] : 0.f;
+  for (int q = 0; q < SUMS; ++q) sums[q].ask(part_row(q), in_parts, lane & 7);
   __builtin_amdgcn_sched_barrier(0);
   // what a wave copies: pieces wid, 8 + wid, ... of 8 rows (chunk c of a row at position c ^ ((row >> 1) & 7))
   const unsigned lds0 = (unsigned)(uintptr_t)smem;
@@ -2215,11 +2429,7 @@ __global__ __launch_bounds__(512, 2) void panel_dma_kernel(const bf16* __restric
 #pragma unroll
   for (int q = 0; q < SUMS; ++q) {
     const int r = q * 64 + wid * 8 + (lane >> 3);
-    float t = (lane & 7) < in_parts ? part[q][0] : 0.f;
-    t += (lane & 7) + 8 < in_parts ? part[q][1] : 0.f;
-    for (int p = (lane & 7) + 16; p < in_parts; p += 8) t += in_ssq[(size_t)min(r, M - 1) * in_parts + p];
-#pragma unroll
-    for (int o = 1; o < 8; o <<= 1) t += __shfl_xor(t, o, MF_WAVE);
+    const float t = sums[q].add(part_row(q), in_parts, lane & 7);
     if ((lane & 7) == 0 && r < RA) fac[r] = in_ssq ? 1.0f / sqrtf(t / (float)K + in_eps) : 1.0f;
   }
 #pragma unroll
@@ -3031,6 +3241,8 @@ static int skinny_product(const void* A, int lda, const void* W, const void* Wt,
   const bf16* w = (const bf16*)W;
   const bf16* wt = (K % 32 == 0 && (uintptr_t)Wt % 16 == 0) ? (const bf16*)Wt : nullptr;
   const bool folds = fused.in_ssq || fused.out_g;
+  if (folds && whole_takes(M, N, K, vec_ok, wt != nullptr, epi, cu_count()))
+    return launch_whole(a, lda, wt, bias, (float*)C, ldc, M, N, K, epi, fused, stream);
   const SkinnyChoice choice = skinny_choice(M, N, K, vec_ok, wt != nullptr, epi, splits, k_per_split, cu_count());
   // at most 16 rows: the register-resident kernel takes a prepared norm and prepares the next one, the
   // rolling kernel prepares the next one; the K-split kernels' second kernel counts its parts otherwise
@@ -3088,7 +3300,8 @@ MF_API int mf_gemm_bf16_skinny(const void* A, int lda, const void* W, const void
 //    product's sums are multiplied by the row's 1 / sqrt(sum / K + eps) before bias and epilogue.
 //  * out_g [N], out_xg [M][N] bf16, out_ssq [M][out_parts]: beside C (32-bit, stored or added
 //    to), bf16(C g) and the sums of C^2 in parts are written: over runs of 256 columns (out_parts =
-//    ceil(N / 256)) for 17 to 64 rows; for at most 16 rows one part per block of the product's one
+//    ceil(N / 256)) for 17 to 64 rows, or one part per block where `whole_kernel` takes them (out_parts at least
+//    `mf_gemm_bf16_whole_parts`, the places past it set to zero); for at most 16 rows one part per block of the product's one
 //    kernel, out_parts at least the number of CUs (the places past the grid are set to zero).
 MF_API int mf_gemm_bf16_skinny_fused(const void* A, int lda, const void* W, const void* Wt, int ldw,
                                      const float* bias, void* C, int ldc, float* part, int M, int N, int K,
@@ -3101,6 +3314,13 @@ MF_API int mf_gemm_bf16_skinny_fused(const void* A, int lda, const void* W, cons
   if (out_g && out_parts < (N + 255) / 256) return (int)hipErrorInvalidValue;
   const FusedNorm fused{in_ssq, in_parts, in_eps, out_g, (bf16*)out_xg, out_ssq, out_parts};
   return skinny_product(A, lda, W, Wt, ldw, bias, C, ldc, part, M, N, K, splits, k_per_split, epi, fused, stream);
+}
+
+// The partial sums of squares a row that `mf_gemm_bf16_skinny_fused` leaves with out_* where one kernel over the whole of K takes
+// the product of 17 to 64 rows (aligned operands and the tiled copy given): one for each of its blocks; 0 where it does not.
+MF_API int mf_gemm_bf16_whole_parts(int M, int N, int K, int n_cu) {
+  if (M <= 0 || N <= 0 || K <= 0 || n_cu <= 0) return 0;
+  return whole_takes(M, N, K, K % 8 == 0, true, EPI_ACC_F32, n_cu) ? whole_plan(M, N, K, n_cu).gx : 0;
 }
 
 // RMS norm of rows of the 32-bit residual stream x (row m of the product is x[row_idx[m]]), then
