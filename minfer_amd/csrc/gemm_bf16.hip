@@ -1504,14 +1504,23 @@ __global__ __launch_bounds__(NW * 64) void rolling16_kernel(const bf16* __restri
   if (epi == EPI_ACC_F32 && e_mine) c_old = ((const float*)C)[(size_t)e_m * ldc + e_n];
   if (fused.out_g && e_mine) e_g = fused.out_g[e_n];       // the next norm's weight, where this product prepares it
   const int R = T / S, rem = T % S;
-  if (R == 0) {       // a slice shorter than the registers hold: step by step
-    for (int s = 0; s < T; ++s) {
-      const bf16x8 a1 = *reinterpret_cast<const bf16x8*>(arow + s * 32);
+  if (R == 0) {       // a slice shorter than the registers hold: all of it asked for at once (in a loop over the slice's length the
+                      // compiler waits for every step: a decode step of one sequence at the 0.5B widths 775 us so, 749 at once)
+    bf16x8 a[S], w[NT][S];
 #pragma unroll
-      for (int j = 0; j < NT; ++j)
-        acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-            a1, *reinterpret_cast<const bf16x8*>(wrow[j] + s * WSTEP), acc[j], 0, 0, 0);
-    }
+    for (int s = 0; s < S; ++s)
+      if (s < T) {
+#pragma unroll
+        for (int j = 0; j < NT; ++j) w[j][s] = *reinterpret_cast<const bf16x8*>(wrow[j] + s * WSTEP);
+        a[s] = *reinterpret_cast<const bf16x8*>(arow + s * 32);
+      }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int s = 0; s < S; ++s)
+      if (s < T) {
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[s], w[j][s], acc[j], 0, 0, 0);
+      }
   } else {
     bf16x8 a[S], w[NT][S];
 #pragma unroll
