@@ -45,16 +45,24 @@ namespace {
 
 // EPI_XIELU: bfloat16 output of the xIELU activation of (sum + bias); the activation's two constants
 // (a_pos, a_neg: z > 0 -> a_pos z^2 + z/2, else a_neg (e^z - 1 - z) + z/2) stand behind the N biases.
-enum { EPI_F32 = 0, EPI_ACC_F32 = 1, EPI_BF16 = 2, EPI_SWIGLU = 3, EPI_XIELU = 4 };
+// EPI_RELU2: bfloat16 output of max(sum + bias, 0)^2.
+enum { EPI_F32 = 0, EPI_ACC_F32 = 1, EPI_BF16 = 2, EPI_SWIGLU = 3, EPI_XIELU = 4, EPI_RELU2 = 5, EPI_LAST = EPI_RELU2 };
 
 __device__ __forceinline__ float xielu_f(float z, float a_pos, float a_neg) {
   return z > 0.f ? fmaf(a_pos * z, z, 0.5f * z) : fmaf(a_neg, expm1f(z) - z, 0.5f * z);
+}
+
+__device__ __forceinline__ float relu2_f(float z) {
+  z = fmaxf(z, 0.f);
+  return z * z;
 }
 
 __device__ __forceinline__ void store_out(void* C, int ldc, int m, int n, float v, int epi,
                                           const float* __restrict__ bias = nullptr, int N = 0) {
   if (epi == EPI_XIELU) {
     ((bf16*)C)[(size_t)m * ldc + n] = (bf16)xielu_f(v, bias[N], bias[N + 1]);
+  } else if (epi == EPI_RELU2) {
+    ((bf16*)C)[(size_t)m * ldc + n] = (bf16)relu2_f(v);
   } else if (epi == EPI_BF16) {
     ((bf16*)C)[(size_t)m * ldc + n] = (bf16)v;
   } else {
@@ -391,10 +399,24 @@ struct DmaTile {
 // A wave's results, acc[i][j]: the lane's row is 16 i + lane % 16, its columns 16 j + 4 (lane / 16) + e.  They go through the
 // wave's own LDS in runs of 32 rows and leave in rows of 16 bytes a lane: straight from the registers every store would be
 // pieces of lines, 2 bytes a lane (506 us for 469 at 2,048 x 37,888 x 3,584).
-template <typename TT>
+// Gate and up rows as they stand, all gates and then all ups (`Halves`; a plain product has none): what a tile takes as its
+// interleaved weight row n, and the activation in the epilogue, y = act(gate, up), times sigmoid(z) of the row where there is one.
+struct Halves {
+  int width;               // gate rows, and up rows behind them; outputs
+  int silu;                // y = silu(gate) up, else the clamped form
+  float limit;
+  const float* z;          // [M] ldz apart, or null
+  int ldz;
+  __device__ __forceinline__ int row(int n) const { return min((n >> 6) * 32 + (n & 31), width - 1) + ((n >> 5) & 1) * width; }
+  __device__ __forceinline__ float act(float g, float u) const {
+    return silu ? g * (1.0f / (1.0f + expf(-g))) * u : clamped_gate(g, u, limit);
+  }
+};
+
+template <typename TT, bool HALVES = false>
 __device__ __forceinline__ void dma_epilogue(floatx4 (&acc)[TT::I][TT::J], unsigned char* __restrict__ own,
                                              const float* __restrict__ bias, void* __restrict__ C, int ldc, int M, int N, int epi,
-                                             int mw, int n0, int wn, int lane) {
+                                             int mw, int n0, int wn, int lane, const Halves& halves = Halves{}) {
   constexpr int J = TT::J, STEP = TT::STEP, COLS = TT::COLS;
   const int row = lane & 15, sub = (lane >> 4) * 4;
   const int b0 = TT::first(wn);
@@ -463,22 +485,31 @@ __device__ __forceinline__ void dma_epilogue(floatx4 (&acc)[TT::I][TT::J], unsig
 #pragma unroll
       for (int h = 0; h < TT::I / 2; ++h) {
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < 2; ++i) {
+          float s = 1.f;
+          if constexpr (HALVES) {
+            const int m = mw + h * 32 + i * 16 + row;
+            if (halves.z && m < M) s = 1.0f / (1.0f + expf(-halves.z[(size_t)m * halves.ldz]));
+          }
 #pragma unroll
           for (int p = 0; p < J / 2; ++p) {
             const int jg = TT::PAIRED ? 2 * p : (p >> 1) * 4 + (p & 1), ju = jg + 2 / STEP;
             bf16x4 v;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = (bf16)act(acc[h * 2 + i][jg][e], acc[h * 2 + i][ju][e]);
+            for (int e = 0; e < 4; ++e) v[e] = (bf16)(HALVES ? act(acc[h * 2 + i][jg][e], acc[h * 2 + i][ju][e]) * s
+                                                             : act(acc[h * 2 + i][jg][e], acc[h * 2 + i][ju][e]));
             *reinterpret_cast<bf16x4*>(st + (i * 16 + row) * LD + p * 16 + sub) = v;
           }
+        }
         leave(std::integral_constant<int, COLS / 2>{}, h, ldc, [&](int c) {
           const int p = c >> 4, b = b0 + (TT::PAIRED ? 2 * p * STEP : (p >> 1) * 4 + (p & 1));
           return (n0 >> 1) + ((b >> 2) * 2 + (b & 1)) * 16 + (c & 15);
         });
       }
     };
-    if (bias) {
+    if constexpr (HALVES) {
+      gated([&](float g, float u) { return halves.act(g, u); });
+    } else if (bias) {
       const float limit = *bias;
       gated([=](float g, float u) { return clamped_gate(g, u, limit); });
     } else {
@@ -503,7 +534,7 @@ __device__ __forceinline__ void dma_epilogue(floatx4 (&acc)[TT::I][TT::J], unsig
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const float z = acc[h * 2 + i][j][e] + b[e];
-          v[e] = (bf16)(epi == EPI_XIELU ? xielu_f(z, ap, an) : z);
+          v[e] = (bf16)(epi == EPI_XIELU ? xielu_f(z, ap, an) : epi == EPI_RELU2 ? relu2_f(z) : z);
         }
         *reinterpret_cast<bf16x4*>(st + (i * 16 + row) * LD + j * 16 + sub) = v;
       }
@@ -512,13 +543,13 @@ __device__ __forceinline__ void dma_epilogue(floatx4 (&acc)[TT::I][TT::J], unsig
   }
 }
 
-template <int BM, int BN, int STAGES, bool GROUPED = false>
+template <int BM, int BN, int STAGES, bool GROUPED = false, bool HALVES = false>
 __global__ __launch_bounds__(512, 2) void tile_dma_kernel(const bf16* __restrict__ A, int lda,
                                                        const bf16* __restrict__ W, int ldw,
                                                        const float* __restrict__ bias, void* __restrict__ C,
                                                        int ldc, int M, int N, int K, int epi, int tiles_m,
                                                        int order, int k_per_split,
-                                                       const RowGroup* __restrict__ groups = nullptr) {
+                                                       const RowGroup* __restrict__ groups = nullptr, Halves halves = Halves{}) {
   using TT = DmaTile<BM, BN>;
   constexpr int ROW = DMA_BK * 2, A_ST = BM * ROW, W_ST = BN * ROW, W_AT = STAGES * A_ST;
   constexpr int I = TT::I, IH = TT::IH, J = TT::J, J0 = TT::J0, J1 = TT::J1, LA = TT::LA, LW0 = TT::LW0, LW1 = TT::LW1, T = TT::T;
@@ -540,8 +571,8 @@ __global__ __launch_bounds__(512, 2) void tile_dma_kernel(const bf16* __restrict
     const int first = __builtin_amdgcn_readfirstlane(groups[bm].first), matrix = __builtin_amdgcn_readfirstlane(groups[bm].matrix);
     M = __builtin_amdgcn_readfirstlane(groups[bm].rows);
     A += (size_t)first * lda;
-    W += (size_t)matrix * N * ldw;
-    C = (float*)C + (size_t)first * ldc;
+    W += (size_t)matrix * (HALVES ? 2 * halves.width : N) * ldw;
+    C = HALVES ? (void*)((bf16*)C + (size_t)first * ldc) : (void*)((float*)C + (size_t)first * ldc);
     bm = 0;
   }
   const int m0 = bm * BM, n0 = bn * BN;
@@ -576,7 +607,7 @@ __global__ __launch_bounds__(512, 2) void tile_dma_kernel(const bf16* __restrict
     const int jh = q < LW0 ? J0 : J1, p = (q < LW0 ? q : q - LW0) * 8 + wid;       // 2 jh pieces a column of waves
     const int b = TT::first(p / (2 * jh)) + ((q < LW0 ? 0 : J0) + (p % (2 * jh)) / 2) * TT::STEP;
     const int r0 = b * 16 + (p & 1) * 8, r = r0 + (lane >> 3);
-    gw[q] = ((unsigned)min(n0 + r, N - 1) * (unsigned)ldw + ((lane & 7) ^ ((r >> 1) & 7)) * 8) * 2u;
+    gw[q] = ((unsigned)(HALVES ? halves.row(n0 + r) : min(n0 + r, N - 1)) * (unsigned)ldw + ((lane & 7) ^ ((r >> 1) & 7)) * 8) * 2u;
     lw[q] = lds0 + W_AT + r0 * ROW;
   }
   auto copy_a = [&](int kt, int st, auto HALF) {
@@ -699,7 +730,7 @@ __global__ __launch_bounds__(512, 2) void tile_dma_kernel(const bf16* __restrict
   if (grp == 0) dma_meet();
   dma_wait<0>();
   dma_meet();
-  dma_epilogue<TT>(acc, smem + wid * TT::OWN, bias, C, ldc, M, N, epi, m0 + wave_m * TT::ROWS, n0, wave_n, lane);
+  dma_epilogue<TT, HALVES>(acc, smem + wid * TT::OWN, bias, C, ldc, M, N, HALVES ? EPI_SWIGLU : epi, m0 + wave_m * TT::ROWS, n0, wave_n, lane, halves);
 }
 
 // The sum of a row's `parts` numbers by LANES lanes that stand side by side (l: the lane's place among them), in two steps so that a
@@ -767,7 +798,7 @@ struct StepTile {
 
 // SCALED: the rows' sums are multiplied by 1 / sqrt(mean + eps) of the row, `in_parts` partial sums of squares of which stand
 // in in_ssq [M][in_parts] (FusedNorm::in_*; one launch, K whole).
-template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, bool GROUPED = false, bool SCALED = false>
+template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, bool GROUPED = false, bool SCALED = false, bool HALVES = false>
 __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void tile_step_kernel(const bf16* __restrict__ A, int lda,
                                                        const bf16* __restrict__ W, int ldw,
                                                        const float* __restrict__ bias, void* __restrict__ C,
@@ -775,7 +806,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void tile_step_kernel(const
                                                        int order, int k_per_split,
                                                        const RowGroup* __restrict__ groups = nullptr,
                                                        const float* __restrict__ in_ssq = nullptr, int in_parts = 0,
-                                                       float in_eps = 0.f) {
+                                                       float in_eps = 0.f, Halves halves = Halves{}) {
   using TT = StepTile<BM, BN, WAVES_M, WAVES_N>;
   constexpr int ROW = DMA_BK * 2, ST = (BM + BN) * ROW, WAVES = TT::WAVES, I = TT::I, J = TT::J, LA = TT::LA, LW = TT::LW;
   int tile, part;
@@ -794,8 +825,8 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void tile_step_kernel(const
     const int first = __builtin_amdgcn_readfirstlane(groups[bm].first), matrix = __builtin_amdgcn_readfirstlane(groups[bm].matrix);
     M = __builtin_amdgcn_readfirstlane(groups[bm].rows);
     A += (size_t)first * lda;
-    W += (size_t)matrix * N * ldw;
-    C = (float*)C + (size_t)first * ldc;
+    W += (size_t)matrix * (HALVES ? 2 * halves.width : N) * ldw;
+    C = HALVES ? (void*)((bf16*)C + (size_t)first * ldc) : (void*)((float*)C + (size_t)first * ldc);
     bm = 0;
   }
   const int m0 = bm * BM, n0 = bn * BN;
@@ -818,7 +849,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void tile_step_kernel(const
 #pragma unroll
   for (int q = 0; q < LW; ++q) {
     const int r = (q * WAVES + wid) * 8 + (lane >> 3);
-    gw[q] = ((unsigned)min(n0 + r, N - 1) * (unsigned)ldw + ((lane & 7) ^ ((r >> 1) & 7)) * 8) * 2u;
+    gw[q] = ((unsigned)(HALVES ? halves.row(n0 + r) : min(n0 + r, N - 1)) * (unsigned)ldw + ((lane & 7) ^ ((r >> 1) & 7)) * 8) * 2u;
   }
   const int nkt = K / DMA_BK;
   auto copy = [&](int kt, int st) {                          // (past the last tile: that one again, never read)
@@ -911,15 +942,15 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void tile_step_kernel(const
       for (int j = 0; j < J; ++j) acc[i][j] *= f;
     }
   }
-  dma_epilogue<TT>(acc, smem + wid * TT::OWN, bias, C, ldc, M, N, epi, m0 + wave_m * TT::ROWS, n0, wave_n, lane);
+  dma_epilogue<TT, HALVES>(acc, smem + wid * TT::OWN, bias, C, ldc, M, N, HALVES ? EPI_SWIGLU : epi, m0 + wave_m * TT::ROWS, n0, wave_n, lane, halves);
 }
 
-template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, bool GROUPED, bool SCALED = false>
+template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, bool GROUPED, bool SCALED = false, bool HALVES = false>
 int launch_tile_step(const bf16* A, int lda, const bf16* W, int ldw, const float* bias, void* C, int ldc, int M, int N, int K, int epi,
                      hipStream_t stream, int splits, int k_per_split, const RowGroup* groups, int n_groups,
-                     const float* in_ssq = nullptr, int in_parts = 0, float in_eps = 0.f) {
+                     const float* in_ssq = nullptr, int in_parts = 0, float in_eps = 0.f, const Halves& halves = Halves{}) {
   using TT = StepTile<BM, BN, WAVES_M, WAVES_N>;
-  auto kern = tile_step_kernel<BM, BN, WAVES_M, WAVES_N, STAGES, GROUPED, SCALED>;
+  auto kern = tile_step_kernel<BM, BN, WAVES_M, WAVES_N, STAGES, GROUPED, SCALED, HALVES>;
   static bool configured = false;
   if (!configured) {
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -929,7 +960,7 @@ int launch_tile_step(const bf16* A, int lda, const bf16* W, int ldw, const float
   }
   const int tiles_m = GROUPED ? n_groups : (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
   kern<<<dim3(tiles_m * tiles_n, splits), 64 * TT::WAVES, TT::template lds<STAGES>(), stream>>>(
-      A, lda, W, ldw, bias, C, ldc, M, N, K, epi, tiles_m, tile_order(tiles_m * tiles_n, splits, M, N, K), k_per_split, groups, in_ssq, in_parts, in_eps);
+      A, lda, W, ldw, bias, C, ldc, M, N, K, epi, tiles_m, tile_order(tiles_m * tiles_n, splits, M, N, K), k_per_split, groups, in_ssq, in_parts, in_eps, halves);
   return mf_launch_status();
 }
 
@@ -941,11 +972,11 @@ int launch_tile64(const bf16* A, int lda, const bf16* W, int ldw, const float* b
                                                           nullptr, 0, in_ssq, in_parts, in_eps);
 }
 
-template <int BM, int BN, int STAGES, bool GROUPED>
+template <int BM, int BN, int STAGES, bool GROUPED, bool HALVES = false>
 int configure_tile_dma() {
   static bool configured = false;
   if (configured) return 0;
-  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(tile_dma_kernel<BM, BN, STAGES, GROUPED>),
+  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(tile_dma_kernel<BM, BN, STAGES, GROUPED, HALVES>),
                                            hipFuncAttributeMaxDynamicSharedMemorySize, DmaTile<BM, BN>::template lds<STAGES>());
   configured = e == hipSuccess;
   return (int)e;
@@ -990,14 +1021,25 @@ int launch_tile(const bf16* A, int lda, const bf16* W, int ldw, const float* bia
                                                            splits, k_per_split);
 }
 
-// The grouped forms: a tile row per entry of `groups` (int32 [n_groups][4] on the device), 32-bit sums stored.
-template <int BM, int BN, int STAGES>
-int launch_grouped_dma(const bf16* A, int lda, const bf16* W, int ldw, float* C, int ldc, const RowGroup* groups, int n_groups,
-                       int N, int K, hipStream_t stream) {
-  if (const int e = configure_tile_dma<BM, BN, STAGES, true>()) return e;
+// The grouped forms: a tile row per entry of `groups` (int32 [n_groups][4] on the device), 32-bit sums stored; or, of matrices of gate
+// and up rows (HALVES), the activation's values in bfloat16.
+template <int BM, int BN, int STAGES, bool HALVES = false>
+int launch_grouped_dma(const bf16* A, int lda, const bf16* W, int ldw, void* C, int ldc, const RowGroup* groups, int n_groups,
+                       int N, int K, hipStream_t stream, const Halves& halves = Halves{}) {
+  if (const int e = configure_tile_dma<BM, BN, STAGES, true, HALVES>()) return e;
   const int tiles_n = (N + BN - 1) / BN;
-  tile_dma_kernel<BM, BN, STAGES, true><<<dim3(n_groups * tiles_n), 512, DmaTile<BM, BN>::template lds<STAGES>(), stream>>>(
-      A, lda, W, ldw, nullptr, C, ldc, 0, N, K, EPI_F32, n_groups, n_groups * tiles_n >= 16, 0, groups);
+  tile_dma_kernel<BM, BN, STAGES, true, HALVES><<<dim3(n_groups * tiles_n), 512, DmaTile<BM, BN>::template lds<STAGES>(), stream>>>(
+      A, lda, W, ldw, nullptr, C, ldc, 0, N, K, EPI_F32, n_groups, n_groups * tiles_n >= 16, 0, groups, halves);
+  return mf_launch_status();
+}
+
+// one product of gate and up rows
+template <int BM, int BN, int STAGES>
+int launch_halves_dma(const bf16* A, int lda, const bf16* W, int ldw, bf16* C, int M, int N, int K, const Halves& halves, hipStream_t stream) {
+  if (const int e = configure_tile_dma<BM, BN, STAGES, false, true>()) return e;
+  const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
+  tile_dma_kernel<BM, BN, STAGES, false, true><<<dim3(tiles_m * tiles_n), 512, DmaTile<BM, BN>::template lds<STAGES>(), stream>>>(
+      A, lda, W, ldw, nullptr, C, halves.width, M, N, K, EPI_SWIGLU, tiles_m, tile_order(tiles_m * tiles_n, 1, M, N, K), 0, nullptr, halves);
   return mf_launch_status();
 }
 
@@ -2474,7 +2516,7 @@ __global__ __launch_bounds__(512, 2) void panel_dma_kernel(const bf16* __restric
     }
     return;
   }
-  const bool half = epi == EPI_BF16 || epi == EPI_XIELU;
+  const bool half = epi == EPI_BF16 || epi == EPI_XIELU || epi == EPI_RELU2;
   const bool vec = ldc % 4 == 0 && (uintptr_t)C % (half ? 8 : 16) == 0;
   for (int x = threadIdx.x; x < M * (BN / 4); x += 512) {
     const int r = x / (BN / 4), c = (x % (BN / 4)) * 4, n = u0 * 32 + c;
@@ -2486,7 +2528,7 @@ __global__ __launch_bounds__(512, 2) void panel_dma_kernel(const bf16* __restric
     if (vec && n + 4 <= N && half) {
       bf16x4 h;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) h[e] = (bf16)(epi == EPI_XIELU ? xielu_f(v[e], bias[N], bias[N + 1]) : v[e]);
+      for (int e = 0; e < 4; ++e) h[e] = (bf16)(epi == EPI_XIELU ? xielu_f(v[e], bias[N], bias[N + 1]) : epi == EPI_RELU2 ? relu2_f(v[e]) : v[e]);
       *reinterpret_cast<bf16x4*>((bf16*)C + (size_t)r * ldc + n) = h;
     } else if (vec && n + 4 <= N) {
       float4* o = reinterpret_cast<float4*>((float*)C + (size_t)r * ldc + n);
@@ -2573,8 +2615,8 @@ __global__ __launch_bounds__(256) void skinny_reduce_kernel(const float* __restr
     v = sum_of_parts(part, stride, (size_t)m * N + n, splits) * rf + (bias ? bias[n] : 0.f);
     if (epi == EPI_XIELU) {
       ((bf16*)C)[(size_t)m * ldc + n] = (bf16)xielu_f(v, bias[N], bias[N + 1]);
-    } else if (epi == EPI_BF16) {
-      ((bf16*)C)[(size_t)m * ldc + n] = (bf16)v;
+    } else if (epi == EPI_BF16 || epi == EPI_RELU2) {
+      ((bf16*)C)[(size_t)m * ldc + n] = (bf16)(epi == EPI_RELU2 ? relu2_f(v) : v);
     } else {
       float* c = (float*)C + (size_t)m * ldc + n;
       if (epi == EPI_ACC_F32) v += *c;
@@ -2636,6 +2678,9 @@ __global__ __launch_bounds__(256) void skinny_reduce4_kernel(const float* __rest
       bf16* c = (bf16*)C + (size_t)m * ldc + n;
       c[0] = (bf16)xielu_f(v.x, ap, an); c[1] = (bf16)xielu_f(v.y, ap, an);
       c[2] = (bf16)xielu_f(v.z, ap, an); c[3] = (bf16)xielu_f(v.w, ap, an);
+    } else if (epi == EPI_RELU2) {
+      bf16* c = (bf16*)C + (size_t)m * ldc + n;
+      c[0] = (bf16)relu2_f(v.x); c[1] = (bf16)relu2_f(v.y); c[2] = (bf16)relu2_f(v.z); c[3] = (bf16)relu2_f(v.w);
     } else if (epi == EPI_BF16) {
       bf16* c = (bf16*)C + (size_t)m * ldc + n;
       c[0] = (bf16)v.x; c[1] = (bf16)v.y; c[2] = (bf16)v.z; c[3] = (bf16)v.w;
@@ -2950,7 +2995,7 @@ TilePlan plan_tiles(int M, int N, int K, bool dma_ok, int epi, int n_cu) {
   const long cu = n_cu > 0 ? n_cu : 1;
   const long nkt = (K + 63) / 64, chunks = (K + 255) / 256;
   const double mn = (double)M * (double)N;
-  const double epi_us = (epi == EPI_ACC_F32 ? 8. : epi == EPI_F32 ? 4. : (epi == EPI_BF16 || epi == EPI_XIELU) ? 2. : 1.) * mn / 4e6;
+  const double epi_us = (epi == EPI_ACC_F32 ? 8. : epi == EPI_F32 ? 4. : (epi == EPI_BF16 || epi == EPI_XIELU || epi == EPI_RELU2) ? 2. : 1.) * mn / 4e6;
   // The kernels through registers have costs of their own: a launch's epilogue is a chain (SwiGLU's stores 4 us, of 16 or 32
   // bits 7, a read and a store 25), the second kernel of a SwiGLU product adds its parts one value at a time, and rows that are
   // no whole 16 bytes are read in eights of single values.  1,888 products of K not in 64s, from 65 x 192 x 100 on: the choice is
@@ -3101,6 +3146,57 @@ MF_API int mf_gemm_bf16_grouped(const void* A, const void* W, float* C, const in
   return (int)hipErrorInvalidValue;
 }
 
+static bool halves_ok(const Halves& h, const void* C, int K, size_t rows, int ld) {
+  return h.width > 0 && C && K > 0 && K % DMA_BK == 0 && rows * (size_t)ld * 2 < (1ull << 32);
+}
+
+// The same of matrices whose rows are `width` gates and then `width` ups (W [matrices][2 width][K]): C [rows][width] =
+// act(gate, up) in bfloat16 from the 32-bit sums, the activations being those of `mf_moe_act` (act 1: silu(gate) up, else the clamped
+// form with `limit`).  No 32-bit intermediate and no kernel of its own for the activation: 2,048 rows over 8 matrices of 8,192 x
+// 2,048 117 + 24 us as two kernels, 120 so (what the smaller stores save, the exponentials take).
+MF_API int mf_gemm_bf16_grouped_gated(const void* A, const void* W, void* C, const int* groups, int n_groups, int width, int K,
+                                      int variant, int act, float limit, hipStream_t stream) {
+  if (n_groups <= 0 || width <= 0) return 0;
+  const Halves h{width, act == 1, limit, nullptr, 0};
+  if (!halves_ok(h, C, K, 2 * (size_t)width, K) || !groups || (uintptr_t)A % 16 || (uintptr_t)W % 16) return (int)hipErrorInvalidValue;
+  const bf16* a = (const bf16*)A;
+  const bf16* w = (const bf16*)W;
+  const RowGroup* g = (const RowGroup*)groups;
+  const int N = (width + 31) / 32 * 64;
+  switch (variant) {
+    case 2:
+      return launch_tile_step<128, 128, 2, 4, 4, true, false, true>(a, K, w, K, nullptr, C, width, 0, N, K, EPI_SWIGLU, stream, 1, 0, g, n_groups,
+                                                                    nullptr, 0, 0.f, h);
+    case 12: return launch_grouped_dma<256, 256, 2, true>(a, K, w, K, C, width, g, n_groups, N, K, stream, h);
+    case 13: return launch_grouped_dma<256, 128, 3, true>(a, K, w, K, C, width, g, n_groups, N, K, stream, h);
+  }
+  return (int)hipErrorInvalidValue;
+}
+
+// One product of that form, M rows, with a factor sigmoid(z) of every row (z [M], ldz apart; null: none): C [M][width].  2,048 rows of
+// 8,192 x 2,048: 62 + 19 us as two kernels, 64 so.
+MF_API int mf_gemm_bf16_gated(const void* A, int lda, const void* W, int ldw, void* C, int M, int width, int K, int act, float limit,
+                              const float* z, int ldz, hipStream_t stream) {
+  if (M <= 0 || width <= 0) return 0;
+  const Halves h{width, act == 1, limit, z, ldz};
+  if (lda < K || ldw < K || lda % 8 || ldw % 8 || !halves_ok(h, C, K, 2 * (size_t)width, ldw) || (size_t)M * lda * 2 >= (1ull << 32) ||
+      (uintptr_t)A % 16 || (uintptr_t)W % 16)
+    return (int)hipErrorInvalidValue;
+  const bf16* a = (const bf16*)A;
+  const bf16* w = (const bf16*)W;
+  bf16* c = (bf16*)C;
+  const int N = (width + 31) / 32 * 64, cu = cu_count();
+  if (cu <= 0) return (int)hipErrorUnknown;
+  const long nkt = K / DMA_BK;
+  int form = FORM_256;
+  for (int f : {FORM_128, FORM_SMALL})
+    if (form_us(f, M, N, nkt, 1, cu) < form_us(form, M, N, nkt, 1, cu)) form = f;
+  if (form == FORM_256) return launch_halves_dma<256, 256, 2>(a, lda, w, ldw, c, M, N, K, h, stream);
+  if (form == FORM_128) return launch_halves_dma<256, 128, 3>(a, lda, w, ldw, c, M, N, K, h, stream);
+  return launch_tile_step<128, 128, 2, 4, 4, false, false, true>(a, lda, w, ldw, nullptr, c, width, M, N, K, EPI_SWIGLU, stream, 1, 0, nullptr, 0,
+                                                                 nullptr, 0, 0.f, h);
+}
+
 // `variant`: 0 picks by shape among the whole-K kernels; 1: 256x256 tile with 4 waves, 2: 128x128,
 // 3: 64x64, 6: 256x128 with 8 waves, 9: 256x256 with 8 waves; through the direct-to-LDS pipeline, K in
 // 64s: 12: 256x256 (SwiGLU: or 256x192), 13: the cheapest of 256x128, 128x256, 128x128 and 64x64 (or the
@@ -3110,7 +3206,7 @@ MF_API int mf_gemm_bf16_grouped(const void* A, const void* W, float* C, const in
 MF_API int mf_gemm_bf16(const void* A, int lda, const void* W, int ldw, const float* bias, void* C,
                         int ldc, int M, int N, int K, int epi, int variant, hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
-  if (K <= 0 || lda < K || ldw < K || epi < 0 || epi > EPI_XIELU || (epi == EPI_XIELU && !bias)) return (int)hipErrorInvalidValue;
+  if (K <= 0 || lda < K || ldw < K || epi < 0 || epi > EPI_LAST || (epi == EPI_XIELU && !bias)) return (int)hipErrorInvalidValue;
   if (epi == EPI_SWIGLU ? (N % 64 != 0 || ldc > N / 2 || ldc <= N / 2 - 32) : ldc < N)
     return (int)hipErrorInvalidValue;
   const int vec_ok = (lda % 8 == 0) && (ldw % 8 == 0) && ((uintptr_t)A % 16 == 0) &&
@@ -3180,7 +3276,7 @@ MF_API int mf_gemm_bf16_splitk(const void* A, int lda, const void* W, int ldw, c
                                int ldc, float* part, int M, int N, int K, int splits, int k_per_split,
                                int epi, int variant, hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
-  if (epi < 0 || epi > EPI_XIELU || (epi == EPI_XIELU && !bias)) return (int)hipErrorInvalidValue;
+  if (epi < 0 || epi > EPI_LAST || (epi == EPI_XIELU && !bias)) return (int)hipErrorInvalidValue;
   if (epi == EPI_SWIGLU ? (N % 64 != 0 || ldc > N / 2 || ldc <= N / 2 - 32) : ldc < N)
     return (int)hipErrorInvalidValue;
   const int rc = mf_gemm_bf16_parts(A, lda, W, ldw, part, M, N, K, splits, k_per_split, variant, stream);
@@ -3238,7 +3334,7 @@ static int skinny_product(const void* A, int lda, const void* W, const void* Wt,
                           void* C, int ldc, float* part, int M, int N, int K, int splits, int k_per_split, int epi,
                           const FusedNorm& fused, hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
-  if (M > 64 || K <= 0 || lda < K || ldw < K || epi < 0 || epi > EPI_XIELU || (epi == EPI_XIELU && !bias) || splits < 1 ||
+  if (M > 64 || K <= 0 || lda < K || ldw < K || epi < 0 || epi > EPI_LAST || (epi == EPI_XIELU && !bias) || splits < 1 ||
       k_per_split % KC != 0 || (long)splits * k_per_split < K || (splits > 1 && !part))
     return (int)hipErrorInvalidValue;
   if (epi == EPI_SWIGLU ? (N % 64 != 0 || ldc > N / 2 || ldc <= N / 2 - 32 || (M > 16 && !part))
@@ -3340,7 +3436,7 @@ MF_API int mf_gemm_bf16_normed(const float* x, int ldx, const int* row_idx, cons
                                const void* W, const void* Wt, int ldw, const float* bias, void* C, int ldc, int M,
                                int N, int K, int epi, hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
-  if (K <= 0 || epi < 0 || epi > EPI_XIELU || (epi == EPI_XIELU && !bias)) return (int)hipErrorInvalidValue;
+  if (K <= 0 || epi < 0 || epi > EPI_LAST || (epi == EPI_XIELU && !bias)) return (int)hipErrorInvalidValue;
   if (ldx % 4 != 0 || ldw % 8 != 0 || (uintptr_t)x % 16 != 0 || (uintptr_t)g % 16 != 0 || (uintptr_t)W % 16 != 0)
     return MF_NOT_BUILT;
   const NormArgs norm{g, row_idx, eps};
@@ -3352,7 +3448,7 @@ MF_API int mf_gemm_bf16_normed(const float* x, int ldx, const int* row_idx, cons
 // for mf_gemm_bf16_splitk with out[1] splits of out[2] of K each.  `aligned`: 16-byte aligned
 // operands with row strides and K in multiples of 8.
 MF_API int mf_gemm_bf16_tile_plan(int M, int N, int K, int aligned, int epi, int n_cu, int* out) {
-  if (!out || M <= 0 || N <= 0 || K <= 0 || epi < 0 || epi > EPI_XIELU || n_cu <= 0) return (int)hipErrorInvalidValue;
+  if (!out || M <= 0 || N <= 0 || K <= 0 || epi < 0 || epi > EPI_LAST || n_cu <= 0) return (int)hipErrorInvalidValue;
   const bool dma_ok = aligned && K % DMA_BK == 0 && (size_t)M * K * 2 < (1ull << 32) && (size_t)N * K * 2 < (1ull << 32);
   const TilePlan plan = plan_tiles(M, N, K, dma_ok, epi, n_cu);
   out[0] = plan.variant;
@@ -3369,7 +3465,7 @@ MF_API int mf_gemm_bf16_tile_plan(int M, int N, int K, int aligned, int epi, int
 // plan's own choice, K split or whole); `n_cu`: compute units of the device.
 MF_API int mf_gemm_bf16_plan(int M, int N, int K, int aligned, int tiled, int epi, int splits, int k_per_split,
                              int normed, int variant, int n_cu, char* name, int cap) {
-  if (!name || cap < 48 || M <= 0 || N <= 0 || K <= 0 || epi < 0 || epi > EPI_XIELU || n_cu <= 0) return (int)hipErrorInvalidValue;
+  if (!name || cap < 48 || M <= 0 || N <= 0 || K <= 0 || epi < 0 || epi > EPI_LAST || n_cu <= 0) return (int)hipErrorInvalidValue;
   const char* what = "";
   if (normed) {
     what = (aligned && stationary_takes(M, N, K, epi, true)) ? "stationary16_kernel(norm)" : "";

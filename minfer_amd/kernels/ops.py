@@ -20,7 +20,7 @@ PAGE = 64          # tokens per cache page (MF_PAGE in csrc/common.h)
 HAVE_PREFILL_ATTENTION = True
 PREFILL_MAX_SHARES = 8  # workgroups that may take the pages of one block of queries of the prompt attention in turn
 PREFILL_MIN_PAGES = 4   # ... each with at least this many pages
-EPI_F32, EPI_ACC_F32, EPI_BF16, EPI_SWIGLU, EPI_XIELU = 0, 1, 2, 3, 4
+EPI_F32, EPI_ACC_F32, EPI_BF16, EPI_SWIGLU, EPI_XIELU, EPI_RELU2 = 0, 1, 2, 3, 4, 5
 
 
 class KernelError(RuntimeError):
@@ -136,6 +136,8 @@ _PROTOTYPES = {
     "gemm_bf16": {
         "mf_gemm_bf16": [_P, c_int, _P, c_int, _P, _P, c_int, c_int, c_int, c_int, c_int, c_int, _P],
         "mf_gemm_bf16_grouped": [_P, _P, _P, _P, c_int, c_int, c_int, c_int, _P],
+        "mf_gemm_bf16_grouped_gated": [_P, _P, _P, _P, c_int, c_int, c_int, c_int, c_int, c_float, _P],
+        "mf_gemm_bf16_gated": [_P, c_int, _P, c_int, _P, c_int, c_int, c_int, c_int, c_float, _P, c_int, _P],
         "mf_gemm_bf16_splitk": [_P, c_int, _P, c_int, _P, _P, c_int, _P, c_int, c_int, c_int, c_int, c_int, c_int,
                                 c_int, _P],
         "mf_gemm_bf16_parts": [_P, c_int, _P, c_int, _P, c_int, c_int, c_int, c_int, c_int, c_int, _P],
@@ -1860,11 +1862,12 @@ def _need_tiled(tiled: Optional[torch.Tensor], name: str, n: int, k: int) -> Non
 
 def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], out: torch.Tensor,
            accumulate: bool = False, variant: int = 0, tiled: Optional[torch.Tensor] = None,
-           xielu: bool = False) -> None:
+           xielu: bool = False, relu2: bool = False) -> None:
     """out (+)= x @ weight^T (+ bias).  weight is [out][in].  float32 weights take the true
     32-bit kernel; bfloat16 weights take the matrix-core kernels (a few rows: the streaming
     kernel).  `out` is float32, or bfloat16 for a bfloat16 product that is stored.  `tiled`:
-    `tile_weight(weight)`, which the kernels for at most 64 rows read instead where they can."""
+    `tile_weight(weight)`, which the kernels for at most 64 rows read instead where they can.  `relu2`: a bfloat16 product's
+    sums go through max(z, 0)^2 before they are rounded."""
     _need(x, "linear.x", _FLOATS)
     _need(weight, "linear.weight", x.dtype)
     m, k = x.shape
@@ -1878,6 +1881,8 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], 
         _need(bias, "linear.bias", torch.float32, (n + 2,))
     elif bias is not None:
         _need(bias, "linear.bias", torch.float32, (n,))
+    if relu2 and (xielu or x.dtype != torch.bfloat16 or out.dtype != torch.bfloat16 or accumulate):
+        raise KernelError("linear(relu2): needs bfloat16 operands and output")
     if m == 0:
         return
     if x.dtype == torch.float32:
@@ -1890,7 +1895,7 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], 
         return
     if accumulate and out.dtype != torch.float32:
         raise KernelError("linear: accumulation needs a float32 output")
-    epi = EPI_XIELU if xielu else (EPI_BF16 if out.dtype == torch.bfloat16 else (EPI_ACC_F32 if accumulate else EPI_F32))
+    epi = EPI_XIELU if xielu else EPI_RELU2 if relu2 else (EPI_BF16 if out.dtype == torch.bfloat16 else (EPI_ACC_F32 if accumulate else EPI_F32))
     aligned = not (x.data_ptr() % 16 or weight.data_ptr() % 16 or k % 8)
     if m <= 64 and variant == 0:
         splits, per = _k_split(m, n, k, False, aligned, tiled=tiled is not None)
@@ -2012,6 +2017,48 @@ def linear_grouped(x: torch.Tensor, weights: torch.Tensor, groups: torch.Tensor,
         raise KernelError(f"linear_grouped: matrices [{n}][{k}], variant {variant}, groups {tuple(groups.shape)}")
     _check(_fn("gemm_bf16", "mf_gemm_bf16_grouped")(x, weights, out, groups, groups.shape[0], n, k, variant,
                                                      _stream()), f"gemm_bf16_grouped {rows}x{n}x{k}")
+
+
+def linear_grouped_gated(x: torch.Tensor, weights: torch.Tensor, groups: torch.Tensor, variant: int, out: torch.Tensor, limit: float,
+                         act: int = 0) -> None:
+    """`linear_grouped` of matrices of gate rows and up rows behind them (`[groups][2 f][k]`), then `moe_act` with weights of
+    one, in one kernel: out[r] = act(gate, up), bfloat16 `[rows][f]`."""
+    rows, k = x.shape
+    f = out.shape[1]
+    _need(x, "linear_grouped_gated.x", torch.bfloat16)
+    _need(weights, "linear_grouped_gated.weights", torch.bfloat16, (weights.shape[0], 2 * f, k))
+    _need(groups, "linear_grouped_gated.groups", torch.int32)
+    _need(out, "linear_grouped_gated.out", torch.bfloat16, (rows, f))
+    if not grouped_takes(x.dtype, 2 * f, k) or variant not in GROUPED_TILES or groups.dim() != 2 or groups.shape[1] != 4:
+        raise KernelError(f"linear_grouped_gated: matrices [{2 * f}][{k}], variant {variant}, groups {tuple(groups.shape)}")
+    _check(_fn("gemm_bf16", "mf_gemm_bf16_grouped_gated")(x, weights, out, groups, groups.shape[0], f, k, variant, int(act), float(limit),
+                                                           _stream()), f"gemm_bf16_grouped_gated {rows}x{f}x{k}")
+
+
+def linear_gated_takes(m: int, f: int, k: int) -> bool:
+    """Whether `linear_gated` is the way to a bfloat16 product of `m` rows with f gates and f ups: more rows than the decode
+    kernels take, K in 64s, and tiles enough to fill the chip with K whole (else K is better cut, and the activation behind it)."""
+    return m > 64 and k % 64 == 0 and 2 * f * k * 2 < 1 << 32 and m * k * 2 < 1 << 32 and tile_plan(m, 2 * f, k, EPI_F32)[1] == 1
+
+
+def linear_gated(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor, limit: float = 0.0, act: int = 0,
+                 gate_logits: Optional[torch.Tensor] = None) -> None:
+    """out = act(gate, up), bfloat16 `[m][f]`, of x and a matrix of f gate rows and f up rows behind them, the activations of
+    `moe_act`, from the 32-bit sums; times sigmoid(gate_logits[r][0]) of every row where given (float32 `[m][any]`)."""
+    m, k = x.shape
+    f = out.shape[1]
+    _need(x, "linear_gated.x", torch.bfloat16)
+    _need(weight, "linear_gated.weight", torch.bfloat16, (2 * f, k))
+    _need(out, "linear_gated.out", torch.bfloat16, (m, f))
+    if gate_logits is not None:
+        _need(gate_logits, "linear_gated.gate_logits", torch.float32)
+        if gate_logits.dim() != 2 or gate_logits.shape[0] != m or gate_logits.shape[1] < 1:
+            raise KernelError(f"linear_gated.gate_logits: {tuple(gate_logits.shape)} for {m} rows")
+    if m == 0:
+        return
+    _check(_fn("gemm_bf16", "mf_gemm_bf16_gated")(x, k, weight, k, out, m, f, k, int(act), float(limit), gate_logits,
+                                                   0 if gate_logits is None else gate_logits.shape[1], _stream()),
+           f"gemm_bf16_gated {m}x{f}x{k}")
 
 
 def interleave_gate_up(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:

@@ -184,3 +184,11 @@ class DenseRelu2(DenseGelu):
     @staticmethod
     def activation(u, y):
         ops.relu2(u, y)
+
+    def forward(self, x, h, ctx, accumulate: bool = True) -> None:
+        if isinstance(x, torch.Tensor) and x.device.type == "cuda" and x.dtype == self.up.weight.dtype == self.rt.dtype == torch.bfloat16:
+            y = torch.empty((x.shape[0], self.inter), dtype=torch.bfloat16, device=x.device)
+            ops.linear(x, self.up.weight, None, y, tiled=self.up.tiled, relu2=True)       # (in the product's epilogue)
+            self.down(y, out=h, accumulate=accumulate)
+        else:
+            super().forward(x, h, ctx, accumulate)

@@ -74,9 +74,15 @@ class SharedExpert:
         return self.up.decode_copy(make, min_row_length) + self.down.decode_copy(make, min_row_length)
 
     def forward(self, x, h, accumulate: bool) -> None:
-        gu = self.up(x, out_dtype=torch.float32)
         y = torch.empty((x.shape[0], self.inter), dtype=self.rt.dtype, device=x.device)
-        ops.gated_expert_act(gu, y)
+        w, pairs = self.up.weight, 2 * self.inter
+        if x.device.type == "cuda" and x.dtype == w.dtype == y.dtype == torch.bfloat16 and ops.linear_gated_takes(x.shape[0], self.inter, self.hidden):
+            # many rows: the rows' own sigmoids first, then the activation in the product's epilogue
+            z = torch.empty((x.shape[0], w.shape[0] - pairs), dtype=torch.float32, device=x.device)
+            ops.linear(x, w[pairs:], None, z)
+            ops.linear_gated(x, w[:pairs], y, act=ops.MOE_ACTS["silu"], gate_logits=z)
+        else:
+            ops.gated_expert_act(self.up(x, out_dtype=torch.float32), y)
         self.down(y, out=h, accumulate=accumulate)
 
 
@@ -181,7 +187,6 @@ class Experts(FeedForward):
         offsets, at = meta[:self.ne], (self.ne + 3) // 4 * 4
         xs = torch.empty((pairs, self.hidden), dtype=x.dtype, device=dev)
         ops.moe_gather(x, chosen, rank, offsets, xs, n_real=self.ne if self.identity else None)
-        gu = torch.empty((pairs, 2 * self.inter), dtype=torch.float32, device=dev)
         y = torch.empty((pairs, self.inter), dtype=self.rt.dtype, device=dev)
         rows = torch.empty((pairs, self.hidden), dtype=torch.float32, device=dev)
         if pairs == 0:
@@ -189,10 +194,10 @@ class Experts(FeedForward):
         elif grouped:
             sizes = [4 * len(t) for t in tables]
             up_groups, down_groups = (meta[at + o:at + o + s].view(-1, 4) for o, s in zip((0, sizes[0]), sizes))
-            ops.linear_grouped(xs, self.gate_up, up_groups, plans[0], gu)
-            ops.moe_act(gu, self._ones(pairs, dev), y, self.limit, self.act)
+            ops.linear_grouped_gated(xs, self.gate_up, up_groups, plans[0], y, self.limit, self.act)
             ops.linear_grouped(y, self.down, down_groups, plans[1], rows)
         else:
+            gu = torch.empty((pairs, 2 * self.inter), dtype=torch.float32, device=dev)
             for e, (gate_up, _) in enumerate(self.experts):
                 if per_expert[e]:
                     gate_up(xs[starts[e]:starts[e + 1]], out=gu[starts[e]:starts[e + 1]])
