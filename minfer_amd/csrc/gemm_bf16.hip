@@ -1680,11 +1680,11 @@ int launch_skinny16(const bf16* A, int lda, const bf16* W, int ldw, const float*
 // and 0.175 us for each of a wave's loads, blocks of a CU added up (measured over 12 shapes of 896 to 18,944, 20 to 64 rows).
 // Hence the choice of `whole_plan`.  q|k|v and o of 32 rows, this / K split or 64 x 64 tiles: 1,152 x 896 3.8 / 8.5 us, 896 x 896
 // 4.3 / 10.2, 2,048 x 1,536 4.7 / 10.5, 2,560 x 2,048 5.9 / 10.7; 896 x 4,864 9.2 / 11.0.
-template <int MT, int NT, int S>
-__global__ __launch_bounds__(512) void whole_kernel(const bf16* __restrict__ A, int lda, const bf16* __restrict__ W,
+template <int MT, int NT, int S, bool TILED>
+__global__ __launch_bounds__(512) void whole_kernel(const bf16* __restrict__ A, int lda, const bf16* __restrict__ W, int ldw,
                                                     const float* __restrict__ bias, float* __restrict__ C, int ldc, int M, int N, int K,
                                                     int accumulate, int rpb, FusedNorm fused) {
-  constexpr int NW = 8, COLS = 16 * NT, RS = COLS + 4, ROWS = 16 * MT;
+  constexpr int NW = 8, COLS = 16 * NT, RS = COLS + 4, ROWS = 16 * MT, WSTEP = TILED ? 512 : 32;
   __shared__ float red[NW][ROWS][RS];
   const int lane = threadIdx.x & 63, r16 = lane & 15;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1697,7 +1697,7 @@ __global__ __launch_bounds__(512) void whole_kernel(const bf16* __restrict__ A, 
 #pragma unroll
   for (int i = 0; i < MT; ++i) arow[i] = A + (size_t)min(m0 + i * 16 + r16, M - 1) * lda + kq;
 #pragma unroll
-  for (int j = 0; j < NT; ++j) wrow[j] = w_operand<true>(W, 0, K, min(n0 + min(j * 16 + r16, rpb - 1), N - 1), kq);
+  for (int j = 0; j < NT; ++j) wrow[j] = w_operand<TILED>(W, ldw, K, min(n0 + min(j * 16 + r16, rpb - 1), N - 1), kq);
   // the epilogue's places of this lane, what it needs of them asked for in front of the stream
   constexpr int PER_WAVE = 64 / COLS, PASS = NW * PER_WAVE, PASSES = (ROWS + PASS - 1) / PASS;
   const int e_c = lane % COLS, e_n = n0 + e_c;
@@ -1722,7 +1722,7 @@ __global__ __launch_bounds__(512) void whole_kernel(const bf16* __restrict__ A, 
   bf16x8 a[S][MT], w[S][NT];
   auto load = [&](int s, int at) {
 #pragma unroll
-    for (int j = 0; j < NT; ++j) w[s][j] = *reinterpret_cast<const bf16x8*>(wrow[j] + (size_t)at * 512);
+    for (int j = 0; j < NT; ++j) w[s][j] = *reinterpret_cast<const bf16x8*>(wrow[j] + (size_t)at * WSTEP);
 #pragma unroll
     for (int i = 0; i < MT; ++i) a[s][i] = *reinterpret_cast<const bf16x8*>(arow[i] + at * 32);
   };
@@ -1813,19 +1813,21 @@ WholePlan whole_plan(int M, int N, int K, int n_cu) {
   return best;
 }
 // Up to 38 loads, where both ways take some 10 us: 896 x 4,864 (38) 9.2 here and 11.0 with K split, 3,584 x 3,584 at 32 rows (42) 11.9
-// and 12.5, 1,536 x 8,960 (70) 16.3 and 13.4.
-bool whole_takes(int M, int N, int K, bool aligned, bool tiled, int epi, int n_cu) {
-  if (M <= 16 || M > 64 || !aligned || !tiled || K % 32 || n_cu <= 0 || (epi != EPI_F32 && epi != EPI_ACC_F32)) return false;
+// and 12.5, 1,536 x 8,960 (70) 16.3 and 13.4.  Whole tiles of weight rows, and not few: below 512 no model has them and a block's share
+// is a row or two.  (With the tiled copy or without, the same sums: the choice does not ask for it.)
+bool whole_takes(int M, int N, int K, bool aligned, int epi, int n_cu) {
+  if (M <= 16 || M > 64 || !aligned || N < 512 || N % 16 || K % 32 || n_cu <= 0 || (epi != EPI_F32 && epi != EPI_ACC_F32)) return false;
   return whole_plan(M, N, K, n_cu).loads <= 38;
 }
 
-int launch_whole(const bf16* A, int lda, const bf16* Wt, const float* bias, float* C, int ldc, int M, int N, int K, int epi,
+template <bool TILED>
+int launch_whole(const bf16* A, int lda, const bf16* W, int ldw, const float* bias, float* C, int ldc, int M, int N, int K, int epi,
                  const FusedNorm& fused, hipStream_t stream) {
   const WholePlan p = whole_plan(M, N, K, cu_count());
   if (fused.out_g && fused.out_parts < p.gx) return MF_NOT_BUILT;
   auto run = [&](auto MT, auto NT) {
-    whole_kernel<decltype(MT)::value, decltype(NT)::value, 8>
-        <<<dim3(p.gx, p.gy), 512, 0, stream>>>(A, lda, Wt, bias, C, ldc, M, N, K, epi == EPI_ACC_F32, p.rpb, fused);
+    whole_kernel<decltype(MT)::value, decltype(NT)::value, 8, TILED>
+        <<<dim3(p.gx, p.gy), 512, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi == EPI_ACC_F32, p.rpb, fused);
   };
   using One = std::integral_constant<int, 1>;
   using Two = std::integral_constant<int, 2>;
@@ -3346,8 +3348,9 @@ static int skinny_product(const void* A, int lda, const void* W, const void* Wt,
   const bf16* w = (const bf16*)W;
   const bf16* wt = (K % 32 == 0 && (uintptr_t)Wt % 16 == 0) ? (const bf16*)Wt : nullptr;
   const bool folds = fused.in_ssq || fused.out_g;
-  if (folds && whole_takes(M, N, K, vec_ok, wt != nullptr, epi, cu_count()))
-    return launch_whole(a, lda, wt, bias, (float*)C, ldc, M, N, K, epi, fused, stream);
+  if (folds && whole_takes(M, N, K, vec_ok, epi, cu_count()))
+    return wt ? launch_whole<true>(a, lda, wt, ldw, bias, (float*)C, ldc, M, N, K, epi, fused, stream)
+              : launch_whole<false>(a, lda, w, ldw, bias, (float*)C, ldc, M, N, K, epi, fused, stream);
   const SkinnyChoice choice = skinny_choice(M, N, K, vec_ok, wt != nullptr, epi, splits, k_per_split, cu_count());
   // at most 16 rows: the register-resident kernel takes a prepared norm and prepares the next one, the
   // rolling kernel prepares the next one; the K-split kernels' second kernel counts its parts otherwise
@@ -3422,10 +3425,10 @@ MF_API int mf_gemm_bf16_skinny_fused(const void* A, int lda, const void* W, cons
 }
 
 // The partial sums of squares a row that `mf_gemm_bf16_skinny_fused` leaves with out_* where one kernel over the whole of K takes
-// the product of 17 to 64 rows (aligned operands and the tiled copy given): one for each of its blocks; 0 where it does not.
+// the product of 17 to 64 rows (aligned operands): one for each of its blocks; 0 where it does not.
 MF_API int mf_gemm_bf16_whole_parts(int M, int N, int K, int n_cu) {
   if (M <= 0 || N <= 0 || K <= 0 || n_cu <= 0) return 0;
-  return whole_takes(M, N, K, K % 8 == 0, true, EPI_ACC_F32, n_cu) ? whole_plan(M, N, K, n_cu).gx : 0;
+  return whole_takes(M, N, K, K % 8 == 0, EPI_ACC_F32, n_cu) ? whole_plan(M, N, K, n_cu).gx : 0;
 }
 
 // RMS norm of rows of the 32-bit residual stream x (row m of the product is x[row_idx[m]]), then

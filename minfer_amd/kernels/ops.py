@@ -2173,20 +2173,20 @@ NORM_AHEAD_16_WIDTHS = (3072, 5120)
 
 @functools.lru_cache(maxsize=4096)
 def _whole_parts(m: int, n: int, k: int, n_cu: int) -> int:
-    """Workgroups in a row of the one kernel over the whole of K that takes a fused product of 17 to 64 rows with the tiled
-    copy, as the library decides it; 0: K is cut over blocks."""
+    """Workgroups in a row of the one kernel over the whole of K that takes a fused product of 17 to 64 rows, as the library
+    decides it; 0: K is cut over blocks."""
     return _fn("gemm_bf16", "mf_gemm_bf16_whole_parts")(m, n, k, n_cu)
 
 
-def norm_sum_parts(n: int, m: int = 64, k: int = 0, tiled: bool = False) -> int:
+def norm_sum_parts(n: int, m: int = 64, k: int = 0) -> int:
     """Partial sums of squares a row of `n` values comes with from a product of `m` rows (see
     `linear_fused`): one per run of 256 columns from 17 rows on (the kernel that adds the parts of a K
     split writes them), one per workgroup of the product's one kernel for at most 16 rows, and from 17 rows on where
-    the product over a K of `k`, given the tiled copy of its weights (`tiled`), is one kernel."""
+    the product over a K of `k` is one kernel (0: not said; the runs)."""
     runs = (n + NORM_SUM_RUN - 1) // NORM_SUM_RUN
     if m <= 16:
         return max(cu_count(), runs)
-    blocks = _whole_parts(m, n, k, cu_count()) if tiled and k else 0
+    blocks = _whole_parts(m, n, k, cu_count()) if k else 0
     return max(runs, (blocks + 3) // 4 * 4)          # (in fours, so that the next product can read them so)
 
 
@@ -2198,7 +2198,7 @@ def linear_fused(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Ten
     it reads its activations in bfloat16, half the bytes, with nothing to convert (at most 16 rows,
     where the norm is otherwise folded into that product's prologue):
 
-    * `norm_out` = (g `[n]`, xg `[m][n]` bfloat16, sums `[m][norm_sum_parts(n, m, k, tiled given)]`): the product stores
+    * `norm_out` = (g `[n]`, xg `[m][n]` bfloat16, sums `[m][norm_sum_parts(n, m, k)]`): the product stores
       or adds into the 32-bit `out` as `linear` does and leaves, beside it, bf16(out g) and the sums
       of out^2 in parts, for the norm with weight g that reads `out` next;
     * `scale_in` = (sums `[m][parts]`, eps): `x` is such an xg, and the product's sums are multiplied
@@ -2243,7 +2243,7 @@ def linear_fused(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Ten
             raise KernelError("linear_fused.norm_out: the product's own output must be float32")
         _need(out_g, "linear_fused.norm_out.g", torch.float32, (n,))
         _need(out_xg, "linear_fused.norm_out.xg", torch.bfloat16, (m, n))
-        _need(out_ssq, "linear_fused.norm_out.sums", torch.float32, (m, norm_sum_parts(n, m, k, tiled is not None)))
+        _need(out_ssq, "linear_fused.norm_out.sums", torch.float32, (m, norm_sum_parts(n, m, k)))
     aligned = not (x.data_ptr() % 16 or weight.data_ptr() % 16 or k % 8)
     splits, per = _k_split(m, n, k, swiglu, aligned, tiled=tiled is not None)
     part = workspace("skinny", splits * m * n, x.device) if (splits > 1 or (swiglu and m > 16)) else None

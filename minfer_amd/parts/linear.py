@@ -124,8 +124,8 @@ class Linear:
         if fold is None or fold[0].numel() != self.out_features:
             return False
         xg = torch.empty(out.shape, dtype=torch.bfloat16, device=out.device)
-        sums = torch.empty((out.shape[0], ops.norm_sum_parts(self.out_features, out.shape[0], self.in_features,
-                                                                  self.tiled is not None)), dtype=torch.float32, device=out.device)
+        sums = torch.empty((out.shape[0], ops.norm_sum_parts(self.out_features, out.shape[0], self.in_features)),
+                           dtype=torch.float32, device=out.device)
         if not ops.linear_fused(x, self.weight, self.bias, out, accumulate=accumulate, tiled=self.tiled,
                                 norm_out=(fold[0], xg, sums)):
             return False
