@@ -2938,6 +2938,17 @@ double rounds_us(long blocks, long slots, double step_us, long nkt, double round
 double form_us(int form, int M, int N, long nkt, int splits, long cu) {
   const DmaForm& f = DMA_FORMS[form];
   const long tiles = (long)((M + f.bm - 1) / f.bm) * ((N + f.bn - 1) / f.bn);
+  if (form == FORM_TINY && nkt * splits < 52) {
+    // Against a K of up to 3,072: blocks of four waves that start at once, two a CU: 0.27 us a k tile while no CU has two, soon 0.52
+    // where some have, no more than the start that every plan pays, and 6 us for a round behind the first; of a K split the
+    // second blocks' stores come late as well.  (Weights from memory, 64 x 64 whole, estimate / measured: 300 x 2,048 x 2,048
+    // 13.6 / 12.1 us, 604 of them 22.5 / 18.9, 604 x 1,536 x 1,536 12.0 / 10.8, 604 x 1,152 x 896 8.9 / 6.7.  Priced like the large tiles
+    // they lost to K split: 300 x 2,048 x 2,048 17.9, 65 x 8,192 x 2,048 15.7 where 64 x 64 take 12.6.)
+    const long slots = cu * f.per_cu, blocks = tiles * splits, rest = blocks % slots;
+    const double last = rest == 0 ? 0. : rest <= cu ? 0.27 : 0.36 + 0.16 * std::min(1., (double)(rest - cu) / 64.);
+    return (double)nkt * ((double)(blocks / slots) * 0.53 + last) - 0.7 + 6. * (double)((blocks - 1) / slots) +
+           (splits > 1 && blocks > cu ? 2.5 : 0.);
+  }
   return rounds_us(tiles * splits, cu * f.per_cu, f.step_us, nkt, ROUND_US, f.low);
 }
 
@@ -2993,7 +3004,16 @@ const char* form_name(int form, bool split) {
 
 int panel_dma_units(int M, int N, int K, int epi, int n_cu);
 
-TilePlan plan_tiles(int M, int N, int K, bool dma_ok, int epi, int n_cu) {
+// What a product with a K of up to 3,072 whole costs beside its own kernel, where the parts of a split would be added by a kernel that
+// runs in any case (`behind`): 1 the rotation, whose second way from memory a split saves, 2 the norm, else a kernel of its own
+// (rmsnorm_kernel: 70 x 896 2.6 us, 604 x 2,048 4.2, 1,200 x 3,584 6.4).  (A longer K is priced without; so are more than 2.2 million
+// results, whose parts cost more than they save: with the norm 1,700 x 2,048 x 1,024 24.0 us whole and 29.5 split.)
+double whole_more(int M, int N, int K, int behind) {
+  const double mn = (double)M * (double)N;
+  return K > 3072 || mn > 2.2e6 || behind == 0 ? 0. : behind == 1 ? 4.5 : 3.2 + mn / 1e6;
+}
+
+TilePlan plan_tiles(int M, int N, int K, bool dma_ok, int epi, int n_cu, int behind = 0) {
   const long cu = n_cu > 0 ? n_cu : 1;
   const long nkt = (K + 63) / 64, chunks = (K + 255) / 256;
   const double mn = (double)M * (double)N;
@@ -3003,7 +3023,8 @@ TilePlan plan_tiles(int M, int N, int K, bool dma_ok, int epi, int n_cu) {
   // no whole 16 bytes are read in eights of single values.  1,888 products of K not in 64s, from 65 x 192 x 100 on: the choice is
   // 0.5 % from the best kernel on average; with the costs of the direct-to-LDS kernels 1.3 %, and SwiGLU of 200 rows against
   // 8,000 of 1,000 34.7 us in two parts for 21.2 whole.
-  const double start_us = dma_ok ? 4. : epi == EPI_ACC_F32 ? 25. : epi == EPI_SWIGLU ? 4. : 7.;
+  const double more_us = dma_ok ? whole_more(M, N, K, behind) : 0.;
+  const double start_us = more_us + (dma_ok ? 4. : epi == EPI_ACC_F32 ? 25. : epi == EPI_SWIGLU ? 4. : 7.);
   const double slow = K % 8 ? 4. : 1.;
   auto tiles = [&](int bm, int bn) { return (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
   auto cut = [&](long parts, int& splits, int& per) {          // K in `parts` runs of whole chunks of 256
@@ -3029,7 +3050,7 @@ TilePlan plan_tiles(int M, int N, int K, bool dma_ok, int epi, int n_cu) {
     if (epi != EPI_SWIGLU) offer(15, 1, K, form(15, 1, nkt) + start_us + epi_us);
     if (const int n0 = main_rows(N, epi))
       offer(16, 1, K, form_us(best_form(0, N_FORMS - 1, M, n0, nkt, 1, cu), M, n0, nkt, 1, cu) +
-                          form_us(best_form(FORM_128, FORM_TINY, M, N - n0, nkt, 1, cu), M, N - n0, nkt, 1, cu) + 2 * start_us + epi_us);
+                          form_us(best_form(FORM_128, FORM_TINY, M, N - n0, nkt, 1, cu), M, N - n0, nkt, 1, cu) + 2 * start_us - more_us + epi_us);
     // many rows against few weight rows and a long K (the down product of a prompt): K cut over
     // the big tiles, each part at least 2,048 of K
     if (epi != EPI_SWIGLU && M >= 768)
@@ -3449,11 +3470,12 @@ MF_API int mf_gemm_bf16_normed(const float* x, int ldx, const int* row_idx, cons
 
 // How a product of more than 64 rows is run: out[0] the variant for mf_gemm_bf16, or with out[1] > 1
 // for mf_gemm_bf16_splitk with out[1] splits of out[2] of K each.  `aligned`: 16-byte aligned
-// operands with row strides and K in multiples of 8.
-MF_API int mf_gemm_bf16_tile_plan(int M, int N, int K, int aligned, int epi, int n_cu, int* out) {
-  if (!out || M <= 0 || N <= 0 || K <= 0 || epi < 0 || epi > EPI_LAST || n_cu <= 0) return (int)hipErrorInvalidValue;
+// operands with row strides and K in multiples of 8.  `behind`: 1 where the kernel behind the product adds its parts on the way (the
+// rotation), 2 where that kernel is the norm of the rows as well, else 0.
+MF_API int mf_gemm_bf16_tile_plan(int M, int N, int K, int aligned, int epi, int n_cu, int behind, int* out) {
+  if (!out || behind < 0 || behind > 2 || M <= 0 || N <= 0 || K <= 0 || epi < 0 || epi > EPI_LAST || n_cu <= 0) return (int)hipErrorInvalidValue;
   const bool dma_ok = aligned && K % DMA_BK == 0 && (size_t)M * K * 2 < (1ull << 32) && (size_t)N * K * 2 < (1ull << 32);
-  const TilePlan plan = plan_tiles(M, N, K, dma_ok, epi, n_cu);
+  const TilePlan plan = plan_tiles(M, N, K, dma_ok, epi, n_cu, behind);
   out[0] = plan.variant;
   out[1] = plan.splits;
   out[2] = plan.k_per_split;

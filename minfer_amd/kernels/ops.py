@@ -150,7 +150,7 @@ _PROTOTYPES = {
         "mf_gemm_bf16_skinny_fused": [_P, c_int, _P, _P, c_int, _P, _P, c_int, _P, c_int, c_int, c_int, c_int,
                                       c_int, c_int, _P, c_int, c_float, _P, _P, _P, c_int, _P],
         "mf_gemm_bf16_plan": [c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_char_p, c_int],
-        "mf_gemm_bf16_tile_plan": [c_int, c_int, c_int, c_int, c_int, c_int, _P],
+        "mf_gemm_bf16_tile_plan": [c_int, c_int, c_int, c_int, c_int, c_int, c_int, _P],
         "mf_gemm_bf16_whole_parts": [c_int, c_int, c_int, c_int],
     },
     "attn_tokens_f32": {
@@ -1786,13 +1786,14 @@ def tile_plan(m: int, n: int, k: int, epi: int, aligned: bool = True, n_cu: Opti
     """(variant, splits, k_per_split) of a bfloat16 product of more than 64 rows, as the library
     chooses among its tile kernels (an estimate of the rounds their tiles take over the CUs); with
     splits > 1, K is cut over blocks and a second kernel adds the parts."""
-    return _tile_plan(m, n, k, epi, bool(aligned), n_cu or cu_count())
+    return _tile_plan(m, n, k, epi, bool(aligned), n_cu or cu_count(), 0)
 
 
 @functools.lru_cache(maxsize=4096)           # (a plan depends on these numbers alone; a prompt asks for each of a few once a layer)
-def _tile_plan(m: int, n: int, k: int, epi: int, aligned: bool, n_cu: int) -> Tuple[int, int, int]:
+def _tile_plan(m: int, n: int, k: int, epi: int, aligned: bool, n_cu: int, behind: int) -> Tuple[int, int, int]:
+    # (behind: 1 where the kernel behind the product adds its parts on the way, 2 where it norms the rows too, else 0)
     out = (c_int * 3)()
-    rc = _fn("gemm_bf16", "mf_gemm_bf16_tile_plan")(m, n, k, 1 if aligned else 0, epi, n_cu, out)
+    rc = _fn("gemm_bf16", "mf_gemm_bf16_tile_plan")(m, n, k, 1 if aligned else 0, epi, n_cu, behind, out)
     if rc != 0:
         raise KernelError(f"tile_plan: error {rc} for m {m}, n {n}, k {k}")
     return out[0], out[1], out[2]
@@ -1919,8 +1920,8 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], 
 
 def linear_parts(x: torch.Tensor, weight: torch.Tensor) -> Optional[torch.Tensor]:
     """The product of more than 64 bfloat16 rows as `linear` would cut it over K, its parts not yet added: float32
-    `[parts][m][n]` in the scratch the next split product reuses (without bias), or None, nothing launched, where `linear`
-    does not cut it."""
+    `[parts][m][n]` in the scratch the next split product reuses (without bias), or None, nothing launched, where it is better
+    not cut."""
     _need(x, "linear_parts.x", torch.bfloat16)
     _need(weight, "linear_parts.weight", torch.bfloat16)
     m, k = x.shape
@@ -1929,7 +1930,7 @@ def linear_parts(x: torch.Tensor, weight: torch.Tensor) -> Optional[torch.Tensor
         raise KernelError(f"linear_parts: x is [{m},{k}], weight is {tuple(weight.shape)}")
     if m <= 64:
         return None
-    variant, splits, per = tile_plan(m, n, k, EPI_F32, not (x.data_ptr() % 16 or weight.data_ptr() % 16 or k % 8))
+    variant, splits, per = _tile_plan(m, n, k, EPI_F32, not (x.data_ptr() % 16 or weight.data_ptr() % 16 or k % 8), cu_count(), 1)
     if splits <= 1:
         return None
     part = workspace("skinny", splits * m * n, x.device)[:splits * m * n].view(splits, m, n)
@@ -1940,15 +1941,15 @@ def linear_parts(x: torch.Tensor, weight: torch.Tensor) -> Optional[torch.Tensor
 
 def linear_norm_out(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], out: torch.Tensor, accumulate: bool,
                     g: torch.Tensor, eps: float) -> Optional[torch.Tensor]:
-    """out (+)= x weight^T (+ bias) for more than 64 bfloat16 rows into float32 `out`, where `linear` would cut the product
+    """out (+)= x weight^T (+ bias) for more than 64 bfloat16 rows into float32 `out`, where the product is better cut
     over K, and out / sqrt(mean(out^2) + eps) g in bfloat16, which the kernel that adds the parts leaves beside it and
     which is returned.  None, nothing launched, for any other shape."""
     m, k = x.shape
     n = weight.shape[0]
     if m <= 64 or x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 or weight.shape[1] != k:
         return None
-    variant, splits, per = tile_plan(m, n, k, EPI_ACC_F32 if accumulate else EPI_F32,
-                                     not (x.data_ptr() % 16 or weight.data_ptr() % 16 or k % 8))
+    variant, splits, per = _tile_plan(m, n, k, EPI_ACC_F32 if accumulate else EPI_F32,
+                                      not (x.data_ptr() % 16 or weight.data_ptr() % 16 or k % 8), cu_count(), 2)
     if splits <= 1:
         return None
     _need(x, "linear_norm_out.x")
