@@ -122,10 +122,13 @@ __device__ __forceinline__ void dma16(const float* base, unsigned off, unsigned 
 
 // SPLIT: sums without bias into this part's slab of C, [parts][M][N]; else the product's own epilogue
 // by_xcd: every XCD takes one contiguous eighth of the tiles of all parts (`tiles_by_xcd`)
-template <bool ACCUMULATE, bool SPLIT>
+// PAIR: W is N gate rows and N up rows behind them, a tile takes 32 of each (16 gates and their 16 ups in turns, so that a lane holds
+// both sums of its outputs) and leaves silu(gate) up, or the clamped form with `limit`: no [M][2 N] intermediate and no kernel to read
+// it (611 rows of 4,864 x 896: 102 + 7.4 us as two kernels, 102 so).
+template <bool ACCUMULATE, bool SPLIT, bool PAIR = false>
 __global__ __launch_bounds__(256) void tile_f32_kernel(const float* __restrict__ A, int lda, const float* __restrict__ W, int ldw,
                                                        const float* __restrict__ bias, float* __restrict__ C, int ldc, int M, int N,
-                                                       int K, int tiles_m, int k_per_split, int by_xcd) {
+                                                       int K, int tiles_m, int k_per_split, int by_xcd, float limit = 0.f) {
   __shared__ __attribute__((aligned(16))) unsigned char smem[T_STAGES * T_STAGE];
   int at = blockIdx.y * gridDim.x + blockIdx.x;
   if (by_xcd) {
@@ -140,7 +143,7 @@ __global__ __launch_bounds__(256) void tile_f32_kernel(const float* __restrict__
     K = min(k_per_split, K - kb);
     C += (size_t)part * M * N;
   }
-  const int m0 = (tile % tiles_m) * T_BM, n0 = (tile / tiles_m) * T_BM;
+  const int m0 = (tile % tiles_m) * T_BM, n0 = (tile / tiles_m) * (PAIR ? T_BM / 2 : T_BM);
   const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = (wid & 1) * 32, wn = (wid >> 1) * 32;
   const int fr = lane & 15, fk = lane >> 4;
@@ -151,7 +154,8 @@ __global__ __launch_bounds__(256) void tile_f32_kernel(const float* __restrict__
   for (int q = 0; q < 2; ++q) {
     const int r = (q * 4 + wid) * 8 + (lane >> 3), c = ((lane & 7) ^ ((r >> 1) & 7)) * 4;
     ga[q] = ((unsigned)min(m0 + r, M - 1) * (unsigned)lda + c) * 4u;
-    gw[q] = ((unsigned)min(n0 + r, N - 1) * (unsigned)ldw + c) * 4u;
+    const int row = PAIR ? min(n0 + (r >> 5) * 16 + (r & 15), N - 1) + ((r >> 4) & 1) * N : min(n0 + r, N - 1);
+    gw[q] = ((unsigned)row * (unsigned)ldw + c) * 4u;
   }
   const int nkt = K / T_BK;
   auto copy = [&](int kt, int st) {               // (past the last tile: that one again, never read)
@@ -216,6 +220,20 @@ __global__ __launch_bounds__(256) void tile_f32_kernel(const float* __restrict__
   for (int i = 0; i < 2; ++i) {
     const int m = m0 + wm + i * 16 + fr;
     if (m >= M) continue;
+    if constexpr (PAIR) {
+      const int n = n0 + wn / 2 + fk * 4;
+      const floatx4 g = acc[i][0] + tot[i][0], u = acc[i][1] + tot[i][1];
+      floatx4 v;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = limit > 0.f ? clamped_gate(g[e], u[e], limit) : g[e] / (1.0f + expf(-g[e])) * u[e];
+      float* c = C + (size_t)m * ldc + n;
+      if (vec && n + 4 <= N) *reinterpret_cast<floatx4*>(c) = v;
+      else
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (n + e < N) c[e] = v[e];
+      continue;
+    }
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       const int n = n0 + wn + j * 16 + fk * 4;
@@ -256,6 +274,60 @@ __global__ __launch_bounds__(256) void add_parts_f32_kernel(const float* __restr
   float* c = C + (size_t)m * ldc + n;
   *c = ACCUMULATE ? *c + v : v;
 }
+
+// The same with the RMS norm of the new rows beside it (C / sqrt(mean(C^2) + eps) g): a block a row, which it holds in registers
+// between the sum of squares and the scaling.  The additions in their order, the norm in that of rmsnorm_kernel.  One launch for two,
+// and the rows are not read again (611 rows of 896 in 5 parts: 4.9 + 5.0 us as two kernels).
+template <int KEEP>
+__global__ __launch_bounds__(256) void add_norm_f32_kernel(const float* __restrict__ part, const float* __restrict__ bias,
+                                                           float* __restrict__ C, int ldc, int M, int N, int splits, int accumulate,
+                                                           const float* __restrict__ g, float eps, float* __restrict__ normed) {
+  __shared__ float scratch[4];
+  const int m = blockIdx.x;
+  const size_t mn = (size_t)M * N;
+  const float* p = part + (size_t)m * N;
+  float* c = C + (size_t)m * ldc;
+  float4 v[KEEP];
+  float ss = 0.f;
+#pragma unroll
+  for (int q = 0; q < KEEP; ++q) {
+    const int n = (q * 256 + threadIdx.x) * 4;
+    v[q] = float4{0.f, 0.f, 0.f, 0.f};
+    if (n < N) {
+      const float4 old = accumulate ? *reinterpret_cast<const float4*>(c + n) : v[q];
+      for (int s0 = 0; s0 < splits; s0 += 8) {
+        float4 x[8];
+#pragma unroll
+        for (int s = 0; s < 8; ++s)
+          x[s] = s0 + s < splits ? *reinterpret_cast<const float4*>(p + (size_t)(s0 + s) * mn + n) : float4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < 8; ++s) { v[q].x += x[s].x; v[q].y += x[s].y; v[q].z += x[s].z; v[q].w += x[s].w; }
+      }
+      if (bias) {
+        const float4 b = *reinterpret_cast<const float4*>(bias + n);
+        v[q] = float4{v[q].x + b.x, v[q].y + b.y, v[q].z + b.z, v[q].w + b.w};
+      }
+      if (accumulate) v[q] = float4{old.x + v[q].x, old.y + v[q].y, old.z + v[q].z, old.w + v[q].w};
+      *reinterpret_cast<float4*>(c + n) = v[q];
+    }
+    ss = fmaf(v[q].x, v[q].x, ss);
+    ss = fmaf(v[q].y, v[q].y, ss);
+    ss = fmaf(v[q].z, v[q].z, ss);
+    ss = fmaf(v[q].w, v[q].w, ss);
+  }
+  ss = block_sum<256>(ss, scratch);
+  const float scale = 1.0f / sqrtf(ss / (float)N + eps);
+#pragma unroll
+  for (int q = 0; q < KEEP; ++q) {
+    const int n = (q * 256 + threadIdx.x) * 4;
+    if (n < N) {
+      const float4 w = *reinterpret_cast<const float4*>(g + n);
+      *reinterpret_cast<float4*>(normed + (size_t)m * N + n) =
+          float4{v[q].x * scale * w.x, v[q].y * scale * w.y, v[q].z * scale * w.z, v[q].w * scale * w.w};
+    }
+  }
+}
+constexpr int ADD_NORM_MAX = 256 * 4 * 16;        // a row's values that a block holds
 
 // How many blocks share a tile's K.  The chip's time is that of the CU with the most tiles, times their k tiles (and some four
 // more a tile for its start), at 0.46 us a k tile where three or more share a CU and somewhat more where two or one do; the
@@ -411,6 +483,58 @@ bool rows_take(int M, int N, int K) {
 MF_API int mf_gemm_f32_splits(int M, int N, int K, int aligned, int n_cu) {
   if (M <= 8 || N <= 0 || K < T_BK || n_cu <= 0 || !aligned || K % T_BK || (size_t)M * K * 4 >= (1ull << 32) || (size_t)N * K * 4 >= (1ull << 32)) return 1;
   return tile_splits(M, N, K, n_cu);
+}
+
+static const int NOT_BUILT = -2;     // an entry point's answer for a shape it has no kernel for; nothing was launched
+
+// The parts of a K split alone, [splits][M][N] without bias, for a kernel behind the product that adds them; `splits` (2 and more) as
+// `mf_gemm_f32_splits` gives it.
+MF_API int mf_gemm_f32_parts(const float* A, int lda, const float* W, int ldw, float* part, int M, int N, int K, int splits,
+                             hipStream_t stream) {
+  if (M <= 0 || N <= 0) return 0;
+  if (K <= 0 || lda < K || ldw < K || splits < 2 || !part) return (int)hipErrorInvalidValue;
+  if (!tile_takes(M, N, K, lda, ldw, A, W)) return NOT_BUILT;
+  const int tiles_m = (M + T_BM - 1) / T_BM, tiles = tiles_m * ((N + T_BM - 1) / T_BM);
+  const int per = (K / T_BK + splits - 1) / splits * T_BK;
+  if ((long)(splits - 1) * per >= K) return (int)hipErrorInvalidValue;
+  tile_f32_kernel<false, true><<<dim3(tiles, splits), 256, 0, stream>>>(A, lda, W, ldw, nullptr, part, N, M, N, K, tiles_m, per,
+                                                                        tiles_by_xcd(M, K, splits));
+  return mf_launch_status();
+}
+
+// The product cut over K into C (stored or added to), with the RMS norm of the new rows beside it, normed [M][N].  N in fours, at most
+// 16,384, every operand 16-byte aligned; NOT_BUILT (nothing launched) for any other.
+MF_API int mf_gemm_f32_norm(const float* A, int lda, const float* W, int ldw, const float* bias, float* C, int ldc, float* part, int M,
+                            int N, int K, int splits, int accumulate, const float* g, float eps, float* normed, hipStream_t stream) {
+  if (M <= 0 || N <= 0) return 0;
+  if (ldc < N || !g || !normed) return (int)hipErrorInvalidValue;
+  if (N % 4 || N > ADD_NORM_MAX || ldc % 4 || (uintptr_t)C % 16 || (uintptr_t)part % 16 || (uintptr_t)bias % 16 || (uintptr_t)g % 16 ||
+      (uintptr_t)normed % 16)
+    return NOT_BUILT;
+  const int rc = mf_gemm_f32_parts(A, lda, W, ldw, part, M, N, K, splits, stream);
+  if (rc) return rc;
+  auto run = [&](auto KEEP) {
+    add_norm_f32_kernel<decltype(KEEP)::value><<<M, 256, 0, stream>>>(part, bias, C, ldc, M, N, splits, accumulate, g, eps, normed);
+  };
+  if (N <= 1024) run(std::integral_constant<int, 1>{});
+  else if (N <= 2048) run(std::integral_constant<int, 2>{});
+  else if (N <= 4096) run(std::integral_constant<int, 4>{});
+  else if (N <= 8192) run(std::integral_constant<int, 8>{});
+  else run(std::integral_constant<int, 16>{});
+  return mf_launch_status();
+}
+
+// C [M][N] = silu(gate) up (limit > 0: the clamped form) of A and W, N gate rows and N up rows behind them; K whole.  NOT_BUILT (nothing
+// launched) where the tiles do not take the operands.
+MF_API int mf_gemm_f32_swiglu(const float* A, int lda, const float* W, int ldw, float* C, int ldc, int M, int N, int K, float limit,
+                              hipStream_t stream) {
+  if (M <= 0 || N <= 0) return 0;
+  if (K <= 0 || lda < K || ldw < K || ldc < N) return (int)hipErrorInvalidValue;
+  if (!tile_takes(M, 2 * N, K, lda, ldw, A, W)) return NOT_BUILT;
+  const int tiles_m = (M + T_BM - 1) / T_BM, tiles = tiles_m * ((N + T_BM / 2 - 1) / (T_BM / 2));
+  tile_f32_kernel<false, false, true><<<tiles, 256, 0, stream>>>(A, lda, W, ldw, nullptr, C, ldc, M, N, K, tiles_m, 0, tiles_by_xcd(M, K, 1),
+                                                                 limit);
+  return mf_launch_status();
 }
 
 MF_API int mf_gemm_f32(const float* A, int lda, const float* W, int ldw, const float* bias, float* C, int ldc, float* part,

@@ -132,6 +132,9 @@ _PROTOTYPES = {
     "gemm_f32": {
         "mf_gemm_f32": [_P, c_int, _P, c_int, _P, _P, c_int, _P, c_int, c_int, c_int, c_int, c_int, _P],
         "mf_gemm_f32_splits": [c_int, c_int, c_int, c_int, c_int],
+        "mf_gemm_f32_parts": [_P, c_int, _P, c_int, _P, c_int, c_int, c_int, c_int, _P],
+        "mf_gemm_f32_norm": [_P, c_int, _P, c_int, _P, _P, c_int, _P, c_int, c_int, c_int, c_int, c_int, _P, c_float, _P, _P],
+        "mf_gemm_f32_swiglu": [_P, c_int, _P, c_int, _P, c_int, c_int, c_int, c_int, c_float, _P],
     },
     "gemm_bf16": {
         "mf_gemm_bf16": [_P, c_int, _P, c_int, _P, _P, c_int, c_int, c_int, c_int, c_int, c_int, _P],
@@ -1919,15 +1922,22 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], 
 
 
 def linear_parts(x: torch.Tensor, weight: torch.Tensor) -> Optional[torch.Tensor]:
-    """The product of more than 64 bfloat16 rows as `linear` would cut it over K, its parts not yet added: float32
+    """The product of more than 64 bfloat16 rows, or of 32-bit rows, as `linear` would cut it over K, its parts not yet added: float32
     `[parts][m][n]` in the scratch the next split product reuses (without bias), or None, nothing launched, where it is better
     not cut."""
-    _need(x, "linear_parts.x", torch.bfloat16)
-    _need(weight, "linear_parts.weight", torch.bfloat16)
+    _need(x, "linear_parts.x", _FLOATS)
+    _need(weight, "linear_parts.weight", x.dtype)
     m, k = x.shape
     n = weight.shape[0]
     if weight.shape[1] != k:
         raise KernelError(f"linear_parts: x is [{m},{k}], weight is {tuple(weight.shape)}")
+    if x.dtype == torch.float32:
+        splits = _f32_splits(m, n, k, not (x.data_ptr() % 16 or weight.data_ptr() % 16 or k % 4), cu_count())
+        if splits <= 1:
+            return None
+        part = torch.empty((splits, m, n), dtype=torch.float32, device=x.device)
+        _check(_fn("gemm_f32", "mf_gemm_f32_parts")(x, k, weight, k, part, m, n, k, splits, _stream()), f"gemm_f32_parts {m}x{n}x{k}")
+        return part
     if m <= 64:
         return None
     variant, splits, per = _tile_plan(m, n, k, EPI_F32, not (x.data_ptr() % 16 or weight.data_ptr() % 16 or k % 8), cu_count(), 1)
@@ -1941,11 +1951,13 @@ def linear_parts(x: torch.Tensor, weight: torch.Tensor) -> Optional[torch.Tensor
 
 def linear_norm_out(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], out: torch.Tensor, accumulate: bool,
                     g: torch.Tensor, eps: float) -> Optional[torch.Tensor]:
-    """out (+)= x weight^T (+ bias) for more than 64 bfloat16 rows into float32 `out`, where the product is better cut
-    over K, and out / sqrt(mean(out^2) + eps) g in bfloat16, which the kernel that adds the parts leaves beside it and
+    """out (+)= x weight^T (+ bias) for more than 64 bfloat16 rows, or 32-bit rows, into float32 `out`, where the product is better cut
+    over K, and out / sqrt(mean(out^2) + eps) g in x's type, which the kernel that adds the parts leaves beside it and
     which is returned.  None, nothing launched, for any other shape."""
     m, k = x.shape
     n = weight.shape[0]
+    if x.dtype == weight.dtype == torch.float32 and weight.shape[1] == k:
+        return _linear_norm_out_f32(x, weight, bias, out, accumulate, g, eps)
     if m <= 64 or x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 or weight.shape[1] != k:
         return None
     variant, splits, per = _tile_plan(m, n, k, EPI_ACC_F32 if accumulate else EPI_F32,
@@ -1967,6 +1979,47 @@ def linear_norm_out(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.
         return None
     _check(rc, f"gemm_bf16_splitk_norm {m}x{n}x{k}")
     return normed
+
+
+def _linear_norm_out_f32(x, weight, bias, out, accumulate: bool, g, eps: float) -> Optional[torch.Tensor]:
+    (m, k), n = x.shape, weight.shape[0]
+    if m == 0:
+        return None
+    splits = _f32_splits(m, n, k, not (x.data_ptr() % 16 or weight.data_ptr() % 16 or k % 4), cu_count())
+    if splits <= 1:
+        return None
+    _need(x, "linear_norm_out.x")
+    _need(weight, "linear_norm_out.weight")
+    _need(out, "linear_norm_out.out", torch.float32, (m, n))
+    _need(g, "linear_norm_out.g", torch.float32, (n,))
+    if bias is not None:
+        _need(bias, "linear_norm_out.bias", torch.float32, (n,))
+    normed = torch.empty((m, n), dtype=torch.float32, device=x.device)
+    part = torch.empty(splits * m * n, dtype=torch.float32, device=x.device)
+    rc = _fn("gemm_f32", "mf_gemm_f32_norm")(x, k, weight, k, bias, out, n, part, m, n, k, splits, 1 if accumulate else 0, g, float(eps),
+                                              normed, _stream())
+    if rc == NOT_BUILT:
+        return None
+    _check(rc, f"gemm_f32_norm {m}x{n}x{k}")
+    return normed
+
+
+def linear_swiglu_f32(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor, limit: float = 0.0) -> bool:
+    """`linear` by gate rows with up rows behind them (`[2 f][k]`) and `swiglu`, in 32 bits and one kernel, for more than 8 rows where K
+    is not cut.  False, nothing launched, for any other shape."""
+    m, k = x.shape
+    f = out.shape[1]
+    _need(x, "linear_swiglu_f32.x", torch.float32)
+    _need(weight, "linear_swiglu_f32.weight", torch.float32, (2 * f, k))
+    _need(out, "linear_swiglu_f32.out", torch.float32, (m, f))
+    aligned = not (x.data_ptr() % 16 or weight.data_ptr() % 16 or k % 4)
+    if m <= 8 or k % 32 or not aligned or _f32_splits(m, 2 * f, k, True, cu_count()) > 1:
+        return False
+    rc = _fn("gemm_f32", "mf_gemm_f32_swiglu")(x, k, weight, k, out, f, m, f, k, float(limit), _stream())
+    if rc == NOT_BUILT:
+        return False
+    _check(rc, f"gemm_f32_swiglu {m}x{f}x{k}")
+    return True
 
 
 # variants of the grouped product: (tile rows, tile columns, blocks a CU, microseconds a k tile of 64 with every CU

@@ -86,7 +86,7 @@ class GQAttention(Mixer):
         tables = self.position.rotation_tables(ctx.max_len)
         # a product cut over K leaves its parts to the kernel that rotates and stores
         parts = None
-        if tables is not None and self.rt.is_bf16 and not ctx.all_decode and self.hd % 8 == 0:
+        if tables is not None and not ctx.all_decode and self.hd % 8 == 0:
             parts = self.qkv.parts(x)
         if parts is not None:
             q = torch.empty_like(o)

@@ -83,7 +83,10 @@ class SwiGLU(FeedForward):
                 ops.linear_swiglu(x.tensor() if isinstance(x, Normed) else x, self.fused, y, tiled=self.fused_tiled,
                                   limit=self.limit_on_device)
         else:
-            ops.swiglu(self.gate_up(x, out_dtype=torch.float32), y, limit=self.limit or 0.0)
+            rows = x.tensor() if isinstance(x, Normed) and x.device.type == "cuda" and self.rt.dtype == self.gate_up.weight.dtype else x
+            if not (isinstance(rows, torch.Tensor) and rows.device.type == "cuda" and rows.dtype == self.gate_up.weight.dtype == y.dtype
+                    == torch.float32 and ops.linear_swiglu_f32(rows, self.gate_up.weight, y, limit=self.limit or 0.0)):
+                ops.swiglu(self.gate_up(rows, out_dtype=torch.float32), y, limit=self.limit or 0.0)
         self.down(y, out=h, accumulate=accumulate, ctx=ctx)
 
 

@@ -93,7 +93,7 @@ class Linear:
             if x.shape[0] <= 64:
                 return None
             x = x.tensor()
-        if x.device.type != "cuda" or x.shape[0] <= 64 or x.dtype != torch.bfloat16 or self.weight.dtype != torch.bfloat16:
+        if x.device.type != "cuda" or x.shape[0] <= 64 or x.dtype != self.weight.dtype:
             return None
         return ops.linear_parts(x, self.weight)
 
@@ -104,9 +104,11 @@ class Linear:
         17 to 64 rows whose K is split over blocks; steps of at most 16 rows in the one-kernel
         forms; steps of more rows whose K is split: there the normed rows themselves).  False: nothing ran."""
         norm = getattr(ctx, "norm_next", None)
-        if norm is None or x.shape[0] == 0 or x.dtype != torch.bfloat16 or out.dtype != torch.float32:
+        if norm is None or x.shape[0] == 0 or out.dtype != torch.float32:
             return False
         if tuning.NO_NORM_AHEAD or x.device.type != "cuda":
+            return False
+        if x.dtype != torch.bfloat16 and (x.shape[0] <= 64 or x.dtype != norm.rt.dtype):
             return False
         if x.shape[0] > 64:
             fold = norm.rms_scale()
