@@ -2241,7 +2241,7 @@ def norm_sum_parts(n: int, m: int = 64, k: int = 0) -> int:
     if m <= 16:
         return max(cu_count(), runs)
     blocks = _whole_parts(m, n, k, cu_count()) if k else 0
-    return max(runs, (blocks + 3) // 4 * 4)          # (in fours, so that the next product can read them so)
+    return max(runs, blocks)
 
 
 def linear_fused(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], out: torch.Tensor,
