@@ -2915,6 +2915,7 @@ enum { FORM_256, FORM_192, FORM_128, FORM_128T, FORM_SMALL, FORM_TINY, N_FORMS }
 constexpr DmaForm DMA_FORMS[N_FORMS] = {{256, 256, 1, 1.36, 0.7}, {256, 192, 1, 1.08, 0.7}, {256, 128, 1, 0.84, 0.9},
                                         {128, 256, 1, 0.84, 0.9}, {128, 128, 1, 0.62, 0.9}, {64, 64, 2, 0.56, 0.55}};
 constexpr double ROUND_US = 5.;
+constexpr int TINY_K = 3264;          // the longest K whose 64 x 64 tiles have the price of `form_us`
 
 // The estimate behind the choice: a kernel's tiles go over its slots (blocks that fit the chip at
 // once) in rounds; a round takes the product's k tiles of 64 times the variant's time per k tile, a last round that is
@@ -2926,15 +2927,20 @@ double rounds_us(long blocks, long slots, double step_us, long nkt, double round
   return ((double)nkt * step_us) * ((double)full + (fill > 0. ? low + (1. - low) * fill : 0.)) + round_us * (double)(full + (fill > 0.));
 }
 
-double form_us(int form, int M, int N, long nkt, int splits, long cu) {
+// (nkt: k tiles of a part; K: the whole product's)
+double form_us(int form, int M, int N, int K, long nkt, int splits, long cu) {
   const DmaForm& f = DMA_FORMS[form];
   const long tiles = (long)((M + f.bm - 1) / f.bm) * ((N + f.bn - 1) / f.bn);
-  if (form == FORM_TINY && nkt * splits < 52) {
-    // Against a K of up to 3,072: blocks of four waves that start at once, two a CU: 0.27 us a k tile while no CU has two, soon 0.52
+  if (form == FORM_TINY && K <= TINY_K) {
+    // Blocks of four waves that start at once, two a CU: 0.27 us a k tile while no CU has two, soon 0.52
     // where some have, no more than the start that every plan pays, and 6 us for a round behind the first; of a K split the
     // second blocks' stores come late as well.  (Weights from memory, 64 x 64 whole, estimate / measured: 300 x 2,048 x 2,048
     // 13.6 / 12.1 us, 604 of them 22.5 / 18.9, 604 x 1,536 x 1,536 12.0 / 10.8, 604 x 1,152 x 896 8.9 / 6.7.  Priced like the large tiles
-    // they lost to K split: 300 x 2,048 x 2,048 17.9, 65 x 8,192 x 2,048 15.7 where 64 x 64 take 12.6.)
+    // they lost to K split: 300 x 2,048 x 2,048 17.9, 65 x 8,192 x 2,048 15.7 where 64 x 64 take 12.6.)  The line is the product's own K, the same for whole and
+    // cut: a line by the k tiles of all parts together gave this price to the whole product of 3,136 to 3,264 and the other one to its
+    // cuts, which K in chunks of 256 takes past the line.  142 products at 3,136 and 3,264 so: 0.94 of the time of what that chose on
+    // the average (88 x 896 x 3,200 13.1 us whole, 9.3 in 5 parts; SwiGLU of 203 x 1,536 x 3,136 the other way, 12.4 and 14.7), 0.86 of what
+    // the large tiles' price for both chose.  Past it both have the large tiles' price.
     const long slots = cu * f.per_cu, blocks = tiles * splits, rest = blocks % slots;
     const double last = rest == 0 ? 0. : rest <= cu ? 0.27 : 0.36 + 0.16 * std::min(1., (double)(rest - cu) / 64.);
     return (double)nkt * ((double)(blocks / slots) * 0.53 + last) - 0.7 + 6. * (double)((blocks - 1) / slots) +
@@ -2944,20 +2950,20 @@ double form_us(int form, int M, int N, long nkt, int splits, long cu) {
 }
 
 // the cheapest of the forms first .. last
-int best_form(int first, int last, int M, int N, long nkt, int splits, long cu) {
+int best_form(int first, int last, int M, int N, int K, long nkt, int splits, long cu) {
   int best = first;
   for (int f = first + 1; f <= last; ++f)
-    if (form_us(f, M, N, nkt, splits, cu) < form_us(best, M, N, nkt, splits, cu)) best = f;
+    if (form_us(f, M, N, K, nkt, splits, cu) < form_us(best, M, N, K, nkt, splits, cu)) best = f;
   return best;
 }
 
 // which tiles variant 12, 13 or 15, or variant 2 cut over K, runs
-int dma_form(int variant, int M, int N, int epi, long nkt, int splits, long cu) {
+int dma_form(int variant, int M, int N, int K, int epi, long nkt, int splits, long cu) {
   switch (variant) {
-    case 12: return epi == EPI_SWIGLU && splits == 1 ? best_form(FORM_256, FORM_192, M, N, nkt, 1, cu) : FORM_256;
+    case 12: return epi == EPI_SWIGLU && splits == 1 ? best_form(FORM_256, FORM_192, M, N, K, nkt, 1, cu) : FORM_256;
     case 15: return FORM_192;
   }
-  return best_form(FORM_128, FORM_TINY, M, N, nkt, splits, cu);
+  return best_form(FORM_128, FORM_TINY, M, N, K, nkt, splits, cu);
 }
 
 int launch_form(int form, const bf16* A, int lda, const bf16* W, int ldw, const float* bias, void* C, int ldc, int M, int N, int K,
@@ -3032,7 +3038,7 @@ TilePlan plan_tiles(int M, int N, int K, bool dma_ok, int epi, int n_cu, int beh
     if (us < best.us) best = TilePlan{variant, splits, per, us};
   };
   auto form = [&](int variant, int splits, long steps) {
-    return form_us(dma_form(variant, M, N, epi, steps, splits, cu), M, N, steps, splits, cu);
+    return form_us(dma_form(variant, M, N, K, epi, steps, splits, cu), M, N, K, steps, splits, cu);
   };
   if (dma_ok) {
     if (M > 64 && panel_dma_units(M, N, K, epi, n_cu)) return TilePlan{13, 1, K, 0.};
@@ -3040,8 +3046,8 @@ TilePlan plan_tiles(int M, int N, int K, bool dma_ok, int epi, int n_cu, int beh
     offer(13, 1, K, form(13, 1, nkt) + start_us + epi_us);
     if (epi != EPI_SWIGLU) offer(15, 1, K, form(15, 1, nkt) + start_us + epi_us);
     if (const int n0 = main_rows(N, epi))
-      offer(16, 1, K, form_us(best_form(0, N_FORMS - 1, M, n0, nkt, 1, cu), M, n0, nkt, 1, cu) +
-                          form_us(best_form(FORM_128, FORM_TINY, M, N - n0, nkt, 1, cu), M, N - n0, nkt, 1, cu) + 2 * start_us - more_us + epi_us);
+      offer(16, 1, K, form_us(best_form(0, N_FORMS - 1, M, n0, K, nkt, 1, cu), M, n0, K, nkt, 1, cu) +
+                          form_us(best_form(FORM_128, FORM_TINY, M, N - n0, K, nkt, 1, cu), M, N - n0, K, nkt, 1, cu) + 2 * start_us - more_us + epi_us);
     // many rows against few weight rows and a long K (the down product of a prompt): K cut over
     // the big tiles, each part at least 2,048 of K
     if (epi != EPI_SWIGLU && M >= 768)
@@ -3204,7 +3210,7 @@ MF_API int mf_gemm_bf16_gated(const void* A, int lda, const void* W, int ldw, vo
   const long nkt = K / DMA_BK;
   int form = FORM_256;
   for (int f : {FORM_128, FORM_SMALL})
-    if (form_us(f, M, N, nkt, 1, cu) < form_us(form, M, N, nkt, 1, cu)) form = f;
+    if (form_us(f, M, N, K, nkt, 1, cu) < form_us(form, M, N, K, nkt, 1, cu)) form = f;
   if (form == FORM_256) return launch_halves_dma<256, 256, 2>(a, lda, w, ldw, c, M, N, K, h, stream);
   if (form == FORM_128) return launch_halves_dma<256, 128, 3>(a, lda, w, ldw, c, M, N, K, h, stream);
   return launch_tile_step<128, 128, 2, 4, 4, false, false, true>(a, lda, w, ldw, nullptr, c, width, M, N, K, EPI_SWIGLU, stream, 1, 0, nullptr, 0,
@@ -3243,10 +3249,10 @@ MF_API int mf_gemm_bf16(const void* A, int lda, const void* W, int ldw, const fl
     const int n0 = main_rows(N, epi), cu = cu_count();
     if (!n0 || !dma_ok || cu <= 0) return (int)hipErrorInvalidValue;
     const long nkt = K / DMA_BK;
-    const int rc = launch_form(best_form(0, N_FORMS - 1, M, n0, nkt, 1, cu), a, lda, w, ldw, bias, C, ldc, M, n0, K, epi, stream);
+    const int rc = launch_form(best_form(0, N_FORMS - 1, M, n0, K, nkt, 1, cu), a, lda, w, ldw, bias, C, ldc, M, n0, K, epi, stream);
     if (rc) return rc;
     void* rest = (char*)C + (size_t)n0 * (epi == EPI_BF16 ? 2 : 4);
-    return launch_form(best_form(FORM_128, FORM_TINY, M, N - n0, nkt, 1, cu), a, lda, w + (size_t)n0 * ldw, ldw, bias ? bias + n0 : nullptr,
+    return launch_form(best_form(FORM_128, FORM_TINY, M, N - n0, K, nkt, 1, cu), a, lda, w + (size_t)n0 * ldw, ldw, bias ? bias + n0 : nullptr,
                        rest, ldc, M, N - n0, K, epi, stream);
   }
   if (epi == EPI_SWIGLU && variant == 3) variant = 2;      // needs two 32-column tiles per wave
@@ -3258,7 +3264,7 @@ MF_API int mf_gemm_bf16(const void* A, int lda, const void* W, int ldw, const fl
     case 9: return launch_tile<256, 256, 128, 64, 64>(a, lda, w, ldw, bias, C, ldc, M, N, K, epi, vec_ok, stream);
     case 12: case 13: case 15:
       if (!dma_ok || (variant == 15 && epi == EPI_SWIGLU)) return (int)hipErrorInvalidValue;
-      return launch_form(dma_form(variant, M, N, epi, K / DMA_BK, 1, cu_count()), a, lda, w, ldw, bias, C, ldc, M, N, K, epi, stream);
+      return launch_form(dma_form(variant, M, N, K, epi, K / DMA_BK, 1, cu_count()), a, lda, w, ldw, bias, C, ldc, M, N, K, epi, stream);
   }
   return (int)hipErrorInvalidValue;
 }
@@ -3280,7 +3286,7 @@ MF_API int mf_gemm_bf16_parts(const void* A, int lda, const void* W, int ldw, fl
   if (variant != 12 && variant != 2) return (int)hipErrorInvalidValue;
   const bool dma_ok = vec_ok && K % DMA_BK == 0 && (size_t)M * lda * 2 < (1ull << 32) && (size_t)N * ldw * 2 < (1ull << 32);
   if (variant == 12 && !dma_ok) return (int)hipErrorInvalidValue;
-  return dma_ok ? launch_form(dma_form(variant, M, N, EPI_F32, k_per_split / DMA_BK, splits, cu_count()), (const bf16*)A, lda,
+  return dma_ok ? launch_form(dma_form(variant, M, N, K, EPI_F32, k_per_split / DMA_BK, splits, cu_count()), (const bf16*)A, lda,
                               (const bf16*)W, ldw, nullptr, part, N, M, N, K, EPI_F32, stream, splits, k_per_split)
                 : launch_tile<128, 128, 64, 64>((const bf16*)A, lda, (const bf16*)W, ldw, nullptr, part, N, M,
                                                 N, K, EPI_F32, vec_ok, stream, splits, k_per_split);
@@ -3504,13 +3510,13 @@ MF_API int mf_gemm_bf16_plan(int M, int N, int K, int aligned, int tiled, int ep
     switch (plan.variant) {
       case 12: case 13: case 15:
         if (plan.variant == 13 && M > 64 && panel_dma_units(M, N, K, epi, n_cu)) what = "panel_dma_kernel";
-        else what = form_name(dma_form(plan.variant, M, N, epi, (split ? plan.k_per_split : K) / DMA_BK, plan.splits, n_cu), split);
+        else what = form_name(dma_form(plan.variant, M, N, K, epi, (split ? plan.k_per_split : K) / DMA_BK, plan.splits, n_cu), split);
         break;
       case 16: what = "tile kernels (the last weight rows apart)"; break;
       case 17: what = "panel_dma_kernel"; break;
       case 9: what = "tile_kernel<256,256>"; break;
       case 2:
-        what = split && dma_ok ? form_name(dma_form(2, M, N, EPI_F32, plan.k_per_split / DMA_BK, plan.splits, n_cu), true)
+        what = split && dma_ok ? form_name(dma_form(2, M, N, K, EPI_F32, plan.k_per_split / DMA_BK, plan.splits, n_cu), true)
                : split         ? "tile_kernel<128,128>(split K)" : "tile_kernel<128,128>";
         break;
       case 3: what = "tile_kernel<64,64>"; break;

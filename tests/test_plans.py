@@ -300,3 +300,34 @@ def test_capped_forms_keep_to_their_registers(dim, v_dim):
     heads = ops.capped_form(13, 2, 1, dim, v_dim, 100, 203, n_cu=256)[0]
     assert (heads, 1) in spills and (heads, 4) in spills and (1, 4) in spills
     assert not {f: n for f, n in spills.items() if f[0] <= heads and n}, spills
+
+
+def test_tile_plan_has_one_price_for_whole_and_cut():
+    """Few tiles against a K around the end of the 64 x 64 tiles' own price: a product that is cut at either end of a run of neighbouring
+    K is cut in between as well (whole, 88 x 896 would be 28 workgroups on 256 CUs, each with the whole chain over K)."""
+    for m, n, epi in itertools.product((65, 88, 100, 128), (256, 512, 896, 1024, 1536, 2048, 2560, 3200),
+                                       (ops.EPI_F32, ops.EPI_ACC_F32, ops.EPI_BF16, ops.EPI_SWIGLU)):
+        ks = range(2944, 3648, 64)
+        cut = [ops.tile_plan(m, n, k, epi, True, n_cu=256)[1] > 1 for k in ks]
+        first, last = cut.index(True), len(cut) - cut[::-1].index(True)
+        assert all(cut[first:last]), (m, n, epi, [k for k, c in zip(ks, cut) if not c])
+    for m, n in ((88, 896), (100, 3200), (128, 2560)):
+        for k in range(3072, 3329, 64):
+            assert ops.tile_plan(m, n, k, ops.EPI_ACC_F32, True, n_cu=256)[1] > 1, (m, n, k)
+
+
+def test_tile_plan_of_a_short_k():
+    """The plans that `test_tile_plan` holds the long and the shortest K to, where the 64 x 64 tiles have their own price and a split is
+    credited with what the kernel behind the product saves: whole chunks, no empty part, K in 64s."""
+    for m, n, k, epi, behind in itertools.product((65, 100, 203, 445, 604, 1024, 2048), (96, 896, 1152, 2048, 4608, 8192),
+                                                  (512, 896, 1536, 2048, 3008, 3072, 3136, 3200, 3264, 3328), (ops.EPI_F32, ops.EPI_ACC_F32),
+                                                  (0, 1, 2)):
+        variant, splits, per = ops._tile_plan(m, n, k, epi, True, 256, behind)
+        assert variant in (2, 12, 13, 15, 16)
+        if splits == 1:
+            assert per == k
+            continue
+        assert variant in (2, 12) and per % 256 == 0 and per >= 512
+        assert splits * per >= k and (splits - 1) * per < k
+        tiles = ((m + 127) // 128) * ((n + 127) // 128)
+        assert variant == 12 or (tiles < 256 and splits * tiles <= 512)
