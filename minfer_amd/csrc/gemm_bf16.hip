@@ -3193,6 +3193,32 @@ MF_API int mf_gemm_bf16_grouped_gated(const void* A, const void* W, void* C, con
   return (int)hipErrorInvalidValue;
 }
 
+// which of the tiles that have the form (256 x 256, 256 x 128, 128 x 128) one product of it takes
+static int gated_form(int M, int N, int K, long cu) {
+  const long nkt = K / DMA_BK;
+  int form = FORM_256;
+  for (int f : {FORM_128, FORM_SMALL})
+    if (form_us(f, M, N, K, nkt, 1, cu) < form_us(form, M, N, K, nkt, 1, cu)) form = f;
+  return form;
+}
+
+// Whether `mf_gemm_bf16_gated`, behind a product of its own for the rows' logits, is the faster way through a matrix of `rows` rows (2 width
+// gates and ups, and the logit's behind them): 1, or 0 where one product of them all and the activation's kernel are.  The estimates of
+// the plans for each of the products, the kernel at 5.5 TB/s; 8 us for what a plan counts as starts and rounds beside them.
+// (The gated form has no 64 x 64 tile, and the logits are a launch or two: 8,208 x 2,048, apart / so: 65 rows 19.0 / 30.5 us, 128 23.9 / 33.1, 203
+// 28.7 / 30.9, 384 29.9 / 33.2, 512 38.6 / 33.1, 2,048 83.9 / 64.6; 2,064 x 2,048: 768 19.6 / 27.2, 2,048 36.7 / 29.7.  245 shapes of 100 to 8,192
+// gates and 256 to 4,096, 65 to 4,096 rows: the choice is 0.5 % above the better way on the average, at most 5 % above two kernels (1,300 rows of
+// 12,304 x 3,072 135 and 142) and 7 % above one (333 of them 54.9 and 51.1).)
+MF_API int mf_gemm_bf16_gated_pays(int M, int width, int rows, int K, int n_cu) {
+  if (M <= 64 || width <= 0 || rows < 2 * width || K <= 0 || K % DMA_BK || n_cu <= 0) return 0;
+  const int N = (width + 31) / 32 * 64, logits = rows - 2 * width;
+  const double act_us = 2.5 + ((double)rows * 4. + (double)width * 2.) * M / 5.5e6;
+  const double apart = plan_tiles(M, rows, K, true, EPI_F32, n_cu).us + act_us;
+  const double joined = form_us(gated_form(M, N, K, n_cu), M, N, K, K / DMA_BK, 1, n_cu) +
+                        (logits ? plan_tiles(M, logits, K, true, EPI_F32, n_cu).us : 0.) + 8.;
+  return joined < apart;
+}
+
 // One product of that form, M rows, with a factor sigmoid(z) of every row (z [M], ldz apart; null: none): C [M][width].  2,048 rows of
 // 8,192 x 2,048: 62 + 19 us as two kernels, 64 so.
 MF_API int mf_gemm_bf16_gated(const void* A, int lda, const void* W, int ldw, void* C, int M, int width, int K, int act, float limit,
@@ -3207,10 +3233,7 @@ MF_API int mf_gemm_bf16_gated(const void* A, int lda, const void* W, int ldw, vo
   bf16* c = (bf16*)C;
   const int N = (width + 31) / 32 * 64, cu = cu_count();
   if (cu <= 0) return (int)hipErrorUnknown;
-  const long nkt = K / DMA_BK;
-  int form = FORM_256;
-  for (int f : {FORM_128, FORM_SMALL})
-    if (form_us(f, M, N, K, nkt, 1, cu) < form_us(form, M, N, K, nkt, 1, cu)) form = f;
+  const int form = gated_form(M, N, K, cu);
   if (form == FORM_256) return launch_halves_dma<256, 256, 2>(a, lda, w, ldw, c, M, N, K, h, stream);
   if (form == FORM_128) return launch_halves_dma<256, 128, 3>(a, lda, w, ldw, c, M, N, K, h, stream);
   return launch_tile_step<128, 128, 2, 4, 4, false, false, true>(a, lda, w, ldw, nullptr, c, width, M, N, K, EPI_SWIGLU, stream, 1, 0, nullptr, 0,

@@ -140,6 +140,7 @@ _PROTOTYPES = {
         "mf_gemm_bf16": [_P, c_int, _P, c_int, _P, _P, c_int, c_int, c_int, c_int, c_int, c_int, _P],
         "mf_gemm_bf16_grouped": [_P, _P, _P, _P, c_int, c_int, c_int, c_int, _P],
         "mf_gemm_bf16_grouped_gated": [_P, _P, _P, _P, c_int, c_int, c_int, c_int, c_int, c_float, _P],
+        "mf_gemm_bf16_gated_pays": [c_int, c_int, c_int, c_int, c_int],
         "mf_gemm_bf16_gated": [_P, c_int, _P, c_int, _P, c_int, c_int, c_int, c_int, c_float, _P, c_int, _P],
         "mf_gemm_bf16_splitk": [_P, c_int, _P, c_int, _P, _P, c_int, _P, c_int, c_int, c_int, c_int, c_int, c_int,
                                 c_int, _P],
@@ -2090,9 +2091,20 @@ def linear_grouped_gated(x: torch.Tensor, weights: torch.Tensor, groups: torch.T
 
 
 def linear_gated_takes(m: int, f: int, k: int) -> bool:
-    """Whether `linear_gated` is the way to a bfloat16 product of `m` rows with f gates and f ups: more rows than the decode
-    kernels take, K in 64s, and tiles enough to fill the chip with K whole (else K is better cut, and the activation behind it)."""
+    """Whether `linear_gated` has a form for a bfloat16 product of `m` rows with f gates and f ups: more rows than the decode
+    kernels take, K in 64s, and a plain product of them is not cut over K (its parts would need their kernel in any case)."""
     return m > 64 and k % 64 == 0 and 2 * f * k * 2 < 1 << 32 and m * k * 2 < 1 << 32 and tile_plan(m, 2 * f, k, EPI_F32)[1] == 1
+
+
+@functools.lru_cache(maxsize=4096)
+def _gated_pays(m: int, f: int, rows: int, k: int, n_cu: int) -> bool:
+    return bool(_fn("gemm_bf16", "mf_gemm_bf16_gated_pays")(m, f, rows, k, n_cu))
+
+
+def linear_gated_pays(m: int, f: int, rows: int, k: int, n_cu: Optional[int] = None) -> bool:
+    """Whether `linear_gated`, with a product of its own for the rows' logits, is faster than one product against all `rows` weight
+    rows (f gates, f ups and the logits' behind them) and `gated_expert_act`, as the library estimates both."""
+    return _gated_pays(m, f, rows, k, n_cu or cu_count())
 
 
 def linear_gated(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor, limit: float = 0.0, act: int = 0,

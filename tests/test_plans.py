@@ -331,3 +331,19 @@ def test_tile_plan_of_a_short_k():
         assert splits * per >= k and (splits - 1) * per < k
         tiles = ((m + 127) // 128) * ((n + 127) // 128)
         assert variant == 12 or (tiles < 256 and splits * tiles <= 512)
+
+
+def test_where_an_activation_joins_its_product():
+    """An expert that every token takes, 4,096 gates and ups of 2,048 and a logit's rows: the activation in the epilogue only from the rows
+    on where the tiles that have it, and the logits' own product, cost less than the plain product's tiles and the activation's kernel."""
+    pays = lambda m, f, k: ops.linear_gated_pays(m, f, 2 * f + 16, k, n_cu=256)
+    for m in (65, 96, 128, 160, 203, 256, 300, 384):
+        assert not pays(m, 4096, 2048), m
+    for m in (512, 1024, 2048, 4096):
+        assert pays(m, 4096, 2048), m
+    for m, f, k in ((65, 1024, 2048), (768, 1024, 2048), (1024, 768, 1024), (1024, 512, 2048), (256, 2048, 1024), (65, 4096, 4096), (64, 4096, 2048),
+                    (1, 4096, 2048)):
+        assert not pays(m, f, k), (m, f, k)
+    for m, f, k in ((2048, 1024, 2048), (2048, 4096, 4096), (1024, 2048, 1024)):
+        assert pays(m, f, k), (m, f, k)
+    assert pays(8192, 1024, 2048) and pays(20000, 5632, 2048)
