@@ -1815,7 +1815,6 @@ template <bool TILED>
 int launch_whole(const bf16* A, int lda, const bf16* W, int ldw, const float* bias, float* C, int ldc, int M, int N, int K, int epi,
                  const FusedNorm& fused, hipStream_t stream) {
   const WholePlan p = whole_plan(M, N, K, cu_count());
-  if (fused.out_g && fused.out_parts < p.gx) return MF_NOT_BUILT;
   auto run = [&](auto MT, auto NT) {
     whole_kernel<decltype(MT)::value, decltype(NT)::value, 8, TILED>
         <<<dim3(p.gx, p.gy), 512, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi == EPI_ACC_F32, p.rpb, fused);
@@ -3389,7 +3388,8 @@ static int skinny_product(const void* A, int lda, const void* W, const void* Wt,
   const bf16* w = (const bf16*)W;
   const bf16* wt = (K % 32 == 0 && (uintptr_t)Wt % 16 == 0) ? (const bf16*)Wt : nullptr;
   const bool folds = fused.in_ssq || fused.out_g;
-  if (folds && whole_takes(M, N, K, vec_ok, epi, cu_count()))
+  // (a caller with places for the sums over runs alone gets those, from the K-split kernels)
+  if (folds && whole_takes(M, N, K, vec_ok, epi, cu_count()) && (!fused.out_g || fused.out_parts >= whole_plan(M, N, K, cu_count()).gx))
     return wt ? launch_whole<true>(a, lda, wt, ldw, bias, (float*)C, ldc, M, N, K, epi, fused, stream)
               : launch_whole<false>(a, lda, w, ldw, bias, (float*)C, ldc, M, N, K, epi, fused, stream);
   const SkinnyChoice choice = skinny_choice(M, N, K, vec_ok, wt != nullptr, epi, splits, k_per_split, cu_count());
@@ -3449,8 +3449,8 @@ MF_API int mf_gemm_bf16_skinny(const void* A, int lda, const void* W, const void
 //    product's sums are multiplied by the row's 1 / sqrt(sum / K + eps) before bias and epilogue.
 //  * out_g [N], out_xg [M][N] bf16, out_ssq [M][out_parts]: beside C (32-bit, stored or added
 //    to), bf16(C g) and the sums of C^2 in parts are written: over runs of 256 columns (out_parts =
-//    ceil(N / 256)) for 17 to 64 rows, or one part per block where `whole_kernel` takes them (out_parts at least
-//    `mf_gemm_bf16_whole_parts`, the places past it set to zero); for at most 16 rows one part per block of the product's one
+//    ceil(N / 256)) for 17 to 64 rows, or one part per block where `whole_kernel` takes them and there are places for that (out_parts at
+//    least `mf_gemm_bf16_whole_parts`, the places past it set to zero; with fewer the K-split kernels run); for at most 16 rows one part per block of the product's one
 //    kernel, out_parts at least the number of CUs (the places past the grid are set to zero).
 MF_API int mf_gemm_bf16_skinny_fused(const void* A, int lda, const void* W, const void* Wt, int ldw,
                                      const float* bias, void* C, int ldc, float* part, int M, int N, int K,

@@ -2265,8 +2265,9 @@ def linear_fused(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Ten
     where the norm is otherwise folded into that product's prologue):
 
     * `norm_out` = (g `[n]`, xg `[m][n]` bfloat16, sums `[m][norm_sum_parts(n, m, k)]`): the product stores
-      or adds into the 32-bit `out` as `linear` does and leaves, beside it, bf16(out g) and the sums
-      of out^2 in parts, for the norm with weight g that reads `out` next;
+      or adds into the 32-bit `out` and leaves, beside it, bf16(out g) and the sums
+      of out^2 in parts, for the norm with weight g that reads `out` next (`out` has the bits that `linear` gives, except where
+      the one kernel over the whole of K runs, whose sums are in another order; with sums `[m][norm_sum_parts(n, m)]` it does not run);
     * `scale_in` = (sums `[m][parts]`, eps): `x` is such an xg, and the product's sums are multiplied
       by the row's 1 / sqrt(sum / k + eps) before the bias and the epilogue; with `swiglu`, `weight`
       is `interleave_gate_up(Wg, Wu)` and out = silu(gate) * up, bfloat16.
@@ -2309,7 +2310,9 @@ def linear_fused(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Ten
             raise KernelError("linear_fused.norm_out: the product's own output must be float32")
         _need(out_g, "linear_fused.norm_out.g", torch.float32, (n,))
         _need(out_xg, "linear_fused.norm_out.xg", torch.bfloat16, (m, n))
-        _need(out_ssq, "linear_fused.norm_out.sums", torch.float32, (m, norm_sum_parts(n, m, k)))
+        runs = norm_sum_parts(n, m)
+        _need(out_ssq, "linear_fused.norm_out.sums", torch.float32,
+              (m, runs if out_ssq.dim() == 2 and out_ssq.shape[1] == runs else norm_sum_parts(n, m, k)))
     aligned = not (x.data_ptr() % 16 or weight.data_ptr() % 16 or k % 8)
     splits, per = _k_split(m, n, k, swiglu, aligned, tiled=tiled is not None)
     part = workspace("skinny", splits * m * n, x.device) if (splits > 1 or (swiglu and m > 16)) else None

@@ -65,3 +65,29 @@ def test_readers_of_many_parts(m, nf, k, parts):
     assert ops.linear_fused(x, w, None, out, swiglu=True, scale_in=(s, 1e-6), tiled=ops.tile_weight(w) if k == 2048 else None)
     want = gate / (1 + torch.exp(-gate)) * up
     assert ((out.double() - want).abs() <= want.abs() * 2.0 ** -8 + 1e-4 * scale ** 2).all()
+
+
+# places for the sums over runs of 256 columns alone, at shapes that the one kernel takes otherwise: the kernels that cut K, whose stream
+# is that of the plain product bit for bit
+@pytest.mark.parametrize("m,n,k", [(20, 896, 4864), (33, 2048, 1536), (64, 912, 896), (17, 512, 512)])
+def test_sums_over_runs(m, n, k):
+    from minfer_amd.kernels import ops
+    runs = ops.norm_sum_parts(n, m)
+    assert runs == (n + 255) // 256 < ops.norm_sum_parts(n, m, k)
+    gen = torch.Generator().manual_seed(m + n + k)
+    x = torch.randn((m, k), generator=gen).to(torch.bfloat16).to(DEV)
+    w = (torch.randn((n, k), generator=gen) * k ** -0.5).to(torch.bfloat16).to(DEV)
+    b, g, base = (torch.randn(s, generator=gen).to(DEV) for s in ((n,), (n,), (m, n)))
+    want, out = base.clone(), base.clone()
+    ops.linear(x, w, b, want, accumulate=True)
+    xg, sums = torch.empty((m, n), dtype=torch.bfloat16, device=DEV), torch.full((m, runs), float("nan"), device=DEV)
+    assert ops.linear_fused(x, w, b, out, accumulate=True, norm_out=(g, xg, sums))
+    if ops.plan_linear(m, n, k)["kernel"].startswith("skinny"):
+        assert torch.equal(out, want)
+    tol = 4 * 2.0 ** -20 * k ** 0.5                                      # 32-bit sums of exact products of size one and below
+    assert (out - (x.double() @ w.double().t() + b.double() + base.double())).abs().max() <= tol
+    assert torch.equal(xg, (out * g).to(torch.bfloat16))
+    squares = torch.nn.functional.pad(out.double() ** 2, (0, -n % 256)).view(m, runs, 256).sum(-1)
+    assert ((sums.double() - squares).abs() <= 1e-5 * squares + 1e-9).all()
+    with pytest.raises(ops.KernelError):
+        ops.linear_fused(x, w, b, out, accumulate=True, norm_out=(g, xg, torch.empty((m, runs + 1), device=DEV)))
