@@ -36,3 +36,22 @@ def test_which_products_take_it():
     with pytest.raises(ops.KernelError):
         x = torch.zeros((128, 64), dtype=torch.bfloat16, device=DEV)
         ops.linear(x, torch.zeros((512, 64), dtype=torch.bfloat16, device=DEV), None, torch.empty((128, 512), device=DEV), variant=16)
+
+
+# as above, rests of up to 64 rows behind one tile and several
+@pytest.mark.parametrize("m,n,k", [(65, 257, 64), (257, 768 + 33, 192), (1030, 1024 + 64, 256), (2048, 8200, 4096)])
+def test_square_of_relu_of_the_last_rows(m, n, k):
+    """max(z, 0)^2 in the epilogues of both launches: the bits of the product in 32 bits, cut the same way, and the activation's kernel."""
+    from minfer_amd.kernels import ops
+    gen = torch.Generator().manual_seed(m + n)
+    x, w = (torch.randn(s, generator=gen).to(torch.bfloat16).to(DEV) for s in ((m, k), (n, k)))
+    b, sums = torch.randn(n, generator=gen).to(DEV), torch.empty((m, n), device=DEV)
+    ops.linear(x, w, b, sums, variant=16)
+    want, out = (torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    ops.relu2(sums, want)
+    ops.linear(x, w, b, out, variant=16, relu2=True)
+    assert torch.equal(out, want)
+    if m == 2048:
+        assert ops.tile_plan(m, n, k, ops.EPI_RELU2, n_cu=256)[0] == 16
+        ops.linear(x, w, b, out.fill_(0), relu2=True)
+        assert torch.equal(out, want)

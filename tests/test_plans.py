@@ -347,3 +347,12 @@ def test_where_an_activation_joins_its_product():
     for m, f, k in ((2048, 1024, 2048), (2048, 4096, 4096), (1024, 2048, 1024)):
         assert pays(m, f, k), (m, f, k)
     assert pays(8192, 1024, 2048) and pays(20000, 5632, 2048)
+
+
+def test_last_weight_rows_apart_whatever_the_epilogue():
+    """A rest of a few weight rows is a launch of its own for every epilogue that takes its columns one by one."""
+    for epi in (ops.EPI_F32, ops.EPI_ACC_F32, ops.EPI_BF16, ops.EPI_RELU2):
+        for m, n, k in ((2048, 8224, 2048), (2048, 8200, 4096), (4096, 8208, 2048)):
+            assert ops.tile_plan(m, n, k, epi, n_cu=256)[0] == 16, (m, n, k, epi)
+    for epi in (ops.EPI_XIELU, ops.EPI_SWIGLU):
+        assert ops.tile_plan(2048, 8256, 2048, epi, n_cu=256)[0] != 16
