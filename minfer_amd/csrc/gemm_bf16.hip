@@ -3103,11 +3103,14 @@ int launch_panel_rows(int J, const bf16* A, int lda, const bf16* W, int ldw, con
 #undef MF_PANEL
 }
 
-// Which kernel a product of at most 64 rows takes.
+// Which kernel a product of at most 64 rows takes (SK_NONE: none has a place for the norms to be folded in).
 enum SkinnyChoice {
   SK_STATIONARY, SK_ROLLING, SK_GUARDED_PAIR, SK_GUARDED_4X2, SK_GUARDED_8X2, SK_GUARDED_8X1, SK_PANEL, SK_RING,
-  SK_STAGED, SK_TILE, SK_PANEL_SHORT
+  SK_STAGED, SK_TILE, SK_PANEL_SHORT, SK_WHOLE, SK_NONE
 };
+// Norms folded in: the activations come with a prepared one, the next one is prepared; of the latter's sums there are places for those
+// over runs of 256 columns alone.
+enum { FOLD_IN = 1, FOLD_OUT = 2, FOLD_RUNS = 4 };
 
 // 17 to 64 rows against a short K: a tile of 64 x 64 over the whole of K, with the norm's factors, the bias and SwiGLU in its
 // epilogue, where the K-split kernels need a second one (32 to 40 rows, K-split and added / one tile kernel: gate|up 9,728 x 896
@@ -3124,12 +3127,15 @@ bool tile64_takes(int M, int N, int K, bool aligned, bool tiled, int epi, int n_
   return K <= 1024 && (!fast_split || M > 32 || K <= 512 || N <= 64 * n_cu);
 }
 
-SkinnyChoice skinny_choice(int M, int N, int K, bool aligned, bool tiled, int epi, int splits, int k_per_split, int n_cu) {
+SkinnyChoice skinny_choice(int M, int N, int K, bool aligned, bool tiled, int epi, int splits, int k_per_split, int n_cu, int folds) {
+  if (folds && !(folds & FOLD_RUNS) && whole_takes(M, N, K, aligned, epi, n_cu)) return SK_WHOLE;
   if (M <= 16 && splits == 1) {
     // the register-resident kernel where it is built; other aligned shapes the rolling K-split
-    // kernel; the rest (and SwiGLU outside the first) the guarded kernel
+    // kernel; the rest (and SwiGLU outside the first) the guarded kernel.  The first takes a prepared norm and prepares
+    // the next one, the second prepares the next one.
     if (aligned && stationary_takes(M, N, K, epi, false)) return SK_STATIONARY;
-    if (aligned && K % 32 == 0 && epi != EPI_SWIGLU) return SK_ROLLING;
+    if (aligned && K % 32 == 0 && epi != EPI_SWIGLU) return folds & FOLD_IN ? SK_NONE : SK_ROLLING;
+    if (folds) return SK_NONE;
     if (epi == EPI_SWIGLU) return SK_GUARDED_PAIR;
     // many weight rows: 4 waves with two 16-row tiles each (less activation traffic per weight
     // byte); a row count that would leave a short second round of 16-row blocks: 8 waves with
@@ -3139,9 +3145,13 @@ SkinnyChoice skinny_choice(int M, int N, int K, bool aligned, bool tiled, int ep
     if (blocks16 > 256 && blocks16 <= 512) return SK_GUARDED_8X2;
     return SK_GUARDED_8X1;
   }
-  if (M > 16 && panel_takes(M, N, K, aligned, epi, n_cu)) return SK_PANEL;
-  if (aligned && panel_dma_units(M, N, K, epi, n_cu) == 3) return SK_PANEL_SHORT;
-  if (tile64_takes(M, N, K, aligned, tiled, epi, n_cu)) return SK_TILE;
+  // (the panel and the tile kernels take a prepared norm and prepare none; of the K-split kernels the second folds norms in)
+  if (M > 16 && panel_takes(M, N, K, aligned, epi, n_cu)) return folds & FOLD_OUT ? SK_NONE : SK_PANEL;
+  if (!(folds & FOLD_OUT)) {
+    if (aligned && panel_dma_units(M, N, K, epi, n_cu) == 3) return SK_PANEL_SHORT;
+    if (tile64_takes(M, N, K, aligned, tiled, epi, n_cu)) return SK_TILE;
+  }
+  if (folds && splits == 1 && epi != EPI_SWIGLU) return SK_NONE;
   return ring_takes(aligned, K, splits, k_per_split) ? SK_RING : SK_STAGED;
 }
 
@@ -3388,18 +3398,15 @@ static int skinny_product(const void* A, int lda, const void* W, const void* Wt,
   const bf16* a = (const bf16*)A;
   const bf16* w = (const bf16*)W;
   const bf16* wt = (K % 32 == 0 && (uintptr_t)Wt % 16 == 0) ? (const bf16*)Wt : nullptr;
-  const bool folds = fused.in_ssq || fused.out_g;
   // (a caller with places for the sums over runs alone gets those, from the K-split kernels)
-  if (folds && whole_takes(M, N, K, vec_ok, epi, cu_count()) && (!fused.out_g || fused.out_parts >= whole_plan(M, N, K, cu_count()).gx))
-    return wt ? launch_whole<true>(a, lda, wt, ldw, bias, (float*)C, ldc, M, N, K, epi, fused, stream)
-              : launch_whole<false>(a, lda, w, ldw, bias, (float*)C, ldc, M, N, K, epi, fused, stream);
-  const SkinnyChoice choice = skinny_choice(M, N, K, vec_ok, wt != nullptr, epi, splits, k_per_split, cu_count());
-  // at most 16 rows: the register-resident kernel takes a prepared norm and prepares the next one, the
-  // rolling kernel prepares the next one; the K-split kernels' second kernel counts its parts otherwise
-  if (folds && M <= 16 && choice != SK_STATIONARY && choice != SK_RING && choice != SK_STAGED &&
-      !(choice == SK_ROLLING && !fused.in_ssq))
-    return MF_NOT_BUILT;
+  const bool runs = fused.out_g && M > 16 && whole_takes(M, N, K, vec_ok, epi, cu_count()) && fused.out_parts < whole_plan(M, N, K, cu_count()).gx;
+  const int folds = (fused.in_ssq ? FOLD_IN : 0) | (fused.out_g ? FOLD_OUT : 0) | (runs ? FOLD_RUNS : 0);
+  const SkinnyChoice choice = skinny_choice(M, N, K, vec_ok, wt != nullptr, epi, splits, k_per_split, cu_count(), folds);
   switch (choice) {
+    case SK_NONE: return MF_NOT_BUILT;
+    case SK_WHOLE:
+      return wt ? launch_whole<true>(a, lda, wt, ldw, bias, (float*)C, ldc, M, N, K, epi, fused, stream)
+                : launch_whole<false>(a, lda, w, ldw, bias, (float*)C, ldc, M, N, K, epi, fused, stream);
     case SK_STATIONARY: return stationary16(a, lda, w, wt, ldw, bias, C, ldc, M, N, K, epi, nullptr, stream, fused);
     case SK_ROLLING:
       return wt ? launch_rolling16<8, 1, 16, false, true>(a, lda, wt, ldw, bias, C, ldc, M, N, K, epi, stream, fused)
@@ -3410,15 +3417,14 @@ static int skinny_product(const void* A, int lda, const void* W, const void* Wt,
     case SK_GUARDED_8X1: return launch_skinny16<8, 1, 8>(a, lda, w, ldw, bias, C, ldc, M, N, K, epi, vec_ok, stream);
     case SK_PANEL:
     case SK_PANEL_SHORT: {
-      // (the panel kernels take a prepared norm and prepare none; 32-bit byte offsets)
-      const int J = (size_t)N * ldw * 2 < (1ull << 32) && !fused.out_g ? panel_dma_units(M, N, K, epi, cu_count()) : 0;
+      // (32-bit byte offsets)
+      const int J = (size_t)N * ldw * 2 < (1ull << 32) ? panel_dma_units(M, N, K, epi, cu_count()) : 0;
       if (J) return launch_panel_rows(J, a, lda, w, ldw, bias, C, ldc, M, N, K, epi, fused, stream);
       if (choice == SK_PANEL_SHORT) break;
       return launch_panel(a, lda, w, wt, ldw, bias, C, ldc, M, N, K, epi, fused, stream);
     }
     case SK_TILE:
-      // (the next norm's sums of squares come from the K-split kernels' second one; operands beyond 4 GB go to them as well)
-      if (fused.out_g || (size_t)N * ldw * 2 >= (1ull << 32)) break;
+      if ((size_t)N * ldw * 2 >= (1ull << 32)) break;          // (operands beyond 4 GB go to the K-split kernels)
       return fused.in_ssq ? launch_tile64<true>(a, lda, w, ldw, bias, C, ldc, M, N, K, epi, stream, 1, 0, fused.in_ssq, fused.in_parts,
                                                 fused.in_eps)
                           : launch_tile64<false>(a, lda, w, ldw, bias, C, ldc, M, N, K, epi, stream, 1, 0);
@@ -3507,16 +3513,22 @@ MF_API int mf_gemm_bf16_tile_plan(int M, int N, int K, int aligned, int epi, int
 // activation rows against `N` weight rows of length `K`; `aligned`: 16-byte aligned operands with
 // row strides and K in multiples of 8; `tiled`: there is the tiled copy; for at most 64 rows `splits`, `k_per_split`: the caller's K
 // split (1, K for none); `normed`: the RMS norm is to be folded in (an empty name then means "no
-// such kernel": norm and product run one after the other); `variant`: of the tile kernels, as `mf_gemm_bf16` takes it (0: the
+// such kernel": norm and product run one after the other); `folds`, at most 64 rows: norms folded in on either side as
+// `mf_gemm_bf16_skinny_fused` does it, 1 a prepared one is taken, 2 the next one is prepared (with places for as many sums a row as the
+// kernels leave; 4 beside it: for those over runs of 256 columns alone); an empty name where it returns MF_NOT_BUILT; `behind`, more rows: as in
+// `mf_gemm_bf16_tile_plan`; `variant`: of the tile kernels, as `mf_gemm_bf16` takes it (0: the
 // plan's own choice, K split or whole); `n_cu`: compute units of the device.
 MF_API int mf_gemm_bf16_plan(int M, int N, int K, int aligned, int tiled, int epi, int splits, int k_per_split,
-                             int normed, int variant, int n_cu, char* name, int cap) {
+                             int normed, int folds, int behind, int variant, int n_cu, char* name, int cap) {
+  if (folds < 0 || folds > 7 || (folds && (normed || M > 64)) || ((folds & FOLD_OUT) && epi != EPI_F32 && epi != EPI_ACC_F32) || behind < 0 ||
+      behind > 2)
+    return (int)hipErrorInvalidValue;
   if (!name || cap < 48 || M <= 0 || N <= 0 || K <= 0 || epi < 0 || epi > EPI_LAST || n_cu <= 0) return (int)hipErrorInvalidValue;
   const char* what = "";
   if (normed) {
     what = (aligned && stationary_takes(M, N, K, epi, true)) ? "stationary16_kernel(norm)" : "";
   } else if (M <= 64 && !variant) {
-    switch (skinny_choice(M, N, K, aligned != 0, tiled != 0 && K % 32 == 0, epi, splits, k_per_split, n_cu)) {
+    switch (skinny_choice(M, N, K, aligned != 0, tiled != 0 && K % 32 == 0, epi, splits, k_per_split, n_cu, folds)) {
       case SK_STATIONARY: what = "stationary16_kernel"; break;
       case SK_ROLLING: what = "rolling16_kernel"; break;
       case SK_GUARDED_PAIR: case SK_GUARDED_4X2: case SK_GUARDED_8X2: case SK_GUARDED_8X1: what = "skinny16_kernel"; break;
@@ -3525,10 +3537,12 @@ MF_API int mf_gemm_bf16_plan(int M, int N, int K, int aligned, int tiled, int ep
       case SK_RING: what = "skinny_ring_kernel"; break;
       case SK_STAGED: what = "skinny_kernel"; break;
       case SK_TILE: what = "tile_step_kernel<64,64>"; break;
+      case SK_WHOLE: what = "whole_kernel"; break;
+      case SK_NONE: break;
     }
   } else {
     const bool dma_ok = aligned && K % DMA_BK == 0 && (size_t)M * K * 2 < (1ull << 32) && (size_t)N * K * 2 < (1ull << 32);
-    const TilePlan plan = variant ? TilePlan{variant, 1, K, 0.} : plan_tiles(M, N, K, dma_ok, epi, n_cu);
+    const TilePlan plan = variant ? TilePlan{variant, 1, K, 0.} : plan_tiles(M, N, K, dma_ok, epi, n_cu, behind);
     const bool split = plan.splits > 1;
     if (variant >= 12 && !dma_ok) return (int)hipErrorInvalidValue;
     switch (plan.variant) {

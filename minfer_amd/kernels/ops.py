@@ -153,7 +153,7 @@ _PROTOTYPES = {
                                 c_int, _P],
         "mf_gemm_bf16_skinny_fused": [_P, c_int, _P, _P, c_int, _P, _P, c_int, _P, c_int, c_int, c_int, c_int,
                                       c_int, c_int, _P, c_int, c_float, _P, _P, _P, c_int, _P],
-        "mf_gemm_bf16_plan": [c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_char_p, c_int],
+        "mf_gemm_bf16_plan": [c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_char_p, c_int],
         "mf_gemm_bf16_tile_plan": [c_int, c_int, c_int, c_int, c_int, c_int, c_int, _P],
         "mf_gemm_bf16_whole_parts": [c_int, c_int, c_int, c_int],
     },
@@ -1817,14 +1817,17 @@ def _k_split(m: int, n: int, k: int, swiglu: bool, aligned: bool, n_cu: Optional
 
 def plan_linear(m: int, n: int, k: int, swiglu: bool = False, normed: bool = False, aligned: bool = True,
                 out_bf16: bool = False, accumulate: bool = False, n_cu: Optional[int] = None,
-                tiled: bool = False, variant: int = 0) -> Dict[str, object]:
-    """Which kernel `linear` / `linear_swiglu` / `linear_normed` runs for a bfloat16 product of
+                tiled: bool = False, variant: int = 0, scale_in: bool = False, norm_out: bool = False,
+                behind: int = 0) -> Dict[str, object]:
+    """Which kernel `linear` / `linear_swiglu` / `linear_normed` / `linear_fused` runs for a bfloat16 product of
     `m` rows against `[n][k]` weights, as the library itself decides it, without launching
     anything: {'kernel': name, 'splits': s, 'k_per_split': per}.  With `normed` an empty name
     means that no kernel folds the norm in at this shape (norm and product then run one after
     the other).  `n` counts the interleaved gate|up rows for `swiglu`; `tiled`: the product is
     given the tiled copy of the weights (it moves the row count from which K is cut over blocks);
-    `variant`: as the one that `linear` is given (a tile kernel's name, K whole)."""
+    `variant`: as the one that `linear` is given (a tile kernel's name, K whole); `scale_in`, `norm_out`: with the norms that
+    `linear_fused` is given (at most 64 rows; an empty name: it returns False); `behind`, more rows: 1 as `linear_parts`, 2 as
+    `linear_norm_out` cuts it (which return None where that is not at all)."""
     n_cu = n_cu or cu_count()
     epi = EPI_SWIGLU if swiglu else (EPI_BF16 if out_bf16 else (EPI_ACC_F32 if accumulate else EPI_F32))
     splits, per = 1, k
@@ -1836,10 +1839,11 @@ def plan_linear(m: int, n: int, k: int, swiglu: bool = False, normed: bool = Fal
     elif m <= 64:
         splits, per = _k_split(m, n, k, swiglu, aligned, n_cu, tiled)
     else:
-        _, splits, per = tile_plan(m, n, k, epi, aligned, n_cu)
+        _, splits, per = _tile_plan(m, n, k, epi, bool(aligned), n_cu, behind)
     name = ctypes.create_string_buffer(64)
     rc = _fn("gemm_bf16", "mf_gemm_bf16_plan")(m, n, k, 1 if aligned else 0, 1 if tiled else 0, epi, splits, per,
-                                               1 if normed else 0, variant, n_cu, name, 64)
+                                               1 if normed else 0, (1 if scale_in else 0) | (2 if norm_out else 0), behind, variant, n_cu,
+                                               name, 64)
     if rc != 0:
         raise KernelError(f"plan_linear: error {rc} for m {m}, n {n}, k {k}")
     return dict(kernel=name.value.decode(), splits=splits, k_per_split=per)

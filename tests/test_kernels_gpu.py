@@ -934,7 +934,7 @@ def test_product_prepares_the_next_norm(ops, m, n, k):
                                           (33, 7168, 5120, False), (17, 1000, 2048, False), (64, 2200, 2048, True),
                                           (8, 4608, 3584, False), (16, 37888, 3584, True), (1, 152064, 3584, False),
                                           (5, 1152, 896, False), (7, 9728, 896, True), (12, 7168, 5120, False),
-                                          (3, 22016, 2048, True)])
+                                          (3, 22016, 2048, True), (17, 1152, 896, False)])
 def test_product_takes_a_prepared_norm(ops, m, n, k, swiglu):
     """The product behind the norm: its activations are bf16(x g), its sums are multiplied by each
     row's 1 / sqrt(sum of the partial sums / k + eps).  Against the formula in float64 with that one
@@ -977,11 +977,11 @@ def test_product_takes_a_prepared_norm(ops, m, n, k, swiglu):
 
 
 # ... and by 64 x 64 tiles over the whole of a short K (one to eight partial sums a row, rows and columns that leave remainders)
-@pytest.mark.parametrize("m,n,k,swiglu", [(17, 1152, 896, False), (40, 1001, 1024, False), (64, 9728, 896, True), (33, 17920, 1536, True),
+@pytest.mark.parametrize("m,n,k,swiglu", [(17, 1160, 896, False), (40, 1001, 1024, False), (64, 9728, 896, True), (33, 17920, 1536, True),
                                           (50, 22016, 2048, True), (64, 515, 64, False), (31, 2000, 192, True)])
 def test_product_takes_a_prepared_norm_in_tiles(ops, m, n, k, swiglu):
     n_run = (n + 63) // 64 * 64 if swiglu else n
-    assert ops.plan_linear(m, n_run, k, swiglu=swiglu)["kernel"] == "tile_step_kernel<64,64>"
+    assert ops.plan_linear(m, n_run, k, swiglu=swiglu, scale_in=True)["kernel"] == "tile_step_kernel<64,64>"
     test_product_takes_a_prepared_norm(ops, m, n, k, swiglu)
 
 

@@ -356,3 +356,30 @@ def test_last_weight_rows_apart_whatever_the_epilogue():
             assert ops.tile_plan(m, n, k, epi, n_cu=256)[0] == 16, (m, n, k, epi)
     for epi in (ops.EPI_XIELU, ops.EPI_SWIGLU):
         assert ops.tile_plan(2048, 8256, 2048, epi, n_cu=256)[0] != 16
+
+
+def test_plan_linear_names_the_kernels_of_folded_norms():
+    """The kernel that a product takes with a norm folded in on either side, "" where `linear_fused` declines; and how a product of many
+    rows is cut where the kernel behind it adds its parts."""
+    p = lambda *a, **k: ops.plan_linear(*a, n_cu=256, **k)["kernel"]
+    both = dict(scale_in=True, norm_out=True)
+    for m, n, k in ((17, 1152, 896), (20, 896, 4864), (64, 2048, 2048), (33, 2048, 1536), (32, 3072, 3072)):
+        for kw in (dict(scale_in=True), dict(norm_out=True), both):
+            assert p(m, n, k, accumulate=True, **kw) == p(m, n, k, tiled=True, **kw) == "whole_kernel", (m, n, k, kw)
+        assert p(m, n, k, accumulate=True) != "whole_kernel"
+        assert p(m, n, k, scale_in=True, out_bf16=True) != "whole_kernel"
+        assert p(m, n + 8, k, norm_out=True) != "whole_kernel"
+    assert p(17, 1152 + 8, 896, scale_in=True) == p(40, 1001, 1024, scale_in=True) == "tile_step_kernel<64,64>"
+    assert p(64, 3584, 3584, norm_out=True) == p(64, 3584, 18944, norm_out=True) == "skinny_ring_kernel"
+    assert p(64, 37888, 3584, swiglu=True, scale_in=True) == "panel_kernel" and p(64, 40960, 3584, norm_out=True) == ""
+    assert p(8, 3584, 18944, norm_out=True, tiled=True) == "rolling16_kernel" and p(8, 3584, 18944, scale_in=True, tiled=True) == ""
+    assert p(8, 3584, 3584, **both) == "stationary16_kernel"
+    for m, n, k in ((8, 300, 200), (20, 300, 200), (64, 64, 256)):
+        assert p(m, n, k, norm_out=True) == "" and p(m, n, k, scale_in=True) == "", (m, n, k)
+    for bad in (dict(norm_out=True, out_bf16=True), dict(norm_out=True, swiglu=True)):
+        with pytest.raises(ops.KernelError):
+            ops.plan_linear(32, 1024, 896, n_cu=256, **bad)
+    for (m, n, k), behind in (((100, 1152, 896), 1), ((300, 896, 896), 2), ((200, 2048, 2048), 1)):
+        assert ops.plan_linear(m, n, k, n_cu=256)["splits"] == 1
+        cut = ops.plan_linear(m, n, k, n_cu=256, behind=behind)
+        assert cut["splits"] > 1 and cut["kernel"].endswith("(split K)")

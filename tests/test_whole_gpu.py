@@ -15,6 +15,8 @@ def test_both_sides(m, n, k):
     from minfer_amd.kernels import ops
     parts = ops.norm_sum_parts(n, m, k)
     assert parts > ops.norm_sum_parts(n, m), "one kernel takes these"
+    for kw in (dict(norm_out=True), dict(scale_in=True), dict(scale_in=True, norm_out=True)):
+        assert ops.plan_linear(m, n, k, accumulate=True, **kw)["kernel"] == "whole_kernel"
     gen = torch.Generator().manual_seed(m + n + k)
     x = torch.randn((m, k), generator=gen).to(torch.bfloat16).to(DEV)
     w = (torch.randn((n, k), generator=gen) * k ** -0.5).to(torch.bfloat16).to(DEV)
