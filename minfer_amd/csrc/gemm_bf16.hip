@@ -3181,14 +3181,14 @@ static bool halves_ok(const Halves& h, const void* C, int K, size_t rows, int ld
 }
 
 // The same of matrices whose rows are `width` gates and then `width` ups (W [matrices][2 width][K]): C [rows][width] =
-// act(gate, up) in bfloat16 from the 32-bit sums, the activations being those of `mf_moe_act` (act 1: silu(gate) up, else the clamped
-// form with `limit`).  No 32-bit intermediate and no kernel of its own for the activation: 2,048 rows over 8 matrices of 8,192 x
+// act(gate, up) in bfloat16 from the 32-bit sums, the activations being those of `mf_moe_act` (act 1: silu(gate) up, 0: the clamped
+// form with `limit`; any other is refused).  No 32-bit intermediate and no kernel of its own for the activation: 2,048 rows over 8 matrices of 8,192 x
 // 2,048 117 + 24 us as two kernels, 120 so (what the smaller stores save, the exponentials take).
 MF_API int mf_gemm_bf16_grouped_gated(const void* A, const void* W, void* C, const int* groups, int n_groups, int width, int K,
                                       int variant, int act, float limit, hipStream_t stream) {
   if (n_groups <= 0 || width <= 0) return 0;
   const Halves h{width, act == 1, limit, nullptr, 0};
-  if (!halves_ok(h, C, K, 2 * (size_t)width, K) || !groups || (uintptr_t)A % 16 || (uintptr_t)W % 16) return (int)hipErrorInvalidValue;
+  if (act < 0 || act > 1 || !halves_ok(h, C, K, 2 * (size_t)width, K) || !groups || (uintptr_t)A % 16 || (uintptr_t)W % 16) return (int)hipErrorInvalidValue;
   const bf16* a = (const bf16*)A;
   const bf16* w = (const bf16*)W;
   const RowGroup* g = (const RowGroup*)groups;
@@ -3229,13 +3229,14 @@ MF_API int mf_gemm_bf16_gated_pays(int M, int width, int rows, int K, int n_cu) 
   return joined < apart;
 }
 
-// One product of that form, M rows, with a factor sigmoid(z) of every row (z [M], ldz apart; null: none): C [M][width].  2,048 rows of
+// One product of that form, M rows, with a factor sigmoid(z) of every row (z [M], ldz apart; null: none): C [M][width].  The clamped form
+// needs a limit above 0.  2,048 rows of
 // 8,192 x 2,048: 62 + 19 us as two kernels, 64 so.
 MF_API int mf_gemm_bf16_gated(const void* A, int lda, const void* W, int ldw, void* C, int M, int width, int K, int act, float limit,
                               const float* z, int ldz, hipStream_t stream) {
   if (M <= 0 || width <= 0) return 0;
   const Halves h{width, act == 1, limit, z, ldz};
-  if (lda < K || ldw < K || lda % 8 || ldw % 8 || !halves_ok(h, C, K, 2 * (size_t)width, ldw) || (size_t)M * lda * 2 >= (1ull << 32) ||
+  if (act < 0 || act > 1 || (act == 0 && !(limit > 0.f)) || lda < K || ldw < K || lda % 8 || ldw % 8 || !halves_ok(h, C, K, 2 * (size_t)width, ldw) || (size_t)M * lda * 2 >= (1ull << 32) ||
       (uintptr_t)A % 16 || (uintptr_t)W % 16)
     return (int)hipErrorInvalidValue;
   const bf16* a = (const bf16*)A;

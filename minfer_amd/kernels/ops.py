@@ -2114,7 +2114,7 @@ def linear_gated_pays(m: int, f: int, rows: int, k: int, n_cu: Optional[int] = N
 def linear_gated(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor, limit: float = 0.0, act: int = 0,
                  gate_logits: Optional[torch.Tensor] = None) -> None:
     """out = act(gate, up), bfloat16 `[m][f]`, of x and a matrix of f gate rows and f up rows behind them, the activations of
-    `moe_act`, from the 32-bit sums; times sigmoid(gate_logits[r][0]) of every row where given (float32 `[m][any]`)."""
+    `moe_act` (the clamped form with a limit above 0), from the 32-bit sums; times sigmoid(gate_logits[r][0]) of every row where given (float32 `[m][any]`)."""
     m, k = x.shape
     f = out.shape[1]
     _need(x, "linear_gated.x", torch.bfloat16)

@@ -87,3 +87,20 @@ def test_square_of_relu(m, n, k):
         assert ((out.double() - ref).abs() <= ref * 2.0 ** -8 + 2 * tol * ref.sqrt() + tol ** 2).all()
         ops.linear(x, w, b, half, tiled=tiled)                           # (which stores nothing else)
         assert torch.isfinite(half.float()).all()
+
+
+def test_activations_that_are_none():
+    """What `moe_act` refuses these refuse, and one product's clamped form without a limit, before anything is launched."""
+    from minfer_amd.kernels import ops
+    x, w = operands(128, 256, 64, 1)
+    groups = torch.tensor(ops.row_groups([128], 2), dtype=torch.int32, device=DEV)
+    out = torch.full((128, 128), 7.0, dtype=torch.bfloat16, device=DEV)
+    for act, limit in ((2, 1.0), (-1, 1.0), (0, 0.0), (0, -1.0), (0, float("nan"))):
+        with pytest.raises(ops.KernelError):
+            ops.linear_gated(x, w, out, limit=limit, act=act)
+    for act in (2, -1):
+        with pytest.raises(ops.KernelError):
+            ops.moe_act(torch.zeros((128, 256), device=DEV), torch.ones((128, 1), device=DEV), out, 1.0, act)
+        with pytest.raises(ops.KernelError):
+            ops.linear_grouped_gated(x, w.view(1, 256, 64), groups, 2, out, 1.0, act)
+    assert (out == 7.0).all()
