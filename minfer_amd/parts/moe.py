@@ -77,7 +77,7 @@ class SharedExpert:
         y = torch.empty((x.shape[0], self.inter), dtype=self.rt.dtype, device=x.device)
         w, pairs = self.up.weight, 2 * self.inter
         if x.device.type == "cuda" and x.dtype == w.dtype == y.dtype == torch.bfloat16 and \
-                ops.linear_gated_takes(x.shape[0], self.inter, self.hidden) and \
+                not (x.data_ptr() % 16 or w.data_ptr() % 16) and ops.linear_gated_takes(x.shape[0], self.inter, self.hidden) and \
                 ops.linear_gated_pays(x.shape[0], self.inter, w.shape[0], self.hidden):
             # many rows: the rows' own logits first, then the activation and their sigmoids in the product's epilogue
             z = torch.empty((x.shape[0], w.shape[0] - pairs), dtype=torch.float32, device=x.device)

@@ -104,3 +104,25 @@ def test_activations_that_are_none():
         with pytest.raises(ops.KernelError):
             ops.linear_grouped_gated(x, w.view(1, 256, 64), groups, 2, out, 1.0, act)
     assert (out == 7.0).all()
+
+
+@pytest.mark.parametrize("offset", [0, 1])
+def test_shared_expert(offset):
+    """The expert every token takes, by the joined kernel and, for rows that stand off 16 bytes, by product and kernel."""
+    from types import SimpleNamespace
+
+    from minfer_amd.kernels import ops
+    from minfer_amd.parts.moe import SharedExpert
+    m, f, k = 1024, 2048, 64
+    assert ops.linear_gated_takes(m, f, k) and ops.linear_gated_pays(m, f, 2 * f + 16, k)
+    flat, w = operands(m * k + 8, 1, 1, 5)[0].view(-1), operands(1, 2 * f + 1, k, 6)[1]
+    x = flat[offset:offset + m * k].view(m, k)
+    down = operands(1, k, f, 7)[1]
+    expert = SharedExpert(dict(stem="e", weight="z", intermediate_size=f), k, SimpleNamespace(dtype=torch.bfloat16))
+    expert.load({"e.gate": w[:f], "e.up": w[f:2 * f], "z": w[2 * f:], "e.down": down}.__getitem__)
+    h = torch.zeros((m, k), device=DEV)
+    expert.forward(x, h, True)
+    z = x.double() @ w.double().t()
+    y = gated(z[:, :f], z[:, f:2 * f], 1, 0.0) / (1 + torch.exp(-z[:, 2 * f:]))
+    want, bound = y @ down.double().t(), y.abs() @ down.double().abs().t() * 2.0 ** -8          # each y rounded to bfloat16
+    assert ((h.double() - want).abs() <= bound + 1e-4).all()
