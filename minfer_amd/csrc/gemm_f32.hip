@@ -551,18 +551,15 @@ MF_API int mf_gemm_f32(const float* A, int lda, const float* W, int ldw, const f
   }
   if (tile_takes(M, N, K, lda, ldw, A, W)) {
     const int tiles_m = (M + T_BM - 1) / T_BM, tiles = tiles_m * ((N + T_BM - 1) / T_BM);
-    const int by_xcd = tiles_by_xcd(M, K, splits);
     if (splits > 1) {
-      const int per = (K / T_BK + splits - 1) / splits * T_BK;
-      if (!part || (long)(splits - 1) * per >= K) return (int)hipErrorInvalidValue;
-      tile_f32_kernel<false, true><<<dim3(tiles, splits), 256, 0, stream>>>(A, lda, W, ldw, nullptr, part, N, M, N, K, tiles_m, per, by_xcd);
-      const int rc = mf_launch_status();
+      const int rc = mf_gemm_f32_parts(A, lda, W, ldw, part, M, N, K, splits, stream);
       if (rc) return rc;
       const unsigned blocks = (unsigned)(((size_t)M * N + 255) / 256);
       if (accumulate) add_parts_f32_kernel<true><<<blocks, 256, 0, stream>>>(part, bias, C, ldc, M, N, splits);
       else add_parts_f32_kernel<false><<<blocks, 256, 0, stream>>>(part, bias, C, ldc, M, N, splits);
       return mf_launch_status();
     }
+    const int by_xcd = tiles_by_xcd(M, K, 1);
     if (accumulate) tile_f32_kernel<true, false><<<tiles, 256, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, tiles_m, 0, by_xcd);
     else tile_f32_kernel<false, false><<<tiles, 256, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, tiles_m, 0, by_xcd);
     return mf_launch_status();
