@@ -1081,7 +1081,6 @@ MF_API int mf_layernorm_join(float* h, const float* y, float alpha, const float*
 }
 
 // ---------------------------------------------------------------- two normed rows, summed
-// out[r] (+)= scale (a[r] / rms(a[r]) wa + b[r] / rms(b[r]) wb), rms with eps inside the root
 // Two sums over a block, each added up as `block_sum` does, behind one pair of barriers.
 template <int NT>
 __device__ __forceinline__ void block_sums(float& a, float& b, float* sa, float* sb) {
@@ -1096,6 +1095,7 @@ __device__ __forceinline__ void block_sums(float& a, float& b, float* sa, float*
   for (int i = 0; i < NT / 64; ++i) { a += sa[i]; b += sb[i]; }
 }
 
+// out[r] (+)= scale (a[r] / rms(a[r]) wa + b[r] / rms(b[r]) wb), rms with eps inside the root
 template <int KEEP>
 __global__ __launch_bounds__(256) void rmsnorm_pair_kernel(const float* __restrict__ a, const float* __restrict__ wa,
                                                            const float* __restrict__ b, const float* __restrict__ wb,

@@ -27,7 +27,7 @@
 // skinny16_kernel) can read the weights from a tiled copy instead (`w_operand`), where the
 // caller has one.
 //
-// Epilogues: 0 store fp32, 1 add into fp32 (residual stream), 2 store bf16, 3 SwiGLU.
+// Epilogues: 0 store fp32, 1 add into fp32 (residual stream), 2 store bf16, 3 SwiGLU, 4 xIELU and 5 the square of relu (both bf16).
 // SwiGLU (y = silu(g) * u, silu(z) = z / (1 + exp(-z)), src/graph/cpu_backend.rs:323-329):
 // the weight rows come interleaved in groups of 64, 32 gate rows then the 32 up rows of the
 // same outputs (the last group padded with zero rows), so a gate column and its up column
@@ -736,7 +736,8 @@ __global__ __launch_bounds__(512, 2) void tile_dma_kernel(const bf16* __restrict
 // The sum of a row's `parts` numbers by LANES lanes that stand side by side (l: the lane's place among them), in two steps so that a
 // kernel asks early and adds late: every lane asks for Q x 4 of them at once, one value a load (with 16-byte loads beside them where
 // the rows allow it the compiler waited for each row's first before the next: a trip to memory for every row of a lane, in front of the
-// product's first copies; gate|up of 37 rows with 84 parts a row 11.2 us so, 9.8 now), and what is left of a longer row when it adds up.  A row without parts (p null) asks for nothing and gives 0.
+// product's first copies; gate|up of 37 rows with 84 parts a row 11.2 us so, 9.8 now), and for what is left of a longer row when it
+// adds up.  A row without parts (p null) asks for nothing and gives 0.
 template <int LANES, int Q>
 struct LanesSum {
   float x[Q][4];
@@ -1416,7 +1417,7 @@ bool ring_takes(bool aligned, int K, int splits, int k_per_split) {
 //    owns some columns; `out_parts` places a row, the ones past the grid set to zero);
 //  * the product that follows takes xg as its activations and multiplies its own sums by the
 //    row's 1 / sqrt(sum / K + eps) in its epilogue (`in_*`), the partial sums of squares added up
-//    in their order.
+//    in a fixed tree.
 // No norm kernel, no pass over the stream between the two products.  The same arithmetic as the
 // fold of the register-resident kernel above (bf16(x g) to the matrix cores, the row's factor in
 // the epilogue).
@@ -1428,7 +1429,7 @@ struct FusedNorm {
   float in_eps;
   const float* out_g;      // [N] weight of the norm that reads the output next (null: none)
   bf16* out_xg;            // [M][N]
-  float* out_ssq;          // [M][ceil(N / 256)], or [M][out_parts] from a one-kernel product of at most 16 rows
+  float* out_ssq;          // [M][out_parts]: a part for every run of 256 columns, or from a one-kernel product for every block; then zeros
   int out_parts;
 };
 
@@ -1803,9 +1804,12 @@ WholePlan whole_plan(int M, int N, int K, int n_cu) {
     }
   return best;
 }
-// Up to 38 loads, where both ways take some 10 us: 896 x 4,864 (38) 9.2 here and 11.0 with K split, 3,584 x 3,584 at 32 rows (42) 11.9
-// and 12.5, 1,536 x 8,960 (70) 16.3 and 13.4.  Whole tiles of weight rows, and not few: below 512 no model has them and a block's share
-// is a row or two.  (With the tiled copy or without, the same sums: the choice does not ask for it.)
+// Up to 38 loads.  K split and added / this, 17, 32, 48 and 64 rows, 17 matrices: up to 38 loads 0.53 to 0.96 of the time (896 x 4,864, 38: 9.3 / 8.9 us
+// at 17 rows, 11.5 / 9.6 at 64), with 40 to 48 0.78 to 1.0 (2,560 x 2,560 at 64 rows 13.8 / 12.2, 3,584 x 3,584 at 32 12.7 / 11.9, 3,072 x 3,072 at 64
+// 13.9 / 13.9), with 56 0.99 to 1.11, from 70 on 1.13 and more (1,536 x 8,960 at 17 rows 13.1 / 14.9): the line is on the safe side of where they
+// meet, some 45 to 50.  At least 512 weight rows, in 16s: not for the kernel's sake, which clamps its rows and would gain there too (500 x 896
+// 6.9 / 4.2 at 17 rows, 384 x 2,048 7.4 / 5.5); widths that no model of this library's has keep the kernels that they had.
+// (With the tiled copy or without, the same sums: the choice does not ask for it.)
 bool whole_takes(int M, int N, int K, bool aligned, int epi, int n_cu) {
   if (M <= 16 || M > 64 || !aligned || N < 512 || N % 16 || K % 32 || n_cu <= 0 || (epi != EPI_F32 && epi != EPI_ACC_F32)) return false;
   return whole_plan(M, N, K, n_cu).loads <= 38;
@@ -3450,8 +3454,8 @@ MF_API int mf_gemm_bf16_skinny(const void* A, int lda, const void* W, const void
 }
 
 // The same with an RMS norm folded in on either side (see FusedNorm), for the shapes whose kernels
-// have a place for it (17 to 64 rows: the whole-K kernel on the reading side, the K-split kernels
-// with more than one split on both; at most 16 rows: the register-resident kernel on both sides,
+// have a place for it (17 to 64 rows: `whole_kernel`, or the K-split kernels with more than one split, on both sides, the tile
+// and the panel kernels on the reading one; at most 16 rows: the register-resident kernel on both sides,
 // the rolling kernel on the writing side); MF_NOT_BUILT (-2), having launched nothing, for any other.
 //  * in_ssq [M][in_parts], in_eps: A holds bf16(x g) of rows x whose sums of squares these are; the
 //    product's sums are multiplied by the row's 1 / sqrt(sum / K + eps) before bias and epilogue.

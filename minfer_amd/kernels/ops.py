@@ -1927,9 +1927,10 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], 
 
 
 def linear_parts(x: torch.Tensor, weight: torch.Tensor) -> Optional[torch.Tensor]:
-    """The product of more than 64 bfloat16 rows, or of 32-bit rows, as `linear` would cut it over K, its parts not yet added: float32
-    `[parts][m][n]` in the scratch the next split product reuses (without bias), or None, nothing launched, where it is better
-    not cut."""
+    """The product of more than 64 bfloat16 rows, or of 32-bit rows, cut over K, its parts not yet added: float32 `[parts][m][n]` (without
+    bias; of bfloat16 rows in the scratch the next split product reuses), or None, nothing launched, where it is better not cut.
+    32-bit rows are cut as `linear` cuts them; bfloat16 rows more often (`plan_linear` with `behind` 1), since the kernel behind the
+    product that adds the parts runs in any case."""
     _need(x, "linear_parts.x", _FLOATS)
     _need(weight, "linear_parts.weight", x.dtype)
     m, k = x.shape

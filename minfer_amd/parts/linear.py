@@ -101,7 +101,7 @@ class Linear:
         """Runs the product with the next norm's input prepared beside it (bf16(out g) and the rows'
         partial sums of squares, left in `ctx.norm_ahead`) where the block has said which norm
         that is, the norm is of the RMS form and the product's kernels have a place for it (steps of
-        17 to 64 rows whose K is split over blocks; steps of at most 16 rows in the one-kernel
+        17 to 64 rows in one kernel over the whole of K or with K split over blocks; steps of at most 16 rows in the one-kernel
         forms; steps of more rows whose K is split: there the normed rows themselves).  False: nothing ran."""
         norm = getattr(ctx, "norm_next", None)
         if norm is None or x.shape[0] == 0 or out.dtype != torch.float32:
