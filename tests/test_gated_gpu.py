@@ -85,6 +85,11 @@ def test_square_of_relu(m, n, k):
         ref = z.clamp(min=0) ** 2
         tol = 4 * 2.0 ** -20 * k ** 0.5                                  # of z: 32-bit sums of exact products of size one and below
         assert ((out.double() - ref).abs() <= ref * 2.0 ** -8 + 2 * tol * ref.sqrt() + tol ** 2).all()
+        if m <= 64 or ops.tile_plan(m, n, k, ops.EPI_RELU2) == ops.tile_plan(m, n, k, ops.EPI_F32):   # K cut alike: the very bits
+            sums, want = torch.empty((m, n), device=DEV), torch.empty_like(out)
+            ops.linear(x, w, b, sums, tiled=tiled)
+            ops.relu2(sums, want)
+            assert torch.equal(out, want)
         ops.linear(x, w, b, half, tiled=tiled)                           # (whose epilogue is the plain one)
         assert ((half.double() - z).abs() <= z.abs() * 2.0 ** -8 + tol).all()
 
