@@ -372,6 +372,13 @@ __device__ __forceinline__ void dma_meet() {
   __builtin_amdgcn_sched_barrier(0);
 }
 
+// Where chunk c (eight k) of weight row n begins in a k tile of 64, in bytes: in the matrix, or in its tiled copy (`w_operand`), where a
+// k tile is two tiles of 32 k, a kilobyte apart, and the next one stands 2 KB on.
+__device__ __forceinline__ unsigned w_copy_at(int n, int ldw, int c, bool tiled) {
+  return tiled ? (unsigned)(n >> 4) * (unsigned)(ldw >> 5) * 1024u + (c >> 2) * 1024u + (n & 15) * 64u + (c & 3) * 16u
+               : ((unsigned)n * (unsigned)ldw + c * 8) * 2u;
+}
+
 // How the 8 waves of a block share a BM x BN tile, in blocks of 16 x 16 results.
 template <int BM, int BN>
 struct DmaTile {
@@ -548,7 +555,7 @@ __global__ __launch_bounds__(512, 2) void tile_dma_kernel(const bf16* __restrict
                                                        const bf16* __restrict__ W, int ldw,
                                                        const float* __restrict__ bias, void* __restrict__ C,
                                                        int ldc, int M, int N, int K, int epi, int tiles_m,
-                                                       int order, int k_per_split,
+                                                       int order, int k_per_split, bool tiled,
                                                        const RowGroup* __restrict__ groups = nullptr, Halves halves = Halves{}) {
   using TT = DmaTile<BM, BN>;
   constexpr int ROW = DMA_BK * 2, A_ST = BM * ROW, W_ST = BN * ROW, W_AT = STAGES * A_ST;
@@ -560,7 +567,7 @@ __global__ __launch_bounds__(512, 2) void tile_dma_kernel(const bf16* __restrict
     // and stores 32-bit sums into its own [M][N] slab of C; another kernel adds the slabs
     const int kb = part * k_per_split;
     A += kb;
-    W += kb;
+    W += tiled ? kb * 16 : kb;
     K = min(k_per_split, K - kb);
     C = (float*)C + (size_t)part * M * N;
   }
@@ -588,6 +595,7 @@ __global__ __launch_bounds__(512, 2) void tile_dma_kernel(const bf16* __restrict
 #pragma unroll
     for (int j = 0; j < J; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
 
+  const int wk = tiled ? 16 * DMA_BK : DMA_BK;               // weights from a k tile to the next
   // What a wave copies: pieces of 8 rows (1 KB), the lane row lane / 8 of a piece and the chunk that belongs at position
   // lane % 8.  Half h of A: the rows of the row blocks h IH .. + IH - 1 of every row of waves; half h of W: the rows of
   // the column blocks of that half of every column of waves.
@@ -607,7 +615,7 @@ __global__ __launch_bounds__(512, 2) void tile_dma_kernel(const bf16* __restrict
     const int jh = q < LW0 ? J0 : J1, p = (q < LW0 ? q : q - LW0) * 8 + wid;       // 2 jh pieces a column of waves
     const int b = TT::first(p / (2 * jh)) + ((q < LW0 ? 0 : J0) + (p % (2 * jh)) / 2) * TT::STEP;
     const int r0 = b * 16 + (p & 1) * 8, r = r0 + (lane >> 3);
-    gw[q] = ((unsigned)(HALVES ? halves.row(n0 + r) : min(n0 + r, N - 1)) * (unsigned)ldw + ((lane & 7) ^ ((r >> 1) & 7)) * 8) * 2u;
+    gw[q] = w_copy_at(HALVES ? halves.row(n0 + r) : min(n0 + r, N - 1), ldw, (lane & 7) ^ ((r >> 1) & 7), tiled);
     lw[q] = lds0 + W_AT + r0 * ROW;
   }
   auto copy_a = [&](int kt, int st, auto HALF) {
@@ -619,7 +627,7 @@ __global__ __launch_bounds__(512, 2) void tile_dma_kernel(const bf16* __restrict
     constexpr int h = decltype(HALF)::value;
 #pragma unroll
     for (int q = h ? LW0 : 0; q < (h ? LW0 + LW1 : LW0); ++q)
-      dma16(W + kt * DMA_BK, gw[q], __builtin_amdgcn_readfirstlane(lw[q] + st * W_ST));
+      dma16(W + kt * wk, gw[q], __builtin_amdgcn_readfirstlane(lw[q] + st * W_ST));
   };
   // fragment reads (16x16x32): row R, chunk 4 ks + fk of its 8, at position chunk ^ ((R >> 1) & 7)
   const int sw = (fr >> 1) & 7;
@@ -795,7 +803,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void tile_step_kernel(const
                                                        const bf16* __restrict__ W, int ldw,
                                                        const float* __restrict__ bias, void* __restrict__ C,
                                                        int ldc, int M, int N, int K, int epi, int tiles_m,
-                                                       int order, int k_per_split,
+                                                       int order, int k_per_split, bool tiled,
                                                        const RowGroup* __restrict__ groups = nullptr,
                                                        const float* __restrict__ in_ssq = nullptr, int in_parts = 0,
                                                        float in_eps = 0.f, Halves halves = Halves{}) {
@@ -806,7 +814,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void tile_step_kernel(const
   if (k_per_split > 0) {                                     // as in tile_dma_kernel
     const int kb = part * k_per_split;
     A += kb;
-    W += kb;
+    W += tiled ? kb * 16 : kb;
     K = min(k_per_split, K - kb);
     C = (float*)C + (size_t)part * M * N;
   }
@@ -841,14 +849,14 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void tile_step_kernel(const
 #pragma unroll
   for (int q = 0; q < LW; ++q) {
     const int r = (q * WAVES + wid) * 8 + (lane >> 3);
-    gw[q] = ((unsigned)(HALVES ? halves.row(n0 + r) : min(n0 + r, N - 1)) * (unsigned)ldw + ((lane & 7) ^ ((r >> 1) & 7)) * 8) * 2u;
+    gw[q] = w_copy_at(HALVES ? halves.row(n0 + r) : min(n0 + r, N - 1), ldw, (lane & 7) ^ ((r >> 1) & 7), tiled);
   }
   const int nkt = K / DMA_BK;
   auto copy = [&](int kt, int st) {                          // (past the last tile: that one again, never read)
-    const int k = min(kt, nkt - 1) * DMA_BK;
+    const int k = min(kt, nkt - 1) * DMA_BK, kw = tiled ? k * 16 : k;
     const unsigned base = lds0 + st * ST + wid * 1024;
 #pragma unroll
-    for (int q = 0; q < LW; ++q) dma16(W + k, gw[q], __builtin_amdgcn_readfirstlane(base + BM * ROW + q * (WAVES * 1024)));
+    for (int q = 0; q < LW; ++q) dma16(W + kw, gw[q], __builtin_amdgcn_readfirstlane(base + BM * ROW + q * (WAVES * 1024)));
 #pragma unroll
     for (int q = 0; q < LA; ++q) dma16(A + k, ga[q], __builtin_amdgcn_readfirstlane(base + q * (WAVES * 1024)));
   };
@@ -940,7 +948,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void tile_step_kernel(const
 template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, bool GROUPED, bool SCALED = false, bool HALVES = false>
 int launch_tile_step(const bf16* A, int lda, const bf16* W, int ldw, const float* bias, void* C, int ldc, int M, int N, int K, int epi,
                      hipStream_t stream, int splits, int k_per_split, const RowGroup* groups, int n_groups,
-                     const float* in_ssq = nullptr, int in_parts = 0, float in_eps = 0.f, const Halves& halves = Halves{}) {
+                     const float* in_ssq = nullptr, int in_parts = 0, float in_eps = 0.f, const Halves& halves = Halves{}, bool tiled = false) {
   using TT = StepTile<BM, BN, WAVES_M, WAVES_N>;
   auto kern = tile_step_kernel<BM, BN, WAVES_M, WAVES_N, STAGES, GROUPED, SCALED, HALVES>;
   static bool configured = false;
@@ -952,16 +960,16 @@ int launch_tile_step(const bf16* A, int lda, const bf16* W, int ldw, const float
   }
   const int tiles_m = GROUPED ? n_groups : (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
   kern<<<dim3(tiles_m * tiles_n, splits), 64 * TT::WAVES, TT::template lds<STAGES>(), stream>>>(
-      A, lda, W, ldw, bias, C, ldc, M, N, K, epi, tiles_m, tile_order(tiles_m * tiles_n, splits, M, N, K), k_per_split, groups, in_ssq, in_parts, in_eps, halves);
+      A, lda, W, ldw, bias, C, ldc, M, N, K, epi, tiles_m, tile_order(tiles_m * tiles_n, splits, M, N, K), k_per_split, tiled, groups, in_ssq, in_parts, in_eps, halves);
   return mf_launch_status();
 }
 
 // 64 x 64: five stages, so that two blocks fit a CU (ten for blocks that have a CU to themselves: level)
 template <bool SCALED>
 int launch_tile64(const bf16* A, int lda, const bf16* W, int ldw, const float* bias, void* C, int ldc, int M, int N, int K, int epi,
-                  hipStream_t stream, int splits, int k_per_split, const float* in_ssq = nullptr, int in_parts = 0, float in_eps = 0.f) {
+                  hipStream_t stream, int splits, int k_per_split, bool tiled, const float* in_ssq = nullptr, int in_parts = 0, float in_eps = 0.f) {
   return launch_tile_step<64, 64, 2, 2, 5, false, SCALED>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi, stream, splits, k_per_split,
-                                                          nullptr, 0, in_ssq, in_parts, in_eps);
+                                                          nullptr, 0, in_ssq, in_parts, in_eps, Halves{}, tiled);
 }
 
 template <int BM, int BN, int STAGES, bool GROUPED, bool HALVES = false>
@@ -976,11 +984,11 @@ int configure_tile_dma() {
 
 template <int BM, int BN, int STAGES>
 int launch_tile_dma(const bf16* A, int lda, const bf16* W, int ldw, const float* bias, void* C, int ldc, int M,
-                    int N, int K, int epi, hipStream_t stream, int splits = 1, int k_per_split = 0) {
+                    int N, int K, int epi, hipStream_t stream, int splits, int k_per_split, bool tiled) {
   if (const int e = configure_tile_dma<BM, BN, STAGES, false>()) return e;
   const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
   tile_dma_kernel<BM, BN, STAGES><<<dim3(tiles_m * tiles_n, splits), 512, DmaTile<BM, BN>::template lds<STAGES>(), stream>>>(
-      A, lda, W, ldw, bias, C, ldc, M, N, K, epi, tiles_m, tile_order(tiles_m * tiles_n, splits, M, N, K), k_per_split, nullptr);
+      A, lda, W, ldw, bias, C, ldc, M, N, K, epi, tiles_m, tile_order(tiles_m * tiles_n, splits, M, N, K), k_per_split, tiled, nullptr);
   return mf_launch_status();
 }
 
@@ -1021,7 +1029,7 @@ int launch_grouped_dma(const bf16* A, int lda, const bf16* W, int ldw, void* C, 
   if (const int e = configure_tile_dma<BM, BN, STAGES, true, HALVES>()) return e;
   const int tiles_n = (N + BN - 1) / BN;
   tile_dma_kernel<BM, BN, STAGES, true, HALVES><<<dim3(n_groups * tiles_n), 512, DmaTile<BM, BN>::template lds<STAGES>(), stream>>>(
-      A, lda, W, ldw, nullptr, C, ldc, 0, N, K, EPI_F32, n_groups, n_groups * tiles_n >= 16, 0, groups, halves);
+      A, lda, W, ldw, nullptr, C, ldc, 0, N, K, EPI_F32, n_groups, n_groups * tiles_n >= 16, 0, false, groups, halves);
   return mf_launch_status();
 }
 
@@ -1031,7 +1039,7 @@ int launch_halves_dma(const bf16* A, int lda, const bf16* W, int ldw, bf16* C, i
   if (const int e = configure_tile_dma<BM, BN, STAGES, false, true>()) return e;
   const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
   tile_dma_kernel<BM, BN, STAGES, false, true><<<dim3(tiles_m * tiles_n), 512, DmaTile<BM, BN>::template lds<STAGES>(), stream>>>(
-      A, lda, W, ldw, nullptr, C, halves.width, M, N, K, EPI_SWIGLU, tiles_m, tile_order(tiles_m * tiles_n, 1, M, N, K), 0, nullptr, halves);
+      A, lda, W, ldw, nullptr, C, halves.width, M, N, K, EPI_SWIGLU, tiles_m, tile_order(tiles_m * tiles_n, 1, M, N, K), 0, false, nullptr, halves);
   return mf_launch_status();
 }
 
@@ -2354,7 +2362,8 @@ struct PanelTile {
 template <int I, int J, int RA, int STAGES, bool TURNS, bool PAIR>
 __global__ __launch_bounds__(512, 2) void panel_dma_kernel(const bf16* __restrict__ A, int lda, const bf16* __restrict__ W, int ldw,
                                                            const float* __restrict__ bias, void* __restrict__ C, int ldc, int M, int N,
-                                                           int K, int epi, const float* __restrict__ in_ssq, int in_parts, float in_eps) {
+                                                           int K, int epi, bool tiled, const float* __restrict__ in_ssq, int in_parts,
+                                                           float in_eps) {
   using T = PanelTile<I, J, RA, STAGES>;
   constexpr int WM = T::WM, BN = T::BN, P = T::P, L = T::L, ST = T::ST, ROW = DMA_BK * 2;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];      // [stage][RA rows of A, BN rows of W][64]
@@ -2399,16 +2408,16 @@ __global__ __launch_bounds__(512, 2) void panel_dma_kernel(const bf16* __restric
     const bool of_a = p * 8 < RA;
     const int row = of_a ? r : weight_row(r - RA);
     lanes[q] = __builtin_amdgcn_ballot_w64(p < P && row < (of_a ? M : N));
-    g[q] = ((unsigned)min(row, (of_a ? M : N) - 1) * (unsigned)(of_a ? lda : ldw) + c * 8) * 2u;
+    g[q] = of_a ? ((unsigned)min(row, M - 1) * (unsigned)lda + c * 8) * 2u : w_copy_at(min(row, N - 1), ldw, c, tiled);
     dst[q] = lds0 + min(p, P - 1) * 1024;
   }
   const int nkt = K / DMA_BK;
   auto copy = [&](int kt, int st) {                          // (past the last tile: that one again, never read)
-    const int k = min(kt, nkt - 1) * DMA_BK;
+    const int k = min(kt, nkt - 1) * DMA_BK, kw = tiled ? k * 16 : k;
 #pragma unroll
     for (int q = 0; q < L; ++q)
       asm volatile("s_mov_b32 m0, %2\n\ts_mov_b64 exec, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1\n\ts_mov_b64 exec, -1" ::"v"(g[q]),
-                   "s"((q * 8 + wid) * 8 < RA ? A + k : W + k), "s"(__builtin_amdgcn_readfirstlane(dst[q] + st * ST)), "s"(lanes[q])
+                   "s"((q * 8 + wid) * 8 < RA ? A + k : W + kw), "s"(__builtin_amdgcn_readfirstlane(dst[q] + st * ST)), "s"(lanes[q])
                    : "m0");
   };
   const int sw = (fr >> 1) & 7;
@@ -2540,7 +2549,7 @@ __global__ __launch_bounds__(512, 2) void panel_dma_kernel(const bf16* __restric
 
 template <int I, int J, int RA, int STAGES, bool TURNS>
 int launch_panel_dma(const bf16* A, int lda, const bf16* W, int ldw, const float* bias, void* C, int ldc, int M, int N, int K, int epi,
-                     const FusedNorm& fused, hipStream_t stream) {
+                     const FusedNorm& fused, bool tiled, hipStream_t stream) {
   using T = PanelTile<I, J, RA, STAGES>;
   auto run = [&](auto PAIR) {
     auto kern = panel_dma_kernel<I, J, RA, STAGES, TURNS, decltype(PAIR)::value>;
@@ -2550,7 +2559,8 @@ int launch_panel_dma(const bf16* A, int lda, const bf16* W, int ldw, const float
       if (e != hipSuccess) return (int)e;
       configured = true;
     }
-    kern<<<((N + 31) / 32 + J - 1) / J, 512, T::LDS, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi, fused.in_ssq, fused.in_parts, fused.in_eps);
+    kern<<<((N + 31) / 32 + J - 1) / J, 512, T::LDS, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi, tiled, fused.in_ssq, fused.in_parts,
+                                                                   fused.in_eps);
     return mf_launch_status();
   };
   return epi == EPI_SWIGLU ? run(std::true_type{}) : run(std::false_type{});
@@ -2969,17 +2979,42 @@ int dma_form(int variant, int M, int N, int K, int epi, long nkt, int splits, lo
   return best_form(FORM_128, FORM_TINY, M, N, K, nkt, splits, cu);
 }
 
-int launch_form(int form, const bf16* A, int lda, const bf16* W, int ldw, const float* bias, void* C, int ldc, int M, int N, int K,
+// A product's weights for the kernels that copy straight into LDS: the matrix, and its tiled copy where the caller has one (null: none).
+// A copy of 8 rows by 64 k is eight whole lines of the one, K elements apart, and of the other two runs of four lines, with the runs of
+// the neighbouring rows and k beside them, which memory gives faster (weights from memory, row-major / tiled: SwiGLU of 22,016 x 2,048, 40 rows
+// 26.1 / 21.8 us, 64 rows 24.0 / 20.5, 100 rows 27.0 / 24.7; 37,888 x 3,584, 64 rows 53.5 / 51.0, 203 rows 73.3 / 72.1, 604 rows 166.1 / 163.1;
+// 3,584 x 18,944, 604 rows in three parts 98.4 / 93.9; 4,608 x 3,584, 2,048 rows 63.9 / 61.2; level where many rows share the weights).
+// Not so 64 x 64 tiles of which no CU has two: their time is a chain of waits, with longer addresses in front of it
+// (2,560 x 2,048, 100 rows 7.4 / 7.7 us, 203 rows 10.0 / 10.4; 1,152 x 896, 604 rows 6.8 / 7.0).
+struct Weights {
+  const bf16* w;
+  const bf16* tiled;
+  int ldw, K;
+  Weights(const void* w_, const void* wt, int ldw_, int K_)
+      : w((const bf16*)w_), tiled(wt && (uintptr_t)wt % 16 == 0 && K_ % DMA_BK == 0 ? (const bf16*)wt : nullptr), ldw(ldw_), K(K_) {}
+  // from weight row n on (in 16s)
+  Weights from(int n) const { return Weights(w + (size_t)n * ldw, tiled ? tiled + (size_t)n * K : nullptr, ldw, K); }
+  const bf16* at(bool t) const { return t ? tiled : w; }
+  int ld(bool t) const { return t ? K : ldw; }
+};
+bool tile64_reads_tiled(const Weights& w, int M, int N, int splits) {
+  return w.tiled && (long)((M + 63) / 64) * ((N + 63) / 64) * splits > cu_count();
+}
+
+int launch_form(int form, const bf16* A, int lda, const Weights& w, const float* bias, void* C, int ldc, int M, int N, int K,
                 int epi, hipStream_t stream, int splits = 1, int k_per_split = 0) {
+  const bool t = form == FORM_TINY ? tile64_reads_tiled(w, M, N, splits) : w.tiled != nullptr;
+  const bf16* W = w.at(t);
+  const int ldw = w.ld(t);
   switch (form) {
-    case FORM_256: return launch_tile_dma<256, 256, 2>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi, stream, splits, k_per_split);
-    case FORM_192: return launch_tile_dma<256, 192, 2>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi, stream, splits, k_per_split);
-    case FORM_128: return launch_tile_dma<256, 128, 3>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi, stream, splits, k_per_split);
-    case FORM_128T: return launch_tile_dma<128, 256, 3>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi, stream, splits, k_per_split);
+    case FORM_256: return launch_tile_dma<256, 256, 2>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi, stream, splits, k_per_split, t);
+    case FORM_192: return launch_tile_dma<256, 192, 2>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi, stream, splits, k_per_split, t);
+    case FORM_128: return launch_tile_dma<256, 128, 3>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi, stream, splits, k_per_split, t);
+    case FORM_128T: return launch_tile_dma<128, 256, 3>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi, stream, splits, k_per_split, t);
   }
-  return form == FORM_SMALL
-             ? launch_tile_step<128, 128, 2, 4, 4, false>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi, stream, splits, k_per_split, nullptr, 0)
-             : launch_tile64<false>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi, stream, splits, k_per_split);
+  return form == FORM_SMALL ? launch_tile_step<128, 128, 2, 4, 4, false>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi, stream, splits, k_per_split,
+                                                                         nullptr, 0, nullptr, 0, 0.f, Halves{}, t)
+                            : launch_tile64<false>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi, stream, splits, k_per_split, t);
 }
 
 // A few weight rows past whole tiles (a gate beside q|k|v, a low-rank factor) can cost a whole round of them: 2,048 rows against
@@ -3099,9 +3134,11 @@ int panel_dma_units(int M, int N, int K, int epi, int n_cu) {
   return M > 50 && M <= 64 && epi == EPI_SWIGLU && K <= 2048 && units > 2 * n_cu && units <= 3 * n_cu ? 3 : 0;
 }
 
-int launch_panel_rows(int J, const bf16* A, int lda, const bf16* W, int ldw, const float* bias, void* C, int ldc, int M, int N, int K,
+int launch_panel_rows(int J, const bf16* A, int lda, const Weights& w, const float* bias, void* C, int ldc, int M, int N, int K,
                       int epi, const FusedNorm& fused, hipStream_t stream) {
-#define MF_PANEL(I_, J_, RA_, STAGES_, TURNS_) launch_panel_dma<I_, J_, RA_, STAGES_, TURNS_>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi, fused, stream)
+  const bool t = w.tiled != nullptr;
+#define MF_PANEL(I_, J_, RA_, STAGES_, TURNS_) \
+  launch_panel_dma<I_, J_, RA_, STAGES_, TURNS_>(A, lda, w.at(t), w.ld(t), bias, C, ldc, M, N, K, epi, fused, t, stream)
   if (M > 64) return MF_PANEL(2, 5, 128, 4, true);
   return J == 5 ? MF_PANEL(1, 5, 64, 5, false) : MF_PANEL(1, 3, 64, 6, false);
 #undef MF_PANEL
@@ -3261,7 +3298,7 @@ MF_API int mf_gemm_bf16_gated(const void* A, int lda, const void* W, int ldw, vo
 // panel kernel where it runs), 15: 256x192 (tests name them),
 // 16: the cheapest of all for the weight rows up to a multiple of 256, and of the small ones for up to 64 behind them; 17: the panel
 // kernel with copies straight into LDS.
-MF_API int mf_gemm_bf16(const void* A, int lda, const void* W, int ldw, const float* bias, void* C,
+MF_API int mf_gemm_bf16(const void* A, int lda, const void* W, const void* Wt, int ldw, const float* bias, void* C,
                         int ldc, int M, int N, int K, int epi, int variant, hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
   if (K <= 0 || lda < K || ldw < K || epi < 0 || epi > EPI_LAST || (epi == EPI_XIELU && !bias)) return (int)hipErrorInvalidValue;
@@ -3278,19 +3315,20 @@ MF_API int mf_gemm_bf16(const void* A, int lda, const void* W, int ldw, const fl
     if (plan.splits > 1) return (int)hipErrorInvalidValue;       // a K split needs the caller's workspace
     variant = plan.variant;
   }
+  const Weights wt(w, Wt, ldw, K);
   if (variant == 17 || (variant == 13 && M > 64 && dma_ok && panel_dma_units(M, N, K, epi, cu_count()))) {
     const int J = panel_dma_units(M, N, K, epi, cu_count());
     if (!J || !dma_ok) return (int)hipErrorInvalidValue;
-    return launch_panel_rows(J, a, lda, w, ldw, bias, C, ldc, M, N, K, epi, FusedNorm{}, stream);
+    return launch_panel_rows(J, a, lda, wt, bias, C, ldc, M, N, K, epi, FusedNorm{}, stream);
   }
   if (variant == 16) {
     const int n0 = main_rows(N, epi), cu = cu_count();
     if (!n0 || !dma_ok || cu <= 0) return (int)hipErrorInvalidValue;
     const long nkt = K / DMA_BK;
-    const int rc = launch_form(best_form(0, N_FORMS - 1, M, n0, K, nkt, 1, cu), a, lda, w, ldw, bias, C, ldc, M, n0, K, epi, stream);
+    const int rc = launch_form(best_form(0, N_FORMS - 1, M, n0, K, nkt, 1, cu), a, lda, wt, bias, C, ldc, M, n0, K, epi, stream);
     if (rc) return rc;
     void* rest = (char*)C + (size_t)n0 * (epi == EPI_BF16 || epi == EPI_RELU2 ? 2 : 4);
-    return launch_form(best_form(FORM_128, FORM_TINY, M, N - n0, K, nkt, 1, cu), a, lda, w + (size_t)n0 * ldw, ldw, bias ? bias + n0 : nullptr,
+    return launch_form(best_form(FORM_128, FORM_TINY, M, N - n0, K, nkt, 1, cu), a, lda, wt.from(n0), bias ? bias + n0 : nullptr,
                        rest, ldc, M, N - n0, K, epi, stream);
   }
   if (epi == EPI_SWIGLU && variant == 3) variant = 2;      // needs two 32-column tiles per wave
@@ -3302,7 +3340,7 @@ MF_API int mf_gemm_bf16(const void* A, int lda, const void* W, int ldw, const fl
     case 9: return launch_tile<256, 256, 128, 64, 64>(a, lda, w, ldw, bias, C, ldc, M, N, K, epi, vec_ok, stream);
     case 12: case 13: case 15:
       if (!dma_ok || (variant == 15 && epi == EPI_SWIGLU)) return (int)hipErrorInvalidValue;
-      return launch_form(dma_form(variant, M, N, K, epi, K / DMA_BK, 1, cu_count()), a, lda, w, ldw, bias, C, ldc, M, N, K, epi, stream);
+      return launch_form(dma_form(variant, M, N, K, epi, K / DMA_BK, 1, cu_count()), a, lda, wt, bias, C, ldc, M, N, K, epi, stream);
   }
   return (int)hipErrorInvalidValue;
 }
@@ -3311,7 +3349,7 @@ MF_API int mf_gemm_bf16(const void* A, int lda, const void* W, int ldw, const fl
 // some 50 tiles for 256 CUs): K is split over `splits` blocks per tile, which store 32-bit sums
 // into part[splits][M][N] (`mf_gemm_bf16_parts`), and skinny_reduce_kernel adds them and runs the epilogue.
 // k_per_split is a multiple of 64.
-MF_API int mf_gemm_bf16_parts(const void* A, int lda, const void* W, int ldw, float* part, int M, int N, int K, int splits,
+MF_API int mf_gemm_bf16_parts(const void* A, int lda, const void* W, const void* Wt, int ldw, float* part, int M, int N, int K, int splits,
                               int k_per_split, int variant, hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
   if (K <= 0 || lda < K || ldw < K || splits < 2 || !part || k_per_split % 64 != 0 || (long)splits * k_per_split < K ||
@@ -3325,19 +3363,19 @@ MF_API int mf_gemm_bf16_parts(const void* A, int lda, const void* W, int ldw, fl
   const bool dma_ok = vec_ok && K % DMA_BK == 0 && (size_t)M * lda * 2 < (1ull << 32) && (size_t)N * ldw * 2 < (1ull << 32);
   if (variant == 12 && !dma_ok) return (int)hipErrorInvalidValue;
   return dma_ok ? launch_form(dma_form(variant, M, N, K, EPI_F32, k_per_split / DMA_BK, splits, cu_count()), (const bf16*)A, lda,
-                              (const bf16*)W, ldw, nullptr, part, N, M, N, K, EPI_F32, stream, splits, k_per_split)
+                              Weights(W, Wt, ldw, K), nullptr, part, N, M, N, K, EPI_F32, stream, splits, k_per_split)
                 : launch_tile<128, 128, 64, 64>((const bf16*)A, lda, (const bf16*)W, ldw, nullptr, part, N, M,
                                                 N, K, EPI_F32, vec_ok, stream, splits, k_per_split);
 }
 
-MF_API int mf_gemm_bf16_splitk(const void* A, int lda, const void* W, int ldw, const float* bias, void* C,
+MF_API int mf_gemm_bf16_splitk(const void* A, int lda, const void* W, const void* Wt, int ldw, const float* bias, void* C,
                                int ldc, float* part, int M, int N, int K, int splits, int k_per_split,
                                int epi, int variant, hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
   if (epi < 0 || epi > EPI_LAST || (epi == EPI_XIELU && !bias)) return (int)hipErrorInvalidValue;
   if (epi == EPI_SWIGLU ? (N % 64 != 0 || ldc > N / 2 || ldc <= N / 2 - 32) : ldc < N)
     return (int)hipErrorInvalidValue;
-  const int rc = mf_gemm_bf16_parts(A, lda, W, ldw, part, M, N, K, splits, k_per_split, variant, stream);
+  const int rc = mf_gemm_bf16_parts(A, lda, W, Wt, ldw, part, M, N, K, splits, k_per_split, variant, stream);
   if (rc) return rc;
   return launch_reduce(part, bias, C, ldc, M, N, K, splits, epi, FusedNorm{}, stream);
 }
@@ -3345,7 +3383,7 @@ MF_API int mf_gemm_bf16_splitk(const void* A, int lda, const void* W, int ldw, c
 // The same into the residual stream (32-bit C, stored or added to), with the RMS norm of the new rows beside it: normed =
 // bfloat16 C / sqrt(mean(C^2) + eps) g, [M][N].  N in fours, at most 16,384, every operand 16-byte aligned; MF_NOT_BUILT
 // (nothing launched) for any other.
-MF_API int mf_gemm_bf16_splitk_norm(const void* A, int lda, const void* W, int ldw, const float* bias, float* C, int ldc,
+MF_API int mf_gemm_bf16_splitk_norm(const void* A, int lda, const void* W, const void* Wt, int ldw, const float* bias, float* C, int ldc,
                                     float* part, int M, int N, int K, int splits, int k_per_split, int accumulate, int variant,
                                     const float* g, float eps, void* normed, hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
@@ -3353,7 +3391,7 @@ MF_API int mf_gemm_bf16_splitk_norm(const void* A, int lda, const void* W, int l
       (uintptr_t)g % 16 || (uintptr_t)normed % 8 || !g || !normed)
     return MF_NOT_BUILT;
   if (ldc < N) return (int)hipErrorInvalidValue;
-  const int rc = mf_gemm_bf16_parts(A, lda, W, ldw, part, M, N, K, splits, k_per_split, variant, stream);
+  const int rc = mf_gemm_bf16_parts(A, lda, W, Wt, ldw, part, M, N, K, splits, k_per_split, variant, stream);
   if (rc) return rc;
   return launch_reduce_norm(part, bias, C, ldc, M, N, splits, accumulate, g, eps, (bf16*)normed, stream);
 }
@@ -3424,15 +3462,18 @@ static int skinny_product(const void* A, int lda, const void* W, const void* Wt,
     case SK_PANEL_SHORT: {
       // (32-bit byte offsets)
       const int J = (size_t)N * ldw * 2 < (1ull << 32) ? panel_dma_units(M, N, K, epi, cu_count()) : 0;
-      if (J) return launch_panel_rows(J, a, lda, w, ldw, bias, C, ldc, M, N, K, epi, fused, stream);
+      if (J) return launch_panel_rows(J, a, lda, Weights(w, wt, ldw, K), bias, C, ldc, M, N, K, epi, fused, stream);
       if (choice == SK_PANEL_SHORT) break;
       return launch_panel(a, lda, w, wt, ldw, bias, C, ldc, M, N, K, epi, fused, stream);
     }
-    case SK_TILE:
+    case SK_TILE: {
       if ((size_t)N * ldw * 2 >= (1ull << 32)) break;          // (operands beyond 4 GB go to the K-split kernels)
-      return fused.in_ssq ? launch_tile64<true>(a, lda, w, ldw, bias, C, ldc, M, N, K, epi, stream, 1, 0, fused.in_ssq, fused.in_parts,
-                                                fused.in_eps)
-                          : launch_tile64<false>(a, lda, w, ldw, bias, C, ldc, M, N, K, epi, stream, 1, 0);
+      const Weights both(w, wt, ldw, K);
+      const bool t = tile64_reads_tiled(both, M, N, 1);
+      return fused.in_ssq ? launch_tile64<true>(a, lda, both.at(t), both.ld(t), bias, C, ldc, M, N, K, epi, stream, 1, 0, t, fused.in_ssq,
+                                                fused.in_parts, fused.in_eps)
+                          : launch_tile64<false>(a, lda, both.at(t), both.ld(t), bias, C, ldc, M, N, K, epi, stream, 1, 0, t);
+    }
     default: break;
   }
   switch ((M + 15) / 16) {

@@ -137,15 +137,15 @@ _PROTOTYPES = {
         "mf_gemm_f32_swiglu": [_P, c_int, _P, c_int, _P, c_int, c_int, c_int, c_int, c_float, _P],
     },
     "gemm_bf16": {
-        "mf_gemm_bf16": [_P, c_int, _P, c_int, _P, _P, c_int, c_int, c_int, c_int, c_int, c_int, _P],
+        "mf_gemm_bf16": [_P, c_int, _P, _P, c_int, _P, _P, c_int, c_int, c_int, c_int, c_int, c_int, _P],
         "mf_gemm_bf16_grouped": [_P, _P, _P, _P, c_int, c_int, c_int, c_int, _P],
         "mf_gemm_bf16_grouped_gated": [_P, _P, _P, _P, c_int, c_int, c_int, c_int, c_int, c_float, _P],
         "mf_gemm_bf16_gated_pays": [c_int, c_int, c_int, c_int, c_int],
         "mf_gemm_bf16_gated": [_P, c_int, _P, c_int, _P, c_int, c_int, c_int, c_int, c_float, _P, c_int, _P],
-        "mf_gemm_bf16_splitk": [_P, c_int, _P, c_int, _P, _P, c_int, _P, c_int, c_int, c_int, c_int, c_int, c_int,
+        "mf_gemm_bf16_splitk": [_P, c_int, _P, _P, c_int, _P, _P, c_int, _P, c_int, c_int, c_int, c_int, c_int, c_int,
                                 c_int, _P],
-        "mf_gemm_bf16_parts": [_P, c_int, _P, c_int, _P, c_int, c_int, c_int, c_int, c_int, c_int, _P],
-        "mf_gemm_bf16_splitk_norm": [_P, c_int, _P, c_int, _P, _P, c_int, _P, c_int, c_int, c_int, c_int, c_int, c_int, c_int,
+        "mf_gemm_bf16_parts": [_P, c_int, _P, _P, c_int, _P, c_int, c_int, c_int, c_int, c_int, c_int, _P],
+        "mf_gemm_bf16_splitk_norm": [_P, c_int, _P, _P, c_int, _P, _P, c_int, _P, c_int, c_int, c_int, c_int, c_int, c_int, c_int,
                                      _P, c_float, _P, _P],
         "mf_gemm_bf16_skinny": [_P, c_int, _P, _P, c_int, _P, _P, c_int, _P, c_int, c_int, c_int, c_int,
                                 c_int, c_int, _P],
@@ -1852,8 +1852,8 @@ def plan_linear(m: int, n: int, k: int, swiglu: bool = False, normed: bool = Fal
 def tile_weight(weight: torch.Tensor) -> torch.Tensor:
     """The tiled copy of a bfloat16 `[n][k]` matrix, k a multiple of 32: `[ceil(n / 16)][k / 32][16][32]`,
     rows padded with zeros to a multiple of 16.  The products of at most 64 rows read their
-    weights a tile (a contiguous kilobyte) per wave and step from it; made once, when a model is
-    loaded, where memory allows a second copy."""
+    weights a tile (a contiguous kilobyte) per wave and step from it, those of more rows copy them from it; made once, when a
+    model is loaded, where memory allows a second copy."""
     _need(weight, "tile_weight.weight", torch.bfloat16)
     n, k = weight.shape
     if k % 32:
@@ -1875,7 +1875,7 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], 
     """out (+)= x @ weight^T (+ bias).  weight is [out][in].  float32 weights take the true
     32-bit kernel; bfloat16 weights take the matrix-core kernels (a few rows: the streaming
     kernel).  `out` is float32, or bfloat16 for a bfloat16 product that is stored.  `tiled`:
-    `tile_weight(weight)`, which the kernels for at most 64 rows read instead where they can.  `relu2`: a bfloat16 product's
+    `tile_weight(weight)`, which the kernels of every number of rows read instead where they can and where it is faster.  `relu2`: a bfloat16 product's
     sums go through max(z, 0)^2 before they are rounded."""
     _need(x, "linear.x", _FLOATS)
     _need(weight, "linear.weight", x.dtype)
@@ -1906,10 +1906,10 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], 
         raise KernelError("linear: accumulation needs a float32 output")
     epi = EPI_XIELU if xielu else EPI_RELU2 if relu2 else (EPI_BF16 if out.dtype == torch.bfloat16 else (EPI_ACC_F32 if accumulate else EPI_F32))
     aligned = not (x.data_ptr() % 16 or weight.data_ptr() % 16 or k % 8)
+    _need_tiled(tiled, "linear.tiled", n, k)
     if m <= 64 and variant == 0:
         splits, per = _k_split(m, n, k, False, aligned, tiled=tiled is not None)
         part = workspace("skinny", splits * m * n, x.device) if splits > 1 else None
-        _need_tiled(tiled, "linear.tiled", n, k)
         _check(_fn("gemm_bf16", "mf_gemm_bf16_skinny")(x, k, weight, tiled, k, bias,
                                                         out, n, part, m, n, k, splits, per,
                                                         epi, _stream()), f"gemm_bf16_skinny {m}x{n}x{k}")
@@ -1918,15 +1918,15 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], 
         variant, splits, per = tile_plan(m, n, k, epi, aligned)
         if splits > 1:
             part = workspace("skinny", splits * m * n, x.device)
-            _check(_fn("gemm_bf16", "mf_gemm_bf16_splitk")(x, k, weight, k, bias, out, n,
+            _check(_fn("gemm_bf16", "mf_gemm_bf16_splitk")(x, k, weight, tiled, k, bias, out, n,
                                                             part, m, n, k, splits, per, epi, variant,
                                                             _stream()), f"gemm_bf16_splitk {m}x{n}x{k}")
             return
-    _check(_fn("gemm_bf16", "mf_gemm_bf16")(x, k, weight, k, bias, out, n, m,
+    _check(_fn("gemm_bf16", "mf_gemm_bf16")(x, k, weight, tiled, k, bias, out, n, m,
                                              n, k, epi, variant, _stream()), f"gemm_bf16 {m}x{n}x{k}")
 
 
-def linear_parts(x: torch.Tensor, weight: torch.Tensor) -> Optional[torch.Tensor]:
+def linear_parts(x: torch.Tensor, weight: torch.Tensor, tiled: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
     """The product of more than 64 bfloat16 rows, or of 32-bit rows, cut over K, its parts not yet added: float32 `[parts][m][n]` (without
     bias; of bfloat16 rows in the scratch the next split product reuses), or None, nothing launched, where it is better not cut.
     32-bit rows are cut as `linear` cuts them; bfloat16 rows more often (`plan_linear` with `behind` 1), since the kernel behind the
@@ -1949,14 +1949,15 @@ def linear_parts(x: torch.Tensor, weight: torch.Tensor) -> Optional[torch.Tensor
     variant, splits, per = _tile_plan(m, n, k, EPI_F32, not (x.data_ptr() % 16 or weight.data_ptr() % 16 or k % 8), cu_count(), 1)
     if splits <= 1:
         return None
+    _need_tiled(tiled, "linear_parts.tiled", n, k)
     part = workspace("skinny", splits * m * n, x.device)[:splits * m * n].view(splits, m, n)
-    _check(_fn("gemm_bf16", "mf_gemm_bf16_parts")(x, k, weight, k, part, m, n, k, splits, per, variant,
+    _check(_fn("gemm_bf16", "mf_gemm_bf16_parts")(x, k, weight, tiled, k, part, m, n, k, splits, per, variant,
                                                    _stream()), f"gemm_bf16_parts {m}x{n}x{k}")
     return part
 
 
 def linear_norm_out(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], out: torch.Tensor, accumulate: bool,
-                    g: torch.Tensor, eps: float) -> Optional[torch.Tensor]:
+                    g: torch.Tensor, eps: float, tiled: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
     """out (+)= x weight^T (+ bias) for more than 64 bfloat16 rows, or 32-bit rows, into float32 `out`, where the product is better cut
     over K, and out / sqrt(mean(out^2) + eps) g in x's type, which the kernel that adds the parts leaves beside it and
     which is returned.  None, nothing launched, for any other shape."""
@@ -1976,9 +1977,10 @@ def linear_norm_out(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.
     _need(g, "linear_norm_out.g", torch.float32, (n,))
     if bias is not None:
         _need(bias, "linear_norm_out.bias", torch.float32, (n,))
+    _need_tiled(tiled, "linear_norm_out.tiled", n, k)
     normed = torch.empty((m, n), dtype=torch.bfloat16, device=x.device)
     part = workspace("skinny", splits * m * n, x.device)
-    rc = _fn("gemm_bf16", "mf_gemm_bf16_splitk_norm")(x, k, weight, k, bias, out, n, part, m, n, k,
+    rc = _fn("gemm_bf16", "mf_gemm_bf16_splitk_norm")(x, k, weight, tiled, k, bias, out, n, part, m, n, k,
                                                       splits, per, 1 if accumulate else 0, variant, g, float(eps),
                                                       normed, _stream())
     if rc == NOT_BUILT:
@@ -2162,10 +2164,10 @@ def linear_swiglu(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor, vari
     if m == 0:
         return
     aligned = not (x.data_ptr() % 16 or weight.data_ptr() % 16 or k % 8)
+    _need_tiled(tiled, "linear_swiglu.tiled", n, k)
     if m <= 64 and variant == 0:
         splits, per = _k_split(m, n, k, True, aligned, tiled=tiled is not None)
         part = workspace("skinny", splits * m * n, x.device) if m > 16 or splits > 1 else None
-        _need_tiled(tiled, "linear_swiglu.tiled", n, k)
         _check(_fn("gemm_bf16", "mf_gemm_bf16_skinny")(x, k, weight, tiled, k, limit, out, nf,
                                                         part, m, n, k, splits, per, EPI_SWIGLU, _stream()),
                f"gemm_bf16_skinny(swiglu) {m}x{n}x{k}")
@@ -2174,11 +2176,11 @@ def linear_swiglu(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor, vari
         variant, splits, per = tile_plan(m, n, k, EPI_SWIGLU, aligned)
         if splits > 1:
             part = workspace("skinny", splits * m * n, x.device)
-            _check(_fn("gemm_bf16", "mf_gemm_bf16_splitk")(x, k, weight, k, limit, out, nf,
+            _check(_fn("gemm_bf16", "mf_gemm_bf16_splitk")(x, k, weight, tiled, k, limit, out, nf,
                                                             part, m, n, k, splits, per, EPI_SWIGLU, variant,
                                                             _stream()), f"gemm_bf16_splitk(swiglu) {m}x{n}x{k}")
             return
-    _check(_fn("gemm_bf16", "mf_gemm_bf16")(x, k, weight, k, limit, out, nf, m, n, k,
+    _check(_fn("gemm_bf16", "mf_gemm_bf16")(x, k, weight, tiled, k, limit, out, nf, m, n, k,
                                              EPI_SWIGLU, variant, _stream()), f"gemm_bf16(swiglu) {m}x{n}x{k}")
 
 

@@ -32,7 +32,7 @@ class Linear:
         return self.weight, self.tiled, self.bias
 
     def decode_copy(self, make: bool, min_row_length: int = 0) -> int:
-        """Bytes of the tiled copy of this matrix, which the products of few rows read faster than
+        """Bytes of the tiled copy of this matrix, which the products (of few rows above all) read faster than
         the matrix itself (0: it has none: 32-bit, a row length that is no multiple of 32, or a
         row shorter than `min_row_length`: the long rows gain most); made when `make`."""
         if self.weight.dtype != torch.bfloat16 or self.in_features % 32 or self.in_features < min_row_length:
@@ -95,7 +95,7 @@ class Linear:
             x = x.tensor()
         if x.device.type != "cuda" or x.shape[0] <= 64 or x.dtype != self.weight.dtype:
             return None
-        return ops.linear_parts(x, self.weight)
+        return ops.linear_parts(x, self.weight, tiled=self.tiled)
 
     def _prepare_norm(self, x: torch.Tensor, out: torch.Tensor, accumulate: bool, ctx) -> bool:
         """Runs the product with the next norm's input prepared beside it (bf16(out g) and the rows'
@@ -114,7 +114,7 @@ class Linear:
             fold = norm.rms_scale()
             if fold is None or fold[0].numel() != self.out_features:
                 return False
-            normed = ops.linear_norm_out(x, self.weight, self.bias, out, accumulate, fold[0], fold[1])
+            normed = ops.linear_norm_out(x, self.weight, self.bias, out, accumulate, fold[0], fold[1], tiled=self.tiled)
             if normed is None:
                 return False
             ctx.norm_ahead = NormAhead(norm, out, normed, None)
