@@ -101,6 +101,15 @@ __device__ __forceinline__ bf16x8 load8_inside(const bf16* __restrict__ base, in
   return *reinterpret_cast<const bf16x8*>(base + (size_t)row * ld + k);
 }
 
+// Weights that no other workgroup reads, marked as read once: a stream of them alone comes at 6.2 TB/s so and at 5.9 without the mark
+// (a plain read of 670 MB by 256 workgroups), and what the step reads again stays in the caches.  With the last loads of a block no
+// longer there only to be dropped, and no wait for the weights in flight in front of an item (microseconds before / after, 8 rows, weights from
+// memory): 37,888 x 3,584 50.5 / 44.2 (6.1 TB/s), 4,608 x 3,584 10.4 / 8.4, 3,584 x 3,584 8.4 / 7.2, 3,584 x 18,944 26.0 / 24.9, 152,064 x 3,584 192 / 172,
+// 9,728 x 896 6.5 / 5.6, 151,936 x 896 63 / 49.  Not for what several tiles of rows read (`whole_kernel`, the prompts' tiles).
+__device__ __forceinline__ bf16x8 load_weights(const bf16* p) {
+  return __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(p));
+}
+
 // The epilogue of a wave's TM x TN tiles of 32 x 32 (D[m][n]: lane holds n = lane % 32,
 // m = 8 (r / 4) + 4 (lane / 32) + r % 4): bias, then store / accumulate / round / SwiGLU.
 template <int TM, int TN>
@@ -156,11 +165,11 @@ __device__ __forceinline__ void tile_epilogue(floatx16 (&acc)[TM][TN], const flo
 // 32 tile rows would share 33).
 __device__ __forceinline__ void tile_position(int tile, int tiles_m, int tiles_n, int& bm, int& bn) {
   constexpr int BAND = 8;
-  const int band = tile / (BAND * tiles_n), first = band * BAND;
+  const int band = (tile / (BAND * tiles_n)), first = band * BAND;
   const int rows = min(tiles_m - first, BAND);
   const int in_band = tile - band * BAND * tiles_n;
-  bm = first + in_band % rows;
-  bn = in_band / rows;
+  bn = (in_band / rows);
+  bm = first + in_band - bn * rows;
 }
 
 // The tile and the part of K that a block of a grid of (tiles, parts) takes.  Workgroups go to the 8 XCDs in turn, each with an
@@ -179,8 +188,9 @@ __device__ __forceinline__ void block_work(int order, int& tile, int& part) {
     const int per = n / 8, rem = n % 8, x = at % 8;
     at = x * per + min(x, rem) + at / 8;
   }
-  part = order == ORDER_PARTS ? at / (int)gridDim.x : blockIdx.y;
-  tile = order == ORDER_PARTS ? at - part * (int)gridDim.x : at;
+  // (a division is vector work; the same in the whole block all the same, and what hangs on it stays in scalar registers so)
+  part = (order == ORDER_PARTS ? at / (int)gridDim.x : blockIdx.y);
+  tile = (order == ORDER_PARTS ? at - part * (int)gridDim.x : at);
 }
 // Part by part where the activations of all of K are half as much again as an XCD's L2 of 4 MB and all parts' tiles are at most two a
 // CU.  (rows x weight rows x K, microseconds with the kernel behind it, the same eighth of every part / part by part: 800 x 1,536 x
@@ -359,6 +369,18 @@ constexpr int DMA_BK = 64;
 __device__ __forceinline__ void dma16(const bf16* base, unsigned off, unsigned lds_byte) {
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds_byte)
                : "m0");
+}
+// The lanes of a mask, of weights that no other workgroup reads (ONCE, see `load_weights`) or of anything else
+template <bool ONCE>
+__device__ __forceinline__ void dma16_lanes(const bf16* base, unsigned off, unsigned lds_byte, unsigned long long lanes) {
+  if constexpr (ONCE)
+    asm volatile("s_mov_b32 m0, %2\n\ts_mov_b64 exec, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt\n\ts_mov_b64 exec, -1" ::"v"(off), "s"(base),
+                 "s"(lds_byte), "s"(lanes)
+                 : "m0");
+  else
+    asm volatile("s_mov_b32 m0, %2\n\ts_mov_b64 exec, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1\n\ts_mov_b64 exec, -1" ::"v"(off), "s"(base),
+                 "s"(lds_byte), "s"(lanes)
+                 : "m0");
 }
 // at most N of this wave's youngest copies are in flight, and all its LDS reads are back
 template <int N>
@@ -745,28 +767,37 @@ __global__ __launch_bounds__(512, 2) void tile_dma_kernel(const bf16* __restrict
 // kernel asks early and adds late: every lane asks for Q x 4 of them at once, one value a load (with 16-byte loads beside them where
 // the rows allow it the compiler waited for each row's first before the next: a trip to memory for every row of a lane, in front of the
 // product's first copies; gate|up of 37 rows with 84 parts a row 11.2 us so, 9.8 now), and for what is left of a longer row when it
-// adds up.  A row without parts (p null) asks for nothing and gives 0.
-template <int LANES, int Q>
+// adds up.  ALL: no load stands behind a condition (a place past the row's end asks for the last one again), for a kernel whose own
+// loads the compiler counts: behind one it counts with the way that has fewer in flight.  Elsewhere places past the end ask for nothing.
+// A row without parts (p null, for all lanes alike) asks for nothing and gives 0.
+template <int LANES, int Q, bool ALL = false>
 struct LanesSum {
   float x[Q][4];
   __device__ __forceinline__ void ask(const float* __restrict__ p, int parts, int l) {
+    if constexpr (!ALL) {
+#pragma unroll
+      for (int q = 0; q < Q; ++q)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[q][e] = 0.f;
+      if (!p) return;
+    }
 #pragma unroll
     for (int q = 0; q < Q; ++q)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) x[q][e] = 0.f;
-    if (!p) return;
-#pragma unroll
-    for (int q = 0; q < Q; ++q)
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if ((q * 4 + e) * LANES + l < parts) x[q][e] = p[(q * 4 + e) * LANES + l];
+      for (int e = 0; e < 4; ++e) {
+        const int i = (q * 4 + e) * LANES + l;
+        if constexpr (ALL) x[q][e] = p ? p[min(i, parts - 1)] : 0.f;
+        else if (i < parts) x[q][e] = p[i];
+      }
   }
   __device__ __forceinline__ float add(const float* __restrict__ p, int parts, int l) const {
     float t = 0.f;
+    if (p) {
+      auto of = [&](int q, int e) { return (q * 4 + e) * LANES + l < parts ? x[q][e] : 0.f; };
 #pragma unroll
-    for (int q = 0; q < Q; ++q) t += (x[q][0] + x[q][1]) + (x[q][2] + x[q][3]);
-    if (p)
+      for (int q = 0; q < Q; ++q) t += (of(q, 0) + of(q, 1)) + (of(q, 2) + of(q, 3));
       for (int i = Q * LANES * 4 + l; i < parts; i += LANES) t += p[i];
+    }
 #pragma unroll
     for (int o = LANES / 2; o > 0; o >>= 1) t += __shfl_xor(t, o, MF_WAVE);
     return t;
@@ -865,8 +896,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void tile_step_kernel(const
   constexpr int GROUPS = (BM + WAVES * 8 - 1) / (WAVES * 8);
   LanesSum<8, 4> sums[SCALED ? GROUPS : 1];
   auto part_row = [&](int q) {
-    const int r = m0 + (q * WAVES + wid) * 8 + (lane >> 3);
-    return r < M ? in_ssq + (size_t)r * in_parts : nullptr;
+    return in_ssq + (size_t)min(m0 + (q * WAVES + wid) * 8 + (lane >> 3), M - 1) * in_parts;      // (rows past M: not stored)
   };
   if constexpr (SCALED) {
 #pragma unroll
@@ -1195,7 +1225,7 @@ __global__ __launch_bounds__(512) void skinny_ring_kernel(const bf16* __restrict
 #pragma unroll
   for (int i = 0; i < MT; ++i) stage[i] = *reinterpret_cast<const bf16x8*>(src[i] + k_begin);
 #pragma unroll
-  for (int s = 0; s < KC / 32; ++s) wr[s] = *reinterpret_cast<const bf16x8*>(wrow + ((k_begin >> 5) + s) * WSTEP);
+  for (int s = 0; s < KC / 32; ++s) wr[s] = load_weights(wrow + ((k_begin >> 5) + s) * WSTEP);
 #pragma unroll
   for (int i = 0; i < MT; ++i)
     *reinterpret_cast<bf16x8*>(&As[(i * 16 + (tid >> 5)) * SK_LD + sk]) = stage[i];
@@ -1204,11 +1234,14 @@ __global__ __launch_bounds__(512) void skinny_ring_kernel(const bf16* __restrict
 #pragma unroll
   for (int i = 0; i < MT; ++i) acc[i] = floatx4{0.f, 0.f, 0.f, 0.f};
   int buf = 0;
-  for (int k0 = k_begin; k0 < k_end; k0 += KC) {
-    const int kn = k0 + KC < k_end ? k0 + KC : k_begin;     // behind the last chunk: the first again, dropped
+  // a chunk's products, the next chunk asked for beside them (behind the last chunk nothing is: 64 KB of weights a block)
+  auto chunk = [&](int kn, auto REFILL) {
+    constexpr bool refill = decltype(REFILL)::value;
+    if constexpr (refill) {
 #pragma unroll
-    for (int i = 0; i < MT; ++i) stage[i] = *reinterpret_cast<const bf16x8*>(src[i] + kn);
-    __builtin_amdgcn_sched_barrier(0);
+      for (int i = 0; i < MT; ++i) stage[i] = *reinterpret_cast<const bf16x8*>(src[i] + kn);
+      __builtin_amdgcn_sched_barrier(0);
+    }
     const bf16* as = As + buf * ROWS * SK_LD;
 #pragma unroll
     for (int s = 0; s < KC / 32; ++s) {
@@ -1217,15 +1250,21 @@ __global__ __launch_bounds__(512) void skinny_ring_kernel(const bf16* __restrict
         const bf16x8 a = *reinterpret_cast<const bf16x8*>(&as[(i * 16 + r16) * SK_LD + s * 32 + kq]);
         acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, wr[s], acc[i], 0, 0, 0);
       }
-      wr[s] = *reinterpret_cast<const bf16x8*>(wrow + ((kn >> 5) + s) * WSTEP);
-      __builtin_amdgcn_sched_barrier(0);      // use a register, then refill it, in this order
+      if constexpr (refill) {
+        wr[s] = load_weights(wrow + ((kn >> 5) + s) * WSTEP);
+        __builtin_amdgcn_sched_barrier(0);    // use a register, then refill it, in this order
+      }
     }
-    buf ^= 1;
+    if constexpr (refill) {
+      buf ^= 1;
 #pragma unroll
-    for (int i = 0; i < MT; ++i)
-      *reinterpret_cast<bf16x8*>(&As[(buf * ROWS + i * 16 + (tid >> 5)) * SK_LD + sk]) = stage[i];
-    __syncthreads();
-  }
+      for (int i = 0; i < MT; ++i)
+        *reinterpret_cast<bf16x8*>(&As[(buf * ROWS + i * 16 + (tid >> 5)) * SK_LD + sk]) = stage[i];
+      __syncthreads();
+    }
+  };
+  for (int kn = k_begin + KC; kn < k_end; kn += KC) chunk(kn, std::true_type{});
+  chunk(0, std::false_type{});
   // D[m][n]: n = lane % 16, m = 4 (lane / 16) + r
 #pragma unroll
   for (int i = 0; i < MT; ++i)
@@ -1444,35 +1483,34 @@ struct FusedNorm {
 // 1 / sqrt(mean(x^2) + eps) of NR rows from their partial sums, K the rows' length, in two steps
 // so that a kernel can ask for the sums early and use them late; all lanes of a wave call both with
 // the same rows (a row outside [0, M) gives 1).  The lanes take the partial sums between them, all
-// rows' loads in flight together, and add up in a fixed tree.
+// rows' loads in flight together, and add up in a fixed tree.  None of the first loads stands behind a condition but `in_ssq` itself
+// (see LanesSum; with a condition a load the 7B shape's gate|up of 8 rows waited two trips to memory before it asked for weights).
 template <int NR>
-__device__ __forceinline__ void row_sums_ask(const FusedNorm& f, const int (&rows)[NR], int M, int lane, float (&t)[NR]) {
-  constexpr int AT_ONCE = 4;             // of a row, asked for at once (as many as a product of one block a CU leaves)
+struct RowSums {
+  static constexpr int AT_ONCE = 4;      // of a row, asked for at once (as many as a product of one block a CU leaves)
   float x[NR][AT_ONCE];
+  __device__ __forceinline__ void ask(const FusedNorm& f, const int (&rows)[NR], int M, int lane) {
 #pragma unroll
-  for (int i = 0; i < NR; ++i)
+    for (int i = 0; i < NR; ++i)
 #pragma unroll
-    for (int q = 0; q < AT_ONCE; ++q)
-      x[i][q] = rows[i] >= 0 && rows[i] < M && lane + q * 64 < f.in_parts ? f.in_ssq[(size_t)rows[i] * f.in_parts + lane + q * 64] : 0.f;
-#pragma unroll
-  for (int i = 0; i < NR; ++i) {
-    t[i] = 0.f;
-#pragma unroll
-    for (int q = 0; q < AT_ONCE; ++q) t[i] += x[i][q];
-    if (rows[i] >= 0 && rows[i] < M)
-      for (int p = lane + AT_ONCE * 64; p < f.in_parts; p += 64) t[i] += f.in_ssq[(size_t)rows[i] * f.in_parts + p];
+      for (int q = 0; q < AT_ONCE; ++q)
+        x[i][q] = f.in_ssq ? f.in_ssq[(size_t)min(max(rows[i], 0), M - 1) * f.in_parts + min(lane + q * 64, f.in_parts - 1)] : 0.f;
   }
-}
-
-template <int NR>
-__device__ __forceinline__ void row_factors_of(const FusedNorm& f, const int (&rows)[NR], int M, int K, float (&t)[NR]) {
+  __device__ __forceinline__ void factors(const FusedNorm& f, const int (&rows)[NR], int M, int K, int lane, float (&t)[NR]) const {
 #pragma unroll
-  for (int i = 0; i < NR; ++i) {
+    for (int i = 0; i < NR; ++i) {
+      const bool row = f.in_ssq && rows[i] >= 0 && rows[i] < M;
+      t[i] = 0.f;
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) t[i] += __shfl_xor(t[i], o, MF_WAVE);
-    t[i] = (rows[i] >= 0 && rows[i] < M) ? 1.0f / sqrtf(t[i] / (float)K + f.in_eps) : 1.f;
+      for (int q = 0; q < AT_ONCE; ++q) t[i] += row && lane + q * 64 < f.in_parts ? x[i][q] : 0.f;
+      if (row)
+        for (int p = lane + AT_ONCE * 64; p < f.in_parts; p += 64) t[i] += f.in_ssq[(size_t)rows[i] * f.in_parts + p];
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) t[i] += __shfl_xor(t[i], o, MF_WAVE);
+      t[i] = row ? 1.0f / sqrtf(t[i] / (float)K + f.in_eps) : 1.f;
+    }
   }
-}
+};
 
 
 // End of a one-kernel product of at most 16 rows that prepares the next norm (FusedNorm::out_*):
@@ -1522,8 +1560,8 @@ __global__ __launch_bounds__(NW * 64) void rolling16_kernel(const bf16* __restri
     return PAIR ? tile_row(j) + r16 : blockIdx.x * rpb + min(j * 16 + r16, rpb - 1);
   };
   const int total = K / 32;
-  const int first = min(wid * steps_per_wave, total);
-  const int T = min(steps_per_wave, total - first);       // steps of this wave
+  const int T = min(steps_per_wave, total - wid * steps_per_wave);       // steps of this wave (none: not above 0)
+  const int first = T > 0 ? wid * steps_per_wave : 0;
   const int kq = first * 32 + (lane >> 4) * 8;
   const bf16* arow = A + (size_t)min(r16, M - 1) * lda + kq;
   const bf16* wrow[NT];
@@ -1545,64 +1583,52 @@ __global__ __launch_bounds__(NW * 64) void rolling16_kernel(const bf16* __restri
   float c_old = 0.f, e_g = 0.f;
   if (epi == EPI_ACC_F32 && e_mine) c_old = ((const float*)C)[(size_t)e_m * ldc + e_n];
   if (fused.out_g && e_mine) e_g = fused.out_g[e_n];       // the next norm's weight, where this product prepares it
-  const int R = T / S, rem = T % S;
-  if (R == 0) {       // a slice shorter than the registers hold: all of it asked for at once (in a loop over the slice's length the
-                      // compiler waits for every step: a decode step of one sequence at the 0.5B widths 775 us so, 749 at once)
-    bf16x8 a[S], w[NT][S];
+  bf16x8 a[S], w[NT][S];
+  auto load = [&](int s, int at) {
+#pragma unroll
+    for (int j = 0; j < NT; ++j) w[j][s] = load_weights(wrow[j] + at * WSTEP);
+    a[s] = *reinterpret_cast<const bf16x8*>(arow + at * 32);
+  };
+  auto multiply = [&](int s) {
+#pragma unroll
+    for (int j = 0; j < NT; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[s], w[j][s], acc[j], 0, 0, 0);
+  };
+  if (steps_per_wave <= S) {   // a slice that the registers hold: all of it asked for at once (in a loop over the slice's length the
+                               // compiler waits for every step: a decode step of one sequence at the 0.5B widths 775 us so, 749 at once)
 #pragma unroll
     for (int s = 0; s < S; ++s)
-      if (s < T) {
-#pragma unroll
-        for (int j = 0; j < NT; ++j) w[j][s] = *reinterpret_cast<const bf16x8*>(wrow[j] + s * WSTEP);
-        a[s] = *reinterpret_cast<const bf16x8*>(arow + s * 32);
-      }
+      if (s < T) load(s, s);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int s = 0; s < S; ++s)
-      if (s < T) {
-#pragma unroll
-        for (int j = 0; j < NT; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[s], w[j][s], acc[j], 0, 0, 0);
-      }
+      if (s < T) multiply(s);
   } else {
-    bf16x8 a[S], w[NT][S];
+    // Rounds of S steps, a register refilled behind its product.  Every refill is there without a condition, so that the compiler can
+    // count what is in flight: past the slice's end it is the last step again (`rolling_steps` chooses S so that there are few).
+    const int last = max(T, 1) - 1;
 #pragma unroll
-    for (int s = 0; s < S; ++s) {
-      a[s] = *reinterpret_cast<const bf16x8*>(arow + s * 32);
-#pragma unroll
-      for (int j = 0; j < NT; ++j) w[j][s] = *reinterpret_cast<const bf16x8*>(wrow[j] + s * WSTEP);
-    }
-    // rounds whose refills all exist: no branch in the body
+    for (int s = 0; s < S; ++s) load(s, min(s, last));
     int base = 0;
-    for (int i = 0; i + 1 < R; ++i, base += S) {
+    for (; base + 2 * S <= T; base += S) {
 #pragma unroll
       for (int s = 0; s < S; ++s) {
-#pragma unroll
-        for (int j = 0; j < NT; ++j) {
-          acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[s], w[j][s], acc[j], 0, 0, 0);
-          w[j][s] = *reinterpret_cast<const bf16x8*>(wrow[j] + (base + S + s) * WSTEP);
-        }
-        a[s] = *reinterpret_cast<const bf16x8*>(arow + (base + S + s) * 32);
+        multiply(s);
+        load(s, base + S + s);
         __builtin_amdgcn_sched_barrier(0);
       }
     }
-    // the last whole round refills only what the remainder needs
+    if (base + S < T) {
 #pragma unroll
-    for (int s = 0; s < S; ++s) {
-#pragma unroll
-      for (int j = 0; j < NT; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[s], w[j][s], acc[j], 0, 0, 0);
-      if (s < rem) {
-        a[s] = *reinterpret_cast<const bf16x8*>(arow + (base + S + s) * 32);
-#pragma unroll
-        for (int j = 0; j < NT; ++j) w[j][s] = *reinterpret_cast<const bf16x8*>(wrow[j] + (base + S + s) * WSTEP);
+      for (int s = 0; s < S; ++s) {
+        multiply(s);
+        load(s, min(base + S + s, last));
+        __builtin_amdgcn_sched_barrier(0);
       }
+      base += S;
     }
 #pragma unroll
-    for (int s = 0; s < S; ++s) {
-      if (s < rem) {
-#pragma unroll
-        for (int j = 0; j < NT; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[s], w[j][s], acc[j], 0, 0, 0);
-      }
-    }
+    for (int s = 0; s < S; ++s)
+      if (base + s < T) multiply(s);
   }
   // D[m][n]: n = lane % 16, m = 4 (lane / 16) + r
 #pragma unroll
@@ -1639,21 +1665,35 @@ __global__ __launch_bounds__(NW * 64) void rolling16_kernel(const bf16* __restri
   if (fused.out_g) norm_part_out<COLS>(fused, sq, e_m, e_c, M);
 }
 
-template <int NW, int NT, int S, bool PAIR = false, bool TILED = false>
+// How many steps `rolling16_kernel` holds for slices of `steps`: at most 16, the one whose rounds have the fewest steps past the end.
+int rolling_steps(int steps) {
+  int best = 16;
+  for (int s = 15; s >= 10 && steps > 16; --s)
+    if ((steps + s - 1) / s * s < (steps + best - 1) / best * best) best = s;
+  return best;
+}
+
+template <bool TILED>
 int launch_rolling16(const bf16* A, int lda, const bf16* W, int ldw, const float* bias, void* C, int ldc,
                      int M, int N, int K, int epi, hipStream_t stream, const FusedNorm& fused = FusedNorm{}) {
+  constexpr int NW = 8;
   const int steps_per_wave = (K / 32 + NW - 1) / NW;
-  int rpb = 16 * NT, blocks = N / 32;
-  if (!PAIR) {
-    const int n_cu = cu_count();
-    if (n_cu <= 0) return (int)hipErrorUnknown;
-    rpb = (N + n_cu - 1) / n_cu;                 // one block per CU when the rows are few
-    rpb = rpb < 1 ? 1 : (rpb > 16 * NT ? 16 * NT : rpb);
-    blocks = (N + rpb - 1) / rpb;
+  const int n_cu = cu_count();
+  if (n_cu <= 0) return (int)hipErrorUnknown;
+  int rpb = (N + n_cu - 1) / n_cu;                 // one block per CU when the rows are few
+  rpb = rpb < 1 ? 1 : (rpb > 16 ? 16 : rpb);
+  const int blocks = (N + rpb - 1) / rpb;
+  if (fused.out_g && blocks > fused.out_parts) return MF_NOT_BUILT;
+  auto run = [&](auto S) {
+    rolling16_kernel<NW, 1, decltype(S)::value, false, TILED><<<blocks, NW * 64, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K,
+                                                                                              steps_per_wave, epi, rpb, fused);
+  };
+#define MF_ROLLING(S_) case S_: run(std::integral_constant<int, S_>{}); break;
+  switch (rolling_steps(steps_per_wave)) {
+    MF_ROLLING(10) MF_ROLLING(11) MF_ROLLING(12) MF_ROLLING(13) MF_ROLLING(14) MF_ROLLING(15)
+    default: run(std::integral_constant<int, 16>{});
   }
-  if (fused.out_g && (PAIR || blocks > fused.out_parts)) return MF_NOT_BUILT;
-  rolling16_kernel<NW, NT, S, PAIR, TILED><<<blocks, NW * 64, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K,
-                                                                           steps_per_wave, epi, rpb, fused);
+#undef MF_ROLLING
   return mf_launch_status();
 }
 
@@ -1680,7 +1720,7 @@ int launch_skinny16(const bf16* A, int lda, const bf16* W, int ldw, const float*
 // and 0.175 us for each of a wave's loads, blocks of a CU added up (measured over 12 shapes of 896 to 18,944, 20 to 64 rows).
 // Hence the choice of `whole_plan`.  q|k|v and o of 32 rows, this / K split or 64 x 64 tiles: 1,152 x 896 3.8 / 8.5 us, 896 x 896
 // 4.3 / 10.2, 2,048 x 1,536 4.7 / 10.5, 2,560 x 2,048 5.9 / 10.7; 896 x 4,864 9.2 / 11.0.
-template <int MT, int NT, int S, bool TILED>
+template <int MT, int NT, int S, bool ONCE, bool TILED>
 __global__ __launch_bounds__(512) void whole_kernel(const bf16* __restrict__ A, int lda, const bf16* __restrict__ W, int ldw,
                                                     const float* __restrict__ bias, float* __restrict__ C, int ldc, int M, int N, int K,
                                                     int accumulate, int rpb, FusedNorm fused) {
@@ -1690,8 +1730,8 @@ __global__ __launch_bounds__(512) void whole_kernel(const bf16* __restrict__ A, 
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int m0 = blockIdx.y * ROWS, n0 = blockIdx.x * rpb;             // rpb: weight rows of a block, as in rolling16_kernel
   const int total = K / 32, share = (total + NW - 1) / NW;
-  const int first = min(wid * share, total);
-  const int T = min(share, total - first);                             // steps of this wave
+  const int T = min(share, total - wid * share);                       // steps of this wave (none: not above 0)
+  const int first = T > 0 ? wid * share : 0, last = max(T, 1) - 1;
   const int kq = first * 32 + (lane >> 4) * 8;
   const bf16 *arow[MT], *wrow[NT];
 #pragma unroll
@@ -1704,10 +1744,10 @@ __global__ __launch_bounds__(512) void whole_kernel(const bf16* __restrict__ A, 
   const bool e_col = e_c < rpb && e_n < N;
   const float e_g = fused.out_g && e_col ? fused.out_g[e_n] : 0.f, e_b = bias && e_col ? bias[e_n] : 0.f;
   float old[PASSES];
-  LanesSum<COLS, 2> sums[PASSES];                                      // of the lane's own row
+  LanesSum<COLS, 2, true> sums[PASSES];                                      // of the lane's own row
   auto part_row = [&](int p) {
-    const int r = p * PASS + wid * PER_WAVE + lane / COLS, m = m0 + r;
-    return fused.in_ssq && r < ROWS && m < M ? fused.in_ssq + (size_t)m * fused.in_parts : nullptr;
+    const int m = m0 + p * PASS + wid * PER_WAVE + lane / COLS;
+    return fused.in_ssq ? fused.in_ssq + (size_t)min(m, M - 1) * fused.in_parts : nullptr;      // (rows past M: not stored)
   };
 #pragma unroll
   for (int p = 0; p < PASSES; ++p) {
@@ -1722,7 +1762,7 @@ __global__ __launch_bounds__(512) void whole_kernel(const bf16* __restrict__ A, 
   bf16x8 a[S][MT], w[S][NT];
   auto load = [&](int s, int at) {
 #pragma unroll
-    for (int j = 0; j < NT; ++j) w[s][j] = *reinterpret_cast<const bf16x8*>(wrow[j] + (size_t)at * WSTEP);
+    for (int j = 0; j < NT; ++j) w[s][j] = *reinterpret_cast<const bf16x8*>(wrow[j] + (size_t)at * WSTEP);      // (the other tiles of rows read them too)
 #pragma unroll
     for (int i = 0; i < MT; ++i) a[s][i] = *reinterpret_cast<const bf16x8*>(arow[i] + at * 32);
   };
@@ -1732,30 +1772,37 @@ __global__ __launch_bounds__(512) void whole_kernel(const bf16* __restrict__ A, 
 #pragma unroll
       for (int j = 0; j < NT; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[s][i], w[s][j], acc[i][j], 0, 0, 0);
   };
+  // All of the slice at once (ONCE: it has at most S steps), or S steps of it and the rest behind their products; no load of a slice that is longer than S stands
+  // behind a condition (see `rolling16_kernel`).
+  if constexpr (ONCE) {
 #pragma unroll
-  for (int s = 0; s < S; ++s)
-    if (s < T) load(s, s);
+    for (int s = 0; s < S; ++s)
+      if (s < T) load(s, s);
+  } else {
+#pragma unroll
+    for (int s = 0; s < S; ++s) load(s, min(s, last));
+  }
 #pragma unroll
   for (int p = 0; p < PASSES; ++p) sums[p].ask(part_row(p), fused.in_parts, e_c);
   __builtin_amdgcn_sched_barrier(0);
-  int base = 0;
-  for (; base + 2 * S <= T; base += S) {                               // rounds whose refills all exist
+  if constexpr (ONCE) {
 #pragma unroll
-    for (int s = 0; s < S; ++s) {
-      multiply(s);
-      load(s, base + S + s);
-      __builtin_amdgcn_sched_barrier(0);
+    for (int s = 0; s < S; ++s)
+      if (s < T) multiply(s);
+  } else {
+    int base = 0;
+    for (; base + S < T; base += S) {
+#pragma unroll
+      for (int s = 0; s < S; ++s) {
+        multiply(s);
+        load(s, min(base + S + s, last));
+        __builtin_amdgcn_sched_barrier(0);
+      }
     }
-  }
-  const int rem = T - base - S;                                        // steps behind those in registers (none if not above 0)
 #pragma unroll
-  for (int s = 0; s < S; ++s) {
-    if (base + s < T) multiply(s);
-    if (s < rem) load(s, base + S + s);
+    for (int s = 0; s < S; ++s)
+      if (base + s < T) multiply(s);
   }
-#pragma unroll
-  for (int s = 0; s < S; ++s)
-    if (s < rem) multiply(s);
   // D[m][n]: n = lane % 16, m = 4 (lane / 16) + r
 #pragma unroll
   for (int i = 0; i < MT; ++i)
@@ -1827,9 +1874,18 @@ template <bool TILED>
 int launch_whole(const bf16* A, int lda, const bf16* W, int ldw, const float* bias, float* C, int ldc, int M, int N, int K, int epi,
                  const FusedNorm& fused, hipStream_t stream) {
   const WholePlan p = whole_plan(M, N, K, cu_count());
+  const int share = (K / 32 + 7) / 8;
   auto run = [&](auto MT, auto NT) {
-    whole_kernel<decltype(MT)::value, decltype(NT)::value, 8, TILED>
-        <<<dim3(p.gx, p.gy), 512, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi == EPI_ACC_F32, p.rpb, fused);
+    auto held = [&](auto S, auto ONCE) {
+      whole_kernel<decltype(MT)::value, decltype(NT)::value, decltype(S)::value, decltype(ONCE)::value, TILED>
+          <<<dim3(p.gx, p.gy), 512, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi == EPI_ACC_F32, p.rpb, fused);
+    };
+    // a slice of up to ten steps at once, or in two rounds (a longer one in more) with few steps past its end
+    if (share <= 4) held(std::integral_constant<int, 4>{}, std::true_type{});
+    else if (share <= 10) held(std::integral_constant<int, 10>{}, std::true_type{});
+    else if (share <= 12) held(std::integral_constant<int, 6>{}, std::false_type{});
+    else if (share <= 16) held(std::integral_constant<int, 8>{}, std::false_type{});
+    else held(std::integral_constant<int, 10>{}, std::false_type{});
   };
   using One = std::integral_constant<int, 1>;
   using Two = std::integral_constant<int, 2>;
@@ -1916,7 +1972,25 @@ __global__ __launch_bounds__(NW * 64) void stationary16_kernel(const void* __res
   auto first_loads = [&](int j) {
     wcur[j] = w_operand<TILED>(Wp, ldw, KK, lane_wrow(c_begin, j), k0);
 #pragma unroll
-    for (int s = 0; s < RING; ++s) w[j][s] = *reinterpret_cast<const bf16x8*>(wcur[j] + s * WSTEP);
+    for (int s = 0; s < RING; ++s) w[j][s] = load_weights(wcur[j] + s * WSTEP);
+  };
+  // The epilogue's place of this lane in an item: wave w adds up the sums of activation rows
+  // [w 64 / COLS, (w + 1) 64 / COLS), all waves at once.  What the epilogue needs from memory (the
+  // bias, and the output's old value where the product is added to it) is asked for an item ahead, in
+  // front of the refills and without a condition (a lane with no place, or no such
+  // operand, reads the head of the weights and drops it): behind the barrier it would make
+  // the wave wait for every load it has in flight, and the kernel's last item for memory; asked for in the item itself and held
+  // there, it made every item wait for the weights in flight before it (gate|up of 8 rows at the 7B widths).
+  const int e_c = lane % COLS, e_m = wid * (64 / COLS) + lane / COLS;
+  float next_old = 0.f, next_bias = 0.f, next_g = 0.f;
+  auto ask_epilogue = [&](int c0) {
+    if constexpr (!PAIR) {
+      const bool mine = c0 + e_c < c_end && e_m < M;
+      const float* none = reinterpret_cast<const float*>(W);
+      next_old = *((mine && epi == EPI_ACC_F32) ? (const float*)C + (size_t)e_m * ldc + c0 + e_c : none);
+      next_bias = *((mine && bias) ? bias + c0 + e_c : none);
+      next_g = *((mine && fused.out_g) ? fused.out_g + c0 + e_c : none);
+    }
   };
   bf16x8 afr[NS];
   float ss = 0.f;
@@ -1957,6 +2031,7 @@ __global__ __launch_bounds__(NW * 64) void stationary16_kernel(const void* __res
         x[s][1] = *reinterpret_cast<const float4*>(xrow + s * 32 + 4);
       }
       __builtin_amdgcn_sched_barrier(0);
+      ask_epilogue(c_begin);
       first_loads(0);
       __builtin_amdgcn_sched_barrier(0);
       *reinterpret_cast<float4*>(&gs[ge0]) = gt0;
@@ -1996,6 +2071,7 @@ __global__ __launch_bounds__(NW * 64) void stationary16_kernel(const void* __res
         __builtin_amdgcn_sched_barrier(0);
       }
       asm volatile("" : "+s"(Wp), "+v"(afr[NS - 1]));     // no weights before the activations are in place
+      ask_epilogue(c_begin);
       first_loads(0);
     }
     ss += __shfl_xor(ss, 16);
@@ -2013,52 +2089,42 @@ __global__ __launch_bounds__(NW * 64) void stationary16_kernel(const void* __res
   constexpr int FR = (16 + NW - 1) / NW;
   int frow[FR];
   float ffac[FR];
+  RowSums<FR> fsums;
 #pragma unroll
   for (int i = 0; i < FR; ++i) frow[i] = (!NORM && fused.in_ssq && wid + NW * i < 16) ? wid + NW * i : -1;
   if constexpr (!NORM) {
-    row_sums_ask<FR>(fused, frow, M, lane, ffac);
+    fsums.ask(fused, frow, M, lane);
+    ask_epilogue(c_begin);
     __builtin_amdgcn_sched_barrier(0);
     first_loads(0);
   }
 #pragma unroll
   for (int j = 1; j < NT; ++j) first_loads(j);
   if constexpr (!NORM) {
-    row_factors_of<FR>(fused, frow, M, KK, ffac);
+    fsums.factors(fused, frow, M, KK, lane, ffac);
     if (lane == 0)
 #pragma unroll
       for (int i = 0; i < FR; ++i)
         if (wid + NW * i < 16) rfac[wid + NW * i] = ffac[i];       // read behind the first item's barrier
   }
   float sq = 0.f;                      // a product that prepares the next norm: squares of this lane's outputs
-  for (int it = 0; it < n_items; ++it) {
-    // The loop body has no branch, so that the compiler can count the loads in flight and wait
-    // for the oldest one only: behind the last item the loads go to the head of the matrix,
-    // the same few lines for every lane, and their values are dropped.
+  // An item.  Its body has no branch, so that the compiler can count the loads in flight and wait for the oldest one only; the last
+  // item, which refills nothing, has a body of its own (loads that went to the head of the matrix there, to be dropped, were
+  // every block's to the same few lines: with `load_weights` 1 us of the 4.8 that q|k|v of 1,152 x 896 took).
+  auto item = [&](int it, auto NEXT) {
+    constexpr bool next = decltype(NEXT)::value;
     const int c0 = c_begin + it * CH;
-    const bool has_next = it + 1 < n_items;
+    if constexpr (next) {
 #pragma unroll
-    for (int j = 0; j < NT; ++j)
-      wrow[j] = w_operand<TILED>(Wp, ldw, KK, has_next ? lane_wrow(c0 + CH, j) : 0, k0);
+      for (int j = 0; j < NT; ++j) wrow[j] = w_operand<TILED>(Wp, ldw, KK, lane_wrow(c0 + CH, j), k0);
+    }
     floatx4 acc[NT];
 #pragma unroll
     for (int j = 0; j < NT; ++j) acc[j] = floatx4{0.f, 0.f, 0.f, 0.f};
-    // The epilogue's place of this lane in this item: wave w adds up the sums of activation rows
-    // [w 64 / COLS, (w + 1) 64 / COLS), all waves at once.  What the epilogue needs from memory (the
-    // bias, and the output's old value where the product is added to it) is asked for here, in
-    // front of the item's refills and without a condition (a lane with no place, or no such
-    // operand, reads the head of the weights and drops it): behind the barrier it would make
-    // the wave wait for every load it has in flight, and the kernel's last item for memory.
-    const int e_c = lane % COLS;
     const int e_n = c0 + e_c;
-    const int e_m = wid * (64 / COLS) + lane / COLS;
     const bool e_mine = !PAIR && e_n < c_end && e_m < M;
-    float c_old = 0.f, e_bias = 0.f, e_g = 0.f;
-    if constexpr (!PAIR) {
-      const float* dummy = reinterpret_cast<const float*>(W);
-      c_old = *((e_mine && epi == EPI_ACC_F32) ? (const float*)C + (size_t)e_m * ldc + e_n : dummy);
-      e_bias = *((e_mine && bias) ? bias + e_n : dummy);
-      e_g = *((e_mine && fused.out_g) ? fused.out_g + e_n : dummy);
-    }
+    const float c_old = next_old, e_bias = next_bias, e_g = next_g;
+    if constexpr (next) ask_epilogue(c0 + CH);
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
 #pragma unroll
@@ -2070,15 +2136,15 @@ __global__ __launch_bounds__(NW * 64) void stationary16_kernel(const void* __res
           asm volatile("" : "+v"(acc[j]) : : "memory");
           __builtin_amdgcn_sched_barrier(0);
         }
-        w[j][s % RING] = s + RING < NS ? *reinterpret_cast<const bf16x8*>(wcur[j] + (s + RING) * WSTEP)
-                                       : *reinterpret_cast<const bf16x8*>(wrow[j] + (s + RING - NS) * WSTEP);
+        if (s + RING < NS) w[j][s % RING] = load_weights(wcur[j] + (s + RING) * WSTEP);
+        else if (next) w[j][s % RING] = load_weights(wrow[j] + (s + RING - NS) * WSTEP);
         __builtin_amdgcn_sched_barrier(0);      // keep "use a register, then refill it" in this order
       }
-      // (held here, or the compiler moves the two loads to where they are used)
-      if (s == 0) asm volatile("" : "+v"(c_old), "+v"(e_bias), "+v"(e_g));
     }
+    if constexpr (next) {
 #pragma unroll
-    for (int j = 0; j < NT; ++j) wcur[j] = wrow[j];
+      for (int j = 0; j < NT; ++j) wcur[j] = wrow[j];
+    }
     // D[m][n]: n = lane % 16, m = 4 (lane / 16) + r
     const int buf = it & 1;
 #pragma unroll
@@ -2123,7 +2189,9 @@ __global__ __launch_bounds__(NW * 64) void stationary16_kernel(const void* __res
         }
       }
     }
-  }
+  };
+  for (int it = 0; it + 1 < n_items; ++it) item(it, std::true_type{});
+  item(n_items - 1, std::false_type{});
   if constexpr (!PAIR)
     if (fused.out_g) norm_part_out<COLS>(fused, sq, wid * (64 / COLS) + lane / COLS, lane % COLS, M);
 }
@@ -2245,16 +2313,17 @@ __global__ __launch_bounds__(512) void panel_kernel(const bf16* __restrict__ A, 
   float ffac[2 * MT];
 #pragma unroll
   for (int i = 0; i < 2 * MT; ++i) frow[i] = fused.in_ssq ? wid + 8 * i : -1;
-  row_sums_ask<2 * MT>(fused, frow, M, lane, ffac);
+  RowSums<2 * MT> fsums;
+  fsums.ask(fused, frow, M, lane);
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int s = 0; s < KC / 32; ++s) {
-    wr[0][s] = *reinterpret_cast<const bf16x8*>(wp[0] + s * WSTEP);
-    wr[1][s] = *reinterpret_cast<const bf16x8*>(wp[1] + s * WSTEP);
+    wr[0][s] = load_weights(wp[0] + s * WSTEP);
+    wr[1][s] = load_weights(wp[1] + s * WSTEP);
   }
   __builtin_amdgcn_sched_barrier(0);
   store_stage(0);
-  row_factors_of<2 * MT>(fused, frow, M, K, ffac);
+  fsums.factors(fused, frow, M, K, lane, ffac);
   if (lane == 0)
 #pragma unroll
     for (int i = 0; i < 2 * MT; ++i) rfac[wid + 8 * i] = ffac[i];
@@ -2287,7 +2356,7 @@ __global__ __launch_bounds__(512) void panel_kernel(const bf16* __restrict__ A, 
 #pragma unroll
         for (int i = 0; i < MT; ++i)
           acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], wr[j][s], acc[j][i], 0, 0, 0);
-        wr[j][s] = *reinterpret_cast<const bf16x8*>(wnext[j] + ((kn >> 5) + s) * WSTEP);
+        wr[j][s] = load_weights(wnext[j] + ((kn >> 5) + s) * WSTEP);
         __builtin_amdgcn_sched_barrier(0);      // use a register, then refill it, in this order
       }
     }
@@ -2392,8 +2461,7 @@ __global__ __launch_bounds__(512, 2) void panel_dma_kernel(const bf16* __restric
   constexpr int SUMS = (RA + 63) / 64;
   LanesSum<8, SUMS == 1 ? 4 : 1> sums[SUMS];
   auto part_row = [&](int q) {
-    const int r = q * 64 + wid * 8 + (lane >> 3);
-    return in_ssq && r < M ? in_ssq + (size_t)r * in_parts : nullptr;
+    return in_ssq ? in_ssq + (size_t)min(q * 64 + wid * 8 + (lane >> 3), M - 1) * in_parts : nullptr;      // (rows past M: not stored)
   };
 #pragma unroll
   for (int q = 0; q < SUMS; ++q) sums[q].ask(part_row(q), in_parts, lane & 7);
@@ -2412,13 +2480,15 @@ __global__ __launch_bounds__(512, 2) void panel_dma_kernel(const bf16* __restric
     dst[q] = lds0 + min(p, P - 1) * 1024;
   }
   const int nkt = K / DMA_BK;
-  auto copy = [&](int kt, int st) {                          // (past the last tile: that one again, never read)
-    const int k = min(kt, nkt - 1) * DMA_BK, kw = tiled ? k * 16 : k;
+  auto copy = [&](int kt, int st) {
+    const int k = kt * DMA_BK, kw = tiled ? k * 16 : k;
+    const bool on = kt < nkt;                                // (else the copies count, and move nothing)
 #pragma unroll
-    for (int q = 0; q < L; ++q)
-      asm volatile("s_mov_b32 m0, %2\n\ts_mov_b64 exec, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1\n\ts_mov_b64 exec, -1" ::"v"(g[q]),
-                   "s"((q * 8 + wid) * 8 < RA ? A + k : W + kw), "s"(__builtin_amdgcn_readfirstlane(dst[q] + st * ST)), "s"(lanes[q])
-                   : "m0");
+    for (int q = 0; q < L; ++q) {
+      const unsigned to = __builtin_amdgcn_readfirstlane(dst[q] + st * ST);
+      if ((q * 8 + wid) * 8 < RA) dma16_lanes<false>(A + k, g[q], to, on ? lanes[q] : 0);
+      else dma16_lanes<true>(W + kw, g[q], to, on ? lanes[q] : 0);
+    }
   };
   const int sw = (fr >> 1) & 7;
   bf16x8 fa[2][I], fw[2][J];
@@ -2605,8 +2675,9 @@ __global__ __launch_bounds__(256) void skinny_reduce_kernel(const float* __restr
   const size_t stride = (size_t)M * N;
   const int frow[1] = {fused.in_ssq ? m : -1};
   float ffac[1];
-  row_sums_ask<1>(fused, frow, M, threadIdx.x & 63, ffac);
-  row_factors_of<1>(fused, frow, M, K, ffac);
+  RowSums<1> fsums;
+  fsums.ask(fused, frow, M, threadIdx.x & 63);
+  fsums.factors(fused, frow, M, K, threadIdx.x & 63, ffac);
   const float rf = ffac[0];
   if (epi == EPI_SWIGLU) {       // n runs over the ldc outputs
     if (n >= ldc) return;
@@ -2660,7 +2731,8 @@ __global__ __launch_bounds__(256) void skinny_reduce4_kernel(const float* __rest
   const size_t stride = (size_t)M * N;
   const int frow[1] = {fused.in_ssq ? m : -1};
   float ffac[1];
-  row_sums_ask<1>(fused, frow, M, threadIdx.x & 63, ffac);
+  RowSums<1> fsums;
+  fsums.ask(fused, frow, M, threadIdx.x & 63);
   float4 v = float4{0.f, 0.f, 0.f, 0.f};
   const bool in = n < N;                                     // N in fours: all four inside, or none
   if (in) {
@@ -2674,7 +2746,7 @@ __global__ __launch_bounds__(256) void skinny_reduce4_kernel(const float* __rest
       for (int j = 0; j < 8; ++j) { v.x += x[j].x; v.y += x[j].y; v.z += x[j].z; v.w += x[j].w; }
     }
   }
-  row_factors_of<1>(fused, frow, M, K, ffac);
+  fsums.factors(fused, frow, M, K, threadIdx.x & 63, ffac);
   if (in) {
     const float rf = ffac[0];
     const float4 b = bias ? *reinterpret_cast<const float4*>(bias + n) : float4{0.f, 0.f, 0.f, 0.f};
@@ -3452,8 +3524,8 @@ static int skinny_product(const void* A, int lda, const void* W, const void* Wt,
                 : launch_whole<false>(a, lda, w, ldw, bias, (float*)C, ldc, M, N, K, epi, fused, stream);
     case SK_STATIONARY: return stationary16(a, lda, w, wt, ldw, bias, C, ldc, M, N, K, epi, nullptr, stream, fused);
     case SK_ROLLING:
-      return wt ? launch_rolling16<8, 1, 16, false, true>(a, lda, wt, ldw, bias, C, ldc, M, N, K, epi, stream, fused)
-                : launch_rolling16<8, 1, 16>(a, lda, w, ldw, bias, C, ldc, M, N, K, epi, stream, fused);
+      return wt ? launch_rolling16<true>(a, lda, wt, ldw, bias, C, ldc, M, N, K, epi, stream, fused)
+                : launch_rolling16<false>(a, lda, w, ldw, bias, C, ldc, M, N, K, epi, stream, fused);
     case SK_GUARDED_PAIR: return launch_skinny16<4, 2, 4, true>(a, lda, w, ldw, bias, C, ldc, M, N, K, epi, vec_ok, stream);
     case SK_GUARDED_4X2: return launch_skinny16<4, 2, 4>(a, lda, w, ldw, bias, C, ldc, M, N, K, epi, vec_ok, stream);
     case SK_GUARDED_8X2: return launch_skinny16<8, 2, 4>(a, lda, w, ldw, bias, C, ldc, M, N, K, epi, vec_ok, stream);
