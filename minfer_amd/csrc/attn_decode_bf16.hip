@@ -98,7 +98,7 @@ __global__ __launch_bounds__(256, ROPE && HD == 32 ? 5 : 1) void attn_decode_ker
   const int n_gc = (G + 15) / 16;
   // Which token, group of heads and split this block has, and how many splits the token's keys go
   // over (`active`, at most its n_splits places in `part`).
-  int t, hg, split, active, p;
+  int t, hg, split, active, p, seq;
   if (base_splits == 0) {
     // Every token has n_splits splits.  Blocks are numbered with the split running fastest, then
     // the group of heads, then the token: consecutive blocks go to consecutive dies, so a
@@ -109,6 +109,7 @@ __global__ __launch_bounds__(256, ROPE && HD == 32 ? 5 : 1) void attn_decode_ker
     t = blockIdx.x / (n_splits * nk * n_gc);
     active = n_splits;
     p = positions[t];
+    seq = seq_of_tok[t];                   // (asked for together)
   } else {
     // The step's tokens (at most 64) share n_tok * base_splits splits, as many blocks per group of
     // heads as without sharing (one per CU is what the plan aims at; a block more on some CUs
@@ -142,13 +143,14 @@ __global__ __launch_bounds__(256, ROPE && HD == 32 ? 5 : 1) void attn_decode_ker
     split = __builtin_amdgcn_readfirstlane(b - (__shfl(behind, t, MF_WAVE) - __shfl(s_i, t, MF_WAVE)));
     active = __builtin_amdgcn_readfirstlane(__shfl(s_i, t, MF_WAVE));
     p = __builtin_amdgcn_readfirstlane(__shfl(p_i, t, MF_WAVE));
+    seq = seq_of_tok[t];
   }
   const int hk = hg / n_gc;
   const int g0 = (hg % n_gc) * 16;
   const int gcount = min(16, G - g0);
   const int h0 = hk * G + g0;
 
-  const int* pt = page_table + (size_t)seq_of_tok[t] * pt_stride;
+  const int* pt = page_table + (size_t)seq * pt_stride;
   const int lo = window > 0 ? max(0, p - window + 1) : 0;
   if (split == 0 && active < n_splits) {
     // the places this token leaves unused say "nothing here" (maximum -inf, sum 0; the merge reads
@@ -236,9 +238,11 @@ __global__ __launch_bounds__(256, ROPE && HD == 32 ? 5 : 1) void attn_decode_ker
       if (q_chunk(u, head, d)) load8<HD>(rq[u], row + (size_t)(h0 + head) * HD, rope.cs, rope.sn, p, d);
     }
     if (own_split) {
-      if (tid * 8 < HD) load8<HD>(rk, row + (size_t)(nh + hk) * HD, rope.cs, rope.sn, p, tid * 8);
-      if (tid < HD) rv = row[(size_t)(nh + nk + hk) * HD + tid];
+      if (w == 0) load8<HD>(rk, row + (size_t)(nh + hk) * HD, rope.cs, rope.sn, p, min(tid * 8, HD - 8));
     }
+    // (without a condition: behind one the compiler waited for all of the rotation before it asked for keys; threads past the head's
+    // end ask for its last value again)
+    rv = row[(size_t)(nh + nk + hk) * HD + min(tid, HD - 1)];
   }
   int page_ahead = 0;                    // of the step after the one in flight
   if (w < n_steps) {
