@@ -8,6 +8,8 @@
 //    their k tiles copied straight into LDS, 16x16x32 MFMA, two groups of four waves a quarter product apart.
 //  * `tile_step_kernel`: the same copies for tiles of 128 x 128 and 64 x 64 (fewer rows, and 17 to 64 rows against a short
 //    K), one barrier a k tile.
+//  * `tile_stream_kernel`: more than 64 rows whose tiles are all on the chip at once, weights from the tiled copy straight into MFMA
+//    operands.
 //  * `tile_kernel`: many rows of any alignment, through registers and double-buffered LDS, 32x32x16 MFMA.
 //  * `reduce_norm_kernel`: adds the parts of a K split into the stream and norms the new rows.
 //  * `stationary16_kernel`: at most 16 rows and K of 896, 1536, 2048, 3584, 4096, 5120 or 8192 (decode):
@@ -1000,6 +1002,190 @@ int launch_tile64(const bf16* A, int lda, const bf16* W, int ldw, const float* b
                   hipStream_t stream, int splits, int k_per_split, bool tiled, const float* in_ssq = nullptr, int in_parts = 0, float in_eps = 0.f) {
   return launch_tile_step<64, 64, 2, 2, 5, false, SCALED>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi, stream, splits, k_per_split,
                                                           nullptr, 0, in_ssq, in_parts, in_eps, Halves{}, tiled);
+}
+
+// ---- tiles that are all on the chip at once: weights straight into MFMA operands
+// What bounds products of some hundred rows is neither the matrix cores nor LDS but what a CU brings in: about 60 GB/s of weights and
+// activations together, whatever form the copies have (k tiles of 64: 128 rows x 128 columns 0.48 us, 96 x 128 0.38, 208 x 128 0.70, 128 x
+// 256 0.78, with 30 blocks on the chip as with 256, four or six k tiles ahead).  So the rows of a tile are what the product has, in 16s, and not
+// 128 or 256; weights, whose tiled copy holds them as the MFMA operands they are, go to registers, four k tiles ahead, each wave its own 32
+// columns; the activations of a k tile go through registers into one of two LDS buffers, and their fragments are read three
+// ahead of the products.  A short way in and out (no LDS at all in the epilogue) makes few parts of a K split pay: the cut kernels
+// alone, in microseconds, `tile_dma_kernel` / this one: 203 x 3,584 x 3,584 16.5 in 7 parts / 13.6 in 3, 203 x 4,608 x 3,584 19.6 in 7 / 16.1
+// in 2, 604 x 2,560 x 2,048 17.3 in 4 / 13.8 in 2, 604 x 2,048 x 2,048 16.4 in 4 / 11.3 in 2, 300 x 896 x 4,864 11.8 in 7 / 9.4 in 9
+// (weights from memory).  SwiGLU products were level at best (300 x 9,728 x 896 12.2 and 12.9) and have none.
+// Tried: 256 columns, weights marked as read once where other rows' tiles read them (slower: 13.7 and 15.3), fragments seven ahead with four
+// LDS buffers (level).
+template <int I>
+__global__ __launch_bounds__(256, 2) void tile_stream_kernel(const bf16* __restrict__ A, int lda, const bf16* __restrict__ Wt,
+                                                                          const float* __restrict__ bias, void* __restrict__ C, int ldc, int M,
+                                                                          int N, int K, int epi, int tiles_m, int tiles, int k_per_split) {
+  constexpr int J = 2, AHEAD = 4, BM = 16 * I, BN = 64 * J, ROW = DMA_BK * 2, BUF = BM * ROW, LA = (I + 1) / 2, STEPS = 2 * I, D = 3, R = 4;
+  static_assert(AHEAD * STEPS % R == 0 && LA < STEPS - D && I + J <= STEPS, "fragments keep their places, a k tile is written before the barrier");
+  __shared__ __attribute__((aligned(16))) unsigned char smem[2 * BUF];      // [buffer][BM rows of A][64]
+  int at = blockIdx.x;
+  {
+    const int n = gridDim.x, per = n / 8, rem = n % 8, x = at % 8;          // (neighbours on one die: a part's tiles of the same weights)
+    at = x * per + min(x, rem) + at / 8;
+  }
+  const int part = at / tiles, tile = at - part * tiles;
+  const int bm = tile % tiles_m, bn = tile / tiles_m;
+  const int k_tiles = K >> 5;                                // tiles of 32 k of a block of weight rows
+  if (k_per_split > 0) {                                     // as in tile_dma_kernel
+    const int kb = part * k_per_split;
+    A += kb;
+    Wt += (size_t)(kb >> 5) * 512;
+    K = min(k_per_split, K - kb);
+    C = (float*)C + (size_t)part * M * N;
+  }
+  const int nkt = K / DMA_BK;
+  const int m0 = bm * BM, n0 = bn * BN;
+  const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int fr = lane & 15, fk = lane >> 4;
+  floatx4 acc[I][J];
+#pragma unroll
+  for (int i = 0; i < I; ++i)
+#pragma unroll
+    for (int j = 0; j < J; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+  unsigned wo[J], ao[LA], aw[LA];                            // bytes: weights, activations, and where the latter go in LDS
+#pragma unroll
+  for (int j = 0; j < J; ++j)
+    wo[j] = (unsigned)min((n0 >> 4) + wid * J + j, (N - 1) >> 4) * (unsigned)k_tiles * 1024u + fr * 64 + fk * 16;
+#pragma unroll
+  for (int q = 0; q < LA; ++q) {
+    const int r = min(q * 32 + (tid >> 3), BM - 1), c = tid & 7;
+    ao[q] = ((unsigned)min(m0 + r, M - 1) * (unsigned)lda + c * 8) * 2u;
+    aw[q] = r * ROW + (c ^ ((r >> 1) & 7)) * 16;
+  }
+  const bool last = I % 2 == 0 || tid < 128;                 // whether the last of a thread's chunks is a row's of the tile
+  bf16x8 w[AHEAD][2][J], a[2][LA], f[R];
+  // (the offsets stay 32 bits wide beside a scalar base only where the compiler cannot take them out of the loop as addresses)
+  auto load = [](const void* base, size_t at, unsigned off) {
+    asm volatile("" : "+v"(off));
+    return *reinterpret_cast<const bf16x8*>((const char*)base + at + off);
+  };
+  auto load_w = [&](int kt, int u, int h, int j) { w[u][h][j] = load(Wt, (size_t)(unsigned)(min(kt, nkt - 1) * 2 + h) * 1024, wo[j]); };
+  auto load_a = [&](int kt, int s, int q) { a[s][q] = load(A, (size_t)(unsigned)min(kt, nkt - 1) * ROW, ao[q]); };
+  auto write_a = [&](int s, int q) {
+    if (q + 1 < LA || last) *reinterpret_cast<bf16x8*>(smem + s * BUF + aw[q]) = a[s][q];
+  };
+  unsigned po[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) po[h] = fr * ROW + ((4 * h + fk) ^ ((fr >> 1) & 7)) * 16;
+  // step s of a k tile: row block s % I, half s / I of its k
+  auto read = [&](int s, int st, int to) { f[to] = *reinterpret_cast<const bf16x8*>(smem + st * BUF + po[s / I] + (s % I) * 16 * ROW); };
+  auto load_tile = [&](int u) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int j = 0; j < J; ++j) load_w(u, u, h, j);
+  };
+#pragma unroll
+  for (int q = 0; q < LA; ++q) load_a(0, 0, q);
+  load_tile(0);
+#pragma unroll
+  for (int q = 0; q < LA; ++q) load_a(1, 1, q);
+#pragma unroll
+  for (int u = 1; u < AHEAD; ++u) load_tile(u);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int q = 0; q < LA; ++q) write_a(0, q);
+#pragma unroll
+  for (int q = 0; q < LA; ++q) load_a(2, 0, q);
+  auto meet = [&]() {                                        // this wave's reads and writes of LDS are done, then everyone's
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    dma_meet();
+  };
+  meet();
+#pragma unroll
+  for (int s = 0; s < D; ++s) read(s, 0, s);
+  // k tile kt in buffer u % 2, its weights in set u.  The next one's activations are written to the other buffer, which every wave
+  // has read to its end by the barrier before; behind this tile's barrier, D steps before its end, the next one's are read.
+  auto pass = [&](int kt, auto U) {
+    constexpr int u = decltype(U)::value, st = u & 1, off = u * STEPS;
+#pragma unroll
+    for (int s = 0; s < STEPS; ++s) {
+      if (s == STEPS - D) meet();
+      read((s + D) % STEPS, s + D < STEPS ? st : st ^ 1, (off + s + D) % R);
+      if (s >= 1 && s <= LA) write_a(st ^ 1, s - 1);
+      if (s >= 2 && s <= LA + 1) load_a(kt + 3, st ^ 1, s - 2);
+      if (s >= I && s < I + J) load_w(kt + AHEAD, u, 0, s - I);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int j = 0; j < J; ++j)
+        acc[s % I][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[u][s / I][j], f[(off + s) % R], acc[s % I][j], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int j = 0; j < J; ++j) load_w(kt + AHEAD, u, 1, j);
+  };
+  using U0 = std::integral_constant<int, 0>;
+  using U1 = std::integral_constant<int, 1>;
+  using U2 = std::integral_constant<int, 2>;
+  using U3 = std::integral_constant<int, 3>;
+  int kt = 0;
+  for (; kt + AHEAD <= nkt; kt += AHEAD) {
+    pass(kt, U0{});
+    pass(kt + 1, U1{});
+    pass(kt + 2, U2{});
+    pass(kt + 3, U3{});
+  }
+  if (kt < nkt) {
+    pass(kt, U0{});
+    if (kt + 1 < nkt) {
+      pass(kt + 1, U1{});
+      if (kt + 2 < nkt) pass(kt + 2, U2{});
+    }
+  }
+  // D: the lane's row is lane % 16, its columns 4 (lane / 16) + e of a block
+  const bool half = epi == EPI_BF16 || epi == EPI_XIELU || epi == EPI_RELU2;
+  const bool vec = ldc % 4 == 0 && (uintptr_t)C % (half ? 8 : 16) == 0;
+  const float ap = epi == EPI_XIELU ? bias[N] : 0.f, an = epi == EPI_XIELU ? bias[N + 1] : 0.f;
+#pragma unroll
+  for (int j = 0; j < J; ++j) {
+    const int n = n0 + (wid * J + j) * 16 + fk * 4;
+    float b[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) b[e] = bias && n + e < N ? bias[n + e] : 0.f;
+#pragma unroll
+    for (int i = 0; i < I; ++i) {
+      const int m = m0 + i * 16 + fr;
+      if (m >= M || n >= N) continue;
+      const float v[4] = {acc[i][j][0] + b[0], acc[i][j][1] + b[1], acc[i][j][2] + b[2], acc[i][j][3] + b[3]};
+      if (!vec || n + 4 > N) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (n + e < N) store_out(C, ldc, m, n + e, v[e], epi, bias, N);
+      } else if (half) {
+        bf16x4 o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = (bf16)(epi == EPI_XIELU ? xielu_f(v[e], ap, an) : epi == EPI_RELU2 ? relu2_f(v[e]) : v[e]);
+        *reinterpret_cast<bf16x4*>((bf16*)C + (size_t)m * ldc + n) = o;
+      } else {
+        float4* o = reinterpret_cast<float4*>((float*)C + (size_t)m * ldc + n);
+        const float4 old = epi == EPI_ACC_F32 ? *o : float4{0.f, 0.f, 0.f, 0.f};
+        *o = float4{old.x + v[0], old.y + v[1], old.z + v[2], old.w + v[3]};
+      }
+    }
+  }
+}
+
+// (variant: VARIANT_STREAM + I)
+constexpr int VARIANT_STREAM = 20;
+int launch_tile_stream(int variant, const bf16* A, int lda, const bf16* Wt, const float* bias, void* C, int ldc, int M, int N, int K, int epi,
+                       hipStream_t stream, int splits = 1, int k_per_split = 0) {
+  if (!Wt || epi == EPI_SWIGLU) return (int)hipErrorInvalidValue;
+  const int bm = (variant - VARIANT_STREAM) * 16, tiles_m = (M + bm - 1) / bm, tiles = tiles_m * ((N + 127) / 128);
+#define MF_STREAM(I_) \
+  case VARIANT_STREAM + I_: \
+    tile_stream_kernel<I_><<<tiles * splits, 256, 0, stream>>>(A, lda, Wt, bias, C, ldc, M, N, K, epi, tiles_m, tiles, k_per_split); \
+    return mf_launch_status();
+  switch (variant) {
+    MF_STREAM(6)
+    MF_STREAM(8)
+  }
+#undef MF_STREAM
+  return (int)hipErrorInvalidValue;
 }
 
 template <int BM, int BN, int STAGES, bool GROUPED, bool HALVES = false>
@@ -3121,7 +3307,12 @@ double whole_more(int M, int N, int K, int behind) {
   return K > 3072 || mn > 2.2e6 || behind == 0 ? 0. : behind == 1 ? 4.5 : 3.2 + mn / 1e6;
 }
 
-TilePlan plan_tiles(int M, int N, int K, bool dma_ok, int epi, int n_cu, int behind = 0) {
+// `tile_stream_kernel`'s tiles: 16 I rows, microseconds a k tile with every CU busy (an eighth less with few), and what a part of a split
+// (on its own; in front of the rotation) and a whole product cost beside what every plan pays.
+struct StreamForm { int i; double step_us, split_us, rotated_us, whole_us; };
+constexpr StreamForm STREAM_FORMS[2] = {{6, 0.44, 4.2, 5.0, 2.0}, {8, 0.51, 4.0, 5.0, 4.0}};
+
+TilePlan plan_tiles(int M, int N, int K, bool dma_ok, int epi, int n_cu, int behind = 0, bool tiled = false) {
   const long cu = n_cu > 0 ? n_cu : 1;
   const long nkt = (K + 63) / 64, chunks = (K + 255) / 256;
   const double mn = (double)M * (double)N;
@@ -3183,6 +3374,29 @@ TilePlan plan_tiles(int M, int N, int K, bool dma_ok, int epi, int n_cu, int beh
       if (splits < 2 || splits * t128 > 2 * cu) continue;
       const double us = dma_ok ? form(2, splits, per / 64) : rounds_us(t128 * splits, 2 * cu, 1.45 * slow, per / 64, 0.);
       offer(2, splits, per, us + parts_us(splits));
+    }
+  // `tile_stream_kernel`, while all its tiles are on the chip at once, in at most eight parts of at least 256 of K.  Whole prompts of 66 to
+  // 2,048 tokens, four models 896 to 3,584 wide, without / with this choice: 2,048 wide 150 tokens 3,723 / 3,562 us, 300 4,731 / 4,640, 604
+  // 6,648 / 6,474, 900 8,118 / 7,946; 1,536 wide 450 tokens 3,223 / 3,154; 3,584 wide 150 tokens 5,186 / 5,089; level elsewhere.  Not in reach of the
+  // lines, a product with the kernel behind it without / with: up to 128 rows (level: the weights' stream), a K below 2,048 except in
+  // front of the rotation (1,536 x 1,536, 800 rows 18.2 / 20.5 us), few weight rows except around 900 rows (896 x 4,864, 180 rows
+  // 13.0 / 15.2, 2,048 rows 33.9 / 35.3; 900 rows of a prompt 2,393 / 2,334).  In front of the rotation a split of this kernel takes the place of another
+  // split only: where the product was whole, the parts cost the rotation more than they save (prompts of 450 tokens, 1,536 wide, 3,225 / 3,348).
+  // Whole up to 1,024 rows: a prompt of 1,400 tokens 2,048 wide 11,156 / 11,279, of 2,048 13,548 / 13,792.
+  const bool enough = behind == 1 || (K >= 2048 && (N >= 1024 || (M >= 700 && M <= 1100)));
+  const bool cut_anyway = best.splits > 1;
+  const double stream_more = behind == 1 ? (K > 3072 ? 9.5 : 4.5) : behind == 2 ? 3.2 + mn / 1e6 : 0.;      // (`whole_more`)
+  if (dma_ok && tiled && epi != EPI_SWIGLU && M > 128 && enough)
+    for (const StreamForm& f : STREAM_FORMS) {
+      const long t = tiles(16 * f.i, 128);
+      for (long parts = 1; parts <= 8 && t * parts <= cu && (parts == 1 || nkt >= 4 * parts); ++parts) {
+        const long steps = (nkt + parts - 1) / parts, splits = (nkt + steps - 1) / steps;
+        if (splits != parts || (splits > 1 ? behind == 1 && !cut_anyway : M > 1024)) continue;
+        const double us = f.step_us * (0.86 + 0.14 * (double)(t * splits) / (double)cu) * (double)steps;
+        offer(VARIANT_STREAM + f.i, (int)splits, splits > 1 ? (int)steps * 64 : K,
+              splits > 1 ? us + (behind == 1 ? f.rotated_us : f.split_us) + parts_us((int)splits)
+                         : us + f.whole_us + start_us - more_us + epi_us + stream_more);
+      }
     }
   return best;
 }
@@ -3403,6 +3617,8 @@ MF_API int mf_gemm_bf16(const void* A, int lda, const void* W, const void* Wt, i
     return launch_form(best_form(FORM_128, FORM_TINY, M, N - n0, K, nkt, 1, cu), a, lda, wt.from(n0), bias ? bias + n0 : nullptr,
                        rest, ldc, M, N - n0, K, epi, stream);
   }
+  if (variant > VARIANT_STREAM)
+    return dma_ok ? launch_tile_stream(variant, a, lda, wt.tiled, bias, C, ldc, M, N, K, epi, stream) : (int)hipErrorInvalidValue;
   if (epi == EPI_SWIGLU && variant == 3) variant = 2;      // needs two 32-column tiles per wave
   switch (variant) {
     case 1: return launch_tile<256, 256, 128, 128>(a, lda, w, ldw, bias, C, ldc, M, N, K, epi, vec_ok, stream);
@@ -3431,9 +3647,13 @@ MF_API int mf_gemm_bf16_parts(const void* A, int lda, const void* W, const void*
                      ((uintptr_t)W % 16 == 0) && (K % 8 == 0);
   // variant 12: 256 x 256 tiles through the direct-to-LDS pipeline (many rows against few weight
   // rows and a long K: the down product of a prompt); 2: the smaller tiles (few rows)
-  if (variant != 12 && variant != 2) return (int)hipErrorInvalidValue;
+  // (and VARIANT_STREAM + I: `tile_stream_kernel`)
+  if (variant != 12 && variant != 2 && variant <= VARIANT_STREAM) return (int)hipErrorInvalidValue;
   const bool dma_ok = vec_ok && K % DMA_BK == 0 && (size_t)M * lda * 2 < (1ull << 32) && (size_t)N * ldw * 2 < (1ull << 32);
-  if (variant == 12 && !dma_ok) return (int)hipErrorInvalidValue;
+  if (variant != 2 && !dma_ok) return (int)hipErrorInvalidValue;
+  if (variant > VARIANT_STREAM)
+    return launch_tile_stream(variant, (const bf16*)A, lda, Weights(W, Wt, ldw, K).tiled, nullptr, part, N, M, N, K, EPI_F32, stream, splits,
+                              k_per_split);
   return dma_ok ? launch_form(dma_form(variant, M, N, K, EPI_F32, k_per_split / DMA_BK, splits, cu_count()), (const bf16*)A, lda,
                               Weights(W, Wt, ldw, K), nullptr, part, N, M, N, K, EPI_F32, stream, splits, k_per_split)
                 : launch_tile<128, 128, 64, 64>((const bf16*)A, lda, (const bf16*)W, ldw, nullptr, part, N, M,
@@ -3615,12 +3835,12 @@ MF_API int mf_gemm_bf16_normed(const float* x, int ldx, const int* row_idx, cons
 
 // How a product of more than 64 rows is run: out[0] the variant for mf_gemm_bf16, or with out[1] > 1
 // for mf_gemm_bf16_splitk with out[1] splits of out[2] of K each.  `aligned`: 16-byte aligned
-// operands with row strides and K in multiples of 8.  `behind`: 1 where the kernel behind the product adds its parts on the way (the
-// rotation), 2 where that kernel is the norm of the rows as well, else 0.
-MF_API int mf_gemm_bf16_tile_plan(int M, int N, int K, int aligned, int epi, int n_cu, int behind, int* out) {
+// operands with row strides and K in multiples of 8; `tiled`: the product is given the tiled copy, 16-byte aligned.  `behind`: 1 where the
+// kernel behind the product adds its parts on the way (the rotation), 2 where that kernel is the norm of the rows as well, else 0.
+MF_API int mf_gemm_bf16_tile_plan(int M, int N, int K, int aligned, int tiled, int epi, int n_cu, int behind, int* out) {
   if (!out || behind < 0 || behind > 2 || M <= 0 || N <= 0 || K <= 0 || epi < 0 || epi > EPI_LAST || n_cu <= 0) return (int)hipErrorInvalidValue;
   const bool dma_ok = aligned && K % DMA_BK == 0 && (size_t)M * K * 2 < (1ull << 32) && (size_t)N * K * 2 < (1ull << 32);
-  const TilePlan plan = plan_tiles(M, N, K, dma_ok, epi, n_cu, behind);
+  const TilePlan plan = plan_tiles(M, N, K, dma_ok, epi, n_cu, behind, tiled != 0);
   out[0] = plan.variant;
   out[1] = plan.splits;
   out[2] = plan.k_per_split;
@@ -3660,7 +3880,7 @@ MF_API int mf_gemm_bf16_plan(int M, int N, int K, int aligned, int tiled, int ep
     }
   } else {
     const bool dma_ok = aligned && K % DMA_BK == 0 && (size_t)M * K * 2 < (1ull << 32) && (size_t)N * K * 2 < (1ull << 32);
-    const TilePlan plan = variant ? TilePlan{variant, 1, K, 0.} : plan_tiles(M, N, K, dma_ok, epi, n_cu, behind);
+    const TilePlan plan = variant ? TilePlan{variant, 1, K, 0.} : plan_tiles(M, N, K, dma_ok, epi, n_cu, behind, tiled != 0);
     const bool split = plan.splits > 1;
     if (variant >= 12 && !dma_ok) return (int)hipErrorInvalidValue;
     switch (plan.variant) {
@@ -3676,6 +3896,8 @@ MF_API int mf_gemm_bf16_plan(int M, int N, int K, int aligned, int tiled, int ep
                : split         ? "tile_kernel<128,128>(split K)" : "tile_kernel<128,128>";
         break;
       case 3: what = "tile_kernel<64,64>"; break;
+      case VARIANT_STREAM + 6: what = split ? "tile_stream_kernel<96>(split K)" : "tile_stream_kernel<96>"; break;
+      case VARIANT_STREAM + 8: what = split ? "tile_stream_kernel<128>(split K)" : "tile_stream_kernel<128>"; break;
       default: return (int)hipErrorInvalidValue;
     }
   }

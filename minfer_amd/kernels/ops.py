@@ -154,7 +154,7 @@ _PROTOTYPES = {
         "mf_gemm_bf16_skinny_fused": [_P, c_int, _P, _P, c_int, _P, _P, c_int, _P, c_int, c_int, c_int, c_int,
                                       c_int, c_int, _P, c_int, c_float, _P, _P, _P, c_int, _P],
         "mf_gemm_bf16_plan": [c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_char_p, c_int],
-        "mf_gemm_bf16_tile_plan": [c_int, c_int, c_int, c_int, c_int, c_int, c_int, _P],
+        "mf_gemm_bf16_tile_plan": [c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, _P],
         "mf_gemm_bf16_whole_parts": [c_int, c_int, c_int, c_int],
     },
     "attn_tokens_f32": {
@@ -1786,18 +1786,19 @@ def _skinny_plan(m: int, n: int, k: int, target_blocks: int, swiglu: bool, tiled
     return (chunks + per - 1) // per, per * 256
 
 
-def tile_plan(m: int, n: int, k: int, epi: int, aligned: bool = True, n_cu: Optional[int] = None) -> Tuple[int, int, int]:
+def tile_plan(m: int, n: int, k: int, epi: int, aligned: bool = True, n_cu: Optional[int] = None,
+              tiled: bool = False) -> Tuple[int, int, int]:
     """(variant, splits, k_per_split) of a bfloat16 product of more than 64 rows, as the library
-    chooses among its tile kernels (an estimate of the rounds their tiles take over the CUs); with
-    splits > 1, K is cut over blocks and a second kernel adds the parts."""
-    return _tile_plan(m, n, k, epi, bool(aligned), n_cu or cu_count(), 0)
+    chooses among its tile kernels (an estimate of the rounds their tiles take over the CUs; one of them reads the
+    tiled copy of the weights alone); with splits > 1, K is cut over blocks and a second kernel adds the parts."""
+    return _tile_plan(m, n, k, epi, bool(aligned), n_cu or cu_count(), 0, bool(tiled))
 
 
 @functools.lru_cache(maxsize=4096)           # (a plan depends on these numbers alone; a prompt asks for each of a few once a layer)
-def _tile_plan(m: int, n: int, k: int, epi: int, aligned: bool, n_cu: int, behind: int) -> Tuple[int, int, int]:
+def _tile_plan(m: int, n: int, k: int, epi: int, aligned: bool, n_cu: int, behind: int, tiled: bool = False) -> Tuple[int, int, int]:
     # (behind: 1 where the kernel behind the product adds its parts on the way, 2 where it norms the rows too, else 0)
     out = (c_int * 3)()
-    rc = _fn("gemm_bf16", "mf_gemm_bf16_tile_plan")(m, n, k, 1 if aligned else 0, epi, n_cu, behind, out)
+    rc = _fn("gemm_bf16", "mf_gemm_bf16_tile_plan")(m, n, k, 1 if aligned else 0, 1 if tiled else 0, epi, n_cu, behind, out)
     if rc != 0:
         raise KernelError(f"tile_plan: error {rc} for m {m}, n {n}, k {k}")
     return out[0], out[1], out[2]
@@ -1839,7 +1840,7 @@ def plan_linear(m: int, n: int, k: int, swiglu: bool = False, normed: bool = Fal
     elif m <= 64:
         splits, per = _k_split(m, n, k, swiglu, aligned, n_cu, tiled)
     else:
-        _, splits, per = _tile_plan(m, n, k, epi, bool(aligned), n_cu, behind)
+        _, splits, per = _tile_plan(m, n, k, epi, bool(aligned), n_cu, behind, bool(tiled))
     name = ctypes.create_string_buffer(64)
     rc = _fn("gemm_bf16", "mf_gemm_bf16_plan")(m, n, k, 1 if aligned else 0, 1 if tiled else 0, epi, splits, per,
                                                1 if normed else 0, (1 if scale_in else 0) | (2 if norm_out else 0), behind, variant, n_cu,
@@ -1862,6 +1863,11 @@ def tile_weight(weight: torch.Tensor) -> torch.Tensor:
     if n16 != n:
         weight = torch.cat([weight, torch.zeros((n16 - n, k), dtype=weight.dtype, device=weight.device)])
     return weight.view(n16 // 16, 16, k // 32, 32).permute(0, 2, 1, 3).contiguous()
+
+
+def _reads_tiled(tiled: Optional[torch.Tensor]) -> bool:
+    """Whether the kernels take the tiled copy where there is one: not off 16 bytes."""
+    return tiled is not None and tiled.data_ptr() % 16 == 0
 
 
 def _need_tiled(tiled: Optional[torch.Tensor], name: str, n: int, k: int) -> None:
@@ -1915,7 +1921,7 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], 
                                                         epi, _stream()), f"gemm_bf16_skinny {m}x{n}x{k}")
         return
     if variant == 0:
-        variant, splits, per = tile_plan(m, n, k, epi, aligned)
+        variant, splits, per = tile_plan(m, n, k, epi, aligned, tiled=_reads_tiled(tiled))
         if splits > 1:
             part = workspace("skinny", splits * m * n, x.device)
             _check(_fn("gemm_bf16", "mf_gemm_bf16_splitk")(x, k, weight, tiled, k, bias, out, n,
@@ -1946,7 +1952,8 @@ def linear_parts(x: torch.Tensor, weight: torch.Tensor, tiled: Optional[torch.Te
         return part
     if m <= 64:
         return None
-    variant, splits, per = _tile_plan(m, n, k, EPI_F32, not (x.data_ptr() % 16 or weight.data_ptr() % 16 or k % 8), cu_count(), 1)
+    variant, splits, per = _tile_plan(m, n, k, EPI_F32, not (x.data_ptr() % 16 or weight.data_ptr() % 16 or k % 8), cu_count(), 1,
+                                      _reads_tiled(tiled))
     if splits <= 1:
         return None
     _need_tiled(tiled, "linear_parts.tiled", n, k)
@@ -1968,7 +1975,7 @@ def linear_norm_out(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.
     if m <= 64 or x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 or weight.shape[1] != k:
         return None
     variant, splits, per = _tile_plan(m, n, k, EPI_ACC_F32 if accumulate else EPI_F32,
-                                      not (x.data_ptr() % 16 or weight.data_ptr() % 16 or k % 8), cu_count(), 2)
+                                      not (x.data_ptr() % 16 or weight.data_ptr() % 16 or k % 8), cu_count(), 2, _reads_tiled(tiled))
     if splits <= 1:
         return None
     _need(x, "linear_norm_out.x")
