@@ -349,7 +349,9 @@ __global__ __launch_bounds__(256) void moe_sparse_down_kernel(const WT* __restri
 // rows.  A workgroup of NW waves owns (expert, 16 output rows) and leaves at once where nobody chose the expert; its
 // waves share K, 64 values a step: A = 16 rows of a matrix (16x16x32 MFMA, a lane two neighbouring runs of 8 values, so
 // that a step reads 128 bytes of every row side by side), B = the rows of the expert's pairs, a column each, with the
-// same order of k.  The waves' sums meet in LDS and are added in the waves' order.
+// same order of k.  The waves' sums meet in LDS and are added in the waves' order.  The matrices are read by one workgroup each and
+// marked as read once, which gives the stream back some 5 % (a plain read 5.9 and 6.2 TB/s): a reply of 8 sequences, 32 steps with three
+// layers of experts 4,096 x 2,048, 18,006 us without and 17,656 with the mark.
 //   UP:  two matrices (gate and up) share B; y[pair][f] gets the activation.
 //   else: rows[pair][n] gets the product.
 template <int NW, bool UP>
@@ -390,7 +392,7 @@ __global__ __launch_bounds__(NW * 64) void moe_sparse_mfma_kernel(const bf16* __
 #pragma unroll
     for (int q = 0; q < 2; ++q) {
 #pragma unroll
-      for (int m = 0; m < MATS; ++m) a[m][q] = *(const bf16x8*)(wr[m] + s * 64 + 8 * q);
+      for (int m = 0; m < MATS; ++m) a[m][q] = __builtin_nontemporal_load((const bf16x8*)(wr[m] + s * 64 + 8 * q));
       b[q] = *(const bf16x8*)(xr + s * 64 + 8 * q);
     }
 #pragma unroll
