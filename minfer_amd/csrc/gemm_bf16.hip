@@ -1607,6 +1607,7 @@ constexpr int stationary_ring(int NS, int NT) {
 }
 
 constexpr int STATIONARY_K7 = 896;       // the one K that runs as 7 waves of 4 steps
+constexpr int STATIONARY_PLAIN_K = 5120; // the longest K without a norm or SwiGLU
 
 bool stationary_takes(int M, int N, int K, int epi, bool normed) {
   if (epi == EPI_SWIGLU && N % 64 != 0) return false;
@@ -1615,9 +1616,9 @@ bool stationary_takes(int M, int N, int K, int epi, bool normed) {
   if (K == STATIONARY_K7) return M <= 16 && (N + 15) / 16 >= 64;
   if (M > 16 || (N + 15) / 16 < 128) return false;
   if (K % 256 != 0) return false;
-  // a K above 5120 without a norm or SwiGLU to fold in (the o product of the widest models): the
+  // a K above STATIONARY_PLAIN_K without a norm or SwiGLU to fold in (the o product of the widest models): the
   // rolling kernel is the faster one there
-  if (K > 5120 && !normed && epi != EPI_SWIGLU) return false;
+  if (K > STATIONARY_PLAIN_K && !normed && epi != EPI_SWIGLU) return false;
   switch (K / 256) {
 #define MF_X(NS_) case NS_:
     MF_STATIONARY_NS(MF_X)
@@ -2167,15 +2168,26 @@ __global__ __launch_bounds__(NW * 64) void stationary16_kernel(const void* __res
   // operand, reads the head of the weights and drops it): behind the barrier it would make
   // the wave wait for every load it has in flight, and the kernel's last item for memory; asked for in the item itself and held
   // there, it made every item wait for the weights in flight before it (gate|up of 8 rows at the 7B widths).
-  const int e_c = lane % COLS, e_m = wid * (64 / COLS) + lane / COLS;
+  // The place is made anew each time: left alone, the compiler carries an address from item to item for every operand and for
+  // every kind of output, and with a K from 5,120 on spilled them; a reload is counted with the weights' loads and comes back behind
+  // them, so every item waited for the weights in flight (8 rows with the norm folded in, tiled copy, microseconds with spills / so:
+  // 152,064 x 6,144 320 / 292, 128,000 x 7,168 306 / 284, 9,216 x 7,168 34.4 / 32.9; level where nothing was spilled).
+  const int e_c = lane % COLS;
+  auto place = [&](int c0, int& m, int& n) {
+    m = PAIR ? wid * 4 + (lane >> 4) : wid * (64 / COLS) + lane / COLS;
+    n = c0 + (PAIR ? r16 : e_c);
+    asm volatile("" : "+v"(m), "+v"(n));
+  };
   float next_old = 0.f, next_bias = 0.f, next_g = 0.f;
   auto ask_epilogue = [&](int c0) {
     if constexpr (!PAIR) {
-      const bool mine = c0 + e_c < c_end && e_m < M;
+      int e_m, e_n;
+      place(c0, e_m, e_n);
+      const bool mine = e_n < c_end && e_m < M;
       const float* none = reinterpret_cast<const float*>(W);
-      next_old = *((mine && epi == EPI_ACC_F32) ? (const float*)C + (size_t)e_m * ldc + c0 + e_c : none);
-      next_bias = *((mine && bias) ? bias + c0 + e_c : none);
-      next_g = *((mine && fused.out_g) ? fused.out_g + c0 + e_c : none);
+      next_old = *((mine && epi == EPI_ACC_F32) ? (const float*)C + (size_t)e_m * ldc + e_n : none);
+      next_bias = *((mine && bias) ? bias + e_n : none);
+      next_g = *((mine && fused.out_g) ? fused.out_g + e_n : none);
     }
   };
   bf16x8 afr[NS];
@@ -2307,8 +2319,6 @@ __global__ __launch_bounds__(NW * 64) void stationary16_kernel(const void* __res
     floatx4 acc[NT];
 #pragma unroll
     for (int j = 0; j < NT; ++j) acc[j] = floatx4{0.f, 0.f, 0.f, 0.f};
-    const int e_n = c0 + e_c;
-    const bool e_mine = !PAIR && e_n < c_end && e_m < M;
     const float c_old = next_old, e_bias = next_bias, e_g = next_g;
     if constexpr (next) ask_epilogue(c0 + CH);
 #pragma unroll
@@ -2348,8 +2358,8 @@ __global__ __launch_bounds__(NW * 64) void stationary16_kernel(const void* __res
     };
     if constexpr (PAIR) {
       static_assert(NT == 2, "a gate tile and an up tile");
-      const int col = c0 + r16;
-      const int m = wid * 4 + (lane >> 4);
+      int col, m;
+      place(c0, m, col);
       if (epi == EPI_SWIGLU && col < c_end && col < ldc && m < M) {
         float g = 0.f, u = 0.f;
 #pragma unroll
@@ -2360,7 +2370,9 @@ __global__ __launch_bounds__(NW * 64) void stationary16_kernel(const void* __res
         ((bf16*)C)[(size_t)m * ldc + col] = (bf16)swiglu_f(g, u, bias);
       }
     } else {
-      if (e_mine) {
+      int e_m, e_n;
+      place(c0, e_m, e_n);
+      if (e_n < c_end && e_m < M) {
         float v = 0.f;
 #pragma unroll
         for (int ww = 0; ww < NW; ++ww) v += red[buf][ww][e_m][e_c];
@@ -2411,12 +2423,14 @@ int launch_stationary16(const void* A, int lda, const bf16* W, int ldw, const fl
     if (fused.in_ssq || fused.out_g) return MF_NOT_BUILT;
     kern<<<grid, NW * 64, smem, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, cols_total, unit, units / grid, units % grid,
                                       epi, *norm, FusedNorm{});
-  } else {
+  } else if constexpr (PAIR || NS * NW * 32 <= STATIONARY_PLAIN_K) {
     if (fused.out_g && (PAIR || grid > fused.out_parts)) return MF_NOT_BUILT;
     stationary16_kernel<NS, RING, NT, PAIR, false, TILED, NW><<<grid, NW * 64, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N,
                                                                              cols_total, unit, units / grid,
                                                                              units % grid, epi,
                                                                              NormArgs{nullptr, nullptr, 0.f}, fused);
+  } else {
+    return MF_NOT_BUILT;
   }
   return mf_launch_status();
 }

@@ -59,3 +59,25 @@ def test_stationary(m, n, k):
         out = base.clone()
         ops.linear(x, w, b, out, accumulate=True, tiled=tiled)
         assert (out - (want + base.double())).abs().max() <= 4 * 2.0 ** -20 * k ** 0.5 + 2.0 ** -22
+
+
+# the same with the norm folded in and with SwiGLU, at the lengths whose weights go through a shorter ring than a slice
+@pytest.mark.parametrize("m,n,k", [(8, 9024, 6144), (16, 4416, 7168), (3, 16384, 5120), (5, 2112, 8192)])
+def test_stationary_of_long_rows(m, n, k):
+    from minfer_amd.kernels import ops
+    x, w, b, _ = _operands(m, n, k)
+    h, gain = x.float(), torch.rand(k, device=DEV) + 0.5
+    h *= 1.0 + 2.0 ** -9                                    # (not the bfloat16 values themselves)
+    xg = (h * gain).to(torch.bfloat16).double()
+    z = xg @ w.double().t() / (h.double().square().mean(-1, keepdim=True) + 1e-6).sqrt()
+    left = []
+    for tiled in (ops.tile_weight(w), None):
+        out, half = torch.empty((m, n), device=DEV), torch.empty((m, n // 2), device=DEV, dtype=torch.bfloat16)
+        assert ops.linear_normed(h, gain, 1e-6, None, w, b, out, tiled=tiled)
+        assert ops.linear_normed(h, gain, 1e-6, None, w, None, half, tiled=tiled, swiglu=True)
+        left.append((out, half))
+    assert all(torch.equal(p, q) for p, q in zip(*left))
+    assert (left[0][0] - (z + b.double())).abs().max() <= 4 * 2.0 ** -20 * k ** 0.5 + 2.0 ** -22
+    gate, up = z.view(m, -1, 2, 32).unbind(2)
+    want = (torch.nn.functional.silu(gate) * up).reshape(m, n // 2)
+    assert (left[0][1].double() - want).abs().max() <= 2.0 ** -8 * want.abs().max() + 2.0 ** -12
