@@ -103,13 +103,16 @@ __device__ __forceinline__ bf16x8 load8_inside(const bf16* __restrict__ base, in
   return *reinterpret_cast<const bf16x8*>(base + (size_t)row * ld + k);
 }
 
-// Weights that no other workgroup reads, marked as read once: a stream of them alone comes at 6.2 TB/s so and at 5.9 without the mark
-// (a plain read of 670 MB by 256 workgroups), and what the step reads again stays in the caches.  With the last loads of a block no
-// longer there only to be dropped, and no wait for the weights in flight in front of an item (microseconds before / after, 8 rows, weights from
-// memory): 37,888 x 3,584 50.5 / 44.2 (6.1 TB/s), 4,608 x 3,584 10.4 / 8.4, 3,584 x 3,584 8.4 / 7.2, 3,584 x 18,944 26.0 / 24.9, 152,064 x 3,584 192 / 172,
-// 9,728 x 896 6.5 / 5.6, 151,936 x 896 63 / 49.  Not for what several tiles of rows read (`whole_kernel`, the prompts' tiles).
+// Weights that no other workgroup reads.  From the tiled copy a load takes whole lines and is marked as read once: what the step reads
+// again stays in the caches (microseconds without / with the mark, 8 rows, weights from memory: 152,064 x 6,144 326 / 292, 152,064 x
+// 3,584 194 / 175, 37,888 x 3,584 49.8 / 47.7, 4,608 x 3,584 10.5 / 9.7, 3,584 x 18,944 26.6 / 25.8; 64 rows, 37,888 x 3,584 53.4 / 48.7).  From the
+// matrix a load takes half a line of each of 16 rows, and the next step takes the other half: marked, the line is fetched twice (marked / not, 8 rows:
+// 152,064 x 6,144 392 / 344, 8,192 x 29,568 117 / 102, 3,584 x 18,944 35.8 / 31.4, 37,888 x 3,584 56.1 / 52.3; 64 rows:
+// 152,064 x 3,584 277 / 245).  Not for what several tiles of rows read (`whole_kernel`, the prompts' tiles).
+template <bool TILED>
 __device__ __forceinline__ bf16x8 load_weights(const bf16* p) {
-  return __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(p));
+  if constexpr (TILED) return __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(p));
+  else return *reinterpret_cast<const bf16x8*>(p);
 }
 
 // The epilogue of a wave's TM x TN tiles of 32 x 32 (D[m][n]: lane holds n = lane % 32,
@@ -372,7 +375,8 @@ __device__ __forceinline__ void dma16(const bf16* base, unsigned off, unsigned l
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds_byte)
                : "m0");
 }
-// The lanes of a mask, of weights that no other workgroup reads (ONCE, see `load_weights`) or of anything else
+// The lanes of a mask, of weights that no other workgroup reads (ONCE, see `load_weights`: a copy takes whole lines from the matrix too; SwiGLU of
+// 37,888 x 3,584 from the matrix, 64 rows, 54.0 / 48.5 us) or of anything else
 template <bool ONCE>
 __device__ __forceinline__ void dma16_lanes(const bf16* base, unsigned off, unsigned lds_byte, unsigned long long lanes) {
   if constexpr (ONCE)
@@ -1411,7 +1415,7 @@ __global__ __launch_bounds__(512) void skinny_ring_kernel(const bf16* __restrict
 #pragma unroll
   for (int i = 0; i < MT; ++i) stage[i] = *reinterpret_cast<const bf16x8*>(src[i] + k_begin);
 #pragma unroll
-  for (int s = 0; s < KC / 32; ++s) wr[s] = load_weights(wrow + ((k_begin >> 5) + s) * WSTEP);
+  for (int s = 0; s < KC / 32; ++s) wr[s] = load_weights<TILED>(wrow + ((k_begin >> 5) + s) * WSTEP);
 #pragma unroll
   for (int i = 0; i < MT; ++i)
     *reinterpret_cast<bf16x8*>(&As[(i * 16 + (tid >> 5)) * SK_LD + sk]) = stage[i];
@@ -1437,7 +1441,7 @@ __global__ __launch_bounds__(512) void skinny_ring_kernel(const bf16* __restrict
         acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, wr[s], acc[i], 0, 0, 0);
       }
       if constexpr (refill) {
-        wr[s] = load_weights(wrow + ((kn >> 5) + s) * WSTEP);
+        wr[s] = load_weights<TILED>(wrow + ((kn >> 5) + s) * WSTEP);
         __builtin_amdgcn_sched_barrier(0);    // use a register, then refill it, in this order
       }
     }
@@ -1773,7 +1777,7 @@ __global__ __launch_bounds__(NW * 64) void rolling16_kernel(const bf16* __restri
   bf16x8 a[S], w[NT][S];
   auto load = [&](int s, int at) {
 #pragma unroll
-    for (int j = 0; j < NT; ++j) w[j][s] = load_weights(wrow[j] + at * WSTEP);
+    for (int j = 0; j < NT; ++j) w[j][s] = load_weights<TILED>(wrow[j] + at * WSTEP);
     a[s] = *reinterpret_cast<const bf16x8*>(arow + at * 32);
   };
   auto multiply = [&](int s) {
@@ -2159,7 +2163,7 @@ __global__ __launch_bounds__(NW * 64) void stationary16_kernel(const void* __res
   auto first_loads = [&](int j) {
     wcur[j] = w_operand<TILED>(Wp, ldw, KK, lane_wrow(c_begin, j), k0);
 #pragma unroll
-    for (int s = 0; s < RING; ++s) w[j][s] = load_weights(wcur[j] + s * WSTEP);
+    for (int s = 0; s < RING; ++s) w[j][s] = load_weights<TILED>(wcur[j] + s * WSTEP);
   };
   // The epilogue's place of this lane in an item: wave w adds up the sums of activation rows
   // [w 64 / COLS, (w + 1) 64 / COLS), all waves at once.  What the epilogue needs from memory (the
@@ -2332,8 +2336,8 @@ __global__ __launch_bounds__(NW * 64) void stationary16_kernel(const void* __res
           asm volatile("" : "+v"(acc[j]) : : "memory");
           __builtin_amdgcn_sched_barrier(0);
         }
-        if (s + RING < NS) w[j][s % RING] = load_weights(wcur[j] + (s + RING) * WSTEP);
-        else if (next) w[j][s % RING] = load_weights(wrow[j] + (s + RING - NS) * WSTEP);
+        if (s + RING < NS) w[j][s % RING] = load_weights<TILED>(wcur[j] + (s + RING) * WSTEP);
+        else if (next) w[j][s % RING] = load_weights<TILED>(wrow[j] + (s + RING - NS) * WSTEP);
         __builtin_amdgcn_sched_barrier(0);      // keep "use a register, then refill it" in this order
       }
     }
@@ -2518,8 +2522,8 @@ __global__ __launch_bounds__(512) void panel_kernel(const bf16* __restrict__ A, 
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int s = 0; s < KC / 32; ++s) {
-    wr[0][s] = load_weights(wp[0] + s * WSTEP);
-    wr[1][s] = load_weights(wp[1] + s * WSTEP);
+    wr[0][s] = load_weights<TILED>(wp[0] + s * WSTEP);
+    wr[1][s] = load_weights<TILED>(wp[1] + s * WSTEP);
   }
   __builtin_amdgcn_sched_barrier(0);
   store_stage(0);
@@ -2556,7 +2560,7 @@ __global__ __launch_bounds__(512) void panel_kernel(const bf16* __restrict__ A, 
 #pragma unroll
         for (int i = 0; i < MT; ++i)
           acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], wr[j][s], acc[j][i], 0, 0, 0);
-        wr[j][s] = load_weights(wnext[j] + ((kn >> 5) + s) * WSTEP);
+        wr[j][s] = load_weights<TILED>(wnext[j] + ((kn >> 5) + s) * WSTEP);
         __builtin_amdgcn_sched_barrier(0);      // use a register, then refill it, in this order
       }
     }

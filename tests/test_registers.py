@@ -49,3 +49,42 @@ def test_products_of_few_rows_spill_nothing(tmp_path):
     few = {n: b for n, b in scratch.items() if any(k + "I" in n for k in kinds)}
     assert all(any(k + "I" in n for n in few) for k in kinds)
     assert not {n: b for n, b in few.items() if b}
+
+
+def _loads_marked_as_read_once(path, folder, names):
+    """Of the named kernels: how many loads of 16 bytes they have, and how many of those are marked."""
+    from minfer_amd.kernels import build
+    objdump = os.path.join(os.path.dirname(os.path.realpath(build._hipcc())), "..", "lib", "llvm", "bin", "llvm-objdump")
+    if not os.path.exists(objdump):
+        pytest.skip("no llvm-objdump beside hipcc")
+    code = os.path.join(folder, "code.o")
+    with open(code, "wb") as f:
+        f.write(_device_code(path))
+    text = subprocess.run([objdump, "-d", "--no-show-raw-insn", "--disassemble-symbols=" + ",".join(names), code], capture_output=True,
+                          text=True, check=True).stdout
+    found, name = {n: [0, 0] for n in names}, None
+    for line in text.splitlines():
+        head = re.match(r"[0-9a-f]+ <(\S+)>:", line)
+        if head:
+            name = head.group(1)
+        elif name in found and re.search(r"\b(global|flat)_load_dwordx4\b", line):
+            found[name][0] += 1
+            found[name][1] += bool(re.search(r"\bnt\b", line))
+    return found
+
+
+def test_only_whole_lines_are_marked_as_read_once(tmp_path):
+    """The kernels of few rows mark the weights that they read from the tiled copy, whose loads take whole lines.  From the matrix a
+    load takes half a line of each row: marked, the line would be fetched again for the other half."""
+    from minfer_amd.kernels import build
+    if not build.is_current("gemm_bf16"):
+        build.compile_library("gemm_bf16")
+    path = build.lib_path("gemm_bf16")
+    tiled = {}                                    # (the last of a kernel's yes-or-no parameters)
+    for n in _scratch_bytes(path, str(tmp_path)):
+        kind = re.search(r"\d(stationary16|rolling16|skinny_ring|panel)_kernelI(?:L[ib]\d+E)*?Lb([01])E(?:Li\dE)?EE", n)
+        if kind:
+            tiled[n] = kind.group(2) == "1"
+    assert len({n for n in tiled if tiled[n]}) == len(tiled) // 2 > 0
+    for n, (loads, marked) in _loads_marked_as_read_once(path, str(tmp_path), sorted(tiled)).items():
+        assert loads > 0 and (marked > 0) == tiled[n], (n, loads, marked)
