@@ -902,7 +902,8 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void tile_step_kernel(const
   constexpr int GROUPS = (BM + WAVES * 8 - 1) / (WAVES * 8);
   LanesSum<8, 4> sums[SCALED ? GROUPS : 1];
   auto part_row = [&](int q) {
-    return in_ssq + (size_t)min(m0 + (q * WAVES + wid) * 8 + (lane >> 3), M - 1) * in_parts;      // (rows past M: not stored)
+    const int r = m0 + (q * WAVES + wid) * 8 + (lane >> 3);  // (rows past M ask for nothing: 9,728 x 896 SwiGLU of 17 rows 8.65 us so and 9.1)
+    return r < M ? in_ssq + (size_t)r * in_parts : nullptr;
   };
   if constexpr (SCALED) {
 #pragma unroll
