@@ -578,12 +578,12 @@ __device__ __forceinline__ void dma_epilogue(floatx4 (&acc)[TT::I][TT::J], unsig
   }
 }
 
-template <int BM, int BN, int STAGES, bool GROUPED = false, bool HALVES = false>
+template <int BM, int BN, int STAGES, bool GROUPED = false, bool HALVES = false, bool TILED = false>
 __global__ __launch_bounds__(512, 2) void tile_dma_kernel(const bf16* __restrict__ A, int lda,
                                                        const bf16* __restrict__ W, int ldw,
                                                        const float* __restrict__ bias, void* __restrict__ C,
                                                        int ldc, int M, int N, int K, int epi, int tiles_m,
-                                                       int order, int k_per_split, bool tiled,
+                                                       int order, int k_per_split,
                                                        const RowGroup* __restrict__ groups = nullptr, Halves halves = Halves{}) {
   using TT = DmaTile<BM, BN>;
   constexpr int ROW = DMA_BK * 2, A_ST = BM * ROW, W_ST = BN * ROW, W_AT = STAGES * A_ST;
@@ -595,7 +595,7 @@ __global__ __launch_bounds__(512, 2) void tile_dma_kernel(const bf16* __restrict
     // and stores 32-bit sums into its own [M][N] slab of C; another kernel adds the slabs
     const int kb = part * k_per_split;
     A += kb;
-    W += tiled ? kb * 16 : kb;
+    W += TILED ? kb * 16 : kb;
     K = min(k_per_split, K - kb);
     C = (float*)C + (size_t)part * M * N;
   }
@@ -623,7 +623,7 @@ __global__ __launch_bounds__(512, 2) void tile_dma_kernel(const bf16* __restrict
 #pragma unroll
     for (int j = 0; j < J; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
 
-  const int wk = tiled ? 16 * DMA_BK : DMA_BK;               // weights from a k tile to the next
+  constexpr int wk = TILED ? 16 * DMA_BK : DMA_BK;           // weights from a k tile to the next
   // What a wave copies: pieces of 8 rows (1 KB), the lane row lane / 8 of a piece and the chunk that belongs at position
   // lane % 8.  Half h of A: the rows of the row blocks h IH .. + IH - 1 of every row of waves; half h of W: the rows of
   // the column blocks of that half of every column of waves.
@@ -643,7 +643,7 @@ __global__ __launch_bounds__(512, 2) void tile_dma_kernel(const bf16* __restrict
     const int jh = q < LW0 ? J0 : J1, p = (q < LW0 ? q : q - LW0) * 8 + wid;       // 2 jh pieces a column of waves
     const int b = TT::first(p / (2 * jh)) + ((q < LW0 ? 0 : J0) + (p % (2 * jh)) / 2) * TT::STEP;
     const int r0 = b * 16 + (p & 1) * 8, r = r0 + (lane >> 3);
-    gw[q] = w_copy_at(HALVES ? halves.row(n0 + r) : min(n0 + r, N - 1), ldw, (lane & 7) ^ ((r >> 1) & 7), tiled);
+    gw[q] = w_copy_at(HALVES ? halves.row(n0 + r) : min(n0 + r, N - 1), ldw, (lane & 7) ^ ((r >> 1) & 7), TILED);
     lw[q] = lds0 + W_AT + r0 * ROW;
   }
   auto copy_a = [&](int kt, int st, auto HALF) {
@@ -835,12 +835,13 @@ struct StepTile {
 
 // SCALED: the rows' sums are multiplied by 1 / sqrt(mean + eps) of the row, `in_parts` partial sums of squares of which stand
 // in in_ssq [M][in_parts] (FusedNorm::in_*; one launch, K whole).
-template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, bool GROUPED = false, bool SCALED = false, bool HALVES = false>
+template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, bool GROUPED = false, bool SCALED = false, bool HALVES = false,
+          bool TILED = false>
 __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void tile_step_kernel(const bf16* __restrict__ A, int lda,
                                                        const bf16* __restrict__ W, int ldw,
                                                        const float* __restrict__ bias, void* __restrict__ C,
                                                        int ldc, int M, int N, int K, int epi, int tiles_m,
-                                                       int order, int k_per_split, bool tiled,
+                                                       int order, int k_per_split,
                                                        const RowGroup* __restrict__ groups = nullptr,
                                                        const float* __restrict__ in_ssq = nullptr, int in_parts = 0,
                                                        float in_eps = 0.f, Halves halves = Halves{}) {
@@ -851,7 +852,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void tile_step_kernel(const
   if (k_per_split > 0) {                                     // as in tile_dma_kernel
     const int kb = part * k_per_split;
     A += kb;
-    W += tiled ? kb * 16 : kb;
+    W += TILED ? kb * 16 : kb;
     K = min(k_per_split, K - kb);
     C = (float*)C + (size_t)part * M * N;
   }
@@ -886,11 +887,11 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void tile_step_kernel(const
 #pragma unroll
   for (int q = 0; q < LW; ++q) {
     const int r = (q * WAVES + wid) * 8 + (lane >> 3);
-    gw[q] = w_copy_at(HALVES ? halves.row(n0 + r) : min(n0 + r, N - 1), ldw, (lane & 7) ^ ((r >> 1) & 7), tiled);
+    gw[q] = w_copy_at(HALVES ? halves.row(n0 + r) : min(n0 + r, N - 1), ldw, (lane & 7) ^ ((r >> 1) & 7), TILED);
   }
   const int nkt = K / DMA_BK;
   auto copy = [&](int kt, int st) {                          // (past the last tile: that one again, never read)
-    const int k = min(kt, nkt - 1) * DMA_BK, kw = tiled ? k * 16 : k;
+    const int k = min(kt, nkt - 1) * DMA_BK, kw = TILED ? k * 16 : k;
     const unsigned base = lds0 + st * ST + wid * 1024;
 #pragma unroll
     for (int q = 0; q < LW; ++q) dma16(W + kw, gw[q], __builtin_amdgcn_readfirstlane(base + BM * ROW + q * (WAVES * 1024)));
@@ -982,12 +983,12 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void tile_step_kernel(const
   dma_epilogue<TT, HALVES>(acc, smem + wid * TT::OWN, bias, C, ldc, M, N, HALVES ? EPI_SWIGLU : epi, m0 + wave_m * TT::ROWS, n0, wave_n, lane, halves);
 }
 
-template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, bool GROUPED, bool SCALED = false, bool HALVES = false>
+template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, bool GROUPED, bool SCALED = false, bool HALVES = false, bool TILED = false>
 int launch_tile_step(const bf16* A, int lda, const bf16* W, int ldw, const float* bias, void* C, int ldc, int M, int N, int K, int epi,
                      hipStream_t stream, int splits, int k_per_split, const RowGroup* groups, int n_groups,
-                     const float* in_ssq = nullptr, int in_parts = 0, float in_eps = 0.f, const Halves& halves = Halves{}, bool tiled = false) {
+                     const float* in_ssq = nullptr, int in_parts = 0, float in_eps = 0.f, const Halves& halves = Halves{}) {
   using TT = StepTile<BM, BN, WAVES_M, WAVES_N>;
-  auto kern = tile_step_kernel<BM, BN, WAVES_M, WAVES_N, STAGES, GROUPED, SCALED, HALVES>;
+  auto kern = tile_step_kernel<BM, BN, WAVES_M, WAVES_N, STAGES, GROUPED, SCALED, HALVES, TILED>;
   static bool configured = false;
   if (!configured) {
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -997,16 +998,16 @@ int launch_tile_step(const bf16* A, int lda, const bf16* W, int ldw, const float
   }
   const int tiles_m = GROUPED ? n_groups : (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
   kern<<<dim3(tiles_m * tiles_n, splits), 64 * TT::WAVES, TT::template lds<STAGES>(), stream>>>(
-      A, lda, W, ldw, bias, C, ldc, M, N, K, epi, tiles_m, tile_order(tiles_m * tiles_n, splits, M, N, K), k_per_split, tiled, groups, in_ssq, in_parts, in_eps, halves);
+      A, lda, W, ldw, bias, C, ldc, M, N, K, epi, tiles_m, tile_order(tiles_m * tiles_n, splits, M, N, K), k_per_split, groups, in_ssq, in_parts, in_eps, halves);
   return mf_launch_status();
 }
 
 // 64 x 64: five stages, so that two blocks fit a CU (ten for blocks that have a CU to themselves: level)
-template <bool SCALED>
+template <bool SCALED, bool TILED>
 int launch_tile64(const bf16* A, int lda, const bf16* W, int ldw, const float* bias, void* C, int ldc, int M, int N, int K, int epi,
-                  hipStream_t stream, int splits, int k_per_split, bool tiled, const float* in_ssq = nullptr, int in_parts = 0, float in_eps = 0.f) {
-  return launch_tile_step<64, 64, 2, 2, 5, false, SCALED>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi, stream, splits, k_per_split,
-                                                          nullptr, 0, in_ssq, in_parts, in_eps, Halves{}, tiled);
+                  hipStream_t stream, int splits, int k_per_split, const float* in_ssq = nullptr, int in_parts = 0, float in_eps = 0.f) {
+  return launch_tile_step<64, 64, 2, 2, 5, false, SCALED, false, TILED>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi, stream, splits, k_per_split,
+                                                                        nullptr, 0, in_ssq, in_parts, in_eps);
 }
 
 // ---- tiles that are all on the chip at once: weights straight into MFMA operands
@@ -1193,23 +1194,23 @@ int launch_tile_stream(int variant, const bf16* A, int lda, const bf16* Wt, cons
   return (int)hipErrorInvalidValue;
 }
 
-template <int BM, int BN, int STAGES, bool GROUPED, bool HALVES = false>
+template <int BM, int BN, int STAGES, bool GROUPED, bool HALVES = false, bool TILED = false>
 int configure_tile_dma() {
   static bool configured = false;
   if (configured) return 0;
-  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(tile_dma_kernel<BM, BN, STAGES, GROUPED, HALVES>),
+  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(tile_dma_kernel<BM, BN, STAGES, GROUPED, HALVES, TILED>),
                                            hipFuncAttributeMaxDynamicSharedMemorySize, DmaTile<BM, BN>::template lds<STAGES>());
   configured = e == hipSuccess;
   return (int)e;
 }
 
-template <int BM, int BN, int STAGES>
+template <int BM, int BN, int STAGES, bool TILED>
 int launch_tile_dma(const bf16* A, int lda, const bf16* W, int ldw, const float* bias, void* C, int ldc, int M,
-                    int N, int K, int epi, hipStream_t stream, int splits, int k_per_split, bool tiled) {
-  if (const int e = configure_tile_dma<BM, BN, STAGES, false>()) return e;
+                    int N, int K, int epi, hipStream_t stream, int splits, int k_per_split) {
+  if (const int e = configure_tile_dma<BM, BN, STAGES, false, false, TILED>()) return e;
   const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
-  tile_dma_kernel<BM, BN, STAGES><<<dim3(tiles_m * tiles_n, splits), 512, DmaTile<BM, BN>::template lds<STAGES>(), stream>>>(
-      A, lda, W, ldw, bias, C, ldc, M, N, K, epi, tiles_m, tile_order(tiles_m * tiles_n, splits, M, N, K), k_per_split, tiled, nullptr);
+  tile_dma_kernel<BM, BN, STAGES, false, false, TILED><<<dim3(tiles_m * tiles_n, splits), 512, DmaTile<BM, BN>::template lds<STAGES>(), stream>>>(
+      A, lda, W, ldw, bias, C, ldc, M, N, K, epi, tiles_m, tile_order(tiles_m * tiles_n, splits, M, N, K), k_per_split, nullptr);
   return mf_launch_status();
 }
 
@@ -1250,7 +1251,7 @@ int launch_grouped_dma(const bf16* A, int lda, const bf16* W, int ldw, void* C, 
   if (const int e = configure_tile_dma<BM, BN, STAGES, true, HALVES>()) return e;
   const int tiles_n = (N + BN - 1) / BN;
   tile_dma_kernel<BM, BN, STAGES, true, HALVES><<<dim3(n_groups * tiles_n), 512, DmaTile<BM, BN>::template lds<STAGES>(), stream>>>(
-      A, lda, W, ldw, nullptr, C, ldc, 0, N, K, EPI_F32, n_groups, n_groups * tiles_n >= 16, 0, false, groups, halves);
+      A, lda, W, ldw, nullptr, C, ldc, 0, N, K, EPI_F32, n_groups, n_groups * tiles_n >= 16, 0, groups, halves);
   return mf_launch_status();
 }
 
@@ -1260,7 +1261,7 @@ int launch_halves_dma(const bf16* A, int lda, const bf16* W, int ldw, bf16* C, i
   if (const int e = configure_tile_dma<BM, BN, STAGES, false, true>()) return e;
   const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
   tile_dma_kernel<BM, BN, STAGES, false, true><<<dim3(tiles_m * tiles_n), 512, DmaTile<BM, BN>::template lds<STAGES>(), stream>>>(
-      A, lda, W, ldw, nullptr, C, halves.width, M, N, K, EPI_SWIGLU, tiles_m, tile_order(tiles_m * tiles_n, 1, M, N, K), 0, false, nullptr, halves);
+      A, lda, W, ldw, nullptr, C, halves.width, M, N, K, EPI_SWIGLU, tiles_m, tile_order(tiles_m * tiles_n, 1, M, N, K), 0, nullptr, halves);
   return mf_launch_status();
 }
 
@@ -3278,20 +3279,27 @@ bool tile64_reads_tiled(const Weights& w, int M, int N, int splits) {
   return w.tiled && (long)((M + 63) / 64) * ((N + 63) / 64) * splits > cu_count();
 }
 
+template <bool T>
+int launch_form_of(int form, const bf16* A, int lda, const Weights& w, const float* bias, void* C, int ldc, int M, int N, int K,
+                   int epi, hipStream_t stream, int splits, int k_per_split) {
+  const bf16* W = w.at(T);
+  const int ldw = w.ld(T);
+  switch (form) {
+    case FORM_256: return launch_tile_dma<256, 256, 2, T>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi, stream, splits, k_per_split);
+    case FORM_192: return launch_tile_dma<256, 192, 2, T>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi, stream, splits, k_per_split);
+    case FORM_128: return launch_tile_dma<256, 128, 3, T>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi, stream, splits, k_per_split);
+    case FORM_128T: return launch_tile_dma<128, 256, 3, T>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi, stream, splits, k_per_split);
+  }
+  return form == FORM_SMALL ? launch_tile_step<128, 128, 2, 4, 4, false, false, false, T>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi, stream, splits,
+                                                                                          k_per_split, nullptr, 0)
+                            : launch_tile64<false, T>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi, stream, splits, k_per_split);
+}
+// (which of the two is known to the compiler: as an argument it cost products from the matrix 0.1 to 0.2 us, 896 x 896 of 100 rows 6.35 and 6.5)
 int launch_form(int form, const bf16* A, int lda, const Weights& w, const float* bias, void* C, int ldc, int M, int N, int K,
                 int epi, hipStream_t stream, int splits = 1, int k_per_split = 0) {
-  const bool t = form == FORM_TINY ? tile64_reads_tiled(w, M, N, splits) : w.tiled != nullptr;
-  const bf16* W = w.at(t);
-  const int ldw = w.ld(t);
-  switch (form) {
-    case FORM_256: return launch_tile_dma<256, 256, 2>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi, stream, splits, k_per_split, t);
-    case FORM_192: return launch_tile_dma<256, 192, 2>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi, stream, splits, k_per_split, t);
-    case FORM_128: return launch_tile_dma<256, 128, 3>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi, stream, splits, k_per_split, t);
-    case FORM_128T: return launch_tile_dma<128, 256, 3>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi, stream, splits, k_per_split, t);
-  }
-  return form == FORM_SMALL ? launch_tile_step<128, 128, 2, 4, 4, false>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi, stream, splits, k_per_split,
-                                                                         nullptr, 0, nullptr, 0, 0.f, Halves{}, t)
-                            : launch_tile64<false>(A, lda, W, ldw, bias, C, ldc, M, N, K, epi, stream, splits, k_per_split, t);
+  return (form == FORM_TINY ? tile64_reads_tiled(w, M, N, splits) : w.tiled != nullptr)
+             ? launch_form_of<true>(form, A, lda, w, bias, C, ldc, M, N, K, epi, stream, splits, k_per_split)
+             : launch_form_of<false>(form, A, lda, w, bias, C, ldc, M, N, K, epi, stream, splits, k_per_split);
 }
 
 // A few weight rows past whole tiles (a gate beside q|k|v, a low-rank factor) can cost a whole round of them: 2,048 rows against
@@ -3780,10 +3788,15 @@ static int skinny_product(const void* A, int lda, const void* W, const void* Wt,
     case SK_TILE: {
       if ((size_t)N * ldw * 2 >= (1ull << 32)) break;          // (operands beyond 4 GB go to the K-split kernels)
       const Weights both(w, wt, ldw, K);
-      const bool t = tile64_reads_tiled(both, M, N, 1);
-      return fused.in_ssq ? launch_tile64<true>(a, lda, both.at(t), both.ld(t), bias, C, ldc, M, N, K, epi, stream, 1, 0, t, fused.in_ssq,
-                                                fused.in_parts, fused.in_eps)
-                          : launch_tile64<false>(a, lda, both.at(t), both.ld(t), bias, C, ldc, M, N, K, epi, stream, 1, 0, t);
+      auto run = [&](auto SCALED, auto T) {
+        constexpr bool t = decltype(T)::value;
+        return launch_tile64<decltype(SCALED)::value, t>(a, lda, both.at(t), both.ld(t), bias, C, ldc, M, N, K, epi, stream, 1, 0, fused.in_ssq,
+                                                         fused.in_parts, fused.in_eps);
+      };
+      using Yes = std::true_type;
+      using No = std::false_type;
+      if (tile64_reads_tiled(both, M, N, 1)) return fused.in_ssq ? run(Yes{}, Yes{}) : run(No{}, Yes{});
+      return fused.in_ssq ? run(Yes{}, No{}) : run(No{}, No{});
     }
     default: break;
   }
