@@ -8,7 +8,7 @@
 //    their k tiles copied straight into LDS, 16x16x32 MFMA, two groups of four waves a quarter product apart.
 //  * `tile_step_kernel`: the same copies for tiles of 128 x 128 and 64 x 64 (fewer rows, and 17 to 64 rows against a short
 //    K), one barrier a k tile.
-//  * `tile_stream_kernel`: more than 64 rows whose tiles are all on the chip at once, weights from the tiled copy straight into MFMA
+//  * `tile_stream_kernel`: more than 128 rows whose tiles are all on the chip at once, weights from the tiled copy straight into MFMA
 //    operands.
 //  * `tile_kernel`: many rows of any alignment, through registers and double-buffered LDS, 32x32x16 MFMA.
 //  * `reduce_norm_kernel`: adds the parts of a K split into the stream and norms the new rows.
@@ -1011,15 +1011,17 @@ int launch_tile64(const bf16* A, int lda, const bf16* W, int ldw, const float* b
 }
 
 // ---- tiles that are all on the chip at once: weights straight into MFMA operands
-// What bounds products of some hundred rows is neither the matrix cores nor LDS but what a CU brings in: about 60 GB/s of weights and
-// activations together, whatever form the copies have (k tiles of 64: 128 rows x 128 columns 0.48 us, 96 x 128 0.38, 208 x 128 0.70, 128 x
-// 256 0.78, with 30 blocks on the chip as with 256, four or six k tiles ahead).  So the rows of a tile are what the product has, in 16s, and not
-// 128 or 256; weights, whose tiled copy holds them as the MFMA operands they are, go to registers, four k tiles ahead, each wave its own 32
+// What bounds products of some hundred rows is neither the matrix cores nor LDS but a chain of waits in each block: a k tile of 64 is 28 KB of
+// weights and activations for 96 x 128 and takes 0.46 us, 32 KB and 0.53 us for 128 x 128, with 30 blocks on the chip as with 256 and four k
+// tiles ahead as with six, 60 GB/s a CU; plain loads bring a CU 75 to 95 GB/s from memory with 30 blocks on the chip (24 with 256: all
+// of them share 6 TB/s) and 140 from an L2 (115 with 256).  A block's time goes with its tile, so the rows of a tile are what the product has, in
+// 16s, and not 128 or 256; weights, whose tiled copy holds them as the MFMA operands they are, go to registers, four k tiles ahead, each wave its own 32
 // columns; the activations of a k tile go through registers into one of two LDS buffers, and their fragments are read three
-// ahead of the products.  A short way in and out (no LDS at all in the epilogue) makes few parts of a K split pay: the cut kernels
-// alone, in microseconds, `tile_dma_kernel` / this one: 203 x 3,584 x 3,584 16.5 in 7 parts / 13.6 in 3, 203 x 4,608 x 3,584 19.6 in 7 / 16.1
-// in 2, 604 x 2,560 x 2,048 17.3 in 4 / 13.8 in 2, 604 x 2,048 x 2,048 16.4 in 4 / 11.3 in 2, 300 x 896 x 4,864 11.8 in 7 / 9.4 in 9
-// (weights from memory).  SwiGLU products were level at best (300 x 9,728 x 896 12.2 and 12.9) and have none.
+// ahead of the products.  A short way in and out (no LDS at all in the epilogue) makes few parts of a K split pay.  Products as the plan runs
+// them, without / with this kernel, in microseconds, weights and activations from memory: with the norm behind them 203 x 3,584 x 3,584 23.8 in 7
+// parts / 21.4 in 3, 150 x 4,096 x 4,096 24.1 in 8 / 20.4 in 4, 900 x 2,048 x 2,048 29.3 in 4 / 24.2 in 2, 150 x 2,048 x 11,008 27.8 in 15 /
+// 23.4 in 8; with the rotation 150 x 4,608 x 3,584 25.8 in 7 / 22.3 in 3; alone 300 x 8,192 x 4,096 42.2 in 2 / 37.7 whole.  SwiGLU products
+// were level at best (300 x 9,728 x 896 12.2 and 12.9) and have none.
 // Tried: 256 columns, weights marked as read once where other rows' tiles read them (slower: 13.7 and 15.3), fragments seven ahead with four
 // LDS buffers (level).
 template <int I>
@@ -3334,10 +3336,17 @@ double whole_more(int M, int N, int K, int behind) {
   return K > 3072 || mn > 2.2e6 || behind == 0 ? 0. : behind == 1 ? 4.5 : 3.2 + mn / 1e6;
 }
 
-// `tile_stream_kernel`'s tiles: 16 I rows, microseconds a k tile with every CU busy (an eighth less with few), and what a part of a split
-// (on its own; in front of the rotation) and a whole product cost beside what every plan pays.
-struct StreamForm { int i; double step_us, split_us, rotated_us, whole_us; };
-constexpr StreamForm STREAM_FORMS[2] = {{6, 0.44, 4.2, 5.0, 2.0}, {8, 0.51, 4.0, 5.0, 4.0}};
+// `tile_stream_kernel`'s tiles of 16 I rows, in microseconds with the kernel behind it: a k tile, what it takes more for the share of the chip and
+// every 10,000 of K, a million results' way to memory and back for every part, and the rest of a whole product and of a cut one, alone, in front of
+// the rotation and in front of the norm (least squares over 3,771 timings at 697 products of 129 to 2,048 rows against 512 to 11,008 of 896 to
+// 28,672, weights and activations from memory: 4 % off on average).
+struct StreamForm { int i; double step_us, wide_us, store_us, whole_us[3], cut_us[3]; };
+constexpr StreamForm STREAM_FORMS[2] = {{6, 0.46, 0.025, 2.3, {3.4, 8.5, 8.3}, {7.5, 8.8, 7.6}},
+                                        {8, 0.53, 0.035, 2.1, {4.6, 10.1, 10.4}, {8.6, 10.2, 8.9}}};
+// The other plans' times over their prices at the same products, from the tiled copy with the kernel behind them, 3 to 8 % off: whole and cut;
+// tiles of 256 and 256 x 128, of 128 x 128, of 64 x 64; alone, rotation, norm.
+constexpr double OF_PRICE[2][3][3] = {{{0.88, 1.07, 0.98}, {0.78, 1.07, 0.89}, {0.95, 1.02, 0.93}},
+                                      {{0.97, 1.03, 1.02}, {0.85, 0.90, 0.86}, {0.95, 1.00, 0.95}}};
 
 TilePlan plan_tiles(int M, int N, int K, bool dma_ok, int epi, int n_cu, int behind = 0, bool tiled = false) {
   const long cu = n_cu > 0 ? n_cu : 1;
@@ -3402,29 +3411,29 @@ TilePlan plan_tiles(int M, int N, int K, bool dma_ok, int epi, int n_cu, int beh
       const double us = dma_ok ? form(2, splits, per / 64) : rounds_us(t128 * splits, 2 * cu, 1.45 * slow, per / 64, 0.);
       offer(2, splits, per, us + parts_us(splits));
     }
-  // `tile_stream_kernel`, while all its tiles are on the chip at once, in at most eight parts of at least 256 of K.  Whole prompts of 66 to
-  // 2,048 tokens, four models 896 to 3,584 wide, without / with this choice: 2,048 wide 150 tokens 3,723 / 3,562 us, 300 4,731 / 4,640, 604
-  // 6,648 / 6,474, 900 8,118 / 7,946; 1,536 wide 450 tokens 3,223 / 3,154; 3,584 wide 150 tokens 5,186 / 5,089; level elsewhere.  Not in reach of the
-  // lines, a product with the kernel behind it without / with: up to 128 rows (level: the weights' stream), a K below 2,048 except in
-  // front of the rotation (1,536 x 1,536, 800 rows 18.2 / 20.5 us), few weight rows except around 900 rows (896 x 4,864, 180 rows
-  // 13.0 / 15.2, 2,048 rows 33.9 / 35.3; 900 rows of a prompt 2,393 / 2,334).  In front of the rotation a split of this kernel takes the place of another
-  // split only: where the product was whole, the parts cost the rotation more than they save (prompts of 450 tokens, 1,536 wide, 3,225 / 3,348).
-  // Whole up to 1,024 rows: a prompt of 1,400 tokens 2,048 wide 11,156 / 11,279, of 2,048 13,548 / 13,792.
-  const bool enough = behind == 1 || (K >= 2048 && (N >= 1024 || (M >= 700 && M <= 1100)));
-  const bool cut_anyway = best.splits > 1;
-  const double stream_more = behind == 1 ? (K > 3072 ? 9.5 : 4.5) : behind == 2 ? 3.2 + mn / 1e6 : 0.;      // (`whole_more`)
-  if (dma_ok && tiled && epi != EPI_SWIGLU && M > 128 && enough)
+  // `tile_stream_kernel`, while all its tiles are on the chip at once, in at most eight parts (more were level) of four k tiles and more on
+  // average: where it takes 3 % less than the plan so far, both as they were timed.  160 of the 697
+  // products go to it (see STREAM_FORMS), 0.980 of the time on average over all, eight of them 1 to 8 % slower than without; 420 others that the prices were not
+  // made from: 0.987, 18 more than 2 % slower, none more than 6 %.  Whole prompts of 37 to 2,048 tokens, 896 to 3,584 wide: within 2 % of lines that
+  // were drawn after such prompts.
+  // Not in the place of 64 x 64 tiles of a K past TINY_K (their price is another: 23 of the 697, level at best, 896 x 4,864 of 150 rows 13.1 and 15.0); in
+  // front of the rotation a split only in the place of another split (level, and prompts of 450 tokens 1,536 wide 3,225 whole and 3,348 cut); not
+  // for up to 128 rows (level: the weights' stream).
+  const int used = !dma_ok ? -1 : best.variant == 16 ? FORM_128 : dma_form(best.variant, M, N, K, epi, best.k_per_split / 64, best.splits, cu);
+  if (dma_ok && tiled && epi != EPI_SWIGLU && M > 128 && !(used == FORM_TINY && K > TINY_K)) {
+    const bool was_cut = best.splits > 1;
+    double us = 0.97 * best.us * OF_PRICE[was_cut][used == FORM_TINY ? 2 : used == FORM_SMALL ? 1 : 0][behind];
     for (const StreamForm& f : STREAM_FORMS) {
       const long t = tiles(16 * f.i, 128);
       for (long parts = 1; parts <= 8 && t * parts <= cu && (parts == 1 || nkt >= 4 * parts); ++parts) {
         const long steps = (nkt + parts - 1) / parts, splits = (nkt + steps - 1) / steps;
-        if (splits != parts || (splits > 1 ? behind == 1 && !cut_anyway : M > 1024)) continue;
-        const double us = f.step_us * (0.86 + 0.14 * (double)(t * splits) / (double)cu) * (double)steps;
-        offer(VARIANT_STREAM + f.i, (int)splits, splits > 1 ? (int)steps * 64 : K,
-              splits > 1 ? us + (behind == 1 ? f.rotated_us : f.split_us) + parts_us((int)splits)
-                         : us + f.whole_us + start_us - more_us + epi_us + stream_more);
+        if (splits != parts || (splits > 1 && behind == 1 && !was_cut)) continue;
+        const double own = (f.step_us + f.wide_us * (double)(t * splits) / (double)cu * (double)K / 1e4) * (double)steps +
+                           f.store_us * (double)splits * mn / 1e6 + (splits > 1 ? f.cut_us : f.whole_us)[behind];
+        if (own < us) best = TilePlan{VARIANT_STREAM + f.i, (int)splits, splits > 1 ? (int)steps * 64 : K, us = own};
       }
     }
+  }
   return best;
 }
 

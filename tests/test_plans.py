@@ -383,3 +383,38 @@ def test_plan_linear_names_the_kernels_of_folded_norms():
         assert ops.plan_linear(m, n, k, n_cu=256)["splits"] == 1
         cut = ops.plan_linear(m, n, k, n_cu=256, behind=behind)
         assert cut["splits"] > 1 and cut["kernel"].endswith("(split K)")
+
+
+def test_tile_plan_with_the_tiled_copy():
+    """With the tiled copy a product takes the plan that it takes without, or the kernel that reads that copy alone: never for SwiGLU, for up
+    to 128 rows or a K not in 64s; all its tiles on the chip at once, at most eight parts, none of them empty."""
+    taken = 0
+    for n_cu, m, n, k, behind in itertools.product((104, 256), (65, 128, 129, 203, 300, 604, 900, 2048), (96, 512, 1001, 2048, 8192),
+                                                   (64, 200, 2048, 3648, 18944), (0, 1, 2)):
+        for epi in (ops.EPI_ACC_F32, ops.EPI_SWIGLU):
+            if epi == ops.EPI_SWIGLU and n % 64:
+                continue
+            plain, (variant, splits, per) = (ops._tile_plan(m, n, k, epi, k % 8 == 0, n_cu, behind, t) for t in (False, True))
+            if (variant, splits, per) == plain:
+                assert variant <= 20
+                continue
+            taken += 1
+            assert variant in (26, 28) and epi != ops.EPI_SWIGLU and m > 128 and k % 64 == 0
+            bm = (variant - 20) * 16
+            assert (m + bm - 1) // bm * ((n + 127) // 128) * splits <= n_cu and 1 <= splits <= 8
+            assert per == k if splits == 1 else per % 64 == 0 and (splits - 1) * per < k <= splits * per
+    assert taken > 50
+
+
+def test_stream_plan_follows_tiles_and_results():
+    """Which kernel a product takes with the tiled copy follows from prices: along the rows it changes where a tile is added (tiles have 64 to 256
+    rows in 32s), and between two such numbers where one price passes another, which is another number for every shape.  (Lines at 700 and 1,100
+    rows were the same two numbers for most of these.)"""
+    changes = {}
+    for n, k, behind in itertools.product((512, 768, 896, 1024), (2048, 3072, 4864, 8192), (0, 2)):
+        plans = [ops._tile_plan(m, n, k, ops.EPI_ACC_F32 if behind else ops.EPI_F32, True, 256, behind, True)[0] > 20 for m in range(129, 1409)]
+        for i in range(1, len(plans)):
+            if plans[i] != plans[i - 1]:
+                changes.setdefault(129 + i, []).append((n, k, behind))
+    assert changes
+    assert not {m: at for m, at in changes.items() if m % 32 != 1 and len(at) > 2}
