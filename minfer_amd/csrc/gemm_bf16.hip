@@ -1724,47 +1724,38 @@ __device__ __forceinline__ void norm_part_out(const FusedNorm& f, float sq, int 
   }
 }
 
-// The same split of the work as skinny16_kernel (a block owns 16 NT weight rows, its waves split
+// The same split of the work as skinny16_kernel (a block owns up to 16 weight rows, its waves split
 // K), for aligned operands and K a multiple of 32, with the loads rolling: a wave holds S steps
 // of weights and activations in registers, and the refill of a register is issued right behind
 // the MFMA that read it, so S steps of loads stay in flight the whole time in half the
 // registers of the two-buffer scheme above.  With K of many thousands and few weight rows
 // (the down projection) the chip is filled by loads in flight, not by blocks, and this is
 // what the time depends on.
-template <int NW, int NT, int S, bool PAIR, bool TILED>
+template <int NW, int S, bool TILED>
 __global__ __launch_bounds__(NW * 64) void rolling16_kernel(const bf16* __restrict__ A, int lda,
                                                             const bf16* __restrict__ W, int ldw,
                                                             const float* __restrict__ bias,
                                                             void* __restrict__ C, int ldc, int M, int N,
                                                             int K, int steps_per_wave, int epi, int rpb,
                                                             FusedNorm fused) {
-  constexpr int COLS = 16 * NT;
+  constexpr int COLS = 16;
   constexpr int RS = COLS + 4;
   constexpr int WSTEP = TILED ? 512 : 32;
   __shared__ float red[NW][16][RS];
   const int lane = threadIdx.x & 63;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);     // the same in the whole wave
   const int r16 = lane & 15;
-  // rpb: weight rows per block (at most 16 NT; fewer when that spreads the rows over every CU:
+  // rpb: weight rows per block (at most 16; fewer when that spreads the rows over every CU:
   // a CU draws only so much from memory, so an idle CU is bandwidth lost).  Lanes past the
   // block's rows read its last row again, from the CU's own cache.
-  auto tile_row = [&](int j) {
-    return PAIR ? (blockIdx.x >> 1) * 64 + (blockIdx.x & 1) * 16 + j * 32 : blockIdx.x * rpb + j * 16;
-  };
-  auto lane_row = [&](int j) {           // the weight row this lane reads in tile j
-    return PAIR ? tile_row(j) + r16 : blockIdx.x * rpb + min(j * 16 + r16, rpb - 1);
-  };
+  const int n0 = blockIdx.x * rpb;
   const int total = K / 32;
   const int T = min(steps_per_wave, total - wid * steps_per_wave);       // steps of this wave (none: not above 0)
   const int first = T > 0 ? wid * steps_per_wave : 0;
   const int kq = first * 32 + (lane >> 4) * 8;
   const bf16* arow = A + (size_t)min(r16, M - 1) * lda + kq;
-  const bf16* wrow[NT];
-#pragma unroll
-  for (int j = 0; j < NT; ++j) wrow[j] = w_operand<TILED>(W, ldw, K, min(lane_row(j), N - 1), kq);
-  floatx4 acc[NT];
-#pragma unroll
-  for (int j = 0; j < NT; ++j) acc[j] = floatx4{0.f, 0.f, 0.f, 0.f};
+  const bf16* wrow = w_operand<TILED>(W, ldw, K, min(n0 + min(r16, rpb - 1), N - 1), kq);
+  floatx4 acc = floatx4{0.f, 0.f, 0.f, 0.f};
   // The epilogue's place of this lane: wave w adds up the sums of activation rows
   // [w 64 / COLS, (w + 1) 64 / COLS), every wave one pass at the same time.  Where the product is
   // added to what the output holds, the old value is asked for here, in front of the whole stream:
@@ -1772,22 +1763,18 @@ __global__ __launch_bounds__(NW * 64) void rolling16_kernel(const bf16* __restri
   constexpr int ROWS_PER_PASS = 64 / COLS;
   static_assert(NW * ROWS_PER_PASS >= 16, "a pass for every activation row");
   const int e_c = lane % COLS;
-  const int e_n = tile_row(e_c >> 4) + (e_c & 15);
+  const int e_n = n0 + e_c;
   const int e_m = wid * ROWS_PER_PASS + lane / COLS;
-  const bool e_mine = e_m < M && e_n < N && (PAIR || e_c < rpb);
+  const bool e_mine = e_m < M && e_n < N && e_c < rpb;
   float c_old = 0.f, e_g = 0.f;
   if (epi == EPI_ACC_F32 && e_mine) c_old = ((const float*)C)[(size_t)e_m * ldc + e_n];
   if (fused.out_g && e_mine) e_g = fused.out_g[e_n];       // the next norm's weight, where this product prepares it
-  bf16x8 a[S], w[NT][S];
+  bf16x8 a[S], w[S];
   auto load = [&](int s, int at) {
-#pragma unroll
-    for (int j = 0; j < NT; ++j) w[j][s] = load_weights<TILED>(wrow[j] + at * WSTEP);
+    w[s] = load_weights<TILED>(wrow + at * WSTEP);
     a[s] = *reinterpret_cast<const bf16x8*>(arow + at * 32);
   };
-  auto multiply = [&](int s) {
-#pragma unroll
-    for (int j = 0; j < NT; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[s], w[j][s], acc[j], 0, 0, 0);
-  };
+  auto multiply = [&](int s) { acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[s], w[s], acc, 0, 0, 0); };
   if (steps_per_wave <= S) {   // a slice that the registers hold: all of it asked for at once (in a loop over the slice's length the
                                // compiler waits for every step: a decode step of one sequence at the 0.5B widths 775 us so, 749 at once)
 #pragma unroll
@@ -1827,23 +1814,8 @@ __global__ __launch_bounds__(NW * 64) void rolling16_kernel(const bf16* __restri
   }
   // D[m][n]: n = lane % 16, m = 4 (lane / 16) + r
 #pragma unroll
-  for (int j = 0; j < NT; ++j)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) red[wid][(lane >> 4) * 4 + r][j * 16 + r16] = acc[j][r];
+  for (int r = 0; r < 4; ++r) red[wid][(lane >> 4) * 4 + r][r16] = acc[r];
   __syncthreads();
-  if (epi == EPI_SWIGLU) {
-    if constexpr (PAIR && NT == 2) {
-      const int col = blockIdx.x * 16 + r16;
-      const int m = wid * 4 + (lane >> 4);
-      if (col < ldc && m < M) {
-        float g = 0.f, u = 0.f;
-#pragma unroll
-        for (int ww = 0; ww < NW; ++ww) { g += red[ww][m][r16]; u += red[ww][m][16 + r16]; }
-        ((bf16*)C)[(size_t)m * ldc + col] = (bf16)swiglu_f(g, u, bias);
-      }
-    }
-    return;
-  }
   float sq = 0.f;
   if (e_mine) {
     float v = bias ? bias[e_n] : 0.f;
@@ -1860,7 +1832,11 @@ __global__ __launch_bounds__(NW * 64) void rolling16_kernel(const bf16* __restri
   if (fused.out_g) norm_part_out<COLS>(fused, sq, e_m, e_c, M);
 }
 
-// How many steps `rolling16_kernel` holds for slices of `steps`: at most 16, the one whose rounds have the fewest steps past the end.
+// How many steps `rolling16_kernel` holds for slices of `steps`: at most 16, the one whose rounds have the fewest steps past the end.  Every length
+// from 10 to 15 has shapes that it pays for (8 rows, tiled copy, weights from memory, microseconds with 16 steps only / 10, 12 and 16 / all):
+// 896 x 4,864 9.25 / 6.8 / 6.8 (10 steps), 2,048 x 5,632 11.0 / 9.4 / 9.1 (11), 2,048 x 11,008 15.8 / 15.7 / 14.9 (11), 1,536 x 8,960 14.0 / 11.65 /
+// 11.65 (12), 2,560 x 9,728 15.4 / 13.9 / 13.5 (13), 8,192 x 29,568 90 / 86 / 84.7 (13), 4,096 x 14,336 24.3 / 23.5 / 22.5 (14), 3,584 x 18,944
+// 29.0 / 29.4 / 27.5 (15).
 int rolling_steps(int steps) {
   int best = 16;
   for (int s = 15; s >= 10 && steps > 16; --s)
@@ -1880,7 +1856,7 @@ int launch_rolling16(const bf16* A, int lda, const bf16* W, int ldw, const float
   const int blocks = (N + rpb - 1) / rpb;
   if (fused.out_g && blocks > fused.out_parts) return MF_NOT_BUILT;
   auto run = [&](auto S) {
-    rolling16_kernel<NW, 1, decltype(S)::value, false, TILED><<<blocks, NW * 64, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K,
+    rolling16_kernel<NW, decltype(S)::value, TILED><<<blocks, NW * 64, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K,
                                                                                               steps_per_wave, epi, rpb, fused);
   };
 #define MF_ROLLING(S_) case S_: run(std::integral_constant<int, S_>{}); break;
