@@ -170,10 +170,10 @@ __device__ __forceinline__ void tile_epilogue(floatx16 (&acc)[TM][TN], const flo
 // 32 tile rows would share 33).
 __device__ __forceinline__ void tile_position(int tile, int tiles_m, int tiles_n, int& bm, int& bn) {
   constexpr int BAND = 8;
-  const int band = (tile / (BAND * tiles_n)), first = band * BAND;
+  const int band = tile / (BAND * tiles_n), first = band * BAND;
   const int rows = min(tiles_m - first, BAND);
   const int in_band = tile - band * BAND * tiles_n;
-  bn = (in_band / rows);
+  bn = in_band / rows;
   bm = first + in_band - bn * rows;
 }
 
@@ -193,9 +193,8 @@ __device__ __forceinline__ void block_work(int order, int& tile, int& part) {
     const int per = n / 8, rem = n % 8, x = at % 8;
     at = x * per + min(x, rem) + at / 8;
   }
-  // (a division is vector work; the same in the whole block all the same, and what hangs on it stays in scalar registers so)
-  part = (order == ORDER_PARTS ? at / (int)gridDim.x : blockIdx.y);
-  tile = (order == ORDER_PARTS ? at - part * (int)gridDim.x : at);
+  part = order == ORDER_PARTS ? at / (int)gridDim.x : blockIdx.y;
+  tile = order == ORDER_PARTS ? at - part * (int)gridDim.x : at;
 }
 // Part by part where the activations of all of K are half as much again as an XCD's L2 of 4 MB and all parts' tiles are at most two a
 // CU.  (rows x weight rows x K, microseconds with the kernel behind it, the same eighth of every part / part by part: 800 x 1,536 x
@@ -2424,8 +2423,11 @@ int launch_stationary16(const void* A, int lda, const bf16* W, int ldw, const fl
 // second kernel.  The share is cut into passes of at most 16 tiles; wave w multiplies tiles w and
 // w + 8 of the pass.  A slot with no tile multiplies the matrix's first bytes, read by all lanes
 // alike, and its sums are dropped: every wave runs the same instructions, so the loads in flight
-// can be counted, and such a load is one look-up in the CU's cache where a tile's (64 lanes in
-// 16 rows) is 64 -- repeating a real tile there made the cache's tag rate the limit.  Weights go
+// can be counted, and such a load is one look-up where a tile's (64 lanes in 16 rows) is 64 -- repeating
+// a real tile there made the cache's tag rate the limit.  They are marked as read once like the others (tiled copy, all loads marked / none /
+// all but the second tile's of a wave, where the slots with no tile are, microseconds: 152,064 x 3,584 17 rows 184 / 197 / 196, 64 rows 211 / 230 / 231; 151,936 x 2,048
+// 48 rows 116 / 130 / 130; SwiGLU 43,008 x 5,120 64 rows 84 / 93 / 92; 151,936 x 896 level).  A body of its own for the last step,
+// with nothing asked for to be dropped, costs the others more than it saves: 184 / 186, 211 / 217, 116 / 121, 84 / 87.  Weights go
 // from HBM straight into MFMA operands through a ring of 16 fragments a wave: the load of the
 // next chunk's fragment is issued right behind the MFMA that frees the register, and runs on
 // into the next pass (a ring of two chunks measured the same).  The activations of a chunk
