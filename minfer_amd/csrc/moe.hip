@@ -345,13 +345,33 @@ __global__ __launch_bounds__(256) void moe_sparse_down_kernel(const WT* __restri
   }
 }
 
+// Lane (c, r) of c in 0..7, r in 0..7 (8 c + r) holds chunk c of row r in a and of row 8 + r in b; behind it the lanes 16 g + i hold of row i
+// chunk 2 g in a and chunk 2 g + 1 in b.  `upper`: whether the lane's r is a row of the upper eight, lane & 8.
+__device__ __forceinline__ void swap_halves(bf16x8& a, bf16x8& b, bool upper) {
+  using intx4 = __attribute__((ext_vector_type(4))) int;
+  intx4 x = __builtin_bit_cast(intx4, a), y = __builtin_bit_cast(intx4, b);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int t = __builtin_amdgcn_update_dpp(0, upper ? x[i] : y[i], 0x128, 0xf, 0xf, false);      // (row_ror:8)
+    if (upper) x[i] = t;
+    else y[i] = t;
+  }
+  a = __builtin_bit_cast(bf16x8, x);
+  b = __builtin_bit_cast(bf16x8, y);
+}
+
 // The same two products on the matrix cores, bfloat16, for rows of a multiple of 64 values and a multiple of 16 output
 // rows.  A workgroup of NW waves owns (expert, 16 output rows) and leaves at once where nobody chose the expert; its
-// waves share K, 64 values a step: A = 16 rows of a matrix (16x16x32 MFMA, a lane two neighbouring runs of 8 values, so
-// that a step reads 128 bytes of every row side by side), B = the rows of the expert's pairs, a column each, with the
-// same order of k.  The waves' sums meet in LDS and are added in the waves' order.  The matrices are read by one workgroup each and
-// marked as read once, which gives the stream back some 5 % (a plain read 5.9 and 6.2 TB/s): a reply of 8 sequences, 32 steps with three
-// layers of experts 4,096 x 2,048, 18,006 us without and 17,656 with the mark.
+// waves share K, 64 values a step: A = 16 rows of a matrix (16x16x32 MFMA), B = the rows of the expert's pairs, a column each.  The waves'
+// sums meet in LDS and are added in the waves' order.
+// What bounds it is the stream of the matrices.  They are read by one workgroup each and marked as read once, so that what the
+// step reads again stays in the caches; a marked load has to take whole lines, or the line is fetched again for what is left of it.  So
+// a load takes 128 bytes of each of 8 rows, and two such loads become two MFMA operands by an exchange within runs of 16 lanes
+// (`swap_halves`): a lane of row r, group g ends with values 16 g .. 16 g + 15 of the step.  Microseconds of both kernels and the sum behind them,
+// parts of the line of 16 rows a load, not marked / marked / whole lines, marked / whole, not marked; matrices from memory: 8 tokens, one of 8
+// experts of 4,096 x 2,048 44.1 / 45.6 / 39.8 / 43.7, two of 8 of 14,336 x 4,096 445 / 532 / 391 / 430, four of 32 of 1,536 x 2,048 88.6 / 98.9 / 79.6 /
+// 88.3; 16 tokens, two of 16 of 1,024 x 1,024 25.9 / 27.9 / 24.3 / 25.9.  A reply of 8 sequences, 32 steps with three layers of experts 4,096 x 2,048:
+// 18,370 / 17,450 / 16,830 / 18,220.  (One token, whose expert of 50 MB lies in the memory-side cache: 17.7 / 21.1 / 21.5 / 18.4.)
 //   UP:  two matrices (gate and up) share B; y[pair][f] gets the activation.
 //   else: rows[pair][n] gets the product.
 template <int NW, bool UP>
@@ -380,7 +400,7 @@ __global__ __launch_bounds__(NW * 64) void moe_sparse_mfma_kernel(const bf16* __
   const bf16* xr = x + (size_t)(UP ? pr / top : pr) * K + 16 * g;
   const bf16* wr[MATS];
 #pragma unroll
-  for (int m = 0; m < MATS; ++m) wr[m] = weights + ((size_t)e * MATS * N + (size_t)m * N + n0 + col) * K + 16 * g;
+  for (int m = 0; m < MATS; ++m) wr[m] = weights + ((size_t)e * MATS * N + (size_t)m * N + n0 + (lane & 7)) * K + 8 * (lane >> 3);
   floatx4 acc[MATS];
 #pragma unroll
   for (int m = 0; m < MATS; ++m) acc[m] = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -392,9 +412,11 @@ __global__ __launch_bounds__(NW * 64) void moe_sparse_mfma_kernel(const bf16* __
 #pragma unroll
     for (int q = 0; q < 2; ++q) {
 #pragma unroll
-      for (int m = 0; m < MATS; ++m) a[m][q] = __builtin_nontemporal_load((const bf16x8*)(wr[m] + s * 64 + 8 * q));
+      for (int m = 0; m < MATS; ++m) a[m][q] = __builtin_nontemporal_load((const bf16x8*)(wr[m] + (size_t)q * 8 * K + s * 64));
       b[q] = *(const bf16x8*)(xr + s * 64 + 8 * q);
     }
+#pragma unroll
+    for (int m = 0; m < MATS; ++m) swap_halves(a[m][0], a[m][1], lane & 8);
 #pragma unroll
     for (int q = 0; q < 2; ++q)
 #pragma unroll

@@ -52,7 +52,8 @@ def test_products_of_few_rows_spill_nothing(tmp_path):
 
 
 def _loads_marked_as_read_once(path, folder, names):
-    """Of the named kernels: how many loads of 16 bytes they have, and how many of those are marked."""
+    """Of the named kernels: how many loads of 16 bytes they have, how many of those are marked, and how many exchanges of values between the
+    lanes l and l ^ 8 of 16."""
     from minfer_amd.kernels import build
     objdump = os.path.join(os.path.dirname(os.path.realpath(build._hipcc())), "..", "lib", "llvm", "bin", "llvm-objdump")
     if not os.path.exists(objdump):
@@ -62,7 +63,7 @@ def _loads_marked_as_read_once(path, folder, names):
         f.write(_device_code(path))
     text = subprocess.run([objdump, "-d", "--no-show-raw-insn", "--disassemble-symbols=" + ",".join(names), code], capture_output=True,
                           text=True, check=True).stdout
-    found, name = {n: [0, 0] for n in names}, None
+    found, name = {n: [0, 0, 0] for n in names}, None
     for line in text.splitlines():
         head = re.match(r"[0-9a-f]+ <(\S+)>:", line)
         if head:
@@ -70,6 +71,8 @@ def _loads_marked_as_read_once(path, folder, names):
         elif name in found and re.search(r"\b(global|flat)_load_dwordx4\b", line):
             found[name][0] += 1
             found[name][1] += bool(re.search(r"\bnt\b", line))
+        elif name in found:
+            found[name][2] += "row_ror:8" in line
     return found
 
 
@@ -86,5 +89,18 @@ def test_only_whole_lines_are_marked_as_read_once(tmp_path):
         if kind:
             tiled[n] = kind.group(2) == "1"
     assert len({n for n in tiled if tiled[n]}) == len(tiled) // 2 > 0
-    for n, (loads, marked) in _loads_marked_as_read_once(path, str(tmp_path), sorted(tiled)).items():
+    for n, (loads, marked, _) in _loads_marked_as_read_once(path, str(tmp_path), sorted(tiled)).items():
         assert loads > 0 and (marked > 0) == tiled[n], (n, loads, marked)
+
+
+def test_experts_marked_loads_take_whole_lines(tmp_path):
+    """The chosen experts' matrices are rows, marked as read once: a load takes 128 bytes of eight of them, and lanes exchange
+    four values of every two such loads to have the rows as MFMA operands."""
+    from minfer_amd.kernels import build
+    if not build.is_current("moe"):
+        build.compile_library("moe")
+    path = build.lib_path("moe")
+    names = sorted(n for n in _scratch_bytes(path, str(tmp_path)) if "moe_sparse_mfma_kernel" in n)
+    assert len(names) == 4
+    for n, (loads, marked, exchanges) in _loads_marked_as_read_once(path, str(tmp_path), names).items():
+        assert loads > marked > 0 and exchanges >= 2 * marked, (n, loads, marked, exchanges)
