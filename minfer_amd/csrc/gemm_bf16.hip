@@ -3394,11 +3394,16 @@ TilePlan plan_tiles(int M, int N, int K, bool dma_ok, int epi, int n_cu, int beh
   // products go to it (see STREAM_FORMS), 0.980 of the time on average over all, eight of them 1 to 8 % slower than without; 420 others that the prices were not
   // made from: 0.987, 18 more than 2 % slower, none more than 6 %.  Whole prompts of 37 to 2,048 tokens, 896 to 3,584 wide: within 2 % of lines that
   // were drawn after such prompts.
+  // Beyond the rows that the prices were made from a whole product in front of the norm has 2.6 us more for every 1,000 rows past 2,200: the norm's own
+  // kernel, a workgroup a row (3,169 rows of 896 x 4,864 52.1 us in parts / 54.1 whole, 4,000 of 768 x 3,072 39.9 / 41.9, 3,372 of 1,000 x 2,816 40.7 /
+  // 45.6; without the term 3 to 6 us under what they take).  Of 60 products of 2,049 to 5,710 rows against 512 to 1,024 of 768 to 4,864 that go to the kernel: 0.915
+  // of the time on average, all but two faster; 2,161 x 640 x 2,560 20.6 / 22.8.
   // Not in the place of 64 x 64 tiles of a K past TINY_K (their price is another: 23 of the 697, level at best, 896 x 4,864 of 150 rows 13.1 and 15.0); in
   // front of the rotation a split only in the place of another split (level, and prompts of 450 tokens 1,536 wide 3,225 whole and 3,348 cut); not
-  // for up to 128 rows (level: the weights' stream).
+  // for up to 128 rows (level: the weights' stream); not for a K below 768, which the prices were not made from and where they are mostly their rests
+  // (1,400 x 1,536, with the norm: K 320 15.75 without and 17.15 with, 512 17.4 and 18.2, 768 19.1 and 18.2).
   const int used = !dma_ok ? -1 : best.variant == 16 ? FORM_128 : dma_form(best.variant, M, N, K, epi, best.k_per_split / 64, best.splits, cu);
-  if (dma_ok && tiled && epi != EPI_SWIGLU && M > 128 && !(used == FORM_TINY && K > TINY_K)) {
+  if (dma_ok && tiled && epi != EPI_SWIGLU && M > 128 && K >= 768 && !(used == FORM_TINY && K > TINY_K)) {
     const bool was_cut = best.splits > 1;
     double us = 0.97 * best.us * OF_PRICE[was_cut][used == FORM_TINY ? 2 : used == FORM_SMALL ? 1 : 0][behind];
     for (const StreamForm& f : STREAM_FORMS) {
@@ -3407,7 +3412,8 @@ TilePlan plan_tiles(int M, int N, int K, bool dma_ok, int epi, int n_cu, int beh
         const long steps = (nkt + parts - 1) / parts, splits = (nkt + steps - 1) / steps;
         if (splits != parts || (splits > 1 && behind == 1 && !was_cut)) continue;
         const double own = (f.step_us + f.wide_us * (double)(t * splits) / (double)cu * (double)K / 1e4) * (double)steps +
-                           f.store_us * (double)splits * mn / 1e6 + (splits > 1 ? f.cut_us : f.whole_us)[behind];
+                           f.store_us * (double)splits * mn / 1e6 + (splits > 1 ? f.cut_us : f.whole_us)[behind] +
+                           (splits == 1 && behind == 2 && M > 2200 ? 0.0026 * (double)(M - 2200) : 0.);
         if (own < us) best = TilePlan{VARIANT_STREAM + f.i, (int)splits, splits > 1 ? (int)steps * 64 : K, us = own};
       }
     }

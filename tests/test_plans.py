@@ -418,3 +418,10 @@ def test_stream_plan_follows_tiles_and_results():
                 changes.setdefault(129 + i, []).append((n, k, behind))
     assert changes
     assert not {m: at for m, at in changes.items() if m % 32 != 1 and len(at) > 2}
+
+
+@pytest.mark.parametrize("m,n,k", [(1400, 1536, 320), (1400, 1536, 512), (3169, 896, 4864), (3379, 896, 4864), (2721, 1024, 4096), (3995, 768, 3072), (3281, 640, 2560), (4310, 640, 2560), (3372, 1000, 2816)])
+def test_stream_plan_in_front_of_the_norm(m, n, k):
+    """A K of a few hundred; and thousands of rows against few weight rows: whole in `tile_stream_kernel` with a norm kernel behind it they took 2 to 12 % longer than in the
+    parts that the kernel with the norm adds."""
+    assert ops._tile_plan(m, n, k, ops.EPI_ACC_F32, True, 256, 2, True) == ops._tile_plan(m, n, k, ops.EPI_ACC_F32, True, 256, 2, False)

@@ -57,7 +57,8 @@ def test_refused():
 
 # the plan's own choice: parts of K in front of the rotation and of the norm, and whole; a last part that is shorter, rows past whole tiles
 @pytest.mark.parametrize("m,n,k,behind", [(470, 2560, 2048, 1), (300, 4608, 3584, 1), (150, 4608, 3584, 1), (257, 1536, 8960, 2), (203, 3584, 3584, 2),
-                                          (150, 2048, 11008, 2), (1000, 1024, 4096, 2), (300, 8192, 4096, 0), (520, 6144, 3584, 0)])
+                                          (150, 2048, 11008, 2), (1000, 1024, 4096, 2), (300, 8192, 4096, 0), (520, 6144, 3584, 0), (2651, 768, 3072, 2),
+                                          (2994, 1024, 4096, 0)])
 def test_planned(m, n, k, behind):
     from minfer_amd.kernels import ops
     x, w, bias = _operands(m, n, k)
