@@ -100,8 +100,9 @@ class DecoderModel:
             yield from block.parts()
 
     def _make_decode_copies(self) -> int:
-        """The parts' second copies of their matrices for the steps of few tokens (a layout that
-        those steps' products read faster): of all matrices where that takes at most a third of
+        """The parts' second copies of their matrices (a layout that products read faster, those of few
+        tokens above all; those of 129 to some 2,000 rows may cut K elsewhere with it than without, so
+        that the sums differ in their last bits): of all matrices where that takes at most a third of
         the device memory that is free once the weights are in place, else of those with rows of
         16,384 and more (the down products, which gain most) under the same condition, else
         none, so that a model that fills the device keeps its memory for the cache.  Returns

@@ -18,7 +18,8 @@ Kernel choice, for measurements (each overrides what `ops` would pick by shape):
                         the lengths (default: shares in proportion to the keys)
 * MF_SKINNY_TARGET=n    blocks the K-split decode product aims at (default: one per CU)
 * MF_NO_SHARED_PAGES=1  a block of queries of the prompt attention keeps all its pages to itself
-* MF_NO_DECODE_COPIES=1 a model keeps no second, tiled copy of its matrices for the steps of few tokens
+* MF_NO_DECODE_COPIES=1 a model keeps no second, tiled copy of its matrices (steps of few tokens, and prompts of more
+                        than 64 tokens, whose sums may then come in another order)
 * MF_NO_FOLD=1          the RMS norm is a kernel of its own instead of being folded into the
                         product that follows it (steps of at most 16 rows)
 * MF_NO_LATENT_MFMA=1   the latent attention runs its plain kernel in bfloat16 as well, not the matrix-core one
