@@ -103,15 +103,15 @@ __device__ __forceinline__ bf16x8 load8_inside(const bf16* __restrict__ base, in
   return *reinterpret_cast<const bf16x8*>(base + (size_t)row * ld + k);
 }
 
-// Weights that no other workgroup reads.  From the tiled copy a load takes whole lines and is marked as read once: what the step reads
+// Weights that no other workgroup reads, marked as read once (ONCE) or not.  From the tiled copy a load takes whole lines and is marked as read once: what the step reads
 // again stays in the caches (microseconds without / with the mark, 8 rows, weights from memory: 152,064 x 6,144 326 / 292, 152,064 x
 // 3,584 194 / 175, 37,888 x 3,584 49.8 / 47.7, 4,608 x 3,584 10.5 / 9.7, 3,584 x 18,944 26.6 / 25.8; 64 rows, 37,888 x 3,584 53.4 / 48.7).  From the
 // matrix a load takes half a line of each of 16 rows, and the next step takes the other half: marked, the line is fetched twice (marked / not, 8 rows:
 // 152,064 x 6,144 392 / 344, 8,192 x 29,568 117 / 102, 3,584 x 18,944 35.8 / 31.4, 37,888 x 3,584 56.1 / 52.3; 64 rows:
-// 152,064 x 3,584 277 / 245).  Not for what several tiles of rows read (`whole_kernel`, the prompts' tiles).
-template <bool TILED>
+// 152,064 x 3,584 277 / 245), except with a short K (`launch_stationary16`).  Not for what several tiles of rows read (`whole_kernel`, the prompts' tiles).
+template <bool ONCE>
 __device__ __forceinline__ bf16x8 load_weights(const bf16* p) {
-  if constexpr (TILED) return __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(p));
+  if constexpr (ONCE) return __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(p));
   else return *reinterpret_cast<const bf16x8*>(p);
 }
 
@@ -2092,7 +2092,8 @@ struct NormArgs {
 // with the step RING further on, of this item or of the next one.
 // NW: waves of a block, each with a slice of NS steps of K: 8, K = 256 NS; or 7 with NS = 4 for a K
 // of 896 (14 heads of 64, the narrowest model of the family), which is no multiple of 256.
-template <int NS, int RING, int NT, bool PAIR, bool NORM, bool TILED, int NW = 8>
+// ONCE: the weights are marked as read once (`load_weights`).
+template <int NS, int RING, int NT, bool PAIR, bool NORM, bool TILED, int NW, bool ONCE>
 __global__ __launch_bounds__(NW * 64) void stationary16_kernel(const void* __restrict__ Av, int lda,
                                                                const bf16* __restrict__ W, int ldw,
                                                                const float* __restrict__ bias,
@@ -2142,7 +2143,7 @@ __global__ __launch_bounds__(NW * 64) void stationary16_kernel(const void* __res
   auto first_loads = [&](int j) {
     wcur[j] = w_operand<TILED>(Wp, ldw, KK, lane_wrow(c_begin, j), k0);
 #pragma unroll
-    for (int s = 0; s < RING; ++s) w[j][s] = load_weights<TILED>(wcur[j] + s * WSTEP);
+    for (int s = 0; s < RING; ++s) w[j][s] = load_weights<ONCE>(wcur[j] + s * WSTEP);
   };
   // The epilogue's place of this lane in an item: wave w adds up the sums of activation rows
   // [w 64 / COLS, (w + 1) 64 / COLS), all waves at once.  What the epilogue needs from memory (the
@@ -2315,8 +2316,8 @@ __global__ __launch_bounds__(NW * 64) void stationary16_kernel(const void* __res
           asm volatile("" : "+v"(acc[j]) : : "memory");
           __builtin_amdgcn_sched_barrier(0);
         }
-        if (s + RING < NS) w[j][s % RING] = load_weights<TILED>(wcur[j] + (s + RING) * WSTEP);
-        else if (next) w[j][s % RING] = load_weights<TILED>(wrow[j] + (s + RING - NS) * WSTEP);
+        if (s + RING < NS) w[j][s % RING] = load_weights<ONCE>(wcur[j] + (s + RING) * WSTEP);
+        else if (next) w[j][s % RING] = load_weights<ONCE>(wrow[j] + (s + RING - NS) * WSTEP);
         __builtin_amdgcn_sched_barrier(0);      // keep "use a register, then refill it" in this order
       }
     }
@@ -2393,29 +2394,42 @@ int launch_stationary16(const void* A, int lda, const bf16* W, int ldw, const fl
   // K keeps 8 to 10 loads of 1 KB in flight per wave, far more than a CU has outstanding anyway.
   constexpr int RING = stationary_ring(NS, NT);
   static_assert(NS % RING == 0 && 4 * NS + 4 * NT * RING <= 200, "activations and weight ring fit the registers");
-  if (norm) {
-    constexpr int smem = NW * NS * 32 * (int)sizeof(float);      // the norm's weight
-    auto kern = stationary16_kernel<NS, RING, NT, PAIR, true, TILED, NW>;
-    static bool configured = false;
-    if (!configured) {
-      hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, smem);
-      if (e != hipSuccess) return (int)e;
-      configured = true;
+  auto run = [&](auto ONCE) {
+    if (norm) {
+      constexpr int smem = NW * NS * 32 * (int)sizeof(float);      // the norm's weight
+      auto kern = stationary16_kernel<NS, RING, NT, PAIR, true, TILED, NW, decltype(ONCE)::value>;
+      static bool configured = false;
+      if (!configured) {
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+        if (e != hipSuccess) return (int)e;
+        configured = true;
+      }
+      if (fused.in_ssq || fused.out_g) return MF_NOT_BUILT;
+      kern<<<grid, NW * 64, smem, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, cols_total, unit, units / grid, units % grid,
+                                            epi, *norm, FusedNorm{});
+    } else if constexpr (PAIR || NS * NW * 32 <= STATIONARY_PLAIN_K) {
+      if (fused.out_g && (PAIR || grid > fused.out_parts)) return MF_NOT_BUILT;
+      stationary16_kernel<NS, RING, NT, PAIR, false, TILED, NW, decltype(ONCE)::value><<<grid, NW * 64, 0, stream>>>(
+          A, lda, W, ldw, bias, C, ldc, M, N, cols_total, unit, units / grid, units % grid, epi, NormArgs{nullptr, nullptr, 0.f}, fused);
+    } else {
+      return MF_NOT_BUILT;
     }
-    if (fused.in_ssq || fused.out_g) return MF_NOT_BUILT;
-    kern<<<grid, NW * 64, smem, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, cols_total, unit, units / grid, units % grid,
-                                      epi, *norm, FusedNorm{});
-  } else if constexpr (PAIR || NS * NW * 32 <= STATIONARY_PLAIN_K) {
-    if (fused.out_g && (PAIR || grid > fused.out_parts)) return MF_NOT_BUILT;
-    stationary16_kernel<NS, RING, NT, PAIR, false, TILED, NW><<<grid, NW * 64, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N,
-                                                                             cols_total, unit, units / grid,
-                                                                             units % grid, epi,
-                                                                             NormArgs{nullptr, nullptr, 0.f}, fused);
+    return mf_launch_status();
+  };
+  // Weights marked as read once: from the tiled copy, and from the matrix where a product that is not SwiGLU has a K of up to 2,048 and a block at
+  // most eight items (of four and of 19 the marked loads are the faster and the slower ones).  Marked / not, weights from memory, no copy,
+  // microseconds, 8 and 16 rows: 2,560 x 896 3.7 / 4.4 and 3.7 / 4.3, 9,216 x 1,024 6.2 / 6.8 and 6.7 / 7.1, 2,048 x 1,536 3.9 / 4.3 and level, 2,560 x 2,048
+  // 4.7 / 5.1 and 5.3 / 5.2, 28,672 x 2,048 27.2 / 28.5 and 28.2 / 29.8, with the norm folded in 2,048 x 1,536 4.8 / 5.2 and 5.7 / 5.8; but
+  // 151,936 x 1,536 with the norm 98.1 / 96.8 and 106.6 / 104.0 (one row 93.6 / 85.9), 3,072 x 2,560 6.2 / 5.9, 4,608 x 3,584 10.1 / 9.85, SwiGLU
+  // 9,728 x 896 6.3 / 6.2, 17,920 x 1,536 13.7 / 13.1 and 14.2 / 13.4.
+  if constexpr (TILED) {
+    return run(std::true_type{});
   } else {
-    return MF_NOT_BUILT;
+    if constexpr (!PAIR && NW * NS * 32 <= 2048)
+      if ((units / grid + 1) * unit <= 8 * 16 * NT) return run(std::true_type{});
+    return run(std::false_type{});
   }
-  return mf_launch_status();
 }
 
 // 17 to 64 rows against a wide matrix (at least 8 tiles of 16 weight rows for every CU): one block

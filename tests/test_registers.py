@@ -76,21 +76,29 @@ def _loads_marked_as_read_once(path, folder, names):
     return found
 
 
-def test_only_whole_lines_are_marked_as_read_once(tmp_path):
+def test_which_weights_are_marked_as_read_once(tmp_path):
     """The kernels of few rows mark the weights that they read from the tiled copy, whose loads take whole lines.  From the matrix a
-    load takes half a line of each row: marked, the line would be fetched again for the other half."""
+    load takes half a line of each row: marked, the line would be fetched again for the other half, and so none is but with a K of up to 2,048
+    in `stationary16_kernel`, where both halves are asked for close together."""
     from minfer_amd.kernels import build
     if not build.is_current("gemm_bf16"):
         build.compile_library("gemm_bf16")
     path = build.lib_path("gemm_bf16")
-    tiled = {}                                    # (the last of a kernel's yes-or-no parameters)
+    once, tiled = {}, 0                           # (the last yes-or-no parameters: the copy; of one kernel the mark behind it)
     for n in _scratch_bytes(path, str(tmp_path)):
-        kind = re.search(r"\d(stationary16|rolling16|skinny_ring|panel)_kernelI(?:L[ib]\d+E)*?Lb([01])E(?:Li\dE)?EE", n)
+        kind = re.search(r"\d(rolling16|skinny_ring|panel)_kernelI(?:L[ib]\d+E)*?Lb([01])EEE", n)
         if kind:
-            tiled[n] = kind.group(2) == "1"
-    assert len({n for n in tiled if tiled[n]}) == len(tiled) // 2 > 0
-    for n, (loads, marked, _) in _loads_marked_as_read_once(path, str(tmp_path), sorted(tiled)).items():
-        assert loads > 0 and (marked > 0) == tiled[n], (n, loads, marked)
+            once[n] = kind.group(2) == "1"
+            tiled += once[n]
+        kind = re.search(r"\d+stationary16_kernelILi(\d+)ELi\d+ELi\d+ELb([01])ELb[01]ELb([01])ELi(\d)ELb([01])EEE", n)
+        if kind:
+            steps, pair, copy, waves, mark = (int(x) for x in kind.groups())
+            once[n] = mark == 1
+            tiled += copy
+            assert mark >= copy and (mark == copy or (not pair and steps * waves * 32 <= 2048)), n
+    assert len(once) > 2 * tiled > 0
+    for n, (loads, marked, _) in _loads_marked_as_read_once(path, str(tmp_path), sorted(once)).items():
+        assert loads > 0 and (marked > 0) == once[n], (n, loads, marked)
 
 
 def test_experts_marked_loads_take_whole_lines(tmp_path):
