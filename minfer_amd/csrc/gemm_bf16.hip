@@ -1730,7 +1730,7 @@ __device__ __forceinline__ void norm_part_out(const FusedNorm& f, float sq, int 
 // registers of the two-buffer scheme above.  With K of many thousands and few weight rows
 // (the down projection) the chip is filled by loads in flight, not by blocks, and this is
 // what the time depends on.
-template <int NW, int S, bool TILED>
+template <int NW, int S, bool ALL, bool TILED>
 __global__ __launch_bounds__(NW * 64) void rolling16_kernel(const bf16* __restrict__ A, int lda,
                                                             const bf16* __restrict__ W, int ldw,
                                                             const float* __restrict__ bias,
@@ -1774,8 +1774,11 @@ __global__ __launch_bounds__(NW * 64) void rolling16_kernel(const bf16* __restri
     a[s] = *reinterpret_cast<const bf16x8*>(arow + at * 32);
   };
   auto multiply = [&](int s) { acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[s], w[s], acc, 0, 0, 0); };
-  if (steps_per_wave <= S) {   // a slice that the registers hold: all of it asked for at once (in a loop over the slice's length the
-                               // compiler waits for every step: a decode step of one sequence at the 0.5B widths 775 us so, 749 at once)
+  // ALL: a slice that the registers hold, all of it asked for at once (in a loop over the slice's length the
+  // compiler waits for every step: a decode step of one sequence at the 0.5B widths 775 us so, 749 at once).  A kernel of its own, for
+  // 4, 8, 12 and 16 steps: with the rounds beside it in one kernel for 16 steps, 16 rows, tiled copy, microseconds together / apart: 1,280 x 2,048
+  // 5.7 / 5.1, 1,152 x 3,584 7.6 / 7.1, 1,536 x 2,560 6.3 / 5.7, 1,024 x 1,024 3.8 / 3.65; 8 rows 4.9 / 4.4, 5.9 / 5.8, 5.0 / 4.8, 3.45 / 3.3.
+  if constexpr (ALL) {
 #pragma unroll
     for (int s = 0; s < S; ++s)
       if (s < T) load(s, s);
@@ -1788,7 +1791,10 @@ __global__ __launch_bounds__(NW * 64) void rolling16_kernel(const bf16* __restri
     // count what is in flight: past the slice's end it is the last step again (`rolling_steps` chooses S so that there are few).
     const int last = max(T, 1) - 1;
 #pragma unroll
-    for (int s = 0; s < S; ++s) load(s, min(s, last));
+    for (int s = 0; s < S; ++s) {
+      load(s, min(s, last));
+      __builtin_amdgcn_sched_barrier(0);         // in the order of their use (left to the compiler: 3,584 x 18,944 of 8 rows 26.2 us, 25.4 so)
+    }
     int base = 0;
     for (; base + 2 * S <= T; base += S) {
 #pragma unroll
@@ -1831,14 +1837,14 @@ __global__ __launch_bounds__(NW * 64) void rolling16_kernel(const bf16* __restri
   if (fused.out_g) norm_part_out<COLS>(fused, sq, e_m, e_c, M);
 }
 
-// How many steps `rolling16_kernel` holds for slices of `steps`: at most 16, the one whose rounds have the fewest steps past the end.  Every length
+// How many steps `rolling16_kernel` holds for slices of `steps` above 16: at most 16, the one whose rounds have the fewest steps past the end.  Every length
 // from 10 to 15 has shapes that it pays for (8 rows, tiled copy, weights from memory, microseconds with 16 steps only / 10, 12 and 16 / all):
 // 896 x 4,864 9.25 / 6.8 / 6.8 (10 steps), 2,048 x 5,632 11.0 / 9.4 / 9.1 (11), 2,048 x 11,008 15.8 / 15.7 / 14.9 (11), 1,536 x 8,960 14.0 / 11.65 /
 // 11.65 (12), 2,560 x 9,728 15.4 / 13.9 / 13.5 (13), 8,192 x 29,568 90 / 86 / 84.7 (13), 4,096 x 14,336 24.3 / 23.5 / 22.5 (14), 3,584 x 18,944
 // 29.0 / 29.4 / 27.5 (15).
 int rolling_steps(int steps) {
   int best = 16;
-  for (int s = 15; s >= 10 && steps > 16; --s)
+  for (int s = 15; s >= 10; --s)
     if ((steps + s - 1) / s * s < (steps + best - 1) / best * best) best = s;
   return best;
 }
@@ -1854,14 +1860,18 @@ int launch_rolling16(const bf16* A, int lda, const bf16* W, int ldw, const float
   rpb = rpb < 1 ? 1 : (rpb > 16 ? 16 : rpb);
   const int blocks = (N + rpb - 1) / rpb;
   if (fused.out_g && blocks > fused.out_parts) return MF_NOT_BUILT;
-  auto run = [&](auto S) {
-    rolling16_kernel<NW, decltype(S)::value, TILED><<<blocks, NW * 64, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K,
+  auto run = [&](auto S, auto ALL) {
+    rolling16_kernel<NW, decltype(S)::value, decltype(ALL)::value, TILED><<<blocks, NW * 64, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K,
                                                                                               steps_per_wave, epi, rpb, fused);
   };
-#define MF_ROLLING(S_) case S_: run(std::integral_constant<int, S_>{}); break;
-  switch (rolling_steps(steps_per_wave)) {
+#define MF_ROLLING(S_) case S_: run(std::integral_constant<int, S_>{}, std::false_type{}); break;
+  if (steps_per_wave <= 4) run(std::integral_constant<int, 4>{}, std::true_type{});
+  else if (steps_per_wave <= 8) run(std::integral_constant<int, 8>{}, std::true_type{});
+  else if (steps_per_wave <= 12) run(std::integral_constant<int, 12>{}, std::true_type{});
+  else if (steps_per_wave <= 16) run(std::integral_constant<int, 16>{}, std::true_type{});
+  else switch (rolling_steps(steps_per_wave)) {
     MF_ROLLING(10) MF_ROLLING(11) MF_ROLLING(12) MF_ROLLING(13) MF_ROLLING(14) MF_ROLLING(15)
-    default: run(std::integral_constant<int, 16>{});
+    default: run(std::integral_constant<int, 16>{}, std::false_type{});
   }
 #undef MF_ROLLING
   return mf_launch_status();
@@ -3256,6 +3266,8 @@ int dma_form(int variant, int M, int N, int K, int epi, long nkt, int splits, lo
 // the neighbouring rows and k beside them, which memory gives faster (weights from memory, row-major / tiled: SwiGLU of 22,016 x 2,048, 40 rows
 // 26.1 / 21.8 us, 64 rows 24.0 / 20.5, 100 rows 27.0 / 24.7; 37,888 x 3,584, 64 rows 53.5 / 51.0, 203 rows 73.3 / 72.1, 604 rows 166.1 / 163.1;
 // 3,584 x 18,944, 604 rows in three parts 98.4 / 93.9; 4,608 x 3,584, 2,048 rows 63.9 / 61.2; level where many rows share the weights).
+// Of 330 other products of 65 to 1,100 rows 0.975 of the time on average, 13 more than 2 % slower, none more than 6 % (6,144 x 8,192, 80
+// rows 30.8 / 32.6), with no line between them; of 260 in 64 x 64 tiles 0.974, one shape slower (28,672 x 512, 17 rows 9.9 / 10.7).
 // Not so 64 x 64 tiles of which no CU has two: their time is a chain of waits, with longer addresses in front of it
 // (2,560 x 2,048, 100 rows 7.4 / 7.7 us, 203 rows 10.0 / 10.4; 1,152 x 896, 604 rows 6.8 / 7.0).
 struct Weights {

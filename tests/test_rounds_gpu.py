@@ -14,8 +14,8 @@ def _operands(m, n, k):
     return x, w, torch.randn(n, generator=gen).to(DEV), torch.randn((m, n), generator=gen).to(DEV)
 
 
-# steps of 32 a wave (eight waves): 1, 2, 16, 17 .. 31, also with waves that have fewer of them
-@pytest.mark.parametrize("k", [32, 96, 416, 3936, 4128, 4352, 4384, 4640, 4864, 5376, 5632, 5920, 6400, 6688, 7424, 7904, 7936])
+# steps of 32 a wave (eight waves): 1, 2, 4, 5, 8, 9, 12, 13, 16, 17 .. 31, also with waves that have fewer of them
+@pytest.mark.parametrize("k", [32, 96, 416, 1024, 1056, 2048, 2080, 3072, 3104, 3936, 4128, 4352, 4384, 4640, 4864, 5376, 5632, 5920, 6400, 6688, 7424, 7904, 7936])
 @pytest.mark.parametrize("m,n", [(1, 80), (16, 896)])
 def test_rolling(m, n, k):
     from minfer_amd.kernels import ops
